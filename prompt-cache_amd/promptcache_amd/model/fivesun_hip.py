@@ -6,9 +6,9 @@ products on the bf16 matrix cores, fp32 accumulation) or float32 (everything in 
 another, each request continuing from what its slot of the ``SlotArena`` holds.  Nothing is padded, and a row reads nothing but
 its own slot, so a request's numbers do not depend on the rest of the step.
 
-What a slot holds differs by layer: an attention layer keeps keys (row by row, normed and rotated) and values (column by column,
-normed and blended), a latent-attention layer ONE row per token -- the normed latent followed by the rotated shared key part --,
-an mLSTM layer its fp32 matrix memory, normaliser and running maximum.
+What a slot holds differs by layer: an attention layer keeps rows ``key | value`` (keys normed and rotated, values normed and
+blended), a latent-attention layer ONE row per token -- the normed latent followed by the rotated shared key part --, an mLSTM
+layer its fp32 matrix memory, normaliser and running maximum.
 
 The residual x is fp32.  Sublayer by sublayer (f = mixer or feed-forward, each between a norm before and a norm after it):
 
@@ -18,13 +18,15 @@ The residual x is fp32.  Sublayer by sublayer (f = mixer or feed-forward, each b
 same projection as the mixer's inputs (or is one projection beside the feed-forward's).
 
     attention   q | k | v | g | r = ONE projection (sigmoid on g | r); pcb_head_prep: per-head RMS norms, rotary pairs (angles as
-                float64 products), value blend with the first blending layer's values, keys / values into the slot's cache;
-                pcb_attn_softmax: keys of the query's own block of positions only, exp(sink_h) in the denominator, one gate per head
+                float64 products), value blend with the first blending layer's values, ``key | value`` rows into the slot's cache;
+                keys of the query's own block of positions only, exp(sink_h) in the denominator, one gate per head: tiles of
+                queries for requests that bring many tokens (pcb_attn_prompt), single rows for the others (pcb_attn_rows)
     latent      q | down | g | r = ONE projection; pcb_head_prep: the latent normed, the shared key part and the queries' rotated
-                parts turned (YaRN frequencies), latent | key part into the slot's row.  The keys' and values' up-projections are
-                folded into the query and the output: q'_h = W_uk,h^T q_h (grouped pcb_linear), attention of [q'_h | q_rot,h] over
-                the cached rows with the latent itself as value (pcb_attn_softmax, one key head, sliding window), o_h = W_uv,h (.)
-                (grouped pcb_linear), times sigmoid(g)
+                parts turned (YaRN frequencies), latent | key part into the slot's row.  A request that brings many tokens has the
+                keys and values of all heads rebuilt from the latents (pcb_linear) and attends in tiles (pcb_attn_prompt, the shared
+                key part read from the cached rows, times sigmoid(g)); for the others the up-projections are folded into the query
+                and the output: q'_h = W_uk,h^T q_h, attention of [q'_h | q_rot,h] over the cached rows with the latent itself as
+                value (pcb_attn_latent, sliding window), o_h = W_uv,h (.), times sigmoid(g).  Heads too wide for the tiles fold always
     mlstm       q | k | v | i | f | g | r = ONE projection; pcb_mlstm: the gated matrix memory token by token; per-head unit RMS,
                 gain, sigmoid(g) (pcb_gated_norm)
     dense ff    act(W_gate h + b) * (W_up h + b) in one projection's epilogue, then W_down (.) + b
@@ -43,7 +45,7 @@ import torch
 from .. import _blocks as B
 from .config import FivesunShape
 from .kv_arena import SlotArena
-from .slot_model import SlotKV, SlotModel  # noqa: F401
+from .slot_model import SlotKV, SlotModel, StepRows  # noqa: F401
 
 ACTS = {"relu": B.ACT_RELU, "silu": B.ACT_SILU, "gelu_tanh": B.ACT_GELU_TANH}
 
@@ -68,6 +70,10 @@ class FivesunHIP(SlotModel):
     GRAPH_MAX_ROWS = 64
     SEGMENT = int(os.environ.get("PC_FS_SEGMENT", "64"))    # a step that brings a request more tokens than this runs its mLSTM layers segment-parallel
     MAX_SEGMENTS = 128      # (segments grow beyond SEGMENT tokens rather than exceed this many per request)
+    # A request that brings at least this many tokens attends in tiles of 64 or 128 queries, another row by row: a tile of 64 with 16
+    # live rows costs what 16 single rows cost (one pass over the keys per head against one per row and 16 heads).
+    PROMPT_ROWS = int(os.environ.get("PC_FS_PROMPT_ROWS", "16"))
+    REBUILD_RATIO = 64      # ... but folds its queries, instead of rebuilding the keys, if it brings less than a 64th of what they number
 
     def __init__(self, shape: FivesunShape, weights: Dict[str, torch.Tensor], device="cuda:0", dtype=torch.bfloat16,
                  decode_headroom: int = 256):
@@ -117,8 +123,10 @@ class FivesunHIP(SlotModel):
                     raise ValueError(f"layer {i}: a latent of up to 256 columns plus a rotated part within 384 together (got {C} + {R})")
                 HQ, HV = l.heads * (l.dim + R), l.heads * l.vdim
                 fr, mag = rotary_frequencies(l.rot_base, R, l.rot_factor, l.yarn_original, l.yarn_fast, l.yarn_slow) if R else (np.zeros(0), 1.0)
+                # (the tiled attention takes heads of up to 256 key and 256 value columns)
                 ent.update(w_in=torch.cat([e(m + "q"), e(m + "dkv"), e(m + "g"), rg], dim=0).contiguous(),
                            b_in=torch.cat([zeros(HQ + C + R + HV), rgb]).contiguous(), act_from=HQ + C + R,
+                           prompts=l.dim + R <= 256 and l.vdim <= 256, w_kv=torch.cat([e(m + "uk"), e(m + "uv")], dim=0).contiguous(),
                            c_gain=f(m + "dkv.norm"), wo=e(m + "o"),
                            # per head: the key up-projection transposed ([C, dim]: it maps a query to the latent's columns) and the
                            # value up-projection as stored ([vdim, C])
@@ -145,25 +153,30 @@ class FivesunHIP(SlotModel):
         self.use_graphs = os.environ.get("PC_FS_GRAPHS", "1") != "0"      # one-token steps replay a captured hipGraph
         self._graphs = {}
         self.max_graphs = 16
-        # cache offsets of a row, one table per distinct (heads, columns) of the row-wise planes and of the column-wise planes
-        att = [l for l in shape.layers if l.kind == "attention"]
-        self._sigs = sorted({(l.kv_heads, l.dim) for l in att} | {(1, l.kv_rank + l.rot_dim) for l in shape.layers if l.kind == "latent_attention"})
-        self._vsigs = sorted({(l.kv_heads, l.vdim) for l in att})
-        # (token, head) row orders of the per-head projections around the latent attention, one table per distinct head count
-        self._perm_heads = sorted({l.heads for l in shape.layers if l.kind == "latent_attention"})
+        # cache offsets of a row, one table per distinct (heads, columns) of the planes
+        self._sigs = sorted({(l.kv_heads, l.dim + l.vdim) for l in shape.layers if l.kind == "attention"} |
+                            {(1, l.kv_rank + l.rot_dim) for l in shape.layers if l.kind == "latent_attention"})
+        latent = [ent for ent in self.layers if ent["cfg"].kind == "latent_attention"]
+        self._rebuilds = any(ent["prompts"] for ent in latent)
+        self._folds = any(not ent["prompts"] for ent in latent)
+        # positions behind a request's first new token whose keys its rebuilding layers need (0: all of them)
+        reach = [ent["cfg"].mask for ent in latent if ent["prompts"]]
+        self._reach = 0 if not reach or min(reach) <= 0 else max(reach)
+        self._wide = any(ent["cfg"].kind == "attention" and ent["cfg"].dim > 256 for ent in self.layers)
+        self._max_heads = max(l.heads for l in shape.layers)
 
     # ---- cache and state -------------------------------------------------------------------------------------------------------
     def new_arena(self, slots: int, cap: int) -> SlotArena:
-        dims, cols, states = [], [], []
+        dims, states = [], []
         for l in self.config.layers:
             if l.kind == "attention":
-                dims.append((l.kv_heads, l.dim)); cols.append((l.kv_heads, l.vdim)); states.append([])
+                dims.append((l.kv_heads, l.dim + l.vdim)); states.append([])
             elif l.kind == "latent_attention":
-                dims.append((1, l.kv_rank + l.rot_dim)); cols.append((0, 0)); states.append([])
+                dims.append((1, l.kv_rank + l.rot_dim)); states.append([])
             else:
-                dims.append((0, 0)); cols.append((0, 0))
+                dims.append((0, 0))
                 states.append([((B.mlstm_state_floats(l.heads, l.dim, l.vdim),), torch.float32)])
-        return SlotArena(dims, slots, cap, self.device, self.dtype, states=states, col_dims=cols)
+        return SlotArena(dims, slots, cap, self.device, self.dtype, states=states)
 
     def kv_bytes_per_token(self) -> int:
         es = 2 if self.dtype == torch.bfloat16 else 4
@@ -178,52 +191,61 @@ class FivesunHIP(SlotModel):
         """Append ``tokens[b]`` behind slot ``slots[b]`` for every b, and return fp32 logits ``[n_wanted, vocab]`` for the places
         ``want[b]`` (indices into ``tokens[b]``; default: each request's last token), in request order.
         ``return_streams``: also the residual stream after each layer, fp32 ``[layers, rows, width]`` (for tests)."""
-        dev, f32 = self.device, torch.float32
-        counts = [len(t) for t in tokens]
-        if len(set(slots)) != len(slots) or len(slots) != len(tokens):
-            raise ValueError("one distinct slot per request")
-        if not counts:
-            return torch.empty((0, self.V), dtype=f32, device=dev)
-        if min(counts) < 1:
-            raise ValueError("every request of a step brings at least one token")
-        T, R = sum(counts), len(counts)
-        if want is None:
-            want = [[c - 1] for c in counts]
-        for s, c in zip(slots, counts):
-            arena.room_for(s, c)
-        starts = [arena.lengths[s] for s in slots]
-        V = self.V
-
-        ids = np.fromiter((t for req in tokens for t in req), dtype=np.int32, count=T)
-        if ids.min() < 0 or ids.max() >= V:
-            raise ValueError("token id outside the vocabulary")
-        for b, ws in enumerate(want):
-            if any(not 0 <= int(w) < counts[b] for w in ws):
-                raise ValueError("a wanted place lies outside its request's tokens")
-        row0 = np.concatenate([[0], np.cumsum(counts)]).astype(np.int64)
-        row_slot = np.repeat(np.asarray(slots, dtype=np.int64), counts)
-        row_pos = np.concatenate([np.arange(c, dtype=np.int64) for c in counts]) + np.repeat(np.asarray(starts, dtype=np.int64), counts)
-        reqs = np.asarray([(s, st, c, int(row0[b])) for b, (s, st, c) in enumerate(zip(slots, starts, counts))], dtype=np.int32)
-        tiles = np.asarray([(s, st + q, min(16, c - q), int(row0[b]) + q) for b, (s, st, c) in enumerate(zip(slots, starts, counts))
-                            for q in range(0, c, 16)], dtype=np.int32).reshape(-1, 4)
+        dev = self.device
+        if not tokens and not slots:
+            return torch.empty((0, self.V), dtype=torch.float32, device=dev)
+        st = StepRows(arena, slots, tokens, want, self.V)
+        T, R, cap, row0, counts, starts = st.T, st.R, arena.cap, st.row0, st.counts, st.starts
         graphed = (self.use_graphs and T <= self.GRAPH_MAX_ROWS and all(c == 1 for c in counts) and num_layers is None
                    and not return_streams)
-        picked = None
-        if graphed and any(len(ws) != 1 for ws in want):
-            picked = [b for b, ws in enumerate(want) for _ in ws]
-        want_rows = np.arange(T, dtype=np.int32) if graphed else \
-            np.asarray([int(row0[b]) + int(w) for b, ws in enumerate(want) for w in ws], dtype=np.int32)
-        # rows of the per-head projections: bucket h holds (token, head h) for every token; perm[h * T + t] = t * H + h
-        perms = [np.concatenate([(np.arange(T, dtype=np.int32) * H + h) for h in range(H)] + [np.arange(H + 1, dtype=np.int32) * T])
-                 for H in self._perm_heads]
+        picked, want_rows = None, st.want_rows
+        if graphed:
+            if any(len(ws) != 1 for ws in st.want):
+                picked = [b for b, ws in enumerate(st.want) for _ in ws]
+            want_rows = np.arange(T, dtype=np.int32)
+        reqs = np.asarray([(s, s0, c, int(row0[b])) for b, (s, s0, c) in enumerate(zip(slots, starts, counts))], dtype=np.int32)
+
+        def row_tiles(rows):
+            return np.stack([st.row_slot[rows], st.row_pos[rows], np.ones(rows.size, np.int64), rows], axis=1).astype(np.int32)
+
+        def rows_of(which):
+            return np.concatenate([np.arange(row0[b], row0[b + 1]) for b in which]).astype(np.int32) if which else np.zeros(0, np.int32)
+
+        # attention: tiles of neighbouring queries for requests that bring many tokens, single rows for the others
+        big = [b for b, c in enumerate(counts) if c >= self.PROMPT_ROWS]
+        # the oldest key that the rebuilding layers need (a whole number of the kernel's blocks of keys)
+        oldest = [max(0, s0 - self._reach + 1) // 64 * 64 if self._reach else 0 for s0 in starts]
+        rebuilt = [b for b in big if self._rebuilds and starts[b] + counts[b] - oldest[b] <= self.REBUILD_RATIO * counts[b]]
+        tile = 64
+        if self.dtype == torch.bfloat16 and sum(-(-counts[b] // 128) for b in big) * self._max_heads >= 512:
+            tile = 128
+
+        def tiles_of(which, base):
+            t = [(base[b], starts[b] + q, min(tile, counts[b] - q), int(row0[b]) + q) for b in which for q in range(0, counts[b], tile)]
+            t.sort(key=lambda t: t[1] + t[2])     # (longer contexts behind the shorter ones: the kernel starts from the last tile)
+            return np.asarray(t, dtype=np.int32).reshape(-1, 4)
+
+        kv_rows, base, at = [], {}, 0
+        for b in rebuilt:
+            n, lo = starts[b] + counts[b], oldest[b]
+            # (whole blocks of 32 rows: the padding repeats the last one; the cached row of position j lies at base + j)
+            src = slots[b] * cap + np.minimum(np.arange(lo, lo + -(-(n - lo) // 32) * 32, dtype=np.int64), n - 1)
+            kv_rows.append(src.astype(np.int32))
+            base[b] = at - lo
+            at += src.size
+        if rebuilt and arena.slots * cap >= 1 << 31:
+            raise ValueError("more than 2^31 cached rows in one plane")
+        s_rows = rows_of([b for b in range(R) if b not in set(big)])
+        f_rows = rows_of([b for b in range(R) if b not in set(rebuilt)])
+        every = np.arange(T, dtype=np.int32)
         # segments of the matrix memories' prefill (only when some request brings more than SEGMENT tokens)
         seg_a = seg_c = chains = np.zeros((0, 4), np.int32)
         seg_end = np.zeros(0, np.int32)
         if max(counts) > self.SEGMENT and any(l.kind == "mlstm" for l in self.config.layers):
             seg = max(self.SEGMENT, -(-max(counts) // self.MAX_SEGMENTS))
             sa, ch = [], []
-            for b, (s, st, c) in enumerate(zip(slots, starts, counts)):
-                ch.append((s, st, len(sa), -(-c // seg)))
+            for b, (s, s0, c) in enumerate(zip(slots, starts, counts)):
+                ch.append((s, s0, len(sa), -(-c // seg)))
                 sa += [(len(sa) + k, 0, min(seg, c - q), int(row0[b]) + q) for k, q in enumerate(range(0, c, seg))]
             seg_a = np.asarray(sa, dtype=np.int32)
             seg_c = seg_a.copy()
@@ -231,22 +253,27 @@ class FivesunHIP(SlotModel):
             chains = np.asarray(ch, dtype=np.int32)
             seg_end = np.full(len(sa), -1, dtype=np.int32)  # a request's last segment leaves the slot's new state
             seg_end[chains[:, 2] + chains[:, 3] - 1] = chains[:, 0]
-        offs = np.stack([row_slot * (g * arena.cap * d) + row_pos * d for g, d in self._sigs] +
-                        [row_slot * (g * d * arena.cap) + row_pos for g, d in self._vsigs]) if self._sigs else np.zeros((0, T), np.int64)
-        # one block: int32 tables, then int64 cache offsets
-        parts32 = [ids, row_pos.astype(np.int32), reqs.reshape(-1), tiles.reshape(-1), want_rows, seg_a.reshape(-1), seg_c.reshape(-1),
-                   chains.reshape(-1), seg_end] + perms
-        n32 = sum(p.size for p in parts32)
+        offs = np.stack([st.row_slot * (g * cap * d) + st.row_pos * d for g, d in self._sigs]) if self._sigs else np.zeros((0, T), np.int64)
+        tables = dict(ids=st.ids, pos=st.row_pos.astype(np.int32), want=want_rows, reqs=reqs, p_tiles=tiles_of(big, slots),
+                      s_tiles=row_tiles(s_rows), l_tiles=tiles_of(rebuilt, base), kv_rows=np.concatenate(kv_rows) if kv_rows else every[:0],
+                      f_tiles=row_tiles(f_rows), f_rows=f_rows if rebuilt else every[:0],
+                      # every row by itself, for layers that fold all rows; tiles of 16 queries, for heads too wide for the others
+                      a_tiles=row_tiles(every) if rebuilt and self._folds else every[:0],
+                      w_tiles=np.asarray([(s, s0 + q, min(16, c - q), int(row0[b]) + q) for b, (s, s0, c) in enumerate(zip(slots, starts, counts))
+                                          for q in range(0, c, 16)], dtype=np.int32).reshape(-1, 4) if self._wide else every[:0],
+                      seg_a=seg_a, seg_c=seg_c, chains=chains, seg_end=seg_end)
+        sizes = {k: v.size for k, v in tables.items()}
+        n32 = sum(sizes.values())
         o64 = (n32 * 4 + 7) // 8 * 8
+        # one block: int32 tables, then int64 cache offsets
         blob = np.empty(o64 + offs.size * 8 + 8, dtype=np.uint8)
-        blob[:n32 * 4].view(np.int32)[:] = np.concatenate(parts32)
+        blob[:n32 * 4].view(np.int32)[:] = np.concatenate([v.reshape(-1) for v in tables.values()])
         blob[o64:o64 + offs.size * 8].view(np.int64)[:] = offs.reshape(-1)
-        dims = dict(T=T, R=R, n_tiles=tiles.shape[0], n_want=int(want_rows.size), n32=n32, o64=o64, n_seg=seg_a.shape[0],
-                    n_chains=chains.shape[0])
+        dims = dict(T=T, R=R, n_want=int(want_rows.size), n32=n32, o64=o64, sizes=sizes, tile=tile)
         res = self._decode_graphed(arena, blob, dims) if graphed else None
         if res is None:
             dblob = torch.from_numpy(blob).to(dev)
-            logits = torch.empty((dims["n_want"], V), dtype=f32, device=dev)
+            logits = torch.empty((dims["n_want"], self.V), dtype=torch.float32, device=dev)
             res = self._run(arena, dblob, dims, logits, num_layers, return_streams)
         for s_, c in zip(slots, counts):
             arena.lengths[s_] += c
@@ -255,18 +282,13 @@ class FivesunHIP(SlotModel):
         return res
 
     def _tables(self, dblob, d):
-        T, R, nt, nw = d["T"], d["R"], d["n_tiles"], d["n_want"]
         i32 = dblob[:d["n32"] * 4].view(torch.int32)
-        at, out = 0, {}
-        ns = d["n_seg"]
-        out["n_seg"], out["n_chains"] = ns, d["n_chains"]
-        for name, n in [("ids", T), ("pos", T), ("reqs", 4 * R), ("tiles", 4 * nt), ("want", nw), ("seg_a", 4 * ns), ("seg_c", 4 * ns),
-                        ("chains", 4 * d["n_chains"]), ("seg_end", ns)] + \
-                       [(("perm", H), T * H + H + 1) for H in self._perm_heads]:
+        at, out = 0, dict(tile=d["tile"], n_seg=d["sizes"]["seg_end"], n_chains=d["sizes"]["chains"] // 4)
+        for name, n in d["sizes"].items():
             out[name] = i32[at:at + n]
             at += n
-        no = len(self._sigs) + len(self._vsigs)
-        out["offs"] = dblob[d["o64"]:d["o64"] + no * T * 8].view(torch.int64).view(no, T)
+        no = len(self._sigs)
+        out["offs"] = dblob[d["o64"]:d["o64"] + no * d["T"] * 8].view(torch.int64).view(no, d["T"])
         return out
 
     def _run(self, arena, dblob, d, logits, num_layers=None, return_streams=False):
@@ -291,7 +313,7 @@ class FivesunHIP(SlotModel):
         for i, lw in enumerate(layers):
             l = lw["cfg"]
             step(lw["norm1"], h)
-            gate, ldg = getattr(self, "_" + l.kind)(arena, i, l, lw, h, y1, tb, T, R, d["n_tiles"])
+            gate, ldg = getattr(self, "_" + l.kind)(arena, i, l, lw, h, y1, tb, T, R)
             pending = dict(y=y1, gate=gate, ldg=ldg, post_gain=lw["norm1b"])
             if l.ff:
                 step(lw["norm2"], h)
@@ -319,68 +341,95 @@ class FivesunHIP(SlotModel):
         B.linear(h, lw["w_in"], P, M=T, bias=lw["b_in"], act_split=lw["act_from"], act2=B.ACT_SIGMOID)
         return P, N
 
-    def _splits(self, arena, n_tiles, heads):
-        # few (tile, head) pairs cannot fill the chip: each is cut into runs of its keys (steps of few rows over long caches)
-        return 1 if n_tiles * heads >= 512 or arena.cap <= 256 else max(1, min(16, 1024 // (n_tiles * heads), arena.cap // 128))
+    def _splits(self, n, head_groups, reach):
+        # few (row, group of heads) pairs cannot fill the chip: each is cut into runs of its keys, as many as blocks of 64 fit what it sees
+        blocks = -(-reach // 64)
+        return 1 if blocks <= 3 else max(1, min(64, 512 // (n * head_groups), blocks))
 
-    def _attention(self, arena, i, l, lw, h, y, tb, T, R, n_tiles):
+    def _attention(self, arena, i, l, lw, h, y, tb, T, R):
         E = self.dtype
         H, G, D, Dv = l.heads, l.kv_heads, l.dim, l.vdim
         HD, GD, GV = H * D, G * D, G * Dv
         P, N = self._project_in(lw, h, T)
-        plane, vplane = arena.planes[i], arena.col_planes[i]
+        plane = arena.planes[i]
         q = self._mat("q_rows", T, HD, E)
         vf = self._mat("v_first", T, GV, torch.float32) if l.v_mix else None
+        row = dict(row_off=tb["offs"][self._sigs.index((G, D + Dv))], head_stride=arena.head_stride(i))
         segs = [B.head_seg(P, N, H, D, q, norm=True, gain=lw["q_gain"], rot_dims=l.rot_dims, ld_dst=HD),
-                B.head_seg(P[:, HD:], N, G, D, plane, norm=True, gain=lw["k_gain"], rot_dims=l.rot_dims,
-                           row_off=tb["offs"][self._sigs.index((G, D))], head_stride=arena.head_stride(i)),
-                B.head_seg(P[:, HD + GD:], N, G, Dv, vplane, norm=True, blend=lw["blend"], other=vf if lw["blend"] is not None else None,
-                           keep=vf if i == self.first_v_mix else None,
-                           row_off=tb["offs"][len(self._sigs) + self._vsigs.index((G, Dv))], head_stride=arena.col_head_stride(i),
-                           col_stride=arena.cap)]
+                B.head_seg(P[:, HD:], N, G, D, plane, norm=True, gain=lw["k_gain"], rot_dims=l.rot_dims, **row),
+                B.head_seg(P[:, HD + GD:], N, G, Dv, plane, norm=True, blend=lw["blend"], other=vf if lw["blend"] is not None else None,
+                           keep=vf if i == self.first_v_mix else None, dst_offset=D, **row)]
         B.head_prep(segs, T, E, pos=tb["pos"], freqs=lw["freqs"], rot_mag=lw["rot_mag"], eps=self.config.norm_eps)
         att = self._mat("mix_out", T, H * Dv, E)
-        splits = self._splits(arena, n_tiles, H)
-        part = self._scratch("attn_part", B.attn_softmax_part(T, H, splits, Dv), torch.float32) if splits > 1 else None
-        B.attn_softmax(q, HD, tb["tiles"], n_tiles, plane, (arena.slot_stride(i), arena.head_stride(i), D), vplane, 0,
-                       (arena.col_slot_stride(i), arena.col_head_stride(i), arena.cap), True, H, G, D, Dv, l.scale, att,
-                       block=l.mask, sink=lw["sink"], gate=P[:, HD + GD + GV:], ldg=N, gate_per_head=True, n_splits=splits, part=part)
+        values, gate = plane.view(-1)[D:], P[:, HD + GD + GV:]
+        ss, hs, rs = arena.slot_stride(i), arena.head_stride(i), D + Dv
+        reach = min(arena.cap, l.mask or arena.cap)
+        if D > 256:
+            n = tb["w_tiles"].numel() // 4
+            splits = 1 if n * H >= 512 or arena.cap <= 256 else max(1, min(16, 1024 // (n * H), arena.cap // 128))
+            part = self._scratch("attn_part", B.attn_softmax_part(T, H, splits, Dv), torch.float32) if splits > 1 else None
+            B.attn_softmax(q, HD, tb["w_tiles"], n, plane, (ss, hs, rs), plane, D, (ss, hs, rs), False, H, G, D, Dv, l.scale, att,
+                           block=l.mask, sink=lw["sink"], gate=gate, ldg=N, gate_per_head=True, n_splits=splits, part=part)
+        else:
+            kw = dict(ldo=H * Dv, block=l.mask, sink=lw["sink"], gate=gate, ldg=N)
+            n = tb["p_tiles"].numel() // 4
+            if n:
+                B.attn_prompt(q, tb["p_tiles"], n, tb["tile"], plane, (rs, hs, ss), values, (rs, hs, ss), H, G, D, Dv, l.scale, att, **kw)
+            n = tb["s_tiles"].numel() // 4
+            if n:
+                splits = self._splits(n, G * -(-H // (16 * G)), reach)
+                part = self._scratch("attn_part", B.attn_softmax_part(n, H, splits, Dv), torch.float32) if splits > 1 else None
+                B.attn_rows(q, tb["s_tiles"], n, plane, (ss, hs, rs), values, (ss, hs, rs), H, G, D, Dv, l.scale, att, gate_per_head=True,
+                            n_splits=splits, part=part, **kw)
         B.linear(att, lw["wo"], y, M=T)
         return P[:, HD + GD + GV + H:], N
 
-    def _latent_attention(self, arena, i, l, lw, h, y, tb, T, R, n_tiles):
+    def _latent_attention(self, arena, i, l, lw, h, y, tb, T, R):
         E = self.dtype
         H, D, Rd, Dv, C = l.heads, l.dim, l.rot_dim, l.vdim, l.kv_rank
-        HQ, HV, CR = H * (D + Rd), H * Dv, C + Rd
+        DR, HQ, HV, CR = D + Rd, H * (D + Rd), H * Dv, C + Rd
         P, N = self._project_in(lw, h, T)
         plane = arena.planes[i]
         off = tb["offs"][self._sigs.index((1, CR))]
-        qn = self._mat("q_rows", T, H * D, E)                 # the queries' unrotated parts, head by head
-        qa = self._mat("q_latent", T, H * CR, E)              # per head [W_uk^T q | rotated part]: a query over the cached rows
-        segs = [B.head_seg(P, N, H, D, qn, src_head_stride=D + Rd, ld_dst=H * D),
-                B.head_seg(P[:, HQ:], N, 1, C, plane, norm=True, gain=lw["c_gain"], row_off=off)]
+        tiled = lw["prompts"] and tb["l_tiles"].numel() > 0
+        f_tiles = tb["f_tiles"] if lw["prompts"] or not tb["a_tiles"].numel() else tb["a_tiles"]
+        n = f_tiles.numel() // 4
+        qa = self._mat("q_latent", T, H * CR, E) if n else None   # per head [W_uk^T q | rotated part]: a query over the cached rows
+        q = self._mat("q_rows", T, HQ, E) if tiled else None      # per head [plain part | rotated part]: a query over rebuilt rows
+        segs = [B.head_seg(P[:, HQ:], N, 1, C, plane, norm=True, gain=lw["c_gain"], row_off=off)]
+        if tiled:
+            segs.append(B.head_seg(P, N, H, D, q, src_head_stride=DR, ld_dst=HQ, head_stride=DR))
         if Rd:
-            segs += [B.head_seg(P[:, D:], N, H, Rd, qa, src_head_stride=D + Rd, rot_dims=Rd, ld_dst=H * CR, head_stride=CR, dst_offset=C),
-                     B.head_seg(P[:, HQ + C:], N, 1, Rd, plane, rot_dims=Rd, row_off=off, dst_offset=C)]
-        B.head_prep(segs, T, E, pos=tb["pos"], freqs=lw["freqs"], rot_mag=lw["rot_mag"], eps=self.config.norm_eps)
-        perm = tb[("perm", H)]
-        rows, goff = perm[:T * H], perm[T * H:]
-        B.linear(qn.view(T * H, D), lw["w_abs"], qa.view(T * H, CR), M=T * H, row_src=rows, row_dst=rows, group_off=goff, n_groups=H,
-                 ldy=CR)
-        ol = self._mat("mix_out", T, H * C, E)
-        one_each = T == R                                    # one token per request: 16 heads share a pass over the slot's rows
-        splits = self._splits(arena, n_tiles, -(-H // 16) if one_each else H)
-        part = self._scratch("attn_part", B.attn_softmax_part(T, H, splits, C), torch.float32) if splits > 1 else None
-        B.attn_softmax(qa, H * CR, tb["tiles"], n_tiles, plane, (arena.slot_stride(i), 0, CR), plane, 0, (arena.slot_stride(i), 0, CR),
-                       False, H, 1, CR, C, l.scale, ol, window=l.mask, n_splits=splits, part=part, head_rows=one_each)
-        ov = self._mat("mix_o32", T, HV, torch.float32)
-        B.linear(ol.view(T * H, C), lw["w_uv"], ov.view(T * H, Dv), M=T * H, row_src=rows, row_dst=rows, group_off=goff, n_groups=H)
-        og = self._mat("mix_gated", T, HV, E)
-        B.gated_norm(ov, None, P[:, HQ + CR:], N, og, self.config.norm_eps, T)
+            segs.append(B.head_seg(P[:, HQ + C:], N, 1, Rd, plane, rot_dims=Rd, row_off=off, dst_offset=C))
+            if tiled:
+                segs.append(B.head_seg(P[:, D:], N, H, Rd, q, src_head_stride=DR, rot_dims=Rd, ld_dst=HQ, head_stride=DR, dst_offset=D))
+            if n:
+                segs.append(B.head_seg(P[:, D:], N, H, Rd, qa, src_head_stride=DR, rot_dims=Rd, ld_dst=H * CR, head_stride=CR, dst_offset=C))
+        for k in range(0, len(segs), 4):
+            B.head_prep(segs[k:k + 4], T, E, pos=tb["pos"], freqs=lw["freqs"], rot_mag=lw["rot_mag"], eps=self.config.norm_eps)
+        og, gate = self._mat("mix_gated", T, HV, E), P[:, HQ + CR:]
+        if n:
+            rows = tb["f_rows"] if tiled and n < T else None
+            B.linear(P, lw["w_abs"], qa, M=n, row_src=rows, row_dst=rows, n_batch=H, ldx=N, x_batch_stride=DR, ldy=H * CR, y_batch_stride=CR)
+            ol = self._mat("mix_out", T, H * C, E)
+            splits = self._splits(n, -(-H // 16), min(arena.cap, l.mask or arena.cap))
+            part = self._scratch("attn_part", B.attn_softmax_part(T, H, splits, C), torch.float32) if splits > 1 else None
+            B.attn_latent(qa, f_tiles, n, plane, arena.slot_stride(i), CR, H, CR, C, l.scale, ol, window=l.mask, n_splits=splits, part=part)
+            ov = self._mat("mix_o32", T, HV, torch.float32)
+            B.linear(ol, lw["w_uv"], ov, M=n, row_src=rows, row_dst=rows, n_batch=H, ldx=H * C, x_batch_stride=C, ldy=HV, y_batch_stride=Dv)
+            B.gated_norm(ov, None, gate, N, og, self.config.norm_eps, T)
+        if tiled:
+            # (after the others: their gate runs over all rows)
+            flat, M, NK = plane.view(-1, CR), tb["kv_rows"].numel(), H * (D + Dv)
+            kv = self._mat("kv_rows", M, NK, E)
+            B.linear(flat, lw["w_kv"], kv, M=M, row_src=tb["kv_rows"], ldx=CR)
+            B.attn_prompt(q, tb["l_tiles"], tb["l_tiles"].numel() // 4, tb["tile"], kv, (NK, D), kv[:, H * D:], (NK, Dv), H, H, DR, Dv, l.scale, og,
+                          ldo=HV, k_tail=flat[:, C:] if Rd else None, tail_row_stride=CR, tail_rows=tb["kv_rows"], tail_dim=Rd, window=l.mask,
+                          gate=gate, ldg=N, gate_cols=True)
         B.linear(og, lw["wo"], y, M=T)
         return P[:, HQ + CR + HV:], N
 
-    def _mlstm(self, arena, i, l, lw, h, y, tb, T, R, n_tiles):
+    def _mlstm(self, arena, i, l, lw, h, y, tb, T, R):
         H, D, Dv = l.heads, l.dim, l.vdim
         HD, HV = H * D, H * Dv
         P, N = self._project_in(lw, h, T)

@@ -480,6 +480,29 @@ def test_prompt_equals_token_by_token_decoding_and_any_portions(name, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n", [15, 16, 17, 64, 65, 129])
+def test_tiled_and_single_rows_beside_one_another(dtype, n):
+    """A request that goes on with n tokens behind 150 (tiled from 16 on, its keys cut at the windows' reach), beside one that decodes
+    and one with three tokens, through layers whose latent heads fit the tiles and one whose heads do not: float32 is held to the
+    oracle at the bound of the whole-model tests above, bfloat16 to the same requests stepped alone token by token."""
+    s = FivesunShape(vocab_size=90, hidden_size=64, norm_eps=1e-6, embed_scale=8.0, layers=[
+        att(4, 2, 32, 32, mask=70, ff=48), lat(4, 40, 24, 32, 48, mask=90, ff=48), lat(2, 230, 40, 20, 32, mask=70), att(2, 1, 264, 16, mask=0)])
+    w = W.make_fivesun_weights(s, seed=4)
+    from promptcache_amd.model.fivesun_hip import FivesunHIP
+    m = FivesunHIP(s, w, device=DEV, dtype=dtype)
+    seqs = [toks(k, s.vocab_size, seed=40 + i) for i, k in enumerate((150 + n, 81, 43))]
+    new = [n, 1, 3]
+    ar = m.new_arena(3, 400)
+    slots = [ar.alloc() for _ in seqs]
+    m.forward_rows(ar, slots, [q[:-k] for q, k in zip(seqs, new)])
+    got = m.forward_rows(ar, slots, [q[-k:] for q, k in zip(seqs, new)], [list(range(k)) for k in new])
+    for i, (q, k) in enumerate(zip(seqs, new)):
+        mine = got[sum(new[:i]):sum(new[:i]) + k]
+        want = oracle_logits(s, w, q)[0][-k:] if dtype == torch.float32 else run_alone(m, q, [1] * len(q))[-k:]
+        assert rel(mine, want) < tol(dtype, 3e-5, 8e-2), i
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("graphs", [True, False])
 def test_unequal_batches_reused_slots_and_states(dtype, graphs):
     """Requests of different lengths step together, some end, newcomers take their slots (keys, values, latents and matrix memories
