@@ -239,9 +239,9 @@ __global__ __launch_bounds__(256) void kv_row_table_kernel(const pc_kv_seg* __re
 // ---- pc_prefill_prologue: everything a captured small-q forward does before its first layer, in ONE launch ------------------
 // Block roles (all of them read the call's PINNED HOST block directly, with system-scope loads: no ordering inside the launch is
 // needed, and the host rewrites the block between replays):
-//   [0, n_tok)            embedding row of token t as the fp32 residual stream          (llama2.py:869; ids from the host block)
-//   n_tok                 the whole block -> its device twin (past length, live rows, ... for the layers' kernels) and the
-//                         (cos, sin) rows of the supplied positions                         (llama2.py:129-147, :204-207)
+//   [0, n_tok)            embedding row of token t as the fp32 residual stream (llama2.py:869; ids from the host block) and its
+//                         (cos, sin) row at the supplied position                           (llama2.py:129-147, :204-207)
+//   n_tok                 the whole block -> its device twin (past length, live rows, ... for the layers' kernels)
 //   n_tok + 1 ..          the staging plan expanded to one pc_kv_row per staged row (pc_kv_row_table), when `rows` is given
 typedef __attribute__((address_space(1))) unsigned long long g64;
 __device__ __forceinline__ unsigned long long host_ld8(const void* p) {
@@ -263,16 +263,59 @@ __device__ __forceinline__ unsigned int host_ld4(const void* p) {
     return __hip_atomic_load((g32*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// Bound by reads over the host link: 2-3 us each, and some thirty million a second in all.  So every word is read once per workgroup,
+// by the lanes of one wave in one instruction; and from 17 tokens on the block is fetched by a launch of its own in front
+// (prologue_fetch_kernel) and `host` is its device twin here: 7 + 6 us for 259 tokens over 8 258 staged rows, 7.6 + 4.3 us for 27
+// over 308, 7.1 us in one launch for 12 over 1 725.  Before, one workgroup computed all rotation rows behind a dependent host read
+// per 256 values and every wave read its words itself: 275, 39 and 28 us.
+__device__ __forceinline__ void fetch_block_part(const PrologueArgs& a, int tid, bool dev_in) {
+    // (o_words is only 4-byte aligned: the block goes over in 4-byte pieces, sixteen reads per thread in flight)
+    const int n = a.nbytes >> 2, from = dev_in ? a.o_words >> 2 : 0;
+    for (int i0 = from + tid; i0 < n; i0 += 16 * 256) {
+        unsigned int v[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const int i = i0 + k * 256;
+            v[k] = host_ld4(a.host + 4 * (i < n ? i : n - 1));
+        }
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const int i = i0 + k * 256;
+            if (i < n) ((unsigned int*)a.dev)[i] = v[k];
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void prologue_fetch_kernel(const PrologueArgs a) {
+    fetch_block_part(a, threadIdx.x, host_ld4(a.host + a.o_words + 20) != 0u);
+}
+
 __global__ __launch_bounds__(256) void prefill_prologue_kernel(const PrologueArgs a) {
     __shared__ pc_kv_seg s_seg[kRowTabMaxSeg];
+    __shared__ unsigned int s_word[4];
     const int b = blockIdx.x, tid = threadIdx.x;
     // words[5] != 0: the caller's token ids and position ids are DEVICE tensors (the reference's calling convention,
     // generation_engine.py:96-97) that it copied into the device twin's ids | pos region on this stream before the launch:
     // read them there, and leave that region alone when the block is fetched
-    const bool dev_in = host_ld4(a.host + a.o_words + 20) != 0u;
     if (b < a.n_tok) {
-        long long id = dev_in ? ((const long long*)a.dev)[b] : (long long)host_ld8(a.host + 8 * b);
+        if (tid < 4) {       // id (two words), position, words[5]
+            const int32_t at = tid < 2 ? 8 * b + 4 * tid : (tid == 2 ? a.o_pos + 4 * b : a.o_words + 20);
+            s_word[tid] = host_ld4(a.host + at);
+        }
+        __syncthreads();
+        long long id = (long long)(((unsigned long long)s_word[1] << 32) | s_word[0]);
+        int pos = (int)s_word[2];
+        if (s_word[3] != 0u) {
+            id = ((const long long*)a.dev)[b];
+            pos = ((const int*)(a.dev + a.o_pos))[b];
+        }
         id = id < 0 ? 0 : (id >= a.vocab ? a.vocab - 1 : id);
+        for (int f = tid; f < a.half_dim; f += 256) {
+            const float ang = __fmul_rn((float)pos, a.inv_freq[f]);                          // as rope_table_kernel (pc_rope.hip)
+            float sn, c;
+            sincosf(ang, &sn, &c);
+            a.cs[(int64_t)b * a.half_dim + f] = make_float2(c, sn);
+        }
         for (int i = tid; i < (a.hidden >> 3); i += 256) {
             const h8g v = *(const h8g*)(a.table + id * a.hidden + i * 8);
             float* o = a.x + (int64_t)b * a.hidden + i * 8;
@@ -282,33 +325,14 @@ __global__ __launch_bounds__(256) void prefill_prologue_kernel(const PrologueArg
         return;
     }
     if (b == a.n_tok) {
-        if (!dev_in) {
-            for (int i = tid; i < a.nbytes / 8; i += 256) ((unsigned long long*)a.dev)[i] = host_ld8(a.host + 8 * i);
-        } else {          // (o_words is only 4-byte aligned: the words and the plan go over in 4-byte pieces)
-            for (int i = a.o_words / 4 + tid; i < a.nbytes / 4; i += 256) ((unsigned int*)a.dev)[i] = host_ld4(a.host + 4 * i);
-        }
-        for (int i = tid; i < a.n_tok * a.half_dim; i += 256) {
-            const int t = i / a.half_dim, f = i - t * a.half_dim;
-            int pos;
-            if (dev_in) {
-                pos = ((const int*)(a.dev + a.o_pos))[t];
-            } else {
-                const unsigned long long w = host_ld8(a.host + a.o_pos + 8 * (t >> 1));  // two int32 positions per 8 bytes
-                pos = (int)((t & 1) ? (w >> 32) : (w & 0xffffffffu));
-            }
-            const float ang = __fmul_rn((float)pos, a.inv_freq[f]);                      // as rope_table_kernel (pc_rope.hip)
-            float sn, c;
-            sincosf(ang, &sn, &c);
-            a.cs[i] = make_float2(c, sn);
-        }
+        if (a.host != a.dev) fetch_block_part(a, tid, host_ld4(a.host + a.o_words + 20) != 0u);
         return;
     }
     if (!a.rows) return;
-    // words[3] = segments, words[4] = rows of the table (o_words is 4-byte aligned: read the two int32 words separately)
-    const unsigned long long w34a = host_ld8(a.host + ((a.o_words + 12) & ~7));
-    const unsigned long long w34b = host_ld8(a.host + ((a.o_words + 16) & ~7));
-    int nseg = (int)(((a.o_words + 12) & 7) ? (w34a >> 32) : (w34a & 0xffffffffu));
-    int total = (int)(((a.o_words + 16) & 7) ? (w34b >> 32) : (w34b & 0xffffffffu));
+    // words[3] = segments, words[4] = rows of the table
+    if (tid < 2) s_word[tid] = host_ld4(a.host + a.o_words + 12 + 4 * tid);
+    __syncthreads();
+    int nseg = (int)s_word[0], total = (int)s_word[1];
     nseg = nseg < 0 ? 0 : (nseg > a.max_seg ? a.max_seg : nseg);
     total = total > a.max_ctx ? a.max_ctx : total;
     for (int i = tid; i < nseg; i += 256) {
@@ -343,6 +367,10 @@ PC_EXPORT int pc_prefill_prologue(const void* host_block, void* dev_block, int32
     a.row_bytes = (uint32_t)head_dim * 2u; a.dst_plane_stride16 = rows ? (uint32_t)(((uint64_t)max_ctx * a.row_bytes) >> 4) : 0u;
     a.max_ctx = max_ctx;
     const int nblk = n_tok + 1 + (rows ? pc_ceil_div(max_ctx, 256) : 0);
+    if (n_tok > 16) {       // (hundreds of workgroups that each wait for the host link; the second launch reads device memory)
+        hipLaunchKernelGGL(prologue_fetch_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, a);
+        a.host = a.dev;
+    }
     hipLaunchKernelGGL(prefill_prologue_kernel, dim3(nblk), dim3(256), 0, (hipStream_t)stream, a);
     return pc_check_launch("prefill_prologue_kernel");
 }

@@ -386,6 +386,51 @@ def test_prefill_prologue_equals_the_separate_launches(T, nseg_plan):
         assert torch.equal(rows, rows2)
 
 
+@pytest.mark.parametrize("T,dev_in", [(16, False), (17, False), (16, True), (17, True), (272, True), (512, False)])
+def test_prefill_prologue_around_the_launch_of_its_own_for_the_block(T, dev_in):
+    """16 tokens (the block is read where it lies on the host) and 17 on (fetched by a launch in front), with more segments than a
+    workgroup has threads, and with ids / positions that the caller already put into the device twin: tables and twin bit for bit
+    what pc_embed_gather, pc_rope_table and the plan itself say."""
+    n = _n()
+    rng = np.random.default_rng(T)
+    hid, vocab, D, cap, max_seg, nseg = 64, 333, 48, 900, 300, 290
+    table = _rand_half((vocab, hid), rng)
+    inv = (1.0 / (10000.0 ** (torch.arange(0, D, 2).float() / D))).to(DEV)
+    o_pos, o_words = 8 * T, 12 * T
+    o_segs = (o_words + 32 + 15) // 16 * 16
+    nbytes = o_segs + 16 * max_seg
+    host = torch.zeros(nbytes, dtype=torch.uint8, pin_memory=True)
+    h = host.numpy()
+    ids, pos = rng.integers(0, vocab, size=T), rng.integers(0, 9000, size=T).astype(np.int32)
+    dev = torch.full((nbytes,), 0xEE, dtype=torch.uint8, device=DEV)
+    if dev_in:
+        dev[:8 * T].view(torch.int64).copy_(torch.from_numpy(ids.astype(np.int64)))
+        dev[o_pos:o_pos + 4 * T].view(torch.int32).copy_(torch.from_numpy(pos))
+    else:
+        h[:8 * T].view(np.int64)[:] = ids
+        h[o_pos:o_pos + 4 * T].view(np.int32)[:] = pos
+    total = 2 * nseg + 5
+    h[o_words:o_words + 32].view(np.int32)[:] = [2 * nseg, 0, T, nseg, total, int(dev_in), 0, 0]
+    sa = h[o_segs:].view(np.dtype([("src", "<u8"), ("dst_row", "<i4"), ("len", "<i4")]))
+    sa["src"][:nseg], sa["dst_row"][:nseg], sa["len"][:nseg] = (1 << 40) + 65536 * np.arange(nseg), 2 * np.arange(nseg), 2
+    arena = torch.zeros(64, dtype=torch.float16, device=DEV)
+    x, cs = torch.full((T, hid), float("nan"), device=DEV), torch.full((T, D // 2, 2), float("nan"), device=DEV)
+    rows = torch.full((cap * 16,), 0xAB, dtype=torch.uint8, device=DEV)
+    n.prefill_prologue(host, dev, nbytes, T, o_pos, o_words, o_segs, max_seg, table, hid, vocab, x, inv, D, cs, rows=rows, dst=arena, max_ctx=cap)
+    torch.cuda.synchronize()
+    assert torch.equal(dev.cpu()[o_words:], host[o_words:])
+    assert np.array_equal(dev[:8 * T].cpu().numpy().view(np.int64), ids) and np.array_equal(dev[o_pos:o_words].cpu().numpy().view(np.int32), pos)
+    assert torch.equal(x, table.float()[torch.from_numpy(ids).to(DEV)])
+    cs2 = torch.empty_like(cs)
+    n.rope_table(torch.from_numpy(pos).to(DEV), inv, cs2, T, D)
+    assert torch.equal(cs.view(torch.int32), cs2.view(torch.int32))
+    got = rows.cpu().numpy().view(np.dtype([("base", "<u8"), ("stride", "<u4"), ("flags", "<u4")]))
+    r = np.arange(total)
+    base = np.where(r < 2 * nseg, (1 << 40) + 65536 * (r // 2) + (r % 2) * 2 * D, arena.data_ptr() + r * 2 * D)
+    assert np.array_equal(got["base"][:total], base.astype(np.uint64)) and (got["base"][total:] == 0xABABABABABABABAB).all()
+    assert (got["stride"][:2 * nseg] == 2 * 2 * D // 16).all()
+
+
 @pytest.mark.parametrize("q_len,stage", [(22, False), (22, True), (9, False), (30, True)])
 def test_tail_mode_streams_sized_for_a_longer_cache_run_empty_without_harm(q_len, stage):
     """tail_stream_splits sizes the streams of a <= 32-row tail-mode launch from the HOST past length (one per key tile); a captured
