@@ -17,22 +17,29 @@
 // partial products meet in the fp32 accumulator, and the epilogue (residual add, SiLU*up, GELU, fp32 store) runs on the
 // accumulator tile -- no [2T][N] fp32 intermediate ever exists.
 //
-// Tile: workgroup = 8 waves (2 per SIMD), block tile 128 (M) x BN (N) x 64 (K), BN = 256 (waves 2 x 4, wave tile
-// 64 x 64) or 128 (waves 4 x 2, wave tile 32 x 64; for launches whose 256-wide grid would leave CUs idle).
-// mfma_f32_32x32x16_f16: per 16-deep k-slab a wave reads 2*MT activation fragments and 2 weight fragments (16 B per
-// lane each, ds_read_b128) for 4*MT MFMAs.
-// Staging: global_load_lds (16 B per lane, 1 KiB per wave-instruction = 8 rows x 128 B of a tile) straight into a
-// double-buffered LDS image, one barrier per K-step: the loads of K-step t+1 are in flight while step t is multiplied.
+// Tile: workgroup = 4 waves (2 x 2), block tile 64 MT (M) x 64 NT (N) x 64 (K), wave tile 32 MT x 32 NT: 128 x 256 with both planes or
+// one, 256 x 256 with one plane over many rows, 128 x 128 for launches whose 256-wide grid would leave CUs idle (launch_dense_tile).
+// What bounds it: power (the matrix cores run these launches at 1.4-1.7 GHz; the same launches on zeros are 1.2-1.3 x faster), LDS bandwidth
+// next.  Per 16-deep k-slab and both planes a wave of 64 x 128 reads 8 KiB of LDS for 16 MFMAs, two waves of 64 x 64 read 12 KiB for as
+// many: the same block tile on eight waves kept the LDS pipe as busy as the matrix pipe.  Eight waves -> four, random data: both planes,
+// 1 737 rows, q|k|v 345 -> 322 us, down 305 -> 286, 32 000 columns 854 -> 797 (1.14 PFLOP/s executed), 3 584 rows down 624 -> 581; one
+// plane, gate|up, 1 737 / 2 940 / 3 584 rows 384 -> 361, 622 -> 577, 760 -> 599 us (256 x 256 tiles, 1.08 PFLOP/s).
+// mfma_f32_32x32x16_f16: per 16-deep k-slab a wave reads MT (2 MT with both planes) activation fragments and NT weight fragments
+// (16 B per lane each, ds_read_b128) for MT NT (2 MT NT) MFMAs.
+// Staging: global_load_lds (16 B per lane, 1 KiB per wave-instruction = 8 rows x 128 B of a tile) straight into a ring of two or three
+// LDS images, one barrier per K-step.  The first half of a wave's instructions for a K-step goes out between the MFMAs behind the barrier
+// that frees its buffer, the second half between those of the next step's first slab.
 // The LDS image keeps 128-byte rows; the 16-byte chunk c of row r sits at chunk position c ^ ((r >> 1) & 7), which
 // makes every ds_read_b128 lane group of a fragment read hit 16 distinct 16-byte bank slots (row-major 128-B rows
 // would be 8-way conflicted).  LDS-DMA writes lane-linearly, so the permutation is applied to the per-lane SOURCE
-// address and again on the read (guide: rule 21, both sides or neither).
+// address and again on the read.
 // Which global weight row lands in which LDS row is free as well (per-lane source address): the SiLU launch puts 32
-// gate rows and the 32 matching up rows side by side in one wave tile, so gate_j and up_j meet in the same lane.
-// Epilogue: the accumulator tile goes through the (now idle) LDS once so that every global store is 16 B per lane on
-// full rows.
-// Grid: 1-D, XCD-aware: block id b runs on XCD b % 8; an XCD owns the weight panels xcd, xcd + 8, ... and walks all
-// M-blocks of a panel before the next one, so a panel is fetched from HBM once and served from that XCD's L2.
+// gate rows and the 32 matching up rows side by side in one 64-column group, so gate_j and up_j meet in the same lane.
+// Epilogue: the accumulator tile goes through the (now idle) LDS, 64 columns of a wave at a time, so that every global store is 16 B per
+// lane on full rows.
+// Grid: 1-D, XCD-aware: block id b runs on XCD b % 8; the tiles are cut into 8 rectangles (px row strips by 8 / px column strips),
+// one per XCD, walked M-block by M-block: the 32 tiles that run on an XCD at a time share few activation rows AND few weight panels
+// (with one column strip each an XCD walks all M-blocks: 2 048 x 8 192 x 2 048 in 256 x 256 tiles 93 us, in 4 x 2 strips 71).
 // Roofline: MFMA.  flops per launch = 2 * (TWO ? 2 : 1) * M * N * K against the 2.5 PFLOP/s dense fp16 peak.
 #include <hip/hip_fp16.h>
 #include <string.h>
@@ -51,8 +58,7 @@ typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 
-constexpr int BM = 128, BK = 64;
-constexpr int kXT = BM * BK * 2;                 // bytes of one activation plane tile (16 KiB)
+constexpr int BK = 64;
 enum { EPI_STORE = 0, EPI_ADD = 1, EPI_SILU = 2, EPI_ROPE = 3, EPI_GELU = 4 };
 
 struct DenseParams {
@@ -71,6 +77,7 @@ struct DenseParams {
     float* y; int64_t ldy;                                 // EPI_STORE / EPI_ADD
     _Float16* oh; _Float16* ol; int64_t ldo;               // EPI_SILU / EPI_GELU output planes
     int32_t M, N, K, mb, nb, nfeat;                        // nfeat: SiLU features (= N / 2)
+    int32_t px, mh, nh;                                    // XCD x owns M-blocks (x % px) mh .. and weight panels (x / px) nh ..
     // split-K (EPI_STORE instantiation only): grid.y slices of `kper` K-steps, slice z stores its partial sums to
     // y + z * slab_stride; dense_reduce_kernel then adds the slabs in fixed order (launch_dense_splitk)
     int32_t kper; int64_t slab_stride;
@@ -87,29 +94,32 @@ __device__ __forceinline__ void glds16(const _Float16* g, char* lds_wave_base) {
                                      (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, 0);
 }
 
-typedef int i4v __attribute__((ext_vector_type(4)));
-typedef int i16v __attribute__((ext_vector_type(16)));
+// the block tile of a launch: W x W waves of 32 MT x 32 NT, S LDS images in the ring (as many as the 160 KiB of a CU hold)
+template <int W, bool TWO, bool NARROW, bool TALL>
+struct Tile {
+    static constexpr int MT = TALL ? 4 : 2, NT = NARROW ? 2 : 4, S = TWO || TALL ? 2 : 3;
+    static constexpr int BM = 32 * W * MT, BN = 32 * W * NT;
+};
 
-template <int WM, int EPI, bool TWO, bool PP, bool LO8 = false>
-__global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseParams p) {
-    static_assert(!(LO8 && (TWO || PP)), "LO8 replaces the fp16 lo plane; lockstep main loop only");
-    constexpr int WN = 8 / WM, MT = BM / (32 * WM), NT = 2, BN = 64 * WN;
-    constexpr int kWT = BN * BK * 2;             // bytes of the weight tile
-    // stage image: Xhi | Xlo | W   (LO8: Xhi | Xlo8 (64-byte rows) | W | W8 (64-byte rows))
-    constexpr int oW = LO8 ? kXT + kXT / 2 : 2 * kXT;
-    constexpr int oW8 = oW + kWT;
-    constexpr int kStage = LO8 ? oW8 + kWT / 2 : 2 * kXT + kWT;
-    constexpr int NXI = 2, NWI = BN / 64;        // staging instructions per wave: 2 per activation plane, BN/64 for W
-    constexpr int NW8 = BN / 128;                // ... and for the int8 weight tile (16 rows x 64 B per instruction); Xlo8: one
-    __shared__ __attribute__((aligned(16))) char lds[2 * kStage];
+// W: waves across and down a workgroup; TWO: both activation planes; NARROW: 128 columns instead of 256; TALL: 256 rows instead of 128
+template <int W, int EPI, bool TWO, bool NARROW, bool TALL>
+__global__ __launch_bounds__(256, 1) void gemm_dense_kernel(const DenseParams p) {
+    static_assert(W == 2 && !(TWO && TALL), "four waves; two planes of 256 rows and their weights do not fit the LDS twice");
+    using T = Tile<W, TWO, NARROW, TALL>;
+    constexpr int MT = T::MT, NT = T::NT, S = T::S;
+    constexpr int PL = TWO ? 2 : 1, BM = T::BM, BN = T::BN, ROWS = PL * BM + BN;
+    constexpr int kStage = ROWS * 128;           // image: Xhi | Xlo | W, 128-byte rows
+    constexpr int NI = ROWS / 32;                // staging instructions per wave: 8 rows each
+    constexpr int NX = PL * BM / 32;             // ... of them for activations
+    __shared__ __attribute__((aligned(16))) char lds[S * kStage];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave / WN, wn = wave - wm * WN;
+    const int wm = wave >> 1, wn = wave & 1;
     // block -> (M-block, weight panel), XCD-aware
-    const int b = blockIdx.x, xcd = b & 7, slot = b >> 3;
-    const int nloc = slot / p.mb, mi = slot - nloc * p.mb, ni = nloc * 8 + xcd;
-    if (ni >= p.nb) return;
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int mi = xcd % p.px * p.mh + slot % p.mh, ni = xcd / p.px * p.nh + slot / p.mh;
+    if (mi >= p.mb || ni >= p.nb) return;
     const int m0 = mi * BM;
     const int K = p.K, nkt = (K + BK - 1) / BK;          // K-steps of the whole product
     const int t0 = blockIdx.y * p.kper;                  // this slice's first K-step (kper = nkt without split-K)
@@ -118,11 +128,11 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseParams p) {
     // global weight row of LDS weight-tile row r; -1 = past the end (clamped source, never stored)
     auto wrow = [&](int r) -> int {
         if (EPI == EPI_SILU) {
-            const int f = (ni * WN + (r >> 6)) * 32 + (r & 31);
+            const int f = (ni * NT + (r >> 6)) * 32 + (r & 31);
             return f < p.nfeat ? ((r >> 5) & 1) * p.nfeat + f : -1;
         }
         if (EPI == EPI_ROPE) {
-            // a wave tile (64 columns) = 32 features d of one head's first half next to their rotary partners d + 64, so
+            // a 64-column group = 32 features d of one head's first half next to their rotary partners d + 64, so
             // x[d] and x[d + 64] meet in the same lane and accumulator index of the two 32-wide MFMA blocks
             const int wt = r >> 6, c = r & 63;
             const int hd = ni * (BN / 128) + (wt >> 1);
@@ -134,68 +144,30 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseParams p) {
         return n < p.N ? n : -1;
     };
 
-    // ---- staging sources: per lane one 16-byte chunk of one row per instruction ----
-    const int srow = lane >> 3, scp = lane & 7;          // row inside the 8-row group, chunk POSITION in the LDS row
-    const _Float16* gx[NXI];
-    const _Float16* gw[NWI];
-    int cx[NXI], cw[NWI];                                // source chunk index (for the K tail)
-    const int64_t lo_delta = TWO ? (p.xl - p.xh) : 0;
+    // ---- staging sources: per lane one 16-byte chunk of one row per instruction; instruction i fills image rows 8 (4 i + wave) .. + 7 ----
+    const int srow = 8 * wave + (lane >> 3);
+    const int cx = (lane & 7) ^ ((srow >> 1) & 7);       // source chunk of the lane (the same in every instruction: 32 rows apart)
+    const _Float16* src[NI];
 #pragma unroll
-    for (int j = 0; j < NXI; ++j) {
-        const int r = wave * 16 + j * 8 + srow;
-        const int gm = (m0 + r < p.M) ? m0 + r : p.M - 1;
-        cx[j] = scp ^ ((r >> 1) & 7);
-        gx[j] = p.xh + (int64_t)gm * p.ldx + cx[j] * 8;
-    }
-#pragma unroll
-    for (int j = 0; j < NWI; ++j) {
-        const int r = wave * (BN / 8) + j * 8 + srow;
-        int gr = wrow(r);
-        gr = gr < 0 ? 0 : gr;
-        cw[j] = scp ^ ((r >> 1) & 7);
-        gw[j] = p.w + (int64_t)gr * p.ldw + cw[j] * 8;
-    }
-    // LO8: one instruction of 16 rows x 64 B per wave for the activation codes, NW8 for the weight codes; lane -> (row, chunk
-    // POSITION); position c of row r holds source chunk c ^ ((r >> 2) & 3): the 16 lanes of every ds_read_b128 group then fall
-    // into 16 distinct 16-byte bank slots (64-byte rows: slot = 4 (r & 3) + position)
-    [[maybe_unused]] const signed char* gx8 = nullptr;
-    [[maybe_unused]] const signed char* gw8[NW8 > 0 ? NW8 : 1];
-    if constexpr (LO8) {
-        const int r = wave * 16 + (lane >> 2);
-        const int gm = (m0 + r < p.M) ? m0 + r : p.M - 1;
-        gx8 = p.xl8 + (int64_t)gm * p.ldx8 + (((lane & 3) ^ ((r >> 2) & 3)) << 4);
-#pragma unroll
-        for (int j = 0; j < NW8; ++j) {
-            const int rw = wave * (BN / 8) + j * 16 + (lane >> 2);
-            int gr = wrow(rw);
-            gr = gr < 0 ? 0 : gr;
-            gw8[j] = p.w8 + (int64_t)gr * p.ldw8 + (((lane & 3) ^ ((rw >> 2) & 3)) << 4);
+    for (int i = 0; i < NI; ++i) {
+        const int r = 32 * i + srow;
+        if (i < NX) {
+            const bool lo = TWO && i >= NX / PL;
+            const int m = m0 + r - (lo ? BM : 0);
+            src[i] = (lo ? p.xl : p.xh) + (int64_t)(m < p.M ? m : p.M - 1) * p.ldx + cx * 8;
+        } else {
+            const int gr = wrow(r - PL * BM);
+            src[i] = p.w + (int64_t)(gr < 0 ? 0 : gr) * p.ldw + cx * 8;
         }
     }
-    const bool ktail = (K % BK) != 0;
-    auto stage = [&](int tl, char* buf) {
+    // chunks past K: zero activations, paired with any finite weight bytes (the row's first chunk)
+    const int last = (K - (nkt - 1) * BK) / 8;           // valid chunks of the product's last K-step (8: a whole one)
+    auto stage = [&](int i, int tl, char* buf) {
         const int t = t0 + tl;
-        const bool tail = ktail && t == nkt - 1;
-        const int64_t ko = (int64_t)t * BK;
-        const int kchunks = tail ? (K - t * BK) / 8 : 8;          // valid 16-byte chunks in this K-step
-#pragma unroll
-        for (int j = 0; j < NXI; ++j) {
-            const bool ok = !tail || cx[j] < kchunks;
-            const _Float16* sh = ok ? gx[j] + ko : p.zeros;
-            glds16(sh, buf + (wave * 16 + j * 8) * 128);
-            if (TWO) glds16(ok ? gx[j] + lo_delta + ko : p.zeros, buf + kXT + (wave * 16 + j * 8) * 128);
-        }
-#pragma unroll
-        for (int j = 0; j < NWI; ++j) {
-            // chunks past K pair with zero activations: any finite weight bytes do (the row's first chunk)
-            const _Float16* sw = (!tail || cw[j] < kchunks) ? gw[j] + ko : gw[j] - cw[j] * 8;
-            glds16(sw, buf + oW + (wave * (BN / 8) + j * 8) * 128);
-        }
-        if constexpr (LO8) {                           // (K % 64 == 0 with LO8: no tail)
-            glds16((const _Float16*)(gx8 + ko), buf + kXT + wave * 1024);
-#pragma unroll
-            for (int j = 0; j < NW8; ++j) glds16((const _Float16*)(gw8[j] + ko), buf + oW8 + (wave * (BN / 8) + j * 16) * 64);
-        }
+        const bool ok = cx < (t == nkt - 1 ? last : 8);
+        const _Float16* g = src[i] + (int64_t)t * BK;
+        if (!ok) g = i < NX ? p.zeros : src[i] - cx * 8;
+        glds16(g, buf + (4 * i + wave) * 1024);
     };
 
     // ---- fragment addressing: lane = (row fr of the 32-row subtile, k-half fh) ----
@@ -203,23 +175,7 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseParams p) {
     int foff[4];
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) foff[ks] = fr * 128 + (((2 * ks + fh) ^ ((fr >> 1) & 7)) << 4);
-    const int a_base = (wm * 32 * MT) * 128;              // + 32*i rows, + kXT for the lo plane
-    const int b_base = oW + (wn * 64) * 128;              // + 32*j rows
-    // LO8: a lane's 16 codes of a 32-deep block kb are chunk 2 kb + fh of its row (A and B pair slot by slot, so which sixteen k
-    // of the block a lane holds is free as long as both sides agree)
-    [[maybe_unused]] int foff8[2];
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) foff8[kb] = fr * 64 + (((2 * kb + fh) ^ ((fr >> 2) & 3)) << 4);
-    [[maybe_unused]] const int a8_base = kXT + (wm * 32 * MT) * 64, b8_base = oW8 + (wn * 64) * 64;
-    [[maybe_unused]] i16v iacc[LO8 ? MT : 1][LO8 ? NT : 1];
-    if constexpr (LO8) {
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-            for (int j = 0; j < NT; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) iacc[i][j][r] = 0;
-    }
+    const int a_base = (wm * 32 * MT) * 128, b_base = (PL * BM + wn * 32 * NT) * 128;
 
     f16v acc[MT][NT];
 #pragma unroll
@@ -230,431 +186,113 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseParams p) {
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
     // ---- main loop: one barrier per K-step, fragment reads one 16-deep slab ahead of the MFMAs ----
-    // Two fragment register sets alternate over the 4 slabs of a K-step.  The reads of slab s+1 are issued in front of
-    // the MFMAs of slab s, so their LDS latency passes under 4*MT MFMAs of 32 cycles each; the last slab of K-step t is
-    // multiplied AFTER the barrier, next to the first reads of K-step t+1 and the LDS-DMA issue of K-step t+2, so the
-    // matrix pipe has work while the workgroup re-synchronises.
-    struct Frags { h8 ah[MT], al[TWO ? MT : 1], bw[NT]; };
-    auto load_frags = [&](Frags& f, const char* buf, int ks) {
-#pragma unroll
-        for (int i = 0; i < MT; ++i) {
-            f.ah[i] = *(const h8*)(buf + a_base + i * 32 * 128 + foff[ks]);
-            if (TWO) f.al[i] = *(const h8*)(buf + kXT + a_base + i * 32 * 128 + foff[ks]);
-        }
-#pragma unroll
-        for (int j = 0; j < NT; ++j) f.bw[j] = *(const h8*)(buf + b_base + j * 32 * 128 + foff[ks]);
-    };
-    auto mfmas = [&](const Frags& f) {
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-            for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.ah[i], f.bw[j], acc[i][j], 0, 0, 0);
-        if (TWO) {
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.al[i], f.bw[j], acc[i][j], 0, 0, 0);
+    // Two fragment register sets alternate over the 4 slabs of a K-step.  The reads of slab s + 1 are issued between the MFMAs of slab
+    // s; the last slab of K-step t is multiplied AFTER the barrier, next to the first reads of K-step t + 1 and the first half of the
+    // LDS-DMA of K-step t + S (its buffer was just freed), whose second half goes out in the next step's first slab.
+    constexpr int R = PL * MT + NT, MF = PL * MT * NT, D0 = NI / 2;
+    struct Frags { h8 a[PL * MT], b[NT]; };
+    auto read_one = [&](Frags& f, const char* buf, int ks, int q) {
+        if (q < NT) {
+            f.b[q] = *(const h8*)(buf + b_base + q * 32 * 128 + foff[ks]);
+        } else {
+            const int pl = (q - NT) / MT, i = (q - NT) % MT;
+            f.a[q - NT] = *(const h8*)(buf + a_base + (pl * BM + i * 32) * 128 + foff[ks]);
         }
     };
-    // Pin the issue order of one (reads of the next slab, MFMAs of this slab) pair: a read in front of every MFMA until
-    // the reads run out.  Left alone, hipcc sinks the ds_reads next to their first use and waits lgkmcnt(0) right
-    // behind them (seen in the ISA: four exposed LDS round trips per K-step).
-    auto interleave = [&]() {
-        // one MFMA, then two reads, until the reads run out: every read of the next slab is in flight at least three
-        // MFMAs (~100 cycles) before the wait in front of that slab's first MFMA
-        constexpr int R = MT * (TWO ? 2 : 1) + NT, MF = MT * NT * (TWO ? 2 : 1);
+    auto mfma_one = [&](const Frags& f, int q) {
+        const int pl = q / (MT * NT), i = q / NT % MT, j = q % NT;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.a[pl * MT + i], f.b[j], acc[i][j], 0, 0, 0);
+    };
+    // the reads that go behind MFMA k of a slab: one to every second MFMA where they fit, else two to each
+    auto reads_behind = [&](Frags& f, const char* buf, int ks, int k) {
+        if constexpr (MF >= 2 * R) {
+            if (k % 2 == 0 && k / 2 < R) read_one(f, buf, ks, k / 2);
+        } else {
+            if (2 * k < R) read_one(f, buf, ks, 2 * k);
+            if (2 * k + 1 < R) read_one(f, buf, ks, 2 * k + 1);
+        }
+    };
+    // (left alone, hipcc sinks the reads next to their first use and waits for them there)
+    auto slab = [&](const Frags& f, Frags& nx, const char* buf, int ks) {
+#pragma unroll
+        for (int q = 0; q < R; ++q) read_one(nx, buf, ks, q);
+#pragma unroll
+        for (int q = 0; q < MF; ++q) mfma_one(f, q);
 #pragma unroll
         for (int k = 0; k < MF; ++k) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                          // one MFMA
-            if (2 * k + 1 < R) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);       // two DS reads
-            else if (2 * k < R) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);      // (an odd one left)
-        }
-    };
-    // The slab multiplied right behind the K-step barrier also carries the LDS-DMA issue of K-step t + 2 (its buffer was just
-    // freed).  Rounds 2-4 issued the 8 (LO8: 11) DMA instructions in one burst in front of that slab's MFMAs: both waves of a SIMD
-    // spend ~60-100 issue cycles per instruction there while the matrix pipe, drained by the barrier, has nothing to do (seen in
-    // the ISA: barrier, 8 x global_load_lds, then the first MFMA).  Round 5 spreads them BETWEEN that slab's MFMAs: one MFMA, two
-    // fragment reads (until they run out), the slab's share of the DMA instructions, next MFMA -- for launches with two fp16 planes
-    // (-0.6 ... -2.6 % per layer at 800 ... 6000 rows); one-plane and int8-residual launches measured 1-5 % SLOWER that way and keep
-    // the burst (profiles/r05_variants.txt).  -DPC_DENSE_SPREAD_DMA=0: the burst everywhere.
-#ifndef PC_DENSE_SPREAD_DMA
-#define PC_DENSE_SPREAD_DMA 1
-#endif
-    // one MFMA / one fragment read / a range of the DMA instructions of a K-step, by index (compile-time after unrolling)
-    auto mfma_one = [&](const Frags& f, int idx) {
-        const int pl = idx / (MT * NT), i = (idx / NT) % MT, j = idx % NT;
-        if (TWO && pl == 1) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.al[i], f.bw[j], acc[i][j], 0, 0, 0);
-        else acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.ah[i], f.bw[j], acc[i][j], 0, 0, 0);
-    };
-    auto read_one = [&](Frags& f, const char* buf, int ks, int idx) {
-        constexpr int NA = MT * (TWO ? 2 : 1);
-        if (idx < NA) {
-            const int i = TWO ? idx >> 1 : idx;
-            if (TWO && (idx & 1)) f.al[i] = *(const h8*)(buf + kXT + a_base + i * 32 * 128 + foff[ks]);
-            else f.ah[i] = *(const h8*)(buf + a_base + i * 32 * 128 + foff[ks]);
-        } else {
-            const int j = idx - NA;
-            f.bw[j] = *(const h8*)(buf + b_base + j * 32 * 128 + foff[ks]);
-        }
-    };
-    auto stage_range = [&](int tl, char* buf, int q0, int q1) {
-        const int t = t0 + tl;
-        const bool tail = ktail && t == nkt - 1;
-        const int64_t ko = (int64_t)t * BK;
-        const int kchunks = tail ? (K - t * BK) / 8 : 8;
-        int q = 0;
-#pragma unroll
-        for (int j = 0; j < NXI; ++j) {
-            const bool ok = !tail || cx[j] < kchunks;
-            if (q >= q0 && q < q1) glds16(ok ? gx[j] + ko : p.zeros, buf + (wave * 16 + j * 8) * 128);
-            ++q;
-            if (TWO) {
-                if (q >= q0 && q < q1) glds16(ok ? gx[j] + lo_delta + ko : p.zeros, buf + kXT + (wave * 16 + j * 8) * 128);
-                ++q;
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < NWI; ++j) {
-            if (q >= q0 && q < q1)
-                glds16((!tail || cw[j] < kchunks) ? gw[j] + ko : gw[j] - cw[j] * 8, buf + oW + (wave * (BN / 8) + j * 8) * 128);
-            ++q;
-        }
-        if constexpr (LO8) {
-            if (q >= q0 && q < q1) glds16((const _Float16*)(gx8 + ko), buf + kXT + wave * 1024);
-            ++q;
-#pragma unroll
-            for (int j = 0; j < NW8; ++j) {
-                if (q >= q0 && q < q1) glds16((const _Float16*)(gw8[j] + ko), buf + oW8 + (wave * (BN / 8) + j * 16) * 64);
-                ++q;
-            }
-        }
-    };
-    if constexpr (PP) {
-        // ---- ping-pong main loop (round 5; the guide's two-waves-per-SIMD regime).  MEASURED SLOWER than the lockstep loop below
-        // on this kernel (0.87-0.90 x with both planes, profiles/r05_dense_pp_ab.txt) in all three forms tried -- fragment reads
-        // waited for inside their load segment; read one phase ahead with hipcc's waits (lgkmcnt(0) every other phase: its
-        // scoreboard merges conservatively at the group branches); read ahead as raw ds_read_b128 with explicit counted waits
-        // (this form) -- kept for A/B behind -DPC_DEV_SWEEPS.  Eight barriers per K-step and one wave per SIMD feeding the
-        // matrix pipe at a time lose to two waves per SIMD interleaving their MFMAs with one barrier per K-step; what is left
-        // between the lockstep loop (1.09-1.15 PFLOP/s executed on random data) and the ~1.3 the guide's 8-phase template
-        // reaches at 4096^3 is not in the wave pairing. ----
-        // The loop above keeps the two waves of a SIMD in lockstep: both issue MFMAs at once (54 % of wave time were issue stalls
-        // behind the shared pipe, profiles/r02_pmc_gemm_dense.txt) and both sit out the barrier and the first fragment reads of
-        // the next K-step together (MFMA pipes busy 63 % of the kernel's cycles).  Here the workgroup's eight waves are two GROUPS
-        // of four (one wave of each group per SIMD) that run the same program ONE BARRIER APART: a K-step is four phases (one
-        // 16-deep slab each), a phase is a LOAD segment (the slab's 6 fragment reads, waited for) and a COMPUTE segment (its 8
-        // MFMAs = 256 matrix-pipe cycles), every segment ends in a raw s_barrier -- so while group 0 is in its compute segment
-        // group 1 is in its load segment and vice versa: the SIMD's matrix pipe always has exactly one wave feeding it, and the
-        // LDS reads, the waits and the barrier latency of one wave pass under the MFMAs of the other.  One fragment register
-        // set instead of two.
-        //   barrier n separates interval n from n + 1.  Group 0: load (t, s) in interval 8t + 2s, compute in 8t + 2s + 1; group 1
-        //   one interval later.  A load segment only ISSUES the fragment reads of the NEXT slab (two register sets); they are
-        //   consumed one phase later, so the segment is a few dozen issue cycles and the LDS latency never sits in front of a
-        //   barrier (first version: reads waited for inside their load segment -- the load segment then took longer than the
-        //   partner's 256-cycle compute segment and the loop ran at ITS pace: 0.81-0.93 x the lockstep loop).
-        //   Slab 0 of K-step t + 1 is read in load (t, 3): group 0 in interval 8t + 6, so K-step t + 1 must have landed, for all
-        //   waves, by barrier 8t + 6: the LDS-DMA goes out in two pieces between MFMAs -- group 0 in compute (t, 0), (t, 1), waited
-        //   for at the end of compute (t, 2); group 1 in load (t, 0) and compute (t, 0), waited for at the end of load (t, 2) -- at
-        //   least two intervals of flight for the last piece.  The buffer it lands in held K-step t - 1, whose last reads (group
-        //   1, issued in its load (t - 1, 2)) are complete at the start of interval 8t: every issue point above lies behind
-        //   barrier 8t + 1.
-        // Same MFMA order per accumulator as the loop above: bit-identical results.
-        constexpr int NI = NXI * (TWO ? 2 : 1) + NWI;          // LDS-DMA instructions per wave and K-step
-        auto stage_piece = [&](int tl, char* buf, int piece) {
-            const int t = t0 + tl;
-            const bool tail = ktail && t == nkt - 1;
-            const int64_t ko = (int64_t)t * BK;
-            const int kchunks = tail ? (K - t * BK) / 8 : 8;
-            const int q0 = piece * NI / 2, q1 = (piece + 1) * NI / 2;
-            int q = 0;
-#pragma unroll
-            for (int j = 0; j < NXI; ++j) {
-                const bool ok = !tail || cx[j] < kchunks;
-                if (q >= q0 && q < q1) glds16(ok ? gx[j] + ko : p.zeros, buf + (wave * 16 + j * 8) * 128);
-                ++q;
-                if (TWO) {
-                    if (q >= q0 && q < q1) glds16(ok ? gx[j] + lo_delta + ko : p.zeros, buf + kXT + (wave * 16 + j * 8) * 128);
-                    ++q;
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < NWI; ++j) {
-                if (q >= q0 && q < q1)
-                    glds16((!tail || cw[j] < kchunks) ? gw[j] + ko : gw[j] - cw[j] * 8, buf + 2 * kXT + (wave * (BN / 8) + j * 8) * 128);
-                ++q;
-            }
-        };
-        const int grp = __builtin_amdgcn_readfirstlane(wave >> 2);
-        Frags fr2[2];                                           // slab s lives in set s & 1: read one phase ahead of its MFMAs
-        // The fragment reads of the ping-pong loop are raw ds_read_b128 statements hipcc does not count: a read issued in load
-        // segment s is consumed in compute segment s + 1 behind an explicit `s_waitcnt lgkmcnt(R)` (R = reads per slab: only
-        // the NEWER slab's reads may still be in flight).  Left to hipcc, the uniform `if (group)` branches between a read and
-        // its use make the waitcnt pass merge its scoreboards conservatively: lgkmcnt(0) in every other phase, i.e. the LDS
-        // latency of the just-issued reads in front of the MFMAs -- what the read-ahead is there to hide.  The loop holds no
-        // other LDS or scalar-memory instruction (checked in the ISA: lgkmcnt counts in order only without SMEM in flight).
-        constexpr int NR = MT * (TWO ? 2 : 1) + NT;
-        const uint32_t lds32 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
-        auto load_frags_raw = [&](Frags& f, uint32_t buf_off, int ks) {
-            const uint32_t aa = lds32 + buf_off + a_base + foff[ks], ab = lds32 + buf_off + b_base + foff[ks];
-#pragma unroll
-            for (int i = 0; i < MT; ++i) {
-                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f.ah[i]) : "v"(aa), "i"(i * 32 * 128));
-                if (TWO) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f.al[i]) : "v"(aa), "i"(kXT + i * 32 * 128));
-            }
-#pragma unroll
-            for (int j = 0; j < NT; ++j) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f.bw[j]) : "v"(ab), "i"(j * 32 * 128));
-        };
-        stage(0, lds);
-        stage(nk > 1 ? 1 : 0, lds + kStage);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // both K-steps (the prologue is not where the time goes)
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-        load_frags_raw(fr2[0], 0, 0);
-        if (grp) {                                              // group 1 runs one interval behind
-            __builtin_amdgcn_sched_barrier(0);
-            __builtin_amdgcn_s_barrier();
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        auto half_a = [&](const Frags& f) {                     // first half of a slab's MFMAs (hi plane; without a lo plane: the first row block)
-#pragma unroll
-            for (int i = 0; i < (TWO ? MT : (MT + 1) / 2); ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.ah[i], f.bw[j], acc[i][j], 0, 0, 0);
-        };
-        auto half_b = [&](const Frags& f) {
-            if (TWO) {
-#pragma unroll
-                for (int i = 0; i < MT; ++i)
-#pragma unroll
-                    for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.al[i], f.bw[j], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                              // one MFMA
+            if (MF >= 2 * R) {
+                if (k < R) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);               // one DS read
             } else {
-#pragma unroll
-                for (int i = (MT + 1) / 2; i < MT; ++i)
-#pragma unroll
-                    for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.ah[i], f.bw[j], acc[i][j], 0, 0, 0);
-            }
-        };
-        for (int t = 0; t < nk; ++t) {
-            char* cur = lds + (t & 1) * kStage;
-            char* nxt = lds + ((t + 1) & 1) * kStage;
-            const int u1 = t + 1 < nk ? t + 1 : nk - 1;         // (clamped: past the end the last K-step goes into the idle buffer again)
-#pragma unroll
-            for (int sl = 0; sl < 4; ++sl) {
-                // ---- load segment: only ISSUES the next slab's fragment reads (slab 0 of K-step t + 1 behind slab 3: its DMA was
-                // waited for two barriers ago); they complete under the partner group's MFMAs and this group's own ----
-                if (sl < 3) load_frags_raw(fr2[(sl + 1) & 1], (t & 1) * kStage, sl + 1);
-                else load_frags_raw(fr2[0], ((t + 1) & 1) * kStage, 0);     // (past the last K-step: the clamped re-load of it, never multiplied)
-                if (grp) {
-                    if (sl == 0) stage_piece(u1, nxt, 0);
-                    if (sl == 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                __builtin_amdgcn_s_barrier();
-                __builtin_amdgcn_sched_barrier(0);
-                // ---- compute segment: the slab read one phase ago; the newer slab's NR reads stay in flight ----
-                static_assert(NR == 6 || NR == 4 || NR == 3, "reads per slab");
-                if constexpr (NR == 6) asm volatile("s_waitcnt lgkmcnt(6)" ::: "memory");
-                else if constexpr (NR == 4) asm volatile("s_waitcnt lgkmcnt(4)" ::: "memory");
-                else asm volatile("s_waitcnt lgkmcnt(3)" ::: "memory");
-                __builtin_amdgcn_sched_barrier(0);
-                __builtin_amdgcn_s_setprio(1);
-                half_a(fr2[sl & 1]);
-                __builtin_amdgcn_sched_barrier(0);
-                if (!grp) {
-                    if (sl < 2) stage_piece(u1, nxt, sl);
-                } else {
-                    if (sl == 0) stage_piece(u1, nxt, 1);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                half_b(fr2[sl & 1]);
-                __builtin_amdgcn_s_setprio(0);
-                if (sl == 2 && !grp) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                __builtin_amdgcn_sched_barrier(0);
-                __builtin_amdgcn_s_barrier();
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (the read-ahead behind the last slab: landed before its registers die)
-        if (!grp) {                                             // group 0 waits for group 1's last compute segment
-            __builtin_amdgcn_s_barrier();
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    } else if constexpr (LO8) {
-        // ---- lockstep main loop with the lo plane on the int8 MFMA (round 5) ----
-        // Per K-step: 16 fp16 MFMAs for the hi plane (as without a lo plane) + 8 v_mfma_i32_32x32x32_i8 for the residual plane
-        // (two 32-deep blocks x MT x NT) instead of 16 more fp16 ones: 24 matrix-pipe slots instead of 32.  One int8 fragment set:
-        // block kb is read one slab ahead of its MFMAs like the fp16 fragments (kb 0 next to slab 0, kb 1 next to slab 2).
-        struct F8 { i4v a[MT], b[NT]; };
-        F8 f8;
-        auto load8 = [&](const char* buf, int kb) {
-#pragma unroll
-            for (int i = 0; i < MT; ++i) f8.a[i] = *(const i4v*)(buf + a8_base + i * 32 * 64 + foff8[kb]);
-#pragma unroll
-            for (int j = 0; j < NT; ++j) f8.b[j] = *(const i4v*)(buf + b8_base + j * 32 * 64 + foff8[kb]);
-        };
-        auto imfmas = [&]() {
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j) iacc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f8.a[i], f8.b[j], iacc[i][j], 0, 0, 0);
-        };
-        // (reads of the next slab, MFMAs of this one): one MFMA, then two reads, until the reads run out
-        auto pin = [&](auto r_, auto mf_) {
-            constexpr int R = decltype(r_)::value, MF = decltype(mf_)::value;
-#pragma unroll
-            for (int k = 0; k < MF; ++k) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 if (2 * k + 1 < R) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
                 else if (2 * k < R) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             }
-        };
-        using RH = std::integral_constant<int, MT + NT>;             // reads of one fp16 slab
-        using RB = std::integral_constant<int, 2 * (MT + NT)>;       // ... plus one int8 block
-        using MH = std::integral_constant<int, MT * NT>;             // MFMAs of one fp16 slab
-        using MB = std::integral_constant<int, 2 * MT * NT>;         // ... plus one int8 block
-        Frags fa, fb;
-        stage(0, lds);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (nk > 1) stage(1, lds + kStage);
-        load_frags(fa, lds, 0);
-        load8(lds, 0);
-        for (int t = 0; t + 1 < nk; ++t) {
-            const char* cur = lds + (t & 1) * kStage;
-            load_frags(fb, cur, 1);
-            mfmas(fa);
-            imfmas();
-            pin(RH{}, MB{});
-            load_frags(fa, cur, 2);
-            load8(cur, 1);
-            mfmas(fb);
-            pin(RB{}, MH{});
-            load_frags(fb, cur, 3);
-            mfmas(fa);
-            imfmas();
-            pin(RH{}, MB{});
+        }
+    };
+    // a slab that also carries the staging instructions [d0, d1) of K-step tl
+    auto slab_staging = [&](const Frags& f, Frags& nx, const char* buf, int ks, int tl, char* to, int d0, int d1) {
+#pragma unroll
+        for (int k = 0; k < MF; ++k) {
+            mfma_one(f, k);
             __builtin_amdgcn_sched_barrier(0);
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __syncthreads();
-            const int tn = t + 2 < nk ? t + 2 : nk - 1;
-            // (the DMA issue spread between this slab's MFMAs -- see the fp16 loop below -- measured SLOWER here: 4177 vs 4136 us per
-            // layer at 6000 rows, profiles/r05_variants.txt)
-            stage(tn, lds + (t & 1) * kStage);
-            load_frags(fa, lds + ((t + 1) & 1) * kStage, 0);
-            load8(lds + ((t + 1) & 1) * kStage, 0);
-            mfmas(fb);
-            pin(RB{}, MH{});
+            reads_behind(nx, buf, ks, k);
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+                if (i >= d0 + k * (d1 - d0) / MF && i < d0 + (k + 1) * (d1 - d0) / MF) stage(i, tl, to);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        {
-            const char* cur = lds + ((nk - 1) & 1) * kStage;
-            load_frags(fb, cur, 1);
-            mfmas(fa);
-            imfmas();
-            pin(RH{}, MB{});
-            load_frags(fa, cur, 2);
-            load8(cur, 1);
-            mfmas(fb);
-            pin(RB{}, MH{});
-            load_frags(fb, cur, 3);
-            mfmas(fa);
-            imfmas();
-            pin(RH{}, MB{});
-            mfmas(fb);
-        }
-        // the residual product joins the fp32 accumulator: y += int_sum * xl8_scale[row] * w8_scale[col]
-        {
-            float wsc[NT];
-#pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                int gr = wrow(wn * 64 + 32 * j + fr);
-                wsc[j] = p.w8_scale[gr < 0 ? 0 : gr];
-            }
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m = m0 + wm * 32 * MT + 32 * i + 8 * (r >> 2) + 4 * fh + (r & 3);
-                    const float xs = p.xl8_scale[m < p.M ? m : p.M - 1];
-#pragma unroll
-                    for (int j = 0; j < NT; ++j) acc[i][j][r] = __builtin_fmaf((float)iacc[i][j][r], xs * wsc[j], acc[i][j][r]);
-                }
-        }
-    } else {
+    };
+    auto clamp = [&](int t) { return t < nk ? t : nk - 1; };        // (past the end the last K-step goes into the idle buffer again)
     Frags fa, fb;
-    stage(0, lds);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (nk > 1) stage(1, lds + kStage);
-    load_frags(fa, lds, 0);
-    for (int t = 0; t + 1 < nk; ++t) {
-        const char* cur = lds + (t & 1) * kStage;
-        load_frags(fb, cur, 1);
-        mfmas(fa);
-        interleave();
-        load_frags(fa, cur, 2);
-        mfmas(fb);
-        interleave();
-        load_frags(fb, cur, 3);
-        mfmas(fa);
-        interleave();
-        // K-step t+1 has landed (this wave's LDS-DMA drained, then everyone's via the barrier), and every wave's reads
-        // of K-step t are complete (__syncthreads waits lgkmcnt(0)): its buffer may be overwritten.  The stage index
-        // is clamped instead of branched on (past the end it re-loads the last K-step into the idle buffer): a branch
-        // here splits the block and hipcc then waits for the fresh reads below before the MFMAs that do not need them.
-        __builtin_amdgcn_sched_barrier(0);      // slab 2's MFMAs stay in front of the barrier: they cover slab 3's reads
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        const int tn = t + 2 < nk ? t + 2 : nk - 1;
-        if constexpr (PC_DENSE_SPREAD_DMA && TWO) {
-            constexpr int MF = MT * NT * (TWO ? 2 : 1), R = MT * (TWO ? 2 : 1) + NT, V = NXI * (TWO ? 2 : 1) + NWI;
-            const char* nb = lds + ((t + 1) & 1) * kStage;
 #pragma unroll
-            for (int k = 0; k < MF; ++k) {
-                mfma_one(fb, k);
-                __builtin_amdgcn_sched_barrier(0);
-                if (2 * k < R) read_one(fa, nb, 0, 2 * k);
-                if (2 * k + 1 < R) read_one(fa, nb, 0, 2 * k + 1);
-                stage_range(tn, lds + (t & 1) * kStage, k * V / MF, (k + 1) * V / MF);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        } else {
-            stage(tn, lds + (t & 1) * kStage);
-            load_frags(fa, lds + ((t + 1) & 1) * kStage, 0);
-            mfmas(fb);
-            interleave();
-        }
+    for (int st = 0; st < S - 1; ++st)
+#pragma unroll
+        for (int i = 0; i < NI; ++i) stage(i, clamp(st), lds + st * kStage);
+#pragma unroll
+    for (int i = 0; i < D0; ++i) stage(i, clamp(S - 1), lds + (S - 1) * kStage);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * NI + D0) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int q = 0; q < R; ++q) read_one(fa, lds, 0, q);
+    int cur = 0, prev = (S - 1) * kStage;                            // images of K-steps t and t + S - 1
+    for (int t = 0; t + 1 < nk; ++t) {
+        slab_staging(fa, fb, lds + cur, 1, clamp(t + S - 1), lds + prev, D0, NI);
+        slab(fb, fa, lds + cur, 2);
+        slab(fa, fb, lds + cur, 3);
+        // K-step t + 1 has landed (S - 2 younger ones may be in flight), for everyone behind the barrier; every wave's reads of K-step t are complete
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * NI) : "memory");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        prev = cur;
+        cur = cur + kStage == S * kStage ? 0 : cur + kStage;
+        slab_staging(fb, fa, lds + cur, 0, clamp(t + S), lds + prev, 0, D0);
     }
-    {
-        const char* cur = lds + ((nk - 1) & 1) * kStage;
-        load_frags(fb, cur, 1);
-        mfmas(fa);
-        interleave();
-        load_frags(fa, cur, 2);
-        mfmas(fb);
-        interleave();
-        load_frags(fb, cur, 3);
-        mfmas(fa);
-        interleave();
-        mfmas(fb);
-    }
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // (the clamped re-load of the last K-step)
+    slab(fa, fb, lds + cur, 1);
+    slab(fb, fa, lds + cur, 2);
+    slab(fa, fb, lds + cur, 3);
+#pragma unroll
+    for (int q = 0; q < MF; ++q) mfma_one(fb, q);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // (clamped re-loads of the last K-step)
 
-    // ---- epilogue: accumulators -> wave-private LDS tile [32*MT][64] fp32 -> full-row global stores ----
+    // ---- epilogue: accumulators -> wave-private LDS tile [32 MT][64] fp32, one 64-column group at a time -> full-row global stores ----
     __syncthreads();                                       // every wave is done with the staging buffers
     float* st = (float*)(lds + wave * (32 * MT * 64 * 4));
+    const int mrow0 = m0 + wm * 32 * MT;
+#pragma unroll
+    for (int half = 0; half < NT / 2; ++half) {
+    const int grp = wn * (NT / 2) + half;                  // the 64-column group inside the block tile
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r)
-                st[(32 * i + 8 * (r >> 2) + 4 * fh + (r & 3)) * 64 + 32 * j + fr] = acc[i][j][r];
-    const int mrow0 = m0 + wm * 32 * MT;
+                st[(32 * i + 8 * (r >> 2) + 4 * fh + (r & 3)) * 64 + 32 * j + fr] = acc[i][2 * half + j][r];
     if (EPI == EPI_SILU) {
         // the wave's 64 columns are [32 gate features | the same 32 up features]: 8 lanes per row, 4 features per lane
-        const int fbase = (ni * WN + wn) * 32 + (lane & 7) * 4;
+        const int fbase = (ni * NT + grp) * 32 + (lane & 7) * 4;
 #pragma unroll
         for (int it = 0; it < 4 * MT; ++it) {
             const int row = it * 8 + (lane >> 3), m = mrow0 + row;
@@ -689,14 +327,14 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseParams p) {
                 if (p.ol) *(h4*)(p.ol + (int64_t)m * p.ldo + fbase) = lo;
             }
         }
-        return;
+        continue;
     }
     if (EPI == EPI_ROPE) {
         // RoPE at the supplied positions (llama2.py:200-213, :357-359) and the KV append (:361-364) on the accumulator tile:
         // 8 lanes per row, a lane holds features d0 .. d0+3 and d0+64 .. d0+67 of head `hd`
-        const int hd = ni * (BN / 128) + (wn >> 1);
-        const int d0 = (wn & 1) * 32 + (lane & 7) * 4;
-        if (hd >= p.H + 2 * p.Hkv) return;
+        const int hd = ni * (BN / 128) + (grp >> 1);
+        const int d0 = (grp & 1) * 32 + (lane & 7) * 4;
+        if (hd >= p.H + 2 * p.Hkv) continue;
         const bool rot = hd < p.H + p.Hkv;
 #pragma unroll
         for (int it = 0; it < 4 * MT; ++it) {
@@ -742,9 +380,9 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseParams p) {
             *(h4*)(dh + 64) = ch;
             if (dl) { *(h4*)dl = al; *(h4*)(dl + 64) = cl; }
         }
-        return;
+        continue;
     }
-    const int n = ni * BN + wn * 64 + (lane & 15) * 4;
+    const int n = ni * BN + grp * 64 + (lane & 15) * 4;
 #pragma unroll
     for (int it = 0; it < 8 * MT; ++it) {
         const int row = it * 4 + (lane >> 4), m = mrow0 + row;
@@ -783,6 +421,7 @@ __global__ __launch_bounds__(512) void gemm_dense_kernel(const DenseParams p) {
             }
         }
     }
+    }
 }
 
 // Split-K tail: y[m][n] (+)= sum_z slab[z][m][n], slabs added in slice order (deterministic), 16 B per lane.
@@ -810,41 +449,42 @@ __global__ __launch_bounds__(256) void dense_reduce_kernel(const float* __restri
 // 16 bytes of zeros for activation chunks past K (device constant: no allocation, graph-capturable)
 __device__ __attribute__((aligned(16))) _Float16 g_zero_chunk[8];
 
-template <int WM, int EPI>
-int launch_dense(DenseParams& p, hipStream_t s, int kslices = 1) {
-    constexpr int BN = 64 * (8 / WM);
-    const int units = (EPI == EPI_SILU) ? pc_ceil_div(p.nfeat, BN / 2) : pc_ceil_div(p.N, BN);
+template <int EPI, bool TWO, bool NARROW, bool TALL>
+int launch_dense_as(DenseParams& p, hipStream_t s, int kslices) {
+    constexpr int BM = Tile<2, TWO, NARROW, TALL>::BM, BN = Tile<2, TWO, NARROW, TALL>::BN;
     p.mb = pc_ceil_div(p.M, BM);
-    p.nb = units;
+    p.nb = (EPI == EPI_SILU) ? pc_ceil_div(p.nfeat, BN / 2) : pc_ceil_div(p.N, BN);
     const int nkt = pc_ceil_div(p.K, BK);
     p.kper = pc_ceil_div(nkt, kslices);
-    const dim3 grid(8 * p.mb * pc_ceil_div(p.nb, 8), pc_ceil_div(nkt, p.kper)), block(512);
-#ifdef PC_DEV_SWEEPS
-    // The ping-pong main loop (PP = true) is a MEASURED NEGATIVE RESULT and only built for A/B (PC_BUILD_FLAGS=-DPC_DEV_SWEEPS,
-    // then PC_DENSE_PP=1; tools/dense_pp_ab.py): bit-identical to the lockstep loop and 0.87-0.90 x its speed at the encode's
-    // shapes with both planes, 0.66-0.83 x on one plane (profiles/r05_dense_pp_ab.txt).
-    const char* e = getenv("PC_DENSE_PP");
-    if (e && e[0] == '1') {
-        if (p.xl) hipLaunchKernelGGL((gemm_dense_kernel<WM, EPI, true, true>), grid, block, 0, s, p);
-        else hipLaunchKernelGGL((gemm_dense_kernel<WM, EPI, false, true>), grid, block, 0, s, p);
-        return pc_check_launch("gemm_dense_kernel");
+    // strips: fewest rounds of an XCD's 32 CUs, then fewest rows (activations of mh M-blocks, weights of the panels 32 tiles reach) per K-step
+    int64_t best = -1;
+    for (int px = 1; px <= 8; px *= 2) {
+        const int mh = pc_ceil_div(p.mb, px), nh = pc_ceil_div(p.nb, 8 / px), reach = mh < 32 ? mh : 32;
+        const int64_t cost = ((int64_t)pc_ceil_div(mh * nh, 32) << 32) + reach * (TWO ? 2 : 1) * BM + pc_ceil_div(32, reach) * BN;
+        if (best < 0 || cost < best) { best = cost; p.px = px; p.mh = mh; p.nh = nh; }
     }
-#endif
-    if (p.xl8) {
+    hipLaunchKernelGGL((gemm_dense_kernel<2, EPI, TWO, NARROW, TALL>), dim3(8 * p.mh * p.nh, pc_ceil_div(nkt, p.kper)), dim3(256), 0, s, p);
+    return pc_check_launch("gemm_dense_kernel");
+}
+
 #ifdef PC_DEV_SWEEPS
-        if constexpr (EPI == EPI_GELU) {               // (no caller: the Falcon / MPT stacks keep the fp16 residual plane)
-            pc_set_error("pc_gemm_dense_lo8: no GELU instantiation");
-            return PC_ERR_ARG;
-        } else {
-            hipLaunchKernelGGL((gemm_dense_kernel<WM, EPI, false, false, true>), grid, block, 0, s, p);
-        }
+#include "pc_gemm_dense_dev.h"
+#endif
+
+// the 128-row tiles, BN = 256 or 128 columns
+template <int BN, int EPI>
+int launch_dense(DenseParams& p, hipStream_t s, int kslices = 1) {
+#ifdef PC_DEV_SWEEPS
+    const char* e = getenv("PC_DENSE_PP");
+    if (p.xl8 || (e && e[0] == '1')) return lockstep::launch<BN == 256 ? 2 : 4, EPI>(p, s, kslices);
 #else
+    if (p.xl8) {
         pc_set_error("pc_gemm_dense: the int8 residual plane (x_lo8) needs a -DPC_DEV_SWEEPS build (csrc/pc_dev.h)");
         return PC_ERR_ARG;
+    }
 #endif
-    } else if (p.xl) hipLaunchKernelGGL((gemm_dense_kernel<WM, EPI, true, false>), grid, block, 0, s, p);
-    else hipLaunchKernelGGL((gemm_dense_kernel<WM, EPI, false, false>), grid, block, 0, s, p);
-    return pc_check_launch("gemm_dense_kernel");
+    if (p.xl) return launch_dense_as<EPI, true, BN == 128, false>(p, s, kslices);
+    return launch_dense_as<EPI, false, BN == 128, false>(p, s, kslices);
 }
 
 // Few-row launches of the N = hidden projections (o_proj, down_proj at a few hundred rows: 64-128 tiles of 128 x 256 for
@@ -856,7 +496,7 @@ int launch_dense_splitk(DenseParams& p, hipStream_t s, float* ws, int64_t ws_byt
     static const int forced_bn = [] { const char* e = getenv("PC_DENSE_BN"); return e ? atoi(e) : 0; }();
     *launched = 0;
     if (!ws || p.xscale || (EPI != EPI_ADD && EPI != EPI_STORE)) return 0;
-    const int nkt = pc_ceil_div(p.K, BK), mb = pc_ceil_div(p.M, BM);
+    const int nkt = pc_ceil_div(p.K, BK), mb = pc_ceil_div(p.M, 128);
     // widest panel whose slices still fill the chip: 256-wide tiles do twice the MFMAs per LDS byte of 128-wide ones
     const int b256 = mb * pc_ceil_div(p.N, 256), b128 = mb * pc_ceil_div(p.N, 128);
     bool narrow = forced_bn ? forced_bn == 128 : false;
@@ -867,7 +507,7 @@ int launch_dense_splitk(DenseParams& p, hipStream_t s, float* ws, int64_t ws_byt
     if (ks < 2 || (int64_t)ks * p.M * p.N * 4 > ws_bytes) return 0;
     float* y = p.y; const int64_t ldy = p.ldy;
     p.y = ws; p.ldy = p.N; p.slab_stride = (int64_t)p.M * p.N;
-    const int rc = narrow ? launch_dense<4, EPI_STORE>(p, s, ks) : launch_dense<2, EPI_STORE>(p, s, ks);
+    const int rc = narrow ? launch_dense<128, EPI_STORE>(p, s, ks) : launch_dense<256, EPI_STORE>(p, s, ks);
     if (rc) return rc;
     const int nslab = pc_ceil_div(pc_ceil_div(p.K, BK), p.kper);
     const int64_t items = (int64_t)p.M * (p.N >> 2);
@@ -886,10 +526,15 @@ int launch_dense_tile(DenseParams& p, hipStream_t s) {
     // profiles/r02_dense_splitk.txt), e.g. 1000 x 4096: 128 wide tiles = one round of half the chip, 256 narrow tiles =
     // one round of all of it
     const int cols = (EPI == EPI_SILU) ? p.nfeat * 2 : p.N;
-    const int mb = pc_ceil_div(p.M, BM);
+    const int mb = pc_ceil_div(p.M, 128);
     const int b256 = mb * pc_ceil_div(cols, 256), b128 = mb * pc_ceil_div(cols, 128);
     const bool narrow = forced ? forced == 128 : (b256 <= 512 && 0.62f * pc_ceil_div(b128, 256) < 1.0f * pc_ceil_div(b256, 256));
-    return narrow ? launch_dense<4, EPI>(p, s) : launch_dense<2, EPI>(p, s);
+    // One plane: 256 x 256 tiles where their whole rounds of the 256 CUs cost less than the 128 x 256 tiles' total.  Per round at K = 4096
+    // (one plane, N = 12288 / 22016 / 32000, 1 737 / 2 940 / 3 584 rows): 95-111 us against 61-70 us, the latter hardly quantised.
+    // (Both planes: 256-row tiles need 32-deep K-steps and gain 4 % at best, 3 584 x 12 288; 128-row tiles throughout.)
+    const int b2 = pc_ceil_div(p.M, 256) * pc_ceil_div(cols, 256);
+    if (!p.xl && !p.xl8 && !forced && !narrow && 1.52f * 256.f * pc_ceil_div(b2, 256) < (float)b256) return launch_dense_as<EPI, false, false, true>(p, s, 1);
+    return narrow ? launch_dense<128, EPI>(p, s) : launch_dense<256, EPI>(p, s);
 }
 
 }  // namespace

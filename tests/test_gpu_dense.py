@@ -61,6 +61,32 @@ def test_dense_store_and_add(M, N, K, two):
 
 # few-row launches of the N = hidden projections take the split-K form when a workspace is supplied (pc_gemm_dense_ws);
 # (1000, 12288, 4096) and (77, 512, 8) do not split (large grid / too few K-steps) and must equal pc_gemm_dense bit for bit
+@pytest.mark.parametrize("M,N,two", [(2001, 8188, False), (2001, 8188, True), (1025, 4100, True), (897, 16388, False)])
+@pytest.mark.parametrize("K", [8, 64, 72, 128, 200, 264])
+def test_dense_tall_tiles_strips_and_short_rings(M, N, K, two):
+    """One to five K-steps (fewer than the ring has images, and a partial last one) through the 256 x 256 tiles of one plane over many
+    rows, through the 128 x 256 tiles and through every cut of the grid into strips, with partial tiles at both edges.  A sum of planes x K
+    fp32 products and additions is off by at most planes x K x 2^-24 of the sum of magnitudes."""
+    n = _n()
+    g = torch.Generator(device="cuda:0").manual_seed(M + K)
+    x = torch.randn((M, K), generator=g, device="cuda:0")
+    hi = x.half()
+    lo = (x - hi.float()).half()
+    w = (torch.randn((N, K), generator=g, device="cuda:0") * 0.05).half()
+    y = torch.full((M, N), float("nan"), device="cuda:0")
+    n.gemm_dense(hi, lo if two else None, w, M, N, K, n.EPI_STORE, y=y)
+    full = hi.double() + (lo.double() if two else 0.0)
+    bound = (2 if two else 1) * K * 2.0 ** -24 * (hi.double().abs() + (lo.double().abs() if two else 0.0)) @ w.double().abs().T
+    assert bool(((y.double() - full @ w.double().T).abs() <= bound).all())
+    if K == 200:
+        N -= N % 8
+        oh, ol = (torch.full((M, N // 2), float("nan"), dtype=torch.float16, device="cuda:0") for _ in range(2))
+        n.gemm_dense(hi, lo if two else None, w[:N].contiguous(), M, N, K, n.EPI_SILU, out_hi=oh, out_lo=ol)
+        want = torch.nn.functional.silu(y[:, :N // 2].double()) * y[:, N // 2:N].double()
+        # (two planes hold 22 bits of the product; the exponential and the quotient are good to a few units in the last place)
+        assert bool(((oh.double() + ol.double() - want).abs() <= 2.0 ** -19 * (want.abs() + 2.0 ** -6)).all())
+
+
 @pytest.mark.parametrize("two", [True, False])
 @pytest.mark.parametrize("M,N,K", [(300, 4096, 4096), (512, 4096, 11008), (130, 260, 1096), (800, 5120, 13824),
                                    (1000, 12288, 4096), (77, 512, 8), (1, 4096, 4096)])
