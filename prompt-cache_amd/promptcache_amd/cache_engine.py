@@ -26,7 +26,7 @@ import torch
 
 from . import _native, parallel
 from .model import LanguageModel
-from .model.kv_arena import KVArena, StagedKV, StagingPlan
+from .model.kv_arena import KVArena, uploaded, StagedKV, StagingPlan
 from .pml import Module, ModuleRef, Path, Prompt, Schema, TokenSequence, UnionModule  # noqa: F401
 
 KVCache = List[Tuple[torch.Tensor, torch.Tensor]]
@@ -471,8 +471,8 @@ class SchemaCache:
         trunk_arena: Optional[KVArena] = None
         if shared:
             job = jobs[0]
-            out = lm(input_ids=torch.tensor([job["token_ids"][:need[0]]], device=dev, dtype=torch.long),
-                     position_ids=torch.tensor([job["position_ids"][:need[0]]], device=dev, dtype=torch.long), use_cache=True,
+            out = lm(input_ids=uploaded([job["token_ids"][:need[0]]], torch.long, dev),
+                     position_ids=uploaded([job["position_ids"][:need[0]]], torch.long, dev), use_cache=True,
                      many_rows=True, kv_only=True)
             trunk_arena = out.past_key_values.arena
             computed_tokens += need[0]
@@ -485,8 +485,8 @@ class SchemaCache:
         for idxs in self._pack(whole, need, batch_size):
             ids_pad, mask = pad_batch([jobs[i]["token_ids"][:need[i]] for i in idxs], lm.eos_token_id)
             pos_pad, _ = pad_batch([jobs[i]["position_ids"][:need[i]] for i in idxs], 0)
-            out = lm(input_ids=torch.tensor(ids_pad, device=dev, dtype=torch.long),
-                     position_ids=torch.tensor(pos_pad, device=dev, dtype=torch.long),
+            out = lm(input_ids=uploaded(ids_pad, torch.long, dev),
+                     position_ids=uploaded(pos_pad, torch.long, dev),
                      attention_mask=torch.tensor(mask, dtype=torch.float16),     # (host: the HIP path only checks it is right-padded)
                      use_cache=True, many_rows=True, kv_only=True)
             arena: KVArena = out.past_key_values.arena
@@ -530,8 +530,8 @@ class SchemaCache:
             if in_place:
                 ids_pad, mask = pad_batch([jobs[i]["token_ids"][prefix[i]:need[i]] for i in idxs], lm.eos_token_id)
                 pos_pad, _ = pad_batch([jobs[i]["position_ids"][prefix[i]:need[i]] for i in idxs], 0)
-                out = lm(input_ids=torch.tensor(ids_pad, device=dev, dtype=torch.long),
-                         position_ids=torch.tensor(pos_pad, device=dev, dtype=torch.long),
+                out = lm(input_ids=uploaded(ids_pad, torch.long, dev),
+                         position_ids=uploaded(pos_pad, torch.long, dev),
                          attention_mask=torch.tensor(mask, dtype=torch.float16),     # (host: the HIP path only checks it is right-padded)
                          use_cache=True, many_rows=True, kv_only=True, shared_prefix=(trunk_arena, pre))
                 arena = out.past_key_values.arena
@@ -561,9 +561,9 @@ class SchemaCache:
             pos_pad, _ = pad_batch([jobs[i]["position_ids"][prefix[i]:need[i]] for i in idxs], 0)
             if full_pos:                                 # ALiBi models take the position id of every key
                 pos_pad = [list(jobs[0]["position_ids"][:n_max]) + row for row in pos_pad]
-            extra = {} if n_same is not None else {"past_lens": torch.tensor(pre, device=dev, dtype=torch.int32)}
-            out = lm(input_ids=torch.tensor(ids_pad, device=dev, dtype=torch.long),
-                     position_ids=torch.tensor(pos_pad, device=dev, dtype=torch.long),
+            extra = {} if n_same is not None else {"past_lens": uploaded(pre, torch.int32, dev)}
+            out = lm(input_ids=uploaded(ids_pad, torch.long, dev),
+                     position_ids=uploaded(pos_pad, torch.long, dev),
                      attention_mask=torch.tensor(mask, dtype=torch.float16),     # (host: the HIP path only checks it is right-padded)
                      past_key_values=arena.views(), use_cache=True, many_rows=True, kv_only=True, **extra)
             arena = out.past_key_values.arena

@@ -35,7 +35,7 @@ import numpy as np
 
 from .. import _native
 from .config import LlamaShape
-from .kv_arena import KVArena, StagedKV, arena_from_past
+from .kv_arena import KVArena, StagedKV, arena_from_past, uploaded
 
 _SEG_DTYPE = np.dtype([("src", "<u8"), ("dst_row", "<i4"), ("len", "<i4")])      # pc_kv_seg
 
@@ -552,7 +552,7 @@ class LlamaHIP:
                     and len(n_pre) == B and trunk.B == 1 and max(n_pre) <= trunk.length):
                 raise ValueError("shared_prefix goes with many_rows=True, explicit position ids, no past_key_values and a one-row "
                                  "trunk arena that holds every prefix")
-            self._shared = (trunk, torch.tensor(list(n_pre), device=dev, dtype=torch.int32), int(max(n_pre)))
+            self._shared = (trunk, uploaded(list(n_pre), torch.int32, dev), int(max(n_pre)))
         arena, past_len = self._resolve_arena(past_key_values, B, q_len, keep_pending=True)
         if many_rows and self.precise_dense and past_key_values is None:
             arena.with_lo()           # a schema-encode pass: keep the residuals of every row it appends
