@@ -267,8 +267,7 @@ __device__ __forceinline__ void scale_frag<bf16_t>(Frag<bf16_t>& f, float s) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const uint32_t w = f.v[e];
-        const uint32_t lo = bf16_bits(s * __uint_as_float(w << 16)), hi = bf16_bits(s * __uint_as_float(w & 0xffff0000u));
-        f.v[e] = lo | (hi << 16);
+        f.v[e] = bf16_pair(s * __uint_as_float(w << 16), s * __uint_as_float(w & 0xffff0000u));
     }
 }
 template <>
@@ -602,8 +601,7 @@ __global__ __launch_bounds__(256) void linear_dma_kernel(pcb_linear_args a) {
                     if (a.out_f32)
                         *reinterpret_cast<f4*>((float*)a.y + at) = v;
                     else
-                        *reinterpret_cast<uint2*>((E*)a.y + at) = uint2{(uint32_t)bf16_bits(v[0]) | ((uint32_t)bf16_bits(v[1]) << 16),
-                                                                        (uint32_t)bf16_bits(v[2]) | ((uint32_t)bf16_bits(v[3]) << 16)};
+                        *reinterpret_cast<uint2*>((E*)a.y + at) = uint2{bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3])};
                 }
             } else {
 #pragma unroll

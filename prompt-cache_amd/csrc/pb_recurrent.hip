@@ -189,7 +189,7 @@ __device__ __forceinline__ void load2(const float* p, float (&o)[2]) {
     o[0] = w.x, o[1] = w.y;
 }
 __device__ __forceinline__ void store2(bf16_t* p, float a, float b) {
-    *reinterpret_cast<uint32_t*>(p) = (uint32_t)bf16_bits(a) | ((uint32_t)bf16_bits(b) << 16);
+    *reinterpret_cast<uint32_t*>(p) = bf16_pair(a, b);
 }
 __device__ __forceinline__ void store2(float* p, float a, float b) { *reinterpret_cast<float2*>(p) = float2{a, b}; }
 

@@ -232,6 +232,26 @@ def matmul32(x, w):
     return torch.matmul(x.float(), w.float().t().contiguous())
 
 
+@pytest.mark.parametrize("M", [3, 40, 300])
+def test_bf16_results_are_the_fp32_results_rounded_to_nearest_even(M):
+    """Sums of two products that fall on, beside and between the halves of a bf16 step, at every exponent, infinities and NaN: a bf16 result is
+    the bits of the same call's fp32 result rounded once."""
+    b, bf, N = B(), torch.bfloat16, 96
+    x, w = torch.zeros(M, 8, dtype=bf, device=DEV), torch.zeros(N, 8, dtype=bf, device=DEV)
+    step = torch.arange(N, device=DEV)
+    x[:, 0] = (1.0 + torch.arange(M, device=DEV) % 128 / 128.0).to(bf)
+    x[:, 1] = 1.0
+    w[:, 0] = torch.exp2((step % 48 * 5 - 120).float()).to(bf)
+    w[:, 1] = w[:, 0] * (step % 7 - 3).to(bf) * 2.0 ** -9                      # 2^-8 of the step at 1: odd multiples of a half and less
+    x[M - 1, 0], x[M // 2, 0] = float("inf"), float("nan")
+    y32, y16 = torch.zeros(M, N, device=DEV), torch.zeros(M, N, dtype=bf, device=DEV)
+    b.linear(x, w, y32, M=M)
+    b.linear(x, w, y16, M=M)
+    want = y32.to(bf)
+    assert torch.equal(torch.isnan(y16), torch.isnan(want)) and torch.equal(torch.nan_to_num(y16), torch.nan_to_num(want))
+    assert bool((y32 != want.float()).any())
+
+
 @pytest.mark.parametrize("M,N", [(2048, 2048), (2000, 2300), (1000, 3300), (300, 1100), (130, 80), (40, 200), (29, 264)])
 @pytest.mark.parametrize("K", [8, 72, 200, 1032])
 def test_many_row_projections_at_every_tile_shape_and_their_edges(M, N, K):
