@@ -11,8 +11,7 @@
 // Y[m][n] = sum_k (Xhi[m][k] + Xlo[m][k]) * W[n][k]       X: split-precision fp16 planes [M][K] (hi = fp16(x),
 //                                                          lo = fp16(x - hi); lo optional), W: nn.Linear [N][K] fp16
 // Why two planes: an fp16 activation costs 2^-12 per projection input, and through 32 layers that alone moves
-// 7b-shape logits by 2-3e-2 against the reference's fp32 CPU path.  Round 1 ran [hi; lo] stacked
-// along the rows of a vendor GEMM and added the halves in separate fp32 passes.  Here both planes meet the SAME weight
+// 7b-shape logits by 2-3e-2 against the reference's fp32 CPU path.  Both planes meet the SAME weight
 // fragment inside one tile pass: a weight fragment is read from LDS once and feeds the hi and the lo MFMA, the two
 // partial products meet in the fp32 accumulator, and the epilogue (residual add, SiLU*up, GELU, fp32 store) runs on the
 // accumulator tile -- no [2T][N] fp32 intermediate ever exists.
@@ -21,18 +20,13 @@
 // one, 256 x 256 with one plane over many rows, 128 x 128 for launches whose 256-wide grid would leave CUs idle (launch_dense_tile).
 // What bounds it: power (the matrix cores run these launches at 1.4-1.7 GHz; the same launches on zeros are 1.2-1.3 x faster), LDS bandwidth
 // next.  Per 16-deep k-slab and both planes a wave of 64 x 128 reads 8 KiB of LDS for 16 MFMAs, two waves of 64 x 64 read 12 KiB for as
-// many: the same block tile on eight waves kept the LDS pipe as busy as the matrix pipe.  Eight waves -> four, random data: both planes,
-// 1 737 rows, q|k|v 345 -> 322 us, down 305 -> 286, 32 000 columns 854 -> 797 (1.14 PFLOP/s executed), 3 584 rows down 624 -> 581; one
-// plane, gate|up, 1 737 / 2 940 / 3 584 rows 384 -> 361, 622 -> 577, 760 -> 599 us (256 x 256 tiles, 1.08 PFLOP/s).
+// many: the same block tile on eight waves kept the LDS pipe as busy as the matrix pipe.  Eight waves with an epilogue that read residuals
+// between its stores -> this kernel, us, random data: both planes, 1 737 rows, q|k|v 329 -> 307, o_proj 113 -> 103, down 288 -> 265
+// (1.18 PFLOP/s executed), 32 000 columns 816 -> 758, 3 584 rows down 598 -> 532; one plane, gate|up, 1 737 / 2 940 / 3 584 rows 370 -> 324,
+// 600 -> 528, 729 -> 561 (256 x 256 tiles, 1.15 PFLOP/s).
 // mfma_f32_32x32x16_f16: per 16-deep k-slab a wave reads MT (2 MT with both planes) activation fragments and NT weight fragments
 // (16 B per lane each, ds_read_b128) for MT NT (2 MT NT) MFMAs.
-// Staging: global_load_lds (16 B per lane, 1 KiB per wave-instruction = 8 rows x 128 B of a tile) straight into a ring of two or three
-// LDS images, one barrier per K-step.  The first half of a wave's instructions for a K-step goes out between the MFMAs behind the barrier
-// that frees its buffer, the second half between those of the next step's first slab.
-// The LDS image keeps 128-byte rows; the 16-byte chunk c of row r sits at chunk position c ^ ((r >> 1) & 7), which
-// makes every ds_read_b128 lane group of a fragment read hit 16 distinct 16-byte bank slots (row-major 128-B rows
-// would be 8-way conflicted).  LDS-DMA writes lane-linearly, so the permutation is applied to the per-lane SOURCE
-// address and again on the read.
+// Staging, LDS image and main loop: mfma_tile_loop.h.
 // Which global weight row lands in which LDS row is free as well (per-lane source address): the SiLU launch puts 32
 // gate rows and the 32 matching up rows side by side in one 64-column group, so gate_j and up_j meet in the same lane.
 // Epilogue: the accumulator tile goes through the (now idle) LDS, 64 columns of a wave at a time, so that every global store is 16 B per
@@ -46,6 +40,7 @@
 
 #include <type_traits>
 
+#include "mfma_tile_loop.h"
 #include "pc_common.h"
 #ifdef PC_DEV_SWEEPS
 #include "pc_dev.h"
@@ -68,12 +63,12 @@ struct DenseParams {
     // LLM.int8 (pc_int8.hip): xh holds activation CODES, xscale[m] = SCA[m] / 127; corr[m][n] (global weight-row index n) is
     // added before the epilogue's nonlinearity when *corr_has != 0
     const float* xscale; const float* corr; int64_t ldc; const int32_t* corr_has;
-    // LO8 (round 5): the lo activation plane as INT8 codes [M][K] with one scale per row (lo ~ code * xl8_scale[m]) against an int8
+    // LO8: the lo activation plane as INT8 codes [M][K] with one scale per row (lo ~ code * xl8_scale[m]) against an int8
     // image of the weights [N][K] with one scale per row (W ~ code * w8_scale[n]): the residual product runs on
     // v_mfma_i32_32x32x32_i8 -- twice the fp16 MFMA rate, exact integer sums -- and joins the fp32 accumulator in the epilogue
     const signed char* xl8; const float* xl8_scale; int64_t ldx8;
     const signed char* w8; const float* w8_scale; int64_t ldw8;
-    const _Float16* zeros;                                 // >= 16 B of zeros: source of activation chunks past K
+    const _Float16* zeros;                                 // >= 16 B of zeros (the -DPC_DEV_SWEEPS kernels' chunks past K)
     float* y; int64_t ldy;                                 // EPI_STORE / EPI_ADD
     _Float16* oh; _Float16* ol; int64_t ldo;               // EPI_SILU / EPI_GELU output planes
     int32_t M, N, K, mb, nb, nfeat;                        // nfeat: SiLU features (= N / 2)
@@ -101,17 +96,149 @@ struct Tile {
     static constexpr int BM = 32 * W * MT, BN = 32 * W * NT;
 };
 
+// The 64 columns of group `grp` (of the launch's weight rows; EPI_SILU: 32 gate and the matching 32 up features, EPI_ROPE: 32 features of a
+// head's first half and their rotary partners), rows mrow0 .. + 32 MT - 1, from a wave's patch to where they go.
+// Loads come before stores and loops are short: a wait for a load behind a store waits for the store's way to memory and back (they count
+// on one counter), and unrolled code that runs once is paid in instruction misses.
+template <int EPI, int MT>
+__device__ __forceinline__ void store_group(const DenseParams& p, char* patch, int lane, int grp, int mrow0) {
+    constexpr bool PAIRS = EPI == EPI_SILU || EPI == EPI_ROPE;
+    constexpr int LPR = PAIRS ? 8 : 16, RPI = 64 / LPR, R = 32 * MT / RPI;       // lanes on a row, rows an access covers, accesses
+    const int pr = lane / LPR, pc = lane % LPR;
+    auto at = [&](int e, int c) { return (f4*)(patch + (RPI * e + pr) * 256 + ((c + pc) ^ ((RPI * e + pr) & 15)) * 16); };
+    auto mrow = [&](int e) { return mrow0 + RPI * e + pr; };
+    auto row = [&](int e) { return mrow(e) < p.M ? mrow(e) : p.M - 1; };
+    const int n = EPI == EPI_SILU ? grp * 32 + pc * 4 : grp * 64 + pc * 4;
+    if (EPI != EPI_ROPE && n >= (EPI == EPI_SILU ? p.nfeat : p.N)) return;
+    if (EPI != EPI_ROPE && p.wscale) {
+#pragma unroll
+        for (int h = 0; h < (EPI == EPI_SILU ? 2 : 1); ++h) {
+            const int col = n + h * p.nfeat;
+            const f4 sv = *(const f4*)(p.wscale + col);
+            const bool corr = p.xscale && *p.corr_has;
+#pragma unroll 1
+            for (int e0 = 0; e0 < R; e0 += 4) {
+                f4 cv[4];
+                float xs[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    xs[e] = p.xscale ? p.xscale[row(e0 + e)] : 1.0f;
+                    cv[e] = corr ? *(const f4*)(p.corr + (int64_t)row(e0 + e) * p.ldc + col) : f4{0.f, 0.f, 0.f, 0.f};
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    f4 v = *at(e0 + e, 8 * h) * sv;
+                    if (p.xscale) v *= xs[e];
+                    if (corr) v += cv[e];
+                    *at(e0 + e, 8 * h) = v;
+                }
+            }
+        }
+    }
+    if constexpr (EPI == EPI_SILU || EPI == EPI_GELU) {
+#pragma unroll 1
+        for (int e0 = 0; e0 < R; e0 += 2)
+#pragma unroll
+            for (int e = e0; e < e0 + 2; ++e) {
+                const f4 v = *at(e, 0), u = EPI == EPI_SILU ? *at(e, 8) : v;
+                h4 hi, lo;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const float s = EPI == EPI_SILU ? (v[k] / (1.0f + __expf(-v[k]))) * u[k]                       // act_fn(gate) * up, llama2.py:242
+                                                    : 0.5f * v[k] * (1.0f + erff(v[k] * 0.70710678118654752f));   // nn.GELU(), falcon.py:726
+                    _Float16 sh, sl;
+                    pc_split(s, sh, sl);
+                    hi[k] = sh; lo[k] = sl;
+                }
+                if (mrow(e) < p.M) {
+                    *(h4*)(p.oh + (int64_t)mrow(e) * p.ldo + n) = hi;
+                    if (p.ol) *(h4*)(p.ol + (int64_t)mrow(e) * p.ldo + n) = lo;
+                }
+            }
+    } else if constexpr (EPI == EPI_ROPE) {
+        // RoPE at the supplied positions (llama2.py:200-213, :357-359) and the KV append (:361-364):
+        // 8 lanes per row, a lane holds features d0 .. d0+3 and d0+64 .. d0+67 of head `hd`
+        const int hd = grp >> 1, d0 = (grp & 1) * 32 + pc * 4;
+        if (hd >= p.H + 2 * p.Hkv) return;
+        const bool rot = hd < p.H + p.Hkv, is_q = hd < p.H;
+        const int kh = rot ? hd - p.H : hd - p.H - p.Hkv;
+#pragma unroll 1
+        for (int e0 = 0; e0 < R; e0 += 8) {
+            f4 w01[8], w23[8];
+            int64_t off[8], off_lo[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int m = row(e0 + e);
+                if (rot) {
+                    w01[e] = *(const f4*)(p.cs + (int64_t)m * 64 + d0);          // (cos, sin) of pairs d0, d0+1
+                    w23[e] = *(const f4*)(p.cs + (int64_t)m * 64 + d0 + 2);      // ... d0+2, d0+3
+                }
+                if (is_q) {
+                    off[e] = off_lo[e] = (int64_t)m * p.q_ts + hd * 128 + d0;
+                } else {
+                    const int b = m / p.q_len, t = m - b * p.q_len;
+                    const int past = p.past_lens ? p.past_lens[b] : p.past_len;
+                    off[e] = b * p.a_bs + kh * p.a_hs + (int64_t)(past + t) * 128 + d0;
+                    off_lo[e] = b * p.lo_bs + kh * p.lo_hs + (int64_t)(past + t - p.lo_row0) * 128 + d0;
+                }
+            }
+            _Float16* dh = is_q ? p.q_hi : rot ? p.k_arena : p.v_arena;
+            _Float16* dl = is_q ? p.q_lo : rot ? p.k_lo : p.v_lo;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const f4 x0 = *at(e0 + e, 0), x1 = *at(e0 + e, 8);
+                f4 a = x0, c = x1;
+                if (rot) {
+                    const float cs_[4] = {w01[e][0], w01[e][2], w23[e][0], w23[e][2]}, sn_[4] = {w01[e][1], w01[e][3], w23[e][1], w23[e][3]};
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        // q*cos + rotate_half(q)*sin (llama2.py:208): the low half pairs with -high, the high half with +low
+                        a[k] = x0[k] * cs_[k] - x1[k] * sn_[k];
+                        c[k] = x1[k] * cs_[k] + x0[k] * sn_[k];
+                    }
+                }
+                h4 ah, al, ch, cl;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    _Float16 t0, t1, t2, t3;
+                    pc_split(a[k], t0, t1);
+                    pc_split(c[k], t2, t3);
+                    ah[k] = t0; al[k] = t1; ch[k] = t2; cl[k] = t3;
+                }
+                if (mrow(e0 + e) >= p.M) continue;
+                *(h4*)(dh + off[e]) = ah;
+                *(h4*)(dh + off[e] + 64) = ch;
+                if (dl) { *(h4*)(dl + off_lo[e]) = al; *(h4*)(dl + off_lo[e] + 64) = cl; }
+            }
+        }
+    } else {
+        float* y = p.y + (int64_t)blockIdx.y * p.slab_stride + n;
+#pragma unroll 1
+        for (int e0 = 0; e0 < R; e0 += 16) {
+            f4 old[16];
+            if (EPI == EPI_ADD)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) old[e] = *(const f4*)(y + (int64_t)row(e0 + e) * p.ldy);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                f4 v = *at(e0 + e, 0);
+                if (EPI == EPI_ADD) v += old[e];
+                if (mrow(e0 + e) < p.M) *(f4*)(y + (int64_t)mrow(e0 + e) * p.ldy) = v;
+            }
+        }
+    }
+}
+
 // W: waves across and down a workgroup; TWO: both activation planes; NARROW: 128 columns instead of 256; TALL: 256 rows instead of 128
 template <int W, int EPI, bool TWO, bool NARROW, bool TALL>
 __global__ __launch_bounds__(256, 1) void gemm_dense_kernel(const DenseParams p) {
     static_assert(W == 2 && !(TWO && TALL), "four waves; two planes of 256 rows and their weights do not fit the LDS twice");
     using T = Tile<W, TWO, NARROW, TALL>;
     constexpr int MT = T::MT, NT = T::NT, S = T::S;
-    constexpr int PL = TWO ? 2 : 1, BM = T::BM, BN = T::BN, ROWS = PL * BM + BN;
-    constexpr int kStage = ROWS * 128;           // image: Xhi | Xlo | W, 128-byte rows
-    constexpr int NI = ROWS / 32;                // staging instructions per wave: 8 rows each
-    constexpr int NX = PL * BM / 32;             // ... of them for activations
-    __shared__ __attribute__((aligned(16))) char lds[S * kStage];
+    using L = mfma_tile::Loop<MT, NT, S, TWO ? 2 : 1>;
+    constexpr int PL = TWO ? 2 : 1, BM = L::BM, BN = L::BN;
+    constexpr int NI = L::NI, NX = PL * BM / 32;                 // staging instructions per wave, of them for activations
+    __shared__ __attribute__((aligned(16))) char lds[S * L::kStage];   // images: Xhi | Xlo | W
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -160,267 +287,58 @@ __global__ __launch_bounds__(256, 1) void gemm_dense_kernel(const DenseParams p)
             src[i] = p.w + (int64_t)(gr < 0 ? 0 : gr) * p.ldw + cx * 8;
         }
     }
-    // chunks past K: zero activations, paired with any finite weight bytes (the row's first chunk)
+    // (chunks past K: the row's first chunk of the K-step, whose products the main loop leaves out)
     const int last = (K - (nkt - 1) * BK) / 8;           // valid chunks of the product's last K-step (8: a whole one)
+    const int64_t past = cx < last ? 0 : -8 * cx;
     auto stage = [&](int i, int tl, char* buf) {
         const int t = t0 + tl;
-        const bool ok = cx < (t == nkt - 1 ? last : 8);
-        const _Float16* g = src[i] + (int64_t)t * BK;
-        if (!ok) g = i < NX ? p.zeros : src[i] - cx * 8;
-        glds16(g, buf + (4 * i + wave) * 1024);
+        glds16(src[i] + ((int64_t)t * BK + (t == nkt - 1 ? past : 0)), buf + (4 * i + wave) * 1024);
     };
-
-    // ---- fragment addressing: lane = (row fr of the 32-row subtile, k-half fh) ----
-    const int fr = lane & 31, fh = lane >> 5;
-    int foff[4];
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) foff[ks] = fr * 128 + (((2 * ks + fh) ^ ((fr >> 1) & 7)) << 4);
-    const int a_base = (wm * 32 * MT) * 128, b_base = (PL * BM + wn * 32 * NT) * 128;
+    const int keep = t0 + nk == nkt ? last : 8;          // chunks of this slice's last K-step
 
     f16v acc[MT][NT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    L::template run<h8>(acc, lds, nk, keep, lane, wm, wn,
+                        [](f16v& c, const h8& a, const h8& w) { c = __builtin_amdgcn_mfma_f32_32x32x16_f16(w, a, c, 0, 0, 0); }, stage);
 
-    // ---- main loop: one barrier per K-step, fragment reads one 16-deep slab ahead of the MFMAs ----
-    // Two fragment register sets alternate over the 4 slabs of a K-step.  The reads of slab s + 1 are issued between the MFMAs of slab
-    // s; the last slab of K-step t is multiplied AFTER the barrier, next to the first reads of K-step t + 1 and the first half of the
-    // LDS-DMA of K-step t + S (its buffer was just freed), whose second half goes out in the next step's first slab.
-    constexpr int R = PL * MT + NT, MF = PL * MT * NT, D0 = NI / 2;
-    struct Frags { h8 a[PL * MT], b[NT]; };
-    auto read_one = [&](Frags& f, const char* buf, int ks, int q) {
-        if (q < NT) {
-            f.b[q] = *(const h8*)(buf + b_base + q * 32 * 128 + foff[ks]);
-        } else {
-            const int pl = (q - NT) / MT, i = (q - NT) % MT;
-            f.a[q - NT] = *(const h8*)(buf + a_base + (pl * BM + i * 32) * 128 + foff[ks]);
-        }
-    };
-    auto mfma_one = [&](const Frags& f, int q) {
-        const int pl = q / (MT * NT), i = q / NT % MT, j = q % NT;
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.a[pl * MT + i], f.b[j], acc[i][j], 0, 0, 0);
-    };
-    // the reads that go behind MFMA k of a slab: one to every second MFMA where they fit, else two to each
-    auto reads_behind = [&](Frags& f, const char* buf, int ks, int k) {
-        if constexpr (MF >= 2 * R) {
-            if (k % 2 == 0 && k / 2 < R) read_one(f, buf, ks, k / 2);
-        } else {
-            if (2 * k < R) read_one(f, buf, ks, 2 * k);
-            if (2 * k + 1 < R) read_one(f, buf, ks, 2 * k + 1);
-        }
-    };
-    // (left alone, hipcc sinks the reads next to their first use and waits for them there)
-    auto slab = [&](const Frags& f, Frags& nx, const char* buf, int ks) {
-#pragma unroll
-        for (int q = 0; q < R; ++q) read_one(nx, buf, ks, q);
-#pragma unroll
-        for (int q = 0; q < MF; ++q) mfma_one(f, q);
-#pragma unroll
-        for (int k = 0; k < MF; ++k) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                              // one MFMA
-            if (MF >= 2 * R) {
-                if (k < R) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);               // one DS read
-            } else {
-                if (2 * k + 1 < R) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-                else if (2 * k < R) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            }
-        }
-    };
-    // a slab that also carries the staging instructions [d0, d1) of K-step tl
-    auto slab_staging = [&](const Frags& f, Frags& nx, const char* buf, int ks, int tl, char* to, int d0, int d1) {
-#pragma unroll
-        for (int k = 0; k < MF; ++k) {
-            mfma_one(f, k);
-            __builtin_amdgcn_sched_barrier(0);
-            reads_behind(nx, buf, ks, k);
-#pragma unroll
-            for (int i = 0; i < NI; ++i)
-                if (i >= d0 + k * (d1 - d0) / MF && i < d0 + (k + 1) * (d1 - d0) / MF) stage(i, tl, to);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-    auto clamp = [&](int t) { return t < nk ? t : nk - 1; };        // (past the end the last K-step goes into the idle buffer again)
-    Frags fa, fb;
-#pragma unroll
-    for (int st = 0; st < S - 1; ++st)
-#pragma unroll
-        for (int i = 0; i < NI; ++i) stage(i, clamp(st), lds + st * kStage);
-#pragma unroll
-    for (int i = 0; i < D0; ++i) stage(i, clamp(S - 1), lds + (S - 1) * kStage);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * NI + D0) : "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-#pragma unroll
-    for (int q = 0; q < R; ++q) read_one(fa, lds, 0, q);
-    int cur = 0, prev = (S - 1) * kStage;                            // images of K-steps t and t + S - 1
-    for (int t = 0; t + 1 < nk; ++t) {
-        slab_staging(fa, fb, lds + cur, 1, clamp(t + S - 1), lds + prev, D0, NI);
-        slab(fb, fa, lds + cur, 2);
-        slab(fa, fb, lds + cur, 3);
-        // K-step t + 1 has landed (S - 2 younger ones may be in flight), for everyone behind the barrier; every wave's reads of K-step t are complete
-        __builtin_amdgcn_sched_barrier(0);
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * NI) : "memory");
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-        prev = cur;
-        cur = cur + kStage == S * kStage ? 0 : cur + kStage;
-        slab_staging(fb, fa, lds + cur, 0, clamp(t + S), lds + prev, 0, D0);
-    }
-    slab(fa, fb, lds + cur, 1);
-    slab(fb, fa, lds + cur, 2);
-    slab(fa, fb, lds + cur, 3);
-#pragma unroll
-    for (int q = 0; q < MF; ++q) mfma_one(fb, q);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // (clamped re-loads of the last K-step)
-
-    // ---- epilogue: accumulators -> wave-private LDS tile [32 MT][64] fp32, one 64-column group at a time -> full-row global stores ----
+    // ---- epilogue: 64 accumulator columns of a wave at a time through an LDS patch of its own -> full-row global stores ----
+    // (the weights are the products' first operand: a lane holds row lane & 31 and the column quads 8 q + 4 (lane >> 5) of a 32 x 32 block;
+    // patch: [32 MT][64] fp32, 16-byte quad c of row r at c ^ (r & 15))
     __syncthreads();                                       // every wave is done with the staging buffers
-    float* st = (float*)(lds + wave * (32 * MT * 64 * 4));
-    const int mrow0 = m0 + wm * 32 * MT;
+    constexpr int P = 32 * MT * 256, PARTS = NT / 2, ROOM = 4 * P * PARTS <= S * L::kStage ? PARTS : 1;   // patches that fit at a time
+    char* patch = lds + wave * (P * ROOM);
+    const int fr = lane & 31, fh = lane >> 5;
+    auto fence = [] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    auto put = [&](auto part, char* to) {
+        constexpr int j = decltype(part)::value;
 #pragma unroll
-    for (int half = 0; half < NT / 2; ++half) {
-    const int grp = wn * (NT / 2) + half;                  // the 64-column group inside the block tile
+        for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+            for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                st[(32 * i + 8 * (r >> 2) + 4 * fh + (r & 3)) * 64 + 32 * j + fr] = acc[i][2 * half + j][r];
-    if (EPI == EPI_SILU) {
-        // the wave's 64 columns are [32 gate features | the same 32 up features]: 8 lanes per row, 4 features per lane
-        const int fbase = (ni * NT + grp) * 32 + (lane & 7) * 4;
-#pragma unroll
-        for (int it = 0; it < 4 * MT; ++it) {
-            const int row = it * 8 + (lane >> 3), m = mrow0 + row;
-            f4 g = *(const f4*)(st + row * 64 + (lane & 7) * 4);
-            f4 u = *(const f4*)(st + row * 64 + 32 + (lane & 7) * 4);
-            if (m < p.M && fbase < p.nfeat) {
-                if (p.wscale) {
-                    const f4 sg = *(const f4*)(p.wscale + fbase), su = *(const f4*)(p.wscale + p.nfeat + fbase);
-                    g[0] *= sg[0]; g[1] *= sg[1]; g[2] *= sg[2]; g[3] *= sg[3];
-                    u[0] *= su[0]; u[1] *= su[1]; u[2] *= su[2]; u[3] *= su[3];
+                for (int q = 0; q < 4; ++q) {
+                    const f16v& c = acc[i][2 * j + h];
+                    *(f4*)(to + (32 * i + fr) * 256 + ((8 * h + 2 * q + fh) ^ (fr & 15)) * 16) = f4{c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]};
                 }
-                if (p.xscale) {
-                    const float xs = p.xscale[m];
-                    g[0] *= xs; g[1] *= xs; g[2] *= xs; g[3] *= xs;
-                    u[0] *= xs; u[1] *= xs; u[2] *= xs; u[3] *= xs;
-                    if (*p.corr_has) {
-                        const f4 cg = *(const f4*)(p.corr + (int64_t)m * p.ldc + fbase);
-                        const f4 cu = *(const f4*)(p.corr + (int64_t)m * p.ldc + p.nfeat + fbase);
-                        g[0] += cg[0]; g[1] += cg[1]; g[2] += cg[2]; g[3] += cg[3];
-                        u[0] += cu[0]; u[1] += cu[1]; u[2] += cu[2]; u[3] += cu[3];
-                    }
-                }
-                h4 hi, lo;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float s = (g[e] / (1.0f + __expf(-g[e]))) * u[e];      // act_fn(gate) * up, llama2.py:242
-                    _Float16 sh, sl;
-                    pc_split(s, sh, sl);
-                    hi[e] = sh; lo[e] = sl;
-                }
-                *(h4*)(p.oh + (int64_t)m * p.ldo + fbase) = hi;
-                if (p.ol) *(h4*)(p.ol + (int64_t)m * p.ldo + fbase) = lo;
-            }
-        }
-        continue;
-    }
-    if (EPI == EPI_ROPE) {
-        // RoPE at the supplied positions (llama2.py:200-213, :357-359) and the KV append (:361-364) on the accumulator tile:
-        // 8 lanes per row, a lane holds features d0 .. d0+3 and d0+64 .. d0+67 of head `hd`
-        const int hd = ni * (BN / 128) + (grp >> 1);
-        const int d0 = (grp & 1) * 32 + (lane & 7) * 4;
-        if (hd >= p.H + 2 * p.Hkv) continue;
-        const bool rot = hd < p.H + p.Hkv;
-#pragma unroll
-        for (int it = 0; it < 4 * MT; ++it) {
-            const int row = it * 8 + (lane >> 3), m = mrow0 + row;
-            const f4 x0 = *(const f4*)(st + row * 64 + (lane & 7) * 4);
-            const f4 x1 = *(const f4*)(st + row * 64 + 32 + (lane & 7) * 4);
-            if (m >= p.M) continue;
-            f4 a = x0, c = x1;
-            if (rot) {
-                const f4 w01 = *(const f4*)(p.cs + (int64_t)m * 64 + d0);          // (cos, sin) of pairs d0, d0+1
-                const f4 w23 = *(const f4*)(p.cs + (int64_t)m * 64 + d0 + 2);      // ... d0+2, d0+3
-                const float cs_[4] = {w01[0], w01[2], w23[0], w23[2]}, sn_[4] = {w01[1], w01[3], w23[1], w23[3]};
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    // q*cos + rotate_half(q)*sin (llama2.py:208): the low half pairs with -high, the high half with +low
-                    a[e] = x0[e] * cs_[e] - x1[e] * sn_[e];
-                    c[e] = x1[e] * cs_[e] + x0[e] * sn_[e];
-                }
-            }
-            h4 ah, al, ch, cl;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                _Float16 t0, t1, t2, t3;
-                pc_split(a[e], t0, t1);
-                pc_split(c[e], t2, t3);
-                ah[e] = t0; al[e] = t1; ch[e] = t2; cl[e] = t3;
-            }
-            _Float16* dh;
-            _Float16* dl = nullptr;
-            if (hd < p.H) {
-                const int64_t off = (int64_t)m * p.q_ts + hd * 128 + d0;
-                dh = p.q_hi + off;
-                if (p.q_lo) dl = p.q_lo + off;
-            } else {
-                const int b = m / p.q_len, t = m - b * p.q_len;
-                const int past = p.past_lens ? p.past_lens[b] : p.past_len;
-                const bool is_k = hd < p.H + p.Hkv;
-                const int kh = is_k ? hd - p.H : hd - p.H - p.Hkv;
-                dh = (is_k ? p.k_arena : p.v_arena) + b * p.a_bs + kh * p.a_hs + (int64_t)(past + t) * 128 + d0;
-                if (p.k_lo) dl = (is_k ? p.k_lo : p.v_lo) + b * p.lo_bs + kh * p.lo_hs + (int64_t)(past + t - p.lo_row0) * 128 + d0;
-            }
-            *(h4*)dh = ah;
-            *(h4*)(dh + 64) = ch;
-            if (dl) { *(h4*)dl = al; *(h4*)(dl + 64) = cl; }
-        }
-        continue;
-    }
-    const int n = ni * BN + grp * 64 + (lane & 15) * 4;
-#pragma unroll
-    for (int it = 0; it < 8 * MT; ++it) {
-        const int row = it * 4 + (lane >> 4), m = mrow0 + row;
-        f4 v = *(const f4*)(st + row * 64 + (lane & 15) * 4);
-        if (m < p.M && n < p.N) {
-            if (p.wscale) {
-                const f4 sv = *(const f4*)(p.wscale + n);
-                v[0] *= sv[0]; v[1] *= sv[1]; v[2] *= sv[2]; v[3] *= sv[3];
-            }
-            if (p.xscale) {
-                const float xs = p.xscale[m];
-                v[0] *= xs; v[1] *= xs; v[2] *= xs; v[3] *= xs;
-                if (*p.corr_has) {
-                    const f4 cv = *(const f4*)(p.corr + (int64_t)m * p.ldc + n);
-                    v[0] += cv[0]; v[1] += cv[1]; v[2] += cv[2]; v[3] += cv[3];
-                }
-            }
-            if (EPI == EPI_GELU) {
-                h4 hi, lo;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float s = 0.5f * v[e] * (1.0f + erff(v[e] * 0.70710678118654752f));   // nn.GELU(), falcon.py:726
-                    _Float16 sh, sl;
-                    pc_split(s, sh, sl);
-                    hi[e] = sh; lo[e] = sl;
-                }
-                *(h4*)(p.oh + (int64_t)m * p.ldo + n) = hi;
-                if (p.ol) *(h4*)(p.ol + (int64_t)m * p.ldo + n) = lo;
-            } else {
-                float* yp = p.y + (int64_t)blockIdx.y * p.slab_stride + (int64_t)m * p.ldy + n;
-                if (EPI == EPI_ADD) {
-                    const f4 old = *(const f4*)yp;
-                    v[0] += old[0]; v[1] += old[1]; v[2] += old[2]; v[3] += old[3];
-                }
-                *(f4*)yp = v;
-            }
-        }
-    }
+    };
+    using First = std::integral_constant<int, 0>;
+    using Second = std::integral_constant<int, PARTS - 1>;
+    const int grp = ni * (BN / 64) + wn * PARTS;           // the wave's first 64-column group
+    put(First{}, patch);
+    if constexpr (ROOM == PARTS) {
+        if constexpr (PARTS == 2) put(Second{}, patch + P);
+        fence();
+#pragma unroll 1
+        for (int j = 0; j < PARTS; ++j) store_group<EPI, MT>(p, patch + j * P, lane, grp + j, m0 + wm * 32 * MT);
+    } else {
+        fence();
+        store_group<EPI, MT>(p, patch, lane, grp, m0 + wm * 32 * MT);
+        fence();
+        put(Second{}, patch);
+        fence();
+        store_group<EPI, MT>(p, patch, lane, grp + 1, m0 + wm * 32 * MT);
     }
 }
 
@@ -446,7 +364,7 @@ __global__ __launch_bounds__(256) void dense_reduce_kernel(const float* __restri
     *(f4*)yp = v;
 }
 
-// 16 bytes of zeros for activation chunks past K (device constant: no allocation, graph-capturable)
+// 16 bytes of zeros (DenseParams::zeros; device constant: no allocation, graph-capturable)
 __device__ __attribute__((aligned(16))) _Float16 g_zero_chunk[8];
 
 template <int EPI, bool TWO, bool NARROW, bool TALL>
@@ -456,13 +374,8 @@ int launch_dense_as(DenseParams& p, hipStream_t s, int kslices) {
     p.nb = (EPI == EPI_SILU) ? pc_ceil_div(p.nfeat, BN / 2) : pc_ceil_div(p.N, BN);
     const int nkt = pc_ceil_div(p.K, BK);
     p.kper = pc_ceil_div(nkt, kslices);
-    // strips: fewest rounds of an XCD's 32 CUs, then fewest rows (activations of mh M-blocks, weights of the panels 32 tiles reach) per K-step
-    int64_t best = -1;
-    for (int px = 1; px <= 8; px *= 2) {
-        const int mh = pc_ceil_div(p.mb, px), nh = pc_ceil_div(p.nb, 8 / px), reach = mh < 32 ? mh : 32;
-        const int64_t cost = ((int64_t)pc_ceil_div(mh * nh, 32) << 32) + reach * (TWO ? 2 : 1) * BM + pc_ceil_div(32, reach) * BN;
-        if (best < 0 || cost < best) { best = cost; p.px = px; p.mh = mh; p.nh = nh; }
-    }
+    const mfma_tile::Strips g = mfma_tile::strips(p.mb, p.nb, (TWO ? 2 : 1) * BM, BN);
+    p.px = g.px; p.mh = g.mh; p.nh = g.nh;
     hipLaunchKernelGGL((gemm_dense_kernel<2, EPI, TWO, NARROW, TALL>), dim3(8 * p.mh * p.nh, pc_ceil_div(nkt, p.kper)), dim3(256), 0, s, p);
     return pc_check_launch("gemm_dense_kernel");
 }
@@ -633,7 +546,7 @@ PC_EXPORT int pc_gemm_dense_lo8(const void* x_hi, int64_t ldx, const void* x_lo8
 
 // The fused q|k|v projection of a many-row pass at head_dim 128 (include/promptcache_hip.h: pc_dense_qkv_args): projection,
 // RoPE at the supplied positions, rotated q as hi / lo planes, rotated k and v appended to the arena (+ residual planes) -- the
-// [M][(H + 2 Hkv) D] fp32 intermediate and the separate pc_rope_append launch of the round-2 encode are gone.
+// [M][(H + 2 Hkv) D] fp32 intermediate and a separate pc_rope_append launch are not needed.
 PC_EXPORT int pc_gemm_dense_qkv_rope(const pc_dense_qkv_args* a, void* stream) {
     PC_REQUIRE(a && a->struct_bytes == (uint32_t)sizeof(pc_dense_qkv_args), PC_ERR_ARG,
                "pc_gemm_dense_qkv_rope: args is NULL or struct_bytes != sizeof(pc_dense_qkv_args) (ABI mismatch)");
