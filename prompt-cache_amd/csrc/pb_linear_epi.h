@@ -1,0 +1,78 @@
+// What pb_linear's kernels do with finished sums (pb_linear.hip, pb_linear_tiles.hip): bias, activation, gated unit, where each element goes.
+#pragma once
+#include "pb_common.h"
+
+namespace pcb {
+
+__device__ __forceinline__ float apply_act(int act, float v, float param) {
+    switch (act) {
+        case PCB_ACT_SILU: return v / (1.0f + expf(-v));
+        case PCB_ACT_SIGMOID: return 1.0f / (1.0f + expf(-v));
+        case PCB_ACT_RELU2: return v > 0.0f ? v * v : 0.0f;
+        case PCB_ACT_SOFTPLUS: return v > 20.0f ? v : log1pf(expf(v));
+        case PCB_ACT_SOFTCAP: return param * tanhf(v / param);
+        case PCB_ACT_RELU: return v > 0.0f ? v : 0.0f;
+        case PCB_ACT_GELU_TANH: return 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)));
+        case PCB_ACT_LOGSIGMOID: return param * (fminf(v, 0.0f) - log1pf(expf(-fabsf(v))));
+        case PCB_ACT_SCALE: return param * v;
+        default: return v;
+    }
+}
+
+// the gated epilogue's function: silu (the default), relu or the tanh-form gelu, which is z sigmoid(2 u) for tanh's argument u.  Kept short:
+// an epilogue too long to unroll would index the accumulators, which throws them out of the registers.
+__device__ __forceinline__ float gate_act(int act, float v) {
+    const float t = act == PCB_ACT_GELU_TANH ? 1.5957691216057308f * (v + 0.044715f * v * v * v) : v;
+    const float s = v / (1.0f + expf(-t));
+    return act == PCB_ACT_RELU ? fmaxf(v, 0.0f) : s;
+}
+
+// where one finished element goes (see pcb_linear_args)
+template <typename E, int EPI>
+__device__ __forceinline__ void put(const pcb_linear_args& a, int m, int n, float v, float cs) {
+    if (EPI == PCB_EPI_SCALE_ADD) {
+        float* y = (float*)a.y + (int64_t)m * a.ldy + n;
+        const float b0 = a.base ? a.base[(int64_t)m * a.ldbase + n] : *y;
+        *y = b0 + cs * v;
+        return;
+    }
+    if (a.split_n3 > 0 && n >= a.split_n3) {
+        ((E*)a.y3)[a.row_off3[m] + (int64_t)(n - a.split_n3) * a.col_stride3] = from_f32<E>(v);
+        return;
+    }
+    if (a.split_n > 0 && n >= a.split_n) {
+        const int c = n - a.split_n;
+        if (a.y2_f32) {
+            ((float*)a.y2)[m * a.head_stride2 + c] = v;
+            return;
+        }
+        E* y = (E*)a.y2 + a.row_off2[m] + (int64_t)(c / a.head_dim2) * a.head_stride2 + c % a.head_dim2;
+        *y = from_f32<E>(v);
+        return;
+    }
+    const int64_t at = (int64_t)(a.row_dst ? a.row_dst[m] : m) * a.ldy + n + (a.n_batch > 0 ? (int64_t)blockIdx.z * a.y_batch_stride : 0);
+    if (a.out_f32)
+        ((float*)a.y)[at] = v;
+    else
+        ((E*)a.y)[at] = from_f32<E>(v);
+}
+
+// columns that pass through act / act2 of a plain store: the split-off parts are stored as they are
+__device__ __forceinline__ int act_end(const pcb_linear_args& a) {
+    return a.split_n > 0 ? a.split_n : (a.split_n3 > 0 ? a.split_n3 : a.N);
+}
+
+// one result element through the epilogue
+template <typename E, int EPI>
+__device__ __forceinline__ void emit(const pcb_linear_args& a, int m, int n, float acc, float acc2, float bv, float cs, float bv2 = 0.0f) {
+    float v = acc + bv;
+    if (EPI == PCB_EPI_STORE && (a.act | a.act2) && n < act_end(a))
+        v = apply_act((a.act_split > 0 && n >= a.act_split) ? a.act2 : a.act, v, a.act_param);
+    if (EPI == PCB_EPI_SILU_MUL) {
+        v = gate_act(a.act, v) * (acc2 + bv2);
+        if (a.row_gate) v *= to_f32(((const E*)a.row_gate)[m * a.ld_row_gate]);
+    }
+    put<E, EPI>(a, m, n, v, cs);
+}
+
+}  // namespace pcb

@@ -1,0 +1,357 @@
+// pb_linear over many rows in bf16: mfma_f32_32x32x16_bf16, four waves (2 x 2) in tiles of 128 x 128, 128 x 256 or 256 x 256 with a whole CU's
+// LDS for their ring, main loop and staging order in mfma_tile_loop.h.
+//
+// What bounds it: at one round of 128 x 128 tiles LDS bandwidth (a wave of 64 x 64 reads as many bytes as its MFMAs take cycles) and the
+// barrier of every K-step, at the larger tiles power.  Against linear_dma_kernel (pb_linear.hip: 16 x 16 MFMAs, two or three images, two
+// workgroups to a CU), us, 2048 rows: 2048 x 2048 29.9 -> 19.9 (0.87 PFLOP/s), K = 8192 93.5 -> 72, 2560 columns 39.8 -> 31, 8192 columns
+// 90.5 -> 65.6 (1.05 PFLOP/s; the gated pair 79.3 -> 60.7), 10272 columns 109 -> 97; 4096 x 4096 x 4096 161 -> 112 (1.23 PFLOP/s).
+#include "mfma_tile_loop.h"
+#include "pb_linear_epi.h"
+#include "pb_linear_tiles.h"
+
+namespace {
+using namespace pcb;
+
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef float f16v __attribute__((ext_vector_type(16)));
+
+struct Grid { int mb, nb, px, mh, nh; };
+
+// The wave's sums in `patch` to where they go: quad pc of rows pr, pr + RPI .. (R of them, RPI = 64 / LPR), row pr = row m0 of the result,
+// columns n .. n + 3 (n0: the wave's first).  First the patch is turned into results in place, then stored.  Short loops on purpose, and no
+// load behind a store:
+// - code that runs once comes in at about 2 bytes per ns (instruction misses): a 256 x 256 tile whose epilogue was unrolled took 20 us
+//   longer than its products;
+// - stores and loads count on one counter, so a wait for a load behind a store waits for the store's way to memory and back (2.4 us).
+template <int EPI, int R>
+__device__ __forceinline__ void store_columns(const pcb_linear_args& a, char* patch, int pr, int pc, int n0, int n, int m0) {
+    typedef bf16_t E;
+    constexpr bool TWO = EPI == PCB_EPI_SILU_MUL;
+    constexpr int LPR = TWO ? 8 : 16, RPI = 64 / LPR;
+    const int M = a.M, N = a.N, whole = act_end(a);                  // columns below `whole` go to y
+    auto at = [&](int e, int c) { return (f4*)(patch + (RPI * e + pr) * 256 + ((c + pc) ^ ((RPI * e + pr) & 15)) * 16); };
+    auto row = [&](int e) { const int m = m0 + RPI * e; return m < M ? m : M - 1; };
+    auto four = [&](const E* p) {
+        f4 b = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (p && n + k < N) b[k] = to_f32(p[n + k]);
+        return b;
+    };
+    const int esz = (EPI == PCB_EPI_SCALE_ADD || a.out_f32) ? 4 : 2;
+    const bool quad = a.ldy % 4 == 0 && (uintptr_t)a.y % (4 * esz) == 0 && n + 4 <= whole &&
+                      (EPI != PCB_EPI_SCALE_ADD || !a.base || (a.ldbase % 4 == 0 && (uintptr_t)a.base % 16 == 0));
+    if (EPI == PCB_EPI_STORE && (a.bias || (a.act | a.act2))) {
+        const int mid = a.act_split > 0 && a.act_split < whole ? a.act_split : whole;
+        f4 bv = four((const E*)a.bias);
+        auto run = [&](auto code, int lo, int hi) {
+#pragma unroll 1
+            for (int e0 = 0; e0 < R; e0 += 4) {
+                f4 v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = *at(e0 + e, 0) + bv;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (n + k >= lo && n + k < hi) v[e][k] = apply_act(decltype(code)::value, v[e][k], a.act_param);
+                    *at(e0 + e, 0) = v[e];
+                }
+            }
+            bv = f4{0.f, 0.f, 0.f, 0.f};
+        };
+        bool added = !a.bias;
+#pragma unroll 1
+        for (int part = 0; part < 2; ++part) {
+            const int act = part ? a.act2 : a.act, lo = part ? mid : 0, hi = part ? whole : mid;
+            if (n0 >= hi || n0 + 4 * LPR <= lo || act == PCB_ACT_NONE) continue;
+            added = true;
+            switch (act) {
+                case PCB_ACT_SILU: run(std::integral_constant<int, PCB_ACT_SILU>{}, lo, hi); break;
+                case PCB_ACT_SIGMOID: run(std::integral_constant<int, PCB_ACT_SIGMOID>{}, lo, hi); break;
+                case PCB_ACT_RELU2: run(std::integral_constant<int, PCB_ACT_RELU2>{}, lo, hi); break;
+                case PCB_ACT_SOFTPLUS: run(std::integral_constant<int, PCB_ACT_SOFTPLUS>{}, lo, hi); break;
+                case PCB_ACT_SOFTCAP: run(std::integral_constant<int, PCB_ACT_SOFTCAP>{}, lo, hi); break;
+                case PCB_ACT_RELU: run(std::integral_constant<int, PCB_ACT_RELU>{}, lo, hi); break;
+                case PCB_ACT_GELU_TANH: run(std::integral_constant<int, PCB_ACT_GELU_TANH>{}, lo, hi); break;
+                case PCB_ACT_LOGSIGMOID: run(std::integral_constant<int, PCB_ACT_LOGSIGMOID>{}, lo, hi); break;
+                default: run(std::integral_constant<int, PCB_ACT_SCALE>{}, lo, hi);
+            }
+        }
+        if (!added) run(std::integral_constant<int, PCB_ACT_NONE>{}, 0, 0);
+    }
+    if (EPI == PCB_EPI_SILU_MUL) {
+        const f4 bv = four((const E*)a.bias), bv2 = four((const E*)a.bias2);
+        auto gate = [&](auto code) {
+#pragma unroll 1
+            for (int e0 = 0; e0 < R; e0 += 4) {
+                f4 v[4], u[4];
+                float rg[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    v[e] = *at(e0 + e, 0) + bv;
+                    u[e] = *at(e0 + e, 8) + bv2;
+                    rg[e] = a.row_gate ? to_f32(((const E*)a.row_gate)[row(e0 + e) * a.ld_row_gate]) : 1.0f;
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) v[e][k] = gate_act(decltype(code)::value, v[e][k]) * u[e][k] * rg[e];
+                    *at(e0 + e, 0) = v[e];
+                }
+            }
+        };
+        if (a.act == PCB_ACT_RELU)
+            gate(std::integral_constant<int, PCB_ACT_RELU>{});
+        else if (a.act == PCB_ACT_GELU_TANH)
+            gate(std::integral_constant<int, PCB_ACT_GELU_TANH>{});
+        else
+            gate(std::integral_constant<int, PCB_ACT_SILU>{});
+    }
+    if (EPI == PCB_EPI_SCALE_ADD) {
+        const float* from = a.base ? a.base : (const float*)a.y;
+        const int64_t ld = a.base ? a.ldbase : a.ldy;
+        const f4 bv = four((const E*)a.bias);
+        f4 cs = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (n + k < N) cs[k] = a.col_scale[n + k];
+        if (quad) {
+#pragma unroll
+            for (int e0 = 0; e0 < R; e0 += 16) {                     // (16 rows' residuals in one wait; R is 16 or 32)
+                f4 b0[16];
+#pragma unroll
+                for (int e = 0; e < 16; ++e) b0[e] = *(const f4*)(from + row(e0 + e) * ld + n);
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    if (m0 + RPI * (e0 + e) < M)
+                        *(f4*)((float*)a.y + (int64_t)(m0 + RPI * (e0 + e)) * a.ldy + n) = b0[e] + cs * (*at(e0 + e, 0) + bv);
+            }
+            return;
+        }
+#pragma unroll 1
+        for (int k = 0; k < 4 && n + k < N; ++k)
+#pragma unroll 1
+            for (int e0 = 0; e0 < R; e0 += 8) {
+                float b0[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) b0[e] = from[row(e0 + e) * ld + n + k];
+                const float ck = a.col_scale[n + k], bk = a.bias ? to_f32(((const E*)a.bias)[n + k]) : 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    float* p = (float*)at(e0 + e, 0) + k;
+                    *p = b0[e] + ck * (*p + bk);
+                }
+            }
+    }
+    auto pack = [](const f4& r) { return uint2{bf16_pair(r[0], r[1]), bf16_pair(r[2], r[3])}; };
+    if (quad && !a.row_dst) {
+        char* y = (char*)a.y + ((int64_t)m0 * a.ldy + n) * esz;
+        const int64_t step = (int64_t)RPI * a.ldy * esz;
+#pragma unroll 1
+        for (int e0 = 0; e0 < R; e0 += 4) {
+            f4 v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = *at(e0 + e, 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e, y += step) {
+                if (m0 + RPI * (e0 + e) >= M) continue;
+                if (esz == 4)
+                    *(f4*)y = v[e];
+                else
+                    *(uint2*)y = pack(v[e]);
+            }
+        }
+        return;
+    }
+    // whole quads in rows of their own: row_dst, the fp32 rows or the heads that split_n begins
+    const bool split = EPI == PCB_EPI_STORE && a.split_n > 0 && n >= a.split_n && n + 4 <= (a.split_n3 > 0 ? a.split_n3 : N) && a.split_n % 4 == 0 &&
+                       a.head_stride2 % 4 == 0 && (a.y2_f32 ? (uintptr_t)a.y2 % 16 == 0 : a.head_dim2 % 4 == 0 && (uintptr_t)a.y2 % 8 == 0);
+    const int c = n - a.split_n;
+    if (quad || split) {
+        const bool wide = split ? a.y2_f32 : esz == 4;
+        const int size = wide ? 4 : 2;
+        char* y = split ? (char*)a.y2 + (a.y2_f32 ? c : (int64_t)(c / a.head_dim2) * a.head_stride2 + c % a.head_dim2) * size : (char*)a.y + (int64_t)n * size;
+#pragma unroll 1
+        for (int e0 = 0; e0 < R; e0 += 8) {
+            int64_t off[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int m = row(e0 + e);
+                off[e] = !split ? a.row_dst[m] * a.ldy : a.y2_f32 ? m * a.head_stride2 : a.row_off2[m];
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                if (m0 + RPI * (e0 + e) >= M) continue;
+                const f4 v = *at(e0 + e, 0);
+                char* p = y + off[e] * size;
+                if (wide) {
+                    *(f4*)p = v;
+                } else if (off[e] % 4 == 0) {
+                    *(uint2*)p = pack(v);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) ((E*)p)[k] = from_f32<E>(v[k]);
+                }
+            }
+        }
+        return;
+    }
+    // element by element: edges, unaligned rows, splits inside a quad, the column-wise destination
+#pragma unroll 1
+    for (int nk = n; nk < n + 4 && nk < N; ++nk) {
+        const bool third = EPI == PCB_EPI_STORE && a.split_n3 > 0 && nk >= a.split_n3;
+        const bool second = EPI == PCB_EPI_STORE && !third && a.split_n > 0 && nk >= a.split_n;
+        const int d = nk - a.split_n;
+        const int64_t col = third ? (int64_t)(nk - a.split_n3) * a.col_stride3
+                            : !second ? nk
+                            : a.y2_f32 ? d
+                                       : (int64_t)(d / a.head_dim2) * a.head_stride2 + d % a.head_dim2;
+        const bool wide = second ? a.y2_f32 : !third && esz == 4;
+        char* y = (char*)(third ? a.y3 : second ? a.y2 : a.y);
+#pragma unroll 1
+        for (int e0 = 0; e0 < R; e0 += 8) {
+            int64_t off[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int m = row(e0 + e);
+                off[e] = col + (third    ? a.row_off3[m]
+                                : second ? a.y2_f32 ? m * a.head_stride2 : a.row_off2[m]
+                                         : (EPI != PCB_EPI_SCALE_ADD && a.row_dst ? a.row_dst[m] : m) * a.ldy);
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                if (m0 + RPI * (e0 + e) >= M) continue;
+                const float r = ((const float*)at(e0 + e, 0))[nk - n];
+                if (wide)
+                    ((float*)y)[off[e]] = r;
+                else
+                    ((E*)y)[off[e]] = from_f32<E>(r);
+            }
+        }
+    }
+}
+
+template <int EPI, int MT, int NT, int S>
+__global__ __launch_bounds__(256, 1) void linear_tile_kernel(const pcb_linear_args a, const Grid g) {
+    typedef bf16_t E;
+    constexpr bool TWO = EPI == PCB_EPI_SILU_MUL;
+    using L = mfma_tile::Loop<MT, NT, S, 1>;
+    constexpr int BM = L::BM, BN = TWO ? L::BN / 2 : L::BN, NI = L::NI;   // BN: result columns
+    __shared__ __attribute__((aligned(16))) char lds[S * L::kStage];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int mi = xcd % g.px * g.mh + slot % g.mh, ni = xcd / g.px * g.nh + slot / g.mh;
+    if (mi >= g.mb || ni >= g.nb) return;
+    const int m_lo = mi * BM, n_lo = ni * BN, K = a.K, N = a.N, nk = (K + 63) / 64;
+
+    // staging: a lane's 16-byte chunk of an instruction's row as a 32-bit offset from the operand's K-step (the address is otherwise uniform)
+    const int srow = 8 * wave + (lane >> 3), cx = (lane & 7) ^ ((srow >> 1) & 7);
+    const int last = (K - (nk - 1) * 64) / 8;                        // chunks of the last K-step (8: a whole one)
+    const E* base[3] = {(const E*)a.x + (int64_t)m_lo * a.ldx, (const E*)a.w + (int64_t)n_lo * a.ldw,
+                        TWO ? (const E*)a.w2 + (int64_t)n_lo * a.ldw : nullptr};
+    uint32_t off[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int r = 32 * i + srow;
+        if (32 * i < BM) {
+            off[i] = (uint32_t)((m_lo + r < a.M ? r : a.M - 1 - m_lo) * (int)a.ldx + cx * 8) * 2u;
+        } else {
+            // (gated: the first half of a wave's columns is W's rows, the second the matching rows of W2)
+            const int c = r - BM, n = TWO ? c / (32 * NT) * 16 * NT + c % (16 * NT) : c;
+            off[i] = (uint32_t)((n_lo + n < N ? n : N - 1 - n_lo) * (int)a.ldw + cx * 8) * 2u;
+        }
+    }
+    // (chunks past K: the row's first of the K-step again, whose products Loop leaves out)
+    const uint32_t past = cx < last ? 0u : (uint32_t)(-16 * cx);
+    auto stage = [&](int i, int t, char* buf) {
+        const int which = 32 * i < BM ? 0 : TWO && (32 * i - BM) / (16 * NT) % 2 ? 2 : 1;
+        const char* s = (const char*)(base[which] + (int64_t)t * 64);
+        const uint32_t o = off[i] + (t == nk - 1 ? past : 0u);
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(s + o),
+                                         (__attribute__((address_space(3))) void*)(buf + (4 * i + wave) * 1024), 16, 0, 0);
+    };
+    f16v acc[MT][NT];
+    // (the weights are the products' first operand: a lane ends up with row lane & 31 and columns 8 q + 4 (lane >> 5) .. + 3 of a block)
+    L::template run<b8>(acc, lds, nk, last, lane, wm, wn,
+                        [](f16v& c, const b8& x, const b8& w) { c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, x, c, 0, 0, 0); }, stage);
+
+    // Results: 64 accumulator columns of a wave go into an LDS patch of its own (16-byte quad c of row r at c ^ (r & 15)), so that neighbouring
+    // lanes store neighbouring columns.  Gated: 32 gate columns and the matching 32 of the other half side by side.
+    __syncthreads();                                                 // (the images are read out)
+    constexpr int P = 32 * MT * 256, PARTS = NT / 2, ROOM = 4 * P * PARTS <= S * L::kStage ? PARTS : 1;   // patches that fit at a time
+    char* patch = lds + wave * (P * ROOM);
+    constexpr int LPR = TWO ? 8 : 16, RPI = 64 / LPR;                // lanes on a row, rows an access covers
+    const int fr = lane & 31, fh = lane >> 5, pr = lane / LPR, pc = lane % LPR;
+    auto fence = [] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    auto put = [&](auto part, char* to) {
+        constexpr int j = decltype(part)::value;
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const f16v& c = acc[i][TWO ? j + h * (NT / 2) : 2 * j + h];
+                    *(f4*)(to + (32 * i + fr) * 256 + ((8 * h + 2 * q + fh) ^ (fr & 15)) * 16) = f4{c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]};
+                }
+    };
+    auto store = [&](int j, char* from) {
+        const int n0 = n_lo + (TWO ? wn * 16 * NT + 32 * j : wn * 32 * NT + 64 * j);
+        if (n0 < N) store_columns<EPI, 32 * MT / RPI>(a, from, pr, pc, n0, n0 + 4 * pc, m_lo + wm * 32 * MT + pr);
+    };
+    using First = std::integral_constant<int, 0>;
+    using Second = std::integral_constant<int, PARTS - 1>;
+    put(First{}, patch);
+    if constexpr (ROOM == PARTS) {
+        if constexpr (PARTS == 2) put(Second{}, patch + P);
+        fence();
+#pragma unroll 1
+        for (int j = 0; j < PARTS; ++j) store(j, patch + j * P);
+    } else {
+        fence();
+        store(0, patch);
+        fence();
+        put(Second{}, patch);
+        fence();
+        store(1, patch);
+    }
+}
+
+template <int EPI, int MT, int NT, int S>
+int launch(const pcb_linear_args& a, hipStream_t stream) {
+    using L = mfma_tile::Loop<MT, NT, S, 1>;
+    const int mb = pcb_ceil_div(a.M, L::BM), nb = pcb_ceil_div(a.N, EPI == PCB_EPI_SILU_MUL ? L::BN / 2 : L::BN);
+    const mfma_tile::Strips s = mfma_tile::strips(mb, nb, L::BM, L::BN);
+    hipLaunchKernelGGL((linear_tile_kernel<EPI, MT, NT, S>), dim3(8 * s.mh * s.nh), dim3(256), 0, stream, a, (Grid{mb, nb, s.px, s.mh, s.nh}));
+    return pcb_check_launch("linear_tile_kernel");
+}
+
+template <int EPI>
+int dispatch(const pcb_linear_args& a, hipStream_t stream) {
+    // The tile whose whole rounds of the 256 CUs cost least.  A round, in us, one workgroup per CU, from K = 64 .. 8192 on a full chip:
+    // 128 x 128 4.5 + 0.53 per K-step, 128 x 256 7 + 0.67, 256 x 256 10 + 1.03 (K = 2048: 21, 28, 43).  2048 rows, K = 2048, the three and
+    // what the rule took: N = 2048 20.0 / 28.0 / 42.7 -> 20.0, 2560 35.0 / 33.3 / 45.7 -> 31, 5136 54 / 59 / 53 -> 50, 8192 84 / 75 / 67 -> 66,
+    // 10272 112 / 95 / 99 -> 97; 6000 rows, K = 512, N = 2048 21.2 / 24.9 / 22.3 -> 21.9.
+    constexpr int C = EPI == PCB_EPI_SILU_MUL ? 2 : 1;               // weight rows per result column
+    auto rounds = [&](int bm, int bn) { return ((int64_t)pcb_ceil_div(a.M, bm) * pcb_ceil_div(C * a.N, bn) + 255) / 256; };
+    const float steps = (float)pcb_ceil_div(a.K, 64);
+    const float square = rounds(128, 128) * (4.5f + 0.53f * steps), wide = rounds(128, 256) * (7.0f + 0.67f * steps),
+                tall = rounds(256, 256) * (10.0f + 1.03f * steps);
+    if (tall <= wide && tall <= square) return launch<EPI, 4, 4, 2>(a, stream);
+    return wide <= square ? launch<EPI, 2, 4, 3>(a, stream) : launch<EPI, 2, 2, 3>(a, stream);
+}
+
+}  // namespace
+
+int pcb_linear_tiles(const pcb_linear_args& a, hipStream_t stream) {
+    switch (a.epilogue) {
+        case PCB_EPI_STORE: return dispatch<PCB_EPI_STORE>(a, stream);
+        case PCB_EPI_SILU_MUL: return dispatch<PCB_EPI_SILU_MUL>(a, stream);
+        default: return dispatch<PCB_EPI_SCALE_ADD>(a, stream);
+    }
+}

@@ -42,7 +42,7 @@ def stale(group: str) -> bool:
         return True
     prefix = pattern.split("*")[0]
     deps = glob.glob(os.path.join(CSRC, pattern)) + glob.glob(os.path.join(CSRC, prefix + "*.h")) + \
-        glob.glob(os.path.join(INCLUDE, "*.h"))
+        glob.glob(os.path.join(CSRC, "mfma_*.h")) + glob.glob(os.path.join(INCLUDE, "*.h"))
     return any(os.path.getmtime(d) > os.path.getmtime(lib) for d in deps)
 
 
@@ -60,12 +60,14 @@ def build(group: str, force: bool = False) -> str:
         srcs = sorted(glob.glob(os.path.join(CSRC, pattern)))
         if not srcs:
             raise RuntimeError(f"no sources match {pattern} under {CSRC}")
-        flags = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-mllvm", "-amdgpu-mfma-vgpr-form",
-                 *extra, *os.environ.get("PC_BUILD_FLAGS", "").split()]
+        flags = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden", *extra,
+                 *os.environ.get("PC_BUILD_FLAGS", "").split()]
         jobs = []
         for src in srcs:
             obj = os.path.join(objdir, os.path.basename(src) + ".o")
-            cmd = [hipcc(), *flags, "-c", src, "-o", obj]
+            # (pb_linear_tiles.hip: up to 256 accumulator registers beside the operands, which only fit as AGPRs)
+            form = [] if os.path.basename(src) == "pb_linear_tiles.hip" else ["-mllvm", "-amdgpu-mfma-vgpr-form"]
+            cmd = [hipcc(), *flags, *form, "-c", src, "-o", obj]
             print("[build]", " ".join(cmd), file=sys.stderr, flush=True)
             jobs.append((obj, cmd, subprocess.Popen(cmd, cwd=os.path.dirname(CSRC), stdout=sys.stderr)))
         for obj, cmd, proc in jobs:

@@ -310,6 +310,50 @@ def test_many_row_projections_of_experts_and_split_destinations(K):
     assert rel(y2[:, pos].permute(1, 0, 2).reshape(R, 84), z[:, 100:184]) < 5e-3 and rel(y3[:, pos].T, z[:, 184:]) < 5e-3
 
 
+@pytest.mark.parametrize("M,N", [(2048, 2052), (1900, 2500), (1900, 4106)])
+@pytest.mark.parametrize("K", [8, 136, 712])
+def test_whole_cu_tiles_and_where_their_results_go(M, N, K):
+    """Launches of each tile size (128 x 128, 128 x 256, 256 x 256) with a ragged last tile both ways and k ranges that end after 1, 2, 1 chunks
+    of a stage: rows scattered, rows that start anywhere, heads in whole quads and at odd offsets, a split inside a quad, fp32 split rows,
+    columns kept column by column, gated rows, the accumulation in place and from unaligned rows."""
+    b, bf = B(), torch.bfloat16
+    x, w, w2 = (rnd(r, K, dtype=bf, seed=i, scale=K ** -0.25) for i, r in ((1, M), (2, N), (3, N)))
+    bias = rnd(N, dtype=bf, seed=4)
+    z, gen = matmul32(x, w), torch.Generator().manual_seed(5)
+    perm = torch.randperm(M, generator=gen).to(DEV)
+    for dtype, tol in ((torch.float32, 2e-6), (bf, 4e-3)):
+        y = torch.zeros(M, N, dtype=dtype, device=DEV)
+        b.linear(x, w, y, M=M, row_dst=perm.to(torch.int32), bias=bias, act=b.ACT_RELU2, act_split=N - 130)
+        t = z + bias.float()
+        assert rel(y[perm], torch.cat([torch.relu(t[:, :N - 130]) ** 2, t[:, N - 130:]], dim=1)) < tol
+        odd = torch.zeros(M, N + 1, dtype=dtype, device=DEV)
+        b.linear(x, w, odd, M=M, ldy=N + 1)
+        assert rel(odd[:, :N], z) < tol and float(odd[:, N].float().abs().max()) == 0.0
+    # heads of 36 columns kept row by row (their rows at multiples of 36, then one element further), 68 columns kept column by column
+    pos = torch.randperm(M, generator=gen).to(DEV)
+    for cut, shift in ((N - 68 - 36 * 11, 0), (N - 68 - 36 * 11, 1), (N - 67 - 36 * 11, 0)):
+        third = cut + 36 * 11
+        y1, y2, y3 = torch.zeros(M, cut, dtype=bf, device=DEV), torch.zeros(11, M * 36 + 4, dtype=bf, device=DEV), torch.zeros(N - third, M, dtype=bf, device=DEV)
+        b.linear(x, w, y1, M=M, split_n=cut, y2=y2, row_off2=pos * 36 + shift, head_dim2=36, head_stride2=M * 36 + 4, split_n3=third, y3=y3,
+                 row_off3=pos.clone(), col_stride3=M)
+        heads = y2[:, shift:M * 36 + shift].view(11, M, 36)[:, pos].permute(1, 0, 2).reshape(M, 396)
+        assert rel(y1, z[:, :cut]) < 4e-3 and rel(heads, z[:, cut:third]) < 4e-3 and rel(y3[:, pos].T, z[:, third:]) < 4e-3
+    for cut, stride in ((N - 70, 72), (N - 72, 76), (N - 71, 71)):
+        y1, y2 = torch.zeros(M, cut, dtype=bf, device=DEV), torch.zeros(M, stride, device=DEV)
+        b.linear(x, w, y1, M=M, split_n=cut, y2=y2, y2_f32=True, head_stride2=stride)
+        assert rel(y1, z[:, :cut]) < 4e-3 and rel(y2[:, :N - cut], z[:, cut:]) < 2e-6
+    gate, g = rnd(M, 3, dtype=bf, seed=6), torch.zeros(M, N, dtype=bf, device=DEV)
+    b.linear(x, w, g, M=M, epilogue=b.EPI_SILU_MUL, w2=w2, act=b.ACT_RELU, row_gate=gate, ld_row_gate=3)
+    assert rel(g, torch.relu(z) * matmul32(x, w2) * gate[:, :1].float()) < 4e-3
+    cs, y = rnd(N, seed=7), rnd(M, N, seed=8)
+    want = y + cs * z
+    b.linear(x, w, y, M=M, epilogue=b.EPI_SCALE_ADD, col_scale=cs)
+    assert rel(y, want) < 2e-6
+    base = rnd(M * N + 1, seed=9)[1:].view(M, N)
+    b.linear(x, w, y, M=M, bias=bias, epilogue=b.EPI_SCALE_ADD, base=base, col_scale=cs)
+    assert rel(y, base + cs * (z + bias.float())) < 2e-6
+
+
 def test_router_scores_are_not_renormalised():
     b, T, n, top = B(), 9, 11, 4
     z = rnd(T, n, seed=3, scale=2.0)
