@@ -5,8 +5,8 @@
 // Tiling: workgroup = 4 waves in a 2 x 2 grid, a wave owns TM x TN result tiles of 16 x 16, so the workgroup covers
 // (32 TM) x (32 TN) of Y.  Per stage of two 32-element k-steps the A and B panels go global -> registers -> LDS (the next stage's
 // loads are in flight while this stage's MFMAs run); waves read their operand fragments from LDS with one 16-byte read per fragment (bf16).
-// bf16 operands that can be read in 16-byte chunks take linear_dma_kernel below instead (large plain launches pb_linear_tiles.hip); fp32, odd
-// sizes and scaled rows this one.
+// Operands that can be read in 16-byte chunks take linear_dma_kernel below instead (large plain launches in bf16 pb_linear_tiles.hip); odd sizes
+// and scaled rows this one.
 #include <type_traits>
 
 #include "pb_linear_epi.h"
@@ -48,6 +48,43 @@ __device__ __forceinline__ u32x4 load_chunk(const E* p, int k, int K, bool vec, 
     }
     return c;
 }
+
+// the lane's elements of a whole k-step, p at element 0 of it in the lane's row (16-byte aligned): k elements 8 group .. + 7 in 16-byte reads.
+// (Both operands use this map, so where an element sits in the k-step does not matter.  fp32 in the map of load_frag is eight 4-byte reads.)
+__device__ __forceinline__ Frag<bf16_t> whole_frag(const bf16_t* p, int group) {
+    Frag<bf16_t> f;
+    f.v = *reinterpret_cast<const u32x4*>(p + 8 * group);
+    return f;
+}
+__device__ __forceinline__ Frag<float> whole_frag(const float* p, int group) {
+    Frag<float> f;
+    const f4 lo = *reinterpret_cast<const f4*>(p + 8 * group), hi = *reinterpret_cast<const f4*>(p + 8 * group + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f.v[e] = lo[e], f.v[4 + e] = hi[e];
+    return f;
+}
+
+// A k-step's products into a pair of sums, odd parts into the second (fp32: shorter chains of roundings -- against 64 bits 0.7 of one chain's
+// error at every size -- and of dependent MFMAs; bf16 has one part); chain: into one, in order of k
+template <typename E>
+struct Sum;
+template <>
+struct Sum<bf16_t> {
+    f4 c = {0.f, 0.f, 0.f, 0.f};
+    __device__ __forceinline__ void add(const Frag<bf16_t>& a, const Frag<bf16_t>& b) { c = mma(a, b, c); }
+    __device__ __forceinline__ void chain(const Frag<bf16_t>& a, const Frag<bf16_t>& b) { add(a, b); }
+    __device__ __forceinline__ f4 total() const { return c; }
+};
+template <>
+struct Sum<float> {
+    f4 c[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
+    __device__ __forceinline__ void add(const Frag<float>& a, const Frag<float>& b) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) c[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[e], b.v[e], c[e & 1], 0, 0, 0);
+    }
+    __device__ __forceinline__ void chain(const Frag<float>& a, const Frag<float>& b) { c[0] = mma(a, b, c[0]); }
+    __device__ __forceinline__ f4 total() const { return c[0] + c[1]; }
+};
 
 template <typename E, int EPI, int TM, int TN>
 __global__ __launch_bounds__(256) void linear_kernel(pcb_linear_args a) {
@@ -177,20 +214,29 @@ __global__ __launch_bounds__(256) void linear_kernel(pcb_linear_args a) {
         const float bv = bias ? to_f32(bias[n]) : 0.0f;
         const float bv2 = (TWO && a.bias2) ? to_f32(((const E*)a.bias2)[n]) : 0.0f;
         const float cs = (EPI == PCB_EPI_SCALE_ADD) ? a.col_scale[n] : 0.0f;
+        Place to[TM][4];
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int m = m_lo + (wm * TM + i) * 16 + 4 * group + r;
-                if (m < m_hi) emit<E, EPI>(a, m, n, acc[i][j][r], TWO ? acc2[i][j][r] : 0.0f, bv, cs, bv2);
+                to[i][r] = place<E, EPI>(a, m < m_hi ? m : m_hi - 1, n);
             }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (m_lo + (wm * TM + i) * 16 + 4 * group + r < m_hi)
+                    put<E, EPI>(to[i][r], finished<E, EPI>(a, to[i][r], n, acc[i][j][r], TWO ? acc2[i][j][r] : 0.0f, bv, bv2), cs);
     }
 }
 
 // ---- few rows: the weights stream once, straight from memory into the matrix cores --------------------------------------------
 // Workgroup = 16 result columns x up to 16 rows; its SKW waves split the k range (k-step s goes to wave s % SKW) and add their
-// partial tiles through LDS.  No LDS staging: a lane's B fragment is 16 contiguous bytes of its weight row, its A fragment 16
-// bytes of its activation row (a handful of rows that stay in cache).
+// partial tiles through LDS.  No LDS staging: a lane's B fragment is 16 contiguous bytes of its weight row (fp32: 32), its A fragment as many of
+// its activation row (a handful of rows that stay in cache).  Bound by the launch and one trip to memory at 4 MB of weights, by the stream at
+// 40 (10 272 x 2 048 bf16, 8 rows: 12.6 us, 3.3 TB/s).  fp32 in 16-byte reads instead of 4-byte ones, us: 1 row, 1024 x 1024 10.0 -> 5.6,
+// 1024 x 4096 32.6 -> 13.4, 5136 x 1024 18.2 -> 9.5, 8 rows 27.6 -> 10.4.
 template <typename E>
 __device__ __forceinline__ void scale_frag(Frag<E>& f, float s);
 template <>
@@ -205,19 +251,6 @@ template <>
 __device__ __forceinline__ void scale_frag<float>(Frag<float>& f, float s) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) f.v[e] *= s;
-}
-
-// the lane's elements of a whole k-step; p points at the first of them
-__device__ __forceinline__ Frag<bf16_t> whole_frag(const bf16_t* p) {
-    Frag<bf16_t> f;
-    f.v = *reinterpret_cast<const u32x4*>(p);
-    return f;
-}
-__device__ __forceinline__ Frag<float> whole_frag(const float* p) {
-    Frag<float> f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) f.v[e] = p[4 * e];
-    return f;
 }
 
 // SKW: waves of a workgroup (eight, or sixteen where few workgroups walk a long k range)
@@ -259,23 +292,31 @@ __global__ __launch_bounds__(64 * SKW) void linear_skinny_kernel(pcb_linear_args
     const E* wrow = W + (int64_t)(b_ok ? n_b : 0) * a.ldw;
     const E* wrow2 = TWO ? W2 + (int64_t)(b_ok ? n_b : 0) * a.ldw : nullptr;
     const E* xrow = X + (int64_t)(a_ok ? (a.row_src ? a.row_src[m_a] : m_a) : 0) * a.ldx;
+    // (the wave that stores asks for everything the epilogue needs before the products)
+    const int n_c = n_lo + l15 < N ? n_lo + l15 : N - 1;
+    float bv = 0.0f, bv2 = 0.0f, cs = 0.0f;
+    Place to[4] = {};
+    if (wave == 0) {
+        if (a.bias) bv = to_f32(((const E*)a.bias)[n_c]);
+        if (TWO && a.bias2) bv2 = to_f32(((const E*)a.bias2)[n_c]);
+        if (EPI == PCB_EPI_SCALE_ADD) cs = a.col_scale[n_c];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) to[r] = place<E, EPI>(a, m_lo + 4 * group + r < m_hi ? m_lo + 4 * group + r : m_hi - 1, n_c);
+    }
     const bool scaled = a.row_scale != nullptr;
     const float xs = (scaled && a_ok) ? a.row_scale[m_a] : 1.0f;
-    f4 acc = f4{0.f, 0.f, 0.f, 0.f}, acc2 = f4{0.f, 0.f, 0.f, 0.f};
+    Sum<E> sum, sum2;
     const int nsteps = (K + 31) / 32;
     // whole k-steps of rows that can be read in 16-byte pieces: nothing between the loads.  (Lanes past the last row or column read row 0
     // or column 0 instead: what they multiply is not stored.)
     int st = wave;
     if (vec && !scaled) {
         const int whole = K / 32;
-        const E* xp = xrow + (sizeof(E) == 2 ? 8 * group : group);
-        const E* wp = wrow + (sizeof(E) == 2 ? 8 * group : group);
-        const E* wp2 = TWO ? wrow2 + (sizeof(E) == 2 ? 8 * group : group) : nullptr;
 #pragma unroll 8
         for (; st < whole; st += SKW) {
-            const Frag<E> fa = whole_frag(xp + 32 * st), fb = whole_frag(wp + 32 * st);
-            acc = mma(fa, fb, acc);
-            if (TWO) acc2 = mma(fa, whole_frag(wp2 + 32 * st), acc2);
+            const Frag<E> fa = whole_frag(xrow + 32 * st, group), fb = whole_frag(wrow + 32 * st, group);
+            sum.add(fa, fb);
+            if (TWO) sum2.add(fa, whole_frag(wrow2 + 32 * st, group));
         }
     }
 #pragma unroll 2
@@ -284,12 +325,10 @@ __global__ __launch_bounds__(64 * SKW) void linear_skinny_kernel(pcb_linear_args
         Frag<E> fa = load_frag(xrow + k0, group, a_ok ? K - k0 : 0, vec);
         if (scaled) scale_frag<E>(fa, xs);
         const Frag<E> fb = load_frag(wrow + k0, group, b_ok ? K - k0 : 0, vec);
-        acc = mma(fa, fb, acc);
-        if (TWO) {
-            const Frag<E> fb2 = load_frag(wrow2 + k0, group, b_ok ? K - k0 : 0, vec);
-            acc2 = mma(fa, fb2, acc2);
-        }
+        sum.chain(fa, fb);
+        if (TWO) sum2.chain(fa, load_frag(wrow2 + k0, group, b_ok ? K - k0 : 0, vec));
     }
+    f4 acc = sum.total(), acc2 = sum2.total();
     red[0][wave][lane] = acc;
     if (TWO) red[1][wave][lane] = acc2;
     __syncthreads();
@@ -303,25 +342,21 @@ __global__ __launch_bounds__(64 * SKW) void linear_skinny_kernel(pcb_linear_args
     }
     const int n = n_lo + l15;
     if (n >= N) return;
-    const E* bias = (const E*)a.bias;
-    const float bv = bias ? to_f32(bias[n]) : 0.0f;
-    const float bv2 = (TWO && a.bias2) ? to_f32(((const E*)a.bias2)[n]) : 0.0f;
-    const float cs = (EPI == PCB_EPI_SCALE_ADD) ? a.col_scale[n] : 0.0f;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int m = m_lo + 4 * group + r;
-        if (m < m_hi) emit<E, EPI>(a, m, n, acc[r], acc2[r], bv, cs, bv2);
-    }
+    for (int r = 0; r < 4; ++r)
+        if (m_lo + 4 * group + r < m_hi) put<E, EPI>(to[r], finished<E, EPI>(a, to[r], n, acc[r], acc2[r], bv, bv2), cs);
 }
 
-// ---- many rows in bf16: both panels travel to LDS by themselves --------------------------------------------------------------------
+// ---- many rows: both panels travel to LDS by themselves ------------------------------------------------------------------------------
 // The same tiles (2 x 2 waves of TM x TN result tiles) for operands whose rows can be read in 16-byte chunks: global_load_lds carries a
-// stage of 64 k elements (1 KiB per wave instruction: 8 rows x 128 bytes) straight into a ring of two or three images, one barrier per stage, so
-// no register and no branch stands between the loads.  Rows past the end repeat the last one (their results are not stored); chunks
-// past K come from a block of zeros.  The 16-byte chunk c of row r sits at position c ^ ((r >> 1) & 7) of its 128-byte row, which spreads
-// a fragment read over all banks; the loads write lane by lane, so the permutation is applied to each lane's source.
+// stage of 128 bytes of k (64 elements of bf16, 32 of fp32; 1 KiB per wave instruction: 8 rows) straight into a ring of two or three images, one
+// barrier per stage, so no register and no branch stands between the loads.  Rows past the end repeat the last one (their results are not
+// stored); chunks past K come from a block of zeros.  The 16-byte chunk c of row r sits at position c ^ ((r >> 1) & 7) of its 128-byte row,
+// which spreads a fragment read over all banks; the loads write lane by lane, so the permutation is applied to each lane's source.
 // A plain launch numbers its tiles panel by panel (all row blocks of a column panel in turn) and gives each XCD one run of them: a
 // panel's weights are fetched into one L2.
+// fp32 through here instead of linear_kernel (one stage in registers, fragments in eight 4-byte LDS reads), us: 600 rows, 2048 x 2048 257 -> 68,
+// 1024 x 1024 120 -> 26, 1024 x 4096 470 -> 91, 5136 x 1024 141 -> 79; 2048 x 2048 x 2048 267 -> 149 (0.115 of 0.157 PFLOP/s).
 __device__ const u32x4 zero_row = {0u, 0u, 0u, 0u};
 
 __device__ __forceinline__ void dma16(const void* g, void* lds_wave_base) {
@@ -329,11 +364,10 @@ __device__ __forceinline__ void dma16(const void* g, void* lds_wave_base) {
                                      0, 0);
 }
 
-template <int EPI, int TM, int TN, int STAGES>
+template <typename E, int EPI, int TM, int TN, int STAGES>
 __global__ __launch_bounds__(256) void linear_dma_kernel(pcb_linear_args a) {
-    typedef bf16_t E;
     constexpr bool TWO = EPI == PCB_EPI_SILU_MUL;
-    constexpr int BM = 32 * TM, BN = 32 * TN, ROWS = BM + (TWO ? 2 : 1) * BN, BK = 64;
+    constexpr int BM = 32 * TM, BN = 32 * TN, ROWS = BM + (TWO ? 2 : 1) * BN, CE = Tile<E>::CE, BK = 8 * CE;
     constexpr int NI = ROWS / 32;                                    // wave instructions per wave and stage
     __shared__ __attribute__((aligned(16))) E img[STAGES][ROWS * BK];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -374,7 +408,7 @@ __global__ __launch_bounds__(256) void linear_dma_kernel(pcb_linear_args a) {
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         const int r = 8 * (4 * i + wave) + (lane >> 3);
-        kc[i] = ((lane & 7) ^ ((r >> 1) & 7)) * 8;
+        kc[i] = ((lane & 7) ^ ((r >> 1) & 7)) * CE;
         if (32 * i < BM) {
             int m = m_lo + r;
             m = m < m_hi ? m : m_hi - 1;
@@ -396,17 +430,19 @@ __global__ __launch_bounds__(256) void linear_dma_kernel(pcb_linear_args a) {
                 dma16(k0 + kc[i] < K ? (const void*)(src[i] + k0 + kc[i]) : (const void*)&zero_row, &img[buf][(4 * i + wave) * 8 * BK]);
         }
     };
-    f4 acc[TM][TN], acc2[TWO ? TM : 1][TWO ? TN : 1];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
-            if (TWO) acc2[i][j] = f4{0.f, 0.f, 0.f, 0.f};
-        }
+    Sum<E> sum[TM][TN], sum2[TWO ? TM : 1][TWO ? TN : 1];
+    // the lane's k elements 8 group .. + 7 of a 32-deep step: one chunk in bf16, two in fp32
     auto frag = [&](int buf, int r, int ks) {
         Frag<E> f;
-        f.v = *reinterpret_cast<const u32x4*>(&img[buf][r * BK + ((4 * ks + group) ^ ((r >> 1) & 7)) * 8]);
+        const E* row = &img[buf][r * BK];
+        const int sw = (r >> 1) & 7;
+        if constexpr (sizeof(E) == 2) {
+            f.v = *reinterpret_cast<const u32x4*>(row + ((4 * ks + group) ^ sw) * CE);
+        } else {
+            const f4 lo = *reinterpret_cast<const f4*>(row + ((2 * group) ^ sw) * CE), hi = *reinterpret_cast<const f4*>(row + ((2 * group + 1) ^ sw) * CE);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) f.v[e] = lo[e], f.v[4 + e] = hi[e];
+        }
         return f;
     };
     // STAGES - 1 stages are in flight: at the top of a step the wave waits for its own part of the stage at hand (loads land in order),
@@ -424,7 +460,7 @@ __global__ __launch_bounds__(256) void linear_dma_kernel(pcb_linear_args a) {
         asm volatile("" ::: "memory");
         if (k0 + (STAGES - 1) * BK < K) fetch(k0 + (STAGES - 1) * BK, buf == 0 ? STAGES - 1 : buf - 1);
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
+        for (int ks = 0; ks < BK / 32; ++ks) {
             Frag<E> fa[TM];
 #pragma unroll
             for (int i = 0; i < TM; ++i) fa[i] = frag(buf, (wm * TM + i) * 16 + l15, ks);
@@ -432,16 +468,24 @@ __global__ __launch_bounds__(256) void linear_dma_kernel(pcb_linear_args a) {
             for (int j = 0; j < TN; ++j) {
                 const Frag<E> fb = frag(buf, BM + (wn * TN + j) * 16 + l15, ks);
 #pragma unroll
-                for (int i = 0; i < TM; ++i) acc[i][j] = mma(fb, fa[i], acc[i][j]);
+                for (int i = 0; i < TM; ++i) sum[i][j].add(fb, fa[i]);
                 if (TWO) {
                     const Frag<E> fb2 = frag(buf, BM + BN + (wn * TN + j) * 16 + l15, ks);
 #pragma unroll
-                    for (int i = 0; i < TM; ++i) acc2[i][j] = mma(fb2, fa[i], acc2[i][j]);
+                    for (int i = 0; i < TM; ++i) sum2[i][j].add(fb2, fa[i]);
                 }
             }
         }
     }
 
+    f4 acc[TM][TN], acc2[TWO ? TM : 1][TWO ? TN : 1];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            acc[i][j] = sum[i][j].total();
+            if (TWO) acc2[i][j] = sum2[i][j].total();
+        }
     // (the weights are the products' first operand: a lane ends up with four neighbouring columns of one row.)
     // Bias, gate and activation first, in the accumulators -- an activation is chosen once, around the loop over them --, then the stores
     const E* bias = (const E*)a.bias;
@@ -506,16 +550,32 @@ __global__ __launch_bounds__(256) void linear_dma_kernel(pcb_linear_args a) {
         for (int part = 0; part < 2; ++part) pass(part ? a.act2 : a.act, part ? mid : 0, part ? end : mid);
     }
     const int whole = act_end(a);                                    // columns that go to y
-    const int esz = (EPI == PCB_EPI_SCALE_ADD || a.out_f32) ? 4 : 2;
+    const int esz = (EPI == PCB_EPI_SCALE_ADD || a.out_f32 || sizeof(E) == 4) ? 4 : 2;
     const bool quads = a.ldy % 4 == 0 && (uintptr_t)a.y % (4 * esz) == 0 && a.y_batch_stride % 4 == 0 &&
                        (EPI != PCB_EPI_SCALE_ADD || !a.base || (a.ldbase % 4 == 0 && (uintptr_t)a.base % 16 == 0));
     const int64_t y0 = a.n_batch > 0 ? (int64_t)blockIdx.z * a.y_batch_stride : 0;
+    // (what the stores need is loaded before the first of them)
+    int64_t dst[TM];
+    f4 base[EPI == PCB_EPI_SCALE_ADD ? TM : 1][EPI == PCB_EPI_SCALE_ADD ? TN : 1], cs[EPI == PCB_EPI_SCALE_ADD ? TN : 1];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        const int mm = m_lo + (wm * TM + i) * 16 + l15, m = mm < m_hi ? mm : m_hi - 1;
+        dst[i] = (int64_t)(EPI != PCB_EPI_SCALE_ADD && a.row_dst ? a.row_dst[m] : m) * a.ldy + y0;
+        if constexpr (EPI == PCB_EPI_SCALE_ADD) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const int n = n_lo + (wn * TN + j) * 16 + 4 * group;
+                if (i == 0) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) cs[j][e] = n + e < N ? a.col_scale[n + e] : 0.0f;
+                }
+                if (quads && n + 4 <= N) base[i][j] = *reinterpret_cast<const f4*>(a.base ? a.base + (int64_t)m * a.ldbase + n : (const float*)a.y + dst[i] + n);
+            }
+        }
+    }
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
         const int n = n_lo + (wn * TN + j) * 16 + 4 * group;
-        float cs[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) cs[e] = EPI == PCB_EPI_SCALE_ADD && n + e < N ? a.col_scale[n + e] : 0.0f;
         const bool quad = quads && n + 4 <= whole;
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
@@ -523,54 +583,64 @@ __global__ __launch_bounds__(256) void linear_dma_kernel(pcb_linear_args a) {
             if (m >= m_hi) continue;
             const f4 v = acc[i][j];
             if (quad) {
-                if (EPI == PCB_EPI_SCALE_ADD) {
-                    f4* y = reinterpret_cast<f4*>((float*)a.y + (int64_t)m * a.ldy + n);
-                    const f4 b0 = a.base ? *reinterpret_cast<const f4*>(a.base + (int64_t)m * a.ldbase + n) : *y;
-                    *y = f4{b0[0] + cs[0] * v[0], b0[1] + cs[1] * v[1], b0[2] + cs[2] * v[2], b0[3] + cs[3] * v[3]};
-                } else {
-                    const int64_t at = (int64_t)(a.row_dst ? a.row_dst[m] : m) * a.ldy + n + y0;
-                    if (a.out_f32)
-                        *reinterpret_cast<f4*>((float*)a.y + at) = v;
-                    else
-                        *reinterpret_cast<uint2*>((E*)a.y + at) = uint2{bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3])};
-                }
+                if constexpr (EPI == PCB_EPI_SCALE_ADD)
+                    *reinterpret_cast<f4*>((float*)a.y + dst[i] + n) = base[i][j] + cs[j] * v;
+                else if (esz == 4)
+                    *reinterpret_cast<f4*>((float*)a.y + dst[i] + n) = v;
+                else
+                    *reinterpret_cast<uint2*>((E*)a.y + dst[i] + n) = uint2{bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3])};
             } else {
+                Place to[4] = {};
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    if (n + e < N) put<E, EPI>(a, m, n + e, v[e], cs[e]);
+                    if (n + e < N) to[e] = place<E, EPI>(a, m, n + e);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < N) put<E, EPI>(to[e], v[e], EPI == PCB_EPI_SCALE_ADD ? cs[EPI == PCB_EPI_SCALE_ADD ? j : 0][e] : 0.0f);
             }
         }
     }
 }
 
-template <int EPI, int TM, int TN, int STAGES>
+template <typename E, int EPI, int TM, int TN, int STAGES>
 int launch_dma(const pcb_linear_args& a, hipStream_t stream) {
     constexpr int BM = 32 * TM, BN = 32 * TN;
     const int nb = pcb_ceil_div(a.N, BN), mb = pcb_ceil_div(a.M, BM);
     const dim3 grid = a.n_groups > 0 ? dim3(nb, mb + a.n_groups) : dim3(8 * pcb_ceil_div(nb * mb, 8), 1, a.n_batch > 0 ? a.n_batch : 1);
-    hipLaunchKernelGGL((linear_dma_kernel<EPI, TM, TN, STAGES>), grid, dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((linear_dma_kernel<E, EPI, TM, TN, STAGES>), grid, dim3(256), 0, stream, a);
     return pcb_check_launch("linear_dma_kernel");
 }
 
-// whether every operand row can be read in 16-byte chunks (bf16)
+// whether every operand row can be read in 16-byte chunks
 bool dma_ok(const pcb_linear_args& a) {
-    return a.dtype == PCB_BF16 && !a.row_scale && a.K % 8 == 0 && a.ldx % 8 == 0 && a.ldw % 8 == 0 && a.w_group_stride % 8 == 0 &&
-           a.x_batch_stride % 8 == 0 && ((uintptr_t)a.x | (uintptr_t)a.w | (uintptr_t)a.w2) % 16 == 0 &&
-           (int64_t)pcb_ceil_div(a.N, 32) * pcb_ceil_div(a.M, 32) < (1 << 30);
+    const int ce = a.dtype == PCB_BF16 ? 8 : 4;
+    return !a.row_scale && a.K % ce == 0 && a.ldx % ce == 0 && a.ldw % ce == 0 && a.w_group_stride % ce == 0 && a.x_batch_stride % ce == 0 &&
+           ((uintptr_t)a.x | (uintptr_t)a.w | (uintptr_t)a.w2) % 16 == 0 && (int64_t)pcb_ceil_div(a.N, 32) * pcb_ceil_div(a.M, 32) < (1 << 30);
 }
 
-template <int EPI>
+template <typename E, int EPI>
 int dispatch_dma(const pcb_linear_args& a, int rows, hipStream_t stream) {
     // the largest tile that still gives every CU a workgroup; grouped launches count the tiles their rows fill
     constexpr int TNW = EPI == PCB_EPI_SILU_MUL ? 2 : 4;
     const int64_t batch = a.n_batch > 0 ? a.n_batch : 1;
     auto tiles = [&](int bm, int bn) { return batch * pcb_ceil_div(a.M, bm) * pcb_ceil_div(a.N, bn); };
+    if constexpr (sizeof(E) == 4) {
+        // fp32 (1 / 16 of the bf16 rate): bound by the matrix cores, so what counts is that all CUs have the same share of tiles.  Whole rounds of
+        // the 256 CUs times a tile's work; a 128 x 128 tile costs 3.8 of 64 x 64 and a 32 x 64 tile 0.575 (us, 64-, 128- and 32-row tiles):
+        // 2048 x 2048 x 2048 158 / 149 / 166, 4096 x 4096, K = 1024 299 / 276 / 317, 1200 x 4096, K = 2048 188 / 267 / 203, 600 x 2564, K = 1024
+        // 44 / 76 / 47, 600 x 2048, K = 2048 79 / 146 / 68, 130 x 1024, K = 1024 25 / 75 / 17.
+        const int64_t extra = a.n_groups / 2;                        // (groups: part tiles)
+        auto rounds = [&](int bm, int bn) { return (batch * (pcb_ceil_div(a.M, bm) + extra) * pcb_ceil_div(a.N, bn) + 255) / 256; };
+        const float large = 3.8f * rounds(128, 32 * TNW), mid = rounds(64, 16 * TNW), small = 0.575f * rounds(32, 16 * TNW);
+        if (rows > 64 && large <= mid && large <= small) return launch_dma<E, EPI, 4, TNW, 2>(a, stream);
+        return rows > 32 && mid <= small ? launch_dma<E, EPI, 2, TNW / 2, 3>(a, stream) : launch_dma<E, EPI, 1, TNW / 2, 3>(a, stream);
+    }
     // (two workgroups of a CU hide each other's loads behind their products; a lone one needs a stage more in flight)
-    if (rows > 64 && tiles(128, 32 * TNW) > 256) return launch_dma<EPI, 4, TNW, 2>(a, stream);
-    if (rows > 64 && tiles(128, 32 * TNW) == 256) return launch_dma<EPI, 4, TNW, 3>(a, stream);
-    if (rows > 32 && tiles(64, 32 * TNW) >= 400) return launch_dma<EPI, 2, TNW, 3>(a, stream);
-    if (rows > 32) return launch_dma<EPI, 2, TNW / 2, 3>(a, stream);
-    return launch_dma<EPI, 1, TNW / 2, 3>(a, stream);
+    if (rows > 64 && tiles(128, 32 * TNW) > 256) return launch_dma<E, EPI, 4, TNW, 2>(a, stream);
+    if (rows > 64 && tiles(128, 32 * TNW) == 256) return launch_dma<E, EPI, 4, TNW, 3>(a, stream);
+    if (rows > 32 && tiles(64, 32 * TNW) >= 400) return launch_dma<E, EPI, 2, TNW, 3>(a, stream);
+    if (rows > 32) return launch_dma<E, EPI, 2, TNW / 2, 3>(a, stream);
+    return launch_dma<E, EPI, 1, TNW / 2, 3>(a, stream);
 }
 
 template <typename E, int EPI, int TM, int TN>
@@ -605,27 +675,28 @@ int dispatch(const pcb_linear_args& a, hipStream_t stream) {
         }
         return pcb_check_launch("linear_skinny_kernel");
     }
-    if (sizeof(E) == 2 && dma_ok(a)) {
+    if (dma_ok(a)) {
         // Plain launches whose 128 x 128 tiles reach more than half of the 256 CUs go to the whole-CU tiles of pb_linear_tiles.hip (row strides
         // such that a tile's rows lie within 32-bit offsets); below, the smaller tiles here give more CUs work: 300 x 2048, K = 2048 (48 tiles)
         // 13.1 us here, 14.9 there, 1024 x 1024 x 1024 (64) 8.3 / 9.6, 1024 x 2048, K = 2048 (128) 15.9 / 16.2, 300 x 8192 (192) 21.4 / 17.4.
         const int weight_rows = a.epilogue == PCB_EPI_SILU_MUL ? 2 * a.N : a.N;
-        if (rows > 64 && a.n_groups == 0 && a.n_batch == 0 && !a.row_src && a.ldx < (1 << 22) && a.ldw < (1 << 22) &&
+        if (sizeof(E) == 2 && rows > 64 && a.n_groups == 0 && a.n_batch == 0 && !a.row_src && a.ldx < (1 << 22) && a.ldw < (1 << 22) &&
             (int64_t)pcb_ceil_div(a.M, 128) * pcb_ceil_div(weight_rows, 128) > 128)
             return pcb_linear_tiles(a, stream);
         switch (a.epilogue) {
-            case PCB_EPI_STORE: return dispatch_dma<PCB_EPI_STORE>(a, rows, stream);
-            case PCB_EPI_SILU_MUL: return dispatch_dma<PCB_EPI_SILU_MUL>(a, rows, stream);
-            default: return dispatch_dma<PCB_EPI_SCALE_ADD>(a, rows, stream);
+            case PCB_EPI_STORE: return dispatch_dma<E, PCB_EPI_STORE>(a, rows, stream);
+            case PCB_EPI_SILU_MUL: return dispatch_dma<E, PCB_EPI_SILU_MUL>(a, rows, stream);
+            default: return dispatch_dma<E, PCB_EPI_SCALE_ADD>(a, rows, stream);
         }
     }
+    auto go = [&](auto epi) {
+        constexpr int EPI = decltype(epi)::value, W = EPI == PCB_EPI_SILU_MUL ? 2 : 1;
+        return big ? launch<E, EPI, 4, 4 / W>(a, stream) : launch<E, EPI, 1, 2 / W>(a, stream);
+    };
     switch (a.epilogue) {
-        case PCB_EPI_STORE:
-            return big ? launch<E, PCB_EPI_STORE, 4, 4>(a, stream) : launch<E, PCB_EPI_STORE, 1, 2>(a, stream);
-        case PCB_EPI_SILU_MUL:
-            return big ? launch<E, PCB_EPI_SILU_MUL, 4, 2>(a, stream) : launch<E, PCB_EPI_SILU_MUL, 1, 1>(a, stream);
-        default:
-            return big ? launch<E, PCB_EPI_SCALE_ADD, 4, 4>(a, stream) : launch<E, PCB_EPI_SCALE_ADD, 1, 2>(a, stream);
+        case PCB_EPI_STORE: return go(std::integral_constant<int, PCB_EPI_STORE>{});
+        case PCB_EPI_SILU_MUL: return go(std::integral_constant<int, PCB_EPI_SILU_MUL>{});
+        default: return go(std::integral_constant<int, PCB_EPI_SCALE_ADD>{});
     }
 }
 

@@ -27,52 +27,55 @@ __device__ __forceinline__ float gate_act(int act, float v) {
     return act == PCB_ACT_RELU ? fmaxf(v, 0.0f) : s;
 }
 
-// where one finished element goes (see pcb_linear_args)
-template <typename E, int EPI>
-__device__ __forceinline__ void put(const pcb_linear_args& a, int m, int n, float v, float cs) {
-    if (EPI == PCB_EPI_SCALE_ADD) {
-        float* y = (float*)a.y + (int64_t)m * a.ldy + n;
-        const float b0 = a.base ? a.base[(int64_t)m * a.ldbase + n] : *y;
-        *y = b0 + cs * v;
-        return;
-    }
-    if (a.split_n3 > 0 && n >= a.split_n3) {
-        ((E*)a.y3)[a.row_off3[m] + (int64_t)(n - a.split_n3) * a.col_stride3] = from_f32<E>(v);
-        return;
-    }
-    if (a.split_n > 0 && n >= a.split_n) {
-        const int c = n - a.split_n;
-        if (a.y2_f32) {
-            ((float*)a.y2)[m * a.head_stride2 + c] = v;
-            return;
-        }
-        E* y = (E*)a.y2 + a.row_off2[m] + (int64_t)(c / a.head_dim2) * a.head_stride2 + c % a.head_dim2;
-        *y = from_f32<E>(v);
-        return;
-    }
-    const int64_t at = (int64_t)(a.row_dst ? a.row_dst[m] : m) * a.ldy + n + (a.n_batch > 0 ? (int64_t)blockIdx.z * a.y_batch_stride : 0);
-    if (a.out_f32)
-        ((float*)a.y)[at] = v;
-    else
-        ((E*)a.y)[at] = from_f32<E>(v);
-}
-
 // columns that pass through act / act2 of a plain store: the split-off parts are stored as they are
 __device__ __forceinline__ int act_end(const pcb_linear_args& a) {
     return a.split_n > 0 ? a.split_n : (a.split_n3 > 0 ? a.split_n3 : a.N);
 }
 
-// one result element through the epilogue
+// Where one finished element goes (see pcb_linear_args) and, for the scaled accumulation, what it is added to.  A kernel asks for all its
+// elements' places before its first store: loads and stores count on one counter, so a load behind a store waits for the store's way to memory.
+struct Place {
+    char* p;
+    bool wide;                                                       // fp32 (else E)
+    float base;                                                      // scaled accumulation: what it is added to; gated epilogue: the row's gate
+};
 template <typename E, int EPI>
-__device__ __forceinline__ void emit(const pcb_linear_args& a, int m, int n, float acc, float acc2, float bv, float cs, float bv2 = 0.0f) {
+__device__ __forceinline__ Place place(const pcb_linear_args& a, int m, int n) {
+    if (EPI == PCB_EPI_SCALE_ADD) {
+        float* y = (float*)a.y + (int64_t)m * a.ldy + n;
+        return Place{(char*)y, true, a.base ? a.base[(int64_t)m * a.ldbase + n] : *y};
+    }
+    if (a.split_n3 > 0 && n >= a.split_n3) return Place{(char*)((E*)a.y3 + a.row_off3[m] + (int64_t)(n - a.split_n3) * a.col_stride3), false, 0.0f};
+    if (a.split_n > 0 && n >= a.split_n) {
+        const int c = n - a.split_n;
+        if (a.y2_f32) return Place{(char*)((float*)a.y2 + m * a.head_stride2 + c), true, 0.0f};
+        return Place{(char*)((E*)a.y2 + a.row_off2[m] + (int64_t)(c / a.head_dim2) * a.head_stride2 + c % a.head_dim2), false, 0.0f};
+    }
+    const int64_t at = (int64_t)(a.row_dst ? a.row_dst[m] : m) * a.ldy + n + (a.n_batch > 0 ? (int64_t)blockIdx.z * a.y_batch_stride : 0);
+    const float gate = EPI == PCB_EPI_SILU_MUL && a.row_gate ? to_f32(((const E*)a.row_gate)[m * a.ld_row_gate]) : 1.0f;
+    return a.out_f32 ? Place{(char*)((float*)a.y + at), true, gate} : Place{(char*)((E*)a.y + at), false, gate};
+}
+template <typename E, int EPI>
+__device__ __forceinline__ void put(const Place& t, float v, float cs) {
+    if (EPI == PCB_EPI_SCALE_ADD)
+        *(float*)t.p = t.base + cs * v;
+    else if (t.wide)
+        *(float*)t.p = v;
+    else
+        *(E*)t.p = from_f32<E>(v);
+}
+
+// one result element through bias, activation and gate
+template <typename E, int EPI>
+__device__ __forceinline__ float finished(const pcb_linear_args& a, const Place& t, int n, float acc, float acc2, float bv, float bv2) {
     float v = acc + bv;
     if (EPI == PCB_EPI_STORE && (a.act | a.act2) && n < act_end(a))
         v = apply_act((a.act_split > 0 && n >= a.act_split) ? a.act2 : a.act, v, a.act_param);
     if (EPI == PCB_EPI_SILU_MUL) {
         v = gate_act(a.act, v) * (acc2 + bv2);
-        if (a.row_gate) v *= to_f32(((const E*)a.row_gate)[m * a.ld_row_gate]);
+        if (a.row_gate) v *= t.base;
     }
-    put<E, EPI>(a, m, n, v, cs);
+    return v;
 }
 
 }  // namespace pcb

@@ -354,6 +354,37 @@ def test_whole_cu_tiles_and_where_their_results_go(M, N, K):
     assert rel(y, base + cs * (z + bias.float())) < 2e-6
 
 
+@pytest.mark.parametrize("M,N", [(1, 70), (9, 64), (16, 130), (40, 100), (130, 260), (600, 2564), (2000, 2040)])
+@pytest.mark.parametrize("K", [4, 30, 36, 68, 516])
+def test_fp32_projections_at_every_tile_and_their_edges(M, N, K):
+    """fp32 rows read in 16-byte pieces (few rows straight into the matrix cores, more through LDS in each tile size) and element by element (K = 30):
+    ragged tiles both ways, k ranges that end inside a step; against sums in 64 bits: a k-step's rounding, sqrt(K) 2^-24 of the terms."""
+    b = B()
+    x, w, w2 = (rnd(r, K, seed=i, scale=K ** -0.25) for i, r in ((1, M), (2, N), (3, N)))
+    bias = rnd(N, seed=4)
+    z, z2 = x.double() @ w.double().T.contiguous(), x.double() @ w2.double().T.contiguous()
+    t = z + bias.double()
+    tol = 2e-6
+    y, perm = torch.zeros(M, N, device=DEV), torch.randperm(M, generator=torch.Generator().manual_seed(5)).to(DEV)
+    b.linear(x, w, y, M=M, bias=bias, act=b.ACT_RELU2, act_split=N // 2, row_dst=perm.to(torch.int32))
+    assert rel(y[perm], torch.cat([torch.relu(t[:, :N // 2]) ** 2, t[:, N // 2:]], dim=1)) < tol
+    gate = rnd(M, 3, seed=6)
+    b.linear(x, w, y, M=M, epilogue=b.EPI_SILU_MUL, w2=w2, bias=bias, act=b.ACT_RELU, row_gate=gate, ld_row_gate=3)
+    assert rel(y, torch.relu(t) * z2 * gate[:, :1].double()) < tol
+    cs, base = rnd(N, seed=7), rnd(M, N, seed=8)
+    y.copy_(base)
+    b.linear(x, w, y, M=M, epilogue=b.EPI_SCALE_ADD, col_scale=cs, bias=bias)
+    assert rel(y, base.double() + cs.double() * t) < tol
+    b.linear(x, w, y, M=M, epilogue=b.EPI_SCALE_ADD, base=base, col_scale=cs)
+    assert rel(y, base.double() + cs.double() * z) < tol
+    cut, third = N - 42, N - 10
+    y1, y2, y3 = torch.zeros(M, cut, device=DEV), torch.zeros(4, M, 8, device=DEV), torch.zeros(10, M, device=DEV)
+    b.linear(x, w, y1, M=M, split_n=cut, y2=y2, row_off2=perm * 8, head_dim2=8, head_stride2=M * 8, split_n3=third, y3=y3, row_off3=perm.clone(),
+             col_stride3=M)
+    heads = y2[:, perm].permute(1, 0, 2).reshape(M, 32)
+    assert rel(y1, z[:, :cut]) < tol and rel(heads, z[:, cut:third]) < tol and rel(y3[:, perm].T, z[:, third:]) < tol
+
+
 def test_router_scores_are_not_renormalised():
     b, T, n, top = B(), 9, 11, 4
     z = rnd(T, n, seed=3, scale=2.0)
