@@ -278,6 +278,18 @@ def test_attention_alone(dtype, H, G, D, window, n, first):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,G,D,window,n,first", [
+    (16, 4, 128, 100, 1070, 0),  # 64 tiles and more: eight waves share a tile's queries; windows that begin inside a 16-key piece of the band
+    (8, 2, 128, 0, 1035, 5),     # no window, the last tile of 6 rows
+    (4, 2, 40, 17, 1030, 0),     # a window of little more than a tile
+    (3, 1, 72, 64, 1100, 70),    # heads padded to the kernel's tier, a sequence that begins past the window
+])
+def test_attention_of_many_tiles(dtype, H, G, D, window, n, first):
+    got, want, _ = _attn_case(dtype, H, G, D, window, n, first)
+    assert rel(got, want) < tol(dtype, 2e-6, 1.5e-2)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("first", [0, 30, 63])           # in a prompt, in a portion, decoded alone
 def test_attention_window_edges_and_far_keys(dtype, first):
     H, G, D, window, n = 4, 2, 16, 25, 64
