@@ -192,9 +192,11 @@ __device__ __forceinline__ void store_group(const DenseParams& p, char* patch, i
                     const float cs_[4] = {w01[e][0], w01[e][2], w23[e][0], w23[e][2]}, sn_[4] = {w01[e][1], w01[e][3], w23[e][1], w23[e][3]};
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {
-                        // q*cos + rotate_half(q)*sin (llama2.py:208): the low half pairs with -high, the high half with +low
-                        a[k] = x0[k] * cs_[k] - x1[k] * sn_[k];
-                        c[k] = x1[k] * cs_[k] + x0[k] * sn_[k];
+                        // q*cos + rotate_half(q)*sin (llama2.py:208): the low half pairs with -high, the high half with +low.  Which product
+                        // stays unrounded is written out: left to the compiler, it changed with the code around it, and with it the last
+                        // bits of every cached key (which the layers behind it turn into 3e-4 of the logits).
+                        a[k] = fmaf(x0[k], cs_[k], -(x1[k] * sn_[k]));
+                        c[k] = fmaf(x1[k], cs_[k], x0[k] * sn_[k]);
                     }
                 }
                 h4 ah, al, ch, cl;

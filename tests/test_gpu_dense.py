@@ -126,6 +126,37 @@ def test_dense_split_k_with_workspace(M, N, K, two):
     assert torch.equal(y, y4)
 
 
+@pytest.mark.parametrize("two", [True, False])
+@pytest.mark.parametrize("M", [5, 130, 700])
+def test_dense_rotation_rounds_one_product(M, two):
+    """The fused q|k|v projection's rotation, bit for bit: x0 cos - round(x1 sin) and x1 cos + round(x0 sin) in one rounding each, on the sums
+    that the plain fp32 store of the same product gives."""
+    n = _n()
+    H, K = 2, 512
+    x, w = _inputs(M, 3 * H * 128, K, seed=M)
+    hi, lo = (torch.from_numpy(p).to(DEV) for p in _split(x))
+    lo, w = lo if two else None, torch.from_numpy(w).to(DEV)
+    ang = 6.28 * torch.rand((M, 64), generator=torch.Generator().manual_seed(M))
+    cs = torch.stack([torch.cos(ang), torch.sin(ang)], dim=-1).to(DEV)
+    q_hi, q_lo = (torch.zeros(M, H, 128, dtype=torch.float16, device=DEV) for _ in range(2))
+    k, v, k_lo, v_lo = (torch.zeros(H, M, 128, dtype=torch.float16, device=DEV) for _ in range(4))
+    n.gemm_dense_qkv_rope(hi, lo, w, K, cs, q_hi, q_lo, H * 128, k, v, H * M * 128, M * 128, 1, H, H, 128, M, 0, M, kv_lo=(k_lo, v_lo, H * M * 128, M * 128, 0))
+    y = torch.empty((M, 3 * H * 128), device=DEV)
+    n.gemm_dense(hi, lo, w, M, 3 * H * 128, K, n.EPI_STORE, y=y)
+    x = y.cpu().numpy().reshape(M, 3, H, 2, 64)
+    c, s = (cs.cpu().numpy()[:, None, None, :, i] for i in (0, 1))
+    x0, x1 = x[:, :2, :, 0], x[:, :2, :, 1]
+
+    def fma(a, b, z):                    # (64 bits of mantissa hold the 48 of the product: one rounding that counts)
+        return (a.astype(np.longdouble) * b.astype(np.longdouble) + z.astype(np.longdouble)).astype(np.float32)
+    a, b = fma(x0, c, -(x1 * s)), fma(x1, c, x0 * s)
+    both = np.concatenate([np.concatenate([a, b], axis=-1), x[:, 2:].reshape(M, 1, H, 128)], axis=1)
+    want_hi = both.astype(np.float16)
+    want_lo = (both - want_hi.astype(np.float32)).astype(np.float16)
+    for i, (h, l) in enumerate(((q_hi, q_lo), (k.transpose(0, 1), k_lo.transpose(0, 1)), (v.transpose(0, 1), v_lo.transpose(0, 1)))):
+        assert np.array_equal(h.cpu().numpy(), want_hi[:, i]) and np.array_equal(l.cpu().numpy(), want_lo[:, i])
+
+
 @pytest.mark.parametrize("M,inter,K", [(128, 128, 64), (300, 11008, 4096), (45, 344, 128), (1030, 1376, 512), (513, 13824, 5120)])
 def test_dense_silu_epilogue(M, inter, K):
     n = _n()
