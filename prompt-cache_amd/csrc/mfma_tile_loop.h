@@ -133,9 +133,10 @@ struct Loop {
     }
 };
 
-// How a grid of mb x nb tiles is cut into 8 rectangles, one per XCD (px row strips by 8 / px column strips of mh x nh tiles): fewest rounds
-// of an XCD's 32 CUs first, then fewest operand rows per K-step (row_cost for a tile's rows, col_cost for its columns) among 32 tiles that
-// run at a time.  Launch 8 mh nh workgroups.
+// How a grid of mb x nb tiles is dealt to the XCDs: cut into 8 rectangles (px row strips by 8 / px column strips of mh x nh tiles), fewest
+// rounds of an XCD's 32 CUs first, then fewest operand rows per K-step (row_cost for a tile's rows, col_cost for its columns) among 32 tiles
+// that run at a time.  Where no cut reaches the rounds of an even share, the tiles go out in 8 runs of mh, column by column (px = 0, nh = 1):
+// 3 x 81 tiles of 128 x 128 are 33 in a rectangle and 31 in a run (257 x 10272, K = 2048: 28.7 us in two rounds, 16.8 in one).  Launch 8 mh nh workgroups.
 struct Strips { int px, mh, nh; };
 static inline Strips strips(int mb, int nb, int row_cost, int col_cost) {
     Strips s{1, mb, (nb + 7) / 8};
@@ -145,7 +146,22 @@ static inline Strips strips(int mb, int nb, int row_cost, int col_cost) {
         const int64_t cost = (((int64_t)mh * nh + 31) / 32 << 32) + (int64_t)reach * row_cost + (int64_t)((32 + reach - 1) / reach) * col_cost;
         if (best < 0 || cost < best) { best = cost; s = Strips{px, mh, nh}; }
     }
+    const int64_t run = ((int64_t)mb * nb + 7) / 8;
+    if ((run + 31) / 32 < best >> 32) s = Strips{0, (int)run, 1};
     return s;
+}
+// the tile of workgroup `block` of such a launch; false: none
+static __device__ __forceinline__ bool tile_of(const Strips& s, int mb, int nb, int block, int& mi, int& ni) {
+    const int xcd = block & 7, slot = block >> 3;
+    if (s.px == 0) {
+        const int t = xcd * s.mh + slot;
+        mi = t % mb;
+        ni = t / mb;
+    } else {
+        mi = xcd % s.px * s.mh + slot % s.mh;
+        ni = xcd / s.px * s.nh + slot / s.mh;
+    }
+    return mi < mb && ni < nb;
 }
 
 }  // namespace mfma_tile

@@ -15,7 +15,7 @@ using namespace pcb;
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 
-struct Grid { int mb, nb, px, mh, nh; };
+struct Grid { int mb, nb; mfma_tile::Strips s; };
 
 // The wave's sums in `patch` to where they go: quad pc of rows pr, pr + RPI .. (R of them, RPI = 64 / LPR), row pr = row m0 of the result,
 // columns n .. n + 3 (n0: the wave's first).  First the patch is turned into results in place, then stored.  Short loops on purpose, and no
@@ -241,9 +241,8 @@ __global__ __launch_bounds__(256, 1) void linear_tile_kernel(const pcb_linear_ar
     __shared__ __attribute__((aligned(16))) char lds[S * L::kStage];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int mi = xcd % g.px * g.mh + slot % g.mh, ni = xcd / g.px * g.nh + slot / g.mh;
-    if (mi >= g.mb || ni >= g.nb) return;
+    int mi, ni;
+    if (!mfma_tile::tile_of(g.s, g.mb, g.nb, blockIdx.x, mi, ni)) return;
     const int m_lo = mi * BM, n_lo = ni * BN, K = a.K, N = a.N, nk = (K + 63) / 64;
 
     // staging: a lane's 16-byte chunk of an instruction's row as a 32-bit offset from the operand's K-step (the address is otherwise uniform)
@@ -327,7 +326,7 @@ int launch(const pcb_linear_args& a, hipStream_t stream) {
     using L = mfma_tile::Loop<MT, NT, S, 1>;
     const int mb = pcb_ceil_div(a.M, L::BM), nb = pcb_ceil_div(a.N, EPI == PCB_EPI_SILU_MUL ? L::BN / 2 : L::BN);
     const mfma_tile::Strips s = mfma_tile::strips(mb, nb, L::BM, L::BN);
-    hipLaunchKernelGGL((linear_tile_kernel<EPI, MT, NT, S>), dim3(8 * s.mh * s.nh), dim3(256), 0, stream, a, (Grid{mb, nb, s.px, s.mh, s.nh}));
+    hipLaunchKernelGGL((linear_tile_kernel<EPI, MT, NT, S>), dim3(8 * s.mh * s.nh), dim3(256), 0, stream, a, (Grid{mb, nb, s}));
     return pcb_check_launch("linear_tile_kernel");
 }
 

@@ -72,7 +72,7 @@ struct DenseParams {
     float* y; int64_t ldy;                                 // EPI_STORE / EPI_ADD
     _Float16* oh; _Float16* ol; int64_t ldo;               // EPI_SILU / EPI_GELU output planes
     int32_t M, N, K, mb, nb, nfeat;                        // nfeat: SiLU features (= N / 2)
-    int32_t px, mh, nh;                                    // XCD x owns M-blocks (x % px) mh .. and weight panels (x / px) nh ..
+    mfma_tile::Strips strips;                              // which tiles (M-block, weight panel) an XCD owns
     // split-K (EPI_STORE instantiation only): grid.y slices of `kper` K-steps, slice z stores its partial sums to
     // y + z * slab_stride; dense_reduce_kernel then adds the slabs in fixed order (launch_dense_splitk)
     int32_t kper; int64_t slab_stride;
@@ -246,9 +246,8 @@ __global__ __launch_bounds__(256, 1) void gemm_dense_kernel(const DenseParams p)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
     // block -> (M-block, weight panel), XCD-aware
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int mi = xcd % p.px * p.mh + slot % p.mh, ni = xcd / p.px * p.nh + slot / p.mh;
-    if (mi >= p.mb || ni >= p.nb) return;
+    int mi, ni;
+    if (!mfma_tile::tile_of(p.strips, p.mb, p.nb, blockIdx.x, mi, ni)) return;
     const int m0 = mi * BM;
     const int K = p.K, nkt = (K + BK - 1) / BK;          // K-steps of the whole product
     const int t0 = blockIdx.y * p.kper;                  // this slice's first K-step (kper = nkt without split-K)
@@ -376,9 +375,8 @@ int launch_dense_as(DenseParams& p, hipStream_t s, int kslices) {
     p.nb = (EPI == EPI_SILU) ? pc_ceil_div(p.nfeat, BN / 2) : pc_ceil_div(p.N, BN);
     const int nkt = pc_ceil_div(p.K, BK);
     p.kper = pc_ceil_div(nkt, kslices);
-    const mfma_tile::Strips g = mfma_tile::strips(p.mb, p.nb, (TWO ? 2 : 1) * BM, BN);
-    p.px = g.px; p.mh = g.mh; p.nh = g.nh;
-    hipLaunchKernelGGL((gemm_dense_kernel<2, EPI, TWO, NARROW, TALL>), dim3(8 * p.mh * p.nh, pc_ceil_div(nkt, p.kper)), dim3(256), 0, s, p);
+    p.strips = mfma_tile::strips(p.mb, p.nb, (TWO ? 2 : 1) * BM, BN);
+    hipLaunchKernelGGL((gemm_dense_kernel<2, EPI, TWO, NARROW, TALL>), dim3(8 * p.strips.mh * p.strips.nh, pc_ceil_div(nkt, p.kper)), dim3(256), 0, s, p);
     return pc_check_launch("gemm_dense_kernel");
 }
 

@@ -126,6 +126,19 @@ def test_dense_split_k_with_workspace(M, N, K, two):
     assert torch.equal(y, y4)
 
 
+@pytest.mark.parametrize("M,N,two", [(300, 20700, True), (257, 20736, False), (1000, 27640, False)])
+def test_dense_tiles_dealt_in_runs(M, N, two):
+    """Grids that no cut into rectangles spreads evenly over the XCDs (3 x 81, 4 x 108 and 8 x 108 tiles): every element is written, and right."""
+    n = _n()
+    x, w = _inputs(M, N, 72, seed=N)
+    hi, lo = (torch.from_numpy(p).to(DEV) for p in _split(x))
+    w, y = torch.from_numpy(w).to(DEV), torch.full((M, N), float("nan"), device=DEV)
+    n.gemm_dense(hi, lo if two else None, w, M, N, 72, n.EPI_STORE, y=y)
+    full = hi.double() + (lo.double() if two else 0.0)
+    bound = (2 if two else 1) * 72 * 2.0 ** -24 * full.abs() @ w.double().abs().T        # (a sum of planes x K products and additions)
+    assert bool(((y.double() - full @ w.double().T).abs() <= bound * 1.01).all())
+
+
 @pytest.mark.parametrize("two", [True, False])
 @pytest.mark.parametrize("M", [5, 130, 700])
 def test_dense_rotation_rounds_one_product(M, two):

@@ -354,6 +354,22 @@ def test_whole_cu_tiles_and_where_their_results_go(M, N, K):
     assert rel(y, base + cs * (z + bias.float())) < 2e-6
 
 
+@pytest.mark.parametrize("M,N", [(257, 10272), (300, 10200), (1100, 4980)])
+@pytest.mark.parametrize("K", [136, 1024])
+def test_whole_cu_tiles_dealt_in_runs(M, N, K):
+    """Grids that no cut into rectangles spreads evenly over the XCDs (3 x 81 and 3 x 80 tiles, the gated pair of 9 x 78): every element is
+    written, and right."""
+    b, bf = B(), torch.bfloat16
+    x, w = (rnd(r, K, dtype=bf, seed=i, scale=K ** -0.25) for i, r in ((1, M), (2, N)))
+    y = torch.full((M, N), float("nan"), device=DEV)
+    b.linear(x, w, y, M=M)
+    assert rel(y, matmul32(x, w)) < 2e-6
+    h, w2 = N // 2, w[N // 2:].contiguous()
+    g = torch.full((M, h), float("nan"), dtype=bf, device=DEV)
+    b.linear(x, w[:h].contiguous(), g, M=M, epilogue=b.EPI_SILU_MUL, w2=w2, act=b.ACT_RELU)
+    assert rel(g, torch.relu(y[:, :h]) * y[:, h:]) < 4e-3
+
+
 @pytest.mark.parametrize("M,N", [(1, 70), (9, 64), (16, 130), (40, 100), (130, 260), (600, 2564), (2000, 2040)])
 @pytest.mark.parametrize("K", [4, 30, 36, 68, 516])
 def test_fp32_projections_at_every_tile_and_their_edges(M, N, K):
