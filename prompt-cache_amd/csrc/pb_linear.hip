@@ -253,8 +253,10 @@ __device__ __forceinline__ void scale_frag<float>(Frag<float>& f, float s) {
     for (int e = 0; e < 8; ++e) f.v[e] *= s;
 }
 
-// SKW: waves of a workgroup (eight, or sixteen where few workgroups walk a long k range)
-template <typename E, int EPI, int SKW>
+// SKW: waves of a workgroup (eight, or sixteen where few workgroups walk a long k range).  LATE (bf16): where a result goes is worked out when it
+// is there, row by row.  Ahead of the products it hides its loads, but holds back the loads of the wave that stores, by 0.2-0.5 us a workgroup:
+// a gain as long as no workgroup waits for another one's place on the chip.
+template <typename E, int EPI, int SKW, bool LATE>
 __global__ __launch_bounds__(64 * SKW) void linear_skinny_kernel(pcb_linear_args a) {
     constexpr bool TWO = EPI == PCB_EPI_SILU_MUL;
     constexpr int CE = Tile<E>::CE;
@@ -292,17 +294,25 @@ __global__ __launch_bounds__(64 * SKW) void linear_skinny_kernel(pcb_linear_args
     const E* wrow = W + (int64_t)(b_ok ? n_b : 0) * a.ldw;
     const E* wrow2 = TWO ? W2 + (int64_t)(b_ok ? n_b : 0) * a.ldw : nullptr;
     const E* xrow = X + (int64_t)(a_ok ? (a.row_src ? a.row_src[m_a] : m_a) : 0) * a.ldx;
-    // (the wave that stores asks for everything the epilogue needs before the products)
+    // (the wave that stores asks for everything the epilogue needs before the products, or before it waits for the other waves)
+    constexpr bool ADD = EPI == PCB_EPI_SCALE_ADD;
     const int n_c = n_lo + l15 < N ? n_lo + l15 : N - 1;
     float bv = 0.0f, bv2 = 0.0f, cs = 0.0f;
     Place to[4] = {};
-    if (wave == 0) {
+    auto columns = [&] {
         if (a.bias) bv = to_f32(((const E*)a.bias)[n_c]);
         if (TWO && a.bias2) bv2 = to_f32(((const E*)a.bias2)[n_c]);
-        if (EPI == PCB_EPI_SCALE_ADD) cs = a.col_scale[n_c];
+        if (ADD) cs = a.col_scale[n_c];
+    };
+    auto places = [&] {
+        columns();
 #pragma unroll
-        for (int r = 0; r < 4; ++r) to[r] = place<E, EPI>(a, m_lo + 4 * group + r < m_hi ? m_lo + 4 * group + r : m_hi - 1, n_c);
-    }
+        for (int r = 0; r < 4; ++r) {
+            const int m = m_lo + 4 * group + r;
+            if (TWO || m < m_hi) to[r] = place<E, EPI>(a, m < m_hi ? m : m_hi - 1, n_c);
+        }
+    };
+    if (!LATE && wave == 0) places();
     const bool scaled = a.row_scale != nullptr;
     const float xs = (scaled && a_ok) ? a.row_scale[m_a] : 1.0f;
     Sum<E> sum, sum2;
@@ -329,6 +339,7 @@ __global__ __launch_bounds__(64 * SKW) void linear_skinny_kernel(pcb_linear_args
         if (TWO) sum2.chain(fa, load_frag(wrow2 + k0, group, b_ok ? K - k0 : 0, vec));
     }
     f4 acc = sum.total(), acc2 = sum2.total();
+    if (LATE && ADD && wave == 0) places();
     red[0][wave][lane] = acc;
     if (TWO) red[1][wave][lane] = acc2;
     __syncthreads();
@@ -342,9 +353,15 @@ __global__ __launch_bounds__(64 * SKW) void linear_skinny_kernel(pcb_linear_args
     }
     const int n = n_lo + l15;
     if (n >= N) return;
+    if (LATE && !ADD) columns();
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-        if (m_lo + 4 * group + r < m_hi) put<E, EPI>(to[r], finished<E, EPI>(a, to[r], n, acc[r], acc2[r], bv, bv2), cs);
+    for (int r = 0; r < 4; ++r) {
+        const int m = m_lo + 4 * group + r;
+        if (m < m_hi) {
+            if (LATE && !ADD) to[r] = place<E, EPI>(a, m, n);
+            put<E, EPI>(to[r], finished<E, EPI>(a, to[r], n, acc[r], acc2[r], bv, bv2), cs);
+        }
+    }
 }
 
 // ---- many rows: both panels travel to LDS by themselves ------------------------------------------------------------------------------
@@ -660,13 +677,21 @@ int dispatch(const pcb_linear_args& a, hipStream_t stream) {
     const bool big = rows > 64 && a.N > 64;
     if (rows <= 16) {
         const dim3 grid(pcb_ceil_div(a.N, 16), pcb_ceil_div(a.M, 16) + (a.n_groups > 0 ? a.n_groups : 0), a.n_batch > 0 ? a.n_batch : 1);
-        const bool deep = a.K >= 2048 && (int64_t)grid.x * grid.y * grid.z <= 192;
+        const int64_t groups = (int64_t)grid.x * grid.y * grid.z;
+        const bool deep = a.K >= 2048 && groups <= 192;
+        // LATE beyond three workgroups a CU, of the gated unit over few k beyond four.  bf16, us, 1 and 8 rows, ahead of the products / late:
+        // K = 1024, 12288 columns (768 workgroups) 6.5 / 6.5 and 7.4 / 7.9, 12800 8.2 / 7.6 and 9.6 / 9.4, 16384 9.0 / 7.7 and 12.1 / 9.5,
+        // 32000 15.6 / 13.9 and 18.8 / 17.6; K = 2048, 13600 columns 17.5 / 13.9 and 22.0 / 18.2; gated, 8 rows, 16384 columns 13.2 / 13.9;
+        // K = 2048, 1 row, 13600 columns 27.4 / 26.4.
+        const bool late = sizeof(E) == 2 && groups > (a.epilogue == PCB_EPI_SILU_MUL && a.K < 2048 ? 1024 : 768);
         auto go = [&](auto epi) {
             constexpr int EPI = decltype(epi)::value;
             if (deep)
-                hipLaunchKernelGGL((linear_skinny_kernel<E, EPI, 16>), grid, dim3(64 * 16), 0, stream, a);
+                hipLaunchKernelGGL((linear_skinny_kernel<E, EPI, 16, false>), grid, dim3(64 * 16), 0, stream, a);
+            else if (late)
+                hipLaunchKernelGGL((linear_skinny_kernel<E, EPI, 8, sizeof(E) == 2>), grid, dim3(64 * 8), 0, stream, a);
             else
-                hipLaunchKernelGGL((linear_skinny_kernel<E, EPI, 8>), grid, dim3(64 * 8), 0, stream, a);
+                hipLaunchKernelGGL((linear_skinny_kernel<E, EPI, 8, false>), grid, dim3(64 * 8), 0, stream, a);
         };
         switch (a.epilogue) {
             case PCB_EPI_STORE: go(std::integral_constant<int, PCB_EPI_STORE>{}); break;

@@ -354,6 +354,36 @@ def test_whole_cu_tiles_and_where_their_results_go(M, N, K):
     assert rel(y, base + cs * (z + bias.float())) < 2e-6
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N", [(1, 12288), (1, 12294), (9, 12300), (16, 20001), (16, 40)])
+def test_few_rows_on_either_side_of_the_late_form(dtype, M, N):
+    """Launches of up to and of more than 768 workgroups, where a row's place is worked out ahead of the products and behind them: rows scattered,
+    a bias and an activation over part of the columns, split-off heads and fp32 rows, gated rows, the accumulation in place and from a base."""
+    b, K = B(), 200
+    x, w, w2 = (rnd(r, K, dtype=dtype, seed=i, scale=K ** -0.25) for i, r in ((1, M), (2, N), (3, N)))
+    bias, z = rnd(N, dtype=dtype, seed=4), matmul32(x, w)
+    tol, t = (4e-3 if dtype == torch.bfloat16 else 2e-6), z + bias.float()
+    perm = torch.randperm(M, generator=torch.Generator().manual_seed(5)).to(DEV)
+    y = torch.zeros(M, N, dtype=dtype, device=DEV)
+    b.linear(x, w, y, M=M, row_dst=perm.to(torch.int32), bias=bias, act=b.ACT_RELU2, act_split=N - 13)
+    assert rel(y[perm], torch.cat([torch.relu(t[:, :N - 13]) ** 2, t[:, N - 13:]], dim=1)) < tol
+    y1, y2 = torch.zeros(M, N - 24, dtype=dtype, device=DEV), torch.zeros(3, M * 8, dtype=dtype, device=DEV)
+    b.linear(x, w, y1, M=M, split_n=N - 24, y2=y2, row_off2=perm * 8, head_dim2=8, head_stride2=M * 8)
+    assert rel(y1, z[:, :N - 24]) < tol and rel(y2.view(3, M, 8)[:, perm].permute(1, 0, 2).reshape(M, 24), z[:, N - 24:]) < tol
+    y2 = torch.zeros(M, 24, device=DEV)
+    b.linear(x, w, y1, M=M, split_n=N - 24, y2=y2, y2_f32=True, head_stride2=24)
+    assert rel(y1, z[:, :N - 24]) < tol and rel(y2, z[:, N - 24:]) < 2e-6
+    gate, g = rnd(M, 3, dtype=dtype, seed=6), torch.zeros(M, N, dtype=dtype, device=DEV)
+    b.linear(x, w, g, M=M, epilogue=b.EPI_SILU_MUL, w2=w2, act=b.ACT_RELU, row_gate=gate, ld_row_gate=3)
+    assert rel(g, torch.relu(z) * matmul32(x, w2) * gate[:, :1].float()) < tol
+    cs, y, base = rnd(N, seed=7), rnd(M, N, seed=8), rnd(M, N, seed=9)
+    want = y + cs * z
+    b.linear(x, w, y, M=M, epilogue=b.EPI_SCALE_ADD, col_scale=cs)
+    assert rel(y, want) < 2e-6
+    b.linear(x, w, y, M=M, bias=bias, epilogue=b.EPI_SCALE_ADD, base=base, col_scale=cs)
+    assert rel(y, base + cs * t) < 2e-6
+
+
 @pytest.mark.parametrize("M,N", [(257, 10272), (300, 10200), (1100, 4980)])
 @pytest.mark.parametrize("K", [136, 1024])
 def test_whole_cu_tiles_dealt_in_runs(M, N, K):
