@@ -807,12 +807,12 @@ def attn_latent(q: torch.Tensor, tiles: torch.Tensor, n_rows: int, cache: torch.
                 vdim: int, scale: float, out: torch.Tensor, *, window: int = 0, sink=None, gate=None, ldg: int = 0, n_splits: int = 1,
                 part=None) -> None:
     """``q`` E [rows, H * dim]; ``cache``: slots of rows whose first ``vdim`` columns are the value; ``tiles`` int32 {slot, position, 1,
-    flat row} per row; ``part`` fp32 of ``attn_softmax_part(rows, H, n_splits, vdim)`` floats when the keys are cut into runs."""
+    flat row} per row; ``part`` fp32 of ``attn_softmax_part(n_rows, H, n_splits, vdim)`` floats when the keys are cut into runs."""
     _want(tiles, torch.int32, "attn_latent tiles"); _want(sink, torch.float32, "attn_latent sink"); _want(part, torch.float32, "attn_latent part")
     assert q.dtype == cache.dtype == out.dtype and q.is_contiguous() and out.is_contiguous() and cache.is_cuda
     assert tiles.numel() >= 4 * n_rows and q.shape[-1] == H * dim and out.shape[-1] == H * vdim and (sink is None or sink.numel() >= H)
     assert gate is None or (gate.dtype == q.dtype and ldg >= H)
-    assert n_splits <= 1 or (part is not None and part.numel() >= attn_softmax_part(out.shape[0], H, n_splits, vdim))
+    assert n_splits <= 1 or (part is not None and part.numel() >= attn_softmax_part(n_rows, H, n_splits, vdim))
     a = AttnLatentArgs(C.sizeof(AttnLatentArgs), _code(q), _p(q), q.shape[-1], _p(tiles), n_rows, _p(cache), slot_stride, row_stride, H, dim, vdim,
                        float(scale), int(window), _p(sink), _p(gate), ldg, _p(out), out.shape[-1], n_splits, _p(part))
     check(load().pcb_attn_latent(C.byref(a), _stream()), "pcb_attn_latent")

@@ -413,7 +413,7 @@ class FivesunHIP(SlotModel):
             B.linear(P, lw["w_abs"], qa, M=n, row_src=rows, row_dst=rows, n_batch=H, ldx=N, x_batch_stride=DR, ldy=H * CR, y_batch_stride=CR)
             ol = self._mat("mix_out", T, H * C, E)
             splits = self._splits(n, -(-H // 16), min(arena.cap, l.mask or arena.cap))
-            part = self._scratch("attn_part", B.attn_softmax_part(T, H, splits, C), torch.float32) if splits > 1 else None
+            part = self._scratch("attn_part", B.attn_softmax_part(n, H, splits, C), torch.float32) if splits > 1 else None
             B.attn_latent(qa, f_tiles, n, plane, arena.slot_stride(i), CR, H, CR, C, l.scale, ol, window=l.mask, n_splits=splits, part=part)
             ov = self._mat("mix_o32", T, HV, torch.float32)
             B.linear(ol, lw["w_uv"], ov, M=n, row_src=rows, row_dst=rows, n_batch=H, ldx=H * C, x_batch_stride=C, ldy=HV, y_batch_stride=Dv)

@@ -330,7 +330,7 @@ class PikadraHIP(SlotModel):
         B.linear(q, lw["w_abs"], qa, M=n, row_src=rows, row_dst=rows, n_batch=H, ldx=H * DR, x_batch_stride=DR, ldy=H * CR, y_batch_stride=CR)
         ol = self._mat("o_latent", T, H * C, E)
         splits = self._splits(arena, n, -(-H // 16))
-        part = self._scratch("attn_part", B.attn_softmax_part(T, H, splits, C), torch.float32) if splits > 1 else None
+        part = self._scratch("attn_part", B.attn_softmax_part(n, H, splits, C), torch.float32) if splits > 1 else None
         B.attn_latent(qa, tiles, n, arena.planes[r], arena.slot_stride(r), CR, H, CR, C, l.scale, ol, sink=lw["sink"], gate=gate, ldg=ldg,
                       n_splits=splits, part=part)
         B.linear(ol, lw["w_uv"], A, M=n, row_src=rows, row_dst=rows, n_batch=H, ldx=H * C, x_batch_stride=C, ldy=ldo, y_batch_stride=Dv)

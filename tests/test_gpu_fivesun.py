@@ -502,6 +502,24 @@ def test_tiled_and_single_rows_beside_one_another(dtype, n):
         assert rel(mine, want) < tol(dtype, 3e-5, 8e-2), i
 
 
+def test_runs_of_a_decoding_row_beside_a_prompt():
+    """One row that decodes over 400 keys of an unwindowed latent layer, cut into runs, beside a prompt of 300: the runs' scratch holds
+    that row's, not the step's, and both requests get what the oracle says."""
+    s = FivesunShape(vocab_size=90, hidden_size=64, norm_eps=1e-6, embed_scale=8.0, layers=[lat(4, 40, 24, 32, 48, mask=0, ff=48)])
+    w = W.make_fivesun_weights(s, seed=4)
+    from promptcache_amd.model.fivesun_hip import FivesunHIP
+    m = FivesunHIP(s, w, device=DEV, dtype=torch.float32)
+    seqs, new = [toks(401, s.vocab_size, seed=60), toks(300, s.vocab_size, seed=61)], [1, 300]
+    ar = m.new_arena(2, 800)
+    slots = [ar.alloc() for _ in seqs]
+    m.forward_rows(ar, slots[:1], [seqs[0][:-1]])
+    got = m.forward_rows(ar, slots, [q[-k:] for q, k in zip(seqs, new)], [list(range(k)) for k in new])
+    splits = m._splits(1, 1, 800)
+    assert splits > 1 and m._buf["attn_part"].numel() <= max(1024, 2 * B().attn_softmax_part(1, 4, splits, 48))
+    for g, q, k in zip((got[:1], got[1:]), seqs, new):
+        assert rel(g, oracle_logits(s, w, q)[0][-k:]) < 3e-5
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("graphs", [True, False])
 def test_unequal_batches_reused_slots_and_states(dtype, graphs):
