@@ -74,6 +74,7 @@ class FivesunHIP(SlotModel):
     # live rows costs what 16 single rows cost (one pass over the keys per head against one per row and 16 heads).
     PROMPT_ROWS = int(os.environ.get("PC_FS_PROMPT_ROWS", "16"))
     REBUILD_RATIO = 64      # ... but folds its queries, instead of rebuilding the keys, if it brings less than a 64th of what they number
+    REBUILD_BYTES = 256 << 20   # rebuilt keys and values that lie in memory at a time: beyond it (32 k rows of 16 heads of 128 + 128) heads take turns
 
     def __init__(self, shape: FivesunShape, weights: Dict[str, torch.Tensor], device="cuda:0", dtype=torch.bfloat16,
                  decode_headroom: int = 256):
@@ -420,12 +421,19 @@ class FivesunHIP(SlotModel):
             B.gated_norm(ov, None, gate, N, og, self.config.norm_eps, T)
         if tiled:
             # (after the others: their gate runs over all rows)
-            flat, M, NK = plane.view(-1, CR), tb["kv_rows"].numel(), H * (D + Dv)
-            kv = self._mat("kv_rows", M, NK, E)
-            B.linear(flat, lw["w_kv"], kv, M=M, row_src=tb["kv_rows"], ldx=CR)
-            B.attn_prompt(q, tb["l_tiles"], tb["l_tiles"].numel() // 4, tb["tile"], kv, (NK, D), kv[:, H * D:], (NK, Dv), H, H, DR, Dv, l.scale, og,
-                          ldo=HV, k_tail=flat[:, C:] if Rd else None, tail_row_stride=CR, tail_rows=tb["kv_rows"], tail_dim=Rd, window=l.mask,
-                          gate=gate, ldg=N, gate_cols=True)
+            flat, M, ew = plane.view(-1, CR), tb["kv_rows"].numel(), D + Dv
+            Hs = max(1, min(H, self.REBUILD_BYTES // (M * ew * plane.element_size())))
+            kv = self._mat("kv_rows", M, Hs * ew, E)
+            for h0 in range(0, H, Hs):
+                n_h = min(Hs, H - h0)
+                if n_h == H:
+                    B.linear(flat, lw["w_kv"], kv, M=M, row_src=tb["kv_rows"], ldx=CR)
+                else:
+                    for at, w in ((0, lw["w_kv"][h0 * D:(h0 + n_h) * D]), (n_h * D, lw["w_kv"][H * D + h0 * Dv:H * D + (h0 + n_h) * Dv])):
+                        B.linear(flat, w, kv[:, at:], M=M, row_src=tb["kv_rows"], ldx=CR, ldy=Hs * ew)
+                B.attn_prompt(q[:, h0 * DR:], tb["l_tiles"], tb["l_tiles"].numel() // 4, tb["tile"], kv, (Hs * ew, D), kv[:, n_h * D:], (Hs * ew, Dv),
+                              n_h, n_h, DR, Dv, l.scale, og[:, h0 * Dv:], ldq=HQ, ldo=HV, k_tail=flat[:, C:] if Rd else None, tail_row_stride=CR,
+                              tail_rows=tb["kv_rows"], tail_dim=Rd, window=l.mask, gate=gate[:, h0 * Dv:], ldg=N, gate_cols=True)
         B.linear(og, lw["wo"], y, M=T)
         return P[:, HQ + CR + HV:], N
 

@@ -502,6 +502,31 @@ def test_tiled_and_single_rows_beside_one_another(dtype, n):
         assert rel(mine, want) < tol(dtype, 3e-5, 8e-2), i
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("dim,rot,vdim", [(40, 24, 32), (13, 6, 9)])
+def test_rebuilt_heads_take_turns_within_their_scratch(dtype, dim, rot, vdim):
+    """The scratch of rebuilt keys and values is as large as it may be, whatever the context: with room for all five heads, for two (the last
+    turn has one) and for less than one, a prompt and what goes on behind it get the same numbers."""
+    s = FivesunShape(vocab_size=90, hidden_size=64, norm_eps=1e-6, embed_scale=8.0, layers=[lat(5, dim, rot, vdim, 48, mask=0, ff=48)])
+    w = W.make_fivesun_weights(s, seed=4)
+    from promptcache_amd.model.fivesun_hip import FivesunHIP
+    tokens = toks(200, s.vocab_size, seed=62)
+    head = 224 * (dim + vdim) * (2 if dtype == torch.bfloat16 else 4)              # 200 rows in whole blocks of 32
+    want = None
+    for room, heads in ((1 << 20, 5), (2 * head, 2), (1, 1)):
+        m = FivesunHIP(s, w, device=DEV, dtype=dtype)
+        m.REBUILD_BYTES = room
+        ar = m.new_arena(1, 256)
+        slot = ar.alloc()
+        m.forward_rows(ar, [slot], [tokens[:100]])
+        got = m.forward_rows(ar, [slot], [tokens[100:]], [list(range(100))])
+        assert m._buf["kv_rows"].numel() <= max(1024, 2 * 224 * heads * (dim + vdim))
+        want = got if want is None else want
+        assert rel(got, want) < tol(dtype, 1e-6, 2e-2)
+    if dtype == torch.float32:
+        assert rel(got, oracle_logits(s, w, tokens)[0][100:]) < 3e-5
+
+
 def test_runs_of_a_decoding_row_beside_a_prompt():
     """One row that decodes over 400 keys of an unwindowed latent layer, cut into runs, beside a prompt of 300: the runs' scratch holds
     that row's, not the step's, and both requests get what the oracle says."""
