@@ -206,25 +206,30 @@ class FivesunHIP(SlotModel):
             want_rows = np.arange(T, dtype=np.int32)
         reqs = np.asarray([(s, s0, c, int(row0[b])) for b, (s, s0, c) in enumerate(zip(slots, starts, counts))], dtype=np.int32)
 
-        def row_tiles(rows):
-            return np.stack([st.row_slot[rows], st.row_pos[rows], np.ones(rows.size, np.int64), rows], axis=1).astype(np.int32)
-
-        def rows_of(which):
-            return np.concatenate([np.arange(row0[b], row0[b + 1]) for b in which]).astype(np.int32) if which else np.zeros(0, np.int32)
-
-        # attention: tiles of neighbouring queries for requests that bring many tokens, single rows for the others
-        big = [b for b, c in enumerate(counts) if c >= self.PROMPT_ROWS]
+        # attention: tiles of neighbouring queries for requests that bring many tokens, single rows for the others.  (A captured step has single
+        # rows only: its launches are those of any step of as many requests.)
+        big = [] if graphed else [b for b, c in enumerate(counts) if c >= self.PROMPT_ROWS]
         # the oldest key that the rebuilding layers need (a whole number of the kernel's blocks of keys)
-        oldest = [max(0, s0 - self._reach + 1) // 64 * 64 if self._reach else 0 for s0 in starts]
+        oldest = [max(0, s0 - self._reach + 1) // 64 * 64 if self._reach else 0 for s0 in starts] if big else []
         rebuilt = [b for b in big if self._rebuilds and starts[b] + counts[b] - oldest[b] <= self.REBUILD_RATIO * counts[b]]
         tile = 64
         if self.dtype == torch.bfloat16 and sum(-(-counts[b] // 128) for b in big) * self._max_heads >= 512:
             tile = 128
+        none = np.zeros(0, np.int32)
+        rows = np.empty((T, 4), dtype=np.int32)                 # every row by itself
+        rows[:, 0], rows[:, 1], rows[:, 2], rows[:, 3] = st.row_slot, st.row_pos, 1, np.arange(T, dtype=np.int32)
+
+        def others(which):                                      # the flat rows of the other requests
+            if not which:
+                return slice(None)
+            mine = np.zeros(R, dtype=bool)
+            mine[which] = True
+            return np.flatnonzero(~np.repeat(mine, counts))
 
         def tiles_of(which, base):
             t = [(base[b], starts[b] + q, min(tile, counts[b] - q), int(row0[b]) + q) for b in which for q in range(0, counts[b], tile)]
             t.sort(key=lambda t: t[1] + t[2])     # (longer contexts behind the shorter ones: the kernel starts from the last tile)
-            return np.asarray(t, dtype=np.int32).reshape(-1, 4)
+            return np.asarray(t, dtype=np.int32).reshape(-1)
 
         kv_rows, base, at = [], {}, 0
         for b in rebuilt:
@@ -236,9 +241,7 @@ class FivesunHIP(SlotModel):
             at += src.size
         if rebuilt and arena.slots * cap >= 1 << 31:
             raise ValueError("more than 2^31 cached rows in one plane")
-        s_rows = rows_of([b for b in range(R) if b not in set(big)])
-        f_rows = rows_of([b for b in range(R) if b not in set(rebuilt)])
-        every = np.arange(T, dtype=np.int32)
+        f_rows = others(rebuilt)
         # segments of the matrix memories' prefill (only when some request brings more than SEGMENT tokens)
         seg_a = seg_c = chains = np.zeros((0, 4), np.int32)
         seg_end = np.zeros(0, np.int32)
@@ -254,22 +257,29 @@ class FivesunHIP(SlotModel):
             chains = np.asarray(ch, dtype=np.int32)
             seg_end = np.full(len(sa), -1, dtype=np.int32)  # a request's last segment leaves the slot's new state
             seg_end[chains[:, 2] + chains[:, 3] - 1] = chains[:, 0]
-        offs = np.stack([st.row_slot * (g * cap * d) + st.row_pos * d for g, d in self._sigs]) if self._sigs else np.zeros((0, T), np.int64)
-        tables = dict(ids=st.ids, pos=st.row_pos.astype(np.int32), want=want_rows, reqs=reqs, p_tiles=tiles_of(big, slots),
-                      s_tiles=row_tiles(s_rows), l_tiles=tiles_of(rebuilt, base), kv_rows=np.concatenate(kv_rows) if kv_rows else every[:0],
-                      f_tiles=row_tiles(f_rows), f_rows=f_rows if rebuilt else every[:0],
-                      # every row by itself, for layers that fold all rows; tiles of 16 queries, for heads too wide for the others
-                      a_tiles=row_tiles(every) if rebuilt and self._folds else every[:0],
-                      w_tiles=np.asarray([(s, s0 + q, min(16, c - q), int(row0[b]) + q) for b, (s, s0, c) in enumerate(zip(slots, starts, counts))
-                                          for q in range(0, c, 16)], dtype=np.int32).reshape(-1, 4) if self._wide else every[:0],
-                      seg_a=seg_a, seg_c=seg_c, chains=chains, seg_end=seg_end)
+        tables = dict(ids=st.ids, pos=rows[:, 1], want=want_rows, reqs=reqs, s_tiles=rows[others(big)])
+        if big:
+            tables.update(p_tiles=tiles_of(big, slots))
+        if rebuilt:
+            # f_: the rows that fold their queries; a_tiles: every row, for layers that fold them all
+            tables.update(l_tiles=tiles_of(rebuilt, base), kv_rows=np.concatenate(kv_rows), f_rows=rows[f_rows, 3], a_tiles=rows if self._folds else none)
+        if rebuilt != big:
+            tables.update(f_tiles=rows[f_rows])
+        if self._wide:                             # tiles of 16 queries, for heads too wide for the others
+            tables.update(w_tiles=np.asarray([(s, s0 + q, min(16, c - q), int(row0[b]) + q) for b, (s, s0, c) in enumerate(zip(slots, starts, counts))
+                                              for q in range(0, c, 16)], dtype=np.int32))
+        if seg_end.size:
+            tables.update(seg_a=seg_a, seg_c=seg_c, chains=chains, seg_end=seg_end)
         sizes = {k: v.size for k, v in tables.items()}
         n32 = sum(sizes.values())
         o64 = (n32 * 4 + 7) // 8 * 8
         # one block: int32 tables, then int64 cache offsets
-        blob = np.empty(o64 + offs.size * 8 + 8, dtype=np.uint8)
-        blob[:n32 * 4].view(np.int32)[:] = np.concatenate([v.reshape(-1) for v in tables.values()])
-        blob[o64:o64 + offs.size * 8].view(np.int64)[:] = offs.reshape(-1)
+        n_off = len(self._sigs) * T
+        blob = np.empty(o64 + n_off * 8 + 8, dtype=np.uint8)
+        np.concatenate([v.reshape(-1) for v in tables.values()], out=blob[:n32 * 4].view(np.int32))
+        offs = blob[o64:o64 + n_off * 8].view(np.int64).reshape(len(self._sigs), T)
+        for k, (g, d) in enumerate(self._sigs):
+            np.add(st.row_slot * (g * cap * d), st.row_pos * d, out=offs[k])
         dims = dict(T=T, R=R, n_want=int(want_rows.size), n32=n32, o64=o64, sizes=sizes, tile=tile)
         res = self._decode_graphed(arena, blob, dims) if graphed else None
         if res is None:
@@ -284,10 +294,14 @@ class FivesunHIP(SlotModel):
 
     def _tables(self, dblob, d):
         i32 = dblob[:d["n32"] * 4].view(torch.int32)
-        at, out = 0, dict(tile=d["tile"], n_seg=d["sizes"]["seg_end"], n_chains=d["sizes"]["chains"] // 4)
-        for name, n in d["sizes"].items():
+        sizes = d["sizes"]
+        at, out = 0, dict(tile=d["tile"], n_seg=sizes.get("seg_end", 0), n_chains=sizes.get("chains", 0) // 4)
+        for name, n in sizes.items():
             out[name] = i32[at:at + n]
             at += n
+        for name in ("p_tiles", "l_tiles", "kv_rows", "f_rows", "a_tiles", "w_tiles"):
+            out.setdefault(name, i32[:0])
+        out.setdefault("f_tiles", out["s_tiles"])  # (the same rows, unless some request is tiled without being rebuilt)
         no = len(self._sigs)
         out["offs"] = dblob[d["o64"]:d["o64"] + no * d["T"] * 8].view(torch.int64).view(no, d["T"])
         return out
@@ -431,9 +445,10 @@ class FivesunHIP(SlotModel):
                 else:
                     for at, w in ((0, lw["w_kv"][h0 * D:(h0 + n_h) * D]), (n_h * D, lw["w_kv"][H * D + h0 * Dv:H * D + (h0 + n_h) * Dv])):
                         B.linear(flat, w, kv[:, at:], M=M, row_src=tb["kv_rows"], ldx=CR, ldy=Hs * ew)
-                B.attn_prompt(q[:, h0 * DR:], tb["l_tiles"], tb["l_tiles"].numel() // 4, tb["tile"], kv, (Hs * ew, D), kv[:, n_h * D:], (Hs * ew, Dv),
-                              n_h, n_h, DR, Dv, l.scale, og[:, h0 * Dv:], ldq=HQ, ldo=HV, k_tail=flat[:, C:] if Rd else None, tail_row_stride=CR,
-                              tail_rows=tb["kv_rows"], tail_dim=Rd, window=l.mask, gate=gate[:, h0 * Dv:], ldg=N, gate_cols=True)
+                qh, oh, gh = (q, og, gate) if not h0 else (q[:, h0 * DR:], og[:, h0 * Dv:], gate[:, h0 * Dv:])
+                B.attn_prompt(qh, tb["l_tiles"], tb["l_tiles"].numel() // 4, tb["tile"], kv, (Hs * ew, D), kv[:, n_h * D:], (Hs * ew, Dv),
+                              n_h, n_h, DR, Dv, l.scale, oh, ldq=HQ, ldo=HV, k_tail=flat[:, C:] if Rd else None, tail_row_stride=CR,
+                              tail_rows=tb["kv_rows"], tail_dim=Rd, window=l.mask, gate=gh, ldg=N, gate_cols=True)
         B.linear(og, lw["wo"], y, M=T)
         return P[:, HQ + CR + HV:], N
 

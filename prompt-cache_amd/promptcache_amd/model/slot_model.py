@@ -74,7 +74,8 @@ class SlotModel:
         return t
 
     def _mat(self, name: str, rows: int, cols: int, dtype) -> torch.Tensor:
-        return self._scratch(name, max(rows, 1) * cols, dtype)[:max(rows, 1) * cols].view(max(rows, 1), cols)
+        rows = max(rows, 1)
+        return self._scratch(name, rows * cols, dtype).as_strided((rows, cols), (cols, 1))
 
     # ---- one-token steps as captured graphs (models whose step is ``_run(arena, device tables, dims, logits)``) ------------------
     def _decode_graphed(self, arena, blob, d):

@@ -94,6 +94,65 @@ def test_arena_serial_numbers_never_repeat():
         del ar
 
 
+def step_tables(m, arena, slots, tokens):
+    """The tables a step of model ``m`` hands its launches, as lists (nothing is launched), and what its block is made of."""
+    seen = []
+    m._run = lambda arena, blob, dims, logits, *_: seen.append((m._tables(blob, dims), dims)) or logits
+    m._decode_graphed = lambda arena, blob, dims: m._run(arena, torch.from_numpy(blob), dims, torch.zeros(dims["T"], m.V))
+    m.forward_rows(arena, slots, tokens)
+    (tb, dims), = seen
+    return {k: v.tolist() if torch.is_tensor(v) else v for k, v in tb.items()}, dims
+
+
+@pytest.mark.parametrize("prompt_rows", [16, 1])
+@pytest.mark.parametrize("news", [[1], [1, 1, 1], [16], [2, 15, 3], [17, 1, 40], [1, 200, 16, 3], [16, 64, 130]])
+def test_step_tables_name_every_row_once(news, prompt_rows):
+    """Which launch of a step takes which row, against the rule in plain words: requests of 16 new tokens and more in tiles, rebuilt where a 64th of
+    their window is new, the others row by row -- and single rows only in a step that may be captured, whatever the knobs say."""
+    from promptcache_amd.model.fivesun_hip import FivesunHIP
+    lat = dict(heads=2, kv_heads=1, kv_rank=24, rot_dim=8, rot_dims=8, vdim=16)
+    s = FivesunShape(vocab_size=50, hidden_size=32, norm_eps=1e-6, layers=[
+        FivesunLayer("attention", heads=2, kv_heads=1, dim=16, vdim=16, mask=64, rot_dims=16), FivesunLayer("latent_attention", dim=16, mask=600, **lat),
+        FivesunLayer("latent_attention", dim=256, mask=80, **lat), FivesunLayer("attention", heads=1, kv_heads=1, dim=264, vdim=8, rot_dims=0)])
+    m = FivesunHIP(s, W.make_fivesun_weights(s, seed=1), device="cpu", dtype=torch.float32)
+    m.PROMPT_ROWS = prompt_rows
+    cap, starts = 4096, [1700, 0, 333, 70][:len(news)]
+    ar = m.new_arena(5, cap)
+    slots = [ar.alloc() for _ in range(5)][5 - len(news):]
+    for b, n in enumerate(starts):
+        ar.lengths[slots[b]] = n
+    tb, dims = step_tables(m, ar, slots, [[7] * n for n in news])
+    T, flat = sum(news), [sum(news[:b]) for b in range(len(news))]
+    row = {flat[b] + i: [slots[b], starts[b] + i, 1, flat[b] + i] for b in range(len(news)) for i in range(news[b])}
+    one = all(n == 1 for n in news)
+    big = [] if one else [b for b, n in enumerate(news) if n >= prompt_rows]
+    low = {b: max(0, starts[b] - 599) // 64 * 64 for b in big}
+    rebuilt = [b for b in big if starts[b] + news[b] - low[b] <= 64 * news[b]]
+    single = [r for b in range(len(news)) if b not in big for r in range(flat[b], flat[b] + news[b])]
+    folded = [r for b in range(len(news)) if b not in rebuilt for r in range(flat[b], flat[b] + news[b])]
+
+    def quads(t):
+        return [t[i:i + 4] for i in range(0, len(t), 4)]
+    assert [tb["pos"][r] for r in range(T)] == [row[r][1] for r in range(T)] and len(tb["ids"]) == T
+    assert quads(tb["s_tiles"]) == [row[r] for r in single] and quads(tb["f_tiles"]) == [row[r] for r in folded]
+    assert tb["f_rows"] == (folded if rebuilt else []) and quads(tb["a_tiles"]) == ([row[r] for r in range(T)] if rebuilt else [])
+    assert sorted(quads(tb["w_tiles"])) == sorted([slots[b], starts[b] + q, min(16, news[b] - q), flat[b] + q] for b in range(len(news)) for q in range(0, news[b], 16))
+    # tiles: every row of theirs once, its own request's; rebuilt rows hold what the window can see of it
+    for tiles, which in ((quads(tb["p_tiles"]), big), (quads(tb["l_tiles"]), rebuilt)):
+        got = sorted(r for t in tiles for r in range(t[3], t[3] + t[2]))
+        assert got == [r for b in which for r in range(flat[b], flat[b] + news[b])] and all(0 < t[2] <= tb["tile"] for t in tiles)
+        assert all(row[t[3]][1] == t[1] for t in tiles)
+    assert all(t[0] == row[t[3]][0] for t in quads(tb["p_tiles"]))
+    for base, p0, n, r in quads(tb["l_tiles"]):
+        b = next(b for b in rebuilt if flat[b] <= r < flat[b] + news[b])
+        assert [tb["kv_rows"][base + j] for j in range(low[b], p0 + n)] == [slots[b] * cap + j for j in range(low[b], p0 + n)]
+    assert [x for x in tb["offs"]] == [[row[r][0] * g * cap * d + row[r][1] * d for r in range(T)] for g, d in m._sigs]
+    if one:                                        # launches of a captured step do not depend on how long its requests are
+        for b in range(len(news)):
+            ar.lengths[slots[b]] = 5 + b
+        assert step_tables(m, ar, slots, [[7] * n for n in news])[1] == dims
+
+
 def test_frequency_tables_follow_the_oracle():
     from promptcache_amd.model.fivesun_hip import rotary_frequencies
     fr, mag = rotary_frequencies(30000.0, 12, 3.0)
