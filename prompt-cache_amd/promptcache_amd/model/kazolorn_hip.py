@@ -271,15 +271,13 @@ class KazolornHIP(SlotModel):
         ent["dev"].copy_(ent["host"], non_blocking=True)
         ent["copied"].record()
         if ent["graph"] is None:
-            from .llama_hip import prime_graph_capture
+            from .llama_hip import graph_capture
             saved, self._buf = self._buf, ent["bufs"]             # the graph owns its scratch: later, larger steps may regrow the shared one
             try:
                 args = (arena, T, ent["dev"], n32, o64, sigs, None, T, T, T, cap, ent["logits"])
                 self._run(*args)                                  # eager first: sizes every scratch buffer, and is this step's result
                 torch.cuda.synchronize()
-                prime_graph_capture(self.device)
-                g = torch.cuda.CUDAGraph()
-                with torch.cuda.graph(g):
+                with graph_capture(self.device) as g:
                     self._run(*args)
                 ent["graph"] = g
             finally:

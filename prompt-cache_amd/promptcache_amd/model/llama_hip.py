@@ -24,6 +24,8 @@ There is no CPU / eager fallback: without the HIP extension this module raises.
 """
 from __future__ import annotations
 
+import contextlib
+import gc
 import math
 import os
 from dataclasses import dataclass
@@ -107,6 +109,23 @@ def prime_graph_capture(device) -> None:
         with torch.cuda.graph(g):
             t.add_(1.0)
     _GRAPH_RNG_PRIMED[idx] = (g, t)
+
+
+@contextlib.contextmanager
+def graph_capture(device):
+    """The block's launches, captured into the graph it is given.  The collector of cyclic garbage stays out meanwhile: whatever graphs,
+    events and pools of memory it found would be released in the middle of the capture, which the runtime forbids -- in a destructor, so the
+    process ends."""
+    prime_graph_capture(device)
+    g = torch.cuda.CUDAGraph()
+    on = gc.isenabled()
+    gc.disable()
+    try:
+        with torch.cuda.graph(g):
+            yield g
+    finally:
+        if on:
+            gc.enable()
 
 
 def lw0_fp16(layers) -> bool:
@@ -1229,9 +1248,7 @@ class LlamaHIP:
             # one eager pass first (loads code objects / sizes the allocator), then capture
             run()
             torch.cuda.synchronize()
-        prime_graph_capture(self.device)
-        g = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(g):
+        with graph_capture(self.device) as g:
             out = run()
         ent[0], ent[2] = g, out
 
@@ -1365,9 +1382,7 @@ class LlamaHIP:
         # writes again and does not touch the loop state
         self._forward_skinny(st["ids"], st["pos"], st["past"], arena, 1, 1, past_len, False, None)
         torch.cuda.synchronize()
-        prime_graph_capture(self.device)
-        g = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(g):
+        with graph_capture(self.device) as g:
             out = self._forward_skinny(st["ids"], st["pos"], st["past"], arena, 1, 1, past_len, False, None)
             n.greedy_advance(out, V, st["ids"], st["pos"], st["past"], st["ring"], st["ctr"])
         ent = (g, out)

@@ -99,15 +99,13 @@ class SlotModel:
         ent["dev"].copy_(ent["host"], non_blocking=True)
         ent["copied"].record()
         if ent["graph"] is None:
-            from .llama_hip import prime_graph_capture
+            from .llama_hip import graph_capture
             saved, self._buf = self._buf, ent["bufs"]             # the graph owns its scratch
             try:
                 self._run(arena, ent["dev"], d, ent["logits"])    # eager first: sizes every scratch buffer, and is this step's result
                 torch.cuda.synchronize()
                 # (capture records the launches without executing them: the recurrent states advance once, by the eager run)
-                prime_graph_capture(self.device)
-                g = torch.cuda.CUDAGraph()
-                with torch.cuda.graph(g):
+                with graph_capture(self.device) as g:
                     self._run(arena, ent["dev"], d, ent["logits"])
                 ent["graph"] = g
             finally:
