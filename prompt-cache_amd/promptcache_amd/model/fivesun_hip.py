@@ -20,9 +20,9 @@ same projection as the mixer's inputs (or is one projection beside the feed-forw
     attention   q | k | v | g | r = ONE projection (sigmoid on g | r); pcb_head_prep: per-head RMS norms, rotary pairs (angles as
                 float64 products), value blend with the first blending layer's values, ``key | value`` rows into the slot's cache;
                 keys of the query's own block of positions only, exp(sink_h) in the denominator, one gate per head: tiles of
-                queries for requests that bring many tokens (pcb_attn_prompt), single rows for the others (pcb_attn_rows)
+                queries where requests bring many tokens for their context (pcb_attn_prompt), single rows elsewhere (pcb_attn_rows)
     latent      q | down | g | r = ONE projection; pcb_head_prep: the latent normed, the shared key part and the queries' rotated
-                parts turned (YaRN frequencies), latent | key part into the slot's row.  A request that brings many tokens has the
+                parts turned (YaRN frequencies), latent | key part into the slot's row.  A request that brings many tokens may have the
                 keys and values of all heads rebuilt from the latents (pcb_linear) and attends in tiles (pcb_attn_prompt, the shared
                 key part read from the cached rows, times sigmoid(g)); for the others the up-projections are folded into the query
                 and the output: q'_h = W_uk,h^T q_h, attention of [q'_h | q_rot,h] over the cached rows with the latent itself as
@@ -37,6 +37,7 @@ from __future__ import annotations
 
 import math
 import os
+from collections import Counter
 from typing import Dict, Optional, Sequence
 
 import numpy as np
@@ -70,11 +71,10 @@ class FivesunHIP(SlotModel):
     GRAPH_MAX_ROWS = 64
     SEGMENT = int(os.environ.get("PC_FS_SEGMENT", "64"))    # a step that brings a request more tokens than this runs its mLSTM layers segment-parallel
     MAX_SEGMENTS = 128      # (segments grow beyond SEGMENT tokens rather than exceed this many per request)
-    # A request that brings at least this many tokens attends in tiles of 64 or 128 queries, another row by row: a tile of 64 with 16
-    # live rows costs what 16 single rows cost (one pass over the keys per head against one per row and 16 heads).
-    PROMPT_ROWS = int(os.environ.get("PC_FS_PROMPT_ROWS", "16"))
-    REBUILD_RATIO = 64      # ... but folds its queries, instead of rebuilding the keys, if it brings less than a 64th of what they number
-    REBUILD_BYTES = 256 << 20   # rebuilt keys and values that lie in memory at a time: beyond it (32 k rows of 16 heads of 128 + 128) heads take turns
+    PROMPT_ROWS = int(os.environ.get("PC_FS_PROMPT_ROWS", "16"))   # a request that brings fewer tokens than this attends row by row (see _tiled)
+    # Rebuilt keys and values that lie in memory at a time: beyond it heads take turns, which leaves part of the chip idle (eight requests of 256
+    # tokens behind 8 000, 541 MB: 3 350 us in one turn, 4 023 in three).  1 GB is 131 k rows of 16 heads of 128 + 128 columns.
+    REBUILD_BYTES = 1 << 30
 
     def __init__(self, shape: FivesunShape, weights: Dict[str, torch.Tensor], device="cuda:0", dtype=torch.bfloat16,
                  decode_headroom: int = 256):
@@ -158,10 +158,12 @@ class FivesunHIP(SlotModel):
         self._sigs = sorted({(l.kv_heads, l.dim + l.vdim) for l in shape.layers if l.kind == "attention"} |
                             {(1, l.kv_rank + l.rot_dim) for l in shape.layers if l.kind == "latent_attention"})
         latent = [ent for ent in self.layers if ent["cfg"].kind == "latent_attention"]
-        self._rebuilds = any(ent["prompts"] for ent in latent)
         self._folds = any(not ent["prompts"] for ent in latent)
+        # what _tiled weighs: (heads, workgroups a row takes in the kernels of single rows, reach, columns rebuilt per key and head), how many layers
+        self._att = Counter((l.heads, l.kv_heads * -(-l.heads // (16 * l.kv_heads)), l.mask, 0) for l in shape.layers if l.kind == "attention" and l.dim <= 256)
+        self._lat = Counter((l.heads, -(-l.heads // 16), l.mask, l.kv_rank * (l.dim + l.vdim)) for l in (ent["cfg"] for ent in latent if ent["prompts"]))
         # positions behind a request's first new token whose keys its rebuilding layers need (0: all of them)
-        reach = [ent["cfg"].mask for ent in latent if ent["prompts"]]
+        reach = [mask for _, _, mask, _ in self._lat]
         self._reach = 0 if not reach or min(reach) <= 0 else max(reach)
         self._wide = any(ent["cfg"].kind == "attention" and ent["cfg"].dim > 256 for ent in self.layers)
         self._max_heads = max(l.heads for l in shape.layers)
@@ -183,6 +185,42 @@ class FivesunHIP(SlotModel):
         es = 2 if self.dtype == torch.bfloat16 else 4
         return sum(l.kv_heads * (l.dim + l.vdim) if l.kind == "attention" else (l.kv_rank + l.rot_dim if l.kind == "latent_attention" else 0)
                    for l in self.config.layers) * es
+
+    def _tiled(self, layers, cand, counts, starts):
+        """Which of the requests ``cand`` attend in tiles of queries in ``layers``; the others go row by row.
+
+        A tile walks its request's keys by itself, so tiles are as slow as the longest context among them, however little of the chip they
+        fill; rows are cut into runs of keys and cost the same each.  In units of a tile's block of 64 keys (2.25 us; fp32 6.6): a row costs
+        1 / 700 a block and workgroup, 470 tiles run at a time (fp32 320), a latent layer's tile block 1.16, its rebuilt block
+        heads * rank * (key + value columns) / 6.5e6, its folded row heads / 4400 for the products around it.  Tiled are the requests up to the
+        context length that makes the sum cheapest.  us, heads of 128, rows / tiles, keys x tokens: 16 heads over 4, 1 024 x 64 23 / 41, x 256
+        79 / 47, 8 000 x 64 121 / 296, x 256 401 / 290, 30 000 x 16 119 / 1 030, x 256 1 384 / 1 039, eight requests of 8 000 x 16 235 / 287, x 64
+        769 / 290; latent of 192, folded / rebuilt: 8 000 x 64 49 / 375, x 512 281 / 381, eight requests of 8 000 x 64 282 / 684, x 256 836 / 723."""
+        if not cand or not layers:
+            return []
+        order = sorted(cand, key=lambda b: starts[b] + counts[b])
+        shortest, longest = starts[order[0]] + counts[order[0]], starts[order[-1]] + counts[order[-1]]
+        if longest <= 512:
+            return cand                            # (a dozen us either way, which the host's part of the step covers)
+        if all(not l[3] and sum(counts[b] for b in cand) * l[1] * shortest >= 1400 * longest for l in layers):
+            return cand                            # (rows would cost twice the longest context's tile)
+        at_a_time = 470.0 if self.dtype == torch.bfloat16 else 320.0
+        cost = [0.0] * (len(order) + 1)            # of the first k in tiles
+        for (heads, groups, mask, rebuilt), n in layers.items():
+            unit = 1.16 if rebuilt else 1.0
+            rows = [counts[b] * (groups * min(starts[b] + 0.5 * counts[b], mask or math.inf) / (64 * 700) + (heads / 4400 if rebuilt else 0.0)) for b in order]
+            rest, longest, all_tiles, rebuild = sum(rows), 0.0, 0.0, 0.0
+            cost[0] += n * (rest + 3.0)            # (3 and 2: the launches)
+            for k, b in enumerate(order):
+                keys = min(starts[b] + counts[b], mask + 64 if mask else math.inf)
+                blocks = -(-keys // 64) * unit
+                longest = max(longest, blocks)
+                all_tiles += -(-counts[b] // 64) * blocks * heads / at_a_time
+                rebuild += min(starts[b] + counts[b], mask + counts[b] if mask else math.inf) / 64 * heads * rebuilt / 6.5e6
+                rest -= rows[k]
+                cost[k + 1] += n * (max(longest, all_tiles) + rebuild + 2.0 + (rest + 3.0 if k + 1 < len(order) else 0.0))
+        best = min(range(len(cost)), key=lambda k: (cost[k], -k))
+        return sorted(order[:best])
 
     # ---- one step ------------------------------------------------------------------------------------------------------------
     @torch.inference_mode()
@@ -208,12 +246,12 @@ class FivesunHIP(SlotModel):
 
         # attention: tiles of neighbouring queries for requests that bring many tokens, single rows for the others.  (A captured step has single
         # rows only: its launches are those of any step of as many requests.)
-        big = [] if graphed else [b for b, c in enumerate(counts) if c >= self.PROMPT_ROWS]
+        cand = [] if graphed else [b for b, c in enumerate(counts) if c >= self.PROMPT_ROWS]
+        big, rebuilt = self._tiled(self._att, cand, counts, starts), self._tiled(self._lat, cand, counts, starts)
         # the oldest key that the rebuilding layers need (a whole number of the kernel's blocks of keys)
-        oldest = [max(0, s0 - self._reach + 1) // 64 * 64 if self._reach else 0 for s0 in starts] if big else []
-        rebuilt = [b for b in big if self._rebuilds and starts[b] + counts[b] - oldest[b] <= self.REBUILD_RATIO * counts[b]]
+        oldest = [max(0, s0 - self._reach + 1) // 64 * 64 if self._reach else 0 for s0 in starts] if rebuilt else []
         tile = 64
-        if self.dtype == torch.bfloat16 and sum(-(-counts[b] // 128) for b in big) * self._max_heads >= 512:
+        if self.dtype == torch.bfloat16 and sum(-(-counts[b] // 128) for b in big or rebuilt) * self._max_heads >= 512:
             tile = 128
         none = np.zeros(0, np.int32)
         rows = np.empty((T, 4), dtype=np.int32)                 # every row by itself
@@ -301,7 +339,7 @@ class FivesunHIP(SlotModel):
             at += n
         for name in ("p_tiles", "l_tiles", "kv_rows", "f_rows", "a_tiles", "w_tiles"):
             out.setdefault(name, i32[:0])
-        out.setdefault("f_tiles", out["s_tiles"])  # (the same rows, unless some request is tiled without being rebuilt)
+        out.setdefault("f_tiles", out["s_tiles"])  # (the same rows, unless other requests are rebuilt than tiled)
         no = len(self._sigs)
         out["offs"] = dblob[d["o64"]:d["o64"] + no * d["T"] * 8].view(torch.int64).view(no, d["T"])
         return out
@@ -356,10 +394,18 @@ class FivesunHIP(SlotModel):
         B.linear(h, lw["w_in"], P, M=T, bias=lw["b_in"], act_split=lw["act_from"], act2=B.ACT_SIGMOID)
         return P, N
 
-    def _splits(self, n, head_groups, reach):
-        # few (row, group of heads) pairs cannot fill the chip: each is cut into runs of its keys, as many as blocks of 64 fit what it sees
-        blocks = -(-reach // 64)
-        return 1 if blocks <= 3 else max(1, min(64, 512 // (n * head_groups), blocks))
+    def _splits(self, n, groups, heads, reach, full=768):
+        """Into how many runs the keys of ``n`` rows are cut (the kernels of single rows: ``n * groups`` workgroups a run, ``full`` of them at a
+        time).  Rounds of the chip times a run's blocks of 64 keys and what starting one costs, and the merge: us, 8 heads over 2, 30 000 keys,
+        cut for 512 workgroups / by this rule: 16 rows 73 / 65, 64 236 / 216, 128 455 / 400, 256 930 / 749, 512 1 678 / 1 381."""
+        blocks, w = -(-reach // 64), n * groups
+        best = (-(-w // full) * (blocks + 2), 1)
+        if blocks > 3:
+            for k in range(1, 5):
+                s = min(64, blocks, full * k // w)
+                if s > 1:
+                    best = min(best, (-(-w * s // full) * (-(-blocks // s) + 2) + 1 + n * heads / 1200, s))
+        return best[1]
 
     def _attention(self, arena, i, l, lw, h, y, tb, T, R):
         E = self.dtype
@@ -392,7 +438,7 @@ class FivesunHIP(SlotModel):
                 B.attn_prompt(q, tb["p_tiles"], n, tb["tile"], plane, (rs, hs, ss), values, (rs, hs, ss), H, G, D, Dv, l.scale, att, **kw)
             n = tb["s_tiles"].numel() // 4
             if n:
-                splits = self._splits(n, G * -(-H // (16 * G)), reach)
+                splits = self._splits(n, G * -(-H // (16 * G)), H, reach, 768 if max(D, Dv) <= 128 else 512)
                 part = self._scratch("attn_part", B.attn_softmax_part(n, H, splits, Dv), torch.float32) if splits > 1 else None
                 B.attn_rows(q, tb["s_tiles"], n, plane, (ss, hs, rs), values, (ss, hs, rs), H, G, D, Dv, l.scale, att, gate_per_head=True,
                             n_splits=splits, part=part, **kw)
@@ -427,7 +473,7 @@ class FivesunHIP(SlotModel):
             rows = tb["f_rows"] if tiled and n < T else None
             B.linear(P, lw["w_abs"], qa, M=n, row_src=rows, row_dst=rows, n_batch=H, ldx=N, x_batch_stride=DR, ldy=H * CR, y_batch_stride=CR)
             ol = self._mat("mix_out", T, H * C, E)
-            splits = self._splits(n, -(-H // 16), min(arena.cap, l.mask or arena.cap))
+            splits = self._splits(n, -(-H // 16), H, min(arena.cap, l.mask or arena.cap), 768 if CR <= 256 else 512)
             part = self._scratch("attn_part", B.attn_softmax_part(n, H, splits, C), torch.float32) if splits > 1 else None
             B.attn_latent(qa, f_tiles, n, plane, arena.slot_stride(i), CR, H, CR, C, l.scale, ol, window=l.mask, n_splits=splits, part=part)
             ov = self._mat("mix_o32", T, HV, torch.float32)

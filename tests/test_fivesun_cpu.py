@@ -105,17 +105,22 @@ def step_tables(m, arena, slots, tokens):
 
 
 @pytest.mark.parametrize("prompt_rows", [16, 1])
+@pytest.mark.parametrize("route", ["all", "tiled", "rebuilt", "last", "none", "rule"])
 @pytest.mark.parametrize("news", [[1], [1, 1, 1], [16], [2, 15, 3], [17, 1, 40], [1, 200, 16, 3], [16, 64, 130]])
-def test_step_tables_name_every_row_once(news, prompt_rows):
-    """Which launch of a step takes which row, against the rule in plain words: requests of 16 new tokens and more in tiles, rebuilt where a 64th of
-    their window is new, the others row by row -- and single rows only in a step that may be captured, whatever the knobs say."""
+def test_step_tables_name_every_row_once(news, route, prompt_rows):
+    """Which launch of a step takes which row, in plain words, whatever requests of 16 new tokens and more attend in tiles and whichever have their
+    keys rebuilt -- and single rows only in a step that may be captured, whatever the knobs say."""
     from promptcache_amd.model.fivesun_hip import FivesunHIP
     lat = dict(heads=2, kv_heads=1, kv_rank=24, rot_dim=8, rot_dims=8, vdim=16)
     s = FivesunShape(vocab_size=50, hidden_size=32, norm_eps=1e-6, layers=[
         FivesunLayer("attention", heads=2, kv_heads=1, dim=16, vdim=16, mask=64, rot_dims=16), FivesunLayer("latent_attention", dim=16, mask=600, **lat),
         FivesunLayer("latent_attention", dim=256, mask=80, **lat), FivesunLayer("attention", heads=1, kv_heads=1, dim=264, vdim=8, rot_dims=0)])
     m = FivesunHIP(s, W.make_fivesun_weights(s, seed=1), device="cpu", dtype=torch.float32)
-    m.PROMPT_ROWS = prompt_rows
+    m.PROMPT_ROWS, rule = prompt_rows, m._tiled
+    pick = dict(all=lambda layers, cand, *_: list(cand), none=lambda *_: [], tiled=lambda layers, cand, *_: list(cand) if layers is m._att else [],
+                rebuilt=lambda layers, cand, *_: list(cand) if layers is m._lat else [], last=lambda layers, cand, *_: cand[-1:], rule=rule)[route]
+    m._tiled = lambda *a: picked.setdefault("att" if a[0] is m._att else "lat", pick(*a))
+    picked = {}
     cap, starts = 4096, [1700, 0, 333, 70][:len(news)]
     ar = m.new_arena(5, cap)
     slots = [ar.alloc() for _ in range(5)][5 - len(news):]
@@ -125,9 +130,9 @@ def test_step_tables_name_every_row_once(news, prompt_rows):
     T, flat = sum(news), [sum(news[:b]) for b in range(len(news))]
     row = {flat[b] + i: [slots[b], starts[b] + i, 1, flat[b] + i] for b in range(len(news)) for i in range(news[b])}
     one = all(n == 1 for n in news)
-    big = [] if one else [b for b, n in enumerate(news) if n >= prompt_rows]
-    low = {b: max(0, starts[b] - 599) // 64 * 64 for b in big}
-    rebuilt = [b for b in big if starts[b] + news[b] - low[b] <= 64 * news[b]]
+    big, rebuilt = picked["att"], picked["lat"]
+    assert all(news[b] >= prompt_rows and not one for b in big + rebuilt)
+    low = {b: max(0, starts[b] - 599) // 64 * 64 for b in rebuilt}
     single = [r for b in range(len(news)) if b not in big for r in range(flat[b], flat[b] + news[b])]
     folded = [r for b in range(len(news)) if b not in rebuilt for r in range(flat[b], flat[b] + news[b])]
 
@@ -151,6 +156,21 @@ def test_step_tables_name_every_row_once(news, prompt_rows):
         for b in range(len(news)):
             ar.lengths[slots[b]] = 5 + b
         assert step_tables(m, ar, slots, [[7] * n for n in news])[1] == dims
+
+
+def test_long_contexts_with_few_new_tokens_are_not_tiled():
+    """The measured sides of the rule: a lone portion over a long context goes row by row, a prompt in tiles, many portions together in tiles,
+    and a portion over a long context does not hold up the prompt beside it (16 heads over 4, a latent of 192)."""
+    from promptcache_amd.model.fivesun_hip import FivesunHIP
+    lat = dict(heads=16, kv_heads=1, kv_rank=192, rot_dim=64, rot_dims=64, dim=128, vdim=128)
+    s = FivesunShape(vocab_size=50, hidden_size=32, norm_eps=1e-6, layers=[
+        FivesunLayer("attention", heads=16, kv_heads=4, dim=128, vdim=128, rot_dims=128), FivesunLayer("latent_attention", **lat)])
+    m = FivesunHIP(s, W.make_fivesun_weights(s, seed=1), device="cpu", dtype=torch.bfloat16)
+    for news, starts, att, latent in [([16], [30000], [], []), ([64], [8000], [], []), ([256], [30000], [0], []), ([2048], [0], [0], [0]),
+                                      ([64] * 8, [8000] * 8, list(range(8)), []), ([256] * 8, [8000] * 8, list(range(8)), list(range(8))),
+                                      ([300] * 8, [0] * 8, list(range(8)), list(range(8))), ([16, 2048], [30000, 0], [1], [1])]:
+        cand = list(range(len(news)))
+        assert m._tiled(m._att, cand, news, starts) == att and m._tiled(m._lat, cand, news, starts) == latent, (news, starts)
 
 
 def test_frequency_tables_follow_the_oracle():

@@ -503,18 +503,58 @@ def test_tiled_and_single_rows_beside_one_another(dtype, n):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n", [16, 64, 65, 129])
+@pytest.mark.parametrize("route", ["all", "tiled", "rebuilt", "none"])
+def test_every_route_of_a_portion_gives_the_same(dtype, n, route):
+    """The steps of the test above with tiles and rebuilt keys wherever they may be, in one kind of layer only, and nowhere: which route is the
+    cheapest depends on sizes that no oracle reaches."""
+    s = FivesunShape(vocab_size=90, hidden_size=64, norm_eps=1e-6, embed_scale=8.0, layers=[
+        att(4, 2, 32, 32, mask=70, ff=48), lat(4, 40, 24, 32, 48, mask=90, ff=48), lat(2, 230, 40, 20, 32, mask=70), att(2, 1, 264, 16, mask=0)])
+    w = W.make_fivesun_weights(s, seed=4)
+    from promptcache_amd.model.fivesun_hip import FivesunHIP
+
+    class Forced(FivesunHIP):
+        on = False
+
+        def _tiled(self, layers, cand, *a):
+            mine = route == "all" or route == ("tiled" if layers is self._att else "rebuilt")
+            return super()._tiled(layers, cand, *a) if not self.on else list(cand) if mine else []
+    m = Forced(s, w, device=DEV, dtype=dtype)
+    seqs = [toks(k, s.vocab_size, seed=40 + i) for i, k in enumerate((150 + n, 81 + n, 43))]
+    new = [n, n, 3]
+    alone = [run_alone(m, q, [1] * len(q))[-k:] for q, k in zip(seqs, new)]
+    m.on = True
+    ar = m.new_arena(3, 400)
+    slots = [ar.alloc() for _ in seqs]
+    m.forward_rows(ar, slots, [q[:-k] for q, k in zip(seqs, new)])
+    got = m.forward_rows(ar, slots, [q[-k:] for q, k in zip(seqs, new)], [list(range(k)) for k in new])
+    for i, (q, k) in enumerate(zip(seqs, new)):
+        want = oracle_logits(s, w, q)[0][-k:] if dtype == torch.float32 else alone[i]
+        assert rel(got[sum(new[:i]):sum(new[:i]) + k], want) < tol(dtype, 3e-5, 8e-2), i
+
+
+def tiling():
+    """The model that attends in tiles, over rebuilt keys, wherever it may."""
+    from promptcache_amd.model.fivesun_hip import FivesunHIP
+
+    class Tiling(FivesunHIP):
+        def _tiled(self, layers, cand, *_):
+            return list(cand)
+    return Tiling
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("dim,rot,vdim", [(40, 24, 32), (13, 6, 9)])
 def test_rebuilt_heads_take_turns_within_their_scratch(dtype, dim, rot, vdim):
     """The scratch of rebuilt keys and values is as large as it may be, whatever the context: with room for all five heads, for two (the last
     turn has one) and for less than one, a prompt and what goes on behind it get the same numbers."""
     s = FivesunShape(vocab_size=90, hidden_size=64, norm_eps=1e-6, embed_scale=8.0, layers=[lat(5, dim, rot, vdim, 48, mask=0, ff=48)])
     w = W.make_fivesun_weights(s, seed=4)
-    from promptcache_amd.model.fivesun_hip import FivesunHIP
     tokens = toks(200, s.vocab_size, seed=62)
     head = 224 * (dim + vdim) * (2 if dtype == torch.bfloat16 else 4)              # 200 rows in whole blocks of 32
     want = None
     for room, heads in ((1 << 20, 5), (2 * head, 2), (1, 1)):
-        m = FivesunHIP(s, w, device=DEV, dtype=dtype)
+        m = tiling()(s, w, device=DEV, dtype=dtype)
         m.REBUILD_BYTES = room
         ar = m.new_arena(1, 256)
         slot = ar.alloc()
@@ -532,14 +572,13 @@ def test_runs_of_a_decoding_row_beside_a_prompt():
     that row's, not the step's, and both requests get what the oracle says."""
     s = FivesunShape(vocab_size=90, hidden_size=64, norm_eps=1e-6, embed_scale=8.0, layers=[lat(4, 40, 24, 32, 48, mask=0, ff=48)])
     w = W.make_fivesun_weights(s, seed=4)
-    from promptcache_amd.model.fivesun_hip import FivesunHIP
-    m = FivesunHIP(s, w, device=DEV, dtype=torch.float32)
+    m = tiling()(s, w, device=DEV, dtype=torch.float32)
     seqs, new = [toks(401, s.vocab_size, seed=60), toks(300, s.vocab_size, seed=61)], [1, 300]
     ar = m.new_arena(2, 800)
     slots = [ar.alloc() for _ in seqs]
     m.forward_rows(ar, slots[:1], [seqs[0][:-1]])
     got = m.forward_rows(ar, slots, [q[-k:] for q, k in zip(seqs, new)], [list(range(k)) for k in new])
-    splits = m._splits(1, 1, 800)
+    splits = m._splits(1, 1, 4, 800)
     assert splits > 1 and m._buf["attn_part"].numel() <= max(1024, 2 * B().attn_softmax_part(1, 4, splits, 48))
     for g, q, k in zip((got[:1], got[1:]), seqs, new):
         assert rel(g, oracle_logits(s, w, q)[0][-k:]) < 3e-5
