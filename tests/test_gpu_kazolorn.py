@@ -21,6 +21,10 @@ F64 = torch.float64
 DTYPES = [torch.float32, torch.bfloat16]
 
 
+def dev_i32(rows):
+    return torch.tensor(rows, dtype=torch.int32, device=DEV).reshape(-1)
+
+
 def rel(got, want):
     got, want = got.detach().to("cpu", F64), want.detach().to("cpu", F64)
     return float((got - want).pow(2).mean().sqrt() / want.pow(2).mean().sqrt().clamp_min(1e-30))
@@ -287,6 +291,32 @@ def test_attention_alone(dtype, H, G, D, window, n, first):
 def test_attention_of_many_tiles(dtype, H, G, D, window, n, first):
     got, want, _ = _attn_case(dtype, H, G, D, window, n, first)
     assert rel(got, want) < tol(dtype, 2e-6, 1.5e-2)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("sink", [True, False])
+@pytest.mark.parametrize("n,rows,few", [(40, 40, 0), (1040, 1040, 0), (90, 3, 4)])     # four waves, eight, the kernel of at most four rows
+def test_rows_that_are_no_numbers_stay_none(dtype, sink, n, rows, few):
+    """A query row with a NaN or an infinity in it gives a row of NaN in every form of the kernels, and the rows beside it what they give
+    without it, bit for bit."""
+    g = torch.Generator().manual_seed(n)
+    H, G, D, window, first, cap = 4, 2, 32, 33, n - rows, n + 3
+    q, k = torch.randn(rows, H * D, generator=g).to(dtype).to(DEV), torch.randn(1, G, cap, D, generator=g).to(dtype).to(DEV)
+    talk = (torch.eye(H) + 0.2 * torch.randn(H, H, generator=g)).to(DEV)
+    tiles = dev_i32([[0, first + t, min(16, rows - t), t] for t in range(0, rows, 16)])
+    t64 = dev_i32([[0, first + t, min(64, rows - t), t] for t in range(0, rows, 64)])
+    scratch = torch.empty(tiles.numel() * 4 * H * B().attn_talk_band(window, n), device=DEV)
+    bad = [rows - 1, rows // 3]
+
+    def attend(x):
+        out = torch.zeros(rows, H * D, dtype=dtype, device=DEV)
+        B().attn_talk(x, tiles, tiles.numel() // 4, k, G * cap * D, cap * D, H, G, D, 0.3, window, n, None, talk, sink, scratch, out, tiles64=t64,
+                      n_tiles64=t64.numel() // 4, max_tile_rows=few)
+        return out
+    clean, x = attend(q), q.clone()
+    x[bad[0], 5 * D // 2], x[bad[1], 3] = float("nan"), float("inf")
+    got, other = attend(x), [r for r in range(rows) if r not in bad]
+    assert bool(torch.isnan(got[bad]).all()) and bool(torch.isfinite(clean).all()) and torch.equal(got[other], clean[other])
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
