@@ -310,7 +310,8 @@ def test_many_row_projections_of_experts_and_split_destinations(K):
     assert rel(y2[:, pos].permute(1, 0, 2).reshape(R, 84), z[:, 100:184]) < 5e-3 and rel(y3[:, pos].T, z[:, 184:]) < 5e-3
 
 
-@pytest.mark.parametrize("M,N", [(2048, 2052), (1900, 2500), (1900, 4106)])
+# tiles of plain stores and accumulations: 128 x 256 at the first three sizes, 128 x 128 at the fourth, 256 x 256 at the last
+@pytest.mark.parametrize("M,N", [(2048, 2052), (1900, 2500), (1900, 4106), (1900, 2044), (1990, 8108)])
 @pytest.mark.parametrize("K", [8, 136, 712])
 def test_whole_cu_tiles_and_where_their_results_go(M, N, K):
     """Launches of each tile size (128 x 128, 128 x 256, 256 x 256) with a ragged last tile both ways and k ranges that end after 1, 2, 1 chunks
