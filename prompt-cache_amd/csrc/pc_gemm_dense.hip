@@ -33,7 +33,8 @@
 // lane on full rows.
 // Grid: 1-D, XCD-aware: block id b runs on XCD b % 8; the tiles are cut into 8 rectangles (px row strips by 8 / px column strips),
 // one per XCD, walked M-block by M-block: the 32 tiles that run on an XCD at a time share few activation rows AND few weight panels
-// (with one column strip each an XCD walks all M-blocks: 2 048 x 8 192 x 2 048 in 256 x 256 tiles 93 us, in 4 x 2 strips 71).
+// (with one column strip each an XCD walks all M-blocks: 2 048 x 8 192 x 2 048 in 256 x 256 tiles 93 us, in 4 x 2 strips 71).  Where no
+// such cut reaches the rounds of an even share, the column-by-column order is dealt to the XCDs in 8 runs (mfma_tile_loop.h).
 // Roofline: MFMA.  flops per launch = 2 * (TWO ? 2 : 1) * M * N * K against the 2.5 PFLOP/s dense fp16 peak.
 #include <hip/hip_fp16.h>
 #include <string.h>
@@ -68,7 +69,6 @@ struct DenseParams {
     // v_mfma_i32_32x32x32_i8 -- twice the fp16 MFMA rate, exact integer sums -- and joins the fp32 accumulator in the epilogue
     const signed char* xl8; const float* xl8_scale; int64_t ldx8;
     const signed char* w8; const float* w8_scale; int64_t ldw8;
-    const _Float16* zeros;                                 // >= 16 B of zeros (the -DPC_DEV_SWEEPS kernels' chunks past K)
     float* y; int64_t ldy;                                 // EPI_STORE / EPI_ADD
     _Float16* oh; _Float16* ol; int64_t ldo;               // EPI_SILU / EPI_GELU output planes
     int32_t M, N, K, mb, nb, nfeat;                        // nfeat: SiLU features (= N / 2)
@@ -89,11 +89,11 @@ __device__ __forceinline__ void glds16(const _Float16* g, char* lds_wave_base) {
                                      (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, 0);
 }
 
-// the block tile of a launch: W x W waves of 32 MT x 32 NT, S LDS images in the ring (as many as the 160 KiB of a CU hold)
-template <int W, bool TWO, bool NARROW, bool TALL>
+// the block tile of a launch: 2 x 2 waves of 32 MT x 32 NT, S LDS images in the ring (as many as the 160 KiB of a CU hold)
+template <bool TWO, bool NARROW, bool TALL>
 struct Tile {
     static constexpr int MT = TALL ? 4 : 2, NT = NARROW ? 2 : 4, S = TWO || TALL ? 2 : 3;
-    static constexpr int BM = 32 * W * MT, BN = 32 * W * NT;
+    static constexpr int BM = 64 * MT, BN = 64 * NT;
 };
 
 // The 64 columns of group `grp` (of the launch's weight rows; EPI_SILU: 32 gate and the matching 32 up features, EPI_ROPE: 32 features of a
@@ -231,11 +231,11 @@ __device__ __forceinline__ void store_group(const DenseParams& p, char* patch, i
     }
 }
 
-// W: waves across and down a workgroup; TWO: both activation planes; NARROW: 128 columns instead of 256; TALL: 256 rows instead of 128
-template <int W, int EPI, bool TWO, bool NARROW, bool TALL>
+// TWO: both activation planes; NARROW: 128 columns instead of 256; TALL: 256 rows instead of 128
+template <int EPI, bool TWO, bool NARROW, bool TALL>
 __global__ __launch_bounds__(256, 1) void gemm_dense_kernel(const DenseParams p) {
-    static_assert(W == 2 && !(TWO && TALL), "four waves; two planes of 256 rows and their weights do not fit the LDS twice");
-    using T = Tile<W, TWO, NARROW, TALL>;
+    static_assert(!(TWO && TALL), "two planes of 256 rows and their weights do not fit the LDS twice");
+    using T = Tile<TWO, NARROW, TALL>;
     constexpr int MT = T::MT, NT = T::NT, S = T::S;
     using L = mfma_tile::Loop<MT, NT, S, TWO ? 2 : 1>;
     constexpr int PL = TWO ? 2 : 1, BM = L::BM, BN = L::BN;
@@ -365,18 +365,15 @@ __global__ __launch_bounds__(256) void dense_reduce_kernel(const float* __restri
     *(f4*)yp = v;
 }
 
-// 16 bytes of zeros (DenseParams::zeros; device constant: no allocation, graph-capturable)
-__device__ __attribute__((aligned(16))) _Float16 g_zero_chunk[8];
-
 template <int EPI, bool TWO, bool NARROW, bool TALL>
 int launch_dense_as(DenseParams& p, hipStream_t s, int kslices) {
-    constexpr int BM = Tile<2, TWO, NARROW, TALL>::BM, BN = Tile<2, TWO, NARROW, TALL>::BN;
+    constexpr int BM = Tile<TWO, NARROW, TALL>::BM, BN = Tile<TWO, NARROW, TALL>::BN;
     p.mb = pc_ceil_div(p.M, BM);
     p.nb = (EPI == EPI_SILU) ? pc_ceil_div(p.nfeat, BN / 2) : pc_ceil_div(p.N, BN);
     const int nkt = pc_ceil_div(p.K, BK);
     p.kper = pc_ceil_div(nkt, kslices);
     p.strips = mfma_tile::strips(p.mb, p.nb, (TWO ? 2 : 1) * BM, BN);
-    hipLaunchKernelGGL((gemm_dense_kernel<2, EPI, TWO, NARROW, TALL>), dim3(8 * p.strips.mh * p.strips.nh, pc_ceil_div(nkt, p.kper)), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((gemm_dense_kernel<EPI, TWO, NARROW, TALL>), dim3(8 * p.strips.mh * p.strips.nh, pc_ceil_div(nkt, p.kper)), dim3(256), 0, s, p);
     return pc_check_launch("gemm_dense_kernel");
 }
 
@@ -387,15 +384,14 @@ int launch_dense_as(DenseParams& p, hipStream_t s, int kslices) {
 // the 128-row tiles, BN = 256 or 128 columns
 template <int BN, int EPI>
 int launch_dense(DenseParams& p, hipStream_t s, int kslices = 1) {
-#ifdef PC_DEV_SWEEPS
-    const char* e = getenv("PC_DENSE_PP");
-    if (p.xl8 || (e && e[0] == '1')) return lockstep::launch<BN == 256 ? 2 : 4, EPI>(p, s, kslices);
-#else
     if (p.xl8) {
+#ifdef PC_DEV_SWEEPS
+        return lockstep::launch<BN == 256 ? 2 : 4, EPI>(p, s, kslices);
+#else
         pc_set_error("pc_gemm_dense: the int8 residual plane (x_lo8) needs a -DPC_DEV_SWEEPS build (csrc/pc_dev.h)");
         return PC_ERR_ARG;
-    }
 #endif
+    }
     if (p.xl) return launch_dense_as<EPI, true, BN == 128, false>(p, s, kslices);
     return launch_dense_as<EPI, false, BN == 128, false>(p, s, kslices);
 }
@@ -481,12 +477,6 @@ int gemm_dense_impl(const void* x_hi, const void* x_lo, int64_t ldx, const void*
         p.xl8 = (const signed char*)lo8->x_lo8; p.xl8_scale = lo8->x_lo8_scale; p.ldx8 = lo8->ldx8;
         p.w8 = (const signed char*)lo8->w8; p.w8_scale = lo8->w8_scale; p.ldw8 = lo8->ldw8;
     }
-    void* z = nullptr;
-    if (hipGetSymbolAddress(&z, HIP_SYMBOL(g_zero_chunk)) != hipSuccess || !z) {
-        pc_set_error("pc_gemm_dense: hipGetSymbolAddress failed");
-        return PC_ERR_ARG;
-    }
-    p.zeros = (const _Float16*)z;
     hipStream_t s = (hipStream_t)stream;
     if (epilogue == EPI_SILU || epilogue == EPI_GELU) {
         PC_REQUIRE(out_hi && ldo % 4 == 0 && ((uintptr_t)out_hi & 7) == 0 && ((uintptr_t)out_lo & 7) == 0, PC_ERR_ARG,
@@ -577,12 +567,6 @@ PC_EXPORT int pc_gemm_dense_qkv_rope(const pc_dense_qkv_args* a, void* stream) {
         p.xl8 = (const signed char*)a->x_lo8; p.xl8_scale = a->x_lo8_scale; p.ldx8 = a->ldx8;
         p.w8 = (const signed char*)a->w8; p.w8_scale = a->w8_scale; p.ldw8 = a->ldw8;
     }
-    void* z = nullptr;
-    if (hipGetSymbolAddress(&z, HIP_SYMBOL(g_zero_chunk)) != hipSuccess || !z) {
-        pc_set_error("pc_gemm_dense_qkv_rope: hipGetSymbolAddress failed");
-        return PC_ERR_ARG;
-    }
-    p.zeros = (const _Float16*)z;
     p.cs = (const float2*)a->cs; p.q_hi = (_Float16*)a->q_hi; p.q_lo = (_Float16*)a->q_lo; p.q_ts = a->q_token_stride;
     p.k_arena = (_Float16*)a->k_arena; p.v_arena = (_Float16*)a->v_arena; p.a_bs = a->arena_batch_stride; p.a_hs = a->arena_head_stride;
     p.k_lo = (_Float16*)a->k_lo; p.v_lo = (_Float16*)a->v_lo; p.lo_bs = a->lo_batch_stride; p.lo_hs = a->lo_head_stride;

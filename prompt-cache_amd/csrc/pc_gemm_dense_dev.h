@@ -1,6 +1,5 @@
-// Dev builds only (-DPC_DEV_SWEEPS; included by pc_gemm_dense.hip): the eight-wave form of the many-row projections with its two measured
-// negative results -- the ping-pong main loop (PC_DENSE_PP=1, tools/dense_pp_ab.py) and the residual activation plane on the int8 MFMA
-// (pc_gemm_dense_lo8, tools/dense_lo8_ab.py).
+// Dev builds only (-DPC_DEV_SWEEPS; included by pc_gemm_dense.hip): the many-row projections with the residual activation plane on the
+// int8 MFMA (pc_gemm_dense_lo8, tools/dense_lo8_ab.py), eight waves and one barrier per K-step.  Needs K % 64 == 0.
 #pragma once
 
 namespace lockstep {
@@ -10,16 +9,15 @@ constexpr int kXT = BM * BK * 2;                 // bytes of one activation plan
 typedef int i4v __attribute__((ext_vector_type(4)));
 typedef int i16v __attribute__((ext_vector_type(16)));
 
-template <int WM, int EPI, bool TWO, bool PP, bool LO8 = false>
+template <int WM, int EPI>
 __global__ __launch_bounds__(512) void lockstep_kernel(const DenseParams p) {
-    static_assert(!(LO8 && (TWO || PP)), "LO8 replaces the fp16 lo plane; lockstep main loop only");
     constexpr int WN = 8 / WM, MT = BM / (32 * WM), NT = 2, BN = 64 * WN;
     constexpr int kWT = BN * BK * 2;             // bytes of the weight tile
-    // stage image: Xhi | Xlo | W   (LO8: Xhi | Xlo8 (64-byte rows) | W | W8 (64-byte rows))
-    constexpr int oW = LO8 ? kXT + kXT / 2 : 2 * kXT;
+    // stage image: Xhi | Xlo8 (64-byte rows) | W | W8 (64-byte rows)
+    constexpr int oW = kXT + kXT / 2;
     constexpr int oW8 = oW + kWT;
-    constexpr int kStage = LO8 ? oW8 + kWT / 2 : 2 * kXT + kWT;
-    constexpr int NXI = 2, NWI = BN / 64;        // staging instructions per wave: 2 per activation plane, BN/64 for W
+    constexpr int kStage = oW8 + kWT / 2;
+    constexpr int NXI = 2, NWI = BN / 64;        // staging instructions per wave: 2 for the activations, BN/64 for W
     constexpr int NW8 = BN / 128;                // ... and for the int8 weight tile (16 rows x 64 B per instruction); Xlo8: one
     __shared__ __attribute__((aligned(16))) char lds[2 * kStage];
 
@@ -31,7 +29,7 @@ __global__ __launch_bounds__(512) void lockstep_kernel(const DenseParams p) {
     const int nloc = slot / p.mb, mi = slot - nloc * p.mb, ni = nloc * 8 + xcd;
     if (ni >= p.nb) return;
     const int m0 = mi * BM;
-    const int K = p.K, nkt = (K + BK - 1) / BK;          // K-steps of the whole product
+    const int nkt = p.K / BK;                            // K-steps of the whole product
     const int t0 = blockIdx.y * p.kper;                  // this slice's first K-step (kper = nkt without split-K)
     const int nk = (p.kper < nkt - t0) ? p.kper : nkt - t0;
 
@@ -58,29 +56,25 @@ __global__ __launch_bounds__(512) void lockstep_kernel(const DenseParams p) {
     const int srow = lane >> 3, scp = lane & 7;          // row inside the 8-row group, chunk POSITION in the LDS row
     const _Float16* gx[NXI];
     const _Float16* gw[NWI];
-    int cx[NXI], cw[NWI];                                // source chunk index (for the K tail)
-    const int64_t lo_delta = TWO ? (p.xl - p.xh) : 0;
 #pragma unroll
     for (int j = 0; j < NXI; ++j) {
         const int r = wave * 16 + j * 8 + srow;
         const int gm = (m0 + r < p.M) ? m0 + r : p.M - 1;
-        cx[j] = scp ^ ((r >> 1) & 7);
-        gx[j] = p.xh + (int64_t)gm * p.ldx + cx[j] * 8;
+        gx[j] = p.xh + (int64_t)gm * p.ldx + (scp ^ ((r >> 1) & 7)) * 8;
     }
 #pragma unroll
     for (int j = 0; j < NWI; ++j) {
         const int r = wave * (BN / 8) + j * 8 + srow;
         int gr = wrow(r);
         gr = gr < 0 ? 0 : gr;
-        cw[j] = scp ^ ((r >> 1) & 7);
-        gw[j] = p.w + (int64_t)gr * p.ldw + cw[j] * 8;
+        gw[j] = p.w + (int64_t)gr * p.ldw + (scp ^ ((r >> 1) & 7)) * 8;
     }
-    // LO8: one instruction of 16 rows x 64 B per wave for the activation codes, NW8 for the weight codes; lane -> (row, chunk
+    // Codes: one instruction of 16 rows x 64 B per wave for the activation codes, NW8 for the weight codes; lane -> (row, chunk
     // POSITION); position c of row r holds source chunk c ^ ((r >> 2) & 3): the 16 lanes of every ds_read_b128 group then fall
     // into 16 distinct 16-byte bank slots (64-byte rows: slot = 4 (r & 3) + position)
-    [[maybe_unused]] const signed char* gx8 = nullptr;
-    [[maybe_unused]] const signed char* gw8[NW8 > 0 ? NW8 : 1];
-    if constexpr (LO8) {
+    const signed char* gx8;
+    const signed char* gw8[NW8];
+    {
         const int r = wave * 16 + (lane >> 2);
         const int gm = (m0 + r < p.M) ? m0 + r : p.M - 1;
         gx8 = p.xl8 + (int64_t)gm * p.ldx8 + (((lane & 3) ^ ((r >> 2) & 3)) << 4);
@@ -92,30 +86,15 @@ __global__ __launch_bounds__(512) void lockstep_kernel(const DenseParams p) {
             gw8[j] = p.w8 + (int64_t)gr * p.ldw8 + (((lane & 3) ^ ((rw >> 2) & 3)) << 4);
         }
     }
-    const bool ktail = (K % BK) != 0;
     auto stage = [&](int tl, char* buf) {
-        const int t = t0 + tl;
-        const bool tail = ktail && t == nkt - 1;
-        const int64_t ko = (int64_t)t * BK;
-        const int kchunks = tail ? (K - t * BK) / 8 : 8;          // valid 16-byte chunks in this K-step
+        const int64_t ko = (int64_t)(t0 + tl) * BK;
 #pragma unroll
-        for (int j = 0; j < NXI; ++j) {
-            const bool ok = !tail || cx[j] < kchunks;
-            const _Float16* sh = ok ? gx[j] + ko : p.zeros;
-            glds16(sh, buf + (wave * 16 + j * 8) * 128);
-            if (TWO) glds16(ok ? gx[j] + lo_delta + ko : p.zeros, buf + kXT + (wave * 16 + j * 8) * 128);
-        }
+        for (int j = 0; j < NXI; ++j) glds16(gx[j] + ko, buf + (wave * 16 + j * 8) * 128);
 #pragma unroll
-        for (int j = 0; j < NWI; ++j) {
-            // chunks past K pair with zero activations: any finite weight bytes do (the row's first chunk)
-            const _Float16* sw = (!tail || cw[j] < kchunks) ? gw[j] + ko : gw[j] - cw[j] * 8;
-            glds16(sw, buf + oW + (wave * (BN / 8) + j * 8) * 128);
-        }
-        if constexpr (LO8) {                           // (K % 64 == 0 with LO8: no tail)
-            glds16((const _Float16*)(gx8 + ko), buf + kXT + wave * 1024);
+        for (int j = 0; j < NWI; ++j) glds16(gw[j] + ko, buf + oW + (wave * (BN / 8) + j * 8) * 128);
+        glds16((const _Float16*)(gx8 + ko), buf + kXT + wave * 1024);
 #pragma unroll
-            for (int j = 0; j < NW8; ++j) glds16((const _Float16*)(gw8[j] + ko), buf + oW8 + (wave * (BN / 8) + j * 16) * 64);
-        }
+        for (int j = 0; j < NW8; ++j) glds16((const _Float16*)(gw8[j] + ko), buf + oW8 + (wave * (BN / 8) + j * 16) * 64);
     };
 
     // ---- fragment addressing: lane = (row fr of the 32-row subtile, k-half fh) ----
@@ -123,44 +102,32 @@ __global__ __launch_bounds__(512) void lockstep_kernel(const DenseParams p) {
     int foff[4];
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) foff[ks] = fr * 128 + (((2 * ks + fh) ^ ((fr >> 1) & 7)) << 4);
-    const int a_base = (wm * 32 * MT) * 128;              // + 32*i rows, + kXT for the lo plane
+    const int a_base = (wm * 32 * MT) * 128;              // + 32*i rows
     const int b_base = oW + (wn * 64) * 128;              // + 32*j rows
-    // LO8: a lane's 16 codes of a 32-deep block kb are chunk 2 kb + fh of its row (A and B pair slot by slot, so which sixteen k
+    // A lane's 16 codes of a 32-deep block kb are chunk 2 kb + fh of its row (A and B pair slot by slot, so which sixteen k
     // of the block a lane holds is free as long as both sides agree)
-    [[maybe_unused]] int foff8[2];
+    int foff8[2];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) foff8[kb] = fr * 64 + (((2 * kb + fh) ^ ((fr >> 2) & 3)) << 4);
-    [[maybe_unused]] const int a8_base = kXT + (wm * 32 * MT) * 64, b8_base = oW8 + (wn * 64) * 64;
-    [[maybe_unused]] i16v iacc[LO8 ? MT : 1][LO8 ? NT : 1];
-    if constexpr (LO8) {
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-            for (int j = 0; j < NT; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) iacc[i][j][r] = 0;
-    }
-
+    const int a8_base = kXT + (wm * 32 * MT) * 64, b8_base = oW8 + (wn * 64) * 64;
+    i16v iacc[MT][NT];
     f16v acc[MT][NT];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+            for (int r = 0; r < 16; ++r) { acc[i][j][r] = 0.f; iacc[i][j][r] = 0; }
 
     // ---- main loop: one barrier per K-step, fragment reads one 16-deep slab ahead of the MFMAs ----
     // Two fragment register sets alternate over the 4 slabs of a K-step.  The reads of slab s+1 are issued in front of
     // the MFMAs of slab s, so their LDS latency passes under 4*MT MFMAs of 32 cycles each; the last slab of K-step t is
     // multiplied AFTER the barrier, next to the first reads of K-step t+1 and the LDS-DMA issue of K-step t+2, so the
     // matrix pipe has work while the workgroup re-synchronises.
-    struct Frags { h8 ah[MT], al[TWO ? MT : 1], bw[NT]; };
+    struct Frags { h8 ah[MT], bw[NT]; };
     auto load_frags = [&](Frags& f, const char* buf, int ks) {
 #pragma unroll
-        for (int i = 0; i < MT; ++i) {
-            f.ah[i] = *(const h8*)(buf + a_base + i * 32 * 128 + foff[ks]);
-            if (TWO) f.al[i] = *(const h8*)(buf + kXT + a_base + i * 32 * 128 + foff[ks]);
-        }
+        for (int i = 0; i < MT; ++i) f.ah[i] = *(const h8*)(buf + a_base + i * 32 * 128 + foff[ks]);
 #pragma unroll
         for (int j = 0; j < NT; ++j) f.bw[j] = *(const h8*)(buf + b_base + j * 32 * 128 + foff[ks]);
     };
@@ -169,239 +136,11 @@ __global__ __launch_bounds__(512) void lockstep_kernel(const DenseParams p) {
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.ah[i], f.bw[j], acc[i][j], 0, 0, 0);
-        if (TWO) {
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.al[i], f.bw[j], acc[i][j], 0, 0, 0);
-        }
     };
-    // Pin the issue order of one (reads of the next slab, MFMAs of this slab) pair: a read in front of every MFMA until
-    // the reads run out.  Left alone, hipcc sinks the ds_reads next to their first use and waits lgkmcnt(0) right
-    // behind them (seen in the ISA: four exposed LDS round trips per K-step).
-    auto interleave = [&]() {
-        // one MFMA, then two reads, until the reads run out: every read of the next slab is in flight at least three
-        // MFMAs (~100 cycles) before the wait in front of that slab's first MFMA
-        constexpr int R = MT * (TWO ? 2 : 1) + NT, MF = MT * NT * (TWO ? 2 : 1);
-#pragma unroll
-        for (int k = 0; k < MF; ++k) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                          // one MFMA
-            if (2 * k + 1 < R) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);       // two DS reads
-            else if (2 * k < R) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);      // (an odd one left)
-        }
-    };
-    // The slab multiplied right behind the K-step barrier also carries the LDS-DMA issue of K-step t + 2 (its buffer was just
-    // freed).  Rounds 2-4 issued the 8 (LO8: 11) DMA instructions in one burst in front of that slab's MFMAs: both waves of a SIMD
-    // spend ~60-100 issue cycles per instruction there while the matrix pipe, drained by the barrier, has nothing to do (seen in
-    // the ISA: barrier, 8 x global_load_lds, then the first MFMA).  Round 5 spreads them BETWEEN that slab's MFMAs: one MFMA, two
-    // fragment reads (until they run out), the slab's share of the DMA instructions, next MFMA -- for launches with two fp16 planes
-    // (-0.6 ... -2.6 % per layer at 800 ... 6000 rows); one-plane and int8-residual launches measured 1-5 % SLOWER that way and keep
-    // the burst (profiles/r05_variants.txt).  -DPC_DENSE_SPREAD_DMA=0: the burst everywhere.
-#ifndef PC_DENSE_SPREAD_DMA
-#define PC_DENSE_SPREAD_DMA 1
-#endif
-    // one MFMA / one fragment read / a range of the DMA instructions of a K-step, by index (compile-time after unrolling)
-    auto mfma_one = [&](const Frags& f, int idx) {
-        const int pl = idx / (MT * NT), i = (idx / NT) % MT, j = idx % NT;
-        if (TWO && pl == 1) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.al[i], f.bw[j], acc[i][j], 0, 0, 0);
-        else acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.ah[i], f.bw[j], acc[i][j], 0, 0, 0);
-    };
-    auto read_one = [&](Frags& f, const char* buf, int ks, int idx) {
-        constexpr int NA = MT * (TWO ? 2 : 1);
-        if (idx < NA) {
-            const int i = TWO ? idx >> 1 : idx;
-            if (TWO && (idx & 1)) f.al[i] = *(const h8*)(buf + kXT + a_base + i * 32 * 128 + foff[ks]);
-            else f.ah[i] = *(const h8*)(buf + a_base + i * 32 * 128 + foff[ks]);
-        } else {
-            const int j = idx - NA;
-            f.bw[j] = *(const h8*)(buf + b_base + j * 32 * 128 + foff[ks]);
-        }
-    };
-    auto stage_range = [&](int tl, char* buf, int q0, int q1) {
-        const int t = t0 + tl;
-        const bool tail = ktail && t == nkt - 1;
-        const int64_t ko = (int64_t)t * BK;
-        const int kchunks = tail ? (K - t * BK) / 8 : 8;
-        int q = 0;
-#pragma unroll
-        for (int j = 0; j < NXI; ++j) {
-            const bool ok = !tail || cx[j] < kchunks;
-            if (q >= q0 && q < q1) glds16(ok ? gx[j] + ko : p.zeros, buf + (wave * 16 + j * 8) * 128);
-            ++q;
-            if (TWO) {
-                if (q >= q0 && q < q1) glds16(ok ? gx[j] + lo_delta + ko : p.zeros, buf + kXT + (wave * 16 + j * 8) * 128);
-                ++q;
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < NWI; ++j) {
-            if (q >= q0 && q < q1)
-                glds16((!tail || cw[j] < kchunks) ? gw[j] + ko : gw[j] - cw[j] * 8, buf + oW + (wave * (BN / 8) + j * 8) * 128);
-            ++q;
-        }
-        if constexpr (LO8) {
-            if (q >= q0 && q < q1) glds16((const _Float16*)(gx8 + ko), buf + kXT + wave * 1024);
-            ++q;
-#pragma unroll
-            for (int j = 0; j < NW8; ++j) {
-                if (q >= q0 && q < q1) glds16((const _Float16*)(gw8[j] + ko), buf + oW8 + (wave * (BN / 8) + j * 16) * 64);
-                ++q;
-            }
-        }
-    };
-    if constexpr (PP) {
-        // ---- ping-pong main loop (round 5; the guide's two-waves-per-SIMD regime).  MEASURED SLOWER than the lockstep loop below
-        // on this kernel (0.87-0.90 x with both planes, profiles/r05_dense_pp_ab.txt) in all three forms tried -- fragment reads
-        // waited for inside their load segment; read one phase ahead with hipcc's waits (lgkmcnt(0) every other phase: its
-        // scoreboard merges conservatively at the group branches); read ahead as raw ds_read_b128 with explicit counted waits
-        // (this form) -- kept for A/B behind -DPC_DEV_SWEEPS.  Eight barriers per K-step and one wave per SIMD feeding the
-        // matrix pipe at a time lose to two waves per SIMD interleaving their MFMAs with one barrier per K-step; what is left
-        // between the lockstep loop (1.09-1.15 PFLOP/s executed on random data) and the ~1.3 the guide's 8-phase template
-        // reaches at 4096^3 is not in the wave pairing. ----
-        // The loop above keeps the two waves of a SIMD in lockstep: both issue MFMAs at once (54 % of wave time were issue stalls
-        // behind the shared pipe, profiles/r02_pmc_gemm_dense.txt) and both sit out the barrier and the first fragment reads of
-        // the next K-step together (MFMA pipes busy 63 % of the kernel's cycles).  Here the workgroup's eight waves are two GROUPS
-        // of four (one wave of each group per SIMD) that run the same program ONE BARRIER APART: a K-step is four phases (one
-        // 16-deep slab each), a phase is a LOAD segment (the slab's 6 fragment reads, waited for) and a COMPUTE segment (its 8
-        // MFMAs = 256 matrix-pipe cycles), every segment ends in a raw s_barrier -- so while group 0 is in its compute segment
-        // group 1 is in its load segment and vice versa: the SIMD's matrix pipe always has exactly one wave feeding it, and the
-        // LDS reads, the waits and the barrier latency of one wave pass under the MFMAs of the other.  One fragment register
-        // set instead of two.
-        //   barrier n separates interval n from n + 1.  Group 0: load (t, s) in interval 8t + 2s, compute in 8t + 2s + 1; group 1
-        //   one interval later.  A load segment only ISSUES the fragment reads of the NEXT slab (two register sets); they are
-        //   consumed one phase later, so the segment is a few dozen issue cycles and the LDS latency never sits in front of a
-        //   barrier (first version: reads waited for inside their load segment -- the load segment then took longer than the
-        //   partner's 256-cycle compute segment and the loop ran at ITS pace: 0.81-0.93 x the lockstep loop).
-        //   Slab 0 of K-step t + 1 is read in load (t, 3): group 0 in interval 8t + 6, so K-step t + 1 must have landed, for all
-        //   waves, by barrier 8t + 6: the LDS-DMA goes out in two pieces between MFMAs -- group 0 in compute (t, 0), (t, 1), waited
-        //   for at the end of compute (t, 2); group 1 in load (t, 0) and compute (t, 0), waited for at the end of load (t, 2) -- at
-        //   least two intervals of flight for the last piece.  The buffer it lands in held K-step t - 1, whose last reads (group
-        //   1, issued in its load (t - 1, 2)) are complete at the start of interval 8t: every issue point above lies behind
-        //   barrier 8t + 1.
-        // Same MFMA order per accumulator as the loop above: bit-identical results.
-        constexpr int NI = NXI * (TWO ? 2 : 1) + NWI;          // LDS-DMA instructions per wave and K-step
-        auto stage_piece = [&](int tl, char* buf, int piece) {
-            const int t = t0 + tl;
-            const bool tail = ktail && t == nkt - 1;
-            const int64_t ko = (int64_t)t * BK;
-            const int kchunks = tail ? (K - t * BK) / 8 : 8;
-            const int q0 = piece * NI / 2, q1 = (piece + 1) * NI / 2;
-            int q = 0;
-#pragma unroll
-            for (int j = 0; j < NXI; ++j) {
-                const bool ok = !tail || cx[j] < kchunks;
-                if (q >= q0 && q < q1) glds16(ok ? gx[j] + ko : p.zeros, buf + (wave * 16 + j * 8) * 128);
-                ++q;
-                if (TWO) {
-                    if (q >= q0 && q < q1) glds16(ok ? gx[j] + lo_delta + ko : p.zeros, buf + kXT + (wave * 16 + j * 8) * 128);
-                    ++q;
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < NWI; ++j) {
-                if (q >= q0 && q < q1)
-                    glds16((!tail || cw[j] < kchunks) ? gw[j] + ko : gw[j] - cw[j] * 8, buf + 2 * kXT + (wave * (BN / 8) + j * 8) * 128);
-                ++q;
-            }
-        };
-        const int grp = __builtin_amdgcn_readfirstlane(wave >> 2);
-        Frags fr2[2];                                           // slab s lives in set s & 1: read one phase ahead of its MFMAs
-        // The fragment reads of the ping-pong loop are raw ds_read_b128 statements hipcc does not count: a read issued in load
-        // segment s is consumed in compute segment s + 1 behind an explicit `s_waitcnt lgkmcnt(R)` (R = reads per slab: only
-        // the NEWER slab's reads may still be in flight).  Left to hipcc, the uniform `if (group)` branches between a read and
-        // its use make the waitcnt pass merge its scoreboards conservatively: lgkmcnt(0) in every other phase, i.e. the LDS
-        // latency of the just-issued reads in front of the MFMAs -- what the read-ahead is there to hide.  The loop holds no
-        // other LDS or scalar-memory instruction (checked in the ISA: lgkmcnt counts in order only without SMEM in flight).
-        constexpr int NR = MT * (TWO ? 2 : 1) + NT;
-        const uint32_t lds32 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
-        auto load_frags_raw = [&](Frags& f, uint32_t buf_off, int ks) {
-            const uint32_t aa = lds32 + buf_off + a_base + foff[ks], ab = lds32 + buf_off + b_base + foff[ks];
-#pragma unroll
-            for (int i = 0; i < MT; ++i) {
-                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f.ah[i]) : "v"(aa), "i"(i * 32 * 128));
-                if (TWO) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f.al[i]) : "v"(aa), "i"(kXT + i * 32 * 128));
-            }
-#pragma unroll
-            for (int j = 0; j < NT; ++j) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f.bw[j]) : "v"(ab), "i"(j * 32 * 128));
-        };
-        stage(0, lds);
-        stage(nk > 1 ? 1 : 0, lds + kStage);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // both K-steps (the prologue is not where the time goes)
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-        load_frags_raw(fr2[0], 0, 0);
-        if (grp) {                                              // group 1 runs one interval behind
-            __builtin_amdgcn_sched_barrier(0);
-            __builtin_amdgcn_s_barrier();
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        auto half_a = [&](const Frags& f) {                     // first half of a slab's MFMAs (hi plane; without a lo plane: the first row block)
-#pragma unroll
-            for (int i = 0; i < (TWO ? MT : (MT + 1) / 2); ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.ah[i], f.bw[j], acc[i][j], 0, 0, 0);
-        };
-        auto half_b = [&](const Frags& f) {
-            if (TWO) {
-#pragma unroll
-                for (int i = 0; i < MT; ++i)
-#pragma unroll
-                    for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.al[i], f.bw[j], acc[i][j], 0, 0, 0);
-            } else {
-#pragma unroll
-                for (int i = (MT + 1) / 2; i < MT; ++i)
-#pragma unroll
-                    for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.ah[i], f.bw[j], acc[i][j], 0, 0, 0);
-            }
-        };
-        for (int t = 0; t < nk; ++t) {
-            char* cur = lds + (t & 1) * kStage;
-            char* nxt = lds + ((t + 1) & 1) * kStage;
-            const int u1 = t + 1 < nk ? t + 1 : nk - 1;         // (clamped: past the end the last K-step goes into the idle buffer again)
-#pragma unroll
-            for (int sl = 0; sl < 4; ++sl) {
-                // ---- load segment: only ISSUES the next slab's fragment reads (slab 0 of K-step t + 1 behind slab 3: its DMA was
-                // waited for two barriers ago); they complete under the partner group's MFMAs and this group's own ----
-                if (sl < 3) load_frags_raw(fr2[(sl + 1) & 1], (t & 1) * kStage, sl + 1);
-                else load_frags_raw(fr2[0], ((t + 1) & 1) * kStage, 0);     // (past the last K-step: the clamped re-load of it, never multiplied)
-                if (grp) {
-                    if (sl == 0) stage_piece(u1, nxt, 0);
-                    if (sl == 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                __builtin_amdgcn_s_barrier();
-                __builtin_amdgcn_sched_barrier(0);
-                // ---- compute segment: the slab read one phase ago; the newer slab's NR reads stay in flight ----
-                static_assert(NR == 6 || NR == 4 || NR == 3, "reads per slab");
-                if constexpr (NR == 6) asm volatile("s_waitcnt lgkmcnt(6)" ::: "memory");
-                else if constexpr (NR == 4) asm volatile("s_waitcnt lgkmcnt(4)" ::: "memory");
-                else asm volatile("s_waitcnt lgkmcnt(3)" ::: "memory");
-                __builtin_amdgcn_sched_barrier(0);
-                __builtin_amdgcn_s_setprio(1);
-                half_a(fr2[sl & 1]);
-                __builtin_amdgcn_sched_barrier(0);
-                if (!grp) {
-                    if (sl < 2) stage_piece(u1, nxt, sl);
-                } else {
-                    if (sl == 0) stage_piece(u1, nxt, 1);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                half_b(fr2[sl & 1]);
-                __builtin_amdgcn_s_setprio(0);
-                if (sl == 2 && !grp) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                __builtin_amdgcn_sched_barrier(0);
-                __builtin_amdgcn_s_barrier();
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (the read-ahead behind the last slab: landed before its registers die)
-        if (!grp) {                                             // group 0 waits for group 1's last compute segment
-            __builtin_amdgcn_s_barrier();
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    } else if constexpr (LO8) {
-        // ---- lockstep main loop with the lo plane on the int8 MFMA (round 5) ----
+    // Pin the issue order of one (reads of the next slab, MFMAs of this slab) pair: one MFMA, then two reads, until the reads run out.
+    // Left alone, hipcc sinks the ds_reads next to their first use and waits lgkmcnt(0) right behind them (seen in the ISA: four
+    // exposed LDS round trips per K-step).
+    {
         // Per K-step: 16 fp16 MFMAs for the hi plane (as without a lo plane) + 8 v_mfma_i32_32x32x32_i8 for the residual plane
         // (two 32-deep blocks x MT x NT) instead of 16 more fp16 ones: 24 matrix-pipe slots instead of 32.  One int8 fragment set:
         // block kb is read one slab ahead of its MFMAs like the fp16 fragments (kb 0 next to slab 0, kb 1 next to slab 2).
@@ -419,7 +158,6 @@ __global__ __launch_bounds__(512) void lockstep_kernel(const DenseParams p) {
 #pragma unroll
                 for (int j = 0; j < NT; ++j) iacc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f8.a[i], f8.b[j], iacc[i][j], 0, 0, 0);
         };
-        // (reads of the next slab, MFMAs of this one): one MFMA, then two reads, until the reads run out
         auto pin = [&](auto r_, auto mf_) {
             constexpr int R = decltype(r_)::value, MF = decltype(mf_)::value;
 #pragma unroll
@@ -458,8 +196,8 @@ __global__ __launch_bounds__(512) void lockstep_kernel(const DenseParams p) {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
             const int tn = t + 2 < nk ? t + 2 : nk - 1;
-            // (the DMA issue spread between this slab's MFMAs -- see the fp16 loop below -- measured SLOWER here: 4177 vs 4136 us per
-            // layer at 6000 rows, profiles/r05_variants.txt)
+            // (the DMA issue spread between this slab's MFMAs measured slower: 4177 vs 4136 us per layer at 6000 rows,
+            // profiles/r05_variants.txt)
             stage(tn, lds + (t & 1) * kStage);
             load_frags(fa, lds + ((t + 1) & 1) * kStage, 0);
             load8(lds + ((t + 1) & 1) * kStage, 0);
@@ -500,64 +238,6 @@ __global__ __launch_bounds__(512) void lockstep_kernel(const DenseParams p) {
                     for (int j = 0; j < NT; ++j) acc[i][j][r] = __builtin_fmaf((float)iacc[i][j][r], xs * wsc[j], acc[i][j][r]);
                 }
         }
-    } else {
-    Frags fa, fb;
-    stage(0, lds);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (nk > 1) stage(1, lds + kStage);
-    load_frags(fa, lds, 0);
-    for (int t = 0; t + 1 < nk; ++t) {
-        const char* cur = lds + (t & 1) * kStage;
-        load_frags(fb, cur, 1);
-        mfmas(fa);
-        interleave();
-        load_frags(fa, cur, 2);
-        mfmas(fb);
-        interleave();
-        load_frags(fb, cur, 3);
-        mfmas(fa);
-        interleave();
-        // K-step t+1 has landed (this wave's LDS-DMA drained, then everyone's via the barrier), and every wave's reads
-        // of K-step t are complete (__syncthreads waits lgkmcnt(0)): its buffer may be overwritten.  The stage index
-        // is clamped instead of branched on (past the end it re-loads the last K-step into the idle buffer): a branch
-        // here splits the block and hipcc then waits for the fresh reads below before the MFMAs that do not need them.
-        __builtin_amdgcn_sched_barrier(0);      // slab 2's MFMAs stay in front of the barrier: they cover slab 3's reads
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        const int tn = t + 2 < nk ? t + 2 : nk - 1;
-        if constexpr (PC_DENSE_SPREAD_DMA && TWO) {
-            constexpr int MF = MT * NT * (TWO ? 2 : 1), R = MT * (TWO ? 2 : 1) + NT, V = NXI * (TWO ? 2 : 1) + NWI;
-            const char* nb = lds + ((t + 1) & 1) * kStage;
-#pragma unroll
-            for (int k = 0; k < MF; ++k) {
-                mfma_one(fb, k);
-                __builtin_amdgcn_sched_barrier(0);
-                if (2 * k < R) read_one(fa, nb, 0, 2 * k);
-                if (2 * k + 1 < R) read_one(fa, nb, 0, 2 * k + 1);
-                stage_range(tn, lds + (t & 1) * kStage, k * V / MF, (k + 1) * V / MF);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        } else {
-            stage(tn, lds + (t & 1) * kStage);
-            load_frags(fa, lds + ((t + 1) & 1) * kStage, 0);
-            mfmas(fb);
-            interleave();
-        }
-    }
-    {
-        const char* cur = lds + ((nk - 1) & 1) * kStage;
-        load_frags(fb, cur, 1);
-        mfmas(fa);
-        interleave();
-        load_frags(fa, cur, 2);
-        mfmas(fb);
-        interleave();
-        load_frags(fb, cur, 3);
-        mfmas(fa);
-        interleave();
-        mfmas(fb);
-    }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // (the clamped re-load of the last K-step)
 
@@ -713,15 +393,12 @@ int launch(DenseParams& p, hipStream_t s, int kslices) {
     const int nkt = pc_ceil_div(p.K, BK);
     p.kper = pc_ceil_div(nkt, kslices);
     const dim3 grid(8 * p.mb * pc_ceil_div(p.nb, 8), pc_ceil_div(nkt, p.kper)), block(512);
-    if (p.xl8) {
-        if constexpr (EPI == EPI_GELU) {               // (no caller: the Falcon / MPT stacks keep the fp16 residual plane)
-            pc_set_error("pc_gemm_dense_lo8: no GELU instantiation");
-            return PC_ERR_ARG;
-        } else {
-            hipLaunchKernelGGL((lockstep_kernel<WM, EPI, false, false, true>), grid, block, 0, s, p);
-        }
-    } else if (p.xl) hipLaunchKernelGGL((lockstep_kernel<WM, EPI, true, true>), grid, block, 0, s, p);
-    else hipLaunchKernelGGL((lockstep_kernel<WM, EPI, false, true>), grid, block, 0, s, p);
+    if constexpr (EPI == EPI_GELU) {                   // (no caller: the Falcon / MPT stacks keep the fp16 residual plane)
+        pc_set_error("pc_gemm_dense_lo8: no GELU instantiation");
+        return PC_ERR_ARG;
+    } else {
+        hipLaunchKernelGGL((lockstep_kernel<WM, EPI>), grid, block, 0, s, p);
+    }
     return pc_check_launch("lockstep_kernel");
 }
 }  // namespace lockstep
