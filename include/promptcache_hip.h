@@ -538,9 +538,10 @@ int pc_gemm_dense_a8(const void* xq, int64_t ldx, const void* w_codes, int64_t l
  * replay that reads it has finished. */
 int pc_fetch_block(const void* host_src, void* dst, int32_t nbytes, void* stream);
 
-/* pc_prefill_prologue -- everything a captured small-q forward does before its first layer, as ONE launch reading the call's pinned
- * host block (layout: int64 ids[n_tok] | int32 pos[n_tok] at o_pos | int32 words[8] at o_words = {past_len, tail base, live rows,
- * segments, rows of the row table, ...} | pc_kv_seg[max_seg] at o_segs): the block copied to its device twin (pc_fetch_block), the
+/* pc_prefill_prologue -- everything a captured small-q forward does before its first layer, read from the call's pinned host block
+ * (one launch up to 16 tokens; above, a first launch fetches the block and a second reads its device twin).  Block layout: int64
+ * ids[n_tok] | int32 pos[n_tok] at o_pos | int32 words[8] at o_words = {past_len, tail base, live rows, segments, rows of the row
+ * table, ...} | pc_kv_seg[max_seg] at o_segs.  The block is copied to its device twin (pc_fetch_block); written are the
  * embedding rows of the tokens as the fp32 residual stream x_out [n_tok][hidden] (embed_tokens, llama2.py:869), the (cos, sin)
  * rows of the supplied positions cs_out [n_tok][head_dim/2][2] (pc_rope_table; llama2.py:129-147, :204-207) and -- when `rows` is
  * given -- the staging plan expanded per staged row (pc_kv_row_table; words[3] segments, words[4] rows).  words[5] != 0: the

@@ -99,8 +99,7 @@ __global__ __launch_bounds__(64 * WV, WV == 8 ? 4 : 1) void talk_scores_kernel(p
     const bool mix = a.talk != nullptr;
     const int nsteps = (D + 31) / 32;
 
-    // the key fragments of PG key heads are requested together (one memory round trip per PG heads, not per head), those of the next subtile's
-    // first heads before this one's scores are stored: a load behind a store waits for the store's way to memory
+    // the key fragments of PG key heads are requested together: one memory round trip per PG heads, not per head
     Frag<E> fk[PG][NST];
     auto keys = [&](int j0, int c0) {
         const int jk = j0 + l15;                                  // the key this lane loads (as a B-operand row)

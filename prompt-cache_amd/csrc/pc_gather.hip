@@ -236,12 +236,13 @@ __global__ __launch_bounds__(256) void kv_row_table_kernel(const pc_kv_seg* __re
     rows[r] = row_entry(s_seg, nseg, r, dst, row_bytes, dst_plane_stride16);
 }
 
-// ---- pc_prefill_prologue: everything a captured small-q forward does before its first layer, in ONE launch ------------------
-// Block roles (all of them read the call's PINNED HOST block directly, with system-scope loads: no ordering inside the launch is
-// needed, and the host rewrites the block between replays):
+// ---- pc_prefill_prologue: everything a captured small-q forward does before its first layer --------------------------------
+// One launch up to 16 tokens, two above.  Block roles (up to 16 tokens all of them read the call's PINNED HOST block directly, with
+// system-scope loads: no ordering inside the launch is needed, and the host rewrites the block between replays; above, the block's
+// device twin, which the launch in front has filled):
 //   [0, n_tok)            embedding row of token t as the fp32 residual stream (llama2.py:869; ids from the host block) and its
 //                         (cos, sin) row at the supplied position                           (llama2.py:129-147, :204-207)
-//   n_tok                 the whole block -> its device twin (past length, live rows, ... for the layers' kernels)
+//   n_tok                 the whole block -> its device twin (past length, live rows, ... for the layers' kernels), up to 16 tokens
 //   n_tok + 1 ..          the staging plan expanded to one pc_kv_row per staged row (pc_kv_row_table), when `rows` is given
 typedef __attribute__((address_space(1))) unsigned long long g64;
 __device__ __forceinline__ unsigned long long host_ld8(const void* p) {

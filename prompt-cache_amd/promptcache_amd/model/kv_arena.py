@@ -18,9 +18,6 @@ from typing import List, Optional, Tuple
 
 import torch
 
-# live arenas by the address of their buffer: a caller that hands back plain views (the reference's GenerationEngine
-# rebuilds the list with k.unsqueeze(0), generation_engine.py:101-102) gets the SAME arena object again -- with its
-# residual tail and the hipGraphs keyed on it -- instead of a fresh reconstruction per call
 def uploaded(rows, dtype, device) -> torch.Tensor:
     """Host numbers as a tensor on ``device`` without waiting for its stream: the copy leaves from pinned memory (which torch keeps
     until it is done).  ``torch.tensor(rows, device=...)`` copies from pageable memory and drains the stream first."""
@@ -29,6 +26,9 @@ def uploaded(rows, dtype, device) -> torch.Tensor:
     return torch.tensor(rows, dtype=dtype, pin_memory=True).to(device, non_blocking=True)
 
 
+# live arenas by the address of their buffer: a caller that hands back plain views (the reference's GenerationEngine
+# rebuilds the list with k.unsqueeze(0), generation_engine.py:101-102) gets the SAME arena object again -- with its
+# residual tail and the hipGraphs keyed on it -- instead of a fresh reconstruction per call
 _LIVE: "weakref.WeakValueDictionary[int, KVArena]" = weakref.WeakValueDictionary()
 
 

@@ -59,8 +59,6 @@ def test_dense_store_and_add(M, N, K, two):
     assert np.array_equal(got2[:, N:], base.cpu().numpy()[:, N:].astype(np.float64))
 
 
-# few-row launches of the N = hidden projections take the split-K form when a workspace is supplied (pc_gemm_dense_ws);
-# (1000, 12288, 4096) and (77, 512, 8) do not split (large grid / too few K-steps) and must equal pc_gemm_dense bit for bit
 @pytest.mark.parametrize("M,N,two", [(2001, 8188, False), (2001, 8188, True), (1025, 4100, True), (897, 16388, False)])
 @pytest.mark.parametrize("K", [8, 64, 72, 128, 200, 264])
 def test_dense_tall_tiles_strips_and_short_rings(M, N, K, two):
@@ -87,6 +85,8 @@ def test_dense_tall_tiles_strips_and_short_rings(M, N, K, two):
         assert bool(((oh.double() + ol.double() - want).abs() <= 2.0 ** -19 * (want.abs() + 2.0 ** -6)).all())
 
 
+# few-row launches of the N = hidden projections take the split-K form when a workspace is supplied (pc_gemm_dense_ws);
+# (1000, 12288, 4096) and (77, 512, 8) do not split (large grid / too few K-steps) and must equal pc_gemm_dense bit for bit
 @pytest.mark.parametrize("two", [True, False])
 @pytest.mark.parametrize("M,N,K", [(300, 4096, 4096), (512, 4096, 11008), (130, 260, 1096), (800, 5120, 13824),
                                    (1000, 12288, 4096), (77, 512, 8), (1, 4096, 4096)])
