@@ -89,11 +89,11 @@ __device__ __forceinline__ void glds16(const _Float16* g, char* lds_wave_base) {
                                      (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, 0);
 }
 
-// the block tile of a launch: 2 x 2 waves of 32 MT x 32 NT, S LDS images in the ring (as many as the 160 KiB of a CU hold)
-template <bool TWO, bool NARROW, bool TALL>
+// the block tile of a launch: W x W waves of 32 MT x 32 NT, S LDS images in the ring (as many as the 160 KiB of a CU hold)
+template <int W, bool TWO, bool NARROW, bool TALL>
 struct Tile {
     static constexpr int MT = TALL ? 4 : 2, NT = NARROW ? 2 : 4, S = TWO || TALL ? 2 : 3;
-    static constexpr int BM = 64 * MT, BN = 64 * NT;
+    static constexpr int BM = 32 * W * MT, BN = 32 * W * NT;
 };
 
 // The 64 columns of group `grp` (of the launch's weight rows; EPI_SILU: 32 gate and the matching 32 up features, EPI_ROPE: 32 features of a
@@ -231,11 +231,11 @@ __device__ __forceinline__ void store_group(const DenseParams& p, char* patch, i
     }
 }
 
-// TWO: both activation planes; NARROW: 128 columns instead of 256; TALL: 256 rows instead of 128
-template <int EPI, bool TWO, bool NARROW, bool TALL>
+// W: waves across and down a workgroup; TWO: both activation planes; NARROW: 128 columns instead of 256; TALL: 256 rows instead of 128
+template <int W, int EPI, bool TWO, bool NARROW, bool TALL>
 __global__ __launch_bounds__(256, 1) void gemm_dense_kernel(const DenseParams p) {
-    static_assert(!(TWO && TALL), "two planes of 256 rows and their weights do not fit the LDS twice");
-    using T = Tile<TWO, NARROW, TALL>;
+    static_assert(W == 2 && !(TWO && TALL), "four waves; two planes of 256 rows and their weights do not fit the LDS twice");
+    using T = Tile<W, TWO, NARROW, TALL>;
     constexpr int MT = T::MT, NT = T::NT, S = T::S;
     using L = mfma_tile::Loop<MT, NT, S, TWO ? 2 : 1>;
     constexpr int PL = TWO ? 2 : 1, BM = L::BM, BN = L::BN;
@@ -367,13 +367,13 @@ __global__ __launch_bounds__(256) void dense_reduce_kernel(const float* __restri
 
 template <int EPI, bool TWO, bool NARROW, bool TALL>
 int launch_dense_as(DenseParams& p, hipStream_t s, int kslices) {
-    constexpr int BM = Tile<TWO, NARROW, TALL>::BM, BN = Tile<TWO, NARROW, TALL>::BN;
+    constexpr int BM = Tile<2, TWO, NARROW, TALL>::BM, BN = Tile<2, TWO, NARROW, TALL>::BN;
     p.mb = pc_ceil_div(p.M, BM);
     p.nb = (EPI == EPI_SILU) ? pc_ceil_div(p.nfeat, BN / 2) : pc_ceil_div(p.N, BN);
     const int nkt = pc_ceil_div(p.K, BK);
     p.kper = pc_ceil_div(nkt, kslices);
     p.strips = mfma_tile::strips(p.mb, p.nb, (TWO ? 2 : 1) * BM, BN);
-    hipLaunchKernelGGL((gemm_dense_kernel<EPI, TWO, NARROW, TALL>), dim3(8 * p.strips.mh * p.strips.nh, pc_ceil_div(nkt, p.kper)), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((gemm_dense_kernel<2, EPI, TWO, NARROW, TALL>), dim3(8 * p.strips.mh * p.strips.nh, pc_ceil_div(nkt, p.kper)), dim3(256), 0, s, p);
     return pc_check_launch("gemm_dense_kernel");
 }
 
