@@ -1244,6 +1244,10 @@ class LlamaHIP:
                 self._gather = None
                 self._pre = None
 
+        # What the captures share is made before the first of them, not in it: memory of a capture's own pool, its counters zeroed by that
+        # graph's replays alone -- and a forward captured ahead (_prewarm) is replayed late or never.
+        if self.ks_o or self.ks_down:
+            self._ks_buffers(self.config.hidden_size)
         if eager_first:
             # one eager pass first (loads code objects / sizes the allocator), then capture
             run()

@@ -86,6 +86,24 @@ def test_config3_codellama_theta1e6_squad_like_entries():
         assert err < TOL
 
 
+def test_counters_that_captures_share_are_made_outside_of_them():
+    """A first prompt of two row tiles: the one-tile forwards are captured behind it before any of them has run, and the arrival counters that they
+    share are zero whichever of them is replayed first."""
+    lm = _lm("llama2-7b", layers=1)
+    m, made = lm.hf_model, []
+
+    class Watched(type(m)):
+        def _ks_buffers(self, hid):
+            if self._ks_state is None:
+                made.append(torch.cuda.is_current_stream_capturing())
+            return super()._ks_buffers(hid)
+
+    m.__class__ = Watched
+    ids = torch.randint(3, 32000, (1, 24), generator=torch.Generator().manual_seed(6))
+    m(input_ids=ids, position_ids=torch.arange(24).unsqueeze(0), use_cache=True)
+    assert made == [False] and any(k[1] == 16 for k in m._graphs) and int(m._ks_state[1].abs().max()) == 0
+
+
 def test_config4_13b_shape_8k_context_dense_path():
     """q ~ 260 > 64 rows: dense projections + the general attention kernel over 8k staged keys."""
     from promptcache_amd import synth
