@@ -42,6 +42,47 @@ __device__ __forceinline__ void block_sum(float (&v)[NV], float* red) {
     }
 }
 
+// The same for kernels that hold their row in registers: sums over a wave by DPP within sixteen lanes and two shuffles, one barrier (a kernel gives
+// each of its sums a `red` of its own).
+template <int NV>
+__device__ __forceinline__ void row_sum(float (&v)[NV], float* red) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        v[i] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v[i]), 0xb1, 0xf, 0xf, true));       // quad_perm [1,0,3,2]
+        v[i] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v[i]), 0x4e, 0xf, 0xf, true));       // quad_perm [2,3,0,1]
+        v[i] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v[i]), 0x141, 0xf, 0xf, true));      // row_half_mirror
+        v[i] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v[i]), 0x140, 0xf, 0xf, true));      // row_mirror
+        v[i] += __shfl_xor(v[i], 16, 64);
+        v[i] += __shfl_xor(v[i], 32, 64);
+    }
+    if (lane == 0) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) red[wave * NV + i] = v[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NV; ++i) v[i] = red[i];
+    for (int w = 1; w < waves; ++w) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) v[i] += red[w * NV + i];
+    }
+}
+__device__ __forceinline__ f4 ld4(const float* p) { return *reinterpret_cast<const f4*>(p); }
+
+// Threads and four-column chunks per thread of a kernel that holds a row of `width` columns in registers; false: too wide.  Few rows (decoding)
+// are one chunk per thread wherever 1024 threads reach: such a launch lasts as long as one row's chain.  Many rows fill the chip anyhow, and 256
+// threads with more chunks each have fewer waves to meet at the barriers.
+inline bool row_threads(int width, int n_rows, int max_chunks, int* threads, int* chunks) {
+    const int pieces = width / 4;
+    int t = n_rows <= 512 || pieces > 256 * max_chunks ? 1024 : 256;
+    if (pieces < t) t = (pieces + 63) / 64 * 64;
+    int c = 1;
+    while (c * t < pieces) c *= 2;
+    *threads = t, *chunks = c;
+    return width % 4 == 0 && c <= max_chunks;
+}
+
 template <typename E>
 __global__ __launch_bounds__(256) void embed_rows_kernel(const E* __restrict__ table, const int32_t* __restrict__ ids,
                                                          float* __restrict__ out, int width, int vocab, float scale = 1.0f) {
@@ -84,6 +125,63 @@ __global__ __launch_bounds__(1024) void mix_norm_kernel(pcb_mix_norm_args a) {
     }
 }
 
+// The same with the row in registers, NC chunks of four columns per thread (width % 4 == 0, rows aligned to the chunks).  Streams and gains are
+// requested together, four streams at a time, so that a launch of one row costs one trip to memory and one sum: one row of 1024, five
+// streams, 6.7 us column by column through LDS, 3.3 so; 2048 rows of 2048, 19.1 and 15.4.
+template <typename E, int NC>
+__global__ __launch_bounds__(1024) void mix_norm_chunks_kernel(pcb_mix_norm_args a) {
+    __shared__ float red[16];
+    const int r = blockIdx.x, W = a.width, nt = a.n_terms;
+    const int64_t src = a.rows ? a.rows[r] : r;
+    const float* __restrict__ hist = a.hist + src * W;
+    const float* __restrict__ coef = a.coef;
+    int c[NC];
+    f4 x[NC], g1[NC], g2[NC];
+    float ss[1] = {0.0f};
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+        c[k] = 4 * (threadIdx.x + k * blockDim.x);
+        const int at = c[k] < W ? c[k] : 0;
+        x[k] = f4{0.f, 0.f, 0.f, 0.f};
+        if (nt == 0) x[k] = ld4(hist + at);
+        if (a.out1) g1[k] = ld4(a.gain1 + at);
+        if (a.out2) g2[k] = ld4(a.gain2 + at);
+    }
+    for (int j0 = 0; j0 < nt; j0 += 4) {
+        f4 v[NC][4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int k = 0; k < NC; ++k)
+                if (j0 + u < nt) v[k][u] = ld4(hist + (j0 + u) * a.hist_stride + (c[k] < W ? c[k] : 0));
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (j0 + u < nt) {
+                const float w = coef[j0 + u];
+#pragma unroll
+                for (int k = 0; k < NC; ++k)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[k][e] += w * v[k][u][e];
+            }
+    }
+#pragma unroll
+    for (int k = 0; k < NC; ++k)
+        if (c[k] < W) {
+            if (a.x_out) *reinterpret_cast<f4*>(a.x_out + (int64_t)r * W + c[k]) = x[k];
+            ss[0] += (x[k][0] * x[k][0] + x[k][1] * x[k][1]) + (x[k][2] * x[k][2] + x[k][3] * x[k][3]);
+        }
+    row_sum<1>(ss, red);
+    const float inv = 1.0f / sqrtf(ss[0] / (float)W + a.eps);
+#pragma unroll
+    for (int k = 0; k < NC; ++k)
+        if (c[k] < W) {
+            const f4 v = x[k] * inv;
+            const int64_t at = (int64_t)r * W + c[k];
+            if (a.out1) store4((E*)a.out1 + at, v[0] * g1[k][0], v[1] * g1[k][1], v[2] * g1[k][2], v[3] * g1[k][3]);
+            if (a.out2) store4((E*)a.out2 + at, v[0] * g2[k][0], v[1] * g2[k][1], v[2] * g2[k][2], v[3] * g2[k][3]);
+        }
+}
+
 template <typename E>
 __global__ __launch_bounds__(1024) void polynorm_kernel(const float* __restrict__ z, const float* __restrict__ coef, E* __restrict__ out,
                                                        float eps, int ff) {
@@ -106,6 +204,49 @@ __global__ __launch_bounds__(1024) void polynorm_kernel(const float* __restrict_
         const float v = zr[c], v2 = v * v;
         out[r * ff + c] = from_f32<E>(i1 * v + i2 * v2 + i3 * (v2 * v) + c3);
     }
+}
+
+// The row in registers, as above: read once.  One row of 4096 5.5 us, 4.1 so; 2048 rows of 8192 30.5, 17.6 so (101 MB).
+template <typename E, int NC>
+__global__ __launch_bounds__(1024) void polynorm_chunks_kernel(const float* __restrict__ z, const float* __restrict__ coef, E* __restrict__ out,
+                                                              float eps, int ff) {
+    __shared__ float red[48];
+    const int64_t r = blockIdx.x;
+    const float* zr = z + r * ff;
+    f4 v[NC];
+    int c[NC];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+        c[k] = 4 * (threadIdx.x + k * blockDim.x);
+        v[k] = f4{0.f, 0.f, 0.f, 0.f};
+        if (c[k] < ff) v[k] = ld4(zr + c[k]);
+    }
+    const float c0 = coef[0], c1 = coef[1], c2 = coef[2], c3 = coef[3];
+    float s[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int k = 0; k < NC; ++k)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float x = v[k][e], x2 = x * x, x3 = x2 * x;
+            s[0] += x2;
+            s[1] += x2 * x2;
+            s[2] += x3 * x3;
+        }
+    row_sum<3>(s, red);
+    const float i1 = c0 / sqrtf(s[0] / (float)ff + eps);
+    const float i2 = c1 / sqrtf(s[1] / (float)ff + eps);
+    const float i3 = c2 / sqrtf(s[2] / (float)ff + eps);
+#pragma unroll
+    for (int k = 0; k < NC; ++k)
+        if (c[k] < ff) {
+            f4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float x = v[k][e], x2 = x * x;
+                o[e] = i1 * x + i2 * x2 + i3 * (x2 * x) + c3;
+            }
+            store4(out + r * ff + c[k], o[0], o[1], o[2], o[3]);
+        }
 }
 
 // one wave per row of router logits: sigmoid scores in LDS, `top` rounds of a wave-wide arg-max
@@ -222,6 +363,23 @@ PCB_EXPORT int pcb_mix_norm(const pcb_mix_norm_args* a, void* stream) {
     if (a->n_rows == 0) return PCB_OK;
     PCB_REQUIRE(a->hist && (a->n_terms == 0 || a->coef) && (!a->out1 || a->gain1) && (!a->out2 || a->gain2), PCB_ERR_ARG,
                 "pcb_mix_norm: null pointer");
+    const uintptr_t e4 = a->dtype == PCB_BF16 ? 8 : 16;              // (four elements of E)
+    int th, nc;
+    if (row_threads(a->width, a->n_rows, 4, &th, &nc) && a->hist_stride % 4 == 0 &&
+        ((uintptr_t)a->hist | (uintptr_t)a->x_out | (uintptr_t)a->gain1 | (uintptr_t)a->gain2) % 16 == 0 &&
+        ((uintptr_t)a->out1 | (uintptr_t)a->out2) % e4 == 0) {
+        auto go = [&](auto e) {
+            using E = decltype(e);
+            if (nc == 1)
+                hipLaunchKernelGGL((mix_norm_chunks_kernel<E, 1>), dim3(a->n_rows), dim3(th), 0, (hipStream_t)stream, *a);
+            else if (nc == 2)
+                hipLaunchKernelGGL((mix_norm_chunks_kernel<E, 2>), dim3(a->n_rows), dim3(th), 0, (hipStream_t)stream, *a);
+            else
+                hipLaunchKernelGGL((mix_norm_chunks_kernel<E, 4>), dim3(a->n_rows), dim3(th), 0, (hipStream_t)stream, *a);
+        };
+        if (a->dtype == PCB_BF16) go(bf16_t{}); else go(0.0f);
+        return pcb_check_launch("mix_norm_chunks_kernel");
+    }
     const size_t lds = (size_t)a->width * sizeof(float);
     // few rows: a row's columns are spread over up to 1024 threads (the loads of a thread's columns are a dependent chain)
     const dim3 threads(a->n_rows <= 512 && a->width > 1024 ? 1024 : 256);
@@ -237,6 +395,22 @@ PCB_EXPORT int pcb_polynorm(const float* z, const float* coef, void* out, int32_
     PCB_REQUIRE(PCB_DTYPE_OK(dtype) && n_rows >= 0 && ff > 0, PCB_ERR_ARG, "pcb_polynorm: bad sizes");
     if (n_rows == 0) return PCB_OK;
     PCB_REQUIRE(z && coef && out, PCB_ERR_ARG, "pcb_polynorm: null pointer");
+    int th, nc;
+    if (row_threads(ff, n_rows, 8, &th, &nc) && (uintptr_t)z % 16 == 0 && (uintptr_t)out % (dtype == PCB_BF16 ? 8 : 16) == 0) {
+        auto go = [&](auto e) {
+            using E = decltype(e);
+            if (nc == 1)
+                hipLaunchKernelGGL((polynorm_chunks_kernel<E, 1>), dim3(n_rows), dim3(th), 0, (hipStream_t)stream, z, coef, (E*)out, eps, ff);
+            else if (nc == 2)
+                hipLaunchKernelGGL((polynorm_chunks_kernel<E, 2>), dim3(n_rows), dim3(th), 0, (hipStream_t)stream, z, coef, (E*)out, eps, ff);
+            else if (nc == 4)
+                hipLaunchKernelGGL((polynorm_chunks_kernel<E, 4>), dim3(n_rows), dim3(th), 0, (hipStream_t)stream, z, coef, (E*)out, eps, ff);
+            else
+                hipLaunchKernelGGL((polynorm_chunks_kernel<E, 8>), dim3(n_rows), dim3(th), 0, (hipStream_t)stream, z, coef, (E*)out, eps, ff);
+        };
+        if (dtype == PCB_BF16) go(bf16_t{}); else go(0.0f);
+        return pcb_check_launch("polynorm_chunks_kernel");
+    }
     const dim3 threads(n_rows <= 512 && ff > 1024 ? 1024 : 256);
     if (dtype == PCB_BF16)
         hipLaunchKernelGGL(polynorm_kernel<bf16_t>, dim3(n_rows), threads, 0, (hipStream_t)stream, z, coef, (bf16_t*)out, eps, ff);
@@ -548,6 +722,114 @@ __global__ __launch_bounds__(1024) void post_norm_kernel(pcb_post_norm_args a) {
     for (int c = threadIdx.x; c < W; c += blockDim.x) o[c] = from_f32<E>(row[c] * inv * a.gain[c]);
 }
 
+// The same with the row in registers (width % 4 == 0, every row aligned to chunks of four columns): both halves' operands are requested before
+// the first sum.  us, column by column through LDS (three dependent trips to memory) and so: 8 rows of 2048 7.2 and 4.6, 2400 rows
+// 23.6 and 16.1 (79 MB: the copy rate).
+template <typename E, int NC>
+__global__ __launch_bounds__(1024) void post_norm_chunks_kernel(pcb_post_norm_args a) {
+    __shared__ float red[3][16];
+    const int r = blockIdx.x, W = a.width;
+    const int64_t src = a.rows ? a.rows[r] : r;
+    const bool write = a.y || a.pair || a.add, norm = a.out && a.gain;
+    float* __restrict__ x = a.x + src * W;
+    const float* __restrict__ y = a.y ? a.y + src * W : nullptr;
+    const float* __restrict__ add = a.add ? a.add + src * W : nullptr;
+    const E* __restrict__ g = a.gate ? (const E*)a.gate + src * a.ldg : nullptr;
+    const float* __restrict__ pair = a.pair ? a.pair + src * a.pair_top * W : nullptr;
+    const float* __restrict__ pw = a.pair ? a.pair_weight + src * a.pair_top : nullptr;
+    int c[NC];
+    f4 t[NC], v[NC], ad[NC], pg[NC], gn[NC], bi[NC];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+        c[k] = 4 * (threadIdx.x + k * blockDim.x);
+        const int at = c[k] < W ? c[k] : 0;
+        t[k] = f4{0.f, 0.f, 0.f, 0.f};
+        if (y) t[k] = ld4(y + at);
+        v[k] = ld4(x + at);
+        if (add) ad[k] = ld4(add + at);
+        if (a.post_gain) pg[k] = ld4(a.post_gain + at);
+        if (norm) gn[k] = ld4(a.gain + at);
+        if (norm && a.layer_norm && a.bias) bi[k] = ld4(a.bias + at);
+    }
+    if (write) {
+        float gt[NC][4];
+#pragma unroll
+        for (int k = 0; k < NC; ++k)
+            if (g) load4(g + (c[k] < W ? c[k] : 0), true, 4, gt[k]);
+        if (pair)
+            for (int j = 0; j < a.pair_top; ++j) {
+                const float w = pw[j];
+#pragma unroll
+                for (int k = 0; k < NC; ++k) {
+                    const f4 pv = ld4(pair + (int64_t)j * W + (c[k] < W ? c[k] : 0));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) t[k][e] += w * pv[e];
+                }
+            }
+        if (g) {
+#pragma unroll
+            for (int k = 0; k < NC; ++k)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) t[k][e] *= gt[k][e];
+        }
+        float inv = 1.0f;
+        if (a.post_gain) {
+            float ss[1] = {0.0f};
+#pragma unroll
+            for (int k = 0; k < NC; ++k)
+                if (c[k] < W) ss[0] += (t[k][0] * t[k][0] + t[k][1] * t[k][1]) + (t[k][2] * t[k][2] + t[k][3] * t[k][3]);
+            row_sum<1>(ss, red[0]);
+            inv = 1.0f / sqrtf(ss[0] / (float)W + a.eps);
+        }
+        const float ys = a.y_scale;
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[k][e] += ys * (a.post_gain ? t[k][e] * inv * pg[k][e] : t[k][e]);
+                if (add) v[k][e] += ad[k][e];
+            }
+            if (!a.rows && c[k] < W) *reinterpret_cast<f4*>(x + c[k]) = v[k];
+        }
+    }
+    if (a.x_out) {
+#pragma unroll
+        for (int k = 0; k < NC; ++k)
+            if (c[k] < W) *reinterpret_cast<f4*>(a.x_out + (int64_t)r * W + c[k]) = v[k];
+    }
+    if (!a.out) return;
+    E* o = (E*)a.out + (int64_t)r * (a.ldo > 0 ? a.ldo : W);
+    float mean = 0.0f, inv = 1.0f;
+    if (norm) {
+        float ss[1];
+        if (a.layer_norm) {
+            ss[0] = 0.0f;
+#pragma unroll
+            for (int k = 0; k < NC; ++k)
+                if (c[k] < W) ss[0] += (v[k][0] + v[k][1]) + (v[k][2] + v[k][3]);
+            row_sum<1>(ss, red[1]);
+            mean = ss[0] / (float)W;
+        }
+        ss[0] = 0.0f;
+#pragma unroll
+        for (int k = 0; k < NC; ++k)
+            if (c[k] < W) {
+                const f4 d = v[k] - mean;
+                ss[0] += (d[0] * d[0] + d[1] * d[1]) + (d[2] * d[2] + d[3] * d[3]);
+            }
+        row_sum<1>(ss, red[2]);
+        inv = 1.0f / sqrtf(ss[0] / (float)W + a.eps);
+    }
+#pragma unroll
+    for (int k = 0; k < NC; ++k)
+        if (c[k] < W) {
+            f4 w = v[k];
+            if (norm) w = (w - mean) * inv * gn[k];
+            if (norm && a.layer_norm && a.bias) w += bi[k];
+            store4(o + c[k], w[0], w[1], w[2], w[3]);
+        }
+}
+
 // one wave per row: scores and choice scores in LDS, group maxima by lanes, then rounds of a wave-wide arg-max
 __global__ __launch_bounds__(256) void router_select_kernel(const float* __restrict__ logits, int n_rows, int n_out, int top, int score_fn,
                                                             const float* __restrict__ correction, int groups, int keep, int renorm,
@@ -769,6 +1051,23 @@ PCB_EXPORT int pcb_post_norm(const pcb_post_norm_args* a, void* stream) {
                 PCB_ERR_ARG, "pcb_post_norm: null pointer (a gate and a norm after the sublayer need its result, a norm its gain)");
     PCB_REQUIRE((!a->pair || (a->pair_weight && a->pair_top > 0)) && (a->ldo == 0 || a->ldo >= a->width), PCB_ERR_ARG,
                 "pcb_post_norm: pairs need their weights and their number per row; output rows may not overlap");
+    const uintptr_t e4 = a->dtype == PCB_BF16 ? 8 : 16;              // (four elements of E)
+    int th, nc;
+    if (row_threads(a->width, a->n_rows, 4, &th, &nc) && (!a->gate || a->ldg % 4 == 0) && a->ldo % 4 == 0 &&
+        ((uintptr_t)a->x | (uintptr_t)a->y | (uintptr_t)a->add | (uintptr_t)a->pair | (uintptr_t)a->post_gain | (uintptr_t)a->gain |
+         (uintptr_t)a->bias | (uintptr_t)a->x_out) % 16 == 0 && ((uintptr_t)a->gate | (uintptr_t)a->out) % e4 == 0) {
+        auto go = [&](auto e) {
+            using E = decltype(e);
+            if (nc == 1)
+                hipLaunchKernelGGL((post_norm_chunks_kernel<E, 1>), dim3(a->n_rows), dim3(th), 0, (hipStream_t)stream, *a);
+            else if (nc == 2)
+                hipLaunchKernelGGL((post_norm_chunks_kernel<E, 2>), dim3(a->n_rows), dim3(th), 0, (hipStream_t)stream, *a);
+            else
+                hipLaunchKernelGGL((post_norm_chunks_kernel<E, 4>), dim3(a->n_rows), dim3(th), 0, (hipStream_t)stream, *a);
+        };
+        if (a->dtype == PCB_BF16) go(bf16_t{}); else go(0.0f);
+        return pcb_check_launch("post_norm_chunks_kernel");
+    }
     const size_t lds = (size_t)a->width * sizeof(float);
     const dim3 threads(a->n_rows <= 512 && a->width > 1024 ? 1024 : 256);
     if (a->dtype == PCB_BF16)
