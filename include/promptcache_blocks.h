@@ -528,6 +528,31 @@ int pcb_mlstm(const pcb_mlstm_args* a, void* stream);
 int pcb_mlstm_chain(const float* local, const float* log_f_sum, float* start, const float* state, int64_t slot_stride, const int32_t* chains,
                     int32_t n_chains, int32_t H, int32_t dim, int32_t vdim, void* stream);
 
+/* pcb_mlstm and the output norm behind it in one, h = pcb_mlstm's output of a (token, head), vdim columns:
+ *   out[row][h * vdim + c] = E( h[c] / sqrt(mean(h^2) + eps) * (gain ? gain[h * vdim + c] : 1) * (gate ? gate[row][h * vdim + c] : 1) )
+ * gate E rows of stride ldg, out E rows of stride ldo. */
+typedef struct pcb_mlstm_norm_args {
+    uint32_t struct_bytes;
+    const float* gain;
+    const void* gate;
+    int64_t ldg;
+    void* out;
+    int64_t ldo;
+    float eps;
+} pcb_mlstm_norm_args;
+
+/* One token per request (reqs as in pcb_mlstm; their token counts are not read): a->out, a->from_nothing, a->log_f_sum and a->end_slots are not
+ * used.  dim, vdim <= 256, one of them <= 128; vdim, ldv multiples of 4, v aligned to four elements. */
+int pcb_mlstm_step(const pcb_mlstm_args* a, const pcb_mlstm_norm_args* o, void* stream);
+
+/* Prompts cut into segments: a->reqs are the segments {segment, -, tokens <= max_tokens, first flat row}, numbered as they lie in the table,
+ * chains as in pcb_mlstm_chain, a->state the slots' states (read where a chain's first position > 0, and left behind its last token), a->end_slots
+ * int32 [n_reqs] the slot of every last segment and -1 elsewhere, a->end_state the same as a->state.  Scratch: local, start fp32
+ * [segments][H][record], f_sum fp32 [segments][H].  a->out, a->from_nothing and a->log_f_sum are not used.  dim, vdim <= 128 and multiples of 8, rows
+ * of q, k, v aligned to 16 bytes, gate and out to four elements; max_tokens <= 256. */
+int pcb_mlstm_prompt(const pcb_mlstm_args* a, const pcb_mlstm_norm_args* o, const int32_t* chains, int32_t n_chains, int32_t max_tokens,
+                     float* local, float* f_sum, float* start, void* stream);
+
 /* Linear attention whose decay changes from token to token, with a matrix state per (slot, head):
  *   S_t = diag(exp(l_t)) S_(t-1) + k_t (s_t v_t)^T,   o_t = S_t^T (q_scale q_t)        (S: [dim][vdim], fp32, zero before position 0)
  * l_t = ld_coef[h] * ld[row][h * dcols + (dcols == 1 ? 0 : d)] is the log decay of key row d (ld_coef null: 1): dcols = dim gives every

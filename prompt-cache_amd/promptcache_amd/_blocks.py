@@ -128,6 +128,11 @@ class MlstmArgs(C.Structure):
                 ("from_nothing", _i32), ("log_f_sum", _vp), ("end_slots", _vp), ("end_state", _vp), ("end_slot_stride", _i64)]
 
 
+class MlstmNormArgs(C.Structure):
+    """``pcb_mlstm_norm_args`` (field for field)."""
+    _fields_ = [("struct_bytes", C.c_uint32), ("gain", _vp), ("gate", _vp), ("ldg", _i64), ("out", _vp), ("ldo", _i64), ("eps", _f32)]
+
+
 class GlaArgs(C.Structure):
     """``pcb_gla_args`` (field for field)."""
     _fields_ = [("struct_bytes", C.c_uint32), ("dtype", _i32),
@@ -207,6 +212,8 @@ SIGNATURES = {
     "pcb_post_norm": (C.c_int, [C.POINTER(PostNormArgs), _vp]),
     "pcb_head_prep": (C.c_int, [C.POINTER(HeadPrepArgs), _vp]),
     "pcb_mlstm": (C.c_int, [C.POINTER(MlstmArgs), _vp]),
+    "pcb_mlstm_step": (C.c_int, [C.POINTER(MlstmArgs), C.POINTER(MlstmNormArgs), _vp]),
+    "pcb_mlstm_prompt": (C.c_int, [C.POINTER(MlstmArgs), C.POINTER(MlstmNormArgs), _vp, _i32, _i32, _vp, _vp, _vp, _vp]),
     "pcb_mlstm_chain": (C.c_int, [_vp, _vp, _vp, _vp, _i64, _vp, _i32, _i32, _i32, _i32, _vp]),
     "pcb_gla": (C.c_int, [C.POINTER(GlaArgs), _vp]),
     "pcb_attn_prompt": (C.c_int, [C.POINTER(AttnPromptArgs), _vp]),
@@ -754,6 +761,59 @@ def mlstm_chain(local: torch.Tensor, log_f_sum: torch.Tensor, start: torch.Tenso
     assert log_f_sum.numel() >= local.shape[0] * H and chains.numel() >= 4 * n_chains
     check(load().pcb_mlstm_chain(_p(local), _p(log_f_sum), _p(start), _p(state), rec, _p(chains), n_chains, H, dim, vdim, _stream()),
           "pcb_mlstm_chain")
+
+
+def _mlstm_normed(name, cols, ld, reqs, n_reqs, state, H, dim, vdim, q_scale, gate_cap, gain, gate, ldg, out, eps, end_slots=None):
+    q, k, v, gi, gf = cols
+    _want(reqs, torch.int32, name + " reqs"); _want(state, torch.float32, name + " state"); _want(gain, torch.float32, name + " gain")
+    _want(end_slots, torch.int32, name + " end_slots")
+    assert end_slots is None or end_slots.numel() >= n_reqs
+    assert q.dtype == k.dtype == v.dtype == gi.dtype == gf.dtype == out.dtype and q.is_cuda and reqs.numel() >= 4 * n_reqs
+    assert gate is None or gate.dtype == out.dtype
+    assert state[0].numel() == mlstm_state_floats(H, dim, vdim) and out.shape[-1] == H * vdim and out.is_contiguous()
+    assert gain is None or gain.numel() == H * vdim
+    a = MlstmArgs(C.sizeof(MlstmArgs), _code(q), _p(q), _p(k), _p(v), _p(gi), _p(gf), ld, ld, ld, ld, ld, _p(reqs), n_reqs, _p(state),
+                  state[0].numel(), H, dim, vdim, float(q_scale), float(gate_cap), None, 0, 0, None, _p(end_slots),
+                  _p(state) if end_slots is not None else None, state[0].numel() if end_slots is not None else 0)
+    return a, MlstmNormArgs(C.sizeof(MlstmNormArgs), _p(gain), _p(gate), ldg, _p(out), H * vdim, float(eps))
+
+
+def mlstm_step_fits(dim: int, vdim: int, ld: int, v: torch.Tensor) -> bool:
+    """Whether ``mlstm_step`` takes these sizes (``v`` a column block of rows ``ld`` elements apart)."""
+    return dim <= 256 and vdim <= 256 and min(dim, vdim) <= 128 and vdim % 4 == 0 and ld % 4 == 0 and v.data_ptr() % (4 * v.element_size()) == 0
+
+
+def mlstm_step(cols, ld: int, reqs: torch.Tensor, n_reqs: int, state: torch.Tensor, H: int, dim: int, vdim: int, q_scale: float, gate_cap: float,
+               gain: Optional[torch.Tensor], gate: Optional[torch.Tensor], ldg: int, out: torch.Tensor, eps: float) -> None:
+    """One token per request through the matrix memory, the norm per head and the gate: ``cols`` = (q, k, v, gi, gf) as in ``mlstm``, ``out``
+    E [rows, H * vdim]."""
+    a, o = _mlstm_normed("mlstm_step", cols, ld, reqs, n_reqs, state, H, dim, vdim, q_scale, gate_cap, gain, gate, ldg, out, eps)
+    check(load().pcb_mlstm_step(C.byref(a), C.byref(o), _stream()), "pcb_mlstm_step")
+
+
+def mlstm_prompt_fits(dim: int, vdim: int, ld: int, cols, gate: torch.Tensor, max_tokens: int) -> bool:
+    """Whether ``mlstm_prompt`` takes these sizes and this alignment (``cols`` and ``gate``: column blocks of rows ``ld`` elements apart)."""
+    es = cols[0].element_size()
+    return dim <= 128 and vdim <= 128 and dim % 8 == 0 and vdim % 8 == 0 and max_tokens <= 256 and ld * es % 16 == 0 and \
+        all(c.data_ptr() % 16 == 0 for c in cols[:3]) and gate.data_ptr() % (4 * es) == 0
+
+
+def mlstm_prompt(cols, ld: int, segments: torch.Tensor, n_segments: int, chains: torch.Tensor, n_chains: int, max_tokens: int, end_slots: torch.Tensor,
+                 state: torch.Tensor, H: int, dim: int, vdim: int, q_scale: float, gate_cap: float, gain: Optional[torch.Tensor],
+                 gate: Optional[torch.Tensor], ldg: int, out: torch.Tensor, eps: float, local: torch.Tensor, f_sum: torch.Tensor,
+                 start: torch.Tensor) -> None:
+    """Prompts in segments of up to ``max_tokens`` tokens, norm and gate included.  ``segments`` int32 {number, -, tokens, first row}; ``chains`` as in
+    ``mlstm_chain``; ``end_slots`` int32: the slot of every request's last segment, -1 elsewhere; scratch ``local``, ``start`` fp32 [segments,
+    mlstm_state_floats], ``f_sum`` fp32 [segments, H]."""
+    a, o = _mlstm_normed("mlstm_prompt", cols, ld, segments, n_segments, state, H, dim, vdim, q_scale, gate_cap, gain, gate, ldg, out, eps, end_slots)
+    _want(chains, torch.int32, "mlstm_prompt chains")
+    rec = mlstm_state_floats(H, dim, vdim)
+    for t, n in ((local, rec), (start, rec), (f_sum, H)):
+        _want(t, torch.float32, "mlstm_prompt scratch")
+        assert t.numel() >= n_segments * n
+    assert chains.numel() >= 4 * n_chains
+    check(load().pcb_mlstm_prompt(C.byref(a), C.byref(o), _p(chains), n_chains, max_tokens, _p(local), _p(f_sum), _p(start), _stream()),
+          "pcb_mlstm_prompt")
 
 
 def gla(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ld: torch.Tensor, lds_: tuple, dcols: int, reqs: torch.Tensor, n_reqs: int,

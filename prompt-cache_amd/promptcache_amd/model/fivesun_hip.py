@@ -27,8 +27,9 @@ same projection as the mixer's inputs (or is one projection beside the feed-forw
                 key part read from the cached rows, times sigmoid(g)); for the others the up-projections are folded into the query
                 and the output: q'_h = W_uk,h^T q_h, attention of [q'_h | q_rot,h] over the cached rows with the latent itself as
                 value (pcb_attn_latent, sliding window), o_h = W_uv,h (.), times sigmoid(g).  Heads too wide for the tiles fold always
-    mlstm       q | k | v | i | f | g | r = ONE projection; pcb_mlstm: the gated matrix memory token by token; per-head unit RMS,
-                gain, sigmoid(g) (pcb_gated_norm)
+    mlstm       q | k | v | i | f | g | r = ONE projection; the gated matrix memory, per-head unit RMS, gain, sigmoid(g): in segments on the
+                matrix cores (pcb_mlstm_prompt), one token per request (pcb_mlstm_step), or, for sizes these do not take, token by
+                token (pcb_mlstm, pcb_gated_norm)
     dense ff    act(W_gate h + b) * (W_up h + b) in one projection's epilogue, then W_down (.) + b
 
 and the logits are ``head . rms(x) g`` for the rows that were asked for.
@@ -69,7 +70,11 @@ def rotary_frequencies(base: float, dims: int, factor: float = 1.0, original: fl
 
 class FivesunHIP(SlotModel):
     GRAPH_MAX_ROWS = 64
-    SEGMENT = int(os.environ.get("PC_FS_SEGMENT", "64"))    # a step that brings a request more tokens than this runs its mLSTM layers segment-parallel
+    # Tokens of a segment of the mLSTM layers.  Where all of them fit the matrix cores' kernels (_mlstm_fits), a step that brings a request more than
+    # FEW_TOKENS runs them in segments, else one that brings more than SEGMENT; the others go token by token.  us, token by token / in segments, 16
+    # heads of 128, one request and eight: 8 tokens 23.1 / 24.3 and 23.9 / 30.6, 16 30.8 / 24.5 and 32.1 / 30.8, 64 78.9 / 32.7 and 81.6 / 42.3.
+    FEW_TOKENS = 12
+    SEGMENT = int(os.environ.get("PC_FS_SEGMENT", "64"))
     MAX_SEGMENTS = 128      # (segments grow beyond SEGMENT tokens rather than exceed this many per request)
     PROMPT_ROWS = int(os.environ.get("PC_FS_PROMPT_ROWS", "16"))   # a request that brings fewer tokens than this attends row by row (see _tiled)
     # Rebuilt keys and values that lie in memory at a time: beyond it heads take turns, which leaves part of the chip idle (eight requests of 256
@@ -166,7 +171,14 @@ class FivesunHIP(SlotModel):
         reach = [mask for _, _, mask, _ in self._lat]
         self._reach = 0 if not reach or min(reach) <= 0 else max(reach)
         self._wide = any(ent["cfg"].kind == "attention" and ent["cfg"].dim > 256 for ent in self.layers)
+        self._chunks = all(self._mlstm_fits(l) for l in shape.layers if l.kind == "mlstm")
         self._max_heads = max(l.heads for l in shape.layers)
+
+    def _mlstm_fits(self, l):
+        """Whether an mLSTM layer's columns of the step's projection are what ``B.mlstm_prompt`` takes (16-byte pieces of up to 128 columns)."""
+        n = 2 * l.heads * l.dim + 2 * l.heads * l.vdim + 2 * l.heads + self.W
+        return l.dim <= 128 and l.vdim <= 128 and l.dim % 8 == 0 and l.vdim % 8 == 0 and l.heads % 2 == 0 and \
+            n % (8 if self.dtype == torch.bfloat16 else 4) == 0
 
     # ---- cache and state -------------------------------------------------------------------------------------------------------
     def new_arena(self, slots: int, cap: int) -> SlotArena:
@@ -280,11 +292,12 @@ class FivesunHIP(SlotModel):
         if rebuilt and arena.slots * cap >= 1 << 31:
             raise ValueError("more than 2^31 cached rows in one plane")
         f_rows = others(rebuilt)
-        # segments of the matrix memories' prefill (only when some request brings more than SEGMENT tokens)
+        # segments of the matrix memories' prefill
         seg_a = seg_c = chains = np.zeros((0, 4), np.int32)
         seg_end = np.zeros(0, np.int32)
-        if max(counts) > self.SEGMENT and any(l.kind == "mlstm" for l in self.config.layers):
-            seg = max(self.SEGMENT, -(-max(counts) // self.MAX_SEGMENTS))
+        seg = max(self.SEGMENT, -(-max(counts) // self.MAX_SEGMENTS))
+        chunks = self._chunks and seg <= 256
+        if max(counts) > (self.FEW_TOKENS if chunks else self.SEGMENT) and any(l.kind == "mlstm" for l in self.config.layers):
             sa, ch = [], []
             for b, (s, s0, c) in enumerate(zip(slots, starts, counts)):
                 ch.append((s, s0, len(sa), -(-c // seg)))
@@ -318,7 +331,8 @@ class FivesunHIP(SlotModel):
         offs = blob[o64:o64 + n_off * 8].view(np.int64).reshape(len(self._sigs), T)
         for k, (g, d) in enumerate(self._sigs):
             np.add(st.row_slot * (g * cap * d), st.row_pos * d, out=offs[k])
-        dims = dict(T=T, R=R, n_want=int(want_rows.size), n32=n32, o64=o64, sizes=sizes, tile=tile)
+        dims = dict(T=T, R=R, n_want=int(want_rows.size), n32=n32, o64=o64, sizes=sizes, tile=tile, ones=max(counts) == 1,
+                    seg=min(seg, max(counts)) if chunks else 0)
         res = self._decode_graphed(arena, blob, dims) if graphed else None
         if res is None:
             dblob = torch.from_numpy(blob).to(dev)
@@ -333,7 +347,7 @@ class FivesunHIP(SlotModel):
     def _tables(self, dblob, d):
         i32 = dblob[:d["n32"] * 4].view(torch.int32)
         sizes = d["sizes"]
-        at, out = 0, dict(tile=d["tile"], n_seg=sizes.get("seg_end", 0), n_chains=sizes.get("chains", 0) // 4)
+        at, out = 0, dict(tile=d["tile"], ones=d["ones"], seg=d["seg"], n_seg=sizes.get("seg_end", 0), n_chains=sizes.get("chains", 0) // 4)
         for name, n in sizes.items():
             out[name] = i32[at:at + n]
             at += n
@@ -502,20 +516,27 @@ class FivesunHIP(SlotModel):
         H, D, Dv = l.heads, l.dim, l.vdim
         HD, HV = H * D, H * Dv
         P, N = self._project_in(lw, h, T)
-        o = self._mat("mix_o32", T, HV, torch.float32)
         cols = (P, P[:, HD:], P[:, 2 * HD:], P[:, 2 * HD + HV:], P[:, 2 * HD + HV + H:], N)
         state, ns = arena.states[i][0], tb["n_seg"]
-        if ns:
-            # every segment from nothing (only the states move), the segments chained, then every segment from its start state
-            rec = B.mlstm_state_floats(H, D, Dv)
-            local, start = self._mat("seg_local", ns, rec, torch.float32), self._mat("seg_start", ns, rec, torch.float32)
-            fsum = self._mat("seg_logf", ns, H, torch.float32)
-            B.mlstm(*cols, tb["seg_a"], ns, local, H, D, Dv, D ** -0.5, l.gate_cap, None, from_nothing=True, log_f_sum=fsum)
-            B.mlstm_chain(local, fsum, start, state, tb["chains"], tb["n_chains"], H, D, Dv)
-            B.mlstm(*cols, tb["seg_c"], ns, start, H, D, Dv, D ** -0.5, l.gate_cap, o, end_slots=tb["seg_end"], end_state=state)
+        rec = B.mlstm_state_floats(H, D, Dv)
+        local, start, fsum = (self._mat("seg_local", ns, rec, torch.float32), self._mat("seg_start", ns, rec, torch.float32),
+                              self._mat("seg_logf", ns, H, torch.float32)) if ns else (None, None, None)
+        gate, on = P[:, 2 * HD + HV + 2 * H:], self._mat("mix_gated", T, HV, self.dtype)
+        tail = (H, D, Dv, D ** -0.5, l.gate_cap)
+        if ns and tb["seg"]:
+            B.mlstm_prompt(cols[:5], N, tb["seg_a"], ns, tb["chains"], tb["n_chains"], tb["seg"], tb["seg_end"], state, *tail, lw["gain"], gate, N, on,
+                           self.config.norm_eps, local, fsum, start)
+        elif tb["ones"] and B.mlstm_step_fits(D, Dv, N, cols[2]):
+            B.mlstm_step(cols[:5], N, tb["reqs"], R, state, *tail, lw["gain"], gate, N, on, self.config.norm_eps)
         else:
-            B.mlstm(*cols, tb["reqs"], R, state, H, D, Dv, D ** -0.5, l.gate_cap, o)
-        on = self._mat("mix_gated", T, HV, self.dtype)
-        B.gated_norm(o, lw["gain"], P[:, 2 * HD + HV + 2 * H:], N, on, self.config.norm_eps, T, group=Dv)
+            o = self._mat("mix_o32", T, HV, torch.float32)
+            if ns:
+                # every segment from nothing (only the states move), the segments chained, then every segment from its start state
+                B.mlstm(*cols, tb["seg_a"], ns, local, *tail, None, from_nothing=True, log_f_sum=fsum)
+                B.mlstm_chain(local, fsum, start, state, tb["chains"], tb["n_chains"], H, D, Dv)
+                B.mlstm(*cols, tb["seg_c"], ns, start, *tail, o, end_slots=tb["seg_end"], end_state=state)
+            else:
+                B.mlstm(*cols, tb["reqs"], R, state, *tail, o)
+            B.gated_norm(o, lw["gain"], gate, N, on, self.config.norm_eps, T, group=Dv)
         B.linear(on, lw["wo"], y, M=T)
         return P[:, 2 * HD + 2 * HV + 2 * H:], N

@@ -1,0 +1,108 @@
+"""pcb_mlstm_prompt and pcb_mlstm_step (the matrix memory in segments on the matrix cores, and one token per request; norm and gate included)
+against the float64 recurrence: segments around the 16-row tiles and the 64-, 128- and 256-token forms, requests that resume, junk in the slots of
+those that do not, forget gates that keep everything, that drop everything and that are closed for good."""
+import pytest
+import torch
+
+from oracle import fivesun_oracle as O
+
+pytestmark = pytest.mark.gpu
+DEV, F64 = "cuda:0", torch.float64
+
+
+def rnd(*shape, seed=0, dtype=torch.float32):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(DEV, dtype)
+
+
+def rel(got, want):
+    got, want = got.to("cpu", F64), want.to("cpu", F64)
+    return float((got - want).norm() / want.norm())
+
+
+def i32(x):
+    return torch.tensor(x, dtype=torch.int32, device=DEV)
+
+
+# fp32 rows: the recurrence's own test holds token by token to 2e-5; products and sums here are fp32 as well.  bf16 rows: the inputs are exact either
+# way, the results are rounded to 8 significant bits: 2^-8 of a value at most.
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 2e-5), (torch.bfloat16, 2.0 ** -8)])
+@pytest.mark.parametrize("H,D,Dv,cap,seg,shift", [(2, 128, 128, 10.0, 64, 3.0), (2, 16, 24, 0.0, 64, 3.0), (4, 72, 128, 0.0, 128, -30.0),
+                                                  (2, 128, 40, 4.0, 256, 6.0), (4, 8, 8, 0.0, 64, 0.0)])
+def test_segments_and_steps_against_the_recurrence(H, D, Dv, cap, seg, shift, dtype, tol):
+    from promptcache_amd import _blocks as B
+    eps, rec = 1e-6, B.mlstm_state_floats(H, D, Dv)
+    counts, starts, slots = [2 * seg + 2, 17, 1, seg, 16, seg - 1], [0, 9, 0, 4, 0, 7], [4, 0, 2, 6, 1, 5]
+    n = sum(counts)
+    N = 2 * H * D + 2 * H * Dv + 2 * H
+    N = -(-N // 8) * 8
+    P = rnd(n + 6, N, seed=1, dtype=dtype)                       # (the last six rows: one more token of every request)
+    gf = P[:, 2 * H * D + H * Dv + H:2 * H * D + H * Dv + 2 * H]
+    gf += shift
+    if cap == 0.0:
+        gf[5::11] = float("-inf")                                # nothing of what came before stays
+    g0 = 2 * H * D + H * Dv + 2 * H
+    gain, gate = 1 + 0.1 * rnd(H * Dv, seed=2), P[:, g0:g0 + H * Dv]
+    state = rnd(7, rec, seed=3)
+    state.view(7, H, -1)[..., -1] = 0.7
+    f = lambda t: t.detach().to("cpu", F64)
+    P6, s6 = f(P), f(state).view(7, H, -1)
+
+    def oracle(rows, st):
+        x, k = P6[rows], len(rows)
+        q, kk, v = x[:, :H * D].view(k, H, D) * D ** -0.5, x[:, H * D:2 * H * D].view(k, H, D), x[:, 2 * H * D:2 * H * D + H * Dv].view(k, H, Dv)
+        gi, gl = x[:, 2 * H * D + H * Dv:2 * H * D + H * Dv + H], x[:, 2 * H * D + H * Dv + H:g0]
+        o, st = O.matrix_memory(q, kk, v, O.soft_cap(gi, cap), torch.nn.functional.logsigmoid(O.soft_cap(gl, cap)), st)
+        return O.unit_rms(o, eps).reshape(k, H * Dv) * f(gain) * x[:, g0:g0 + H * Dv], st
+
+    segs, chains, ends, row = [], [], [], 0
+    for c, s0, slot in zip(counts, starts, slots):
+        chains.append((slot, s0, len(segs), -(-c // seg)))
+        for q in range(0, c, seg):
+            segs.append((len(segs), 0, min(seg, c - q), row + q))
+            ends.append(slot if q + seg >= c else -1)
+        row += c
+    ns = len(segs)
+    cols = (P, P[:, H * D:], P[:, 2 * H * D:], P[:, 2 * H * D + H * Dv:], P[:, 2 * H * D + H * Dv + H:])
+    out = torch.zeros(n + 6, H * Dv, device=DEV, dtype=dtype)
+    nan = lambda *s: torch.full(s, float("nan"), device=DEV)
+    tail = (H, D, Dv, D ** -0.5, cap, gain, gate, N, out, eps)
+    assert B.mlstm_prompt_fits(D, Dv, N, cols, gate, seg) and B.mlstm_step_fits(D, Dv, N, cols[2])
+    untouched = state[3].clone()
+    B.mlstm_prompt(cols, N, i32(segs), ns, i32(chains), len(chains), seg, i32(ends), state, *tail, nan(ns, rec), nan(ns, H), nan(ns, rec))
+    want, after, row = [], [], 0
+    for c, s0, slot in zip(counts, starts, slots):
+        st = (s6[slot][:, :D * Dv].reshape(H, D, Dv), s6[slot][:, D * Dv:D * Dv + D], s6[slot][:, -1]) if s0 else None
+        o, st = oracle(list(range(row, row + c)), st)
+        want.append(o), after.append(st)
+        got = state[slot].view(H, -1)
+        assert rel(got[:, :D * Dv].reshape(H, D, Dv), st[0]) < 2e-5 and rel(got[:, D * Dv:-1], st[1]) < 2e-5
+        assert torch.allclose(f(got[:, -1]), st[2], rtol=1e-5, atol=1e-5)
+        row += c
+    assert rel(out[:n], torch.cat(want)) < tol and torch.equal(state[3], untouched)
+    # one more token each
+    B.mlstm_step(cols, N, i32([(s, s0 + c, 1, n + b) for b, (s, s0, c) in enumerate(zip(slots, starts, counts))]), 6, state, *tail)
+    for b, slot in enumerate(slots):
+        o, st = oracle([n + b], after[b])
+        got = state[slot].view(H, -1)
+        assert rel(out[n + b], o[0]) < tol and rel(got[:, :D * Dv].reshape(H, D, Dv), st[0]) < 2e-5 and rel(got[:, D * Dv:-1], st[1]) < 2e-5
+    # a first token: the slot's junk is not read
+    B.mlstm_step(cols, N, i32([(3, 0, 1, n)]), 1, state, *tail)
+    assert rel(out[n], oracle([n], None)[0][0]) < tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("D,Dv", [(200, 100), (60, 252)])
+def test_steps_of_wide_heads(D, Dv, dtype):
+    from promptcache_amd import _blocks as B
+    H, eps = 3, 1e-6
+    N = 2 * H * D + H * Dv + 2 * H + 2
+    P, state = rnd(5, N, seed=1, dtype=dtype), rnd(5, B.mlstm_state_floats(H, D, Dv), seed=2)
+    state.view(5, H, -1)[..., -1] = 0.2
+    cols = (P, P[:, H * D:], P[:, 2 * H * D:], P[:, 2 * H * D + H * Dv:], P[:, 2 * H * D + H * Dv + H:])
+    reqs, ref = i32([(4, 3, 1, 0), (1, 0, 1, 1), (0, 8, 1, 4)]), state.clone()
+    out, raw, want = (torch.zeros(5, H * Dv, device=DEV, dtype=t) for t in (dtype, torch.float32, dtype))
+    B.mlstm(*cols, N, reqs, 3, ref, H, D, Dv, D ** -0.5, 5.0, raw)
+    B.gated_norm(raw, None, None, 0, want, eps, 5, group=Dv)
+    assert B.mlstm_step_fits(D, Dv, N, cols[2])
+    B.mlstm_step(cols, N, reqs, 3, state, H, D, Dv, D ** -0.5, 5.0, None, None, 0, out, eps)
+    assert rel(state, ref) < 1e-6 and rel(out, want) < (1e-5 if dtype == torch.float32 else 2.0 ** -8)
