@@ -193,6 +193,15 @@ typedef struct pcb_attn_talk_args {
 int32_t pcb_attn_talk_band(int32_t window, int32_t max_kv_len);
 int pcb_attn_talk(const pcb_attn_talk_args* a, void* stream);
 
+/* The same for tiles of one row each (decoding) in one launch; scratch, tiles64 and max_tile_rows are not used.  part: fp32
+ * [pcb_attn_talk_rows_part(n_tiles, H, head_dim)], aligned to 8 bytes; counters: int32 [n_tiles], zero before the first launch that is given them and
+ * left zero by every launch; launches that may run at the same time need a part and counters of their own.  pcb_attn_talk_rows_fits: which sizes it
+ * takes (1, 2, 4 or 8 heads to a key head, head_dim <= 128 and a multiple of 8, head_dim / 8 * Hkv <= 256); q, cache and their strides are multiples of
+ * 16 bytes. */
+int32_t pcb_attn_talk_rows_fits(int32_t dtype, int32_t H, int32_t Hkv, int32_t head_dim);
+int64_t pcb_attn_talk_rows_part(int32_t n_rows, int32_t H, int32_t head_dim);
+int pcb_attn_talk_rows(const pcb_attn_talk_args* a, float* part, int64_t part_floats, int32_t* counters, void* stream);
+
 /* ---- residual streams, norms, routers of designs with several residual streams --------------------------------------------- */
 
 /* out[s][r][:] = fp32(table[ids[r]]) + fp32(pos_table[positions[r]]) for every stream s < n_streams (pos_table null: no

@@ -8,8 +8,9 @@
 //      [row][head][key, from band_key0 of the row on] -- no softmax state, hence no coupling between key tiles: the grid runs over key blocks too.
 //   2. talk_values_kernel: per (up to 64 queries, head): one sweep over the band with a running maximum and denominator per row
 //      (the sink enters as a score of 0), P V on the matrix cores with the keys as values; bf16 runs P as a hi + lo pair so the
-//      fp32 weights are not rounded.  Tiles of at most 4 rows (decoding) take talk_values_few_kernel: fp32 multiply-adds over
+//      fp32 weights are not rounded.  Tiles of at most 4 rows take talk_values_few_kernel: fp32 multiply-adds over
 //      coalesced key rows, no matrix cores.
+// Single rows (decoding) of the usual sizes go through one launch without a band instead: pb_attn_talk_rows.hip.
 #include <type_traits>
 
 #include "pb_common.h"

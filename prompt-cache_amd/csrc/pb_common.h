@@ -171,6 +171,30 @@ __device__ __forceinline__ void store4(bf16_t* p, float a, float b, float c, flo
 }
 __device__ __forceinline__ void store4(float* p, float a, float b, float c, float d) { *reinterpret_cast<float4*>(p) = float4{a, b, c, d}; }
 
+// eight neighbouring elements (16-byte aligned) as a lane's part of a k-step in which lane group g holds the elements 8 g .. 8 g + 7.  (For bf16 that
+// is lane_k; two fp32 operands that both use it are as good.)  at8: element e as a float.
+__device__ __forceinline__ Frag<bf16_t> load8(const bf16_t* p) {
+    Frag<bf16_t> f;
+    f.v = *reinterpret_cast<const u32x4*>(p);
+    return f;
+}
+__device__ __forceinline__ Frag<float> load8(const float* p) {
+    Frag<float> f;
+    const f4 a = *reinterpret_cast<const f4*>(p), b = *reinterpret_cast<const f4*>(p + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f.v[e] = a[e], f.v[4 + e] = b[e];
+    return f;
+}
+__device__ __forceinline__ float at8(const Frag<bf16_t>& f, int e) {
+    return __uint_as_float(e & 1 ? f.v[e >> 1] & 0xffff0000u : f.v[e >> 1] << 16);
+}
+__device__ __forceinline__ float at8(const Frag<float>& f, int e) { return f.v[e]; }
+__device__ __forceinline__ void zero8(Frag<bf16_t>& f) { f.v = u32x4{0u, 0u, 0u, 0u}; }
+__device__ __forceinline__ void zero8(Frag<float>& f) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f.v[e] = 0.0f;
+}
+
 // result tile: lane l holds column (l & 15), rows 4 * (l >> 4) + r, r = 0..3
 
 }  // namespace pcb

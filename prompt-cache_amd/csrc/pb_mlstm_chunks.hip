@@ -29,28 +29,6 @@ __device__ __forceinline__ float soft_cap(float z, float cap) { return cap > 0.0
 __device__ __forceinline__ float log_sigmoid(float z) { return fminf(z, 0.0f) - log1pf(expf(-fabsf(z))); }
 __device__ __forceinline__ f4 mma4(float a, float b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
-// eight neighbouring elements (16-byte aligned; states, which lie at any float: load8u)
-__device__ __forceinline__ Frag<bf16_t> load8(const bf16_t* p) {
-    Frag<bf16_t> f;
-    f.v = *reinterpret_cast<const u32x4*>(p);
-    return f;
-}
-__device__ __forceinline__ Frag<float> load8(const float* p) {
-    Frag<float> f;
-    const f4 a = *reinterpret_cast<const f4*>(p), b = *reinterpret_cast<const f4*>(p + 4);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) f.v[e] = a[e], f.v[4 + e] = b[e];
-    return f;
-}
-__device__ __forceinline__ float at8(const Frag<bf16_t>& f, int e) {
-    return __uint_as_float(e & 1 ? f.v[e >> 1] & 0xffff0000u : f.v[e >> 1] << 16);
-}
-__device__ __forceinline__ float at8(const Frag<float>& f, int e) { return f.v[e]; }
-__device__ __forceinline__ void zero8(Frag<bf16_t>& f) { f.v = u32x4{0u, 0u, 0u, 0u}; }
-__device__ __forceinline__ void zero8(Frag<float>& f) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) f.v[e] = 0.0f;
-}
 __device__ __forceinline__ void load2(const bf16_t* p, float (&o)[2]) {
     const uint32_t w = *reinterpret_cast<const uint32_t*>(p);
     o[0] = __uint_as_float(w << 16), o[1] = __uint_as_float(w & 0xffff0000u);

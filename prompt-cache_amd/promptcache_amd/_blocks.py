@@ -198,6 +198,9 @@ SIGNATURES = {
     "pcb_moe_combine": (C.c_int, [_vp, _vp, _vp, _i32, _i32, _i32, _vp]),
     "pcb_attn_talk_band": (C.c_int32, [_i32, _i32]),
     "pcb_attn_talk": (C.c_int, [C.POINTER(AttnTalkArgs), _vp]),
+    "pcb_attn_talk_rows_fits": (C.c_int32, [_i32, _i32, _i32, _i32]),
+    "pcb_attn_talk_rows_part": (_i64, [_i32, _i32, _i32]),
+    "pcb_attn_talk_rows": (C.c_int, [C.POINTER(AttnTalkArgs), _vp, _i64, _vp, _vp]),
     "pcb_embed_pos_rows": (C.c_int, [_vp, _vp, _i32, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _i32, _vp]),
     "pcb_hyper_norm": (C.c_int, [C.POINTER(HyperNormArgs), _vp]),
     "pcb_gated_norm": (C.c_int, [_vp, _i64, _vp, _vp, _i64, _vp, _i64, _i32, _f32, _i32, _i32, _i32, _i32, _vp, _i64, _vp, _i32, _vp]),
@@ -455,6 +458,32 @@ def attn_talk(q: torch.Tensor, tiles: torch.Tensor, n_tiles: int, cache: torch.T
         _want(tiles64, torch.int32, "attn_talk tiles64")
         assert tiles64.numel() >= 4 * n_tiles64 > 0
     check(load().pcb_attn_talk(C.byref(a), _stream()), "pcb_attn_talk")
+
+
+def attn_talk_rows_fits(dtype: torch.dtype, H: int, Hkv: int, head_dim: int) -> bool:
+    """Whether ``attn_talk_rows`` takes these sizes."""
+    return bool(load().pcb_attn_talk_rows_fits(DTYPES[dtype], H, Hkv, head_dim))
+
+
+def attn_talk_rows_part(n_rows: int, H: int, head_dim: int) -> int:
+    return int(load().pcb_attn_talk_rows_part(n_rows, H, head_dim))
+
+
+def attn_talk_rows(q: torch.Tensor, tiles: torch.Tensor, n_tiles: int, cache: torch.Tensor, slot_stride: int, head_stride: int,
+                   H: int, Hkv: int, head_dim: int, scale: float, window: int, max_kv_len: int, slopes, talk, sink: bool,
+                   part: torch.Tensor, counters: torch.Tensor, out: torch.Tensor) -> None:
+    """``attn_talk`` for tiles of one row each; ``part`` fp32 [attn_talk_rows_part], ``counters`` int32 [n_tiles], zero and left zero."""
+    _want(tiles, torch.int32, "attn_talk_rows tiles"); _want(part, torch.float32, "attn_talk_rows part")
+    _want(counters, torch.int32, "attn_talk_rows counters"); _want(slopes, torch.float32, "attn_talk_rows slopes")
+    _want(talk, torch.float32, "attn_talk_rows talk")
+    assert q.dtype == cache.dtype == out.dtype and q.is_contiguous() and out.is_contiguous() and cache.is_cuda
+    assert tiles.numel() >= 4 * n_tiles and q.shape[-1] == H * head_dim and out.shape[-1] == H * head_dim and counters.numel() >= n_tiles
+    assert slopes is None or slopes.numel() == H
+    assert talk is None or talk.numel() == H * H
+    a = AttnTalkArgs(C.sizeof(AttnTalkArgs), _code(q), _p(q), q.shape[-1], _p(tiles), n_tiles, _p(cache), slot_stride,
+                     head_stride, H, Hkv, head_dim, float(scale), int(window), int(max_kv_len), _p(slopes), _p(talk), int(sink),
+                     None, 0, _p(out), out.shape[-1], None, 0, 1)
+    check(load().pcb_attn_talk_rows(C.byref(a), _p(part), part.numel(), _p(counters), _stream()), "pcb_attn_talk_rows")
 
 
 # ---- blocks of designs with several residual streams, gated / recurrent mixers and group-limited routers ----------------------

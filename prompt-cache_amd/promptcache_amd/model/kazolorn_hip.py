@@ -71,7 +71,7 @@ class KazolornHIP(SlotModel):
                        wqk=torch.cat([e(p + "mix.q"), e(p + "mix.k")], dim=0).contiguous(),
                        bqk=torch.cat([e(p + "mix.q.b"), e(p + "mix.k.b")], dim=0).contiguous(),
                        talk=f(p + "mix.talk"), wo=e(p + "mix.o"), bo=e(p + "mix.o.b"),
-                       slopes=distance_slopes(l.heads).to(dev))
+                       slopes=distance_slopes(l.heads).to(dev), rows=B.attn_talk_rows_fits(dtype, l.heads, l.kv_heads, l.dim))
             if ent["dwa"].numel() < i + 2:
                 raise ValueError(f"{p}dwa has {ent['dwa'].numel()} weights, layer {i} sums {i + 2} streams")
             ent["dwa"] = ent["dwa"].reshape(-1)[:i + 2].contiguous()
@@ -252,7 +252,7 @@ class KazolornHIP(SlotModel):
         from pinned memory refreshes; every launch dimension is sized for the arena's row capacity instead of the current
         lengths.  Returns None when the score band of such a launch would be too large (the caller then runs eagerly)."""
         cap = arena.cap
-        worst = max(16 * T * l.heads * B.attn_talk_band(l.window, cap) for l in self.config.layers)
+        worst = max((16 * T * lw["cfg"].heads * B.attn_talk_band(lw["cfg"].window, cap) for lw in self.layers if not lw["rows"]), default=0)
         if worst > ATTN_SCRATCH_FLOATS // 4:
             return None
         key = (T, arena.serial, arena.generation)
@@ -288,6 +288,11 @@ class KazolornHIP(SlotModel):
         return ent["logits"].clone()
 
     def _attention(self, q, att, tiles, n_tiles, tiles_d, tiles64_d, n64, plane, arena, i, l, lw, max_kv, max_rows=0):
+        if max_rows == 1 and lw["rows"]:
+            part = self._scratch("talk_part", B.attn_talk_rows_part(n_tiles, l.heads, l.dim), torch.float32)
+            B.attn_talk_rows(q, tiles_d, n_tiles, plane, arena.slot_stride(i), arena.head_stride(i), l.heads, l.kv_heads, l.dim, l.scale,
+                             l.window, max_kv, lw["slopes"], lw["talk"], True, part, self._counters("talk_counters", n_tiles), att)
+            return
         band = B.attn_talk_band(l.window, max_kv)
         per_tile = 16 * l.heads * band
         chunk = max(1, ATTN_SCRATCH_FLOATS // per_tile)

@@ -77,6 +77,14 @@ class SlotModel:
         rows = max(rows, 1)
         return self._scratch(name, rows * cols, dtype).as_strided((rows, cols), (cols, 1))
 
+    def _counters(self, name: str, n: int) -> torch.Tensor:
+        """At least ``n`` int32 counters that launches find at zero and leave at zero.  They are made by an eager run (a capture only ever
+        follows one with the same scratch), never inside a capture, whose replays would be the only ones to clear them."""
+        t = self._buf.get(name)
+        if t is None or t.numel() < n:
+            t = self._buf[name] = torch.zeros(max(n, 64), dtype=torch.int32, device=self.device)
+        return t
+
     # ---- one-token steps as captured graphs (models whose step is ``_run(arena, device tables, dims, logits)``) ------------------
     def _decode_graphed(self, arena, blob, d):
         """A step of T requests with one token each, replayed from a hipGraph captured per (T, arena planes).  What changes
