@@ -364,6 +364,84 @@ __global__ __launch_bounds__(64 * SKW) void linear_skinny_kernel(pcb_linear_args
     }
 }
 
+// Few rows of a plain or batched launch whose rows can be read in 16-byte pieces, whole k-steps; R = 16 / PARTS rows at most.  PARTS runs of k lie side
+// by side in one product: the operands' row (and column) i stands for row i % R of run i / R, so the R x R blocks on the result's diagonal hold the
+// runs' sums of R columns each, and what lies beside them is thrown away.  A workgroup then has R columns instead of 16: twice or four times the
+// workgroups where 16 columns each would leave CUs idle, and as many more loads under way per column.  Eight waves split k; a wave requests U k-steps
+// at a time (a loop of single steps waits for each).  LATE: as above.
+// us, the kernel above / this, 1 row bf16: 1024 x 1024 3.9 / 2.9, 1024 x 4096 8.0 / 4.3, 32000 x 2048 31.4 / 24.0 (5.5 TB/s); 8 rows bf16: 2048 x 2048
+// 6.3 / 4.9, 2048 x 4096 9.2 / 6.8, gated 4096 x 2048 11.4 / 9.5, 5136 x 2048 10.1 / 8.6; fp32: 1 row 1024 x 4096 13.5 / 6.5, 32000 x 2048 58.9 / 43.8,
+// 8 rows 2048 x 2048 10.4 / 7.2, 32000 x 2048 70.4 / 57.1, 16 rows 10272 x 2048 33.2 / 26.4.
+template <typename E, int EPI, int PARTS, int U, bool LATE>
+__global__ __launch_bounds__(512) void linear_parts_kernel(pcb_linear_args a) {
+    constexpr bool TWO = EPI == PCB_EPI_SILU_MUL, ADD = EPI == PCB_EPI_SCALE_ADD;
+    constexpr int R = 16 / PARTS, SKW = 8;
+    __shared__ f4 red[TWO ? 2 : 1][SKW][64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, group = lane >> 4, l15 = lane & 15;
+    const int K = a.K, N = a.N, n_lo = blockIdx.x * R, g = a.n_batch > 0 ? blockIdx.z : 0;
+    const int run = l15 / R, i = l15 % R;
+    const int n_b = n_lo + i < N ? n_lo + i : N - 1, m_a = i < a.M ? i : a.M - 1;
+    const E* X = (const E*)a.x + g * a.x_batch_stride;
+    const int64_t w_at = g * a.w_group_stride + n_b * a.ldw + 32 * run + 8 * group;
+    const E* wrow = (const E*)a.w + w_at;
+    const E* wrow2 = TWO ? (const E*)a.w2 + w_at : nullptr;
+    const E* xrow = X + (int64_t)(a.row_src ? a.row_src[m_a] : m_a) * a.ldx + 32 * run + 8 * group;
+    // (the lanes that store: rows m0 .. m0 + 3 of column n_b, run 0)
+    const int m0 = 4 * group;
+    float bv = 0.0f, bv2 = 0.0f, cs = 0.0f;
+    Place to[4] = {};
+    const bool stores = wave == 0 && m0 < R && run == 0;
+    auto places = [&] {
+        if (a.bias) bv = to_f32(((const E*)a.bias)[n_b]);
+        if (TWO && a.bias2) bv2 = to_f32(((const E*)a.bias2)[n_b]);
+        if (ADD) cs = a.col_scale[n_b];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (TWO || m0 + r < a.M) to[r] = place<E, EPI>(a, m0 + r < a.M ? m0 + r : a.M - 1, n_b);
+    };
+    if (!LATE && stores) places();
+    Sum<E> sum, sum2;
+    const int steps = K / (32 * PARTS);
+    for (int s0 = wave; s0 < steps; s0 += U * SKW) {
+        Frag<E> fa[U], fb[U], fc[TWO ? U : 1];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (s0 + u * SKW < steps) {                                // (uniform over the wave)
+                const int k = 32 * PARTS * (s0 + u * SKW);
+                fb[u] = load8(wrow + k);
+                if (TWO) fc[u] = load8(wrow2 + k);
+                fa[u] = load8(xrow + k);
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (s0 + u * SKW < steps) {
+                sum.add(fa[u], fb[u]);
+                if (TWO) sum2.add(fa[u], fc[u]);
+            }
+    }
+    if (LATE && stores) places();
+    red[0][wave][lane] = sum.total();
+    if (TWO) red[1][wave][lane] = sum2.total();
+    __syncthreads();
+    if (wave != 0) return;
+    f4 acc[2];
+#pragma unroll
+    for (int t = 0; t < (TWO ? 2 : 1); ++t) {
+        acc[t] = red[t][0][lane];
+#pragma unroll
+        for (int w = 1; w < SKW; ++w) acc[t] += red[t][w][lane];
+        // run p of column i: lane R i.. of the rows p R ..: (16 R / 4 + R) lanes further per run
+#pragma unroll
+        for (int o = PARTS / 2; o > 0; o >>= 1)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[t][r] += __shfl(acc[t][r], (lane + o * (4 * R + R)) & 63, 64);
+    }
+    if (!stores || n_lo + i >= N) return;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        if (m0 + r < a.M) put<E, EPI>(to[r], finished<E, EPI>(a, to[r], n_b, acc[0][r], TWO ? acc[1][r] : 0.0f, bv, bv2), cs);
+}
+
 // ---- many rows: both panels travel to LDS by themselves ------------------------------------------------------------------------------
 // The same tiles (2 x 2 waves of TM x TN result tiles) for operands whose rows can be read in 16-byte chunks: global_load_lds carries a
 // stage of 128 bytes of k (64 elements of bf16, 32 of fp32; 1 KiB per wave instruction: 8 rows) straight into a ring of two or three images, one
@@ -684,6 +762,56 @@ int dispatch(const pcb_linear_args& a, hipStream_t stream) {
         // 32000 15.6 / 13.9 and 18.8 / 17.6; K = 2048, 13600 columns 17.5 / 13.9 and 22.0 / 18.2; gated, 8 rows, 16384 columns 13.2 / 13.9;
         // K = 2048, 1 row, 13600 columns 27.4 / 26.4.
         const bool late = sizeof(E) == 2 && groups > (a.epilogue == PCB_EPI_SILU_MUL && a.K < 2048 ? 1024 : 768);
+        // Runs side by side: four where up to four rows leave no more than three workgroups a CU so, else two, and for more than four rows not where 16
+        // columns each are one round of the chip and eight are two (us, 8 rows, K = 2048, one run / two: 3072 columns bf16 6.3 / 6.7, fp32 9.5 / 10.8;
+        // 5136 9.8 / 8.6 and 16.5 / 14.5) or beyond 1024 workgroups (fp32: 768; 7424 columns 10.7 / 10.4 and 18.1 / 18.7, 32000 34.1 / 35.1 and
+        // 57.1 / 64.4).  A run has eight k-steps at least.  bf16 of more than eight rows over a deep k of few columns stays with sixteen waves above
+        // (16 rows, 2048 x 4096: 10.8, here 11.2).
+        const int es = sizeof(E), batch = a.n_batch > 0 ? a.n_batch : 1;
+        const bool pieces = a.n_groups == 0 && !a.row_scale && a.K % 32 == 0 && a.ldx * es % 16 == 0 && a.ldw * es % 16 == 0 &&
+                            a.x_batch_stride * es % 16 == 0 && a.w_group_stride * es % 16 == 0 &&
+                            ((uintptr_t)a.x | (uintptr_t)a.w | (uintptr_t)(a.epilogue == PCB_EPI_SILU_MUL ? a.w2 : nullptr)) % 16 == 0;
+        if (pieces && !(es == 2 && a.M > 8 && deep)) {
+            const int64_t four = (int64_t)batch * pcb_ceil_div(a.N, 4), two = (int64_t)batch * pcb_ceil_div(a.N, 8);
+            int parts = 1;
+            if (a.M <= 4 && four <= 768 && a.K % 128 == 0 && a.K >= 1024)
+                parts = 4;
+            else if (a.M <= 8 && a.K % 64 == 0 && a.K >= 512 && (a.M <= 4 || two <= 256 || (two > 400 && two <= (es == 2 ? 1024 : 768))))
+                parts = 2;
+            auto go = [&](auto epi, auto p, auto u, auto late) {
+                hipLaunchKernelGGL((linear_parts_kernel<E, decltype(epi)::value, decltype(p)::value, decltype(u)::value, decltype(late)::value>),
+                                   dim3(pcb_ceil_div(a.N, 16 / decltype(p)::value), 1, batch), dim3(512), 0, stream, a);
+            };
+            using One = std::integral_constant<int, 1>;
+            using Two = std::integral_constant<int, 2>;
+            using Four = std::integral_constant<int, 4>;
+            using Steps = std::integral_constant<int, sizeof(E) == 2 ? 4 : 2>;             // (fp32: more in flight costs workgroups)
+            using Deep = std::integral_constant<int, sizeof(E) == 2 ? 8 : 2>;
+            auto kind = [&](auto epi, auto late) {
+                if (parts == 4)
+                    go(epi, Four{}, Steps{}, late);
+                else if (parts == 2)
+                    go(epi, Two{}, Steps{}, late);
+                else if (a.K >= 2048)
+                    go(epi, One{}, Deep{}, late);
+                else
+                    go(epi, One{}, Steps{}, late);
+            };
+            // (where results go, worked out behind the products: -0.1 to -0.3 us from K = 1024 on, +0.2 below; gated units only where 16 columns each
+            // fill the chip, 16 rows x 4096, K = 2048 11.1 against 12.5; what a scaled accumulation adds to is asked for ahead of them)
+            if (a.epilogue == PCB_EPI_SILU_MUL && parts == 1)
+                go(std::integral_constant<int, PCB_EPI_SILU_MUL>{}, One{}, Steps{}, std::true_type{});
+            else if (a.epilogue == PCB_EPI_SILU_MUL)
+                parts == 4 ? go(std::integral_constant<int, PCB_EPI_SILU_MUL>{}, Four{}, Steps{}, std::false_type{})
+                           : go(std::integral_constant<int, PCB_EPI_SILU_MUL>{}, Two{}, Steps{}, std::false_type{});
+            else if (a.epilogue == PCB_EPI_SCALE_ADD)
+                kind(std::integral_constant<int, PCB_EPI_SCALE_ADD>{}, std::false_type{});
+            else if (a.K >= 1024)
+                kind(std::integral_constant<int, PCB_EPI_STORE>{}, std::true_type{});
+            else
+                kind(std::integral_constant<int, PCB_EPI_STORE>{}, std::false_type{});
+            return pcb_check_launch("linear_parts_kernel");
+        }
         auto go = [&](auto epi) {
             constexpr int EPI = decltype(epi)::value;
             if (deep)
