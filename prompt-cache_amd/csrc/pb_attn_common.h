@@ -2,8 +2,22 @@
 #pragma once
 #include "pb_common.h"
 
+// bf16 prompts of the usual head counts in one pass without a band (pb_attn_talk_prompt.hip): which calls it takes, and the launch
+bool pcb_talk_prompt_fits(const pcb_attn_talk_args& a);
+int pcb_talk_prompt(const pcb_attn_talk_args& a, hipStream_t stream);
+
 #ifdef __HIPCC__
 namespace pcb {
+
+// e^x of a score less its row's maximum (x <= 0, -infinity for a key the row does not see): 2^(x log2 e) on the hardware's exp2, the product's
+// rounding put back (log2 e in two parts), so that the error does not grow with |x|.  Seven instructions; below e^-87 it is 0.  NaN stays NaN
+// (v_maximum3_f32; fmaxf would return the bound for it).
+__device__ __forceinline__ float exp_le0(float x) {
+    x = __builtin_elementwise_maximum(x, -200.0f);
+    const float p = x * 1.44269502e+00f, lo = __builtin_fmaf(x, 1.92596303e-08f, __builtin_fmaf(x, 1.44269502e+00f, -p));
+    const float e = __builtin_amdgcn_exp2f(p);
+    return __builtin_fmaf(e, lo * 6.93147182e-01f, e);
+}
 
 // eight softmax weights of a lane.  bf16: a hi + lo pair of bf16 values (two MFMAs), so that they are not rounded to 8 bits; fp32: as
 // they are

@@ -10,10 +10,11 @@
 //      (the sink enters as a score of 0), P V on the matrix cores with the keys as values; bf16 runs P as a hi + lo pair so the
 //      fp32 weights are not rounded.  Tiles of at most 4 rows take talk_values_few_kernel: fp32 multiply-adds over
 //      coalesced key rows, no matrix cores.
-// Single rows (decoding) of the usual sizes go through one launch without a band instead: pb_attn_talk_rows.hip.
+// Single rows (decoding) of the usual sizes go through one launch without a band instead: pb_attn_talk_rows.hip; so do bf16 prompts with heads of 128
+// columns, four to a key head: pb_attn_talk_prompt.hip.
 #include <type_traits>
 
-#include "pb_common.h"
+#include "pb_attn_common.h"
 
 namespace {
 using namespace pcb;
@@ -25,16 +26,6 @@ struct TileRec {
 // The key that position 0 of row i's band stands for: the row's first visible key, down to a multiple of 16, so that sixteen keys of a tile are a
 // whole 64-byte piece of the band and four are a 16-byte read.
 __device__ __forceinline__ int band_key0(int i, int window) { return i - window + 1 > 0 ? (i - window + 1) & ~15 : 0; }
-
-// e^x of a score less its row's maximum (x <= 0, -infinity for a key the row does not see): 2^(x log2 e) on the hardware's exp2, the product's
-// rounding put back (log2 e in two parts), so that the error does not grow with |x|.  Seven instructions; below e^-87 it is 0.  NaN stays NaN
-// (v_maximum3_f32; fmaxf would return the bound for it).
-__device__ __forceinline__ float exp_le0(float x) {
-    x = __builtin_elementwise_maximum(x, -200.0f);
-    const float p = x * 1.44269502e+00f, lo = __builtin_fmaf(x, 1.92596303e-08f, __builtin_fmaf(x, 1.44269502e+00f, -p));
-    const float e = __builtin_amdgcn_exp2f(p);
-    return __builtin_fmaf(e, lo * 6.93147182e-01f, e);
-}
 
 // ---- 1. scores ---------------------------------------------------------------------------------------------------------------
 // Workgroup = one 16-query tile x KC keys (128, or 64 when the launch has few tiles: decoding); a wave owns 16-key subtiles of
@@ -584,5 +575,7 @@ PCB_EXPORT int pcb_attn_talk(const pcb_attn_talk_args* a, void* stream) {
     PCB_REQUIRE(a->scratch_floats >= (int64_t)a->n_tiles * 16 * a->H * band, PCB_ERR_ARG,
                 "pcb_attn_talk: scratch holds %lld floats, %lld needed", (long long)a->scratch_floats,
                 (long long)a->n_tiles * 16 * a->H * band);
+    // (every size measured is faster there: 100 rows 30 -> 18 us, 2048 rows 111 -> 72; tiles of at most four rows have a values kernel of their own)
+    if ((a->max_tile_rows <= 0 || a->max_tile_rows > FEW_ROWS) && pcb_talk_prompt_fits(*a)) return pcb_talk_prompt(*a, (hipStream_t)stream);
     return a->dtype == PCB_BF16 ? run<pcb::bf16_t>(*a, band, (hipStream_t)stream) : run<float>(*a, band, (hipStream_t)stream);
 }
