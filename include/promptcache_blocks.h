@@ -136,6 +136,13 @@ typedef struct pcb_linear_args {
     int32_t y2_f32;
 } pcb_linear_args;
 int pcb_linear(const pcb_linear_args* a, void* stream);
+/* pcb_linear(a), pcb_linear(b) for two products of the same rows' count that do not need one another: one launch where both are of few rows (a a plain
+ * store, b that or gated), else those two. */
+int pcb_linear_pair(const pcb_linear_args* a, const pcb_linear_args* b, void* stream);
+/* Two scaled accumulations into the same rows (same M, N, y, ldy; b without a base of its own): pcb_linear(a), then pcb_linear(b), in one launch where
+ * there are few rows.  z (fp32 [M][b->K], may be null): b's input is pcb_polynorm(z, coef, eps); b->x is then scratch of that shape, which may or may not
+ * be written. */
+int pcb_linear_add2(const pcb_linear_args* a, const pcb_linear_args* b, const float* z, const float* coef, float eps, void* stream);
 
 /* out[r][f] = c0 * z/rms(z) + c1 * z^2/rms(z^2) + c2 * z^3/rms(z^3) + c3 over row r of z (fp32 [n_rows][ff]), rms with eps inside the
  * root; coef = {c0, c1, c2, c3} fp32 on the device; out is E. */

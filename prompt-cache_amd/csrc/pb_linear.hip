@@ -9,7 +9,7 @@
 // and scaled rows this one.
 #include <type_traits>
 
-#include "pb_linear_epi.h"
+#include "pb_linear_parts.h"
 #include "pb_linear_tiles.h"
 
 namespace {
@@ -63,28 +63,6 @@ __device__ __forceinline__ Frag<float> whole_frag(const float* p, int group) {
     for (int e = 0; e < 4; ++e) f.v[e] = lo[e], f.v[4 + e] = hi[e];
     return f;
 }
-
-// A k-step's products into a pair of sums, odd parts into the second (fp32: shorter chains of roundings -- against 64 bits 0.7 of one chain's
-// error at every size -- and of dependent MFMAs; bf16 has one part); chain: into one, in order of k
-template <typename E>
-struct Sum;
-template <>
-struct Sum<bf16_t> {
-    f4 c = {0.f, 0.f, 0.f, 0.f};
-    __device__ __forceinline__ void add(const Frag<bf16_t>& a, const Frag<bf16_t>& b) { c = mma(a, b, c); }
-    __device__ __forceinline__ void chain(const Frag<bf16_t>& a, const Frag<bf16_t>& b) { add(a, b); }
-    __device__ __forceinline__ f4 total() const { return c; }
-};
-template <>
-struct Sum<float> {
-    f4 c[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
-    __device__ __forceinline__ void add(const Frag<float>& a, const Frag<float>& b) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) c[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[e], b.v[e], c[e & 1], 0, 0, 0);
-    }
-    __device__ __forceinline__ void chain(const Frag<float>& a, const Frag<float>& b) { c[0] = mma(a, b, c[0]); }
-    __device__ __forceinline__ f4 total() const { return c[0] + c[1]; }
-};
 
 template <typename E, int EPI, int TM, int TN>
 __global__ __launch_bounds__(256) void linear_kernel(pcb_linear_args a) {
@@ -364,82 +342,14 @@ __global__ __launch_bounds__(64 * SKW) void linear_skinny_kernel(pcb_linear_args
     }
 }
 
-// Few rows of a plain or batched launch whose rows can be read in 16-byte pieces, whole k-steps; R = 16 / PARTS rows at most.  PARTS runs of k lie side
-// by side in one product: the operands' row (and column) i stands for row i % R of run i / R, so the R x R blocks on the result's diagonal hold the
-// runs' sums of R columns each, and what lies beside them is thrown away.  A workgroup then has R columns instead of 16: twice or four times the
-// workgroups where 16 columns each would leave CUs idle, and as many more loads under way per column.  Eight waves split k; a wave requests U k-steps
-// at a time (a loop of single steps waits for each).  LATE: as above.
+// The few-row products of pb_linear_parts.h, a launch of their own.  LATE: as above.
 // us, the kernel above / this, 1 row bf16: 1024 x 1024 3.9 / 2.9, 1024 x 4096 8.0 / 4.3, 32000 x 2048 31.4 / 24.0 (5.5 TB/s); 8 rows bf16: 2048 x 2048
 // 6.3 / 4.9, 2048 x 4096 9.2 / 6.8, gated 4096 x 2048 11.4 / 9.5, 5136 x 2048 10.1 / 8.6; fp32: 1 row 1024 x 4096 13.5 / 6.5, 32000 x 2048 58.9 / 43.8,
 // 8 rows 2048 x 2048 10.4 / 7.2, 32000 x 2048 70.4 / 57.1, 16 rows 10272 x 2048 33.2 / 26.4.
 template <typename E, int EPI, int PARTS, int U, bool LATE>
 __global__ __launch_bounds__(512) void linear_parts_kernel(pcb_linear_args a) {
-    constexpr bool TWO = EPI == PCB_EPI_SILU_MUL, ADD = EPI == PCB_EPI_SCALE_ADD;
-    constexpr int R = 16 / PARTS, SKW = 8;
-    __shared__ f4 red[TWO ? 2 : 1][SKW][64];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, group = lane >> 4, l15 = lane & 15;
-    const int K = a.K, N = a.N, n_lo = blockIdx.x * R, g = a.n_batch > 0 ? blockIdx.z : 0;
-    const int run = l15 / R, i = l15 % R;
-    const int n_b = n_lo + i < N ? n_lo + i : N - 1, m_a = i < a.M ? i : a.M - 1;
-    const E* X = (const E*)a.x + g * a.x_batch_stride;
-    const int64_t w_at = g * a.w_group_stride + n_b * a.ldw + 32 * run + 8 * group;
-    const E* wrow = (const E*)a.w + w_at;
-    const E* wrow2 = TWO ? (const E*)a.w2 + w_at : nullptr;
-    const E* xrow = X + (int64_t)(a.row_src ? a.row_src[m_a] : m_a) * a.ldx + 32 * run + 8 * group;
-    // (the lanes that store: rows m0 .. m0 + 3 of column n_b, run 0)
-    const int m0 = 4 * group;
-    float bv = 0.0f, bv2 = 0.0f, cs = 0.0f;
-    Place to[4] = {};
-    const bool stores = wave == 0 && m0 < R && run == 0;
-    auto places = [&] {
-        if (a.bias) bv = to_f32(((const E*)a.bias)[n_b]);
-        if (TWO && a.bias2) bv2 = to_f32(((const E*)a.bias2)[n_b]);
-        if (ADD) cs = a.col_scale[n_b];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            if (TWO || m0 + r < a.M) to[r] = place<E, EPI>(a, m0 + r < a.M ? m0 + r : a.M - 1, n_b);
-    };
-    if (!LATE && stores) places();
-    Sum<E> sum, sum2;
-    const int steps = K / (32 * PARTS);
-    for (int s0 = wave; s0 < steps; s0 += U * SKW) {
-        Frag<E> fa[U], fb[U], fc[TWO ? U : 1];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (s0 + u * SKW < steps) {                                // (uniform over the wave)
-                const int k = 32 * PARTS * (s0 + u * SKW);
-                fb[u] = load8(wrow + k);
-                if (TWO) fc[u] = load8(wrow2 + k);
-                fa[u] = load8(xrow + k);
-            }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (s0 + u * SKW < steps) {
-                sum.add(fa[u], fb[u]);
-                if (TWO) sum2.add(fa[u], fc[u]);
-            }
-    }
-    if (LATE && stores) places();
-    red[0][wave][lane] = sum.total();
-    if (TWO) red[1][wave][lane] = sum2.total();
-    __syncthreads();
-    if (wave != 0) return;
-    f4 acc[2];
-#pragma unroll
-    for (int t = 0; t < (TWO ? 2 : 1); ++t) {
-        acc[t] = red[t][0][lane];
-#pragma unroll
-        for (int w = 1; w < SKW; ++w) acc[t] += red[t][w][lane];
-        // run p of column i: lane R i.. of the rows p R ..: (16 R / 4 + R) lanes further per run
-#pragma unroll
-        for (int o = PARTS / 2; o > 0; o >>= 1)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[t][r] += __shfl(acc[t][r], (lane + o * (4 * R + R)) & 63, 64);
-    }
-    if (!stores || n_lo + i >= N) return;
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-        if (m0 + r < a.M) put<E, EPI>(to[r], finished<E, EPI>(a, to[r], n_b, acc[0][r], TWO ? acc[1][r] : 0.0f, bv, bv2), cs);
+    __shared__ f4 red[EPI == PCB_EPI_SILU_MUL ? 2 : 1][8][64];
+    parts_block<E, EPI, PARTS, U, LATE>(a, blockIdx.x, red);
 }
 
 // ---- many rows: both panels travel to LDS by themselves ------------------------------------------------------------------------------
@@ -768,10 +678,7 @@ int dispatch(const pcb_linear_args& a, hipStream_t stream) {
         // 57.1 / 64.4).  A run has eight k-steps at least.  bf16 of more than eight rows over a deep k of few columns stays with sixteen waves above
         // (16 rows, 2048 x 4096: 10.8, here 11.2).
         const int es = sizeof(E), batch = a.n_batch > 0 ? a.n_batch : 1;
-        const bool pieces = a.n_groups == 0 && !a.row_scale && a.K % 32 == 0 && a.ldx * es % 16 == 0 && a.ldw * es % 16 == 0 &&
-                            a.x_batch_stride * es % 16 == 0 && a.w_group_stride * es % 16 == 0 &&
-                            ((uintptr_t)a.x | (uintptr_t)a.w | (uintptr_t)(a.epilogue == PCB_EPI_SILU_MUL ? a.w2 : nullptr)) % 16 == 0;
-        if (pieces && !(es == 2 && a.M > 8 && deep)) {
+        if (pcb_linear_pieces(a) && !(es == 2 && a.M > 8 && deep)) {
             const int64_t four = (int64_t)batch * pcb_ceil_div(a.N, 4), two = (int64_t)batch * pcb_ceil_div(a.N, 8);
             int parts = 1;
             if (a.M <= 4 && four <= 768 && a.K % 128 == 0 && a.K >= 1024)
@@ -855,7 +762,7 @@ int dispatch(const pcb_linear_args& a, hipStream_t stream) {
 
 }  // namespace
 
-PCB_EXPORT int pcb_linear(const pcb_linear_args* a, void* stream) {
+int pcb_linear_check(const pcb_linear_args* a) {
     PCB_REQUIRE(a && a->struct_bytes == sizeof(pcb_linear_args), PCB_ERR_ARG, "pcb_linear: struct size mismatch");
     PCB_REQUIRE(a->dtype == PCB_BF16 || a->dtype == PCB_F32, PCB_ERR_ARG, "pcb_linear: unknown dtype");
     PCB_REQUIRE(a->M >= 0 && a->N > 0 && a->K > 0 && a->ldx >= a->K && a->ldw >= a->K, PCB_ERR_ARG, "pcb_linear: bad sizes");
@@ -890,5 +797,11 @@ PCB_EXPORT int pcb_linear(const pcb_linear_args* a, void* stream) {
                                      a->col_stride3 > 0 && (a->split_n > 0 || a->ldy >= a->split_n3)),
                 PCB_ERR_ARG, "pcb_linear: bad column-wise destination");
     PCB_REQUIRE(a->split_n > 0 || a->split_n3 > 0 || a->epilogue == PCB_EPI_SCALE_ADD || a->ldy >= a->N, PCB_ERR_ARG, "pcb_linear: ldy < N");
+    return PCB_OK;
+}
+
+PCB_EXPORT int pcb_linear(const pcb_linear_args* a, void* stream) {
+    const int rc = pcb_linear_check(a);
+    if (rc != PCB_OK || a->M == 0) return rc;
     return a->dtype == PCB_BF16 ? dispatch<pcb::bf16_t>(*a, (hipStream_t)stream) : dispatch<float>(*a, (hipStream_t)stream);
 }

@@ -1,0 +1,119 @@
+// Products of a few rows with runs of k side by side (pb_linear.hip, pb_linear_pair.hip).
+#pragma once
+#include "pb_linear_epi.h"
+
+namespace pcb {
+
+// A k-step's products into a pair of sums, odd parts into the second (fp32: shorter chains of roundings -- against 64 bits 0.7 of one chain's
+// error at every size -- and of dependent MFMAs; bf16 has one part); chain: into one, in order of k
+template <typename E>
+struct Sum;
+template <>
+struct Sum<bf16_t> {
+    f4 c = {0.f, 0.f, 0.f, 0.f};
+    __device__ __forceinline__ void add(const Frag<bf16_t>& a, const Frag<bf16_t>& b) { c = mma(a, b, c); }
+    __device__ __forceinline__ void chain(const Frag<bf16_t>& a, const Frag<bf16_t>& b) { add(a, b); }
+    __device__ __forceinline__ f4 total() const { return c; }
+};
+template <>
+struct Sum<float> {
+    f4 c[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
+    __device__ __forceinline__ void add(const Frag<float>& a, const Frag<float>& b) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) c[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[e], b.v[e], c[e & 1], 0, 0, 0);
+    }
+    __device__ __forceinline__ void chain(const Frag<float>& a, const Frag<float>& b) { c[0] = mma(a, b, c[0]); }
+    __device__ __forceinline__ f4 total() const { return c[0] + c[1]; }
+};
+
+// Few rows of a plain or batched launch whose rows can be read in 16-byte pieces, whole k-steps; R = 16 / PARTS rows at most.  PARTS runs of k lie side
+// by side in one product: the operands' row (and column) i stands for row i % R of run i / R, so the R x R blocks on the result's diagonal hold the
+// runs' sums of R columns each, and what lies beside them is thrown away.  A workgroup then has R columns instead of 16: twice or four times the
+// workgroups where 16 columns each would leave CUs idle, and as many more loads under way per column.  Eight waves split k; a wave requests U k-steps
+// at a time (a loop of single steps waits for each).
+
+// the waves' sums: lane R i .. of run 0 ends up with what it stores (rows m0 = 4 (lane >> 4) .. + 3 of column lane & 15)
+template <int PARTS>
+__device__ __forceinline__ f4 parts_total(const f4 (*red)[64], int lane) {
+    constexpr int R = 16 / PARTS;
+    f4 acc = red[0][lane];
+#pragma unroll
+    for (int w = 1; w < 8; ++w) acc += red[w][lane];
+    // run p of column i: lane R i.. of the rows p R ..: (16 R / 4 + R) lanes further per run
+#pragma unroll
+    for (int o = PARTS / 2; o > 0; o >>= 1)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[r] += __shfl(acc[r], (lane + o * (4 * R + R)) & 63, 64);
+    return acc;
+}
+
+// Workgroup `block` of such a launch, 512 threads; red: [EPI gated ? 2 : 1][8][64].  LATE: where a result goes is worked out behind the products.
+template <typename E, int EPI, int PARTS, int U, bool LATE>
+__device__ __forceinline__ void parts_block(const pcb_linear_args& a, int block, f4 (*red)[8][64]) {
+    constexpr bool TWO = EPI == PCB_EPI_SILU_MUL, ADD = EPI == PCB_EPI_SCALE_ADD;
+    constexpr int R = 16 / PARTS, SKW = 8;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, group = lane >> 4, l15 = lane & 15;
+    const int K = a.K, N = a.N, n_lo = block * R, g = a.n_batch > 0 ? blockIdx.z : 0;
+    const int run = l15 / R, i = l15 % R;
+    const int n_b = n_lo + i < N ? n_lo + i : N - 1, m_a = i < a.M ? i : a.M - 1;
+    const E* X = (const E*)a.x + g * a.x_batch_stride;
+    const int64_t w_at = g * a.w_group_stride + n_b * a.ldw + 32 * run + 8 * group;
+    const E* wrow = (const E*)a.w + w_at;
+    const E* wrow2 = TWO ? (const E*)a.w2 + w_at : nullptr;
+    const E* xrow = X + (int64_t)(a.row_src ? a.row_src[m_a] : m_a) * a.ldx + 32 * run + 8 * group;
+    // (the lanes that store: rows m0 .. m0 + 3 of column n_b, run 0)
+    const int m0 = 4 * group;
+    float bv = 0.0f, bv2 = 0.0f, cs = 0.0f;
+    Place to[4] = {};
+    const bool stores = wave == 0 && m0 < R && run == 0;
+    auto places = [&] {
+        if (a.bias) bv = to_f32(((const E*)a.bias)[n_b]);
+        if (TWO && a.bias2) bv2 = to_f32(((const E*)a.bias2)[n_b]);
+        if (ADD) cs = a.col_scale[n_b];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (TWO || m0 + r < a.M) to[r] = place<E, EPI>(a, m0 + r < a.M ? m0 + r : a.M - 1, n_b);
+    };
+    if (!LATE && stores) places();
+    Sum<E> sum, sum2;
+    const int steps = K / (32 * PARTS);
+    for (int s0 = wave; s0 < steps; s0 += U * SKW) {
+        Frag<E> fa[U], fb[U], fc[TWO ? U : 1];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (s0 + u * SKW < steps) {                                // (uniform over the wave)
+                const int k = 32 * PARTS * (s0 + u * SKW);
+                fb[u] = load8(wrow + k);
+                if (TWO) fc[u] = load8(wrow2 + k);
+                fa[u] = load8(xrow + k);
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (s0 + u * SKW < steps) {
+                sum.add(fa[u], fb[u]);
+                if (TWO) sum2.add(fa[u], fc[u]);
+            }
+    }
+    if (LATE && stores) places();
+    red[0][wave][lane] = sum.total();
+    if (TWO) red[1][wave][lane] = sum2.total();
+    __syncthreads();
+    if (wave != 0) return;
+    const f4 acc = parts_total<PARTS>(red[0], lane), acc2 = TWO ? parts_total<PARTS>(red[TWO], lane) : f4{};
+    if (!stores || n_lo + i >= N) return;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        if (m0 + r < a.M) put<E, EPI>(to[r], finished<E, EPI>(a, to[r], n_b, acc[r], acc2[r], bv, bv2), cs);
+}
+
+}  // namespace pcb
+
+// PCB_OK when the arguments are valid (pb_linear.hip)
+int pcb_linear_check(const pcb_linear_args* a);
+// whether a launch's rows can be read in 16-byte pieces, whole k-steps
+inline bool pcb_linear_pieces(const pcb_linear_args& a) {
+    const int es = a.dtype == PCB_BF16 ? 2 : 4;
+    return a.n_groups == 0 && !a.row_scale && a.K % 32 == 0 && a.ldx * es % 16 == 0 && a.ldw * es % 16 == 0 && a.x_batch_stride * es % 16 == 0 &&
+           a.w_group_stride * es % 16 == 0 &&
+           ((uintptr_t)a.x | (uintptr_t)a.w | (uintptr_t)(a.epilogue == PCB_EPI_SILU_MUL ? a.w2 : nullptr)) % 16 == 0;
+}

@@ -192,6 +192,8 @@ SIGNATURES = {
     "pcb_embed_scaled_rows": (C.c_int, [_vp, _i32, _vp, _f32, _vp, _i32, _i32, _i32, _vp]),
     "pcb_mix_norm": (C.c_int, [C.POINTER(MixNormArgs), _vp]),
     "pcb_linear": (C.c_int, [C.POINTER(LinearArgs), _vp]),
+    "pcb_linear_pair": (C.c_int, [C.POINTER(LinearArgs), C.POINTER(LinearArgs), _vp]),
+    "pcb_linear_add2": (C.c_int, [C.POINTER(LinearArgs), C.POINTER(LinearArgs), _vp, _vp, _f32, _vp]),
     "pcb_polynorm": (C.c_int, [_vp, _vp, _vp, _i32, _f32, _i32, _i32, _vp]),
     "pcb_router_topk": (C.c_int, [_vp, _i32, _i32, _i32, _vp, _vp, _vp]),
     "pcb_moe_plan": (C.c_int, [_vp, _vp, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp]),
@@ -328,14 +330,14 @@ def mix_norm(hist: torch.Tensor, n_streams: int, coef: Optional[torch.Tensor], g
     check(load().pcb_mix_norm(C.byref(a), _stream()), "pcb_mix_norm")
 
 
-def linear(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, *, M: int, epilogue: int = EPI_STORE, bias=None, w2=None,
-           row_src=None, row_scale=None, group_off=None, n_groups: int = 0, row_dst=None, base=None, col_scale=None,
-           split_n: int = 0, y2=None, row_off2=None, head_dim2: int = 0, head_stride2: int = 0, split_n3: int = 0, y3=None,
-           row_off3=None, col_stride3: int = 0, act: int = ACT_NONE,
-           act_split: int = 0, act2: int = ACT_NONE, act_param: float = 0.0, ldy: Optional[int] = None, bias2=None,
-           ldx: Optional[int] = None, n_batch: int = 0, x_batch_stride: int = 0, y_batch_stride: int = 0, row_gate=None,
-           ld_row_gate: int = 1, y2_f32: bool = False) -> None:
-    """``w``: [N, K], or [groups, N, K] with ``group_off``.  ``x``: [rows, K] of the weights' element type.  ``act`` (and ``act2``
+def linear_args(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, *, M: int, epilogue: int = EPI_STORE, bias=None, w2=None,
+                row_src=None, row_scale=None, group_off=None, n_groups: int = 0, row_dst=None, base=None, col_scale=None,
+                split_n: int = 0, y2=None, row_off2=None, head_dim2: int = 0, head_stride2: int = 0, split_n3: int = 0, y3=None,
+                row_off3=None, col_stride3: int = 0, act: int = ACT_NONE,
+                act_split: int = 0, act2: int = ACT_NONE, act_param: float = 0.0, ldy: Optional[int] = None, bias2=None,
+                ldx: Optional[int] = None, n_batch: int = 0, x_batch_stride: int = 0, y_batch_stride: int = 0, row_gate=None,
+                ld_row_gate: int = 1, y2_f32: bool = False) -> LinearArgs:
+    """What ``linear`` and the calls of two products take, checked.  ``w``: [N, K], or [groups, N, K] with ``group_off``.  ``x``: [rows, K] of the weights' element type.  ``act`` (and ``act2``
     from column ``act_split`` on): the element-wise function of a plain store.  ``ldy``: row stride of ``y`` when it is a
     column block of a wider matrix.  ``n_batch``: that many products at once, ``w`` [n_batch, N, K], their inputs / outputs
     ``x_batch_stride`` / ``y_batch_stride`` elements apart (``ldx`` / ``ldy`` given).  ``row_gate``: E, one factor per row of the gated
@@ -393,12 +395,34 @@ def linear(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, *, M: int, epilogu
     if split_n3:
         _want(row_off3, torch.int64, "linear row_off3")
         assert y3 is not None and y3.dtype == w.dtype and row_off3.numel() >= M and col_stride3 > 0 and split_n3 > split_n
-    a = LinearArgs(C.sizeof(LinearArgs), code, epilogue, _p(x), K if ldx is None else ldx, _p(row_src), _p(row_scale), _p(w), _p(w2), K, _p(bias),
-                   M, N, K, _p(group_off), n_groups, N * K if (n_groups or n_batch) else 0, _p(y), y.shape[-1] if ldy is None else ldy, out_f32,
+    return LinearArgs(C.sizeof(LinearArgs), code, epilogue, _p(x), K if ldx is None else ldx, _p(row_src), _p(row_scale), _p(w), _p(w2), K, _p(bias),
+                      M, N, K, _p(group_off), n_groups, N * K if (n_groups or n_batch) else 0, _p(y), y.shape[-1] if ldy is None else ldy, out_f32,
                    _p(row_dst), _p(base), N, _p(col_scale), split_n, _p(y2), _p(row_off2), head_dim2, head_stride2,
                    split_n3, _p(y3), _p(row_off3), col_stride3, int(act), int(act_split), int(act2), float(act_param), _p(bias2),
                    n_batch, x_batch_stride, y_batch_stride, _p(row_gate), ld_row_gate, int(y2_f32))
+
+
+def linear_run(a: LinearArgs) -> None:
     check(load().pcb_linear(C.byref(a), _stream()), "pcb_linear")
+
+
+def linear(*args, **kw) -> None:
+    """One product: arguments as ``linear_args``."""
+    linear_run(linear_args(*args, **kw))
+
+
+def linear_pair(a: LinearArgs, b: LinearArgs) -> None:
+    """Two products (``linear_args``) of the same number of rows that do not need one another."""
+    check(load().pcb_linear_pair(C.byref(a), C.byref(b), _stream()), "pcb_linear_pair")
+
+
+def linear_add2(a: LinearArgs, b: LinearArgs, z: Optional[torch.Tensor] = None, coef: Optional[torch.Tensor] = None, eps: float = 0.0) -> None:
+    """Two scaled accumulations (``linear_args``) into the same rows; with ``z`` (fp32) the second one's input is ``polynorm(z, coef, eps)``, its ``x``
+    scratch for that."""
+    if z is not None:
+        _want(z, torch.float32, "linear_add2 z"); _want(coef, torch.float32, "linear_add2 coef")
+        assert coef.numel() == 4 and z.shape[-1] == b.K and z.shape[0] >= b.M
+    check(load().pcb_linear_add2(C.byref(a), C.byref(b), _p(z), _p(coef), float(eps), _stream()), "pcb_linear_add2")
 
 
 def polynorm(z: torch.Tensor, coef: torch.Tensor, out: torch.Tensor, eps: float, n_rows: int) -> None:

@@ -385,10 +385,10 @@ class FivesunHIP(SlotModel):
             if l.ff:
                 step(lw["norm2"], h)
                 rg = self._mat("ff_gate", T, W, E)
-                B.linear(h, lw["rg2"], rg, M=T, bias=lw["rg2b"], act=B.ACT_SIGMOID)
                 mid = self._mat("ff_mid", T, l.ff, E)
-                B.linear(h, lw["w_gate"], mid, M=T, epilogue=B.EPI_SILU_MUL, w2=lw["w_up"], bias=lw["b_gate"], bias2=lw["b_up"],
-                         act=ACTS[l.act])
+                B.linear_pair(B.linear_args(h, lw["rg2"], rg, M=T, bias=lw["rg2b"], act=B.ACT_SIGMOID),
+                              B.linear_args(h, lw["w_gate"], mid, M=T, epilogue=B.EPI_SILU_MUL, w2=lw["w_up"], bias=lw["b_gate"], bias2=lw["b_up"],
+                                            act=ACTS[l.act]))
                 B.linear(mid, lw["w_down"], y2, M=T, bias=lw["b_down"])
                 pending = dict(y=y2, gate=rg, ldg=W, post_gain=lw["norm2b"])
             if streams is not None:

@@ -205,19 +205,23 @@ class KazolornHIP(SlotModel):
             HD, GD = l.heads * l.dim, l.kv_heads * l.dim
             q = self._mat("q", T, HD, E)
             plane = arena.planes[i]
-            B.linear(h1, lw["wqk"], q, M=T, bias=lw["bqk"], split_n=HD, y2=plane, row_off2=offs_d[sigs.index((l.kv_heads, l.dim))],
-                     head_dim2=l.dim, head_stride2=arena.head_stride(i))
+            qk = B.linear_args(h1, lw["wqk"], q, M=T, bias=lw["bqk"], split_n=HD, y2=plane, row_off2=offs_d[sigs.index((l.kv_heads, l.dim))],
+                               head_dim2=l.dim, head_stride2=arena.head_stride(i))
+            if l.mlp_kind == "dense":
+                # (both halves of a layer start from the same input: their products go out two by two)
+                z, act = self._mat("z", T, l.ff, f32), self._mat("act", T, l.ff, E)
+                B.linear_pair(qk, B.linear_args(h2, lw["up"], z, M=T))
+            else:
+                B.linear_run(qk)
             att = self._mat("att", T, HD, E)
             self._attention(q, att, tiles, n_tiles, tiles_d, tiles64_d, n64, plane, arena, i, l, lw, max_kv,
                             max_rows=1 if n_tiles == T else (int(tiles[:, 2].max()) if tiles is not None and n64 == n_tiles else 0))
-            B.linear(att, lw["wo"], hist[i + 1], M=T, epilogue=B.EPI_SCALE_ADD, bias=lw["bo"], base=base, col_scale=lw["ls1"])
+            wo = B.linear_args(att, lw["wo"], hist[i + 1], M=T, epilogue=B.EPI_SCALE_ADD, bias=lw["bo"], base=base, col_scale=lw["ls1"])
             if l.mlp_kind == "dense":
-                z = self._mat("z", T, l.ff, f32)
-                B.linear(h2, lw["up"], z, M=T)
-                act = self._mat("act", T, l.ff, E)
-                B.polynorm(z, lw["act"], act, eps, T)
-                B.linear(act, lw["down"], hist[i + 1], M=T, epilogue=B.EPI_SCALE_ADD, col_scale=lw["ls2"])
-            elif l.mlp_kind == "moe":
+                B.linear_add2(wo, B.linear_args(act, lw["down"], hist[i + 1], M=T, epilogue=B.EPI_SCALE_ADD, col_scale=lw["ls2"]), z, lw["act"], eps)
+                continue
+            B.linear_run(wo)
+            if l.mlp_kind == "moe":
                 P = T * l.top
                 ex = self._scratch("moe_i", 3 * P + l.experts + 1, torch.int32)
                 sc = self._scratch("moe_f", 2 * P, f32)
