@@ -7,6 +7,8 @@
 // position in the thousands costs no bits of the angle -- and its waves then take the heads in turn: one pass for the sum of
 // squares, one that norms, blends, turns and stores.  A lane owns the two columns of a pair, so a rotation never crosses lanes
 // (and a segment may work in place).
+//
+// Heads of whole 16-byte chunks go through head_prep_chunks_kernel: a lane has eight neighbouring columns (four pairs), 16, 32 or 64 lanes a head.
 #include "pb_common.h"
 
 namespace {
@@ -120,6 +122,149 @@ __global__ __launch_bounds__(256) void head_prep_kernel(pcb_head_prep_args a) {
         prep_heads<E, false>(a, s, row, cs, sn, red);
 }
 
+// The same for heads of up to 512 columns whose chunks of eight can be read and written at once, neighbouring pairs turning.  Workgroup = RW rows: its
+// threads make the rows' turns (one float64 sincos each, where the kernel above makes them again for every segment), its waves take tasks of one row and
+// 64 lanes' heads of a segment; a task's row is requested before the one in front of it is worked on, the first before the turns.
+// What bounds it: bytes (2048 rows: 30 MB, 6 us at the copy rate) behind a launch and a sincos of 3.5 us.  us, the kernel above / this, 16 heads of 128
+// over 4, bf16: 1 row 3.9 / 3.6, 300 rows 9.1 / 4.6, 2048 rows 22.5 / 10.1 (18 with four waves a workgroup); a latent's four segments 3.2 / 3.4, 6.5 / 4.1,
+// 21.8 / 10.2; fp32, 2048 rows 25.1 / 14.2.
+constexpr int TURNS = 512;                                       // turns of a workgroup's rows
+
+__host__ __device__ __forceinline__ int lanes_of(int head_dim) { return head_dim <= 64 ? 8 : head_dim <= 128 ? 16 : head_dim <= 256 ? 32 : 64; }
+__host__ __device__ __forceinline__ int tasks_of(const pcb_head_prep_seg& s) {
+    const int per = 64 / lanes_of(s.head_dim);
+    return (s.heads + per - 1) / per;
+}
+
+struct Tasks {
+    int32_t first[5];                                            // a row's tasks: of segment i first[i] .. first[i + 1] - 1
+};
+
+template <typename E>
+__global__ __launch_bounds__(512) void head_prep_chunks_kernel(pcb_head_prep_args a, Tasks f, int rw, int np) {
+    __shared__ float cs[TURNS], sn[TURNS];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t row0 = (int64_t)blockIdx.x * rw;
+    const int waves = blockDim.x >> 6, n_tasks = f.first[4], rows = a.n_rows - row0 < rw ? (int)(a.n_rows - row0) : rw, tasks = rows * n_tasks;
+    const int step = waves * gridDim.y;
+    struct Task {
+        int seg, r, h, c;                                        // segment, row of the workgroup, the lane's head and first column
+        bool on;
+        Frag<E> x;
+    };
+    auto load = [&](int t, Task& k) {
+        k.on = false;
+        if (t >= tasks) return;
+        k.r = rw > 1 ? t / n_tasks : 0;
+        int at = t - k.r * n_tasks;
+        k.seg = (at >= f.first[1]) + (at >= f.first[2]) + (at >= f.first[3]);
+        at -= f.first[k.seg];
+        const pcb_head_prep_seg& s = a.seg[k.seg];
+        const int lph = lanes_of(s.head_dim);
+        k.h = at * (64 / lph) + lane / lph;
+        k.c = 8 * (lane % lph);
+        k.on = k.h < s.heads && k.c < s.head_dim;
+        zero8(k.x);
+        if (k.on) k.x = load8((const E*)s.src + (row0 + k.r) * s.ld_src + (int64_t)k.h * s.src_head_stride + k.c);
+    };
+    int t = wave + waves * blockIdx.y;
+    Task cur;
+    load(t, cur);
+    if (np > 0) {
+        for (int e = threadIdx.x; e < rows * np; e += blockDim.x) {
+            const int r = rw > 1 ? e / np : 0, i = e - r * np;
+            if (a.table) {
+                cs[e] = a.table[(row0 + r) * 2 * np + i];
+                sn[e] = a.table[(row0 + r) * 2 * np + np + i];
+            } else {
+                double sv, cv;
+                sincos((double)a.pos[row0 + r] * a.freqs[i], &sv, &cv);
+                cs[e] = (float)cv * a.rot_mag;
+                sn[e] = (float)sv * a.rot_mag;
+            }
+        }
+        __syncthreads();
+    }
+    for (; t < tasks; t += step) {
+        Task next;
+        load(t + step, next);
+        const pcb_head_prep_seg& s = a.seg[cur.seg];
+        const int64_t row = row0 + cur.r;
+        const int D = s.head_dim;
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = at8(cur.x, e);
+        if (s.norm) {
+            float ss = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+            ss += __shfl_xor(ss, 1, 64);
+            ss += __shfl_xor(ss, 2, 64);
+            ss += __shfl_xor(ss, 4, 64);
+            if (D > 64) ss += __shfl_xor(ss, 8, 64);
+            if (D > 128) ss += __shfl_xor(ss, 16, 64);
+            if (D > 256) ss += __shfl_xor(ss, 32, 64);
+            const float inv = 1.0f / sqrtf(ss / (float)D + a.eps);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] *= inv;
+        }
+        if (cur.on) {
+            auto eight = [](const float* p, float (&o)[8]) {
+                const f4 lo = *reinterpret_cast<const f4*>(p), hi = *reinterpret_cast<const f4*>(p + 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = lo[e], o[4 + e] = hi[e];
+            };
+            if (s.gain) {
+                float g[8];
+                eight(s.gain + cur.c, g);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] *= g[e];
+            }
+            if (s.blend) {
+                float o[8];
+                eight(s.other + row * s.ld_other + (int64_t)cur.h * D + cur.c, o);
+                const float lam = s.blend[0];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = (1.0f - lam) * v[e] + lam * o[e];
+            }
+            if (s.keep) {
+                float* k = s.keep + row * s.ld_keep + (int64_t)cur.h * D + cur.c;
+                *reinterpret_cast<f4*>(k) = f4{v[0], v[1], v[2], v[3]};
+                *reinterpret_cast<f4*>(k + 4) = f4{v[4], v[5], v[6], v[7]};
+            }
+            const int i = (cur.c - s.rot_off) / 2;
+            if (cur.c >= s.rot_off && 2 * i < s.rot_dims) {
+                const float* c = cs + cur.r * np + i;
+                const float* n = sn + cur.r * np + i;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float u = v[2 * e], w = v[2 * e + 1];
+                    v[2 * e] = u * c[e] - w * n[e];
+                    v[2 * e + 1] = w * c[e] + u * n[e];
+                }
+            }
+            E* d = (E*)s.dst + (s.row_off ? s.row_off[row] : row * s.ld_dst) + (int64_t)cur.h * s.head_stride + cur.c;
+            if ((uintptr_t)d % 16 == 0) {
+                store4(d, v[0], v[1], v[2], v[3]);
+                store4(d + 4, v[4], v[5], v[6], v[7]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) d[e] = from_f32<E>(v[e]);
+            }
+        }
+        cur = next;
+    }
+}
+
+// whether a segment's heads are whole chunks of eight columns, read and written 16 bytes at a time
+bool chunks_ok(const pcb_head_prep_args& a, const pcb_head_prep_seg& s) {
+    const int64_t es = a.dtype == PCB_BF16 ? 2 : 4;
+    auto whole = [](int64_t bytes) { return bytes % 16 == 0; };
+    return s.head_dim % 8 == 0 && s.head_dim <= 512 && s.col_stride == 1 && whole((uintptr_t)s.src) && whole(s.ld_src * es) && whole(s.src_head_stride * es) &&
+           whole((uintptr_t)s.gain) && (!s.blend || (whole((uintptr_t)s.other) && whole(s.ld_other * 4))) &&
+           (!s.keep || (whole((uintptr_t)s.keep) && whole(s.ld_keep * 4))) && (s.rot_dims == 0 || (!a.rot_half && s.rot_off % 8 == 0 && s.rot_dims % 8 == 0));
+}
+
 __global__ __launch_bounds__(256) void rot_table_kernel(const int32_t* __restrict__ pos, const double* __restrict__ freqs, float mag,
                                                         float* __restrict__ out, int n_rows, int np) {
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -162,6 +307,23 @@ PCB_EXPORT int pcb_head_prep(const pcb_head_prep_args* a, void* stream) {
     }
     if (a->n_rows == 0) return PCB_OK;
     PCB_REQUIRE(rot == 0 || a->table || (a->pos && a->freqs), PCB_ERR_ARG, "pcb_head_prep: a rotation needs positions and frequencies");
+    bool chunks = rot <= 2 * TURNS;
+    Tasks f{};
+    for (int i = 0; i < 4; ++i) {
+        chunks = chunks && (i >= a->n_segs || chunks_ok(*a, a->seg[i]));
+        f.first[i + 1] = f.first[i] + (i < a->n_segs ? tasks_of(a->seg[i]) : 0);
+    }
+    if (chunks) {
+        // (few rows: a row's tasks are spread over workgroups of four waves; many: a workgroup of eight has up to four rows' turns)
+        const int np = rot / 2, rw = a->n_rows >= 1024 ? (np <= 64 ? 4 : np <= 128 ? 2 : 1) : 1;
+        const bool few = a->n_rows <= 64;
+        const dim3 grid(pcb_ceil_div(a->n_rows, rw), few ? pcb_ceil_div(f.first[4], 4) : 1), threads(few ? 256 : 512);
+        if (a->dtype == PCB_BF16)
+            hipLaunchKernelGGL(head_prep_chunks_kernel<pcb::bf16_t>, grid, threads, 0, (hipStream_t)stream, *a, f, rw, np);
+        else
+            hipLaunchKernelGGL(head_prep_chunks_kernel<float>, grid, threads, 0, (hipStream_t)stream, *a, f, rw, np);
+        return pcb_check_launch("head_prep_chunks_kernel");
+    }
     // (few rows: a row's heads are spread over workgroups, so that a wave has one)
     int most = 1;
     for (int i = 0; i < a->n_segs; ++i) most = a->seg[i].heads > most ? a->seg[i].heads : most;
