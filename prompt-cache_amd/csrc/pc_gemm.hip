@@ -60,6 +60,24 @@ int launch_MT(int epi, const GemmParams& p, int T, int units, hipStream_t s) {
 // preceding pc_gemm_skinny left behind -- the residual add of llama2.py:638 / :644 happens here, in place.
 // LN = true: torch.nn.LayerNorm instead (Falcon, falcon.py:757): mean removed (two passes over the register-resident
 // row, no cancellation), bias `b` added after the gain.
+// Gains and bias are requested with the row, ahead of the residual's store: stores and loads count on one counter, so a load behind that store waits for
+// its way to memory.  The sums over a wave's lanes go without LDS where the machine can (the same pairs, hence the same bits).
+// What bounds it: the launch (2.4 us), one row a CU, one trip to memory, one (LN: two) sums over the workgroup.  us, loads and sums as they were / so, hidden
+// 4096, four slabs: 27 rows 4.66 / 4.36 and LN 5.35 / 4.66, 256 rows 9.16 / 9.01; hidden 8192, 1 row 5.88 / 5.09.
+__device__ __forceinline__ float lanes_sum(float v) {
+    auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(s32[0]) + __uint_as_float(s32[1]);
+    auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(s16[0]) + __uint_as_float(s16[1]);
+    auto dpp = [](float x, auto ctrl) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, 0xf, 0xf, true));
+    };
+    v += dpp(v, std::integral_constant<int, 0x128>{});           // lane ^ 8 (the row of 16 turned by eight)
+    v += __shfl_xor(v, 4);
+    v += dpp(v, std::integral_constant<int, 0x4e>{});            // lane ^ 2
+    v += dpp(v, std::integral_constant<int, 0xb1>{});            // lane ^ 1
+    return v;
+}
 template <int G, bool LN = false>   // G = 8-element groups per thread: the whole row stays in registers between the passes
 __global__ __launch_bounds__(256) void rmsnorm_frag_kernel(float* __restrict__ x, const _Float16* __restrict__ w,
                                                            _Float16* __restrict__ of_hi, _Float16* __restrict__ of_lo,
@@ -72,6 +90,7 @@ __global__ __launch_bounds__(256) void rmsnorm_frag_kernel(float* __restrict__ x
     const int nv = hidden >> 3;
     float* xr = x + (int64_t)row * hidden;
     f4 va[G], vb[G];
+    h8 gw[G], bw[G];
     float ss = 0.f;
 #pragma unroll
     for (int k = 0; k < G; ++k) {
@@ -82,6 +101,10 @@ __global__ __launch_bounds__(256) void rmsnorm_frag_kernel(float* __restrict__ x
             va[k] = *(const f4*)(xr + i * 8);
             vb[k] = *(const f4*)(xr + i * 8 + 4);
         }
+        const int ic = i < nv ? i : nv - 1;
+        gw[k] = *(const h8*)(w + ic * 8);
+        bw[k] = h8{0, 0, 0, 0, 0, 0, 0, 0};
+        if (LN && b) bw[k] = *(const h8*)(b + ic * 8);
     }
     if (nslabs > 0) {
         // CH slabs at a time: all of their loads are issued before the first add (clamped, unconditional), so a chunk
@@ -129,8 +152,7 @@ __global__ __launch_bounds__(256) void rmsnorm_frag_kernel(float* __restrict__ x
 #pragma unroll
         for (int k = 0; k < G; ++k)       // lanes past the end of the row hold zeros
             sm += va[k][0] + va[k][1] + va[k][2] + va[k][3] + vb[k][0] + vb[k][1] + vb[k][2] + vb[k][3];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) sm += __shfl_xor(sm, o);
+        sm = lanes_sum(sm);
         if ((tid & 63) == 0) redm[tid >> 6] = sm;
         __syncthreads();
         mu = (redm[0] + redm[1] + redm[2] + redm[3]) / (float)hidden;
@@ -146,8 +168,7 @@ __global__ __launch_bounds__(256) void rmsnorm_frag_kernel(float* __restrict__ x
     for (int k = 0; k < G; ++k)
         ss += va[k][0] * va[k][0] + va[k][1] * va[k][1] + va[k][2] * va[k][2] + va[k][3] * va[k][3] +
               vb[k][0] * vb[k][0] + vb[k][1] * vb[k][1] + vb[k][2] * vb[k][2] + vb[k][3] * vb[k][3];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+    ss = lanes_sum(ss);
     if ((tid & 63) == 0) red[tid >> 6] = ss;
     __syncthreads();
     const float rs = rsqrtf((red[0] + red[1] + red[2] + red[3]) / (float)hidden + eps);
@@ -156,14 +177,11 @@ __global__ __launch_bounds__(256) void rmsnorm_frag_kernel(float* __restrict__ x
     for (int k = 0; k < G; ++k) {
         const int i = tid + k * 256;
         if (i < nv) {
-            const h8 gw = *(const h8*)(w + i * 8);
-            h8 bw = {0, 0, 0, 0, 0, 0, 0, 0};
-            if (LN && b) bw = *(const h8*)(b + i * 8);
             h8 hi, lo;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                float v = (float)gw[e] * ((e < 4 ? va[k][e] : vb[k][e - 4]) * rs);
-                if (LN) v += (float)bw[e];
+                float v = (float)gw[k][e] * ((e < 4 ? va[k][e] : vb[k][e - 4]) * rs);
+                if (LN) v += (float)bw[k][e];
                 _Float16 vh, vl;
                 pc_split(v, vh, vl);
                 hi[e] = vh; lo[e] = vl;
