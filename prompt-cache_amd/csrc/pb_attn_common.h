@@ -19,6 +19,14 @@ __device__ __forceinline__ float exp_le0(float x) {
     return __builtin_fmaf(e, lo * 6.93147182e-01f, e);
 }
 
+// the largest over the four lane groups (16 lanes apart)
+__device__ __forceinline__ float max4(float v) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
 // eight softmax weights of a lane.  bf16: a hi + lo pair of bf16 values (two MFMAs), so that they are not rounded to 8 bits; fp32: as
 // they are
 template <typename E>
@@ -33,17 +41,14 @@ struct PFrag<float> {
 };
 
 __device__ __forceinline__ void make_p(PFrag<bf16_t>& f, const float (&p)[8]) {
-    // hi = the upper 16 bits of p as they stand, lo = the rest, cut to 16 bits: hi + lo carries 16 bits of p's mantissa (p is a
-    // finite non-negative weight, so no rounding carry or NaN needs care)
-    uint32_t h[8], l[8];
+    // hi = p, lo = what that leaves, both rounded to nearest: hi + lo carries 17 bits of p's mantissa.  Six instructions a pair of weights; cutting the upper
+    // 16 bits off instead took twelve.
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const uint32_t u = __float_as_uint(p[e]);
-        h[e] = u >> 16;
-        l[e] = __float_as_uint(p[e] - __uint_as_float(u & 0xffff0000u)) >> 16;
+    for (int e = 0; e < 4; ++e) {
+        const uint32_t w = bf16_pair(p[2 * e], p[2 * e + 1]);
+        f.hi.v[e] = w;
+        f.lo.v[e] = bf16_pair(p[2 * e] - __uint_as_float(w << 16), p[2 * e + 1] - __uint_as_float(w & 0xffff0000u));
     }
-    f.hi.v = u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
-    f.lo.v = u32x4{l[0] | (l[1] << 16), l[2] | (l[3] << 16), l[4] | (l[5] << 16), l[6] | (l[7] << 16)};
 }
 __device__ __forceinline__ void make_p(PFrag<float>& f, const float (&p)[8]) {
 #pragma unroll

@@ -6,11 +6,14 @@
 // flight while this one is worked on) and serve all 64 QT queries.  Both products are "swapped" as in pb_attn_soft.hip:
 //   S^T = K Q^T   K operand: 16-byte reads of LDS key rows; the lane's column is its query,
 //   O^T = V^T P^T V operand: transposed LDS reads of the same row-major value tile (bf16), P straight from the lane's registers.
-// A wave's queries are its own from start to end, so nothing is merged at the end.  Waves whose queries all precede a block skip its
+// A wave's queries are its own from start to end, so nothing is merged at the end -- except where two halves of four waves (KG = 2) share the key blocks
+// of a tile in turn: the second half's results pass through LDS then.  Waves whose queries all precede a block skip its
 // products; only blocks that straddle a query's own position or a window's edge pay for masks.  The keys' last tail_dim columns may be
 // shared by all heads (one rotated part per token): they are then fetched from rows of their own, through an index table if given.
 // Keys and values may also lie in a slot's cache, and a query may see its window or its block of positions only.
 // Workgroups of one head are neighbours eight apart in launch order: they share that head's keys and values in one XCD's L2.
+#include <type_traits>
+
 #include "pb_attn_common.h"
 
 namespace {
@@ -36,8 +39,8 @@ __device__ __forceinline__ int oldest(const pcb_attn_prompt_args& a, int i) {
 }
 
 // KSQ: 32-element k-steps of the key size; VB: 16-column blocks of the value size; BK: keys per block
-template <typename E, int KSQ, int VB, int QT, int BK>
-__global__ __launch_bounds__(64 * PW) void attn_prompt_kernel(pcb_attn_prompt_args a) {
+template <typename E, int KSQ, int VB, int QT, int BK, int KG>
+__global__ __launch_bounds__(64 * PW * KG) void attn_prompt_kernel(pcb_attn_prompt_args a) {
     constexpr int CE = 16 / sizeof(E);
     constexpr int KC = KSQ * 32, VC = VB * 16;                       // columns of the tiles
     constexpr int KLD = KC + CE, VLD = v_ld<E>(VC);
@@ -45,9 +48,11 @@ __global__ __launch_bounds__(64 * PW) void attn_prompt_kernel(pcb_attn_prompt_ar
     constexpr int KCH = KC / CE / LPR, VCH = VC / CE / LPR;          // 16-byte chunks per thread
     static_assert(KC / CE % LPR == 0 && VC / CE % LPR == 0, "whole chunks per thread");
     constexpr int NKT = BK / 16, NK2 = BK / 32;
-    __shared__ __attribute__((aligned(16))) E Ks[BK * KLD];
-    __shared__ __attribute__((aligned(16))) E Vs[BK * VLD];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, c = lane & 15;
+    __shared__ __attribute__((aligned(16))) E lds[KG][BK * KLD + BK * VLD];
+    const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * PW));       // the wave's share of the key blocks
+    E* const Ks = lds[kg];
+    E* const Vs = lds[kg] + BK * KLD;
+    const int tid = threadIdx.x & (64 * PW - 1), lane = tid & 63, wave = tid >> 6, g = lane >> 4, c = lane & 15;
     const int h = blockIdx.x, hk = h / (a.H / a.Hkv);
     // (tiles from the last to the first: within a request later tiles see more keys, and the long ones should not start last)
     const int32_t* tile = a.tiles + 4 * (gridDim.y - 1 - blockIdx.y);
@@ -130,8 +135,9 @@ __global__ __launch_bounds__(64 * PW) void attn_prompt_kernel(pcb_attn_prompt_ar
             }
         }
     };
-    if (plain) fetch(kb_lo);
-    for (int kb = kb_lo; kb <= kb_hi; ++kb) {
+    if (plain) fetch(kb_lo + kg < kb_hi ? kb_lo + kg : kb_hi);
+    for (int kb0 = kb_lo; kb0 <= kb_hi; kb0 += KG) {
+        const int kb = kb0 + kg;                                     // (past the last: the block in front of it again, not used)
         __syncthreads();                                             // the previous block's reads are done
         if (plain) {
 #pragma unroll
@@ -139,12 +145,12 @@ __global__ __launch_bounds__(64 * PW) void attn_prompt_kernel(pcb_attn_prompt_ar
 #pragma unroll
             for (int i = 0; i < VCH; ++i) *reinterpret_cast<u32x4*>(&Vs[lr * VLD + lc + i * LPR * CE]) = rv[i];
         } else {
-            fetch(kb);                                               // (odd sizes: element by element, straight into LDS)
+            fetch(kb < kb_hi ? kb : kb_hi);                          // (odd sizes: element by element, straight into LDS)
         }
         __syncthreads();
-        if (plain && kb < kb_hi) fetch(kb + 1);
+        if (plain && kb0 + KG <= kb_hi) fetch(kb + KG < kb_hi ? kb + KG : kb_hi);
         const int k0 = kb * BK;
-        if (!busy || k0 > w_last || k0 + BK - 1 < w_lo) continue;
+        if (!busy || kb > kb_hi || k0 > w_last || k0 + BK - 1 < w_lo) continue;
 
         f4 s[QT][NKT];
 #pragma unroll
@@ -175,8 +181,7 @@ __global__ __launch_bounds__(64 * PW) void attn_prompt_kernel(pcb_attn_prompt_ar
                     s[qt][kt][r] = v;
                     bm = fmaxf(bm, v);
                 }
-            bm = fmaxf(bm, __shfl_xor(bm, 16, 64));
-            bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
+            bm = max4(bm);
             const float m_new = fmaxf(m[qt], bm);
             const float m_use = m_new == NEG ? 0.0f : m_new;
             const float alpha = __builtin_amdgcn_exp2f(m[qt] - m_use);          // (m = -inf: 0)
@@ -208,6 +213,34 @@ __global__ __launch_bounds__(64 * PW) void attn_prompt_kernel(pcb_attn_prompt_ar
 #pragma unroll
                 for (int qt = 0; qt < QT; ++qt) o[qt][vb] = mma_p(vf, pf[qt][k2], o[qt][vb]);
             }
+    }
+    if constexpr (KG == 2) {
+        // the second half's sums, maxima and denominators through LDS (a lane's own: both halves hold them alike)
+        float* const half = reinterpret_cast<float*>(lds) + wave * (QT * (4 * VB + 2) * 64) + lane;
+        static_assert((int)sizeof(lds) >= PW * QT * (4 * VB + 2) * 64 * 4, "room for a half's results");
+        __syncthreads();
+        if (kg == 1) {
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt) {
+                float* const h1 = half + qt * (4 * VB + 2) * 64;
+#pragma unroll
+                for (int e = 0; e < 4 * VB; ++e) h1[e * 64] = o[qt][e >> 2][e & 3];
+                h1[4 * VB * 64] = m[qt];
+                h1[(4 * VB + 1) * 64] = l[qt];
+            }
+        }
+        __syncthreads();
+        if (kg == 1) return;
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {
+            const float* const h1 = half + qt * (4 * VB + 2) * 64;
+            const float m1 = h1[4 * VB * 64], top = fmaxf(m[qt], m1), use = top == NEG ? 0.0f : top;
+            const float f0 = __builtin_amdgcn_exp2f(m[qt] - use), f1 = __builtin_amdgcn_exp2f(m1 - use);
+            l[qt] = l[qt] * f0 + h1[(4 * VB + 1) * 64] * f1;
+#pragma unroll
+            for (int e = 0; e < 4 * VB; ++e) o[qt][e >> 2][e & 3] = o[qt][e >> 2][e & 3] * f0 + h1[e * 64] * f1;
+            m[qt] = top;
+        }
     }
     if (!busy) return;
 #pragma unroll
@@ -253,11 +286,30 @@ __global__ __launch_bounds__(64 * PW) void attn_prompt_kernel(pcb_attn_prompt_ar
 
 template <typename E, int KSQ, int VB, int BK>
 int launch(const pcb_attn_prompt_args& a, hipStream_t stream) {
-    const dim3 grid(a.H, a.n_tiles), block(64 * PW);
-    if (sizeof(E) == 2 && a.tile_rows == 128)
-        hipLaunchKernelGGL((attn_prompt_kernel<E, KSQ, VB, sizeof(E) == 2 ? 2 : 1, BK>), grid, block, 0, stream, a);
-    else
-        hipLaunchKernelGGL((attn_prompt_kernel<E, KSQ, VB, 1, BK>), grid, block, 0, stream, a);
+    const dim3 grid(a.H, a.n_tiles);
+    auto go = [&](auto qt, auto kg) {
+        constexpr int Q = decltype(qt)::value, G = decltype(kg)::value;
+        hipLaunchKernelGGL((attn_prompt_kernel<E, KSQ, VB, Q, BK, G>), grid, dim3(64 * PW * G), 0, stream, a);
+    };
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
+    if constexpr (sizeof(E) == 2)
+        if (a.tile_rows == 128) {
+            go(Two{}, One{});
+            return pcb_check_launch("attn_prompt_kernel");
+        }
+    // Two halves while the chip has a CU for every tile and head, keys of up to 128 columns also two of them (the longest tile's chain of blocks is what a
+    // launch takes: 2.3 us a block of 64); beyond, a CU is better off with workgroups of four waves.  us, one half / two, bf16: 16 heads of 128, 1024 rows
+    // 36 / 26, 600 rows 24 / 17, 2048 rows in blocks of 1024 (512 workgroups) 46 / 35, 8 x 300 rows (640) 20 / 29, 5000 rows 205 / 296; 192-column keys,
+    // 8 heads, 2048 rows 44 / 33, 16 heads 54 / 65; fp32, 8 heads: 2 x 300 rows 36 / 34, 2048 rows 105 / 94, 16 heads 170 / 116.
+    const int64_t wgs = (int64_t)a.H * a.n_tiles;
+    if constexpr (VB <= 8) {
+        if (wgs <= (KSQ <= 4 ? 512 : 256)) {
+            go(One{}, Two{});
+            return pcb_check_launch("attn_prompt_kernel");
+        }
+    }
+    go(One{}, One{});
     return pcb_check_launch("attn_prompt_kernel");
 }
 

@@ -132,8 +132,7 @@ __global__ __launch_bounds__(64 * LW) void attn_rows_kernel(pcb_attn_rows_args a
                 bm = fmaxf(bm, s[kt][r]);
             }
         }
-        bm = fmaxf(bm, __shfl_xor(bm, 16, 64));
-        bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
+        bm = max4(bm);
         const float m_new = fmaxf(m, bm);
         const float m_use = m_new == NEG ? 0.0f : m_new;
         const float alpha = __builtin_amdgcn_exp2f(m - m_use);       // (m = -inf: 0)

@@ -30,14 +30,6 @@ __device__ __forceinline__ int key_spread(int j) { return (((j & 7) ^ (j >> 1 & 
 // blocks 2 and 3.
 __device__ __forceinline__ int row_spread(int b, int r) { return (r >> 1) ^ (b & 1); }
 
-// over the four lane groups
-__device__ __forceinline__ float max4(float v) {
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-
 // HKV key heads (H = 4 HKV).  `parts` workgroups share the keys of the same rows: each leaves [part][row][head]{D sums} and, behind all of these,
 // {maximum, denominator} in the scratch, to be merged by talk_merge_kernel.
 template <int HKV, int NU>
