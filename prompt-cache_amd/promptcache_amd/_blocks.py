@@ -268,7 +268,8 @@ def _p(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current device's current stream as a handle (see ``_native.current_stream``)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _code(t: torch.Tensor) -> int:

