@@ -92,7 +92,6 @@ class MptHIP(LlamaHIP):
                  **_unused) -> CausalLMOutput:
         dev = self.device
         self._kv_only = bool(kv_only)
-        input_ids = input_ids.to(dev)
         B, q_len = input_ids.shape
         arena, past_len = self._resolve_arena(past_key_values, B, q_len)
         if many_rows and self.precise_dense and past_key_values is None:
@@ -101,8 +100,8 @@ class MptHIP(LlamaHIP):
         if position_ids is None:
             if past_len:
                 raise ValueError("MPT needs the position id of every cached key (use_full_position_ids, mpt.py:172)")
-            position_ids = torch.arange(q_len, device=dev).unsqueeze(0).expand(B, q_len)
-        position_ids = position_ids.to(dev).reshape(B, -1)
+            position_ids = torch.arange(q_len, device=input_ids.device).unsqueeze(0).expand(B, q_len)
+        position_ids = position_ids.reshape(B, -1)
         if position_ids.shape[1] != kv_len:
             raise ValueError(f"MPT got {position_ids.shape[1]} position ids for {kv_len} keys: pass the full position ids "
                              "(CacheEngine.process(..., return_full_position_ids=True), mpt.py:172)")
@@ -125,6 +124,8 @@ class MptHIP(LlamaHIP):
         mid = self.skinny and not encode_pass and T <= self.MID_MAX_ROWS and \
             not (many_rows and self.precise_dense and T > self.SKINNY_MAX_ROWS)
         self._lo_mode = self._tail_mode(arena, q_len, past_len) if (graphed or mid) else 0
+        if not (graphed and ids.device.type == "cpu" and position_ids.device.type == "cpu"):      # (from the host: _graphed_mpt's own upload)
+            ids, position_ids = ids.to(dev), position_ids.to(dev)
         if graphed:
             logits = self._graphed_mpt(ids, position_ids, arena, B, q_len, past_len, last_token_only, num_layers)
         else:
@@ -152,16 +153,29 @@ class MptHIP(LlamaHIP):
         else:
             if len(self._graphs) >= self.max_graphs:
                 self._graphs.pop(next(iter(self._graphs)))   # evict the least recently used
-            st_ids = torch.zeros(B * q_len, dtype=torch.int64, device=self.device)
-            st_kpos = torch.zeros((B, self._kpos_cols(arena.cap)), dtype=torch.float32, device=self.device)
-            st_past = torch.zeros(2, dtype=torch.int32, device=self.device)      # {past_len, base of the residual tail}
-            ent = [None, st_ids, st_kpos, st_past, None]
-        _, st_ids, st_kpos, st_past, out = ent
-        st_ids.copy_(ids)
-        st_kpos[:, :kv_len].copy_(position_ids)           # int64 -> fp32 on the fly
-        st_past[0:1].fill_(past_len)
-        if mode == 2:
-            st_past[1:2].fill_(arena.tail_base)
+            # the step's inputs in one block: {past_len, base of the residual tail}, ids, positions -- and its image in pinned memory
+            cols = self._kpos_cols(arena.cap)
+            at = 16 + (8 * B * q_len + 15) // 16 * 16
+            sides = [torch.zeros(at + 4 * B * cols, dtype=torch.uint8, **kw) for kw in (dict(device=self.device), dict(pin_memory=True))]
+            views = [(t[16:16 + 8 * B * q_len].view(torch.int64), t[at:].view(torch.float32).view(B, cols), t[:8].view(torch.int32)) for t in sides]
+            ent = [None, *views[0], None, sides, views[1], torch.cuda.Event()]
+        _, st_ids, st_kpos, st_past, out, sides, (h_ids, h_kpos, h_past), copied = ent
+        if ids.device.type == "cpu" and position_ids.device.type == "cpu":
+            # from the host in one copy: sums, conversions and fills on the device were eight launches of 5 us of host time each, the uploads two waits
+            copied.synchronize()                          # (the previous upload has left the pinned block)
+            h_ids.copy_(ids)
+            h_kpos[:, :kv_len].copy_(position_ids)        # int64 -> fp32 on the fly
+            h_past[0] = past_len
+            if mode == 2:
+                h_past[1] = arena.tail_base
+            sides[0].copy_(sides[1], non_blocking=True)
+            copied.record()
+        else:
+            st_ids.copy_(ids)
+            st_kpos[:, :kv_len].copy_(position_ids)
+            st_past[0:1].fill_(past_len)
+            if mode == 2:
+                st_past[1:2].fill_(arena.tail_base)
         if fresh:
             self._forward_skinny(st_ids, st_kpos, st_past, arena, B, q_len, past_len, last_token_only, num_layers)
             torch.cuda.synchronize()
