@@ -5,7 +5,8 @@
 // Tiling: workgroup = 4 waves in a 2 x 2 grid, a wave owns TM x TN result tiles of 16 x 16, so the workgroup covers
 // (32 TM) x (32 TN) of Y.  Per stage of two 32-element k-steps the A and B panels go global -> registers -> LDS (the next stage's
 // loads are in flight while this stage's MFMAs run); waves read their operand fragments from LDS with one 16-byte read per fragment (bf16).
-// Operands that can be read in 16-byte chunks take linear_dma_kernel below instead (large plain launches in bf16 pb_linear_tiles.hip); odd sizes
+// Operands that can be read in 16-byte chunks take linear_dma_kernel below instead (large plain launches in bf16 pb_linear_tiles.hip, those of few tiles
+// pb_linear_waves.hip); odd sizes
 // and scaled rows this one.
 #include <type_traits>
 
@@ -636,6 +637,9 @@ int dispatch_dma(const pcb_linear_args& a, int rows, hipStream_t stream) {
         // 44 / 76 / 47, 600 x 2048, K = 2048 79 / 146 / 68, 130 x 1024, K = 1024 25 / 75 / 17.
         const int64_t extra = a.n_groups / 2;                        // (groups: part tiles)
         auto rounds = [&](int bm, int bn) { return (batch * (pcb_ceil_div(a.M, bm) + extra) * pcb_ceil_div(a.N, bn) + 255) / 256; };
+        // (32 x 32 tiles, three to a CU, up to 768 of them: 600 x 1024, K = 1024 25.8 -> 21.5, 300 x 1024 18.1 -> 16.3, 200 x 2564 26.5 -> 22.1, 600 x 512,
+        // K = 512 10.3 -> 9.6; 600 x 2564 (1539) 42.9, 45.1 so.  What is below a round of the chip or deep is with pb_linear_waves.hip.)
+        if (EPI != PCB_EPI_SILU_MUL && a.n_groups == 0 && batch * pcb_ceil_div(a.M, 32) * pcb_ceil_div(a.N, 32) <= 768) return launch_dma<E, EPI, 1, 1, 3>(a, stream);
         const float large = 3.8f * rounds(128, 32 * TNW), mid = rounds(64, 16 * TNW), small = 0.575f * rounds(32, 16 * TNW);
         if (rows > 64 && large <= mid && large <= small) return launch_dma<E, EPI, 4, TNW, 2>(a, stream);
         return rows > 32 && mid <= small ? launch_dma<E, EPI, 2, TNW / 2, 3>(a, stream) : launch_dma<E, EPI, 1, TNW / 2, 3>(a, stream);
@@ -736,6 +740,7 @@ int dispatch(const pcb_linear_args& a, hipStream_t stream) {
         return pcb_check_launch("linear_skinny_kernel");
     }
     if (dma_ok(a)) {
+        if (pcb_linear_waves_fits(a)) return pcb_linear_waves(a, stream);
         // Plain launches whose 128 x 128 tiles reach more than half of the 256 CUs go to the whole-CU tiles of pb_linear_tiles.hip (row strides
         // such that a tile's rows lie within 32-bit offsets); below, the smaller tiles here give more CUs work: 300 x 2048, K = 2048 (48 tiles)
         // 13.1 us here, 14.9 there, 1024 x 1024 x 1024 (64) 8.3 / 9.6, 1024 x 2048, K = 2048 (128) 15.9 / 16.2, 300 x 8192 (192) 21.4 / 17.4.

@@ -5,3 +5,7 @@
 #include "pb_common.h"
 
 int pcb_linear_tiles(const pcb_linear_args& a, hipStream_t stream);
+// ... and those over some tens or hundreds of rows (pb_linear_waves.hip): which launches whose rows can be read in 16-byte chunks it is the better for
+int64_t pcb_linear_waves_tiles(const pcb_linear_args& a);
+bool pcb_linear_waves_fits(const pcb_linear_args& a);
+int pcb_linear_waves(const pcb_linear_args& a, hipStream_t stream);
