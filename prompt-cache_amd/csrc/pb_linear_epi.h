@@ -27,6 +27,11 @@ __device__ __forceinline__ float gate_act(int act, float v) {
     return act == PCB_ACT_RELU ? fmaxf(v, 0.0f) : s;
 }
 
+// Sigmoid and silu of a result that is rounded to bf16: v_exp_f32 and v_rcp_f32, four instructions where expf and a division are some forty (256 of them
+// a thread are 20 us at the end of a 256 x 256 tile).  Good to 2^-19 for |v| <= 20, a thousandth of the rounding's half place; 0 and 1, and what is no
+// number, as above.
+__device__ __forceinline__ float rounded_sigmoid(float v) { return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(v * -1.44269504f)); }
+
 // columns that pass through act / act2 of a plain store: the split-off parts are stored as they are
 __device__ __forceinline__ int act_end(const pcb_linear_args& a) {
     return a.split_n > 0 ? a.split_n : (a.split_n3 > 0 ? a.split_n3 : a.N);
