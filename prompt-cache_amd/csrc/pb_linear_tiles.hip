@@ -1,11 +1,11 @@
-// pb_linear over many rows in bf16: mfma_f32_32x32x16_bf16, four waves (2 x 2) in tiles of 128 x 128, 128 x 256 or 256 x 256 with a whole CU's
+// pb_linear over many rows in bf16: mfma_f32_32x32x16_bf16, four waves (2 x 2) in tiles of 128 or 256 rows x 128, 192 or 256 columns with a whole CU's
 // LDS for their ring, main loop and staging order in mfma_tile_loop.h.
 //
 // What bounds it: at one round of 128 x 128 tiles LDS bandwidth (a wave of 64 x 64 reads as many bytes as its MFMAs take cycles) and the
 // barrier of every K-step, at the larger tiles power.  Against linear_dma_kernel (pb_linear.hip: 16 x 16 MFMAs, two or three images, two
 // workgroups to a CU), us, 2048 rows: 2048 x 2048 29.9 -> 19.9 (0.87 PFLOP/s), K = 8192 93.5 -> 72, 2560 columns 39.8 -> 31, 8192 columns
 // 90.5 -> 65.6 (1.05 PFLOP/s; the gated pair 79.3 -> 60.7); 4096 x 4096 x 4096 161 -> 112 (1.23 PFLOP/s).  With a sigmoid on half of the columns: 5136
-// columns 73.7 -> 60.5, 10272 133 -> 117.5 since results that are rounded to bf16 take the machine's exponential and reciprocal.
+// columns 73.7 -> 56, 10272 133 -> 113 since results that are rounded to bf16 take the machine's exponential and reciprocal.
 #include "mfma_tile_loop.h"
 #include "pb_linear_epi.h"
 #include "pb_linear_tiles.h"
@@ -251,7 +251,8 @@ __global__ __launch_bounds__(256, 1) void linear_tile_kernel(const pcb_linear_ar
     constexpr bool TWO = EPI == PCB_EPI_SILU_MUL;
     using L = mfma_tile::Loop<MT, NT, S, 1>;
     constexpr int BM = L::BM, BN = TWO ? L::BN / 2 : L::BN, NI = L::NI;   // BN: result columns
-    __shared__ __attribute__((aligned(16))) char lds[S * L::kStage];
+    constexpr int P = 32 * MT * 256;                                 // bytes of a patch (see below)
+    __shared__ __attribute__((aligned(16))) char lds[S * L::kStage > 4 * P ? S * L::kStage : 4 * P];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
     int mi, ni;
@@ -292,7 +293,7 @@ __global__ __launch_bounds__(256, 1) void linear_tile_kernel(const pcb_linear_ar
     // Results: 64 accumulator columns of a wave go into an LDS patch of its own (16-byte quad c of row r at c ^ (r & 15)), so that neighbouring
     // lanes store neighbouring columns.  Gated: 32 gate columns and the matching 32 of the other half side by side.
     __syncthreads();                                                 // (the images are read out)
-    constexpr int P = 32 * MT * 256, PARTS = NT / 2, ROOM = 4 * P * PARTS <= S * L::kStage ? PARTS : 1;   // patches that fit at a time
+    constexpr int PARTS = (NT + 1) / 2, ROOM = 4 * P * PARTS <= S * L::kStage ? PARTS : 1;   // patches that fit at a time
     char* patch = lds + wave * (P * ROOM);
     constexpr int LPR = TWO ? 8 : 16, RPI = 64 / LPR;                // lanes on a row, rows an access covers
     const int fr = lane & 31, fh = lane >> 5, pr = lane / LPR, pc = lane % LPR;
@@ -308,12 +309,15 @@ __global__ __launch_bounds__(256, 1) void linear_tile_kernel(const pcb_linear_ar
             for (int h = 0; h < 2; ++h)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const f16v& c = acc[i][TWO ? j + h * (NT / 2) : 2 * j + h];
+                    constexpr bool ODD = NT % 2 != 0 && j == PARTS - 1;          // (the last half patch of an odd number of blocks)
+                    if (ODD && h == 1) continue;
+                    const f16v& c = acc[i][ODD ? NT - 1 : TWO ? j + h * (NT / 2) : 2 * j + h];
                     *(f4*)(to + (32 * i + fr) * 256 + ((8 * h + 2 * q + fh) ^ (fr & 15)) * 16) = f4{c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]};
                 }
     };
     auto store = [&](int j, char* from) {
         const int n0 = n_lo + (TWO ? wn * 16 * NT + 32 * j : wn * 32 * NT + 64 * j);
+        if (NT % 2 != 0 && j == PARTS - 1 && pc >= 8) return;
         if (n0 < N) store_columns<EPI, 32 * MT / RPI>(a, from, pr, pc, n0, n0 + 4 * pc, m_lo + wm * 32 * MT + pr);
     };
     using First = std::integral_constant<int, 0>;
@@ -346,16 +350,24 @@ int launch(const pcb_linear_args& a, hipStream_t stream) {
 template <int EPI>
 int dispatch(const pcb_linear_args& a, hipStream_t stream) {
     // The tile whose whole rounds of the 256 CUs cost least.  A round, in us, one workgroup per CU, from K = 64 .. 8192 on a full chip:
-    // 128 x 128 4.5 + 0.53 per K-step, 128 x 256 7 + 0.67, 256 x 256 10 + 1.03 (K = 2048: 21, 28, 43).  2048 rows, K = 2048, the three and
-    // what the rule took: N = 2048 20.0 / 28.0 / 42.7 -> 20.0, 2560 35.0 / 33.3 / 45.7 -> 31, 5136 54 / 59 / 53 -> 50, 8192 84 / 75 / 67 -> 66,
-    // 10272 112 / 95 / 99 -> 97; 6000 rows, K = 512, N = 2048 21.2 / 24.9 / 22.3 -> 21.9.
+    // 128 x 128 4.5 + 0.53 per K-step, 128 x 192 5.6 + 0.645, 128 x 256 7 + 0.67, 256 x 192 8 + 0.95, 256 x 256 10 + 1.03 (K = 2048: 21, 26, 28, 38, 43).
+    // 2048 rows, K = 2048, 128 x 128 / 128 x 256 / 256 x 256 and what the rule took: N = 2048 20.0 / 28.0 / 42.7 -> 20.0, 8192 84 / 75 / 67 -> 66;
+    // 6000 rows, K = 512, N = 2048 21.2 / 24.9 / 22.3 -> 21.9.  Without and with the two of 192 columns: 2048 rows, N = 2560 31.7 / 29.9, 5136 55.3 / 49.7,
+    // 10272 106 / 102; 1500 x 3072 31.3 / 25.4; 4096 x 2560 52.0 / 45.4; 2400 x 2048, K = 8192 102 / 91.  (The gated unit's halves are whole pairs of
+    // 32-column blocks: not 192.)
     constexpr int C = EPI == PCB_EPI_SILU_MUL ? 2 : 1;               // weight rows per result column
     auto rounds = [&](int bm, int bn) { return ((int64_t)pcb_ceil_div(a.M, bm) * pcb_ceil_div(C * a.N, bn) + 255) / 256; };
     const float steps = (float)pcb_ceil_div(a.K, 64);
     const float square = rounds(128, 128) * (4.5f + 0.53f * steps), wide = rounds(128, 256) * (7.0f + 0.67f * steps),
                 tall = rounds(256, 256) * (10.0f + 1.03f * steps);
-    if (tall <= wide && tall <= square) return launch<EPI, 4, 4, 2>(a, stream);
-    return wide <= square ? launch<EPI, 2, 4, 3>(a, stream) : launch<EPI, 2, 2, 3>(a, stream);
+    const float least = tall <= wide && tall <= square ? tall : wide <= square ? wide : square;
+    if constexpr (C == 1) {
+        const float wide192 = rounds(128, 192) * (5.6f + 0.645f * steps), tall192 = rounds(256, 192) * (8.0f + 0.95f * steps);
+        if (tall192 < least && tall192 <= wide192) return launch<EPI, 4, 3, 2>(a, stream);
+        if (wide192 < least) return launch<EPI, 2, 3, 3>(a, stream);
+    }
+    if (tall == least) return launch<EPI, 4, 4, 2>(a, stream);
+    return wide == least ? launch<EPI, 2, 4, 3>(a, stream) : launch<EPI, 2, 2, 3>(a, stream);
 }
 
 }  // namespace
