@@ -7,12 +7,13 @@
 //            which is what the mixing's product (weights in fp32, v_mfma_f32_16x16x4_f32) wants as an operand: nothing is moved in between
 //   softmax  the mixed scores come out as lane = lane head, registers = neighbouring keys; the four waves agree on the maxima through LDS
 //   values   weights as a hi + lo pair of bf16 through LDS, values by transposed reads of the key tile
-// The next keys are requested into registers before a tile is worked on.
+// The next keys are requested into registers before a tile is worked on and pass into the second of two tiles in LDS beside the exchange of the maxima, so
+// that a tile's values and the next one's scores have no barrier between them.
 //
-// What bounds it: a tile's chain (scores, maxima, weights, values, four barriers) at two waves per SIMD: matrix cores busy 26 %, vector unit 31 %, LDS 24 %
+// What bounds it: a tile's chain (scores, maxima, weights, values, three barriers) at two waves per SIMD: matrix cores busy 27 %, vector unit 33 %, LDS 25 %
 // of the time; LDS bank conflicts, 23 % before the spreads below, are 1 %.  us (scores into a band of memory and values behind it, then here), window 1024:
-// 2048 rows of 16 heads 110.6 and 71.7, 8 heads 72.7 and 43.1, 4 heads 60.7 and 32.5; 6 x 300 rows of 16 heads 50.8 and 30.1, 100 rows 30.4 and 18.2, 9 rows
-// 29.5 and 15.0; 200 rows of 16 heads behind 1000 keys 70.7 and 34.
+// 2048 rows of 16 heads 110.6 and 68.5, 8 heads 72.7 and 41.6, 4 heads 60.7 and 31.6; 6 x 300 rows of 16 heads 50.8 and 28.7, 100 rows 30.4 and 17.4, 9 rows
+// 29.5 and 14.3; 200 rows of 16 heads behind 1000 keys 70.7 and 32.  One tile in LDS and four barriers: 16 heads 72.4, 8 heads 41.8, 4 heads 32.4.
 #include <type_traits>
 
 #include "pb_attn_common.h"
@@ -37,9 +38,10 @@ __global__ __launch_bounds__(256 * NU, 2) void talk_prompt_kernel(pcb_attn_talk_
     constexpr int H = 4 * HKV, UQ = 16 / HKV, WQ = NU * UQ;      // queries of a unit, of a workgroup
     constexpr int RP = 16 * NU, NCH = KT * HKV / RP;              // key rows staged at a time; 16-byte chunks of a key tile per thread
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    bf16_t* const Ks = reinterpret_cast<bf16_t*>(lds);           // [HKV][KT][D]
+    bf16_t* Ks = reinterpret_cast<bf16_t*>(lds);                 // [HKV][KT][D], two of them
+    bf16_t* Kn = Ks + HKV * KT * D;                              // the next tile's
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), sub = wave & 3, unit = wave >> 2, g = lane >> 4, l15 = lane & 15;
-    bf16_t* const Ps = Ks + HKV * KT * D + unit * 2 * 64 * KT;   // the unit's weights: [hi, lo][4][16 rows][KT]
+    bf16_t* const Ps = Kn + HKV * KT * D + unit * 2 * 64 * KT;   // the unit's weights: [hi, lo][4][16 rows][KT]
     const int32_t* const t = tiles + 4 * (gridDim.x - 1 - blockIdx.x);        // (later rows see more keys: they start first)
     const int w_rows = t[2] - WQ * (int)blockIdx.y, w_first = t[1] + WQ * (int)blockIdx.y;
     if (w_rows <= 0) return;                                     // (uniform over the workgroup)
@@ -97,13 +99,16 @@ __global__ __launch_bounds__(256 * NU, 2) void talk_prompt_kernel(pcb_attn_talk_
 #pragma unroll
     for (int n = 0; n < 8; ++n) acc[n] = f4{0.f, 0.f, 0.f, 0.f};
 
-    for (int j0 = j_lo; j0 < j_hi; j0 += KT) {
+    auto stage = [&](bf16_t* K) {
 #pragma unroll
         for (int u = 0; u < NCH; ++u) {
             const int j = (tid >> 4) + RP * (u % (KT / RP));
-            *reinterpret_cast<u32x4*>(Ks + ((u / (KT / RP)) * KT + j) * D + 8 * ((tid & 15) ^ key_spread(j & 15))) = next[u];
+            *reinterpret_cast<u32x4*>(K + ((u / (KT / RP)) * KT + j) * D + 8 * ((tid & 15) ^ key_spread(j & 15))) = next[u];
         }
-        __syncthreads();
+    };
+    stage(Ks);
+    __syncthreads();
+    for (int j0 = j_lo; j0 < j_hi; j0 += KT) {
         if (j0 + KT < j_hi) fetch(j0 + KT);
 
         const int js = j0 + 16 * sub;                            // this wave's keys
@@ -152,8 +157,10 @@ __global__ __launch_bounds__(256 * NU, 2) void talk_prompt_kernel(pcb_attn_talk_
         auto place = [&](int b, int r, int c, int w) {           // chunk c (of the wave's 32 keys) of row r in block b, the half that wave w writes
             return Ps + (b * 16 + r) * KT + 8 * ((4 * (w >> 1) + c) ^ row_spread(b, r)) + 4 * ((w & 1) ^ (b >> 1));
         };
+        __syncthreads();                                         // (the tile before is read out: its weights and its keys)
 #pragma unroll
         for (int x = 0; x < 2; ++x) *reinterpret_cast<float2*>(place(sub, l15, x, g)) = make_float2(top[2 * x], top[2 * x + 1]);
+        if (j0 + KT < j_hi) stage(Kn);
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < 4; ++k)
@@ -211,8 +218,10 @@ __global__ __launch_bounds__(256 * NU, 2) void talk_prompt_kernel(pcb_attn_talk_
                 acc[n] = mma(pl, fv, acc[n]);
             }
         }
-        __syncthreads();
+        bf16_t* const k = Ks;
+        Ks = Kn, Kn = k;
     }
+    __syncthreads();
 
     // denominators: over the lane groups and the four waves
     float* const sums = reinterpret_cast<float*>(Ps);
@@ -284,7 +293,7 @@ int pcb_talk_prompt(const pcb_attn_talk_args& a, hipStream_t stream) {
     const int n_tiles = a.tiles64 ? a.n_tiles64 : a.n_tiles, tile_rows = a.tiles64 ? 64 : 16;
     const int n_rows = 16 * a.n_tiles;                           // (what the scratch is laid out for)
     auto go = [&](auto hkv, auto nu) {
-        constexpr int HKV = decltype(hkv)::value, NU = decltype(nu)::value, LDS = (HKV * KT * D + NU * 2 * 64 * KT) * 2, WQ = NU * 16 / HKV;
+        constexpr int HKV = decltype(hkv)::value, NU = decltype(nu)::value, LDS = 2 * (2 * HKV * KT * D + NU * 2 * 64 * KT), WQ = NU * 16 / HKV;
         static const hipError_t raised =
             hipFuncSetAttribute(reinterpret_cast<const void*>(talk_prompt_kernel<HKV, NU>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
         (void)raised;
