@@ -44,7 +44,8 @@ struct __attribute__((packed, aligned(4))) Floats4 {
 __device__ __forceinline__ double up(double v, int o) { return __shfl_up(v, o, 64); }
 
 // one wave: the gates of the segment's n tokens, lane l the NT tokens from l NT on.  b[u] = li - F, F[u] = the running sum, 64 bits; tokens past n
-// have b = -infinity.  (A log forget gate below -1e8 counts as -1e8: what it forgets is gone either way, and sums and differences stay finite.)
+// have b = -infinity, as those with a closed input gate (li = -infinity): nothing of them is taken, a segment of such tokens alone leaves S' = n' = 0 and
+// m' = -infinity.  (A log forget gate below -1e8 counts as -1e8: what it forgets is gone either way, and sums and differences stay finite.)
 template <typename E, int NT>
 __device__ __forceinline__ void segment_gates(const pcb_mlstm_args& a, int64_t row0, int n, int h, int lane, double (&b)[NT], double (&F)[NT]) {
     const E* gi = (const E*)a.gi + row0 * a.ldgi + h;
@@ -99,7 +100,7 @@ __global__ __launch_bounds__(256) void mlstm_local_kernel(pcb_mlstm_args a, floa
             top = x > top ? x : top;
         }
 #pragma unroll
-        for (int u = 0; u < NT; ++u) ws[lane * NT + u] = lane * NT + u < n ? expf((float)(b[u] - top)) : 0.0f;
+        for (int u = 0; u < NT; ++u) ws[lane * NT + u] = b[u] == -__builtin_inf() ? 0.0f : expf((float)(b[u] - top));      // (top may be -infinity too)
         if (lane == 63) {                                                  // (its running sum is the whole segment's)
             f_sum[(int64_t)blockIdx.x * a.H + h] = (float)F[NT - 1];
             st[rec - 1] = (float)(F[NT - 1] + top);
@@ -272,7 +273,7 @@ __global__ __launch_bounds__(256 * NT, NT > 1 ? 1 : sizeof(E) == 2 ? 3 : 2) void
             M = b[u] > M ? b[u] : M;
             const float hi = (float)b[u], Hi = (float)M;
             bh[t] = hi;
-            bl[t] = t < n ? (float)(b[u] - (double)hi) : 0.0f;
+            bl[t] = b[u] == -__builtin_inf() ? 0.0f : (float)(b[u] - (double)hi);
             Mh[t] = Hi;
             Ml[t] = (float)(M - (double)Hi);
             em[t] = expf(-(float)(F[u] + M));

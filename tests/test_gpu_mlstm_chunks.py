@@ -106,3 +106,49 @@ def test_steps_of_wide_heads(D, Dv, dtype):
     assert B.mlstm_step_fits(D, Dv, N, cols[2])
     B.mlstm_step(cols, N, reqs, 3, state, H, D, Dv, D ** -0.5, 5.0, None, None, 0, out, eps)
     assert rel(state, ref) < 1e-6 and rel(out, want) < (1e-5 if dtype == torch.float32 else 2.0 ** -8)
+
+
+def layer(H, D, Dv, n, dtype, shift=3.0):
+    """Columns of n random tokens, their strides' row length, gate and gain."""
+    N = -(-(2 * H * D + 2 * H * Dv + 2 * H) // 8) * 8
+    P = rnd(n, N, seed=1, dtype=dtype)
+    P[:, 2 * H * D + H * Dv + H:2 * H * D + H * Dv + 2 * H] += shift
+    g0 = 2 * H * D + H * Dv + 2 * H
+    return (P, P[:, H * D:], P[:, 2 * H * D:], P[:, 2 * H * D + H * Dv:], P[:, 2 * H * D + H * Dv + H:]), N, P[:, g0:g0 + H * Dv], 1 + 0.1 * rnd(H * Dv, seed=2)
+
+
+def one_prompt(cols, N, H, D, Dv, n, seg, state, slot, pos0, gain, gate):
+    from promptcache_amd import _blocks as B
+    rec, starts = B.mlstm_state_floats(H, D, Dv), range(0, n, seg)
+    ns, nan = len(starts), lambda *s: torch.full(s, float("nan"), device=DEV)
+    out = torch.zeros(n, H * Dv, device=DEV, dtype=cols[0].dtype)
+    B.mlstm_prompt(cols, N, i32([(i, 0, min(seg, n - q), q) for i, q in enumerate(starts)]), ns, i32([(slot, pos0, 0, ns)]), 1, seg,
+                   i32([-1] * (ns - 1) + [slot]), state, H, D, Dv, D ** -0.5, 0.0, gain, gate, N, out, 1e-6, nan(ns, rec), nan(ns, H), nan(ns, rec))
+    return out
+
+
+# (bounds as above)
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 2e-5), (torch.bfloat16, 2.0 ** -8)])
+@pytest.mark.parametrize("closed", ["one token", "the first token", "a whole segment", "a last segment of one token", "every token", "every other token"])
+@pytest.mark.parametrize("pos0", [0, 5])
+def test_closed_input_gates(closed, pos0, dtype, tol):
+    from promptcache_amd import _blocks as B
+    H, D, Dv, seg = 2, 64, 40, 32
+    n = 2 * seg + 1
+    cols, N, gate, gain = layer(H, D, Dv, n, dtype)
+    shut = {"one token": [5], "the first token": [0], "a whole segment": range(seg, 2 * seg), "a last segment of one token": [2 * seg], "every token": range(n),
+            "every other token": range(1, n, 2)}[closed]
+    cols[3][list(shut), :H] = float("-inf")
+    state = rnd(2, B.mlstm_state_floats(H, D, Dv), seed=3)
+    state.view(2, H, -1)[..., -1] = 0.7
+    f = lambda t: t.detach().to("cpu", F64)
+    s6, x = f(state[1]).view(H, -1), [f(c) for c in cols]
+    st = (s6[:, :D * Dv].reshape(H, D, Dv), s6[:, D * Dv:-1], s6[:, -1]) if pos0 else None
+    o, (S, nv, m) = O.matrix_memory(x[0][:, :H * D].view(n, H, D) * D ** -0.5, x[1][:, :H * D].view(n, H, D), x[2][:, :H * Dv].view(n, H, Dv), x[3][:, :H],
+                                    torch.nn.functional.logsigmoid(x[4][:, :H]), st)
+    want = O.unit_rms(o, 1e-6).reshape(n, H * Dv) * f(gain) * f(gate)
+    got = f(one_prompt(cols, N, H, D, Dv, n, seg, state, 1, pos0, gain, gate))
+    near = lambda a, b, t: bool(torch.isfinite(a).all()) and float((a - b).norm()) <= t * float(b.norm())      # (from nothing, no token: all zeros)
+    after = f(state[1]).view(H, -1)
+    assert near(got, want, tol)
+    assert near(after[:, :D * Dv].reshape(H, D, Dv), S, 2e-5) and near(after[:, D * Dv:-1], nv, 2e-5) and torch.allclose(after[:, -1], m, rtol=1e-5, atol=1e-5)
