@@ -211,6 +211,39 @@ __global__ __launch_bounds__(256) void mlstm_starts_kernel(const float* __restri
         if (e0 + 256 * u < elems) st[e0 + 256 * u] = v[u];
 }
 
+// A row's last tile holds tokens behind it: of weight 0, but 0 times infinity (or times what is no number) is none.  Such values are taken out of the tile,
+// and what they belong to -- their column, from their token's own row on -- is set to NaN.  v: the lane's tokens `first` .. + 3 of the tile, eight columns.
+__device__ __forceinline__ bool finite(float x) { return fabsf(x) < __builtin_inff(); }
+__device__ __forceinline__ void clear(Frag<bf16_t>& f, int e) { f.v[e >> 1] &= e & 1 ? 0xffffu : 0xffff0000u; }
+__device__ __forceinline__ void clear(Frag<float>& f, int e) { f.v[e] = 0.0f; }
+template <typename E>
+__device__ __forceinline__ bool all_finite(const Frag<E> (&v)[4]) {
+    float z = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) z = __builtin_fmaf(at8(v[r], c), 0.0f, z);
+    return z == 0.0f;
+}
+template <typename E>
+__device__ __forceinline__ void keep_behind(Frag<E> (&v)[4], f4 (&acc)[8], int first) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        int j = 16;
+#pragma unroll
+        for (int r = 3; r >= 0; --r)
+            if (!finite(at8(v[r], c))) {
+                j = first + r;
+                clear(v[r], c);
+            }
+        j = min(j, __shfl_xor(j, 16, 64));
+        j = min(j, __shfl_xor(j, 32, 64));
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (first + e >= j) acc[c][e] = __builtin_nanf("");
+    }
+}
+
 // ---- 3. the rows ----------------------------------------------------------------------------------------------------------------------------------
 // A wave owns 16 rows.  The norm's and the gate's part is that of pcb_gated_norm with a norm per head.
 template <typename E, int NT>
@@ -332,6 +365,7 @@ __global__ __launch_bounds__(256 * NT, NT > 1 ? 1 : sizeof(E) == 2 ? 3 : 2) void
     }
     float ps = 0.0f;
     for (int j0 = 0; j0 <= t0; j0 += 16) {
+        if (j0 == t0 && __any(!all_finite(fv))) keep_behind(fv, acc, 4 * group);
         f4 s = f4{0.f, 0.f, 0.f, 0.f};
         Frag<E> v[4];
 #pragma unroll

@@ -152,3 +152,19 @@ def test_closed_input_gates(closed, pos0, dtype, tol):
     after = f(state[1]).view(H, -1)
     assert near(got, want, tol)
     assert near(after[:, :D * Dv].reshape(H, D, Dv), S, 2e-5) and near(after[:, D * Dv:-1], nv, 2e-5) and torch.allclose(after[:, -1], m, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("at", [0, 7, 15, 16, 37, 49])
+def test_a_value_that_is_no_number_leaves_earlier_rows_alone(at, bad, dtype):
+    from promptcache_amd import _blocks as B
+    H, D, Dv, n = 2, 64, 72, 50
+    cols, N, gate, gain = layer(H, D, Dv, n, dtype)
+    rec = B.mlstm_state_floats(H, D, Dv)
+    clean = one_prompt(cols, N, H, D, Dv, n, 64, torch.zeros(2, rec, device=DEV), 1, 0, gain, gate)
+    cols[2][at, Dv + 3] = bad                                    # (head 1)
+    got = one_prompt(cols, N, H, D, Dv, n, 64, torch.zeros(2, rec, device=DEV), 1, 0, gain, gate)
+    # the rows in front of it and the other head: to the rounding of sums in another order
+    assert bool(torch.isfinite(got[:at]).all()) and bool(torch.isfinite(got[:, :Dv]).all()) and not bool(torch.isfinite(got[at:, Dv + 3]).any())
+    assert rel(got[:, :Dv], clean[:, :Dv]) == 0 and (at == 0 or rel(got[:at], clean[:at]) < (1e-6 if dtype == torch.float32 else 2.0 ** -9))
