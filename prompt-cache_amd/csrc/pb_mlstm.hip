@@ -108,7 +108,9 @@ __global__ __launch_bounds__(256) void mlstm_kernel(pcb_mlstm_args a) {
             const int t = blk * TB + tt, pb = t & 1;
             const float li = gs[b][tt][0], lf = gs[b][tt][1];
             const float m_new = fmaxf(lf + m, li);
-            const float keep = expf(lf + m - m_new), take = expf(li - m_new);      // (m = -inf: keep = 0)
+            // (m = -inf: keep = 0; a segment that starts from nothing with closed input gates stays at nothing: m_new = -inf, both 0)
+            const float at = m_new == -__builtin_inff() ? 0.0f : m_new;
+            const float keep = expf(lf + m - at), take = expf(li - at);
             m = m_new;
             f_sum += lf;
             float acc = 0.0f, accn = 0.0f;
@@ -185,7 +187,8 @@ __global__ __launch_bounds__(256) void mlstm_chain_kernel(const float* __restric
         if (g + 1 == seg0 + n_seg) break;
         const float F = f_sum[(int64_t)g * H + h], ml = lc[elems];
         const float m_new = fmaxf(F + mm, ml);
-        const float keep = expf(F + mm - m_new), take = expf(ml - m_new);
+        const float at = m_new == -__builtin_inff() ? 0.0f : m_new;      // (everything forgotten, nothing taken)
+        const float keep = expf(F + mm - at), take = expf(ml - at);
 #pragma unroll
         for (int u = 0; u < 4; ++u)
             if (e0 + 256 * u < elems) v[u] = keep * v[u] + take * lc[e0 + 256 * u];

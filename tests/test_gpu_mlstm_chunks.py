@@ -168,3 +168,29 @@ def test_a_value_that_is_no_number_leaves_earlier_rows_alone(at, bad, dtype):
     # the rows in front of it and the other head: to the rounding of sums in another order
     assert bool(torch.isfinite(got[:at]).all()) and bool(torch.isfinite(got[:, :Dv]).all()) and not bool(torch.isfinite(got[at:, Dv + 3]).any())
     assert rel(got[:, :Dv], clean[:, :Dv]) == 0 and (at == 0 or rel(got[:at], clean[:at]) < (1e-6 if dtype == torch.float32 else 2.0 ** -9))
+
+
+@pytest.mark.parametrize("shut", [[0], [40], [32, 33, 50], range(32, 64), range(65)])
+@pytest.mark.parametrize("pos0", [0, 5])
+def test_closed_input_gates_token_by_token(shut, pos0):
+    """The segments of sizes that the matrix cores' kernels do not take: from nothing, chained, each from its start."""
+    from promptcache_amd import _blocks as B
+    H, D, Dv, seg, n = 2, 136, 40, 32, 65
+    cols, N, _, _ = layer(H, D, Dv, n, torch.float32)
+    cols[3][list(shut), :H] = float("-inf")
+    rec, f = B.mlstm_state_floats(H, D, Dv), lambda t: t.detach().to("cpu", F64)
+    state = rnd(2, rec, seed=3)
+    state.view(2, H, -1)[..., -1] = 0.7
+    s6, x = f(state[1]).view(H, -1), [f(c) for c in cols]
+    st = (s6[:, :D * Dv].reshape(H, D, Dv), s6[:, D * Dv:-1], s6[:, -1]) if pos0 else None
+    want, (S, nv, m) = O.matrix_memory(x[0][:, :H * D].view(n, H, D) * D ** -0.5, x[1][:, :H * D].view(n, H, D), x[2][:, :H * Dv].view(n, H, Dv), x[3][:, :H],
+                                       torch.nn.functional.logsigmoid(x[4][:, :H]), st)
+    local, start, fsum, out = torch.empty(3, rec, device=DEV), torch.empty(3, rec, device=DEV), torch.empty(3, H, device=DEV), torch.zeros(n, H * Dv, device=DEV)
+    tail = (H, D, Dv, D ** -0.5, 0.0)
+    B.mlstm(*cols, N, i32([(g, 0, min(seg, n - g * seg), g * seg) for g in range(3)]), 3, local, *tail, None, from_nothing=True, log_f_sum=fsum)
+    B.mlstm_chain(local, fsum, start, state, i32([(1, pos0, 0, 3)]), 1, H, D, Dv)
+    B.mlstm(*cols, N, i32([(g, 1, min(seg, n - g * seg), g * seg) for g in range(3)]), 3, start, *tail, out, end_slots=i32([-1, -1, 1]), end_state=state)
+    near = lambda a, b: bool(torch.isfinite(a).all()) and float((a - b).norm()) <= 2e-5 * float(b.norm())
+    after = f(state[1]).view(H, -1)
+    assert near(f(out), want.reshape(n, H * Dv)) and near(after[:, :D * Dv].reshape(H, D, Dv), S) and near(after[:, D * Dv:-1], nv)
+    assert torch.allclose(after[:, -1], m, rtol=1e-5, atol=1e-5)
