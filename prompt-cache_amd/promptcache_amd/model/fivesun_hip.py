@@ -71,9 +71,7 @@ def rotary_frequencies(base: float, dims: int, factor: float = 1.0, original: fl
 class FivesunHIP(SlotModel):
     GRAPH_MAX_ROWS = 64
     # Tokens of a segment of the mLSTM layers.  Where all of them fit the matrix cores' kernels (_mlstm_fits), a step that brings a request more than
-    # FEW_TOKENS runs them in segments, else one that brings more than SEGMENT; the others go token by token.  us, token by token / in segments, 16
-    # heads of 128, one request and eight: 8 tokens 23.1 / 24.3 and 23.9 / 30.6, 16 30.8 / 24.5 and 32.1 / 30.8, 64 78.9 / 32.7 and 81.6 / 42.3.
-    FEW_TOKENS = 12
+    # _few_tokens() runs them in segments, else one that brings more than SEGMENT; the others go token by token.
     SEGMENT = int(os.environ.get("PC_FS_SEGMENT", "64"))
     MAX_SEGMENTS = 128      # (segments grow beyond SEGMENT tokens rather than exceed this many per request)
     PROMPT_ROWS = int(os.environ.get("PC_FS_PROMPT_ROWS", "16"))   # a request that brings fewer tokens than this attends row by row (see _tiled)
@@ -173,6 +171,18 @@ class FivesunHIP(SlotModel):
         self._wide = any(ent["cfg"].kind == "attention" and ent["cfg"].dim > 256 for ent in self.layers)
         self._chunks = all(self._mlstm_fits(l) for l in shape.layers if l.kind == "mlstm")
         self._max_heads = max(l.heads for l in shape.layers)
+
+    @staticmethod
+    def _few_tokens(requests, heads, dim, vdim):
+        """Up to how many tokens a request (the longest of the step) the memory is faster token by token.  That costs a fixed time a token until its
+        workgroups (one per request, head and 64 value columns) are more than two a CU; segments cost the same for 2 as for 16 tokens, and in
+        proportion to requests x heads.  us, token by token / in segments, heads of 128: 16 of them 8 tokens 23.0 / 24.6, 10 25.7 / 24.6; 128 13 tokens
+        30.0 / 31.1, 16 33 / 31; 256 20 tokens 40 / 44, 24 44 / 44; 640 9 tokens 82 / 67 (bf16), 1280 13 157 / 166 (fp32); heads of 64: 16 of them 14 tokens
+        20.2 / 20.9, 16 22.0 / 20.9; 320 28 tokens 33 / 36 (fp32), 1024 32 tokens 52 / 62; 128 x 64, 288 of them 22 tokens 41 / 47."""
+        n = requests * heads
+        if dim <= 64:
+            return 15 + n // 20
+        return 14 if vdim > 64 and n > 256 else min(26, 8 + n // 16)
 
     def _mlstm_fits(self, l):
         """Whether an mLSTM layer's columns of the step's projection are what ``B.mlstm_prompt`` takes (16-byte pieces of up to 128 columns)."""
@@ -297,7 +307,9 @@ class FivesunHIP(SlotModel):
         seg_end = np.zeros(0, np.int32)
         seg = max(self.SEGMENT, -(-max(counts) // self.MAX_SEGMENTS))
         chunks = self._chunks and seg <= 256
-        if max(counts) > (self.FEW_TOKENS if chunks else self.SEGMENT) and any(l.kind == "mlstm" for l in self.config.layers):
+        few = [min(self.SEGMENT, self._few_tokens(len(counts), l.heads, l.dim, l.vdim) if chunks else self.SEGMENT)
+               for l in self.config.layers if l.kind == "mlstm"]
+        if few and max(counts) > max(few):
             sa, ch = [], []
             for b, (s, s0, c) in enumerate(zip(slots, starts, counts)):
                 ch.append((s, s0, len(sa), -(-c // seg)))

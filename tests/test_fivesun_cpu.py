@@ -347,3 +347,14 @@ def test_oracle_gated_sublayer_and_feed_forward():
     assert torch.allclose(O.gated_sublayer(x, lambda hh: O.dense_ff(hh, p, "m."), p, "l.", "2", 1e-5), want, atol=1e-12)
     z = torch.tensor([-1.0, 0.5, 2.0], dtype=F)
     assert torch.allclose(O.activation("gelu_tanh")(z), 0.5 * z * (1 + torch.tanh(math.sqrt(2 / math.pi) * (z + 0.044715 * z ** 3))))
+
+
+@pytest.mark.parametrize("requests,heads,dim,vdim,tokens,segments", [
+    # where one of the two ways through the matrix memory was measured to be the faster by 8 % or more
+    (1, 16, 128, 128, 8, False), (1, 16, 128, 128, 16, True), (8, 8, 128, 128, 8, False), (8, 16, 128, 128, 8, False), (8, 16, 128, 128, 24, True),
+    (32, 8, 128, 128, 16, False), (8, 32, 128, 128, 16, False), (8, 32, 128, 128, 32, True), (40, 16, 128, 128, 15, True), (80, 16, 128, 128, 11, False),
+    (24, 12, 128, 64, 22, False), (24, 12, 128, 64, 40, True), (1, 16, 64, 64, 10, False), (1, 16, 64, 64, 20, True), (32, 16, 64, 64, 24, False),
+    (40, 8, 64, 64, 28, False), (32, 32, 64, 64, 32, False), (32, 4, 64, 64, 32, True)])
+def test_few_tokens_go_through_the_matrix_memory_one_by_one(requests, heads, dim, vdim, tokens, segments):
+    from promptcache_amd.model.fivesun_hip import FivesunHIP
+    assert (tokens > FivesunHIP._few_tokens(requests, heads, dim, vdim)) == segments
