@@ -181,8 +181,10 @@ class FivesunHIP(SlotModel):
         20.2 / 20.9, 16 22.0 / 20.9; 320 28 tokens 33 / 36 (fp32), 1024 32 tokens 52 / 62; 128 x 64, 288 of them 22 tokens 41 / 47."""
         n = requests * heads
         if dim <= 64:
-            return 15 + n // 20
-        return 14 if vdim > 64 and n > 256 else min(26, 8 + n // 16)
+            return 15 + n // 24
+        if vdim > 64 and n > 256:
+            return 12 if n <= 1024 else 14
+        return min(22, 8 + n * dim * dim // (1 << 18))
 
     def _mlstm_fits(self, l):
         """Whether an mLSTM layer's columns of the step's projection are what ``B.mlstm_prompt`` takes (16-byte pieces of up to 128 columns)."""
