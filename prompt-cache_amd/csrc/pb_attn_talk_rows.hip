@@ -1,6 +1,7 @@
 // pcb_attn_talk_rows: the attention of pcb_attn_talk for single rows (one new token per request), in one launch.
 //
-// Workgroup = one row x KPW of the keys it sees (a multiple of 64, such that a row has at most 16 workgroups), all heads, 64 keys at a time:
+// Workgroup = one row x KPW of the keys it sees (a multiple of 64, such that a row has at most max_parts workgroups; by the row's own position, since a
+// captured step launches for the cache's capacity), all heads, 64 keys at a time:
 //   scores   a wave takes 16 keys against every head: K Q^T on the matrix cores, the heads of one key head as columns; with scale and distance
 //            bias into LDS
 //   mixing   a lane per key, a wave for every fourth head: the heads' sums are lane-local, maximum and denominator of a head are sums over the wave
@@ -11,7 +12,8 @@
 //
 // What bounds it: latency -- one trip to memory, three barriers, one more trip where rows are merged.  us, one row, 8 heads of 128 over 2, 45 keys:
 // scores through the band and the values behind them 13.5 + 12.4 (two launches, 2 and 8 workgroups), 7.8 here.
-// 16 heads over 4, window 1024: 8 rows of 1500 keys 46.6 and 21.0, 64 rows 85.7 and 41.5; no window, one row of 8000 keys 219.8 and 66.5.
+// 16 heads over 4, window 1024: 8 rows of 1500 keys 46.6 and 21.0, 64 rows 85.7 and 41.5; no window, one row of 8000 keys 219.8 and 50.2; one row of 1000
+// keys in a cache of 16384, 45.6 and 20.4 (110.8 with a workgroup's keys by the capacity).
 #include <type_traits>
 
 #include "pb_common.h"
@@ -20,7 +22,13 @@ namespace {
 using namespace pcb;
 
 constexpr int KB = 64;                 // keys at a time
-constexpr int MAX_PARTS = 16;
+// Workgroups that a row of `blocks` blocks of 64 keys may have, of n_rows rows: eight where the rows alone fill the chip, else sixteen, up to four rows
+// over more than 48 blocks 32 (where each query head has its own keys a block of 16 heads in fp32 takes 20 us).  us, eight / sixteen, 64 rows of 1000 keys:
+// 32 heads of 64 columns 61 / 90, 16 of 128 40 / 44; sixteen / 32, one row of 8000 keys: 16 heads over 4 67 / 50, 16 heads of 64 with keys of their own
+// in fp32 173 / 100 (111 through the band); 2000 keys 27 / 30.
+__host__ __device__ __forceinline__ int max_parts(int n_rows, int blocks) { return n_rows <= 4 ? (blocks > 48 ? 32 : 16) : n_rows <= 48 ? 16 : 8; }
+
+constexpr int ANY = 1 << 20;            // (as many blocks as there may be)
 
 // Hand-over between workgroups of one launch: stores that go through to memory, s_waitcnt vmcnt(0) (stores count there on gfx9), barrier, one relaxed
 // arrival; loads that bypass this CU's caches.
@@ -46,7 +54,7 @@ __device__ __forceinline__ float dpp(float v) {
 }
 
 template <typename E, int HMAX, int REP>
-__global__ __launch_bounds__(256, 2) void talk_rows_kernel(pcb_attn_talk_args a, int kpw, float* __restrict__ part, uint32_t* __restrict__ counters) {
+__global__ __launch_bounds__(256, 2) void talk_rows_kernel(pcb_attn_talk_args a, float* __restrict__ part, uint32_t* __restrict__ counters) {
     constexpr int PG = 2;                                         // key heads whose fragments are requested together
     constexpr int VB = sizeof(E) == 2 ? 8 : 4;           // key rows of a thread in flight
     constexpr int HP = HMAX / 4;                         // heads a wave mixes
@@ -69,6 +77,7 @@ __global__ __launch_bounds__(256, 2) void talk_rows_kernel(pcb_attn_talk_args a,
     const int32_t* t = a.tiles + 4 * blockIdx.x;
     const int slot = t[0], i = t[1], row = t[3];
     const int j_min = a.window > 0 && i - a.window + 1 > 0 ? i - a.window + 1 : 0;
+    const int blocks = (i - j_min + KB) / KB, most = max_parts(gridDim.x, blocks), kpw = KB * ((blocks + most - 1) / most);
     const int parts = (i - j_min + kpw) / kpw;           // workgroups of this row
     if ((int)blockIdx.y >= parts) return;                // (uniform over the workgroup)
     const int j_lo = j_min + kpw * blockIdx.y, j_hi = j_lo + kpw <= i ? j_lo + kpw - 1 : i;      // its keys, j_hi included
@@ -249,8 +258,8 @@ __global__ __launch_bounds__(256, 2) void talk_rows_kernel(pcb_attn_talk_args a,
     }
     __syncthreads();
     E* out = (E*)a.out + (int64_t)row * a.ldo;
-    const int rec = HD + 2 * H;
-    float* mine = part + ((int64_t)blockIdx.x * MAX_PARTS + blockIdx.y) * rec;
+    const int rec = HD + 2 * H, stride = max_parts(gridDim.x, ANY);
+    float* mine = part + ((int64_t)blockIdx.x * stride + blockIdx.y) * rec;
 #pragma unroll 1
     for (int e = 2 * tid; e < HD; e += 512) {
         float v0 = 0.0f, v1 = 0.0f;
@@ -280,24 +289,35 @@ __global__ __launch_bounds__(256, 2) void talk_rows_kernel(pcb_attn_talk_args a,
     }
     __syncthreads();
     if (!last_s) return;
-    const float* all = part + (int64_t)blockIdx.x * MAX_PARTS * rec;
+    const float* all = part + (int64_t)blockIdx.x * stride * rec;
     float* w_s = red;                                    // [parts][H]: a part's weight over the row's denominator
     if (tid < H) {
-        float2 ml[MAX_PARTS];
         float m = a.sink ? 0.0f : -INFINITY, l = 0.0f;
+        auto ask = [&](int b0, float2(&ml)[16]) {
 #pragma unroll
-        for (int b = 0; b < MAX_PARTS; ++b) ml[b] = get2(all + (int64_t)(b < parts ? b : 0) * rec + HD + 2 * tid);
+            for (int b = 0; b < 16; ++b) ml[b] = get2(all + (int64_t)(b0 + b < parts ? b0 + b : 0) * rec + HD + 2 * tid);
 #pragma unroll
-        for (int b = 0; b < MAX_PARTS; ++b) m = b < parts ? fmaxf(m, ml[b].x) : m;
+            for (int b = 0; b < 16; ++b) m = b0 + b < parts ? fmaxf(m, ml[b].x) : m;
+        };
+        auto weigh = [&](int b0, float2(&ml)[16]) {
 #pragma unroll
-        for (int b = 0; b < MAX_PARTS; ++b) {
-            ml[b].x = b < parts ? expf(ml[b].x - m) : 0.0f;
-            if (b < parts) l += ml[b].x * ml[b].y;
-        }
+            for (int b = 0; b < 16; ++b) {
+                ml[b].x = b0 + b < parts ? expf(ml[b].x - m) : 0.0f;
+                if (b0 + b < parts) l += ml[b].x * ml[b].y;
+            }
+        };
+        float2 lo[16], hi[16];
+        ask(0, lo);
+        if (parts > 16) ask(16, hi);
+        weigh(0, lo);
+        if (parts > 16) weigh(16, hi);
         if (a.sink) l += expf(-m);
         const float inv = 1.0f / l;
 #pragma unroll
-        for (int b = 0; b < MAX_PARTS; ++b) w_s[b * H + tid] = ml[b].x * inv;
+        for (int b = 0; b < 16; ++b) {
+            w_s[b * H + tid] = lo[b].x * inv;
+            if (parts > 16) w_s[(16 + b) * H + tid] = hi[b].x * inv;
+        }
     }
     __syncthreads();
 #pragma unroll 1
@@ -324,19 +344,17 @@ __global__ __launch_bounds__(256, 2) void talk_rows_kernel(pcb_attn_talk_args a,
 template <typename E>
 int run(const pcb_attn_talk_args& a, float* part, uint32_t* counters, hipStream_t stream) {
     const int rep = a.H / a.Hkv, most = a.window > 0 && a.window < a.max_kv_len ? a.window : a.max_kv_len;
-    const int kpw = KB * pcb_ceil_div(pcb_ceil_div(most, KB), MAX_PARTS);
-    const dim3 grid(a.n_tiles, pcb_ceil_div(most, kpw));
+    const int blocks = pcb_ceil_div(most, KB), parts = max_parts(a.n_tiles, blocks);
+    const dim3 grid(a.n_tiles, blocks < parts ? blocks : parts);
     const int slices = 256 / (a.head_dim / 8 * a.Hkv);
     size_t lds = (size_t)slices * a.H * a.head_dim * sizeof(float);            // (8 KiB times the query heads of a key head, at most)
-    if (lds < MAX_PARTS * (size_t)a.H * sizeof(float)) lds = MAX_PARTS * (size_t)a.H * sizeof(float);
+    if (lds < 32 * (size_t)a.H * sizeof(float)) lds = 32 * (size_t)a.H * sizeof(float);
     auto go = [&](auto hmax, auto r) {
         auto kern = talk_rows_kernel<E, decltype(hmax)::value, decltype(r)::value>;
-        static bool raised = false;
-        if (lds > 32 * 1024 && !raised) {
-            (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);
-            raised = true;
-        }
-        hipLaunchKernelGGL(kern, grid, dim3(256), lds, stream, a, kpw, part, counters);
+        static const hipError_t raised =
+            hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);
+        (void)raised;
+        hipLaunchKernelGGL(kern, grid, dim3(256), lds, stream, a, part, counters);
     };
     auto heads = [&](auto r) {
         if (a.H <= 8)
@@ -365,7 +383,7 @@ bool fits(int dtype, int H, int Hkv, int D) {
 
 PCB_EXPORT int32_t pcb_attn_talk_rows_fits(int32_t dtype, int32_t H, int32_t Hkv, int32_t head_dim) { return fits(dtype, H, Hkv, head_dim); }
 PCB_EXPORT int64_t pcb_attn_talk_rows_part(int32_t n_rows, int32_t H, int32_t head_dim) {
-    return (int64_t)n_rows * MAX_PARTS * ((int64_t)H * head_dim + 2 * H);
+    return (int64_t)n_rows * max_parts(n_rows, ANY) * ((int64_t)H * head_dim + 2 * H);
 }
 
 PCB_EXPORT int pcb_attn_talk_rows(const pcb_attn_talk_args* a, float* part, int64_t part_floats, int32_t* counters, void* stream) {

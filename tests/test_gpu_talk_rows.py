@@ -86,3 +86,25 @@ def test_single_rows_as_the_general_form_gives_them(dtype, sink, mixed):
     x[0, 3], x[2, 40] = float("nan"), float("inf")
     bad = attend(x, cache, talk, tiles, cap, H, G, D, window, None, sink, counters)
     assert torch.equal(torch.isnan(bad), torch.isnan(general(x))) and torch.equal(bad[[1, 3]], got[[1, 3]]) and bool(torch.isnan(bad[[0, 2]]).any())
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 4e-6), (torch.bfloat16, 1.5e-2)])
+@pytest.mark.parametrize("n,places", [(1, [3300]), (4, [3071, 3072, 64, 7000]), (5, [3300, 0, 1023, 1024, 4100]), (49, [1024 + 61 * b for b in range(49)])])
+def test_a_rows_share_of_workgroups_does_not_depend_on_the_capacity(n, places, dtype, tol):
+    """Eight, sixteen and 32 workgroups to a row; launched for a cache much longer than any row, as captured steps are, and for the longest row."""
+    H, G, D = 4, 2, 64
+    q, cache, talk, tiles, cap, want = case(dtype, H, G, D, 0, places)
+    slopes, out = O.head_slopes(H).float().to(DEV), []
+    counters = torch.zeros(n, dtype=torch.int32, device=DEV)
+    for longest in (max(places) + 1, 1 << 20):
+        got, part = torch.zeros_like(q), torch.full((B().attn_talk_rows_part(n, H, D),), float("nan"), device=DEV)
+        B().attn_talk_rows(q, tiles.reshape(-1), n, cache, G * cap * D, cap * D, H, G, D, 0.3, 0, longest, slopes, talk, True, part, counters, got)
+        assert rel(got, want) < tol and not bool(counters.any())
+        out.append(got)
+        used = part.view(n, -1, H * D + 2 * H).isfinite().all(-1).sum(1)
+        for r, p in enumerate(places):                           # (records that a row's workgroups left: none from one alone)
+            blocks = p // 64 + 1
+            most = 8 if n > 48 else 32 if n <= 4 and blocks > 48 else 16
+            per = -(-blocks // most)
+            assert int(used[r]) == (0 if blocks <= per else -(-blocks // per)), (r, p)
+    assert torch.equal(out[0], out[1])
