@@ -344,9 +344,7 @@ __global__ __launch_bounds__(64 * SKW) void linear_skinny_kernel(pcb_linear_args
 }
 
 // The few-row products of pb_linear_parts.h, a launch of their own.  LATE: as above.
-// us, the kernel above / this, 1 row bf16: 1024 x 1024 3.9 / 2.9, 1024 x 4096 8.0 / 4.3, 32000 x 2048 31.4 / 24.0 (5.5 TB/s); 8 rows bf16: 2048 x 2048
-// 6.3 / 4.9, 2048 x 4096 9.2 / 6.8, gated 4096 x 2048 11.4 / 9.5, 5136 x 2048 10.1 / 8.6; fp32: 1 row 1024 x 4096 13.5 / 6.5, 32000 x 2048 58.9 / 43.8,
-// 8 rows 2048 x 2048 10.4 / 7.2, 32000 x 2048 70.4 / 57.1, 16 rows 10272 x 2048 33.2 / 26.4.
+// (few_rows() below says which launches take it, and what both cost)
 template <typename E, int EPI, int PARTS, int U, bool LATE>
 __global__ __launch_bounds__(512) void linear_parts_kernel(pcb_linear_args a) {
     __shared__ f4 red[EPI == PCB_EPI_SILU_MUL ? 2 : 1][8][64];
@@ -639,7 +637,8 @@ int dispatch_dma(const pcb_linear_args& a, int rows, hipStream_t stream) {
         auto rounds = [&](int bm, int bn) { return (batch * (pcb_ceil_div(a.M, bm) + extra) * pcb_ceil_div(a.N, bn) + 255) / 256; };
         // (32 x 32 tiles, three to a CU, up to 768 of them: 600 x 1024, K = 1024 25.8 -> 21.5, 300 x 1024 18.1 -> 16.3, 200 x 2564 26.5 -> 22.1, 600 x 512,
         // K = 512 10.3 -> 9.6; 600 x 2564 (1539) 42.9, 45.1 so.  What is below a round of the chip or deep is with pb_linear_waves.hip.)
-        if (EPI != PCB_EPI_SILU_MUL && a.n_groups == 0 && batch * pcb_ceil_div(a.M, 32) * pcb_ceil_div(a.N, 32) <= 768) return launch_dma<E, EPI, 1, 1, 3>(a, stream);
+        if constexpr (EPI != PCB_EPI_SILU_MUL)
+            if (a.n_groups == 0 && batch * pcb_ceil_div(a.M, 32) * pcb_ceil_div(a.N, 32) <= 768) return launch_dma<E, EPI, 1, 1, 3>(a, stream);
         const float large = 3.8f * rounds(128, 32 * TNW), mid = rounds(64, 16 * TNW), small = 0.575f * rounds(32, 16 * TNW);
         if (rows > 64 && large <= mid && large <= small) return launch_dma<E, EPI, 4, TNW, 2>(a, stream);
         return rows > 32 && mid <= small ? launch_dma<E, EPI, 2, TNW / 2, 3>(a, stream) : launch_dma<E, EPI, 1, TNW / 2, 3>(a, stream);
@@ -660,6 +659,47 @@ int launch(const pcb_linear_args& a, hipStream_t stream) {
     return pcb_check_launch("linear_kernel");
 }
 
+// Which kernel takes a launch of up to sixteen rows: parts runs of k side by side in linear_parts_kernel (0: linear_skinny_kernel), late: where results
+// go is worked out behind the products.  Measured with weights from memory at 4067 points, 64 .. 32000 columns, K = 64 .. 8192, 1 to 16 rows, every
+// epilogue, both types: on average 1.2 % behind the fastest of them all, nowhere more than 8 % behind linear_skinny_kernel.  us below: linear_skinny_kernel /
+// one run / two / four, the faster of late and not.  (g1, g2, g4: workgroups of 16, 8 and 4 columns.)
+struct FewRows {
+    int parts;
+    bool late;
+};
+FewRows few_rows(const pcb_linear_args& a) {
+    const bool bf = a.dtype == PCB_BF16, gated = a.epilogue == PCB_EPI_SILU_MUL, add = a.epilogue == PCB_EPI_SCALE_ADD;
+    if (!pcb_linear_pieces(a)) return {0, false};
+    const int64_t batch = a.n_batch > 0 ? a.n_batch : 1, g1 = batch * pcb_ceil_div(a.N, 16), g2 = batch * pcb_ceil_div(a.N, 8),
+                  g4 = batch * pcb_ceil_div(a.N, 4);
+    // Late beyond three workgroups a CU (the gated unit in bf16 two), stores in bf16 also over K >= 512.  bf16, 32000 x 512, 4 rows added: not late 11.7,
+    // late 10.0; fp32 gated 11000 x 64 6.4, 7.6.
+    const FewRows skinny = {0, false},
+                  one = {1, (g1 > (gated && bf ? 512 : 768) && (bf || !gated || a.K >= 512)) || (bf && a.epilogue == PCB_EPI_STORE && a.K >= 512)};
+    // gated, many columns over next to no k: fp32 11000 x 64 5.4 / 6.4
+    if (gated && a.K < 128) return g1 > 512 ? skinny : one;
+    // more than eight rows in bf16: the kernel above over a deep k of few columns (its sixteen waves) or of more than a round of the chip.  16 rows, K = 4096:
+    // 2048 columns 11.3 / 12.2, 4096 13.7 / 13.3, 5120 19.8 / 22.2, gated 4096 20.3 / 21.8, 5120 34.8 / 31.6
+    if (a.M > 8) return bf && a.K >= 2048 && (g1 <= (gated && a.K >= 4096 ? 256 : 192) || (g1 > 256 && !gated)) ? skinny : one;
+    // four runs up to three workgroups a CU.  1 row bf16: 2048 x 4096 8.5 / 8.4 / 5.9 / 5.7, 3072 x 2048 6.2 / 5.7 / 5.6 / 5.1; 4 rows, 3072 x 2048 6.5 / 6.3 / 6.3 /
+    // 6.2, gated 10.3 / 10.5 / 9.5 / 8.6, 3072 x 1024 5.6 / 4.5 / 4.9 / 4.8, gated 6.8 / 6.5 / 6.6 / 6.5; 1 row fp32 1024 x 2048 9.0 / 7.5 / 5.3 / 4.5
+    const bool late = a.epilogue == PCB_EPI_STORE ? bf || a.M <= 2 : gated && bf;
+    if (a.M <= 4 && a.K % 128 == 0 && a.K >= (gated && bf ? 2048 : 1024) && g4 <= (a.M <= 2 || gated || a.K >= 2048 ? 768 : 512)) return {4, late};
+    // two runs, of more than four rows not where 16 columns each are one round of the chip and eight are two (there the kernel above over a deep k: 8 rows,
+    // K = 4096, 2048 columns 9.6 / 10.3 / 7.1, 2560 9.8 / 10.6 / 10.6, 4096 13.6 / 11.6 / 11.3, 8192 18.3 / 20.1 / 20.4, 16384 35.8 / 36.0 / 36.4)
+    if (a.K % 64 != 0 || a.K < (bf ? 1024 : 512)) return one;
+    if (a.M > 4 && !gated) {
+        const bool hole = g2 > 256 && g2 <= 400;
+        if (bf && a.K >= 4096 && (hole || (g2 > 768 && g2 <= 1400))) return skinny;
+        if (hole) return one;
+    }
+    // ... and while the chip has places for them: accumulations in bf16 8 rows, 4096 x 1024 5.6 / 4.9 / 5.1, 8192 x 1024 6.7 / 7.0 / 7.5, 8192 x 2048 10.8 / 11.7 /
+    // 11.5; stores in bf16 at any size (32000 x 2048, 1 row 30.0 / 27.8 / 23.6, 4 rows 31.8 / 30.2 / 28.8); fp32, K = 2048, 4 rows, 8192 columns 20.1 / 17.3 /
+    // 17.5, 8 rows, 6144 20.4 / 16.9 / 15.8, 8192 21.8 / 18.1 / 19.9; 4 rows added, K = 512, 4096 columns 5.7 / 5.0 / 5.2, 8192 7.3 / 6.4 / 6.9
+    const int64_t most = bf ? (!add ? INT64_MAX : a.K < 2048 ? 640 : a.M > 4 ? 768 : INT64_MAX) : add && a.K < 1024 ? 640 : a.M <= 4 ? 1024 : 768;
+    return g2 <= most ? FewRows{2, late} : one;
+}
+
 template <typename E>
 int dispatch(const pcb_linear_args& a, hipStream_t stream) {
     // rows per group decide the row tile: many rows -> 128-row panels, few -> 32-row panels (the weights stream once)
@@ -671,56 +711,36 @@ int dispatch(const pcb_linear_args& a, hipStream_t stream) {
         const dim3 grid(pcb_ceil_div(a.N, 16), pcb_ceil_div(a.M, 16) + (a.n_groups > 0 ? a.n_groups : 0), a.n_batch > 0 ? a.n_batch : 1);
         const int64_t groups = (int64_t)grid.x * grid.y * grid.z;
         const bool deep = a.K >= 2048 && groups <= 192;
-        // LATE beyond three workgroups a CU, of the gated unit over few k beyond four.  bf16, us, 1 and 8 rows, ahead of the products / late:
-        // K = 1024, 12288 columns (768 workgroups) 6.5 / 6.5 and 7.4 / 7.9, 12800 8.2 / 7.6 and 9.6 / 9.4, 16384 9.0 / 7.7 and 12.1 / 9.5,
-        // 32000 15.6 / 13.9 and 18.8 / 17.6; K = 2048, 13600 columns 17.5 / 13.9 and 22.0 / 18.2; gated, 8 rows, 16384 columns 13.2 / 13.9;
-        // K = 2048, 1 row, 13600 columns 27.4 / 26.4.
+        // LATE beyond three workgroups a CU, of the gated unit over few k beyond four.  Of the launches that come this far (groups, odd rows, many columns
+        // over a deep k), bf16, us, ahead of the products / late: stores 8 rows, 16384 x 1000 15.5 / 12.8, x 2024 28.8 / 22.1, x 4096 44.1 / 35.0, 32000 x 4096
+        // 62.1 / 59.7; 8 groups of 2048 x 1024, one row each 13.4 / 10.2; accumulations 16384 x 1000 11.8 / 11.9, 32000 x 4096 64.4 / 59.5; gated, 1 row,
+        // 16384 x 1000 23.4 / 22.2, 8 rows 26.2 / 25.7, 32000 x 2024 67.9 / 66.6, x 4096 111.6 / 117.9.
         const bool late = sizeof(E) == 2 && groups > (a.epilogue == PCB_EPI_SILU_MUL && a.K < 2048 ? 1024 : 768);
-        // Runs side by side: four where up to four rows leave no more than three workgroups a CU so, else two, and for more than four rows not where 16
-        // columns each are one round of the chip and eight are two (us, 8 rows, K = 2048, one run / two: 3072 columns bf16 6.3 / 6.7, fp32 9.5 / 10.8;
-        // 5136 9.8 / 8.6 and 16.5 / 14.5) or beyond 1024 workgroups (fp32: 768; 7424 columns 10.7 / 10.4 and 18.1 / 18.7, 32000 34.1 / 35.1 and
-        // 57.1 / 64.4).  A run has eight k-steps at least.  bf16 of more than eight rows over a deep k of few columns stays with sixteen waves above
-        // (16 rows, 2048 x 4096: 10.8, here 11.2).
-        const int es = sizeof(E), batch = a.n_batch > 0 ? a.n_batch : 1;
-        if (pcb_linear_pieces(a) && !(es == 2 && a.M > 8 && deep)) {
-            const int64_t four = (int64_t)batch * pcb_ceil_div(a.N, 4), two = (int64_t)batch * pcb_ceil_div(a.N, 8);
-            int parts = 1;
-            if (a.M <= 4 && four <= 768 && a.K % 128 == 0 && a.K >= 1024)
-                parts = 4;
-            else if (a.M <= 8 && a.K % 64 == 0 && a.K >= 512 && (a.M <= 4 || two <= 256 || (two > 400 && two <= (es == 2 ? 1024 : 768))))
-                parts = 2;
-            auto go = [&](auto epi, auto p, auto u, auto late) {
-                hipLaunchKernelGGL((linear_parts_kernel<E, decltype(epi)::value, decltype(p)::value, decltype(u)::value, decltype(late)::value>),
-                                   dim3(pcb_ceil_div(a.N, 16 / decltype(p)::value), 1, batch), dim3(512), 0, stream, a);
+        const FewRows few = few_rows(a);
+        if (few.parts > 0) {
+            auto go = [&](auto epi, auto p, auto late) {
+                constexpr int EPI = decltype(epi)::value, P = decltype(p)::value;
+                // (fp32: more k-steps in flight cost workgroups)
+                hipLaunchKernelGGL((linear_parts_kernel<E, EPI, P, sizeof(E) == 2 ? 4 : 2, decltype(late)::value>),
+                                   dim3(pcb_ceil_div(a.N, 16 / P), 1, a.n_batch > 0 ? a.n_batch : 1), dim3(512), 0, stream, a);
             };
             using One = std::integral_constant<int, 1>;
             using Two = std::integral_constant<int, 2>;
             using Four = std::integral_constant<int, 4>;
-            using Steps = std::integral_constant<int, sizeof(E) == 2 ? 4 : 2>;             // (fp32: more in flight costs workgroups)
-            using Deep = std::integral_constant<int, sizeof(E) == 2 ? 8 : 2>;
-            auto kind = [&](auto epi, auto late) {
-                if (parts == 4)
-                    go(epi, Four{}, Steps{}, late);
-                else if (parts == 2)
-                    go(epi, Two{}, Steps{}, late);
-                else if (a.K >= 2048)
-                    go(epi, One{}, Deep{}, late);
-                else
-                    go(epi, One{}, Steps{}, late);
+            auto kind = [&](auto epi) {
+                // (what few_rows() does not ask for is not built: runs side by side are late in a plain store, in bf16 in the gated unit)
+                constexpr bool LATE = decltype(epi)::value == PCB_EPI_STORE || (sizeof(E) == 2 && decltype(epi)::value == PCB_EPI_SILU_MUL);
+                if (few.parts == 1)
+                    return few.late ? go(epi, One{}, std::true_type{}) : go(epi, One{}, std::false_type{});
+                if constexpr (LATE)
+                    if (few.late) return few.parts == 4 ? go(epi, Four{}, std::true_type{}) : go(epi, Two{}, std::true_type{});
+                if constexpr (!LATE || sizeof(E) == 4) few.parts == 4 ? go(epi, Four{}, std::false_type{}) : go(epi, Two{}, std::false_type{});
             };
-            // (where results go, worked out behind the products: -0.1 to -0.3 us from K = 1024 on, +0.2 below; gated units only where 16 columns each
-            // fill the chip, 16 rows x 4096, K = 2048 11.1 against 12.5; what a scaled accumulation adds to is asked for ahead of them)
-            if (a.epilogue == PCB_EPI_SILU_MUL && parts == 1)
-                go(std::integral_constant<int, PCB_EPI_SILU_MUL>{}, One{}, Steps{}, std::true_type{});
-            else if (a.epilogue == PCB_EPI_SILU_MUL)
-                parts == 4 ? go(std::integral_constant<int, PCB_EPI_SILU_MUL>{}, Four{}, Steps{}, std::false_type{})
-                           : go(std::integral_constant<int, PCB_EPI_SILU_MUL>{}, Two{}, Steps{}, std::false_type{});
-            else if (a.epilogue == PCB_EPI_SCALE_ADD)
-                kind(std::integral_constant<int, PCB_EPI_SCALE_ADD>{}, std::false_type{});
-            else if (a.K >= 1024)
-                kind(std::integral_constant<int, PCB_EPI_STORE>{}, std::true_type{});
-            else
-                kind(std::integral_constant<int, PCB_EPI_STORE>{}, std::false_type{});
+            switch (a.epilogue) {
+                case PCB_EPI_STORE: kind(std::integral_constant<int, PCB_EPI_STORE>{}); break;
+                case PCB_EPI_SILU_MUL: kind(std::integral_constant<int, PCB_EPI_SILU_MUL>{}); break;
+                default: kind(std::integral_constant<int, PCB_EPI_SCALE_ADD>{});
+            }
             return pcb_check_launch("linear_parts_kernel");
         }
         auto go = [&](auto epi) {

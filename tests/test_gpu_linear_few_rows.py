@@ -64,3 +64,21 @@ def test_few_rows_of_a_batch(M, N, K, n, dtype):
     B().linear(x, w, y, M=M, n_batch=n, ldx=n * K, x_batch_stride=K, ldy=n * N, y_batch_stride=N)
     want = torch.stack([x.to(F64)[:, i * K:(i + 1) * K] @ w[i].to(F64).T for i in range(n)], 1).reshape(M, n * N)
     assert rel(y, want) < 1e-6
+
+
+# sizes on both sides of the rule's other borders: one run late and not, a deep k of few and of many columns, four runs' and two runs' last sizes
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M", [2, 4, 7, 12])
+@pytest.mark.parametrize("N,K", [(12300, 64), (12300, 96), (8250, 480), (8200, 512), (6200, 960), (2600, 4096), (4100, 4096), (8300, 4096)])
+def test_few_rows_at_the_rules_other_borders(M, N, K, dtype):
+    b, f = B(), lambda t: t.to(F64)
+    low = 1e-6 if dtype == torch.float32 else 2.0 ** -8
+    x, w, w2 = rnd(M, K, seed=1, dtype=dtype), rnd(N, K, seed=2, dtype=dtype) * 0.1, rnd(N, K, seed=5, dtype=dtype) * 0.1
+    z, out, y = f(x) @ f(w).T, torch.empty(M, N, dtype=dtype, device=DEV), rnd(M, N, seed=6)
+    b.linear(x, w, out, M=M)
+    assert rel(out, z) < low
+    b.linear(x, w, out, M=M, epilogue=b.EPI_SILU_MUL, w2=w2, act=b.ACT_RELU)
+    assert rel(out, z.relu() * (f(x) @ f(w2).T)) < max(low, 2e-6)
+    scale, want = rnd(N, seed=7), f(y)
+    b.linear(x, w, y, M=M, epilogue=b.EPI_SCALE_ADD, col_scale=scale)
+    assert rel(y, want + f(scale) * z) < 1e-6
