@@ -171,10 +171,13 @@ int64_t pcb_linear_waves_tiles(const pcb_linear_args& a) {
 // 130 x 4096, K = 1024 (640) 8.8 / 10.4.
 // fp32: a round of the chip, and three over a deep k.  37 x 1024, K = 1024 17.5 / 9.5, K = 4096 60 / 25; 64 x 2048 gated, K = 1024 18.9 / 10.7;
 // 300 x 2048, K = 2048 (640) 47.6 / 39.9, 75 x 4096 gated (768) 52 / 45; 130 x 5136 (805) 50.5 / 52.9.
+// A wave has to have two chunks of k at least for its own ring to be worth the sums at the end, beyond 192 workgroups bf16 four: bf16 17 x 2048, K = 256
+// 4.0 / 4.4, 17 x 11000 (344) K = 256 4.6 / 6.2, K = 512 5.7 / 6.9, 128 x 4096 (512) K = 512 6.2 / 6.7, gated 17 x 4096 (256) 6.1 / 6.5; fp32 64 x 512, K = 64 3.9 / 4.7.
 bool pcb_linear_waves_fits(const pcb_linear_args& a) {
     if (a.n_groups > 0) return false;
     const int64_t wgs = pcb_linear_waves_tiles(a) * (a.n_batch > 0 ? a.n_batch : 1);
-    return a.dtype == PCB_BF16 ? wgs <= 512 : wgs <= 256 || (wgs <= 768 && a.K >= 2048);
+    if (a.dtype != PCB_BF16) return a.K >= 256 && (wgs <= 256 || (wgs <= 768 && a.K >= 2048));
+    return a.K >= 1024 ? wgs <= 512 : a.K >= 512 && wgs <= 192;
 }
 
 // Three images to a wave's ring (96 KB: one workgroup a CU); two where bf16 has two workgroups a CU (300 x 1024, K = 1024: 6.7 us, 9.1 with three; 200 x
