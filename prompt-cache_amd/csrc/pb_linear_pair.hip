@@ -162,10 +162,10 @@ int pair(const pcb_linear_args& a, const pcb_linear_args& b, hipStream_t stream)
         return pcb_check_launch("linear_pair_kernel");
     };
     // Two runs of k side by side (up to eight rows) while both products together have no more than 8192 weight rows, beyond that up to four rows, not
-    // with a gated bf16 unit.  Weights from memory, us, one run / two: 1 row bf16, 1280 + 4096 columns, K = 1024 5.9 / 5.5, K = 512 3.9 / 4.1; 2560 + 8192,
+    // with a gated bf16 unit.  Weights from memory, us, one run / two: 1 row bf16, 1280 + 4096 columns, K = 1024 5.9 / 5.5, 640 + 2048, K = 512 3.9 / 4.1; 2560 + 8192,
     // K = 2048 12.9 / 11.2, 8 rows 14.7 / 15.5; 1024 and 2048 gated, K = 1024, 8 rows 6.7 / 6.1, fp32 9.9 / 8.8; 2048 and 4096 gated, K = 2048, 1 row
     // 12.1 / 12.3, 2 rows fp32 21.8 / 19.7, 8 rows 13.5 / 14.9.  (Four runs lose 2 to 20 % against two at each of these.)  As launches of their own,
-    // the first of each pair: 8.0, 6.7, 13.9, 18.6, 9.7, 12.8, 13.0, 23.6, 15.0.
+    // the first of each pair: 8.1, 6.4, 13.9, 19.3, 9.9, 13.2, 13.7, 23.3, 16.0.
     const bool gated = b.epilogue == PCB_EPI_SILU_MUL;
     const int64_t w_rows = (int64_t)a.N + (gated ? 2 : 1) * (int64_t)b.N;
     const bool two = a.M <= 8 && a.K >= 1024 && b.K >= 1024 && splits(a, 2) && splits(b, 2) &&
@@ -196,7 +196,12 @@ PCB_EXPORT int pcb_linear_pair(const pcb_linear_args* a, const pcb_linear_args* 
     if (rc != PCB_OK) return rc;
     const bool one = a->dtype == b->dtype && a->M == b->M && a->M > 0 && a->M <= 16 && a->n_batch == 0 && b->n_batch == 0 && a->epilogue == PCB_EPI_STORE &&
                      b->epilogue != PCB_EPI_SCALE_ADD && pcb_linear_pieces(*a) && pcb_linear_pieces(*b);
-    if (!one) {
+    // (A gated unit in bf16 only up to 80 MB of weights: alone it is faster then.  us, two launches / one, 8 rows, residual gate and gated unit of a width:
+    // 2048 15.9 / 14.3, 2560 (66 MB) 24.4 / 21.6, 3072 (94 MB) 28.9 / 29.8, 1 row 13.6 / 12.8, 19.4 / 18.9, 23.4 / 26.5.  9 and 16 rows: bf16 2048 18.7 / 14.7 and
+    // 20.0 / 16.0, 2560 29.2 / 22.2 and 32.9 / 25.2; fp32 2048 27.5 / 23.6 and 29.1 / 26.5; plain, 2560 + 8192
+    // columns, K = 2048, bf16 18.9 / 15.1 and 20.8 / 17.6.)
+    const bool heavy = a->dtype == PCB_BF16 && b->epilogue == PCB_EPI_SILU_MUL && ((int64_t)a->N * a->K + 2 * (int64_t)b->N * b->K) * 2 > 80000000;
+    if (!one || heavy) {
         rc = pcb_linear(a, stream);
         return rc == PCB_OK ? pcb_linear(b, stream) : rc;
     }
@@ -216,7 +221,10 @@ PCB_EXPORT int pcb_linear_add2(const pcb_linear_args* a, const pcb_linear_args* 
     // 11.2 / 7.3, 4 rows 12.7 / 8.9, 8 rows 15.0 / 12.1; 2048 columns, K = 2048 and 8192 18.1 / 14.3, 4 rows 21.7 / 20.7, 8 rows 22.3 / 21.7, fp32 34.0 / 30.2.
     const bool pieces = pcb_linear_pieces(*a) && pcb_linear_pieces(*b) && !a->row_src && !b->row_src && (!z || (uintptr_t)z % 16 == 0);
     const int parts = a->M <= 4 && splits(*a, 4) && splits(*b, 4) && pcb_ceil_div(a->N, 4) <= 768 ? 4 : a->M <= 8 && splits(*a, 2) && splits(*b, 2) ? 2 : 0;
-    if (pieces && parts)
+    // In bf16 three rows and more only up to 56 MB of weights: 4 rows, 2048 columns, K = 2048 and 8192 (42 MB) as launches of their own 21.8, here 20.9, 2560 and
+    // 10240 (66 MB) 31.6 / 35.7, 4096 and 16384 48.3 / 53.9, 8 rows 56.1 / 68.8; 1 row 24.5 / 23.0, 43.9 / 42.5; 4 rows fp32 48.4 / 47.7, 86.7 / 81.6.
+    const bool heavy = a->dtype == PCB_BF16 && a->M > 2 && (int64_t)a->N * ((int64_t)a->K + b->K) * 2 > 56000000;
+    if (pieces && parts && !heavy)
         return a->dtype == PCB_BF16 ? add2<pcb::bf16_t>(*a, *b, z, coef, eps, parts, (hipStream_t)stream)
                                     : add2<float>(*a, *b, z, coef, eps, parts, (hipStream_t)stream);
     rc = pcb_linear(a, stream);
