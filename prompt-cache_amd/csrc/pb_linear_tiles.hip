@@ -5,7 +5,7 @@
 // barrier of every K-step, at the larger tiles power.  Against linear_dma_kernel (pb_linear.hip: 16 x 16 MFMAs, two or three images, two
 // workgroups to a CU), us, 2048 rows: 2048 x 2048 29.9 -> 19.9 (0.87 PFLOP/s), K = 8192 93.5 -> 72, 2560 columns 39.8 -> 31, 8192 columns
 // 90.5 -> 65.6 (1.05 PFLOP/s; the gated pair 79.3 -> 60.7); 4096 x 4096 x 4096 161 -> 112 (1.23 PFLOP/s).  With a sigmoid on half of the columns: 5136
-// columns 73.7 -> 56, 10272 133 -> 113 since results that are rounded to bf16 take the machine's exponential and reciprocal.
+// columns 77.6 -> 63.0, 10272 132 -> 124 since it and silu do without expf's and the division's cases (over_one_plus_exp; and 192-column tiles).
 #include "mfma_tile_loop.h"
 #include "pb_linear_epi.h"
 #include "pb_linear_tiles.h"
@@ -42,29 +42,37 @@ __device__ __forceinline__ void store_columns(const pcb_linear_args& a, char* pa
     const int esz = (EPI == PCB_EPI_SCALE_ADD || a.out_f32) ? 4 : 2;
     const bool quad = a.ldy % 4 == 0 && (uintptr_t)a.y % (4 * esz) == 0 && n + 4 <= whole &&
                       (EPI != PCB_EPI_SCALE_ADD || !a.base || (a.ldbase % 4 == 0 && (uintptr_t)a.base % 16 == 0));
+    auto largest = [](const f4(&v)[4]) {                             // (what is no number does not count: it stays none either way)
+        float top = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) top = fmaxf(top, fabsf(v[e][k]));
+        return top;
+    };
     if (EPI == PCB_EPI_STORE && (a.bias || (a.act | a.act2))) {
         const int mid = a.act_split > 0 && a.act_split < whole ? a.act_split : whole;
         f4 bv = four((const E*)a.bias);
-        // (codes below 0: the form for results that are rounded to bf16)
-        auto act_of = [&](auto code, float x) {
-            constexpr int A = decltype(code)::value;
-            if constexpr (A == -PCB_ACT_SIGMOID) return rounded_sigmoid(x);
-            else if constexpr (A == -PCB_ACT_SILU) return x * rounded_sigmoid(x);
-            else return apply_act(A, x, a.act_param);
-        };
         auto run = [&](auto code, int lo, int hi) {
 #pragma unroll 1
             for (int e0 = 0; e0 < R; e0 += 4) {
                 f4 v[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = *at(e0 + e, 0) + bv;
+                auto each = [&](auto f) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
+                    for (int e = 0; e < 4; ++e) {
 #pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        if (n + k >= lo && n + k < hi) v[e][k] = act_of(code, v[e][k]);
-                    *at(e0 + e, 0) = v[e];
-                }
+                        for (int k = 0; k < 4; ++k)
+                            if (n + k >= lo && n + k < hi) v[e][k] = f(v[e][k]);
+                        *at(e0 + e, 0) = v[e];
+                    }
+                };
+                constexpr int A = decltype(code)::value;
+                if ((A == PCB_ACT_SIGMOID || A == PCB_ACT_SILU) && largest(v) <= PLAIN_EXP)
+                    each([](float x) { return over_one_plus_exp(A == PCB_ACT_SILU ? x : 1.0f, x); });
+                else
+                    each([&](float x) { return apply_act(A, x, a.act_param); });
             }
             bv = f4{0.f, 0.f, 0.f, 0.f};
         };
@@ -74,9 +82,7 @@ __device__ __forceinline__ void store_columns(const pcb_linear_args& a, char* pa
             const int act = part ? a.act2 : a.act, lo = part ? mid : 0, hi = part ? whole : mid;
             if (n0 >= hi || n0 + 4 * LPR <= lo || act == PCB_ACT_NONE) continue;
             added = true;
-            switch (a.out_f32 || (act != PCB_ACT_SIGMOID && act != PCB_ACT_SILU) ? act : -act) {
-                case -PCB_ACT_SILU: run(std::integral_constant<int, -PCB_ACT_SILU>{}, lo, hi); break;
-                case -PCB_ACT_SIGMOID: run(std::integral_constant<int, -PCB_ACT_SIGMOID>{}, lo, hi); break;
+            switch (act) {
                 case PCB_ACT_SILU: run(std::integral_constant<int, PCB_ACT_SILU>{}, lo, hi); break;
                 case PCB_ACT_SIGMOID: run(std::integral_constant<int, PCB_ACT_SIGMOID>{}, lo, hi); break;
                 case PCB_ACT_RELU2: run(std::integral_constant<int, PCB_ACT_RELU2>{}, lo, hi); break;
@@ -103,21 +109,25 @@ __device__ __forceinline__ void store_columns(const pcb_linear_args& a, char* pa
                     u[e] = *at(e0 + e, 8) + bv2;
                     rg[e] = a.row_gate ? to_f32(((const E*)a.row_gate)[row(e0 + e) * a.ld_row_gate]) : 1.0f;
                 }
+                auto each = [&](auto f) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
+                    for (int e = 0; e < 4; ++e) {
 #pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        v[e][k] = (decltype(code)::value < 0 ? v[e][k] * rounded_sigmoid(v[e][k]) : gate_act(decltype(code)::value, v[e][k])) * u[e][k] * rg[e];
-                    *at(e0 + e, 0) = v[e];
-                }
+                        for (int k = 0; k < 4; ++k) v[e][k] = f(v[e][k]) * u[e][k] * rg[e];
+                        *at(e0 + e, 0) = v[e];
+                    }
+                };
+                constexpr int A = decltype(code)::value;
+                if (A == PCB_ACT_SILU && largest(v) <= PLAIN_EXP)
+                    each([](float x) { return over_one_plus_exp(x, x); });
+                else
+                    each([](float x) { return gate_act(A, x); });
             }
         };
         if (a.act == PCB_ACT_RELU)
             gate(std::integral_constant<int, PCB_ACT_RELU>{});
         else if (a.act == PCB_ACT_GELU_TANH)
             gate(std::integral_constant<int, PCB_ACT_GELU_TANH>{});
-        else if (!a.out_f32)
-            gate(std::integral_constant<int, -PCB_ACT_SILU>{});
         else
             gate(std::integral_constant<int, PCB_ACT_SILU>{});
     }
