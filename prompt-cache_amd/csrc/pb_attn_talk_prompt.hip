@@ -75,8 +75,9 @@ __global__ __launch_bounds__(256 * NU, 2) void talk_prompt_kernel(pcb_attn_talk_
             if (rq < nq) fq[c][st] = load8((const bf16_t*)a.q + (int64_t)(row0 + rq) * a.ldq + (4 * (c % HKV) + (l15 >> 2)) * D + 32 * st + 8 * g);
         }
     }
-    // Scores are kept in units of ln 2, so that a weight is one v_exp_f32: scale and log2 e go into the mixing's weights, and the distance bias, which is
-    // linear, is mixed once.
+    // Scores are kept in units of ln 2, so that a weight is one v_exp_f32: scale and log2 e go into the mixing's weights (rounded once, from 64 bits), and the
+    // distance bias, which is linear, is mixed once.  That leaves out the roundings of every head's scaled and biased score: the weights' error against
+    // 64 bits is 0.2 to 1.0 of that of scores mixed from those (2048 keys of 16 heads 3.2e-6, 1.5e-5 that way; no bias 2.7e-7, 2.8e-7).
     const double log2e = 1.4426950408889634;
     const int my = l15 % H;                                      // this lane's head
     const int i0 = q0 + 4 * (l15 / H);                           // position of its query 0

@@ -1,19 +1,23 @@
 // pcb_mlstm: the matrix memory of an mLSTM layer, token by token.  Per (slot, head): S [dim][vdim], a normaliser n [dim] and a
 // running maximum m of the log gates, all fp32 (see pcb_mlstm_args for the recurrence).
 //
-// One workgroup = one request x one head x 64 value columns.  Wave p of its four owns the key rows d = p DPT .. (p + 1) DPT - 1 and
-// lane j the value column: a thread keeps its DPT entries S[d][j] in registers for the whole request, and the matching entries of
-// n as well (every lane of a wave holds the same ones, which spares a broadcast per token).  Tokens arrive in blocks of TB: the
+// One workgroup = one request x one head x NB blocks of 64 value columns, four waves each.  Wave p of a block's four owns the key rows
+// d = p DPT .. (p + 1) DPT - 1 and lane j the value column: a thread keeps its DPT entries S[d][j] in registers for the whole request, and the
+// matching entries of n as well (every lane of a wave holds the same ones, which spares a broadcast per token).  Beyond 128 value columns there
+// are several launches, the first columns last: n and m, which all of them read and are moved in place, are written by that one alone.  Tokens arrive in blocks of TB: the
 // whole block's q, k, v and gates are requested at once (one memory round trip per block, and the next block's while the current
 // one is worked on), staged in LDS -- q scaled, the gates already through cap / logsigmoid --, and the block's tokens then run
 // from LDS alone: every thread advances the running maximum by itself, updates its slice, leaves partial sums of S^T q and n . q
-// in LDS (two alternating sets, so one barrier per token), and wave 0 adds the four parts and stores the output row.
+// in LDS (two alternating sets, so one barrier per token), and a block's wave 0 adds the four parts and stores its
+// columns of the output row.
 //
 // A long prompt is cut into segments that run side by side (pcb_mlstm_args.from_nothing, pcb_mlstm_chain): with the stabilised
 // state (S, n, m) standing for the true sums exp(m) S and exp(m) n, a segment that starts from nothing (S = n = 0, m = -inf) leaves
 // its own contribution (S', n', m') and the sum F of its log forget gates, and a state (S, n, m) carried over it becomes
 //   m'' = max(F + m, m'),   S'' = exp(F + m - m'') S + exp(m' - m'') S',   n'' likewise
 // which is what the token-by-token recurrence gives, since its running maximum unrolls to exactly that maximum.
+#include <type_traits>
+
 #include "pb_common.h"
 
 namespace {
@@ -25,19 +29,20 @@ __device__ __forceinline__ float log_sigmoid(float z) { return fminf(z, 0.0f) - 
 constexpr int TB = 8;          // tokens per staged block
 
 // OUT false: only the states move (the first pass over segments) -- no products with q, no partial sums, no barrier per token
-template <typename E, int DPT, bool OUT>
-__global__ __launch_bounds__(256) void mlstm_kernel(pcb_mlstm_args a) {
-    constexpr int DM = 4 * DPT;                 // key rows the workgroup can hold (>= dim)
-    constexpr int QN = TB * DM / 256;           // q (and k) elements a thread fetches per block
-    constexpr int VN = TB * 64 / 256;           // v elements a thread fetches per block
+template <typename E, int DPT, int NB, bool OUT>
+__global__ __launch_bounds__(256 * NB) void mlstm_kernel(pcb_mlstm_args a, int col0) {
+    constexpr int DM = 4 * DPT, NT = 256 * NB, VC = 64 * NB;      // key rows the workgroup can hold (>= dim), threads, value columns
+    constexpr int QN = TB * DM / NT;            // q (and k) elements a thread fetches per block
+    constexpr int VN = TB * VC / NT;            // v elements a thread fetches per block
     __shared__ __attribute__((aligned(16))) float qs[2][TB][DM], ks[2][TB][DM];
-    __shared__ float vs[2][TB][64], gs[2][TB][2];
-    __shared__ float part_o[2][4][64], part_n[2][4];
-    const int tid = threadIdx.x, lane = tid & 63, p = tid >> 6;
+    __shared__ float vs[2][TB][VC], gs[2][TB][2];
+    __shared__ float part_o[2][4][VC], part_n[2][4];
+    const int tid = threadIdx.x, lane = tid & 63, p = tid >> 6 & 3, jv = (tid >> 8) * 64 + lane;
     const int32_t* rq = a.reqs + 4 * blockIdx.x;
     const int slot = rq[0], pos0 = rq[1], count = rq[2], row0 = rq[3];
     const int h = blockIdx.y, dim = a.dim, vdim = a.vdim;
-    const int j0 = blockIdx.z * 64, j = j0 + lane;
+    const int j = col0 + jv;
+    const bool first = col0 == 0 && tid < 256;                    // (of these columns: who leaves n and m)
     const bool col = j < vdim;
     float* st = a.state + (int64_t)slot * a.slot_stride + (int64_t)h * ((int64_t)dim * vdim + dim + 1);
     float* st_n = st + (int64_t)dim * vdim;
@@ -55,7 +60,7 @@ __global__ __launch_bounds__(256) void mlstm_kernel(pcb_mlstm_args a) {
 
     const E* q = (const E*)a.q + (int64_t)row0 * a.ldq + (int64_t)h * dim;
     const E* k = (const E*)a.k + (int64_t)row0 * a.ldk + (int64_t)h * dim;
-    const E* v = (const E*)a.v + (int64_t)row0 * a.ldv + (int64_t)h * vdim + j0;
+    const E* v = (const E*)a.v + (int64_t)row0 * a.ldv + (int64_t)h * vdim + col0;
     const E* gi = (const E*)a.gi + (int64_t)row0 * a.ldgi + h;
     const E* gf = (const E*)a.gf + (int64_t)row0 * a.ldgf + h;
     // a block in flight: this thread's share of its q, k, v and (threads 0 .. TB-1) one token's gates
@@ -64,15 +69,15 @@ __global__ __launch_bounds__(256) void mlstm_kernel(pcb_mlstm_args a) {
         const int t0 = blk * TB;
 #pragma unroll
         for (int i = 0; i < QN; ++i) {
-            const int e = tid + 256 * i, tt = e / DM, d = e % DM;
+            const int e = tid + NT * i, tt = e / DM, d = e % DM;
             const bool ok = d < dim && t0 + tt < count;
             rq_[i] = (OUT && ok) ? to_f32(q[(int64_t)(t0 + tt) * a.ldq + d]) * a.q_scale : 0.0f;
             rk_[i] = ok ? to_f32(k[(int64_t)(t0 + tt) * a.ldk + d]) : 0.0f;
         }
 #pragma unroll
         for (int i = 0; i < VN; ++i) {
-            const int e = tid + 256 * i, tt = e >> 6, jj = e & 63;
-            rv_[i] = (j0 + jj < vdim && t0 + tt < count) ? to_f32(v[(int64_t)(t0 + tt) * a.ldv + jj]) : 0.0f;
+            const int e = tid + NT * i, tt = e / VC, jj = e % VC;
+            rv_[i] = (col0 + jj < vdim && t0 + tt < count) ? to_f32(v[(int64_t)(t0 + tt) * a.ldv + jj]) : 0.0f;
         }
         if (tid < TB && t0 + tid < count) {
             rgi = to_f32(gi[(int64_t)(t0 + tid) * a.ldgi]);
@@ -82,14 +87,14 @@ __global__ __launch_bounds__(256) void mlstm_kernel(pcb_mlstm_args a) {
     auto stage = [&](int b) {
 #pragma unroll
         for (int i = 0; i < QN; ++i) {
-            const int e = tid + 256 * i;
+            const int e = tid + NT * i;
             if (OUT) qs[b][e / DM][e % DM] = rq_[i];
             ks[b][e / DM][e % DM] = rk_[i];
         }
 #pragma unroll
         for (int i = 0; i < VN; ++i) {
-            const int e = tid + 256 * i;
-            vs[b][e >> 6][e & 63] = rv_[i];
+            const int e = tid + NT * i;
+            vs[b][e / VC][e % VC] = rv_[i];
         }
         if (tid < TB) {
             gs[b][tid][0] = soft_cap(rgi, a.gate_cap);
@@ -114,7 +119,7 @@ __global__ __launch_bounds__(256) void mlstm_kernel(pcb_mlstm_args a) {
             m = m_new;
             f_sum += lf;
             float acc = 0.0f, accn = 0.0f;
-            const float tv = take * vs[b][tt][lane];
+            const float tv = take * vs[b][tt][jv];
             const float4* k4 = reinterpret_cast<const float4*>(&ks[b][tt][p * DPT]);     // (rows past dim were staged as zeros)
             const float4* q4 = reinterpret_cast<const float4*>(&qs[b][tt][p * DPT]);
 #pragma unroll
@@ -133,17 +138,18 @@ __global__ __launch_bounds__(256) void mlstm_kernel(pcb_mlstm_args a) {
                 }
             }
             if (!OUT) continue;
-            part_o[pb][p][lane] = acc;
-            if (lane == 0) part_n[pb][p] = accn;
+            part_o[pb][p][jv] = acc;
+            if (tid < 256 && lane == 0) part_n[pb][p] = accn;
             __syncthreads();
             if (p == 0 && col) {
-                const float num = (part_o[pb][0][lane] + part_o[pb][1][lane]) + (part_o[pb][2][lane] + part_o[pb][3][lane]);
+                const float num = (part_o[pb][0][jv] + part_o[pb][1][jv]) + (part_o[pb][2][jv] + part_o[pb][3][jv]);
                 const float nq_dot = (part_n[pb][0] + part_n[pb][1]) + (part_n[pb][2] + part_n[pb][3]);
                 const float den = fmaxf(fabsf(nq_dot), expf(-m_new)) + 1e-6f;
                 a.out[(int64_t)(row0 + t) * a.ldo + (int64_t)h * vdim + j] = num / den;
             }
         }
     }
+    __syncthreads();                                       // (n and m are read by every wave, written by one block's: all tokens are through by now)
     // where the request's last state goes: its own record, or (the last segment of a prompt) the slot it belongs to
     if (a.end_slots && a.end_slots[blockIdx.x] >= 0) {
         st = a.end_state + (int64_t)a.end_slots[blockIdx.x] * a.end_slot_stride + (int64_t)h * ((int64_t)dim * vdim + dim + 1);
@@ -154,10 +160,10 @@ __global__ __launch_bounds__(256) void mlstm_kernel(pcb_mlstm_args a) {
         const int d = p * DPT + i;
         if (d < dim) {
             if (col) st[(int64_t)d * vdim + j] = S[i];
-            if (blockIdx.z == 0 && lane == 0) st_n[d] = nv[i];
+            if (first && lane == 0) st_n[d] = nv[i];
         }
     }
-    if (blockIdx.z == 0 && tid == 0) {
+    if (first && tid == 0) {
         st_n[dim] = m;
         if (a.log_f_sum) a.log_f_sum[(int64_t)blockIdx.x * a.H + h] = f_sum;
     }
@@ -198,22 +204,24 @@ __global__ __launch_bounds__(256) void mlstm_chain_kernel(const float* __restric
 
 template <typename E>
 int dispatch(const pcb_mlstm_args& a, hipStream_t stream) {
-    const dim3 grid(a.n_reqs, a.H, pcb_ceil_div(a.vdim, 64)), block(256);
-    if (a.out) {
+    auto go = [&](auto dpt, auto nb) {
+        constexpr int DPT = decltype(dpt)::value, NB = decltype(nb)::value;
+        for (int col0 = (a.vdim - 1) / (64 * NB) * (64 * NB); col0 >= 0; col0 -= 64 * NB) {
+            if (a.out)
+                hipLaunchKernelGGL((mlstm_kernel<E, DPT, NB, true>), dim3(a.n_reqs, a.H), dim3(256 * NB), 0, stream, a, col0);
+            else
+                hipLaunchKernelGGL((mlstm_kernel<E, DPT, NB, false>), dim3(a.n_reqs, a.H), dim3(256 * NB), 0, stream, a, col0);
+        }
+    };
+    auto rows = [&](auto nb) {
         if (a.dim <= 64)
-            hipLaunchKernelGGL((mlstm_kernel<E, 16, true>), grid, block, 0, stream, a);
+            go(std::integral_constant<int, 16>{}, nb);
         else if (a.dim <= 128)
-            hipLaunchKernelGGL((mlstm_kernel<E, 32, true>), grid, block, 0, stream, a);
+            go(std::integral_constant<int, 32>{}, nb);
         else
-            hipLaunchKernelGGL((mlstm_kernel<E, 64, true>), grid, block, 0, stream, a);
-    } else {
-        if (a.dim <= 64)
-            hipLaunchKernelGGL((mlstm_kernel<E, 16, false>), grid, block, 0, stream, a);
-        else if (a.dim <= 128)
-            hipLaunchKernelGGL((mlstm_kernel<E, 32, false>), grid, block, 0, stream, a);
-        else
-            hipLaunchKernelGGL((mlstm_kernel<E, 64, false>), grid, block, 0, stream, a);
-    }
+            go(std::integral_constant<int, 64>{}, nb);
+    };
+    a.vdim <= 64 ? rows(std::integral_constant<int, 1>{}) : rows(std::integral_constant<int, 2>{});
     return pcb_check_launch("mlstm_kernel");
 }
 

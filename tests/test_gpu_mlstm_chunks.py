@@ -194,3 +194,34 @@ def test_closed_input_gates_token_by_token(shut, pos0):
     after = f(state[1]).view(H, -1)
     assert near(f(out), want.reshape(n, H * Dv)) and near(after[:, :D * Dv].reshape(H, D, Dv), S) and near(after[:, D * Dv:-1], nv)
     assert torch.allclose(after[:, -1], m, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 2e-5), (torch.bfloat16, 2e-5)])
+@pytest.mark.parametrize("H,D,Dv,R,count", [(8, 16, 128, 200, 3), (16, 40, 70, 80, 9), (4, 136, 200, 96, 2), (3, 8, 300, 24, 1)])
+def test_more_workgroups_than_run_at_once(H, D, Dv, R, count, dtype, tol):
+    """Several blocks of value columns share a head's n and m, which move in place: a block that starts when another one has ended must not see them moved.
+    (Against each request by itself: launches that the chip has room for.)"""
+    from promptcache_amd import _blocks as B
+    n = R * count
+    cols, N, _, _ = layer(H, D, Dv, n, dtype)
+    rec = B.mlstm_state_floats(H, D, Dv)
+    state = rnd(R, rec, seed=3)
+    state.view(R, H, -1)[..., -1] = 0.7
+    ref, out, want = state.clone(), torch.zeros(n, H * Dv, device=DEV), torch.zeros(n, H * Dv, device=DEV)
+    tail = (H, D, Dv, D ** -0.5, 0.0)
+    reqs = [(r, 5, count, r * count) for r in range(R)]
+    B.mlstm(*cols, N, i32(reqs), R, state, *tail, out)
+    for r in reqs:
+        B.mlstm(*cols, N, i32([r]), 1, ref, *tail, want)
+    assert torch.equal(out, want) and torch.equal(state, ref)
+    # ... and a few of them against the recurrence
+    f = lambda t: t.detach().to("cpu", F64)
+    s0, x = rnd(R, rec, seed=3), [f(c) for c in cols]
+    s0.view(R, H, -1)[..., -1] = 0.7
+    for r in (0, R // 2, R - 1):
+        rows, s6 = slice(r * count, (r + 1) * count), f(s0[r]).view(H, -1)
+        o, (S, nv, m) = O.matrix_memory(x[0][rows, :H * D].view(count, H, D) * D ** -0.5, x[1][rows, :H * D].view(count, H, D),
+                                        x[2][rows, :H * Dv].view(count, H, Dv), x[3][rows, :H], torch.nn.functional.logsigmoid(x[4][rows, :H]),
+                                        (s6[:, :D * Dv].reshape(H, D, Dv), s6[:, D * Dv:-1], s6[:, -1]))
+        after = f(state[r]).view(H, -1)
+        assert rel(f(out[rows]), o.reshape(count, H * Dv)) < tol and rel(after[:, :D * Dv].reshape(H, D, Dv), S) < tol and rel(after[:, D * Dv:-1], nv) < tol
