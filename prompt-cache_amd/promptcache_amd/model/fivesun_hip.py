@@ -175,10 +175,10 @@ class FivesunHIP(SlotModel):
     @staticmethod
     def _few_tokens(requests, heads, dim, vdim):
         """Up to how many tokens a request (the longest of the step) the memory is faster token by token.  That costs a fixed time a token until its
-        workgroups (one per request, head and 64 value columns) are more than two a CU; segments cost the same for 2 as for 16 tokens, and in
-        proportion to requests x heads.  us, token by token / in segments, heads of 128: 16 of them 8 tokens 23.0 / 24.6, 10 25.7 / 24.6; 128 13 tokens
-        30.0 / 31.1, 16 33 / 31; 256 20 tokens 40 / 44, 24 44 / 44; 640 9 tokens 82 / 67 (bf16), 1280 13 157 / 166 (fp32); heads of 64: 16 of them 14 tokens
-        20.2 / 20.9, 16 22.0 / 20.9; 320 28 tokens 33 / 36 (fp32), 1024 32 tokens 52 / 62; 128 x 64, 288 of them 22 tokens 41 / 47."""
+        workgroups (one per request and head) are more than fit the chip at once; segments cost the same for 2 as for 16 tokens, and in proportion to
+        requests x heads.  us, token by token / in segments, heads of 128: 16 of them 8 tokens 22.1 / 24.6, 10 25.1 / 24.8; 128 13 tokens 29.2 / 31.3, 16
+        31.5 / 31.3; 256 20 tokens 38.7 / 44.6, 24 42.7 / 44.6; 640 13 85 / 67 (bf16), 1280 13 139 / 167 (fp32); heads of 64: 16 of them 14 tokens
+        20.4 / 21.1, 16 21.7 / 21.1; 320 28 tokens 34 / 36 (fp32), 1024 32 tokens 54 / 76; 128 x 64, 288 of them 22 tokens 41 / 47."""
         n = requests * heads
         if dim <= 64:
             return 15 + n // 24
