@@ -845,11 +845,16 @@ def mlstm_step(cols, ld: int, reqs: torch.Tensor, n_reqs: int, state: torch.Tens
     check(load().pcb_mlstm_step(C.byref(a), C.byref(o), _stream()), "pcb_mlstm_step")
 
 
-def mlstm_prompt_fits(dim: int, vdim: int, ld: int, cols, gate: torch.Tensor, max_tokens: int) -> bool:
-    """Whether ``mlstm_prompt`` takes these sizes and this alignment (``cols`` and ``gate``: column blocks of rows ``ld`` elements apart)."""
-    es = cols[0].element_size()
+def mlstm_prompt_takes(dim: int, vdim: int, ld: int, es: int, cols_at, gate_at: int, max_tokens: int) -> bool:
+    """Whether ``mlstm_prompt`` takes these sizes: q, k, v and the gate lie ``cols_at`` and ``gate_at`` bytes behind a multiple of 16 bytes, rows ``ld``
+    elements of ``es`` bytes apart."""
     return dim <= 128 and vdim <= 128 and dim % 8 == 0 and vdim % 8 == 0 and max_tokens <= 256 and ld * es % 16 == 0 and \
-        all(c.data_ptr() % 16 == 0 for c in cols[:3]) and gate.data_ptr() % (4 * es) == 0
+        all(c % 16 == 0 for c in cols_at) and gate_at % (4 * es) == 0
+
+
+def mlstm_prompt_fits(dim: int, vdim: int, ld: int, cols, gate: torch.Tensor, max_tokens: int) -> bool:
+    """The same of ``cols`` and ``gate`` themselves (column blocks of rows ``ld`` elements apart)."""
+    return mlstm_prompt_takes(dim, vdim, ld, cols[0].element_size(), [c.data_ptr() for c in cols[:3]], gate.data_ptr(), max_tokens)
 
 
 def mlstm_prompt(cols, ld: int, segments: torch.Tensor, n_segments: int, chains: torch.Tensor, n_chains: int, max_tokens: int, end_slots: torch.Tensor,

@@ -187,10 +187,10 @@ class FivesunHIP(SlotModel):
         return min(22, 8 + n * dim * dim // (1 << 18))
 
     def _mlstm_fits(self, l):
-        """Whether an mLSTM layer's columns of the step's projection are what ``B.mlstm_prompt`` takes (16-byte pieces of up to 128 columns)."""
-        n = 2 * l.heads * l.dim + 2 * l.heads * l.vdim + 2 * l.heads + self.W
-        return l.dim <= 128 and l.vdim <= 128 and l.dim % 8 == 0 and l.vdim % 8 == 0 and l.heads % 2 == 0 and \
-            n % (8 if self.dtype == torch.bfloat16 else 4) == 0
+        """Whether an mLSTM layer's columns of the step's projection (q | k | v | i | f | gate | residual gate) are what ``B.mlstm_prompt`` takes."""
+        HD, HV, es = l.heads * l.dim, l.heads * l.vdim, 2 if self.dtype == torch.bfloat16 else 4
+        gate = 2 * HD + HV + 2 * l.heads
+        return B.mlstm_prompt_takes(l.dim, l.vdim, gate + HV + self.W, es, (0, es * HD, 2 * es * HD), es * gate, 1)
 
     # ---- cache and state -------------------------------------------------------------------------------------------------------
     def new_arena(self, slots: int, cap: int) -> SlotArena:

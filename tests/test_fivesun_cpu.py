@@ -358,3 +358,22 @@ def test_oracle_gated_sublayer_and_feed_forward():
 def test_few_tokens_go_through_the_matrix_memory_one_by_one(requests, heads, dim, vdim, tokens, segments):
     from promptcache_amd.model.fivesun_hip import FivesunHIP
     assert (tokens > FivesunHIP._few_tokens(requests, heads, dim, vdim)) == segments
+
+
+@pytest.mark.parametrize("heads,dim,vdim,width,dtype,fits", [
+    (16, 128, 128, 2048, torch.bfloat16, True), (16, 128, 128, 2048, torch.float32, True), (2, 16, 24, 64, torch.float32, True), (2, 16, 24, 64, torch.bfloat16, False),
+    (3, 128, 128, 2048, torch.bfloat16, False), (4, 136, 64, 512, torch.bfloat16, False), (4, 64, 60, 512, torch.float32, False), (4, 64, 64, 508, torch.bfloat16, False)])
+def test_layers_and_calls_share_the_rule_of_what_goes_in_segments(heads, dim, vdim, width, dtype, fits):
+    """What a model decides from a layer's sizes is what the call says of the same columns."""
+    from types import SimpleNamespace
+    from promptcache_amd import _blocks as B
+    from promptcache_amd.model.fivesun_hip import FivesunHIP
+    layer = FivesunLayer("mlstm", heads=heads, kv_heads=heads, dim=dim, vdim=vdim, ff=16)
+    assert FivesunHIP._mlstm_fits(SimpleNamespace(dtype=dtype, W=width), layer) == fits
+    at = [0, heads * dim, 2 * heads * dim]
+    gate = 2 * heads * dim + heads * vdim + 2 * heads
+    n = gate + heads * vdim + width
+    es = torch.empty(0, dtype=dtype).element_size()
+    mem = torch.empty(2 * n + 16, dtype=dtype)
+    mem = mem[(-mem.data_ptr() % 16) // es:]
+    assert B.mlstm_prompt_fits(dim, vdim, n, [mem[a:] for a in at], mem[gate:], 64) == fits
