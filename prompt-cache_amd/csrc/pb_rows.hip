@@ -70,17 +70,15 @@ __device__ __forceinline__ void row_sum(float (&v)[NV], float* red) {
 }
 __device__ __forceinline__ f4 ld4(const float* p) { return *reinterpret_cast<const f4*>(p); }
 
-// Threads and four-column chunks per thread of a kernel that holds a row of `width` columns in registers; false: too wide.  Few rows (decoding)
-// are one chunk per thread wherever 1024 threads reach: such a launch lasts as long as one row's chain.  Many rows fill the chip anyhow, and 256
-// threads with more chunks each have fewer waves to meet at the barriers.
+// Threads and four-column chunks per thread (one, two, four, .. up to max_chunks: what a kernel's registers hold for 1024 threads) of a kernel that holds
+// a row of `width` columns in registers; false: too wide.  Few rows (decoding) are one chunk per thread wherever 1024 threads reach: such a launch
+// lasts as long as one row's chain.  Many rows fill the chip anyhow, and fewer threads with more chunks each have fewer waves to meet at the barriers.
 inline bool row_threads(int width, int n_rows, int max_chunks, int* threads, int* chunks) {
-    const int pieces = width / 4;
-    int t = n_rows <= 512 || pieces > 256 * max_chunks ? 1024 : 256;
-    if (pieces < t) t = (pieces + 63) / 64 * 64;
+    const int pieces = width / 4, t0 = n_rows <= 512 ? 1024 : 256;
     int c = 1;
-    while (c * t < pieces) c *= 2;
-    *threads = t, *chunks = c;
-    return width % 4 == 0 && c <= max_chunks;
+    while (c * t0 < pieces && c < max_chunks) c *= 2;
+    *threads = (pieces + 64 * c - 1) / (64 * c) * 64, *chunks = c;
+    return width % 4 == 0 && *threads <= 1024;
 }
 
 template <typename E>
@@ -91,8 +89,9 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(const E* __restrict__ t
     id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
     const E* src = table + (int64_t)id * width;
     float* dst = out + (int64_t)r * width;
-    // (eight columns a thread where the rows are whole 16-byte pieces: 1 row of 2048 bf16 2.6 us one by one, 2.2 so; 2400 rows 7.9, 6.9)
-    if (width % 8 == 0 && ((uintptr_t)table | (uintptr_t)out) % 16 == 0) {
+    // (eight columns a thread where the rows are whole 16-byte pieces and give every thread some: 1 row of 2048 bf16 2.6 us one by one, 2.2 so; 2400 rows
+    // 7.9, 6.9; 4096 rows of 1024 6.2, 6.9)
+    if (width >= 2048 && width % 8 == 0 && ((uintptr_t)table | (uintptr_t)out) % 16 == 0) {
         for (int c = 8 * threadIdx.x; c < width; c += 2048) {
             const Frag<E> v = load8(src + c);
             store4(dst + c, scale * at8(v, 0), scale * at8(v, 1), scale * at8(v, 2), scale * at8(v, 3));
@@ -375,17 +374,15 @@ PCB_EXPORT int pcb_mix_norm(const pcb_mix_norm_args* a, void* stream) {
                 "pcb_mix_norm: null pointer");
     const uintptr_t e4 = a->dtype == PCB_BF16 ? 8 : 16;              // (four elements of E)
     int th, nc;
-    if (row_threads(a->width, a->n_rows, 4, &th, &nc) && a->hist_stride % 4 == 0 &&
+    if (row_threads(a->width, a->n_rows, 2, &th, &nc) && a->hist_stride % 4 == 0 &&
         ((uintptr_t)a->hist | (uintptr_t)a->x_out | (uintptr_t)a->gain1 | (uintptr_t)a->gain2) % 16 == 0 &&
         ((uintptr_t)a->out1 | (uintptr_t)a->out2) % e4 == 0) {
         auto go = [&](auto e) {
             using E = decltype(e);
             if (nc == 1)
                 hipLaunchKernelGGL((mix_norm_chunks_kernel<E, 1>), dim3(a->n_rows), dim3(th), 0, (hipStream_t)stream, *a);
-            else if (nc == 2)
-                hipLaunchKernelGGL((mix_norm_chunks_kernel<E, 2>), dim3(a->n_rows), dim3(th), 0, (hipStream_t)stream, *a);
             else
-                hipLaunchKernelGGL((mix_norm_chunks_kernel<E, 4>), dim3(a->n_rows), dim3(th), 0, (hipStream_t)stream, *a);
+                hipLaunchKernelGGL((mix_norm_chunks_kernel<E, 2>), dim3(a->n_rows), dim3(th), 0, (hipStream_t)stream, *a);
         };
         if (a->dtype == PCB_BF16) go(bf16_t{}); else go(0.0f);
         return pcb_check_launch("mix_norm_chunks_kernel");
@@ -734,7 +731,8 @@ __global__ __launch_bounds__(1024) void post_norm_kernel(pcb_post_norm_args a) {
 
 // The same with the row in registers (width % 4 == 0, every row aligned to chunks of four columns): both halves' operands are requested before
 // the first sum.  us, column by column through LDS (three dependent trips to memory) and so: 8 rows of 2048 7.2 and 4.6, 2400 rows
-// 23.6 and 16.1 (79 MB: the copy rate).
+// 23.6 and 16.1 (79 MB: the copy rate), 2048 rows of 4096 33.6 and 28.3 (four chunks a thread do not fit the registers: 45.0).  Rows beyond 8192 columns take the
+// kernel above (300 rows of 12288 19.6, 34.1 in four chunks).
 template <typename E, int NC>
 __global__ __launch_bounds__(1024) void post_norm_chunks_kernel(pcb_post_norm_args a) {
     __shared__ float red[3][16];
@@ -1063,17 +1061,15 @@ PCB_EXPORT int pcb_post_norm(const pcb_post_norm_args* a, void* stream) {
                 "pcb_post_norm: pairs need their weights and their number per row; output rows may not overlap");
     const uintptr_t e4 = a->dtype == PCB_BF16 ? 8 : 16;              // (four elements of E)
     int th, nc;
-    if (row_threads(a->width, a->n_rows, 4, &th, &nc) && (!a->gate || a->ldg % 4 == 0) && a->ldo % 4 == 0 &&
+    if (row_threads(a->width, a->n_rows, 2, &th, &nc) && (!a->gate || a->ldg % 4 == 0) && a->ldo % 4 == 0 &&
         ((uintptr_t)a->x | (uintptr_t)a->y | (uintptr_t)a->add | (uintptr_t)a->pair | (uintptr_t)a->post_gain | (uintptr_t)a->gain |
          (uintptr_t)a->bias | (uintptr_t)a->x_out) % 16 == 0 && ((uintptr_t)a->gate | (uintptr_t)a->out) % e4 == 0) {
         auto go = [&](auto e) {
             using E = decltype(e);
             if (nc == 1)
                 hipLaunchKernelGGL((post_norm_chunks_kernel<E, 1>), dim3(a->n_rows), dim3(th), 0, (hipStream_t)stream, *a);
-            else if (nc == 2)
-                hipLaunchKernelGGL((post_norm_chunks_kernel<E, 2>), dim3(a->n_rows), dim3(th), 0, (hipStream_t)stream, *a);
             else
-                hipLaunchKernelGGL((post_norm_chunks_kernel<E, 4>), dim3(a->n_rows), dim3(th), 0, (hipStream_t)stream, *a);
+                hipLaunchKernelGGL((post_norm_chunks_kernel<E, 2>), dim3(a->n_rows), dim3(th), 0, (hipStream_t)stream, *a);
         };
         if (a->dtype == PCB_BF16) go(bf16_t{}); else go(0.0f);
         return pcb_check_launch("post_norm_chunks_kernel");

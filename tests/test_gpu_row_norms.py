@@ -59,3 +59,9 @@ def test_rows_held_in_registers(rows, width, dtype, tol):
     z = f(x0)
     want = f(c)[0] * unit(z, eps) + f(c)[1] * unit(z ** 2, eps) + f(c)[2] * unit(z ** 3, eps) + f(c)[3]
     assert rel(out, want) < tol
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-6), (torch.bfloat16, 2.0 ** -8)])
+@pytest.mark.parametrize("rows,width", [(2, 4224), (2, 8192), (2, 8196), (2, 12288), (515, 3072), (513, 4100), (514, 5128), (513, 8192), (513, 8200)])
+def test_rows_of_two_chunks_a_thread_and_wider(rows, width, dtype, tol):
+    test_rows_held_in_registers(rows, width, dtype, tol)
