@@ -643,6 +643,7 @@ typedef struct pcb_attn_prompt_args {
     int32_t gate_cols;
     int32_t slots;
     int64_t k_slot_stride, v_slot_stride;
+    int32_t longest; /* (0: unknown; may be left out of struct_bytes) last position + 1 of the tile that ends last: speed alone depends on it */
 } pcb_attn_prompt_args;
 int pcb_attn_prompt(const pcb_attn_prompt_args* a, void* stream);
 

@@ -12,6 +12,8 @@
 // shared by all heads (one rotated part per token): they are then fetched from rows of their own, through an index table if given.
 // Keys and values may also lie in a slot's cache, and a query may see its window or its block of positions only.
 // Workgroups of one head are neighbours eight apart in launch order: they share that head's keys and values in one XCD's L2.
+#include <cstddef>
+#include <cstring>
 #include <type_traits>
 
 #include "pb_attn_common.h"
@@ -39,8 +41,10 @@ __device__ __forceinline__ int oldest(const pcb_attn_prompt_args& a, int i) {
 }
 
 // KSQ: 32-element k-steps of the key size; VB: 16-column blocks of the value size; BK: keys per block
+// (192 key columns in bf16: two waves a SIMD and their registers, not three -- a tile's loads lie further ahead)
 template <typename E, int KSQ, int VB, int QT, int BK, int KG>
-__global__ __launch_bounds__(64 * PW * KG) void attn_prompt_kernel(pcb_attn_prompt_args a) {
+__global__ __launch_bounds__(64 * PW * KG) __attribute__((amdgpu_waves_per_eu(1, sizeof(E) == 2 && KSQ == 6 && QT == 1 && KG == 1 ? 2 : 8)))
+void attn_prompt_kernel(pcb_attn_prompt_args a) {
     constexpr int CE = 16 / sizeof(E);
     constexpr int KC = KSQ * 32, VC = VB * 16;                       // columns of the tiles
     constexpr int KLD = KC + CE, VLD = v_ld<E>(VC);
@@ -284,6 +288,22 @@ __global__ __launch_bounds__(64 * PW * KG) void attn_prompt_kernel(pcb_attn_prom
     }
 }
 
+// Two halves where the longest tile's chain of key blocks is what a launch takes (2.3 us a block of 64), that is where tiles are long and the chip has a CU for
+// every tile and head.  With up to two of them a CU only where some tiles are much longer than others, that is not where a window cuts all of them alike; beyond,
+// a CU is better off with workgroups of four waves, and tiles of a few blocks pay for the second half without using it.  us, one half / two, bf16, 128
+// columns: 16 heads, 64 rows 7.4 / 8.5, 150 rows 10.8 / 10.8, 300 16.3 / 14.9, 600 24 / 17, 1024 36 / 26, 2048 46 / 35, 2048 with a window of 256 20.7 / 25.9; 32 x 64 rows
+// 10.0 / 14.9; 8 heads 16 x 200 rows 14.8 / 20.3, 3 x 700 (264 workgroups) 27 / 23, 8 x 300 (320) 17.2 / 19.8; 192 columns, 8 heads, 2048 rows 44 / 33; fp32 8 heads,
+// 64 rows 13.8 / 16.9, 300 rows 35 / 35, 600 60 / 55, 2048 rows 105 / 94, 16 heads 170 / 116.
+bool two_halves(const pcb_attn_prompt_args& a, int bk) {
+    const int64_t wgs = (int64_t)a.H * a.n_tiles;
+    const bool alike = a.window > 0 && a.longest > a.window + a.tile_rows;
+    int seen = alike ? a.window + a.tile_rows : a.longest;
+    if (a.block > 0 && a.block < seen) seen = a.block;
+    const int blocks = pcb_ceil_div(seen, bk);
+    const bool bf = a.dtype == PCB_BF16;
+    return wgs <= 256 ? blocks >= (bf ? 4 : 10) : wgs <= 512 && !alike && blocks >= (bf ? 10 : 17);
+}
+
 template <typename E, int KSQ, int VB, int BK>
 int launch(const pcb_attn_prompt_args& a, hipStream_t stream) {
     const dim3 grid(a.H, a.n_tiles);
@@ -298,13 +318,8 @@ int launch(const pcb_attn_prompt_args& a, hipStream_t stream) {
             go(Two{}, One{});
             return pcb_check_launch("attn_prompt_kernel");
         }
-    // Two halves while the chip has a CU for every tile and head, keys of up to 128 columns also two of them (the longest tile's chain of blocks is what a
-    // launch takes: 2.3 us a block of 64); beyond, a CU is better off with workgroups of four waves.  us, one half / two, bf16: 16 heads of 128, 1024 rows
-    // 36 / 26, 600 rows 24 / 17, 2048 rows in blocks of 1024 (512 workgroups) 46 / 35, 8 x 300 rows (640) 20 / 29, 5000 rows 205 / 296; 192-column keys,
-    // 8 heads, 2048 rows 44 / 33, 16 heads 54 / 65; fp32, 8 heads: 2 x 300 rows 36 / 34, 2048 rows 105 / 94, 16 heads 170 / 116.
-    const int64_t wgs = (int64_t)a.H * a.n_tiles;
     if constexpr (VB <= 8) {
-        if (wgs <= (KSQ <= 4 ? 512 : 256)) {
+        if (two_halves(a, BK)) {
             go(One{}, Two{});
             return pcb_check_launch("attn_prompt_kernel");
         }
@@ -324,8 +339,12 @@ int dispatch(const pcb_attn_prompt_args& a, hipStream_t stream) {
 
 }  // namespace
 
-PCB_EXPORT int pcb_attn_prompt(const pcb_attn_prompt_args* a, void* stream) {
-    PCB_REQUIRE(a && a->struct_bytes == sizeof(pcb_attn_prompt_args), PCB_ERR_ARG, "pcb_attn_prompt: struct size mismatch");
+PCB_EXPORT int pcb_attn_prompt(const pcb_attn_prompt_args* given, void* stream) {
+    PCB_REQUIRE(given && (given->struct_bytes == sizeof(pcb_attn_prompt_args) || given->struct_bytes == offsetof(pcb_attn_prompt_args, longest)), PCB_ERR_ARG,
+                "pcb_attn_prompt: struct size mismatch");
+    pcb_attn_prompt_args whole = {};
+    std::memcpy(&whole, given, given->struct_bytes);
+    const pcb_attn_prompt_args* const a = &whole;
     PCB_REQUIRE(a->dtype == PCB_BF16 || a->dtype == PCB_F32, PCB_ERR_ARG, "pcb_attn_prompt: unknown dtype");
     PCB_REQUIRE(a->n_tiles >= 0 && a->n_tiles <= 65535 && a->H > 0 && a->Hkv > 0 && a->H % a->Hkv == 0 && a->dim > 0 && a->dim <= 256 &&
                     a->vdim > 0 && a->vdim <= 256 && a->tail_dim >= 0 && a->tail_dim < a->dim && a->ldq >= (int64_t)a->H * a->dim &&

@@ -151,7 +151,7 @@ class AttnPromptArgs(C.Structure):
                 ("v", _vp), ("v_row_stride", _i64), ("v_head_stride", _i64),
                 ("H", _i32), ("Hkv", _i32), ("dim", _i32), ("vdim", _i32), ("scale", _f32), ("window", _i32),
                 ("sink", _vp), ("gate", _vp), ("ldg", _i64), ("out", _vp), ("ldo", _i64),
-                ("block", _i32), ("gate_cols", _i32), ("slots", _i32), ("k_slot_stride", _i64), ("v_slot_stride", _i64)]
+                ("block", _i32), ("gate_cols", _i32), ("slots", _i32), ("k_slot_stride", _i64), ("v_slot_stride", _i64), ("longest", _i32)]
 
 
 class AttnLatentArgs(C.Structure):
@@ -903,10 +903,11 @@ def gla(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ld: torch.Tensor, lds
 def attn_prompt(q: torch.Tensor, tiles: torch.Tensor, n_tiles: int, tile_rows: int, k: torch.Tensor, k_strides, v: torch.Tensor, v_strides,
                 H: int, Hkv: int, dim: int, vdim: int, scale: float, out: torch.Tensor, *, ldo: int, ldq: Optional[int] = None, k_tail=None,
                 tail_row_stride: int = 0, tail_rows=None, tail_dim: int = 0, window: int = 0, sink=None, gate=None, ldg: int = 0,
-                block: int = 0, gate_cols: bool = False) -> None:
+                block: int = 0, gate_cols: bool = False, longest: int = 0) -> None:
     """``k_strides`` / ``v_strides``: (row, head) strides in elements of the key and value rows -- or (row, head, slot) strides: the tiles
     then name slots; ``tail_rows``: int32 row of ``k_tail`` per key row; ``gate``: E, one number per row and head (or, ``gate_cols``, per
-    element); ``block`` > 0: a key is seen inside the query's own block of that many positions only."""
+    element); ``block`` > 0: a key is seen inside the query's own block of that many positions only; ``longest``: positions up to the last
+    query's, where the caller knows (few tiles over long contexts go faster then)."""
     _want(tiles, torch.int32, "attn_prompt tiles"); _want(sink, torch.float32, "attn_prompt sink"); _want(tail_rows, torch.int32, "attn_prompt tail_rows")
     assert q.dtype == k.dtype == v.dtype == out.dtype and q.is_cuda and k.is_cuda and v.is_cuda and out.is_cuda
     ldq = q.shape[-1] if ldq is None else ldq
@@ -918,7 +919,7 @@ def attn_prompt(q: torch.Tensor, tiles: torch.Tensor, n_tiles: int, tile_rows: i
     a = AttnPromptArgs(C.sizeof(AttnPromptArgs), _code(q), _p(q), ldq, _p(tiles), n_tiles, tile_rows, _p(k), k_strides[0], k_strides[1],
                        _p(k_tail), tail_row_stride, _p(tail_rows), tail_dim, _p(v), v_strides[0], v_strides[1], H, Hkv, dim, vdim, float(scale),
                        int(window), _p(sink), _p(gate), ldg, _p(out), ldo, int(block), int(gate_cols), int(slots), k_strides[2] if slots else 0,
-                       v_strides[2] if slots else 0)
+                       v_strides[2] if slots else 0, int(longest))
     check(load().pcb_attn_prompt(C.byref(a), _stream()), "pcb_attn_prompt")
 
 

@@ -346,6 +346,7 @@ class FivesunHIP(SlotModel):
         for k, (g, d) in enumerate(self._sigs):
             np.add(st.row_slot * (g * cap * d), st.row_pos * d, out=offs[k])
         dims = dict(T=T, R=R, n_want=int(want_rows.size), n32=n32, o64=o64, sizes=sizes, tile=tile, ones=max(counts) == 1,
+                    longest=max((starts[b] + counts[b] for b in {*big, *rebuilt}), default=0),
                     seg=min(seg, max(counts)) if chunks else 0)
         res = self._decode_graphed(arena, blob, dims) if graphed else None
         if res is None:
@@ -361,7 +362,8 @@ class FivesunHIP(SlotModel):
     def _tables(self, dblob, d):
         i32 = dblob[:d["n32"] * 4].view(torch.int32)
         sizes = d["sizes"]
-        at, out = 0, dict(tile=d["tile"], ones=d["ones"], seg=d["seg"], n_seg=sizes.get("seg_end", 0), n_chains=sizes.get("chains", 0) // 4)
+        at, out = 0, dict(tile=d["tile"], longest=d["longest"], ones=d["ones"], seg=d["seg"], n_seg=sizes.get("seg_end", 0),
+                           n_chains=sizes.get("chains", 0) // 4)
         for name, n in sizes.items():
             out[name] = i32[at:at + n]
             at += n
@@ -463,7 +465,8 @@ class FivesunHIP(SlotModel):
             kw = dict(ldo=H * Dv, block=l.mask, sink=lw["sink"], gate=gate, ldg=N)
             n = tb["p_tiles"].numel() // 4
             if n:
-                B.attn_prompt(q, tb["p_tiles"], n, tb["tile"], plane, (rs, hs, ss), values, (rs, hs, ss), H, G, D, Dv, l.scale, att, **kw)
+                B.attn_prompt(q, tb["p_tiles"], n, tb["tile"], plane, (rs, hs, ss), values, (rs, hs, ss), H, G, D, Dv, l.scale, att,
+                              longest=tb["longest"], **kw)
             n = tb["s_tiles"].numel() // 4
             if n:
                 splits = self._splits(n, G * -(-H // (16 * G)), H, reach, 768 if max(D, Dv) <= 128 else 512)
@@ -522,7 +525,7 @@ class FivesunHIP(SlotModel):
                 qh, oh, gh = (q, og, gate) if not h0 else (q[:, h0 * DR:], og[:, h0 * Dv:], gate[:, h0 * Dv:])
                 B.attn_prompt(qh, tb["l_tiles"], tb["l_tiles"].numel() // 4, tb["tile"], kv, (Hs * ew, D), kv[:, n_h * D:], (Hs * ew, Dv),
                               n_h, n_h, DR, Dv, l.scale, oh, ldq=HQ, ldo=HV, k_tail=flat[:, C:] if Rd else None, tail_row_stride=CR,
-                              tail_rows=tb["kv_rows"], tail_dim=Rd, window=l.mask, gate=gh, ldg=N, gate_cols=True)
+                              tail_rows=tb["kv_rows"], tail_dim=Rd, window=l.mask, gate=gh, ldg=N, gate_cols=True, longest=tb["longest"])
         B.linear(og, lw["wo"], y, M=T)
         return P[:, HQ + CR + HV:], N
 

@@ -195,7 +195,8 @@ class PikadraHIP(SlotModel):
         blob = np.empty(o64 + offs.size * 8, dtype=np.uint8)
         blob[:n32 * 4].view(np.int32)[:] = np.concatenate([v.reshape(-1) for v in tables.values()])
         blob[o64:].view(np.int64)[:] = offs.reshape(-1)
-        dims = dict(T=T, R=st.R, n_want=int(want_rows.size), n32=n32, o64=o64, sizes=sizes, tile=tile)
+        dims = dict(T=T, R=st.R, n_want=int(want_rows.size), n32=n32, o64=o64, sizes=sizes, tile=tile,
+                    longest=max((st.starts[b] + st.counts[b] for b in big), default=0))
         res = self._decode_graphed(arena, blob, dims) if graphed else None
         if res is None:
             dblob = torch.from_numpy(blob).to(dev)
@@ -222,7 +223,7 @@ class PikadraHIP(SlotModel):
         dev, E, f32 = self.device, self.dtype, torch.float32
         W, T = self.W, d["T"]
         tb = self._tables(dblob, d)
-        tb["tile"] = d["tile"]
+        tb["tile"], tb["longest"] = d["tile"], d["longest"]
         runs = self.runs if num_layers is None else self.runs[:num_layers]
         cfg, eps = self.config, self.config.norm_eps
         x = self._mat("x", T, W, f32)
@@ -316,7 +317,7 @@ class PikadraHIP(SlotModel):
         B.linear(flat, lw["w_kv"], kv, M=M, row_src=tb["kv_rows"], ldx=CR)
         B.attn_prompt(q, tb["p_tiles"], tb["p_tiles"].numel() // 4, tb["tile"], kv, (NK, D), kv[:, H * D:], (NK, Dv), H, H, D + R, Dv, l.scale, A,
                       ldo=ldo, k_tail=flat[:, C:] if R else None, tail_row_stride=CR, tail_rows=tb["kv_rows"], tail_dim=R, sink=lw["sink"],
-                      gate=gate, ldg=ldg)
+                      gate=gate, ldg=ldg, longest=tb["longest"])
 
     def _folded(self, arena, r, lw, q, A, ldo, gate, ldg, tb, tiles, n, rows, T, rot, turned):
         E, l = self.dtype, lw["cfg"]

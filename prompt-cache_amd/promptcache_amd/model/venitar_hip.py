@@ -224,7 +224,8 @@ class VenitarHIP(SlotModel):
         blob = np.empty(o64 + offs.size * 8 + 8, dtype=np.uint8)
         blob[:n32 * 4].view(np.int32)[:] = np.concatenate([v.reshape(-1) for v in tables.values()])
         blob[o64:o64 + offs.size * 8].view(np.int64)[:] = offs.reshape(-1)
-        dims = dict(T=T, R=R, n_want=int(want_rows.size), n32=n32, o64=o64, sizes=sizes, tile=tile, single=single)
+        dims = dict(T=T, R=R, n_want=int(want_rows.size), n32=n32, o64=o64, sizes=sizes, tile=tile, single=single,
+                    longest=max((st.starts[b] + st.counts[b] for b in big), default=0))
         res = self._decode_graphed(arena, blob, dims) if graphed else None
         if res is None:
             dblob = torch.from_numpy(blob).to(dev)
@@ -238,7 +239,7 @@ class VenitarHIP(SlotModel):
 
     def _tables(self, dblob, d):
         i32 = dblob[:d["n32"] * 4].view(torch.int32)
-        at, out = 0, dict(tile=d["tile"], single=d["single"], R=d["R"])
+        at, out = 0, dict(tile=d["tile"], longest=d["longest"], single=d["single"], R=d["R"])
         for name, n in d["sizes"].items():
             out[name] = i32[at:at + n]
             at += n
@@ -356,7 +357,7 @@ class VenitarHIP(SlotModel):
         n = tb["p_tiles"].numel() // 4
         if n:
             B.attn_prompt(q, tb["p_tiles"], n, tb["tile"], plane, (rs, hs, ss), values, (rs, hs, ss), H, G, D, Dv, a.scale, out,
-                          gate_cols=kw.get("gate") is not None, **kw)
+                          gate_cols=kw.get("gate") is not None, longest=tb["longest"], **kw)
         n = tb["s_tiles"].numel() // 4
         if n:
             # few (row, key head) pairs cannot fill the chip: each is cut into runs of its keys, as many as the visible blocks of 64 allow

@@ -41,3 +41,14 @@ def test_both_sides_of_the_split(rows, H, block, window, dim, vdim, dtype, tol):
             w = torch.softmax(torch.cat([w, sink[h].to(F64).expand(n, 1)], 1), -1)[:, :n]
             want, got = w @ V[:, h // 2], out[s:s + n, h * vdim:(h + 1) * vdim].to(F64)
             assert float((got - want).norm() / want.norm()) < tol, (s, h)
+
+
+# (`longest` decides who shares a tile's blocks: what the launch is told of a longer context than there is changes its speed alone)
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 3e-6), (torch.bfloat16, 4e-3)])
+@pytest.mark.parametrize("dim,vdim", [(128, 128), (64, 64), (192, 128), (100, 60)])
+@pytest.mark.parametrize("rows,H,block,window", [([1, 63, 64, 65, 130], 4, 0, 0), ([600], 4, 512, 0), ([600], 4, 0, 300), ([600] * 3, 16, 0, 0), ([600] * 3, 24, 0, 0)])
+def test_two_halves_of_a_tile(rows, H, block, window, dim, vdim, dtype, tol, monkeypatch):
+    import functools
+    from promptcache_amd import _blocks as B
+    monkeypatch.setattr(B, "attn_prompt", functools.partial(B.attn_prompt, longest=2000))
+    test_both_sides_of_the_split(rows, H, block, window, dim, vdim, dtype, tol)

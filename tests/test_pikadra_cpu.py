@@ -282,3 +282,14 @@ def test_blocks_reject_bad_arguments_on_the_host():
     assert linear(split_n=2, y2=16, y2_f32=1, head_stride2=1) == -2001 and b"split destination" in err()
     p = b.PostNormArgs(struct_bytes=ctypes.sizeof(b.PostNormArgs), x=16, eps=1e-6, n_rows=2, width=8, y_scale=1.0, pair=16)
     assert lb.pcb_post_norm(ctypes.byref(p), None) == -2001 and b"pairs" in err()
+
+
+def test_prompt_attention_takes_arguments_without_their_last_field():
+    """``longest`` was appended: callers that do not know it leave it out of ``struct_bytes``."""
+    from promptcache_amd import _blocks as b
+    lb, size = b.load(build_missing=False), ctypes.sizeof(b.AttnPromptArgs)
+    for n, taken in ((size, True), (b.AttnPromptArgs.longest.offset, True), (size - 4, False), (size + 8, False)):
+        a = b.AttnPromptArgs(struct_bytes=n, ldq=48, n_tiles=1, tile_rows=64, k_row_stride=48, k_head_stride=24, v_row_stride=48, v_head_stride=24, H=2,
+                             Hkv=2, dim=24, vdim=24, scale=1.0, ldo=48)
+        assert lb.pcb_attn_prompt(ctypes.byref(a), None) == -2001
+        assert (b"null pointer" if taken else b"struct size") in lb.pcb_last_error_string()
