@@ -694,9 +694,11 @@ FewRows few_rows(const pcb_linear_args& a) {
         if (hole) return one;
     }
     // ... and while the chip has places for them: accumulations in bf16 8 rows, 4096 x 1024 5.6 / 4.9 / 5.1, 8192 x 1024 6.7 / 7.0 / 7.5, 8192 x 2048 10.8 / 11.7 /
-    // 11.5; stores in bf16 at any size (32000 x 2048, 1 row 30.0 / 27.8 / 23.6, 4 rows 31.8 / 30.2 / 28.8); fp32, K = 2048, 4 rows, 8192 columns 20.1 / 17.3 /
-    // 17.5, 8 rows, 6144 20.4 / 16.9 / 15.8, 8192 21.8 / 18.1 / 19.9; 4 rows added, K = 512, 4096 columns 5.7 / 5.0 / 5.2, 8192 7.3 / 6.4 / 6.9
-    const int64_t most = bf ? (!add ? INT64_MAX : a.K < 2048 ? 640 : a.M > 4 ? 768 : INT64_MAX) : add && a.K < 1024 ? 640 : a.M <= 4 ? 1024 : 768;
+    // 11.5; stores in bf16 up to six rows at any size (32000 x 2048, 1 row 30.0 / 27.8 / 23.6, 5 rows 32.1 / 31.1 / 29.8, 8 rows 34.3 / 34.6 / 35.1), in fp32 two (2 rows
+    // 33.7 / 27.0 / 26.4); fp32, K = 2048, 4 rows, 8192 columns 20.1 / 17.3 / 17.5, 8 rows, 6144 20.4 / 16.9 / 15.8, 8192 21.8 / 18.1 / 19.9; 4 rows added, K = 512, 4096
+    // columns 5.7 / 5.0 / 5.2, 8192 7.3 / 6.4 / 6.9
+    const bool any = bf ? (add ? a.K >= 2048 && a.M <= 4 : gated || a.M <= 6) : a.epilogue == PCB_EPI_STORE && a.M <= 2;
+    const int64_t most = any ? INT64_MAX : add ? (a.K < (bf ? 2048 : 1024) ? 640 : bf || a.M > 4 ? 768 : 1024) : bf || a.M <= 4 ? 1024 : 768;
     return g2 <= most ? FewRows{2, late} : one;
 }
 
