@@ -575,7 +575,7 @@ PCB_EXPORT int pcb_attn_talk(const pcb_attn_talk_args* a, void* stream) {
     PCB_REQUIRE(a->scratch_floats >= (int64_t)a->n_tiles * 16 * a->H * band, PCB_ERR_ARG,
                 "pcb_attn_talk: scratch holds %lld floats, %lld needed", (long long)a->scratch_floats,
                 (long long)a->n_tiles * 16 * a->H * band);
-    // (every size measured is faster there: 100 rows 30 -> 18 us, 2048 rows 111 -> 72; tiles of at most four rows have a values kernel of their own)
+    // (every size measured is faster there: 100 rows 30 -> 18 us, 2048 rows 111 -> 69; tiles of at most four rows have a values kernel of their own)
     if ((a->max_tile_rows <= 0 || a->max_tile_rows > FEW_ROWS) && pcb_talk_prompt_fits(*a)) return pcb_talk_prompt(*a, (hipStream_t)stream);
     return a->dtype == PCB_BF16 ? run<pcb::bf16_t>(*a, band, (hipStream_t)stream) : run<float>(*a, band, (hipStream_t)stream);
 }

@@ -661,7 +661,7 @@ int launch(const pcb_linear_args& a, hipStream_t stream) {
 
 // Which kernel takes a launch of up to sixteen rows: parts runs of k side by side in linear_parts_kernel (0: linear_skinny_kernel), late: where results
 // go is worked out behind the products.  Measured with weights from memory at 4067 points, 64 .. 32000 columns, K = 64 .. 8192, 1 to 16 rows, every
-// epilogue, both types: on average 1.2 % behind the fastest of them all, nowhere more than 8 % behind linear_skinny_kernel.  us below: linear_skinny_kernel /
+// epilogue, both types: on average 1.3 % behind the fastest of them all, nowhere more than 8 % behind linear_skinny_kernel.  us below: linear_skinny_kernel /
 // one run / two / four, the faster of late and not.  (g1, g2, g4: workgroups of 16, 8 and 4 columns.)
 struct FewRows {
     int parts;
