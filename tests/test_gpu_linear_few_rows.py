@@ -69,7 +69,7 @@ def test_few_rows_of_a_batch(M, N, K, n, dtype):
 # sizes on both sides of the rule's other borders: one run late and not, a deep k of few and of many columns, four runs' and two runs' last sizes
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("M", [2, 4, 7, 12])
-@pytest.mark.parametrize("N,K", [(12300, 64), (12300, 96), (8250, 480), (8200, 512), (6200, 960), (2600, 4096), (4100, 4096), (8300, 4096)])
+@pytest.mark.parametrize("N,K", [(12300, 64), (12300, 96), (8250, 480), (8200, 512), (8200, 1024), (6200, 960), (2600, 4096), (4100, 4096), (8300, 4096)])
 def test_few_rows_at_the_rules_other_borders(M, N, K, dtype):
     b, f = B(), lambda t: t.to(F64)
     low = 1e-6 if dtype == torch.float32 else 2.0 ** -8
