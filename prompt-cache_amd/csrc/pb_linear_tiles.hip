@@ -1,8 +1,8 @@
-// pb_linear over many rows in bf16: mfma_f32_32x32x16_bf16, four waves (2 x 2) in tiles of 128 or 256 rows x 128, 192 or 256 columns with a whole CU's
-// LDS for their ring, main loop and staging order in mfma_tile_loop.h.
+// pb_linear over many rows in bf16: four waves (2 x 2) in tiles of 128 or 256 rows x 128, 192 or 256 columns with a whole CU's
+// LDS for their ring, main loop and staging order in mfma_tile_loop.h (16 x 16 MFMA blocks, 32 x 32 in the 128 x 128 tiles).
 //
-// What bounds it: at one round of 128 x 128 tiles LDS bandwidth (a wave of 64 x 64 reads as many bytes as its MFMAs take cycles) and the
-// barrier of every K-step, at the larger tiles power.  Against linear_dma_kernel (pb_linear.hip: 16 x 16 MFMAs, two or three images, two
+// What bounds it: power (at 128 x 128 LDS bandwidth nearly as much: a wave of 64 x 64 reads as many bytes as its MFMAs take cycles; eight waves in two
+// halves of k, or four and five images, take 10 % fewer clocks a K-step and the same time).  Against linear_dma_kernel (pb_linear.hip: 16 x 16 MFMAs, two or three images, two
 // workgroups to a CU), us, 2048 rows: 2048 x 2048 29.9 -> 19.9 (0.87 PFLOP/s), K = 8192 93.5 -> 72, 2560 columns 39.8 -> 31, 8192 columns
 // 90.5 -> 65.6 (1.05 PFLOP/s; the gated pair 79.3 -> 60.7); 4096 x 4096 x 4096 161 -> 112 (1.23 PFLOP/s).  With a sigmoid on half of the columns: 5136
 // columns 77.6 -> 63.0, 10272 132 -> 124 since it and silu do without expf's and the division's cases (over_one_plus_exp; and 192-column tiles).
@@ -14,7 +14,6 @@ namespace {
 using namespace pcb;
 
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
-typedef float f16v __attribute__((ext_vector_type(16)));
 
 struct Grid { int mb, nb; mfma_tile::Strips s; };
 
@@ -255,11 +254,11 @@ __device__ __forceinline__ void store_columns(const pcb_linear_args& a, char* pa
     }
 }
 
-template <int EPI, int MT, int NT, int S>
+template <int EPI, int MT, int NT, int S, int BLK>
 __global__ __launch_bounds__(256, 1) void linear_tile_kernel(const pcb_linear_args a, const Grid g) {
     typedef bf16_t E;
     constexpr bool TWO = EPI == PCB_EPI_SILU_MUL;
-    using L = mfma_tile::Loop<MT, NT, S, 1>;
+    using L = mfma_tile::Loop<MT, NT, S, 1, BLK>;
     constexpr int BM = L::BM, BN = TWO ? L::BN / 2 : L::BN, NI = L::NI;   // BN: result columns
     constexpr int P = 32 * MT * 256;                                 // bytes of a patch (see below)
     __shared__ __attribute__((aligned(16))) char lds[S * L::kStage > 4 * P ? S * L::kStage : 4 * P];
@@ -295,10 +294,15 @@ __global__ __launch_bounds__(256, 1) void linear_tile_kernel(const pcb_linear_ar
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(s + o),
                                          (__attribute__((address_space(3))) void*)(buf + (4 * i + wave) * 1024), 16, 0, 0);
     };
-    f16v acc[MT][NT];
-    // (the weights are the products' first operand: a lane ends up with row lane & 31 and columns 8 q + 4 (lane >> 5) .. + 3 of a block)
-    L::template run<b8>(acc, lds, nk, last, lane, wm, wn,
-                        [](f16v& c, const b8& x, const b8& w) { c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, x, c, 0, 0, 0); }, stage);
+    typename L::Acc acc[L::MB][L::NB];
+    // (the weights are the products' first operand: a lane ends up with a row of a block and four neighbouring columns, BLK = 32: four times four)
+    auto mma = [](typename L::Acc& c, const b8& x, const b8& w) {
+        if constexpr (BLK == 16)
+            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x, c, 0, 0, 0);
+        else
+            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, x, c, 0, 0, 0);
+    };
+    L::template run<b8>(acc, lds, nk, last, lane, wm, wn, mma, stage);
 
     // Results: 64 accumulator columns of a wave go into an LDS patch of its own (16-byte quad c of row r at c ^ (r & 15)), so that neighbouring
     // lanes store neighbouring columns.  Gated: 32 gate columns and the matching 32 of the other half side by side.
@@ -306,24 +310,25 @@ __global__ __launch_bounds__(256, 1) void linear_tile_kernel(const pcb_linear_ar
     constexpr int PARTS = (NT + 1) / 2, ROOM = 4 * P * PARTS <= S * L::kStage ? PARTS : 1;   // patches that fit at a time
     char* patch = lds + wave * (P * ROOM);
     constexpr int LPR = TWO ? 8 : 16, RPI = 64 / LPR;                // lanes on a row, rows an access covers
-    const int fr = lane & 31, fh = lane >> 5, pr = lane / LPR, pc = lane % LPR;
+    const int fr = lane % BLK, pr = lane / LPR, pc = lane % LPR;
     auto fence = [] {
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
     };
     auto put = [&](auto part, char* to) {
         constexpr int j = decltype(part)::value;
+        constexpr int H = 32 / BLK;                                  // blocks of 32 columns
+        constexpr bool ODD = NT % 2 != 0 && j == PARTS - 1;          // (the last half patch of an odd number of them)
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
+        for (int i = 0; i < L::MB; ++i)
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
+            for (int h = 0; h < (ODD ? H : 2 * H); ++h) {
+                const typename L::Acc& c = acc[i][ODD ? L::NB - H + h : TWO ? H * j + h / H * (L::NB / 2) + h % H : 2 * H * j + h];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    constexpr bool ODD = NT % 2 != 0 && j == PARTS - 1;          // (the last half patch of an odd number of blocks)
-                    if (ODD && h == 1) continue;
-                    const f16v& c = acc[i][ODD ? NT - 1 : TWO ? j + h * (NT / 2) : 2 * j + h];
-                    *(f4*)(to + (32 * i + fr) * 256 + ((8 * h + 2 * q + fh) ^ (fr & 15)) * 16) = f4{c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]};
-                }
+                for (int q = 0; q < BLK * BLK / 256; ++q)
+                    *(f4*)(to + (BLK * i + fr) * 256 + ((BLK / 4 * h + mfma_tile::quad_of<BLK>(q, lane)) ^ (fr & 15)) * 16) =
+                        f4{c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]};
+            }
     };
     auto store = [&](int j, char* from) {
         const int n0 = n_lo + (TWO ? wn * 16 * NT + 32 * j : wn * 32 * NT + 64 * j);
@@ -348,12 +353,12 @@ __global__ __launch_bounds__(256, 1) void linear_tile_kernel(const pcb_linear_ar
     }
 }
 
-template <int EPI, int MT, int NT, int S>
+template <int EPI, int MT, int NT, int S, int BLK = (MT * NT > 4 ? 16 : 32)>
 int launch(const pcb_linear_args& a, hipStream_t stream) {
-    using L = mfma_tile::Loop<MT, NT, S, 1>;
+    using L = mfma_tile::Loop<MT, NT, S, 1, BLK>;
     const int mb = pcb_ceil_div(a.M, L::BM), nb = pcb_ceil_div(a.N, EPI == PCB_EPI_SILU_MUL ? L::BN / 2 : L::BN);
     const mfma_tile::Strips s = mfma_tile::strips(mb, nb, L::BM, L::BN);
-    hipLaunchKernelGGL((linear_tile_kernel<EPI, MT, NT, S>), dim3(8 * s.mh * s.nh), dim3(256), 0, stream, a, (Grid{mb, nb, s}));
+    hipLaunchKernelGGL((linear_tile_kernel<EPI, MT, NT, S, BLK>), dim3(8 * s.mh * s.nh), dim3(256), 0, stream, a, (Grid{mb, nb, s}));
     return pcb_check_launch("linear_tile_kernel");
 }
 

@@ -24,7 +24,8 @@
 // between its stores -> this kernel, us, random data: both planes, 1 737 rows, q|k|v 329 -> 307, o_proj 113 -> 103, down 288 -> 265
 // (1.18 PFLOP/s executed), 32 000 columns 816 -> 758, 3 584 rows down 598 -> 532; one plane, gate|up, 1 737 / 2 940 / 3 584 rows 370 -> 324,
 // 600 -> 528, 729 -> 561 (256 x 256 tiles, 1.15 PFLOP/s).
-// mfma_f32_32x32x16_f16: per 16-deep k-slab a wave reads MT (2 MT with both planes) activation fragments and NT weight fragments
+// mfma_f32_16x16x32_f16 (32x32x16 in the 128 x 128 tiles of one plane; which and why: mfma_tile_loop.h).  Per 32 x 32 results and 16 of k: MT (2 MT with both
+// planes) activation fragments and NT weight fragments
 // (16 B per lane each, ds_read_b128) for MT NT (2 MT NT) MFMAs.
 // Staging, LDS image and main loop: mfma_tile_loop.h.
 // Which global weight row lands in which LDS row is free as well (per-lane source address): the SiLU launch puts 32
@@ -92,7 +93,7 @@ __device__ __forceinline__ void glds16(const _Float16* g, char* lds_wave_base) {
 // the block tile of a launch: W x W waves of 32 MT x 32 NT, S LDS images in the ring (as many as the 160 KiB of a CU hold)
 template <int W, bool TWO, bool NARROW, bool TALL>
 struct Tile {
-    static constexpr int MT = TALL ? 4 : 2, NT = NARROW ? 2 : 4, S = TWO || TALL ? 2 : 3;
+    static constexpr int MT = TALL ? 4 : 2, NT = NARROW ? 2 : 4, S = TWO || TALL ? 2 : 3, BLK = TWO || !NARROW ? 16 : 32;
     static constexpr int BM = 32 * W * MT, BN = 32 * W * NT;
 };
 
@@ -237,7 +238,7 @@ __global__ __launch_bounds__(256, 1) void gemm_dense_kernel(const DenseParams p)
     static_assert(W == 2 && !(TWO && TALL), "four waves; two planes of 256 rows and their weights do not fit the LDS twice");
     using T = Tile<W, TWO, NARROW, TALL>;
     constexpr int MT = T::MT, NT = T::NT, S = T::S;
-    using L = mfma_tile::Loop<MT, NT, S, TWO ? 2 : 1>;
+    using L = mfma_tile::Loop<MT, NT, S, TWO ? 2 : 1, T::BLK>;
     constexpr int PL = TWO ? 2 : 1, BM = L::BM, BN = L::BN;
     constexpr int NI = L::NI, NX = PL * BM / 32;                 // staging instructions per wave, of them for activations
     __shared__ __attribute__((aligned(16))) char lds[S * L::kStage];   // images: Xhi | Xlo | W
@@ -261,7 +262,7 @@ __global__ __launch_bounds__(256, 1) void gemm_dense_kernel(const DenseParams p)
         }
         if (EPI == EPI_ROPE) {
             // a 64-column group = 32 features d of one head's first half next to their rotary partners d + 64, so
-            // x[d] and x[d + 64] meet in the same lane and accumulator index of the two 32-wide MFMA blocks
+            // x[d] and x[d + 64] meet in the same row of a patch, 32 columns apart
             const int wt = r >> 6, c = r & 63;
             const int hd = ni * (BN / 128) + (wt >> 1);
             const int d = (c < 32) ? (wt & 1) * 32 + c : 64 + (wt & 1) * 32 + (c - 32);
@@ -297,31 +298,38 @@ __global__ __launch_bounds__(256, 1) void gemm_dense_kernel(const DenseParams p)
     };
     const int keep = t0 + nk == nkt ? last : 8;          // chunks of this slice's last K-step
 
-    f16v acc[MT][NT];
-    L::template run<h8>(acc, lds, nk, keep, lane, wm, wn,
-                        [](f16v& c, const h8& a, const h8& w) { c = __builtin_amdgcn_mfma_f32_32x32x16_f16(w, a, c, 0, 0, 0); }, stage);
+    typename L::Acc acc[L::MB][L::NB];
+    auto mma = [](typename L::Acc& c, const h8& a, const h8& w) {
+        if constexpr (T::BLK == 16)
+            c = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, a, c, 0, 0, 0);
+        else
+            c = __builtin_amdgcn_mfma_f32_32x32x16_f16(w, a, c, 0, 0, 0);
+    };
+    L::template run<h8>(acc, lds, nk, keep, lane, wm, wn, mma, stage);
 
     // ---- epilogue: 64 accumulator columns of a wave at a time through an LDS patch of its own -> full-row global stores ----
-    // (the weights are the products' first operand: a lane holds row lane & 31 and the column quads 8 q + 4 (lane >> 5) of a 32 x 32 block;
+    // (the weights are the products' first operand: a lane holds a row of a block and four neighbouring columns, in 32 x 32 blocks four times four;
     // patch: [32 MT][64] fp32, 16-byte quad c of row r at c ^ (r & 15))
     __syncthreads();                                       // every wave is done with the staging buffers
     constexpr int P = 32 * MT * 256, PARTS = NT / 2, ROOM = 4 * P * PARTS <= S * L::kStage ? PARTS : 1;   // patches that fit at a time
     char* patch = lds + wave * (P * ROOM);
-    const int fr = lane & 31, fh = lane >> 5;
+    const int fr = lane % T::BLK;
     auto fence = [] {
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
     };
     auto put = [&](auto part, char* to) {
         constexpr int j = decltype(part)::value;
+        constexpr int H = 64 / T::BLK;                     // blocks of 64 columns
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
+        for (int i = 0; i < L::MB; ++i)
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
+            for (int h = 0; h < H; ++h)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const f16v& c = acc[i][2 * j + h];
-                    *(f4*)(to + (32 * i + fr) * 256 + ((8 * h + 2 * q + fh) ^ (fr & 15)) * 16) = f4{c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]};
+                for (int q = 0; q < T::BLK * T::BLK / 256; ++q) {
+                    const typename L::Acc& c = acc[i][H * j + h];
+                    *(f4*)(to + (T::BLK * i + fr) * 256 + ((T::BLK / 4 * h + mfma_tile::quad_of<T::BLK>(q, lane)) ^ (fr & 15)) * 16) =
+                        f4{c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]};
                 }
     };
     using First = std::integral_constant<int, 0>;

@@ -85,6 +85,33 @@ def test_dense_tall_tiles_strips_and_short_rings(M, N, K, two):
         assert bool(((oh.double() + ol.double() - want).abs() <= 2.0 ** -19 * (want.abs() + 2.0 ** -6)).all())
 
 
+@pytest.mark.parametrize("two", [True, False])
+@pytest.mark.parametrize("M,N", [(1025, 4100), (2001, 8188), (300, 1028)])
+@pytest.mark.parametrize("K", [8, 24, 48, 56, 88, 104, 160, 184])
+def test_dense_k_ranges_that_end_inside_a_slab_keep_infinities(M, N, two, K):
+    """The chunks of a last K-step past K are staged from the row's first ones of that step and left out of the products: an infinity there stays
+    the infinity that the sums make of it (no infinity times zero), and the other rows are finite and right (as above, planes x K x 2^-24 of the
+    magnitudes; 128 x 256, 256 x 256 and 128 x 128 tiles, one plane and two)."""
+    n = _n()
+    g = torch.Generator(device="cuda:0").manual_seed(K)
+    x = torch.randn((M, K), generator=g, device="cuda:0")
+    hi = x.half()
+    lo = (x - hi.float()).half()
+    w = (torch.rand((N, K), generator=g, device="cuda:0") + 0.5).half()
+    k = (K - 1) // 64 * 64
+    hi[7, k], hi[M - 1, k] = float("inf"), -float("inf")
+    lo[7, k] = lo[M - 1, k] = 0.0
+    y = torch.full((M, N), float("nan"), device="cuda:0")
+    n.gemm_dense(hi, lo if two else None, w, M, N, K, n.EPI_STORE, y=y)
+    assert bool((y[7] == float("inf")).all()) and bool((y[M - 1] == -float("inf")).all())
+    hi[7, k] = hi[M - 1, k] = 0.0
+    rest = torch.ones(M, dtype=torch.bool, device="cuda:0")
+    rest[7] = rest[M - 1] = False
+    full = hi.double() + (lo.double() if two else 0.0)
+    bound = (2 if two else 1) * K * 2.0 ** -24 * (hi.double().abs() + (lo.double().abs() if two else 0.0)) @ w.double().abs().T
+    assert bool(((y.double() - full @ w.double().T).abs() <= bound)[rest].all())
+
+
 # few-row launches of the N = hidden projections take the split-K form when a workspace is supplied (pc_gemm_dense_ws);
 # (1000, 12288, 4096) and (77, 512, 8) do not split (large grid / too few K-steps) and must equal pc_gemm_dense bit for bit
 @pytest.mark.parametrize("two", [True, False])
