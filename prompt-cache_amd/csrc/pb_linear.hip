@@ -490,120 +490,7 @@ __global__ __launch_bounds__(256) void linear_dma_kernel(pcb_linear_args a) {
             acc[i][j] = sum[i][j].total();
             if (TWO) acc2[i][j] = sum2[i][j].total();
         }
-    // (the weights are the products' first operand: a lane ends up with four neighbouring columns of one row.)
-    // Bias, gate and activation first, in the accumulators -- an activation is chosen once, around the loop over them --, then the stores
-    const E* bias = (const E*)a.bias;
-    const E* bias2 = TWO ? (const E*)a.bias2 : nullptr;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-        const int n = n_lo + (wn * TN + j) * 16 + 4 * group;
-        if (bias || TWO) {
-            float bv[4], bv2[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const bool in = n + e < N;
-                bv[e] = bias && in ? to_f32(bias[n + e]) : 0.0f;
-                bv2[e] = TWO && bias2 && in ? to_f32(bias2[n + e]) : 0.0f;
-            }
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                float rg = 1.0f;
-                if (TWO && a.row_gate) {
-                    const int m = m_lo + (wm * TM + i) * 16 + l15;
-                    rg = to_f32(((const E*)a.row_gate)[(m < m_hi ? m : m_hi - 1) * a.ld_row_gate]);
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    acc[i][j][e] += bv[e];
-                    if (TWO) acc[i][j][e] = gate_act(a.act, acc[i][j][e]) * (acc2[TWO ? i : 0][TWO ? j : 0][e] + bv2[e]) * rg;
-                }
-            }
-        }
-    }
-    if (EPI == PCB_EPI_STORE && (a.act | a.act2)) {
-        const int end = act_end(a), mid = a.act_split > 0 && a.act_split < end ? a.act_split : end;
-        auto run = [&](auto code, int lo, int hi) {
-            constexpr int A = decltype(code)::value;
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const int n = n_lo + (wn * TN + j) * 16 + 4 * group;
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (n + e >= lo && n + e < hi) {
-#pragma unroll
-                        for (int i = 0; i < TM; ++i) acc[i][j][e] = apply_act(A, acc[i][j][e], a.act_param);
-                    }
-            }
-        };
-        auto pass = [&](int act, int lo, int hi) {
-            if (n_lo >= hi || n_lo + BN <= lo) return;
-            switch (act) {
-                case PCB_ACT_SILU: run(std::integral_constant<int, PCB_ACT_SILU>{}, lo, hi); break;
-                case PCB_ACT_SIGMOID: run(std::integral_constant<int, PCB_ACT_SIGMOID>{}, lo, hi); break;
-                case PCB_ACT_RELU2: run(std::integral_constant<int, PCB_ACT_RELU2>{}, lo, hi); break;
-                case PCB_ACT_SOFTPLUS: run(std::integral_constant<int, PCB_ACT_SOFTPLUS>{}, lo, hi); break;
-                case PCB_ACT_SOFTCAP: run(std::integral_constant<int, PCB_ACT_SOFTCAP>{}, lo, hi); break;
-                case PCB_ACT_RELU: run(std::integral_constant<int, PCB_ACT_RELU>{}, lo, hi); break;
-                case PCB_ACT_GELU_TANH: run(std::integral_constant<int, PCB_ACT_GELU_TANH>{}, lo, hi); break;
-                case PCB_ACT_LOGSIGMOID: run(std::integral_constant<int, PCB_ACT_LOGSIGMOID>{}, lo, hi); break;
-                case PCB_ACT_SCALE: run(std::integral_constant<int, PCB_ACT_SCALE>{}, lo, hi); break;
-                default: break;
-            }
-        };
-#pragma unroll 1
-        for (int part = 0; part < 2; ++part) pass(part ? a.act2 : a.act, part ? mid : 0, part ? end : mid);
-    }
-    const int whole = act_end(a);                                    // columns that go to y
-    const int esz = (EPI == PCB_EPI_SCALE_ADD || a.out_f32 || sizeof(E) == 4) ? 4 : 2;
-    const bool quads = a.ldy % 4 == 0 && (uintptr_t)a.y % (4 * esz) == 0 && a.y_batch_stride % 4 == 0 &&
-                       (EPI != PCB_EPI_SCALE_ADD || !a.base || (a.ldbase % 4 == 0 && (uintptr_t)a.base % 16 == 0));
-    const int64_t y0 = a.n_batch > 0 ? (int64_t)blockIdx.z * a.y_batch_stride : 0;
-    // (what the stores need is loaded before the first of them)
-    int64_t dst[TM];
-    f4 base[EPI == PCB_EPI_SCALE_ADD ? TM : 1][EPI == PCB_EPI_SCALE_ADD ? TN : 1], cs[EPI == PCB_EPI_SCALE_ADD ? TN : 1];
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-        const int mm = m_lo + (wm * TM + i) * 16 + l15, m = mm < m_hi ? mm : m_hi - 1;
-        dst[i] = (int64_t)(EPI != PCB_EPI_SCALE_ADD && a.row_dst ? a.row_dst[m] : m) * a.ldy + y0;
-        if constexpr (EPI == PCB_EPI_SCALE_ADD) {
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const int n = n_lo + (wn * TN + j) * 16 + 4 * group;
-                if (i == 0) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) cs[j][e] = n + e < N ? a.col_scale[n + e] : 0.0f;
-                }
-                if (quads && n + 4 <= N) base[i][j] = *reinterpret_cast<const f4*>(a.base ? a.base + (int64_t)m * a.ldbase + n : (const float*)a.y + dst[i] + n);
-            }
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-        const int n = n_lo + (wn * TN + j) * 16 + 4 * group;
-        const bool quad = quads && n + 4 <= whole;
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-            const int m = m_lo + (wm * TM + i) * 16 + l15;
-            if (m >= m_hi) continue;
-            const f4 v = acc[i][j];
-            if (quad) {
-                if constexpr (EPI == PCB_EPI_SCALE_ADD)
-                    *reinterpret_cast<f4*>((float*)a.y + dst[i] + n) = base[i][j] + cs[j] * v;
-                else if (esz == 4)
-                    *reinterpret_cast<f4*>((float*)a.y + dst[i] + n) = v;
-                else
-                    *reinterpret_cast<uint2*>((E*)a.y + dst[i] + n) = uint2{bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3])};
-            } else {
-                Place to[4] = {};
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (n + e < N) to[e] = place<E, EPI>(a, m, n + e);
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (n + e < N) put<E, EPI>(to[e], v[e], EPI == PCB_EPI_SCALE_ADD ? cs[EPI == PCB_EPI_SCALE_ADD ? j : 0][e] : 0.0f);
-            }
-        }
-    }
+    finish_tile<E, EPI, TM, TN>(a, acc, acc2, m_lo, m_hi, n_lo, wm, wn, group, l15);
 }
 
 template <typename E, int EPI, int TM, int TN, int STAGES>
@@ -762,6 +649,7 @@ int dispatch(const pcb_linear_args& a, hipStream_t stream) {
         return pcb_check_launch("linear_skinny_kernel");
     }
     if (dma_ok(a)) {
+        if (sizeof(E) == 4 && pcb_linear_split_fits(a)) return pcb_linear_split(a, stream);
         if (pcb_linear_waves_fits(a)) return pcb_linear_waves(a, stream);
         // Plain launches whose 128 x 128 tiles reach more than half of the 256 CUs go to the whole-CU tiles of pb_linear_tiles.hip (row strides
         // such that a tile's rows lie within 32-bit offsets); below, the smaller tiles here give more CUs work: 300 x 2048, K = 2048 (48 tiles)

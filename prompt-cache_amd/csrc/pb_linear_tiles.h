@@ -9,3 +9,6 @@ int pcb_linear_tiles(const pcb_linear_args& a, hipStream_t stream);
 int64_t pcb_linear_waves_tiles(const pcb_linear_args& a);
 bool pcb_linear_waves_fits(const pcb_linear_args& a);
 int pcb_linear_waves(const pcb_linear_args& a, hipStream_t stream);
+// ... and those in fp32 of so many tiles that splitting their operands pays (pb_linear_split.hip)
+bool pcb_linear_split_fits(const pcb_linear_args& a);
+int pcb_linear_split(const pcb_linear_args& a, hipStream_t stream);

@@ -401,6 +401,60 @@ def test_whole_cu_tiles_dealt_in_runs(M, N, K):
     assert rel(g, torch.relu(y[:, :h]) * y[:, h:]) < 4e-3
 
 
+# tiles of 64 x 64, 64 x 128 and 128 x 128 (weight rows), a ragged last one both ways
+@pytest.mark.parametrize("M,N", [(587, 1026), (587, 2562), (587, 5134)])
+@pytest.mark.parametrize("K", [4, 28, 64, 100, 520])
+def test_fp32_products_in_parts_and_what_is_no_number(M, N, K):
+    """fp32 products on the bf16 matrix cores: no further from 64 bits than 32-term sums rounded to fp32 are (sqrt(K / 32) 2^-24 of the magnitudes, times
+    four), over rows of very different sizes; gathered rows, the gated unit, batches and the accumulation; an infinity, a NaN and the largest numbers
+    give what fp32 sums of them give, in their own row and column only."""
+    b = B()
+    x, w, w2 = (rnd(r, K, seed=i, scale=K ** -0.25) for i, r in ((1, M), (2, N), (3, N)))
+    x = x * 2.0 ** torch.linspace(-40, 40, M, device=DEV).round()[:, None]
+    mag, z = x.double().abs() @ w.double().abs().T.contiguous(), x.double() @ w.double().T.contiguous()
+    y = torch.full((M, N), float("nan"), device=DEV)
+    b.linear(x, w, y, M=M)
+    bound = 4 * (K / 32 + 1) ** 0.5 * 2.0 ** -24
+    assert bool(((y.double() - z).abs() <= bound * mag).all())
+    src = torch.randperm(M, generator=torch.Generator().manual_seed(5)).to(DEV)
+    y2 = torch.full((M, N), float("nan"), device=DEV)
+    b.linear(x, w, y2, M=M, row_src=src.to(torch.int32))
+    assert torch.equal(y2, y[src])
+    x1 = rnd(M, K, seed=7, scale=K ** -0.25)
+    h = N // 2
+    t, u = x1.double() @ w[:h].double().T.contiguous(), x1.double() @ w2[:h].double().T.contiguous()
+    g = torch.full((M, h), float("nan"), device=DEV)
+    b.linear(x1, w[:h].contiguous(), g, M=M, epilogue=b.EPI_SILU_MUL, w2=w2[:h].contiguous(), act=b.ACT_RELU)
+    assert rel(g, torch.relu(t) * u) < 2e-6
+    cs, acc = rnd(N, seed=8), rnd(M, N, seed=9)
+    want = acc.double() + cs.double() * (x1.double() @ w.double().T.contiguous())
+    b.linear(x1, w, acc, M=M, epilogue=b.EPI_SCALE_ADD, col_scale=cs)
+    assert rel(acc, want) < 2e-6
+    yb = torch.full((2, M, N), float("nan"), device=DEV)
+    xb, wb = torch.stack([x1, x]), torch.stack([w, w2])
+    b.linear(xb, wb, yb, M=M, n_batch=2, ldx=K, ldy=N, x_batch_stride=M * K, y_batch_stride=M * N)
+    assert rel(yb[0], x1.double() @ w.double().T.contiguous()) < 2e-6
+    assert bool(((yb[1].double() - x.double() @ w2.double().T.contiguous()).abs() <= bound * (x.double().abs() @ w2.double().abs().T.contiguous())).all())
+    tiny = x1 * 2.0 ** -112                                          # (parts below the smallest normal number)
+    b.linear(tiny, w, y, M=M)
+    assert rel(y.double() * 2.0 ** 112, x1.double() @ w.double().T.contiguous()) < 2e-6
+    # an infinity among the rows, one among the weights (positive partners), a NaN, a row and a weight close to the largest number
+    bad, wbad = x1.clone(), w.abs().contiguous()
+    bad[3, K - 1], bad[70, 0], bad[M - 1, K // 2] = float("inf"), float("nan"), 3.4e38
+    bad[3, :K - 1] = 0.25
+    wbad[5] = 0.0
+    wbad[5, K - 1] = 2.0 ** -20
+    wbad[N - 1, 0] = float("inf")
+    y = torch.zeros(M, N, device=DEV)
+    b.linear(bad, wbad, y, M=M)
+    z = bad.double() @ wbad.double().T.contiguous()
+    z = torch.where(z.abs() > 3.4028235677973366e38, torch.full_like(z, float("inf")) * z.sign(), z)
+    assert torch.equal(torch.isnan(y), torch.isnan(z)) and torch.equal(torch.isinf(y), torch.isinf(z)) and torch.equal(y[torch.isinf(y)].double(), z[torch.isinf(z)])
+    ok = torch.isfinite(z)
+    mag = torch.nan_to_num(bad.double().abs(), 0.0, 0.0) @ torch.nan_to_num(wbad.double().abs(), 0.0, 0.0).T.contiguous()
+    assert bool(((y.double() - z).abs() <= bound * mag)[ok].all())
+
+
 @pytest.mark.parametrize("M,N", [(1, 70), (9, 64), (16, 130), (40, 100), (130, 260), (600, 2564), (2000, 2040)])
 @pytest.mark.parametrize("K", [4, 30, 36, 68, 516])
 def test_fp32_projections_at_every_tile_and_their_edges(M, N, K):
