@@ -705,6 +705,51 @@ typedef struct pcb_attn_rows_args {
 } pcb_attn_rows_args;
 int pcb_attn_rows(const pcb_attn_rows_args* a, void* stream);
 
+/* One decoding step of an attention layer behind its projection: pcb_head_prep of the step's rows, pcb_attn_rows (latent: pcb_attn_latent) over what is cached and
+ * the new row itself; n_splits and part as there (n_splits > 1: a second launch merges).  Every row is the only one of its slot in the step.  tile r = {slot, position, 1, flat row} (int32 x 4, device).
+ * p: projected rows, ldp apart; queries from column q_at on, q_head_stride apart: unit-RMS norm, q_gain, a turn of the first rot_dims columns (neighbouring pairs,
+ * freqs float64 [rot_dims / 2], times rot_mag); keys from k_at on, k_cols apart, likewise with k_gain; values from v_at on: norm, kept in fp32 in keep (may be null) and
+ * mixed with other's by blend[0] (may be null; as in pcb_head_prep_seg).  The new key and value go to k / v as in pcb_attn_rows_args.
+ * latent: one key head whose row is (latent of vdim columns, normed, k_gain | dim - vdim turned columns), from k_at on; the values are its first vdim columns (v = k);
+ * queries: folded parts of vdim columns in q (head h of row r at r ldq + h dim), the turned parts from q_at on.
+ * gate: E, one number per row and head, or null.  pcb_attn_step_fits: whether heads of these sizes are taken. */
+typedef struct pcb_attn_step_args {
+    uint32_t struct_bytes;
+    int32_t dtype;
+    const void* p;
+    int64_t ldp, q_at, q_head_stride, k_at, k_cols, v_at;
+    const void* q;
+    int64_t ldq;
+    const int32_t* tiles;
+    int32_t n_rows;
+    void* k;
+    int64_t k_slot_stride, k_head_stride, k_row_stride;
+    void* v;
+    int64_t v_slot_stride, v_head_stride, v_row_stride;
+    int32_t H, Hkv, dim, vdim, latent;
+    float scale;
+    int32_t window, block;
+    const float* sink;
+    const void* gate;
+    int64_t ldg;
+    void* out;
+    int64_t ldo;
+    const float *q_gain, *k_gain;
+    float eps;
+    int32_t rot_dims;
+    const double* freqs;
+    float rot_mag;
+    const float* blend;
+    const float* other;
+    int64_t ld_other;
+    float* keep;
+    int64_t ld_keep;
+    int32_t n_splits;
+    float* part;
+} pcb_attn_step_args;
+int pcb_attn_step(const pcb_attn_step_args* a, void* stream);
+int pcb_attn_step_fits(int32_t dtype, int32_t H, int32_t Hkv, int32_t dim, int32_t vdim, int32_t rot_dims, int32_t latent);
+
 /* Recurrences with a matrix state S [dim][vdim] per (slot, head), fp32, zero before position 0.  Per token and head h:
  *   q = q_scale q^, k = k_scale k^        q^, k^: E rows with head h / (H / Hk) at column (h / (H / Hk)) * dim; unit_norm: divided by
  *                                         sqrt(sum of squares + unit_eps); rot_dims > 0: turned in halves by the row's cosines and

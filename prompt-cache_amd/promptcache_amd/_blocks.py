@@ -173,6 +173,19 @@ class AttnRowsArgs(C.Structure):
                 ("sink", _vp), ("gate", _vp), ("ldg", _i64), ("gate_per_head", _i32), ("out", _vp), ("ldo", _i64), ("n_splits", _i32), ("part", _vp)]
 
 
+class AttnStepArgs(C.Structure):
+    """``pcb_attn_step_args`` (field for field)."""
+    _fields_ = [("struct_bytes", C.c_uint32), ("dtype", _i32),
+                ("p", _vp), ("ldp", _i64), ("q_at", _i64), ("q_head_stride", _i64), ("k_at", _i64), ("k_cols", _i64), ("v_at", _i64),
+                ("q", _vp), ("ldq", _i64), ("tiles", _vp), ("n_rows", _i32),
+                ("k", _vp), ("k_slot_stride", _i64), ("k_head_stride", _i64), ("k_row_stride", _i64),
+                ("v", _vp), ("v_slot_stride", _i64), ("v_head_stride", _i64), ("v_row_stride", _i64),
+                ("H", _i32), ("Hkv", _i32), ("dim", _i32), ("vdim", _i32), ("latent", _i32), ("scale", _f32), ("window", _i32), ("block", _i32),
+                ("sink", _vp), ("gate", _vp), ("ldg", _i64), ("out", _vp), ("ldo", _i64), ("q_gain", _vp), ("k_gain", _vp), ("eps", _f32),
+                ("rot_dims", _i32), ("freqs", _vp), ("rot_mag", _f32), ("blend", _vp), ("other", _vp), ("ld_other", _i64), ("keep", _vp),
+                ("ld_keep", _i64), ("n_splits", _i32), ("part", _vp)]
+
+
 class RecArgs(C.Structure):
     """``pcb_rec_args`` (field for field)."""
     _fields_ = [("struct_bytes", C.c_uint32), ("dtype", _i32),
@@ -224,6 +237,8 @@ SIGNATURES = {
     "pcb_attn_prompt": (C.c_int, [C.POINTER(AttnPromptArgs), _vp]),
     "pcb_attn_latent": (C.c_int, [C.POINTER(AttnLatentArgs), _vp]),
     "pcb_attn_rows": (C.c_int, [C.POINTER(AttnRowsArgs), _vp]),
+    "pcb_attn_step": (_i32, [C.POINTER(AttnStepArgs), _vp]),
+    "pcb_attn_step_fits": (_i32, [_i32] * 7),
     "pcb_rot_table": (C.c_int, [_vp, _vp, _f32, _vp, _i32, _i32, _vp]),
     "pcb_conv_step": (C.c_int, [_vp, _i64, _vp, _vp, _i32, _i32, _vp, _i32, _vp, _i64, _vp, _i64, _i32, _i32, _vp]),
     "pcb_rec_scratch": (C.c_int64, [_i32, _i32, _i32]),
@@ -955,6 +970,41 @@ def attn_rows(q: torch.Tensor, tiles: torch.Tensor, n_rows: int, k: torch.Tensor
                      *(int(x) for x in v_strides), H, Hkv, dim, vdim, float(scale), int(window), int(block), _p(sink), _p(gate), ldg,
                      int(gate_per_head), _p(out), ldo, n_splits, _p(part))
     check(load().pcb_attn_rows(C.byref(a), _stream()), "pcb_attn_rows")
+
+
+def attn_step_fits(dtype: torch.dtype, H: int, Hkv: int, dim: int, vdim: int, rot_dims: int, latent: bool = False) -> bool:
+    """Whether ``attn_step`` takes heads of these sizes."""
+    return bool(load().pcb_attn_step_fits(BF16 if dtype == torch.bfloat16 else F32, H, Hkv, dim, vdim, rot_dims, int(latent)))
+
+
+def attn_step(p: torch.Tensor, tiles: torch.Tensor, n_rows: int, k: torch.Tensor, k_strides, v: torch.Tensor, v_strides, H: int, Hkv: int, dim: int,
+              vdim: int, scale: float, out: torch.Tensor, *, q_at: int, q_head_stride: int, k_at: int, v_at: int = 0, q=None, q_gain=None, k_gain=None,
+              eps: float, rot_dims: int = 0, freqs=None, rot_mag: float = 1.0, blend=None, other=None, keep=None, window: int = 0, block: int = 0, sink=None,
+              gate=None, ldg: int = 0, n_splits: int = 1, part=None) -> None:
+    """A decoding step of an attention layer behind its projection ``p`` [rows, columns]: ``head_prep`` of queries, keys and values and ``attn_rows`` over the cached rows
+    and the new one; with ``q`` [rows, H * dim] (the folded queries) ``attn_latent``'s form: one key head, its first ``vdim`` columns the values.  Every row is
+    the only one of its slot.  ``k_strides`` / ``v_strides``: (slot, head, row) strides; ``other`` / ``keep``: fp32 [rows, Hkv * vdim]; ``gate``: E, one number per row and head;
+    ``n_splits`` / ``part`` as in ``attn_rows``."""
+    latent = q is not None
+    _want(tiles, torch.int32, "attn_step tiles"); _want(sink, torch.float32, "attn_step sink"); _want(freqs, torch.float64, "attn_step freqs")
+    for t, nm in ((q_gain, "q_gain"), (k_gain, "k_gain"), (blend, "blend"), (other, "other"), (keep, "keep")):
+        _want(t, torch.float32, "attn_step " + nm)
+    assert p.dtype == k.dtype == v.dtype == out.dtype and p.is_contiguous() and out.is_contiguous() and p.shape[0] >= n_rows and out.shape[0] >= n_rows
+    assert tiles.numel() >= 4 * n_rows and out.shape[-1] == H * vdim and (sink is None or sink.numel() >= H)
+    assert q_at + (H - 1) * q_head_stride + (dim - vdim if latent else dim) <= p.shape[-1]
+    assert k_at + (dim if latent else Hkv * dim) <= p.shape[-1] and (latent or v_at + Hkv * vdim <= p.shape[-1])
+    assert rot_dims == 0 or freqs.numel() >= rot_dims // 2
+    assert (q_gain is None or q_gain.numel() >= dim) and (k_gain is None or k_gain.numel() >= (vdim if latent else dim))
+    assert not latent or (q.dtype == p.dtype and q.is_contiguous() and q.shape[-1] == H * dim and q.shape[0] >= n_rows)
+    assert all(t is None or (t.shape[-1] == Hkv * vdim and t.shape[0] >= n_rows) for t in (other, keep)) and (blend is None or other is not None)
+    assert gate is None or (gate.dtype == p.dtype and ldg >= H)
+    _want(part, torch.float32, "attn_step part")
+    assert n_splits <= 1 or (part is not None and part.numel() >= attn_softmax_part(n_rows, H, n_splits, vdim))
+    a = AttnStepArgs(C.sizeof(AttnStepArgs), _code(p), _p(p), p.shape[-1], q_at, q_head_stride, k_at, dim, v_at, _p(q), q.shape[-1] if latent else 0, _p(tiles),
+                     n_rows, _p(k), *(int(x) for x in k_strides), _p(v), *(int(x) for x in v_strides), H, Hkv, dim, vdim, int(latent), float(scale),
+                     int(window), int(block), _p(sink), _p(gate), ldg, _p(out), out.shape[-1], _p(q_gain), _p(k_gain), float(eps), rot_dims, _p(freqs),
+                     float(rot_mag), _p(blend), _p(other), Hkv * vdim, _p(keep), Hkv * vdim, n_splits, _p(part))
+    check(load().pcb_attn_step(C.byref(a), _stream()), "pcb_attn_step")
 
 
 def rot_table(pos: torch.Tensor, freqs: torch.Tensor, mag: float, out: torch.Tensor, n_rows: int) -> None:

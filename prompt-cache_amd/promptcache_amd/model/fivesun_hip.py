@@ -443,8 +443,19 @@ class FivesunHIP(SlotModel):
         HD, GD, GV = H * D, G * D, G * Dv
         P, N = self._project_in(lw, h, T)
         plane = arena.planes[i]
-        q = self._mat("q_rows", T, HD, E)
         vf = self._mat("v_first", T, GV, torch.float32) if l.v_mix else None
+        reach = min(arena.cap, l.mask or arena.cap)
+        if tb["ones"] and B.attn_step_fits(E, H, G, D, Dv, l.rot_dims):      # (a row's own key is the only new one it sees)
+            splits = self._splits(T, G * -(-H // (16 * G)), H, reach)
+            att, strides = self._mat("mix_out", T, H * Dv, E), (arena.slot_stride(i), arena.head_stride(i), D + Dv)
+            part = self._scratch("attn_part", B.attn_softmax_part(T, H, splits, Dv), torch.float32) if splits > 1 else None
+            B.attn_step(P, tb["s_tiles"], T, plane, strides, plane.view(-1)[D:], strides, H, G, D, Dv, l.scale, att, q_at=0, q_head_stride=D, k_at=HD,
+                        v_at=HD + GD, q_gain=lw["q_gain"], k_gain=lw["k_gain"], eps=self.config.norm_eps, rot_dims=l.rot_dims, freqs=lw["freqs"],
+                        rot_mag=lw["rot_mag"], blend=lw["blend"], other=vf if lw["blend"] is not None else None,
+                        keep=vf if i == self.first_v_mix else None, block=l.mask, sink=lw["sink"], gate=P[:, HD + GD + GV:], ldg=N, n_splits=splits, part=part)
+            B.linear(att, lw["wo"], y, M=T)
+            return P[:, HD + GD + GV + H:], N
+        q = self._mat("q_rows", T, HD, E)
         row = dict(row_off=tb["offs"][self._sigs.index((G, D + Dv))], head_stride=arena.head_stride(i))
         segs = [B.head_seg(P, N, H, D, q, norm=True, gain=lw["q_gain"], rot_dims=l.rot_dims, ld_dst=HD),
                 B.head_seg(P[:, HD:], N, G, D, plane, norm=True, gain=lw["k_gain"], rot_dims=l.rot_dims, **row),
@@ -454,7 +465,6 @@ class FivesunHIP(SlotModel):
         att = self._mat("mix_out", T, H * Dv, E)
         values, gate = plane.view(-1)[D:], P[:, HD + GD + GV:]
         ss, hs, rs = arena.slot_stride(i), arena.head_stride(i), D + Dv
-        reach = min(arena.cap, l.mask or arena.cap)
         if D > 256:
             n = tb["w_tiles"].numel() // 4
             splits = 1 if n * H >= 512 or arena.cap <= 256 else max(1, min(16, 1024 // (n * H), arena.cap // 128))
@@ -487,6 +497,19 @@ class FivesunHIP(SlotModel):
         f_tiles = tb["f_tiles"] if lw["prompts"] or not tb["a_tiles"].numel() else tb["a_tiles"]
         n = f_tiles.numel() // 4
         qa = self._mat("q_latent", T, H * CR, E) if n else None   # per head [W_uk^T q | rotated part]: a query over the cached rows
+        reach = min(arena.cap, l.mask or arena.cap)
+        splits = self._splits(n, -(-H // 16), H, reach, 768 if CR <= 256 else 512) if n else 0
+        if tb["ones"] and n == T and B.attn_step_fits(E, H, 1, CR, C, Rd, True):
+            B.linear(P, lw["w_abs"], qa, M=T, n_batch=H, ldx=N, x_batch_stride=DR, ldy=H * CR, y_batch_stride=CR)
+            ol, strides = self._mat("mix_out", T, H * C, E), (arena.slot_stride(i), 0, CR)
+            B.attn_step(P, f_tiles, T, plane, strides, plane, strides, H, 1, CR, C, l.scale, ol, q_at=D, q_head_stride=DR, k_at=HQ, q=qa, k_gain=lw["c_gain"],
+                        eps=self.config.norm_eps, rot_dims=Rd, freqs=lw["freqs"], rot_mag=lw["rot_mag"], window=l.mask, n_splits=splits,
+                        part=self._scratch("attn_part", B.attn_softmax_part(n, H, splits, C), torch.float32) if splits > 1 else None)
+            og, ov = self._mat("mix_gated", T, HV, E), self._mat("mix_o32", T, HV, torch.float32)
+            B.linear(ol, lw["w_uv"], ov, M=T, n_batch=H, ldx=H * C, x_batch_stride=C, ldy=HV, y_batch_stride=Dv)
+            B.gated_norm(ov, None, P[:, HQ + CR:], N, og, self.config.norm_eps, T)
+            B.linear(og, lw["wo"], y, M=T)
+            return P[:, HQ + CR + HV:], N
         q = self._mat("q_rows", T, HQ, E) if tiled else None      # per head [plain part | rotated part]: a query over rebuilt rows
         segs = [B.head_seg(P[:, HQ:], N, 1, C, plane, norm=True, gain=lw["c_gain"], row_off=off)]
         if tiled:
@@ -504,7 +527,6 @@ class FivesunHIP(SlotModel):
             rows = tb["f_rows"] if tiled and n < T else None
             B.linear(P, lw["w_abs"], qa, M=n, row_src=rows, row_dst=rows, n_batch=H, ldx=N, x_batch_stride=DR, ldy=H * CR, y_batch_stride=CR)
             ol = self._mat("mix_out", T, H * C, E)
-            splits = self._splits(n, -(-H // 16), H, min(arena.cap, l.mask or arena.cap), 768 if CR <= 256 else 512)
             part = self._scratch("attn_part", B.attn_softmax_part(n, H, splits, C), torch.float32) if splits > 1 else None
             B.attn_latent(qa, f_tiles, n, plane, arena.slot_stride(i), CR, H, CR, C, l.scale, ol, window=l.mask, n_splits=splits, part=part)
             ov = self._mat("mix_o32", T, HV, torch.float32)
