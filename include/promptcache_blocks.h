@@ -18,6 +18,7 @@ extern "C" {
 
 #define PCB_ABI_VERSION 6
 #define PCB_OK 0
+#define PCB_NOT_TAKEN 1 /* pcb_norm_linear only: sizes or alignments it does not take; nothing was launched */
 #define PCB_ERR_ARG (-2001)
 #define PCB_ERR_HIP_BASE (-3000)
 
@@ -749,6 +750,33 @@ typedef struct pcb_attn_step_args {
 } pcb_attn_step_args;
 int pcb_attn_step(const pcb_attn_step_args* a, void* stream);
 int pcb_attn_step_fits(int32_t dtype, int32_t H, int32_t Hkv, int32_t dim, int32_t vdim, int32_t rot_dims, int32_t latent);
+
+/* A step's residual rows, their norm and the one or two products (b may be null) that read the normed rows, in one launch:
+ *   table       x[r] = scale * fp32(table[ids[r]])                                   (table E [vocab][K], as pcb_embed_scaled_rows)
+ *   n_terms > 0 x[r] = sum_j coef[j] * x[j][r]                                       (streams x_stride elements apart, as pcb_mix_norm)
+ *   y           t = y[r] * gate[r];  x[r] + t / sqrt(mean(t^2) + eps) * post_gain    (gate E, rows ldg apart, as pcb_post_norm)
+ *   x_out[r] = x[r];  the products' rows are x[r] / sqrt(mean(x[r]^2) + eps) * gain (b's: gain2) as E; a->x and b->x are only checked, not read
+ * x_out is none of the rows read.  a is a plain store, b one or, with y, a gated unit.  PCB_NOT_TAKEN: beyond a few rows of a
+ * few thousand elements, not in whole 16-byte pieces, or so many columns that launches of their own are faster. */
+typedef struct pcb_row_norm_args {
+    uint32_t struct_bytes;
+    const float* x;
+    int64_t x_stride;
+    const float* coef;
+    int32_t n_terms;
+    const void* table;
+    const int32_t* ids;
+    int32_t vocab;
+    float scale;
+    const float* y;
+    const void* gate;
+    int64_t ldg;
+    const float* post_gain;
+    const float *gain, *gain2;
+    float* x_out;
+    float eps;
+} pcb_row_norm_args;
+int pcb_norm_linear(const pcb_row_norm_args* n, const pcb_linear_args* a, const pcb_linear_args* b, void* stream);
 
 /* Recurrences with a matrix state S [dim][vdim] per (slot, head), fp32, zero before position 0.  Per token and head h:
  *   q = q_scale q^, k = k_scale k^        q^, k^: E rows with head h / (H / Hk) at column (h / (H / Hk)) * dim; unit_norm: divided by

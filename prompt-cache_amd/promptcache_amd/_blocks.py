@@ -17,6 +17,7 @@ _lib: Optional[C.CDLL] = None
 BF16, F32 = 0, 1
 EPI_STORE, EPI_SILU_MUL, EPI_SCALE_ADD = 0, 1, 2
 ACT_NONE, ACT_SILU, ACT_SIGMOID, ACT_RELU2, ACT_SOFTPLUS, ACT_SOFTCAP, ACT_RELU, ACT_GELU_TANH, ACT_LOGSIGMOID, ACT_SCALE = range(10)
+NOT_TAKEN, NORM_LINEAR_MAX = 1, 4096                               # (what norm_linear takes: rows x columns)
 NORM_NONE, NORM_RMS, NORM_DYT = 0, 1, 2
 SCORE_SIGMOID, SCORE_SOFTMAX = 0, 1
 ABI_VERSION = 6
@@ -186,6 +187,13 @@ class AttnStepArgs(C.Structure):
                 ("ld_keep", _i64), ("n_splits", _i32), ("part", _vp)]
 
 
+class RowNormArgs(C.Structure):
+    """``pcb_row_norm_args`` (field for field)."""
+    _fields_ = [("struct_bytes", C.c_uint32), ("x", _vp), ("x_stride", _i64), ("coef", _vp), ("n_terms", _i32),
+                ("table", _vp), ("ids", _vp), ("vocab", _i32), ("scale", _f32), ("y", _vp), ("gate", _vp), ("ldg", _i64), ("post_gain", _vp),
+                ("gain", _vp), ("gain2", _vp), ("x_out", _vp), ("eps", _f32)]
+
+
 class RecArgs(C.Structure):
     """``pcb_rec_args`` (field for field)."""
     _fields_ = [("struct_bytes", C.c_uint32), ("dtype", _i32),
@@ -205,6 +213,7 @@ SIGNATURES = {
     "pcb_embed_scaled_rows": (C.c_int, [_vp, _i32, _vp, _f32, _vp, _i32, _i32, _i32, _vp]),
     "pcb_mix_norm": (C.c_int, [C.POINTER(MixNormArgs), _vp]),
     "pcb_linear": (C.c_int, [C.POINTER(LinearArgs), _vp]),
+    "pcb_norm_linear": (C.c_int, [C.POINTER(RowNormArgs), C.POINTER(LinearArgs), C.POINTER(LinearArgs), _vp]),
     "pcb_linear_pair": (C.c_int, [C.POINTER(LinearArgs), C.POINTER(LinearArgs), _vp]),
     "pcb_linear_add2": (C.c_int, [C.POINTER(LinearArgs), C.POINTER(LinearArgs), _vp, _vp, _f32, _vp]),
     "pcb_polynorm": (C.c_int, [_vp, _vp, _vp, _i32, _f32, _i32, _i32, _vp]),
@@ -439,6 +448,30 @@ def linear_add2(a: LinearArgs, b: LinearArgs, z: Optional[torch.Tensor] = None, 
         _want(z, torch.float32, "linear_add2 z"); _want(coef, torch.float32, "linear_add2 coef")
         assert coef.numel() == 4 and z.shape[-1] == b.K and z.shape[0] >= b.M
     check(load().pcb_linear_add2(C.byref(a), C.byref(b), _p(z), _p(coef), float(eps), _stream()), "pcb_linear_add2")
+
+
+def norm_linear(a: LinearArgs, b: Optional[LinearArgs], gain: torch.Tensor, gain2: Optional[torch.Tensor], x_out: torch.Tensor, *, eps: float, x=None, coef=None,
+                n_terms: int = 0, table=None, ids=None, scale: float = 1.0, y=None, gate=None, ldg: int = 0, post_gain=None) -> bool:
+    """Residual rows -- of a ``table``, the sum of ``n_terms`` streams ``x`` [streams, rows, width], or ``x`` and a gated sublayer's result ``y`` behind its norm
+    -- into ``x_out``, and one or two products (``linear_args``) of the normed rows.  False: not of the sizes that one launch takes, nothing done."""
+    M, W = a.M, a.K
+    for t, nm in ((gain, "gain"), (gain2, "gain2"), (x_out, "x_out"), (x, "x"), (coef, "coef"), (y, "y"), (post_gain, "post_gain")):
+        _want(t, torch.float32, "norm_linear " + nm)
+    _want(ids, torch.int32, "norm_linear ids")
+    assert gain.numel() == W and (gain2 is None or gain2.numel() == W) and (post_gain is None or post_gain.numel() == W) and x_out.numel() >= M * W
+    assert (table is not None) + (n_terms > 0) + (y is not None) == 1
+    if table is not None:
+        assert _code(table) == a.dtype and table.is_contiguous() and table.shape[1] == W and ids.numel() >= M
+    elif y is not None:
+        assert x.numel() >= M * W and y.numel() >= M * W and _code(gate) == a.dtype and _reach(gate) >= (M - 1) * ldg + W
+    else:
+        assert x.dim() == 3 and x.shape[0] >= n_terms and x.shape[1] >= M and x.shape[2] == W and coef.numel() >= n_terms
+    n = RowNormArgs(C.sizeof(RowNormArgs), _p(x), x.stride(0) if n_terms else 0, _p(coef), n_terms, _p(table), _p(ids), table.shape[0] if table is not None else 0,
+                    float(scale), _p(y), _p(gate), ldg, _p(post_gain), _p(gain), _p(gain2), _p(x_out), float(eps))
+    rc = load().pcb_norm_linear(C.byref(n), C.byref(a), None if b is None else C.byref(b), _stream())
+    if rc != NOT_TAKEN:
+        check(rc, "pcb_norm_linear")
+    return rc != NOT_TAKEN
 
 
 def polynorm(z: torch.Tensor, coef: torch.Tensor, out: torch.Tensor, eps: float, n_rows: int) -> None:

@@ -381,30 +381,47 @@ class FivesunHIP(SlotModel):
         tb = self._tables(dblob, d)
         layers = self.layers if num_layers is None else self.layers[:num_layers]
         eps = self.config.norm_eps
-        x = self._mat("x", T, W, f32)
+        x, spare = self._mat("x", T, W, f32), self._mat("x_next", T, W, f32)
         h = self._mat("h", T, W, E)
         y1, y2 = self._mat("y1", T, W, f32), self._mat("y2", T, W, f32)
         streams = torch.empty((len(layers), T, W), dtype=f32, device=dev) if return_streams else None
-        B.embed_scaled_rows(self.embed, tb["ids"], self.config.embed_scale, x)
+        rows = dict(table=self.embed, ids=tb["ids"], scale=self.config.embed_scale)      # where x comes from, until it is there
         pending = {}                               # the sublayer result that is still to be gated, normed and added to x
 
         def step(gain, out, **kw):
-            nonlocal pending
+            nonlocal rows, pending
+            if rows:
+                B.embed_scaled_rows(*rows.values(), x)
             B.post_norm(x, gain=gain, out=out, eps=eps, n_rows=kw.pop("n_rows", T), **pending, **kw)
-            pending = {}
+            rows, pending = {}, {}
+
+        def project(gain, a, b=None):
+            """The products ``a`` and, where given, ``b`` of the normed rows: for one or two rows the norm goes into their launch."""
+            nonlocal x, spare, rows, pending
+            if T * W <= B.NORM_LINEAR_MAX and (rows or pending):
+                to = x if rows else spare
+                if B.norm_linear(a, b, gain, gain if b else None, to, eps=eps, **(rows or dict(x=x, **pending))):
+                    x, spare = to, x if to is spare else spare
+                    rows, pending = {}, {}
+                    return
+            step(gain, h)
+            if b:
+                B.linear_pair(a, b)
+            else:
+                B.linear_run(a)
 
         for i, lw in enumerate(layers):
             l = lw["cfg"]
-            step(lw["norm1"], h)
-            gate, ldg = getattr(self, "_" + l.kind)(arena, i, l, lw, h, y1, tb, T, R)
+            P = self._mat("mix_in", T, lw["w_in"].shape[0], E)
+            project(lw["norm1"], B.linear_args(h, lw["w_in"], P, M=T, bias=lw["b_in"], act_split=lw["act_from"], act2=B.ACT_SIGMOID))
+            gate, ldg = getattr(self, "_" + l.kind)(arena, i, l, lw, P, y1, tb, T, R)
             pending = dict(y=y1, gate=gate, ldg=ldg, post_gain=lw["norm1b"])
             if l.ff:
-                step(lw["norm2"], h)
                 rg = self._mat("ff_gate", T, W, E)
                 mid = self._mat("ff_mid", T, l.ff, E)
-                B.linear_pair(B.linear_args(h, lw["rg2"], rg, M=T, bias=lw["rg2b"], act=B.ACT_SIGMOID),
-                              B.linear_args(h, lw["w_gate"], mid, M=T, epilogue=B.EPI_SILU_MUL, w2=lw["w_up"], bias=lw["b_gate"], bias2=lw["b_up"],
-                                            act=ACTS[l.act]))
+                project(lw["norm2"], B.linear_args(h, lw["rg2"], rg, M=T, bias=lw["rg2b"], act=B.ACT_SIGMOID),
+                        B.linear_args(h, lw["w_gate"], mid, M=T, epilogue=B.EPI_SILU_MUL, w2=lw["w_up"], bias=lw["b_gate"], bias2=lw["b_up"],
+                                      act=ACTS[l.act]))
                 B.linear(mid, lw["w_down"], y2, M=T, bias=lw["b_down"])
                 pending = dict(y=y2, gate=rg, ldg=W, post_gain=lw["norm2b"])
             if streams is not None:
@@ -417,13 +434,7 @@ class FivesunHIP(SlotModel):
             B.linear(hn, self.head, logits, M=nw)
         return (logits, streams) if return_streams else logits
 
-    # ---- mixers (each leaves its result in y, fp32 [T, W], and returns where the residual gate's sigmoid lies) --------------------
-    def _project_in(self, lw, h, T):
-        N = lw["w_in"].shape[0]
-        P = self._mat("mix_in", T, N, self.dtype)
-        B.linear(h, lw["w_in"], P, M=T, bias=lw["b_in"], act_split=lw["act_from"], act2=B.ACT_SIGMOID)
-        return P, N
-
+    # ---- mixers (each gets its projected rows P, leaves its result in y, fp32 [T, W], and returns where the residual gate's sigmoid lies) --------------------
     def _splits(self, n, groups, heads, reach, full=768):
         """Into how many runs the keys of ``n`` rows are cut (the kernels of single rows: ``n * groups`` workgroups a run, ``full`` of them at a
         time).  Rounds of the chip times a run's blocks of 64 keys and what starting one costs, and the merge: us, 8 heads over 2, 30 000 keys,
@@ -437,11 +448,11 @@ class FivesunHIP(SlotModel):
                     best = min(best, (-(-w * s // full) * (-(-blocks // s) + 2) + 1 + n * heads / 1200, s))
         return best[1]
 
-    def _attention(self, arena, i, l, lw, h, y, tb, T, R):
+    def _attention(self, arena, i, l, lw, P, y, tb, T, R):
         E = self.dtype
         H, G, D, Dv = l.heads, l.kv_heads, l.dim, l.vdim
         HD, GD, GV = H * D, G * D, G * Dv
-        P, N = self._project_in(lw, h, T)
+        N = P.shape[1]
         plane = arena.planes[i]
         vf = self._mat("v_first", T, GV, torch.float32) if l.v_mix else None
         reach = min(arena.cap, l.mask or arena.cap)
@@ -486,11 +497,11 @@ class FivesunHIP(SlotModel):
         B.linear(att, lw["wo"], y, M=T)
         return P[:, HD + GD + GV + H:], N
 
-    def _latent_attention(self, arena, i, l, lw, h, y, tb, T, R):
+    def _latent_attention(self, arena, i, l, lw, P, y, tb, T, R):
         E = self.dtype
         H, D, Rd, Dv, C = l.heads, l.dim, l.rot_dim, l.vdim, l.kv_rank
         DR, HQ, HV, CR = D + Rd, H * (D + Rd), H * Dv, C + Rd
-        P, N = self._project_in(lw, h, T)
+        N = P.shape[1]
         plane = arena.planes[i]
         off = tb["offs"][self._sigs.index((1, CR))]
         tiled = lw["prompts"] and tb["l_tiles"].numel() > 0
@@ -551,10 +562,10 @@ class FivesunHIP(SlotModel):
         B.linear(og, lw["wo"], y, M=T)
         return P[:, HQ + CR + HV:], N
 
-    def _mlstm(self, arena, i, l, lw, h, y, tb, T, R):
+    def _mlstm(self, arena, i, l, lw, P, y, tb, T, R):
         H, D, Dv = l.heads, l.dim, l.vdim
         HD, HV = H * D, H * Dv
-        P, N = self._project_in(lw, h, T)
+        N = P.shape[1]
         cols = (P, P[:, HD:], P[:, 2 * HD:], P[:, 2 * HD + HV:], P[:, 2 * HD + HV + H:], N)
         state, ns = arena.states[i][0], tb["n_seg"]
         rec = B.mlstm_state_floats(H, D, Dv)

@@ -187,32 +187,35 @@ class KazolornHIP(SlotModel):
         x = self._mat("x", T, W, f32)
         h1, h2 = self._mat("h1", T, W, E), self._mat("h2", T, W, E)
         streams = torch.empty((L, T, W), dtype=f32, device=dev) if return_streams else None
-        B.embed_rows(self.embed, ids_d, hist[0])
         eps = self.config.norm_eps
 
         for i, lw in enumerate(layers):
             l = lw["cfg"]
             has_ff = l.mlp_kind is not None
-            if i == 0:
-                B.mix_norm(hist, 1, None, lw["g1"], h1, lw.get("g2"), h2 if has_ff else None, eps=eps, n_rows=T)
-                base = hist[0]
-            else:
-                B.mix_norm(hist, i + 1, layers[i - 1]["dwa"], lw["g1"], h1, lw.get("g2"), h2 if has_ff else None, x_out=x,
-                           eps=eps, n_rows=T)
-                base = x
-                if streams is not None:
-                    streams[i - 1].copy_(x)
+            base = x if i else hist[0]
             HD, GD = l.heads * l.dim, l.kv_heads * l.dim
             q = self._mat("q", T, HD, E)
             plane = arena.planes[i]
             qk = B.linear_args(h1, lw["wqk"], q, M=T, bias=lw["bqk"], split_n=HD, y2=plane, row_off2=offs_d[sigs.index((l.kv_heads, l.dim))],
                                head_dim2=l.dim, head_stride2=arena.head_stride(i))
+            up = None
             if l.mlp_kind == "dense":
-                # (both halves of a layer start from the same input: their products go out two by two)
                 z, act = self._mat("z", T, l.ff, f32), self._mat("act", T, l.ff, E)
-                B.linear_pair(qk, B.linear_args(h2, lw["up"], z, M=T))
-            else:
-                B.linear_run(qk)
+                up = B.linear_args(h2, lw["up"], z, M=T)
+            rows = dict(x=hist, n_terms=i + 1, coef=layers[i - 1]["dwa"]) if i else dict(table=self.embed, ids=ids_d)
+            # (one or two rows: the embedding or the streams' sum and the norms in the launch of the layer's first products)
+            if not (up and T * W <= B.NORM_LINEAR_MAX and B.norm_linear(qk, up, lw["g1"], lw["g2"], base, eps=eps, **rows)):
+                if not i:
+                    B.embed_rows(self.embed, ids_d, hist[0])
+                B.mix_norm(hist, i + 1, layers[i - 1]["dwa"] if i else None, lw["g1"], h1, lw.get("g2"), h2 if has_ff else None, x_out=x if i else None,
+                           eps=eps, n_rows=T)
+                # (both halves of a layer start from the same input: their products go out two by two)
+                if up:
+                    B.linear_pair(qk, up)
+                else:
+                    B.linear_run(qk)
+            if i and streams is not None:
+                streams[i - 1].copy_(x)
             att = self._mat("att", T, HD, E)
             self._attention(q, att, tiles, n_tiles, tiles_d, tiles64_d, n64, plane, arena, i, l, lw, max_kv,
                             max_rows=1 if n_tiles == T else (int(tiles[:, 2].max()) if tiles is not None and n64 == n_tiles else 0))
