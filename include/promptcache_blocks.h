@@ -713,7 +713,9 @@ int pcb_attn_rows(const pcb_attn_rows_args* a, void* stream);
  * mixed with other's by blend[0] (may be null; as in pcb_head_prep_seg).  The new key and value go to k / v as in pcb_attn_rows_args.
  * latent: one key head whose row is (latent of vdim columns, normed, k_gain | dim - vdim turned columns), from k_at on; the values are its first vdim columns (v = k);
  * queries: folded parts of vdim columns in q (head h of row r at r ldq + h dim), the turned parts from q_at on.
- * gate: E, one number per row and head, or null.  pcb_attn_step_fits: whether heads of these sizes are taken. */
+ * gate: E, one number per row and head, or null.  pcb_attn_step_fits: whether heads of these sizes are taken.
+ * up (latent, may be null): E [H][up_dim][vdim], up_dim <= 128 in eights; the merging launch (any n_splits, part is needed) takes head h's result, unrounded, through
+ * up[h] and stores it times up_gate (E [rows], ld_up_gate apart) as out (H * up_dim columns). */
 typedef struct pcb_attn_step_args {
     uint32_t struct_bytes;
     int32_t dtype;
@@ -747,6 +749,10 @@ typedef struct pcb_attn_step_args {
     int64_t ld_keep;
     int32_t n_splits;
     float* part;
+    const void* up;
+    int32_t up_dim;
+    const void* up_gate;
+    int64_t ld_up_gate;
 } pcb_attn_step_args;
 int pcb_attn_step(const pcb_attn_step_args* a, void* stream);
 int pcb_attn_step_fits(int32_t dtype, int32_t H, int32_t Hkv, int32_t dim, int32_t vdim, int32_t rot_dims, int32_t latent);

@@ -259,7 +259,7 @@ __global__ __launch_bounds__(64 * LW) void attn_step_kernel(pcb_attn_step_args a
     l += __shfl_xor(l, 32, 64);
     if (c >= n_h) return;
     const int h = h0 + c;
-    if (a.n_splits > 1) {                                            // as the merging launches of pcb_attn_rows and pcb_attn_latent read it
+    if (a.n_splits > 1 || (LATENT && a.up)) {                        // as the merging launches of pcb_attn_rows and pcb_attn_latent read it
         const int64_t run = ((int64_t)blockIdx.x * a.H + h) * a.n_splits + blockIdx.z;
         if (wave == 0 && g == 0) *reinterpret_cast<float2*>(a.part + (int64_t)a.n_rows * a.H * a.n_splits * vdim + 2 * run) = float2{m, l};
 #pragma unroll
@@ -325,6 +325,68 @@ __global__ __launch_bounds__(128) void attn_step_merge_kernel(pcb_attn_step_args
     }
 }
 
+// The same for a latent's runs with the heads' own up-projections and gates behind it: one workgroup per (row, head), the head's rows of `up` on their way while the
+// runs are merged, four lanes an output.  What bounds it: the way of the runs and of up's 49 KB to a CU.  A merge, a launch of H small products and one of gates were
+// 14 us of a step (8 rows, 16 heads of 128 over a latent of 192, 5 runs), this is 8.
+template <typename E>
+__global__ __launch_bounds__(256) void attn_step_up_kernel(pcb_attn_step_args a) {
+    constexpr int AHEAD = 8, PASS = 2, CH = 6;                       // 64 outputs a pass, chunks of 32 columns
+    __shared__ float fac[64];
+    __shared__ __attribute__((aligned(16))) float merged[32 * CH];
+    const int tid = threadIdx.x, lane = tid & 63, h = blockIdx.y, vdim = a.vdim, up = a.up_dim, Z = a.n_splits > 1 ? a.n_splits : 1;
+    const int64_t run = ((int64_t)blockIdx.x * a.H + h) * Z;
+    const float* pp = a.part + run * vdim;
+    const float* ml = a.part + (int64_t)a.n_rows * a.H * Z * vdim + 2 * run;
+    const int64_t row = a.tiles[4 * blockIdx.x + 3];
+    const int c0 = tid < vdim ? tid : 0;
+    const float2 mz = *reinterpret_cast<const float2*>(ml + 2 * (lane < Z ? lane : 0));
+    float first[AHEAD];
+#pragma unroll
+    for (int z = 0; z < AHEAD; ++z) first[z] = pp[(int64_t)(z < Z ? z : 0) * vdim + c0];
+    E gate[PASS];
+    Frag<E> w[PASS][CH];
+#pragma unroll
+    for (int p = 0; p < PASS; ++p) {
+        const int j = 64 * p + tid / 4 < up ? 64 * p + tid / 4 : up - 1;
+        gate[p] = ((const E*)a.up_gate)[row * a.ld_up_gate + (int64_t)h * up + j];
+        const E* wr = (const E*)a.up + ((int64_t)h * up + j) * vdim;
+#pragma unroll
+        for (int i = 0; i < CH; ++i) w[p][i] = load8(wr + (32 * i < vdim ? 32 * i : 0) + 8 * (tid & 3));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };      // (what is under way stays so)
+    if (tid < 64) {
+        const float m = lane < Z ? mz.x : -__builtin_inff(), l = lane < Z ? mz.y : 0.0f;
+        const float f = __builtin_amdgcn_exp2f(m - wave_max(m));     // (the row sees itself: the largest is a number)
+        fac[lane] = f / wave_sum(f * l);
+    }
+    barrier();
+    if (tid < vdim) {
+        float o = 0.0f;
+#pragma unroll
+        for (int z = 0; z < AHEAD; ++z)
+            if (z < Z) o += fac[z] * first[z];
+#pragma unroll 8
+        for (int z = AHEAD; z < Z; ++z) o += fac[z] * pp[(int64_t)z * vdim + tid];      // (an empty run left zeros)
+        merged[tid] = o;
+    }
+    barrier();
+#pragma unroll
+    for (int p = 0; p < PASS; ++p) {
+        const int j = 64 * p + tid / 4;
+        float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < CH; ++i)
+            if (32 * i < vdim)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) acc[e & 3] += at8(w[p][i], e) * merged[32 * i + 8 * (tid & 3) + e];
+        float o = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+        o += __shfl_xor(o, 1, 64);
+        o += __shfl_xor(o, 2, 64);
+        if ((tid & 3) == 0 && j < up) ((E*)a.out)[row * a.ldo + (int64_t)h * up + j] = from_f32<E>(o * to_f32(gate[p]));
+    }
+}
+
 template <typename E>
 int dispatch(const pcb_attn_step_args& a, hipStream_t stream) {
     const int per = a.H / a.Hkv;
@@ -335,7 +397,10 @@ int dispatch(const pcb_attn_step_args& a, hipStream_t stream) {
         hipLaunchKernelGGL((attn_step_kernel<E, 2, 1, false>), grid, block, 0, stream, a);
     else
         hipLaunchKernelGGL((attn_step_kernel<E, 4, 2, false>), grid, block, 0, stream, a);
-    if (a.n_splits > 1) hipLaunchKernelGGL(attn_step_merge_kernel<E>, dim3(a.n_rows, a.H), dim3(128), 0, stream, a);
+    if (a.up)
+        hipLaunchKernelGGL(attn_step_up_kernel<E>, dim3(a.n_rows, a.H), dim3(256), 0, stream, a);
+    else if (a.n_splits > 1)
+        hipLaunchKernelGGL(attn_step_merge_kernel<E>, dim3(a.n_rows, a.H), dim3(128), 0, stream, a);
     return pcb_check_launch("attn_step_kernel");
 }
 
@@ -357,10 +422,13 @@ PCB_EXPORT int pcb_attn_step(const pcb_attn_step_args* a, void* stream) {
     if (a->n_rows == 0) return PCB_OK;
     PCB_REQUIRE(a->p && a->tiles && a->k && a->v && a->out && (a->rot_dims == 0 || a->freqs) && (!a->latent || a->q), PCB_ERR_ARG, "pcb_attn_step: null pointer");
     PCB_REQUIRE((!a->blend || (a->other && a->ld_other >= (int64_t)a->Hkv * a->vdim)) && (!a->keep || a->ld_keep >= (int64_t)a->Hkv * a->vdim) &&
-                    (!a->gate || a->ldg >= a->H) && a->ldo >= (int64_t)a->H * a->vdim && (!a->latent || a->ldq >= (int64_t)a->H * a->dim) &&
+                    (!a->gate || a->ldg >= a->H) && a->ldo >= (int64_t)a->H * (a->up ? a->up_dim : a->vdim) && (!a->latent || a->ldq >= (int64_t)a->H * a->dim) &&
                     a->k_cols >= (a->latent ? 0 : a->dim) && a->k_row_stride >= a->dim && a->v_row_stride >= a->vdim && a->k_slot_stride >= 0 && a->k_head_stride >= 0 &&
                     a->v_slot_stride >= 0 && a->v_head_stride >= 0 && a->q_head_stride >= 0 && a->q_at >= 0 && a->k_at >= 0 && a->v_at >= 0,
                 PCB_ERR_ARG, "pcb_attn_step: bad strides");
+    PCB_REQUIRE(!a->up || (a->latent && !a->sink && !a->gate && a->up_gate && a->up_dim > 0 && a->up_dim <= 128 && a->up_dim % 8 == 0 && a->part &&
+                           (uintptr_t)a->up % 16 == 0 && a->ld_up_gate >= (int64_t)a->H * a->up_dim),
+                PCB_ERR_ARG, "pcb_attn_step: up-projections of a latent's heads, up to 128 columns in eights, with their gates and scratch");
     PCB_REQUIRE(a->n_splits <= 1 || (a->part && (uintptr_t)a->part % 16 == 0 && a->n_splits <= 64), PCB_ERR_ARG, "pcb_attn_step: up to 64 runs, with their scratch");
     const int es = a->dtype == PCB_BF16 ? 2 : 4;
     const int64_t whole = a->k_slot_stride | a->k_head_stride | a->k_row_stride | a->v_slot_stride | a->v_head_stride | a->v_row_stride | a->ldo | (a->latent ? a->ldq : 0);

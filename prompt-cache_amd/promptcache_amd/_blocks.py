@@ -184,7 +184,7 @@ class AttnStepArgs(C.Structure):
                 ("H", _i32), ("Hkv", _i32), ("dim", _i32), ("vdim", _i32), ("latent", _i32), ("scale", _f32), ("window", _i32), ("block", _i32),
                 ("sink", _vp), ("gate", _vp), ("ldg", _i64), ("out", _vp), ("ldo", _i64), ("q_gain", _vp), ("k_gain", _vp), ("eps", _f32),
                 ("rot_dims", _i32), ("freqs", _vp), ("rot_mag", _f32), ("blend", _vp), ("other", _vp), ("ld_other", _i64), ("keep", _vp),
-                ("ld_keep", _i64), ("n_splits", _i32), ("part", _vp)]
+                ("ld_keep", _i64), ("n_splits", _i32), ("part", _vp), ("up", _vp), ("up_dim", _i32), ("up_gate", _vp), ("ld_up_gate", _i64)]
 
 
 class RowNormArgs(C.Structure):
@@ -1013,17 +1013,18 @@ def attn_step_fits(dtype: torch.dtype, H: int, Hkv: int, dim: int, vdim: int, ro
 def attn_step(p: torch.Tensor, tiles: torch.Tensor, n_rows: int, k: torch.Tensor, k_strides, v: torch.Tensor, v_strides, H: int, Hkv: int, dim: int,
               vdim: int, scale: float, out: torch.Tensor, *, q_at: int, q_head_stride: int, k_at: int, v_at: int = 0, q=None, q_gain=None, k_gain=None,
               eps: float, rot_dims: int = 0, freqs=None, rot_mag: float = 1.0, blend=None, other=None, keep=None, window: int = 0, block: int = 0, sink=None,
-              gate=None, ldg: int = 0, n_splits: int = 1, part=None) -> None:
+              gate=None, ldg: int = 0, n_splits: int = 1, part=None, up=None, up_gate=None, ld_up_gate: int = 0) -> None:
     """A decoding step of an attention layer behind its projection ``p`` [rows, columns]: ``head_prep`` of queries, keys and values and ``attn_rows`` over the cached rows
     and the new one; with ``q`` [rows, H * dim] (the folded queries) ``attn_latent``'s form: one key head, its first ``vdim`` columns the values.  Every row is
     the only one of its slot.  ``k_strides`` / ``v_strides``: (slot, head, row) strides; ``other`` / ``keep``: fp32 [rows, Hkv * vdim]; ``gate``: E, one number per row and head;
-    ``n_splits`` / ``part`` as in ``attn_rows``."""
+    ``n_splits`` / ``part`` as in ``attn_rows``; ``up`` [H, columns, vdim] (latent): head h's result goes on through ``up[h]``, times ``up_gate``
+    (E [rows, H * columns]), into ``out``."""
     latent = q is not None
     _want(tiles, torch.int32, "attn_step tiles"); _want(sink, torch.float32, "attn_step sink"); _want(freqs, torch.float64, "attn_step freqs")
     for t, nm in ((q_gain, "q_gain"), (k_gain, "k_gain"), (blend, "blend"), (other, "other"), (keep, "keep")):
         _want(t, torch.float32, "attn_step " + nm)
     assert p.dtype == k.dtype == v.dtype == out.dtype and p.is_contiguous() and out.is_contiguous() and p.shape[0] >= n_rows and out.shape[0] >= n_rows
-    assert tiles.numel() >= 4 * n_rows and out.shape[-1] == H * vdim and (sink is None or sink.numel() >= H)
+    assert tiles.numel() >= 4 * n_rows and out.shape[-1] == H * (vdim if up is None else up.shape[1]) and (sink is None or sink.numel() >= H)
     assert q_at + (H - 1) * q_head_stride + (dim - vdim if latent else dim) <= p.shape[-1]
     assert k_at + (dim if latent else Hkv * dim) <= p.shape[-1] and (latent or v_at + Hkv * vdim <= p.shape[-1])
     assert rot_dims == 0 or freqs.numel() >= rot_dims // 2
@@ -1032,11 +1033,13 @@ def attn_step(p: torch.Tensor, tiles: torch.Tensor, n_rows: int, k: torch.Tensor
     assert all(t is None or (t.shape[-1] == Hkv * vdim and t.shape[0] >= n_rows) for t in (other, keep)) and (blend is None or other is not None)
     assert gate is None or (gate.dtype == p.dtype and ldg >= H)
     _want(part, torch.float32, "attn_step part")
-    assert n_splits <= 1 or (part is not None and part.numel() >= attn_softmax_part(n_rows, H, n_splits, vdim))
+    assert up is None or (up.dtype == p.dtype == up_gate.dtype and up.is_contiguous() and up.dim() == 3 and up.shape[0] == H and up.shape[2] == vdim and
+                          _reach(up_gate) >= (n_rows - 1) * ld_up_gate + H * up.shape[1])
+    assert (n_splits <= 1 and up is None) or (part is not None and part.numel() >= attn_softmax_part(n_rows, H, n_splits, vdim))
     a = AttnStepArgs(C.sizeof(AttnStepArgs), _code(p), _p(p), p.shape[-1], q_at, q_head_stride, k_at, dim, v_at, _p(q), q.shape[-1] if latent else 0, _p(tiles),
                      n_rows, _p(k), *(int(x) for x in k_strides), _p(v), *(int(x) for x in v_strides), H, Hkv, dim, vdim, int(latent), float(scale),
                      int(window), int(block), _p(sink), _p(gate), ldg, _p(out), out.shape[-1], _p(q_gain), _p(k_gain), float(eps), rot_dims, _p(freqs),
-                     float(rot_mag), _p(blend), _p(other), Hkv * vdim, _p(keep), Hkv * vdim, n_splits, _p(part))
+                     float(rot_mag), _p(blend), _p(other), Hkv * vdim, _p(keep), Hkv * vdim, n_splits, _p(part), _p(up), 0 if up is None else up.shape[1], _p(up_gate), ld_up_gate)
     check(load().pcb_attn_step(C.byref(a), _stream()), "pcb_attn_step")
 
 

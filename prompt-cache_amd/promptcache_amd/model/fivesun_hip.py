@@ -435,18 +435,24 @@ class FivesunHIP(SlotModel):
         return (logits, streams) if return_streams else logits
 
     # ---- mixers (each gets its projected rows P, leaves its result in y, fp32 [T, W], and returns where the residual gate's sigmoid lies) --------------------
-    def _splits(self, n, groups, heads, reach, full=768):
+    def _splits(self, n, groups, heads, reach, full=768, unit=64, merged=False):
         """Into how many runs the keys of ``n`` rows are cut (the kernels of single rows: ``n * groups`` workgroups a run, ``full`` of them at a
-        time).  Rounds of the chip times a run's blocks of 64 keys and what starting one costs, and the merge: us, 8 heads over 2, 30 000 keys,
-        cut for 512 workgroups / by this rule: 16 rows 73 / 65, 64 236 / 216, 128 455 / 400, 256 930 / 749, 512 1 678 / 1 381."""
-        blocks, w = -(-reach // 64), n * groups
+        time).  Rounds of the chip times a run's blocks of ``unit`` keys and what starting one costs, and the merge, unless that is a launch anyhow (``merged``):
+        us, 8 heads over 2, 30 000 keys, cut for 512 workgroups / by this rule: 16 rows 73 / 65, 64 236 / 216, 128 455 / 400, 256 930 / 749, 512 1 678 / 1 381."""
+        blocks, w, join = -(-reach // unit), n * groups, 0 if merged else 1 + n * heads / 1200
         best = (-(-w // full) * (blocks + 2), 1)
-        if blocks > 3:
+        if blocks > (1 if merged else 3):
             for k in range(1, 5):
                 s = min(64, blocks, full * k // w)
                 if s > 1:
-                    best = min(best, (-(-w * s // full) * (-(-blocks // s) + 2) + 1 + n * heads / 1200, s))
+                    best = min(best, (-(-w * s // full) * (-(-blocks // s) + 2) + join, s))
         return best[1]
+
+    def _step_splits(self, n, groups, heads, reach, full=768, merged=False):
+        """The same for a step's single tokens: in fp32, whose blocks are 32 keys, by these while every block finds a CU of its own.  us a step, width 1024, 64 / 32: one
+        of 150 keys 191 / 169, two of 300 183 / 178, of 1000 184 / 180, eight of 300 234 / 229, of 1000 (512 blocks) 234 / 240, 32 of 300 (640) 366 / 368."""
+        unit = 32 if self.dtype == torch.float32 and n * groups * -(-reach // 32) <= 256 else 64
+        return self._splits(n, groups, heads, reach, full, unit, merged)
 
     def _attention(self, arena, i, l, lw, P, y, tb, T, R):
         E = self.dtype
@@ -457,7 +463,7 @@ class FivesunHIP(SlotModel):
         vf = self._mat("v_first", T, GV, torch.float32) if l.v_mix else None
         reach = min(arena.cap, l.mask or arena.cap)
         if tb["ones"] and B.attn_step_fits(E, H, G, D, Dv, l.rot_dims):      # (a row's own key is the only new one it sees)
-            splits = self._splits(T, G * -(-H // (16 * G)), H, reach)
+            splits = self._step_splits(T, G * -(-H // (16 * G)), H, reach)
             att, strides = self._mat("mix_out", T, H * Dv, E), (arena.slot_stride(i), arena.head_stride(i), D + Dv)
             part = self._scratch("attn_part", B.attn_softmax_part(T, H, splits, Dv), torch.float32) if splits > 1 else None
             B.attn_step(P, tb["s_tiles"], T, plane, strides, plane.view(-1)[D:], strides, H, G, D, Dv, l.scale, att, q_at=0, q_head_stride=D, k_at=HD,
@@ -509,18 +515,27 @@ class FivesunHIP(SlotModel):
         n = f_tiles.numel() // 4
         qa = self._mat("q_latent", T, H * CR, E) if n else None   # per head [W_uk^T q | rotated part]: a query over the cached rows
         reach = min(arena.cap, l.mask or arena.cap)
-        splits = self._splits(n, -(-H // 16), H, reach, 768 if CR <= 256 else 512) if n else 0
+        full = 768 if CR <= 256 else 512
         if tb["ones"] and n == T and B.attn_step_fits(E, H, 1, CR, C, Rd, True):
             B.linear(P, lw["w_abs"], qa, M=T, n_batch=H, ldx=N, x_batch_stride=DR, ldy=H * CR, y_batch_stride=CR)
-            ol, strides = self._mat("mix_out", T, H * C, E), (arena.slot_stride(i), 0, CR)
-            B.attn_step(P, f_tiles, T, plane, strides, plane, strides, H, 1, CR, C, l.scale, ol, q_at=D, q_head_stride=DR, k_at=HQ, q=qa, k_gain=lw["c_gain"],
-                        eps=self.config.norm_eps, rot_dims=Rd, freqs=lw["freqs"], rot_mag=lw["rot_mag"], window=l.mask, n_splits=splits,
-                        part=self._scratch("attn_part", B.attn_softmax_part(n, H, splits, C), torch.float32) if splits > 1 else None)
-            og, ov = self._mat("mix_gated", T, HV, E), self._mat("mix_o32", T, HV, torch.float32)
-            B.linear(ol, lw["w_uv"], ov, M=T, n_batch=H, ldx=H * C, x_batch_stride=C, ldy=HV, y_batch_stride=Dv)
-            B.gated_norm(ov, None, P[:, HQ + CR:], N, og, self.config.norm_eps, T)
+            # the heads' up-projections and gates ride in the launch that merges: us a step of 16 heads, bf16, without / with it: one of 300 keys 212 / 206, 8 of 300
+            # 287 / 281, 32 of 100 360 / 356, 64 of 60 397 / 396; 8 heads, fp32, two of 300 189 / 183
+            up = T <= 64 and Dv <= 128 and Dv % 8 == 0
+            splits = self._step_splits(T, -(-H // 16), H, reach, full, up)
+            strides, og, gate = (arena.slot_stride(i), 0, CR), self._mat("mix_gated", T, HV, E), P[:, HQ + CR:]
+            kw = dict(q_at=D, q_head_stride=DR, k_at=HQ, q=qa, k_gain=lw["c_gain"], eps=self.config.norm_eps, rot_dims=Rd, freqs=lw["freqs"],
+                      rot_mag=lw["rot_mag"], window=l.mask, n_splits=splits)
+            part = self._scratch("attn_part", B.attn_softmax_part(n, H, splits, C), torch.float32)
+            if up:
+                B.attn_step(P, f_tiles, T, plane, strides, plane, strides, H, 1, CR, C, l.scale, og, part=part, up=lw["w_uv"], up_gate=gate, ld_up_gate=N, **kw)
+            else:
+                ol, ov = self._mat("mix_out", T, H * C, E), self._mat("mix_o32", T, HV, torch.float32)
+                B.attn_step(P, f_tiles, T, plane, strides, plane, strides, H, 1, CR, C, l.scale, ol, part=part, **kw)
+                B.linear(ol, lw["w_uv"], ov, M=T, n_batch=H, ldx=H * C, x_batch_stride=C, ldy=HV, y_batch_stride=Dv)
+                B.gated_norm(ov, None, gate, N, og, self.config.norm_eps, T)
             B.linear(og, lw["wo"], y, M=T)
             return P[:, HQ + CR + HV:], N
+        splits = self._splits(n, -(-H // 16), H, reach, full) if n else 0
         q = self._mat("q_rows", T, HQ, E) if tiled else None      # per head [plain part | rotated part]: a query over rebuilt rows
         segs = [B.head_seg(P[:, HQ:], N, 1, C, plane, norm=True, gain=lw["c_gain"], row_off=off)]
         if tiled:

@@ -98,8 +98,9 @@ def test_heads(dtype, H, G, D, Dv, rot, block, window, splits):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("H,C,R,window", [(16, 192, 64, 0), (20, 64, 32, 100), (3, 32, 8, 0), (2, 160, 0, 33)])
-@pytest.mark.parametrize("splits", [1, 4])
-def test_latent(dtype, H, C, R, window, splits):
+@pytest.mark.parametrize("splits,up", [(1, 0), (4, 0), (1, 72), (4, 128), (11, 8), (64, 120)])
+def test_latent(dtype, H, C, R, window, splits, up):
+    """``up``: the heads' up-projections and gates in the merging launch."""
     b, n, cap, eps, D = B(), len(POS), 304, 1e-6, 24
     CR, DR, HQ = C + R, D + R, H * (D + R)
     P = rnd(n, HQ + CR + 8, seed=1, dtype=dtype)
@@ -112,11 +113,15 @@ def test_latent(dtype, H, C, R, window, splits):
     tiles = torch.tensor([[slot[r], POS[r], 1, r] for r in range(n)], dtype=torch.int32, device=DEV).reshape(-1)
     gain, out = rnd(C, seed=4), torch.zeros(n, H * C, dtype=dtype, device=DEV)
     freqs = torch.tensor([100.0 ** (-2 * i / max(R, 1)) for i in range(R // 2)], dtype=F64, device=DEV)
-    part = torch.full((b.attn_softmax_part(n, H, splits, C),), float("nan"), device=DEV) if splits > 1 else None
+    part = torch.full((b.attn_softmax_part(n, H, splits, C),), float("nan"), device=DEV) if splits > 1 or up else None
+    kw = {}
+    if up:
+        w, gate, out = rnd(H, up, C, seed=5, dtype=dtype, scale=C ** -0.5), rnd(n, H * up + 8, seed=6, dtype=dtype), torch.zeros(n, H * up, dtype=dtype, device=DEV)
+        kw = dict(up=w, up_gate=gate[:, 3:], ld_up_gate=H * up + 8)
     assert b.attn_step_fits(dtype, H, 1, CR, C, R, True)
     scale = 0.5 * CR ** -0.5
     b.attn_step(P, tiles, n, plane, (cap * CR, 0, CR), plane, (cap * CR, 0, CR), H, 1, CR, C, scale, out, q_at=D, q_head_stride=DR, k_at=HQ, q=qa, k_gain=gain,
-                eps=eps, rot_dims=R, freqs=freqs if R else None, rot_mag=0.75, window=window, n_splits=splits, part=part)
+                eps=eps, rot_dims=R, freqs=freqs if R else None, rot_mag=0.75, window=window, n_splits=splits, part=part, **kw)
     pos = torch.tensor(POS, device=DEV)
     c = unit(P[:, HQ:HQ + C], eps) * gain.to(F64)
     k = torch.cat([c, turned(P[:, None, HQ + C:HQ + CR].to(F64), pos, freqs, 0.75)[:, 0]], -1)
@@ -129,7 +134,9 @@ def test_latent(dtype, H, C, R, window, splits):
         full[slot[r], POS[r]] = new[r]
     full = full[:, None].expand(-1, H, -1, -1)
     want = attended(q.to(dtype).to(F64), full, full[..., :C], POS, slot, scale, [max(0, p - window + 1) if window else 0 for p in POS], None)
-    got = out.view(n, H, C).to(F64)
+    if up:
+        want = (w.to(F64) @ want[..., None])[..., 0] * gate[:, 3:3 + H * up].to(F64).view(n, H, up)
+    got = out.view(n, H, up or C).to(F64)
     assert float((got - want).norm() / want.norm()) < (6e-3 if dtype == torch.bfloat16 else 4e-6)
 
 
