@@ -58,6 +58,8 @@ typedef struct pcb_mix_norm_args {
     int32_t width;
 } pcb_mix_norm_args;
 int pcb_mix_norm(const pcb_mix_norm_args* a, void* stream);
+/* pcb_embed_scaled_rows into x_out and pcb_mix_norm of these rows (hist and rows null, n_terms 0) at once. */
+int pcb_embed_norm(const void* table, const int32_t* ids, float scale, int32_t vocab, const pcb_mix_norm_args* a, void* stream);
 
 /* Y = A W^T (+ bias), A = gathered / scaled rows of X.  W is [N][K] row-major (nn.Linear layout).
  *

@@ -191,6 +191,47 @@ __global__ __launch_bounds__(1024) void mix_norm_chunks_kernel(pcb_mix_norm_args
         }
 }
 
+// Embedding rows as the first stream and their norms, laid out as above: the row need not come back from memory, and a step is a launch shorter.  us, as two
+// launches / here, two norms: bf16 1 row of 1024 4.4 / 3.0, 8 of 2048 5.0 / 3.4, 600 8.3 / 5.5, 2048 16.8 / 12.1; one norm 2400 17.5 / 11.7, fp32 600 of 1024 7.4 / 4.2.
+template <typename E, int NC>
+__global__ __launch_bounds__(1024) void embed_norm_kernel(const E* __restrict__ table, const int32_t* __restrict__ ids, float scale, int vocab,
+                                                          pcb_mix_norm_args a) {
+    __shared__ float red[16];
+    const int r = blockIdx.x, W = a.width;
+    int id = ids[r];
+    id = id < 0 ? 0 : id >= vocab ? vocab - 1 : id;
+    const E* src = table + (int64_t)id * W;
+    int c[NC];
+    f4 x[NC], g1[NC], g2[NC];
+    float ss[1] = {0.0f};
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+        c[k] = 4 * (threadIdx.x + k * blockDim.x);
+        const int at = c[k] < W ? c[k] : 0;
+        float v[4];
+        load4(src + at, true, 4, v);
+        if (a.out1) g1[k] = ld4(a.gain1 + at);
+        if (a.out2) g2[k] = ld4(a.gain2 + at);
+        x[k] = scale * f4{v[0], v[1], v[2], v[3]};
+    }
+#pragma unroll
+    for (int k = 0; k < NC; ++k)
+        if (c[k] < W) {
+            *reinterpret_cast<f4*>(a.x_out + (int64_t)r * W + c[k]) = x[k];
+            ss[0] += (x[k][0] * x[k][0] + x[k][1] * x[k][1]) + (x[k][2] * x[k][2] + x[k][3] * x[k][3]);
+        }
+    row_sum<1>(ss, red);
+    const float inv = 1.0f / sqrtf(ss[0] / (float)W + a.eps);
+#pragma unroll
+    for (int k = 0; k < NC; ++k)
+        if (c[k] < W) {
+            const f4 v = x[k] * inv;
+            const int64_t at = (int64_t)r * W + c[k];
+            if (a.out1) store4((E*)a.out1 + at, v[0] * g1[k][0], v[1] * g1[k][1], v[2] * g1[k][2], v[3] * g1[k][3]);
+            if (a.out2) store4((E*)a.out2 + at, v[0] * g2[k][0], v[1] * g2[k][1], v[2] * g2[k][2], v[3] * g2[k][3]);
+        }
+}
+
 template <typename E>
 __global__ __launch_bounds__(1024) void polynorm_kernel(const float* __restrict__ z, const float* __restrict__ coef, E* __restrict__ out,
                                                        float eps, int ff) {
@@ -395,6 +436,34 @@ PCB_EXPORT int pcb_mix_norm(const pcb_mix_norm_args* a, void* stream) {
     else
         hipLaunchKernelGGL(mix_norm_kernel<float>, dim3(a->n_rows), threads, lds, (hipStream_t)stream, *a);
     return pcb_check_launch("mix_norm_kernel");
+}
+
+PCB_EXPORT int pcb_embed_norm(const void* table, const int32_t* ids, float scale, int32_t vocab, const pcb_mix_norm_args* a, void* stream) {
+    PCB_REQUIRE(a && a->struct_bytes == sizeof(pcb_mix_norm_args), PCB_ERR_ARG, "pcb_embed_norm: struct size mismatch");
+    PCB_REQUIRE(PCB_DTYPE_OK(a->dtype) && a->n_rows >= 0 && a->width > 0 && a->width <= 16384 && vocab > 0 && a->n_terms == 0 && !a->rows && !a->hist, PCB_ERR_ARG,
+                "pcb_embed_norm: bad sizes (width <= 16384), or rows of streams");
+    if (a->n_rows == 0) return PCB_OK;
+    PCB_REQUIRE(table && ids && a->x_out && (!a->out1 || a->gain1) && (!a->out2 || a->gain2), PCB_ERR_ARG, "pcb_embed_norm: null pointer");
+    const uintptr_t e4 = a->dtype == PCB_BF16 ? 8 : 16;              // (four elements of E)
+    int th, nc;
+    if (row_threads(a->width, a->n_rows, 2, &th, &nc) && ((uintptr_t)a->x_out | (uintptr_t)a->gain1 | (uintptr_t)a->gain2) % 16 == 0 &&
+        ((uintptr_t)a->out1 | (uintptr_t)a->out2 | (uintptr_t)table) % e4 == 0) {
+        auto go = [&](auto e) {
+            using E = decltype(e);
+            if (nc == 1)
+                hipLaunchKernelGGL((embed_norm_kernel<E, 1>), dim3(a->n_rows), dim3(th), 0, (hipStream_t)stream, (const E*)table, ids, scale, vocab, *a);
+            else
+                hipLaunchKernelGGL((embed_norm_kernel<E, 2>), dim3(a->n_rows), dim3(th), 0, (hipStream_t)stream, (const E*)table, ids, scale, vocab, *a);
+        };
+        if (a->dtype == PCB_BF16) go(bf16_t{}); else go(0.0f);
+        return pcb_check_launch("embed_norm_kernel");
+    }
+    const int rc = pcb_embed_scaled_rows(table, a->dtype, ids, scale, a->x_out, a->n_rows, a->width, vocab, stream);
+    if (rc != PCB_OK) return rc;
+    pcb_mix_norm_args rest = *a;
+    rest.hist = a->x_out;
+    rest.x_out = nullptr;
+    return pcb_mix_norm(&rest, stream);
 }
 
 PCB_EXPORT int pcb_polynorm(const float* z, const float* coef, void* out, int32_t dtype, float eps, int32_t n_rows, int32_t ff,

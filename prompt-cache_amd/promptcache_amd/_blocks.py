@@ -212,6 +212,7 @@ SIGNATURES = {
     "pcb_embed_rows": (C.c_int, [_vp, _i32, _vp, _vp, _i32, _i32, _i32, _vp]),
     "pcb_embed_scaled_rows": (C.c_int, [_vp, _i32, _vp, _f32, _vp, _i32, _i32, _i32, _vp]),
     "pcb_mix_norm": (C.c_int, [C.POINTER(MixNormArgs), _vp]),
+    "pcb_embed_norm": (C.c_int, [_vp, _vp, _f32, _i32, C.POINTER(MixNormArgs), _vp]),
     "pcb_linear": (C.c_int, [C.POINTER(LinearArgs), _vp]),
     "pcb_norm_linear": (C.c_int, [C.POINTER(RowNormArgs), C.POINTER(LinearArgs), C.POINTER(LinearArgs), _vp]),
     "pcb_linear_pair": (C.c_int, [C.POINTER(LinearArgs), C.POINTER(LinearArgs), _vp]),
@@ -353,6 +354,20 @@ def mix_norm(hist: torch.Tensor, n_streams: int, coef: Optional[torch.Tensor], g
                     n_streams if coef is not None else 0, _p(x_out), _p(rows), _p(gain1), _p(out1), _p(gain2), _p(out2),
                     float(eps), n, W)
     check(load().pcb_mix_norm(C.byref(a), _stream()), "pcb_mix_norm")
+
+
+def embed_norm(table: torch.Tensor, ids: torch.Tensor, scale: float, x_out: torch.Tensor, gain1: torch.Tensor, out1: torch.Tensor,
+               gain2: Optional[torch.Tensor] = None, out2: Optional[torch.Tensor] = None, *, eps: float) -> None:
+    """``embed_scaled_rows`` into ``x_out`` (fp32 [rows, width]) and ``mix_norm`` of these rows at once."""
+    n, W = x_out.shape
+    _want(ids, torch.int32, "embed_norm ids"); _want(x_out, torch.float32, "embed_norm x_out")
+    assert ids.numel() >= n and table.shape[1] == W and table.is_contiguous() and x_out.is_contiguous()
+    for g, o in ((gain1, out1), (gain2, out2)):
+        if o is not None:
+            _want(g, torch.float32, "embed_norm gain")
+            assert g.numel() == W and o.is_contiguous() and o.shape[-1] == W and o.numel() >= n * W and o.dtype == table.dtype
+    a = MixNormArgs(C.sizeof(MixNormArgs), _code(table), None, 0, None, 0, _p(x_out), None, _p(gain1), _p(out1), _p(gain2), _p(out2), float(eps), n, W)
+    check(load().pcb_embed_norm(_p(table), _p(ids), float(scale), table.shape[0], C.byref(a), _stream()), "pcb_embed_norm")
 
 
 def linear_args(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, *, M: int, epilogue: int = EPI_STORE, bias=None, w2=None,

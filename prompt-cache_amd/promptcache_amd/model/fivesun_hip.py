@@ -404,7 +404,11 @@ class FivesunHIP(SlotModel):
                     x, spare = to, x if to is spare else spare
                     rows, pending = {}, {}
                     return
-            step(gain, h)
+            if rows:
+                B.embed_norm(*rows.values(), x, gain, h, eps=eps)
+                rows = {}
+            else:
+                step(gain, h)
             if b:
                 B.linear_pair(a, b)
             else:

@@ -205,10 +205,11 @@ class KazolornHIP(SlotModel):
             rows = dict(x=hist, n_terms=i + 1, coef=layers[i - 1]["dwa"]) if i else dict(table=self.embed, ids=ids_d)
             # (one or two rows: the embedding or the streams' sum and the norms in the launch of the layer's first products)
             if not (up and T * W <= B.NORM_LINEAR_MAX and B.norm_linear(qk, up, lw["g1"], lw["g2"], base, eps=eps, **rows)):
-                if not i:
-                    B.embed_rows(self.embed, ids_d, hist[0])
-                B.mix_norm(hist, i + 1, layers[i - 1]["dwa"] if i else None, lw["g1"], h1, lw.get("g2"), h2 if has_ff else None, x_out=x if i else None,
-                           eps=eps, n_rows=T)
+                norms = (lw["g1"], h1, lw.get("g2"), h2 if has_ff else None)
+                if i:
+                    B.mix_norm(hist, i + 1, layers[i - 1]["dwa"], *norms, x_out=x, eps=eps, n_rows=T)
+                else:
+                    B.embed_norm(self.embed, ids_d, 1.0, hist[0], *norms, eps=eps)
                 # (both halves of a layer start from the same input: their products go out two by two)
                 if up:
                     B.linear_pair(qk, up)

@@ -107,3 +107,19 @@ def test_norm_linear(dtype, kind, M, K, N1, N2):
         z = torch.empty_like(y1)
         B.linear(h, w1, z, M=M, bias=b1, **kw)
         close(y1, z.to(d))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,W", [(1, 4), (3, 260), (2, 2048), (700, 1024), (1, 8192), (5, 16384), (4, 1001), (513, 512)])
+@pytest.mark.parametrize("both", [False, True])
+def test_embed_norm(dtype, rows, W, both):
+    table, ids = rand(40, W, dtype=dtype), torch.tensor([(11 * r + 41) % 45 - 2 for r in range(rows)], dtype=torch.int32, device=DEV)
+    g1, g2 = rand(W, sd=0.1) + 1, rand(W, sd=0.1) + 1
+    x, o1, o2 = torch.empty(rows, W, device=DEV), torch.empty(rows, W, dtype=dtype, device=DEV), torch.empty(rows, W, dtype=dtype, device=DEV)
+    B.embed_norm(table, ids, 0.75, x, g1, o1, g2 if both else None, o2 if both else None, eps=1e-5)
+    want = 0.75 * table.float()[ids.clamp(0, 39).long()]
+    assert torch.equal(x, want)
+    for g, o in ((g1, o1), (g2, o2))[:1 + both]:
+        n = rms(want.double(), g.double())
+        # (fp32: a sum of squares, a root, a quotient and two products; bf16: the result's rounding)
+        assert ((o.double() - n).abs() <= (2.0 ** -21 if dtype == torch.float32 else 2.0 ** -8) * n.abs() + 1e-30).all()
