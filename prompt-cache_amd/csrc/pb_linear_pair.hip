@@ -5,6 +5,7 @@
 #include <type_traits>
 
 #include "pb_linear_parts.h"
+#include "pb_linear_tiles.h"
 
 namespace {
 using namespace pcb;
@@ -202,6 +203,7 @@ PCB_EXPORT int pcb_linear_pair(const pcb_linear_args* a, const pcb_linear_args* 
     // columns, K = 2048, bf16 18.9 / 15.1 and 20.8 / 17.6.)
     const bool heavy = a->dtype == PCB_BF16 && b->epilogue == PCB_EPI_SILU_MUL && ((int64_t)a->N * a->K + 2 * (int64_t)b->N * b->K) * 2 > 80000000;
     if (!one || heavy) {
+        if (a->M > 64 && pcb_linear_tiles_pair(*a, *b, (hipStream_t)stream, &rc)) return rc;
         rc = pcb_linear(a, stream);
         return rc == PCB_OK ? pcb_linear(b, stream) : rc;
     }

@@ -5,6 +5,8 @@
 #include "pb_common.h"
 
 int pcb_linear_tiles(const pcb_linear_args& a, hipStream_t stream);
+// two products of the same rows in one grid where that is the better (false: it is not, nothing was launched)
+bool pcb_linear_tiles_pair(const pcb_linear_args& a, const pcb_linear_args& b, hipStream_t stream, int* rc);
 // ... and those over some tens or hundreds of rows (pb_linear_waves.hip): which launches whose rows can be read in 16-byte chunks it is the better for
 int64_t pcb_linear_waves_tiles(const pcb_linear_args& a);
 bool pcb_linear_waves_fits(const pcb_linear_args& a);

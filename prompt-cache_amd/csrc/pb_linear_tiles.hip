@@ -7,7 +7,7 @@
 // 90.5 -> 65.6 (1.05 PFLOP/s; the gated pair 79.3 -> 60.7); 4096 x 4096 x 4096 161 -> 112 (1.23 PFLOP/s).  With a sigmoid on half of the columns: 5136
 // columns 77.6 -> 63.0, 10272 132 -> 124 since it and silu do without expf's and the division's cases (over_one_plus_exp; and 192-column tiles).
 #include "mfma_tile_loop.h"
-#include "pb_linear_epi.h"
+#include "pb_linear_parts.h"
 #include "pb_linear_tiles.h"
 
 namespace {
@@ -254,18 +254,19 @@ __device__ __forceinline__ void store_columns(const pcb_linear_args& a, char* pa
     }
 }
 
+template <int MT, int NT, int S, int BLK>
+constexpr int kTileLds = S * mfma_tile::Loop<MT, NT, S, 1, BLK>::kStage > 4 * 32 * MT * 256 ? S * mfma_tile::Loop<MT, NT, S, 1, BLK>::kStage : 4 * 32 * MT * 256;
+
+// tile (mi, ni) of a product
 template <int EPI, int MT, int NT, int S, int BLK>
-__global__ __launch_bounds__(256, 1) void linear_tile_kernel(const pcb_linear_args a, const Grid g) {
+__device__ __forceinline__ void tile_block(const pcb_linear_args& a, int mi, int ni, char* lds) {
     typedef bf16_t E;
     constexpr bool TWO = EPI == PCB_EPI_SILU_MUL;
     using L = mfma_tile::Loop<MT, NT, S, 1, BLK>;
     constexpr int BM = L::BM, BN = TWO ? L::BN / 2 : L::BN, NI = L::NI;   // BN: result columns
     constexpr int P = 32 * MT * 256;                                 // bytes of a patch (see below)
-    __shared__ __attribute__((aligned(16))) char lds[S * L::kStage > 4 * P ? S * L::kStage : 4 * P];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
-    int mi, ni;
-    if (!mfma_tile::tile_of(g.s, g.mb, g.nb, blockIdx.x, mi, ni)) return;
     const int m_lo = mi * BM, n_lo = ni * BN, K = a.K, N = a.N, nk = (K + 63) / 64;
 
     // staging: a lane's 16-byte chunk of an instruction's row as a 32-bit offset from the operand's K-step (the address is otherwise uniform)
@@ -353,36 +354,84 @@ __global__ __launch_bounds__(256, 1) void linear_tile_kernel(const pcb_linear_ar
     }
 }
 
+template <int EPI, int MT, int NT, int S, int BLK>
+__global__ __launch_bounds__(256, 1) void linear_tile_kernel(const pcb_linear_args a, const Grid g) {
+    __shared__ __attribute__((aligned(16))) char lds[kTileLds<MT, NT, S, BLK>];
+    int mi, ni;
+    if (mfma_tile::tile_of(g.s, g.mb, g.nb, blockIdx.x, mi, ni)) tile_block<EPI, MT, NT, S, BLK>(a, mi, ni, lds);
+}
+
+// two products of the same rows in one grid: the first na column blocks are the first product's
+template <int EPI, int MT, int NT, int S, int BLK>
+__global__ __launch_bounds__(256, 1) void linear_tile_pair_kernel(const pcb_linear_args a, const pcb_linear_args b, const Grid g, int na) {
+    __shared__ __attribute__((aligned(16))) char lds[kTileLds<MT, NT, S, BLK>];
+    int mi, ni;
+    if (!mfma_tile::tile_of(g.s, g.mb, g.nb, blockIdx.x, mi, ni)) return;
+    if (ni < na)
+        tile_block<PCB_EPI_STORE, MT, NT, S, BLK>(a, mi, ni, lds);
+    else
+        tile_block<EPI, MT, NT, S, BLK>(b, mi, ni - na, lds);
+}
+
+// (b: the second product of a pair, the first one is a plain store)
 template <int EPI, int MT, int NT, int S, int BLK = (MT * NT > 4 ? 16 : 32)>
-int launch(const pcb_linear_args& a, hipStream_t stream) {
+int launch(const pcb_linear_args& a, const pcb_linear_args* b, hipStream_t stream) {
     using L = mfma_tile::Loop<MT, NT, S, 1, BLK>;
-    const int mb = pcb_ceil_div(a.M, L::BM), nb = pcb_ceil_div(a.N, EPI == PCB_EPI_SILU_MUL ? L::BN / 2 : L::BN);
+    constexpr int BN = EPI == PCB_EPI_SILU_MUL ? L::BN / 2 : L::BN;
+    const int mb = pcb_ceil_div(a.M, L::BM), na = b ? pcb_ceil_div(a.N, L::BN) : 0, nb = na + pcb_ceil_div(b ? b->N : a.N, BN);
     const mfma_tile::Strips s = mfma_tile::strips(mb, nb, L::BM, L::BN);
-    hipLaunchKernelGGL((linear_tile_kernel<EPI, MT, NT, S, BLK>), dim3(8 * s.mh * s.nh), dim3(256), 0, stream, a, (Grid{mb, nb, s}));
+    const dim3 grid(8 * s.mh * s.nh);
+    if constexpr (EPI != PCB_EPI_SCALE_ADD)
+        if (b) {
+            hipLaunchKernelGGL((linear_tile_pair_kernel<EPI, MT, NT, S, BLK>), grid, dim3(256), 0, stream, a, *b, (Grid{mb, nb, s}), na);
+            return pcb_check_launch("linear_tile_pair_kernel");
+        }
+    hipLaunchKernelGGL((linear_tile_kernel<EPI, MT, NT, S, BLK>), grid, dim3(256), 0, stream, a, (Grid{mb, nb, s}));
     return pcb_check_launch("linear_tile_kernel");
 }
 
-template <int EPI>
-int dispatch(const pcb_linear_args& a, hipStream_t stream) {
-    // The tile whose whole rounds of the 256 CUs cost least.  A round, in us, one workgroup per CU, from K = 64 .. 8192 on a full chip:
-    // 128 x 128 4.5 + 0.53 per K-step, 128 x 192 5.6 + 0.645, 128 x 256 7 + 0.67, 256 x 192 8 + 0.95, 256 x 256 10 + 1.03 (K = 2048: 21, 26, 28, 38, 43).
-    // 2048 rows, K = 2048, 128 x 128 / 128 x 256 / 256 x 256 and what the rule took: N = 2048 20.0 / 28.0 / 42.7 -> 20.0, 8192 84 / 75 / 67 -> 66;
-    // 6000 rows, K = 512, N = 2048 21.2 / 24.9 / 22.3 -> 21.9.  Without and with the two of 192 columns: 2048 rows, N = 2560 31.7 / 29.9, 5136 55.3 / 49.7,
-    // 10272 106 / 102; 1500 x 3072 31.3 / 25.4; 4096 x 2560 52.0 / 45.4; 2400 x 2048, K = 8192 102 / 91.  (The gated unit's halves are whole pairs of
-    // 32-column blocks: not 192.)
-    constexpr int C = EPI == PCB_EPI_SILU_MUL ? 2 : 1;               // weight rows per result column
-    auto rounds = [&](int bm, int bn) { return ((int64_t)pcb_ceil_div(a.M, bm) * pcb_ceil_div(C * a.N, bn) + 255) / 256; };
+// The tile whose whole rounds of the 256 CUs cost least.  A round, in us, one workgroup per CU, from K = 64 .. 8192 on a full chip:
+// 128 x 128 4.5 + 0.53 per K-step, 128 x 192 5.6 + 0.645, 128 x 256 7 + 0.67, 256 x 192 8 + 0.95, 256 x 256 10 + 1.03 (K = 2048: 21, 26, 28, 38, 43).
+// 2048 rows, K = 2048, 128 x 128 / 128 x 256 / 256 x 256 and what the rule took: N = 2048 20.0 / 28.0 / 42.7 -> 20.0, 8192 84 / 75 / 67 -> 66;
+// 6000 rows, K = 512, N = 2048 21.2 / 24.9 / 22.3 -> 21.9.  Without and with the two of 192 columns: 2048 rows, N = 2560 31.7 / 29.9, 5136 55.3 / 49.7,
+// 10272 106 / 102; 1500 x 3072 31.3 / 25.4; 4096 x 2560 52.0 / 45.4; 2400 x 2048, K = 8192 102 / 91.  (The gated unit's halves are whole pairs of
+// 32-column blocks: not 192.)
+enum Shape { SQUARE, WIDE192, WIDE, TALL192, TALL };
+int choose(const pcb_linear_args& a, const pcb_linear_args* b) {
+    const bool gated = (b ? b : &a)->epilogue == PCB_EPI_SILU_MUL;
+    auto cols = [](const pcb_linear_args& q) { return q.epilogue == PCB_EPI_SILU_MUL ? 2 * q.N : q.N; };      // weight rows
+    auto rounds = [&](int bm, int bn) { return ((int64_t)pcb_ceil_div(a.M, bm) * (pcb_ceil_div(cols(a), bn) + (b ? pcb_ceil_div(cols(*b), bn) : 0)) + 255) / 256; };
     const float steps = (float)pcb_ceil_div(a.K, 64);
     const float square = rounds(128, 128) * (4.5f + 0.53f * steps), wide = rounds(128, 256) * (7.0f + 0.67f * steps),
                 tall = rounds(256, 256) * (10.0f + 1.03f * steps);
     const float least = tall <= wide && tall <= square ? tall : wide <= square ? wide : square;
-    if constexpr (C == 1) {
+    if (!gated) {
         const float wide192 = rounds(128, 192) * (5.6f + 0.645f * steps), tall192 = rounds(256, 192) * (8.0f + 0.95f * steps);
-        if (tall192 < least && tall192 <= wide192) return launch<EPI, 4, 3, 2>(a, stream);
-        if (wide192 < least) return launch<EPI, 2, 3, 3>(a, stream);
+        if (tall192 < least && tall192 <= wide192) return TALL192;
+        if (wide192 < least) return WIDE192;
     }
-    if (tall == least) return launch<EPI, 4, 4, 2>(a, stream);
-    return wide == least ? launch<EPI, 2, 4, 3>(a, stream) : launch<EPI, 2, 2, 3>(a, stream);
+    return tall == least ? TALL : wide == least ? WIDE : SQUARE;
+}
+
+template <int EPI>
+int dispatch(const pcb_linear_args& a, hipStream_t stream) {
+    const int shape = choose(a, nullptr);
+    if constexpr (EPI != PCB_EPI_SILU_MUL) {
+        if (shape == TALL192) return launch<EPI, 4, 3, 2>(a, nullptr, stream);
+        if (shape == WIDE192) return launch<EPI, 2, 3, 3>(a, nullptr, stream);
+    }
+    if (shape == TALL) return launch<EPI, 4, 4, 2>(a, nullptr, stream);
+    return shape == WIDE ? launch<EPI, 2, 4, 3>(a, nullptr, stream) : launch<EPI, 2, 2, 3>(a, nullptr, stream);
+}
+
+template <int EPI>
+int dispatch_pair(const pcb_linear_args& a, const pcb_linear_args& b, int shape, hipStream_t stream) {
+    if constexpr (EPI != PCB_EPI_SILU_MUL) {
+        if (shape == TALL192) return launch<EPI, 4, 3, 2>(a, &b, stream);
+        if (shape == WIDE192) return launch<EPI, 2, 3, 3>(a, &b, stream);
+    }
+    if (shape == TALL) return launch<EPI, 4, 4, 2>(a, &b, stream);
+    return shape == WIDE ? launch<EPI, 2, 4, 3>(a, &b, stream) : launch<EPI, 2, 2, 3>(a, &b, stream);
 }
 
 }  // namespace
@@ -393,4 +442,32 @@ int pcb_linear_tiles(const pcb_linear_args& a, hipStream_t stream) {
         case PCB_EPI_SILU_MUL: return dispatch<PCB_EPI_SILU_MUL>(a, stream);
         default: return dispatch<PCB_EPI_SCALE_ADD>(a, stream);
     }
+}
+
+// Two products in one grid fill the rounds that each leaves part empty.  What a grid takes, us: whole rounds, half a round for a part of one and the rest of it
+// in proportion (a full chip runs at a lower clock), and the activations behind the last products, 0.056 a number and thread: one grid where that is the
+// lesser, by 3 %, than the two products' (gated units beyond 128 rows only).  Over 138 sizes of 65 .. 4800 rows 0.1 % behind the better of the two, two of
+// them by 11 and 13 %.  Apart / in one, us, 2560 and 8192 fp32 columns, K = 2048: 255 rows 38.1 / 25.1, 377 40.1 / 25.4, 679 52.4 / 35.0, 1484 77.8 / 57.7, 2195 120 / 103; 2048
+// with a sigmoid and a gated 4096: 142 rows 32.3 / 24.7, 558 50.9 / 40.1, 2195 124 / 106 (1805 83 / 102: apart); 640 and 2048, K = 512: 310 rows 12.0 / 9.0.
+static float grid_us(const pcb_linear_args& a, const pcb_linear_args* b, int shape) {
+    static constexpr struct { int bm, bn; float base, step; } T[] = {
+        {128, 128, 4.8f, 0.57f}, {128, 192, 7.0f, 0.77f}, {128, 256, 11.0f, 0.88f}, {256, 192, 10.0f, 1.3f}, {256, 256, 12.7f, 1.5f}};
+    const auto& t = T[shape];
+    auto blocks = [&](const pcb_linear_args& q) { return (int64_t)pcb_ceil_div(q.epilogue == PCB_EPI_SILU_MUL ? 2 * q.N : q.N, t.bn); };
+    auto acts = [&](const pcb_linear_args& q) { return q.epilogue == PCB_EPI_SILU_MUL ? 0.5f : (q.act | q.act2) ? 1.0f : 0.0f; };
+    const int64_t tiles = pcb_ceil_div(a.M, t.bm) * (blocks(a) + (b ? blocks(*b) : 0)), rest = tiles % 256;
+    const float round = t.base + t.step * (float)pcb_ceil_div(a.K, 64), act = b && acts(*b) > acts(a) ? acts(*b) : acts(a);
+    return round * ((float)(tiles / 256) + (rest ? 0.5f + (float)rest / 512.0f : 0.0f)) + 0.056f * act * (float)(t.bm * t.bn / 256);
+}
+
+bool pcb_linear_tiles_pair(const pcb_linear_args& a, const pcb_linear_args& b, hipStream_t stream, int* rc) {
+    auto fits = [](const pcb_linear_args& q) {
+        return q.dtype == PCB_BF16 && q.M > 64 && q.n_groups == 0 && q.n_batch == 0 && !q.row_src && q.ldx < (1 << 22) && q.ldw < (1 << 22) && pcb_linear_pieces(q);
+    };
+    const bool gated = b.epilogue == PCB_EPI_SILU_MUL;
+    if (!fits(a) || !fits(b) || a.M != b.M || a.K != b.K || a.epilogue != PCB_EPI_STORE || b.epilogue == PCB_EPI_SCALE_ADD || (gated && a.M <= 128)) return false;
+    const int shape = choose(a, &b);
+    if (grid_us(a, &b, shape) >= 0.97f * (grid_us(a, nullptr, choose(a, nullptr)) + grid_us(b, nullptr, choose(b, nullptr)))) return false;
+    *rc = gated ? dispatch_pair<PCB_EPI_SILU_MUL>(a, b, shape, stream) : dispatch_pair<PCB_EPI_STORE>(a, b, shape, stream);
+    return true;
 }
