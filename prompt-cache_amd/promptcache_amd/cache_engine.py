@@ -125,7 +125,7 @@ class PromptCache:
         self.last_gather_events = None
         self.last_gather_tokens = 0
         # Leave the copy to the first forward over the staged buffer (set by CacheEngine for models whose cached-prefill
-        # attention stages while it reads, ``supports_fused_gather``): update() then only records WHAT is staged
+        # attention stages while it reads, ``supports_fused_gather``, or whose forward copies first, ``defers_staging``): update() then only records WHAT is staged
         # (``KVArena.pending``); the rows arrive with the first ``lm()`` call -- or with one pc_kv_gather launch as soon as
         # somebody looks at the returned views.  TTFT (cache_time + the first lm() call) moves the K/V once instead of
         # gather read + gather write + attention read.
@@ -695,7 +695,8 @@ class CacheEngine:
         self.prompt_cache = PromptCache(max_ctx_length=max_ctx_length, num_layers=num_layers, num_head=num_head,
                                         head_dim=head_dim, target_device=self.target_device)
         # PC_DEFER_GATHER=0: PromptCache.update copies at once, as rounds 1-3 did
-        self.prompt_cache.defer_gather = bool(getattr(getattr(lm, "hf_model", None), "supports_fused_gather", False)) and \
+        model = getattr(lm, "hf_model", None)
+        self.prompt_cache.defer_gather = bool(getattr(model, "supports_fused_gather", False) or getattr(model, "defers_staging", False)) and \
             os.environ.get("PC_DEFER_GATHER", "1") != "0"
 
     def add_schema(self, schema: Union[str, Schema], batch_size: int = 1, max_tokens: Optional[int] = None,

@@ -37,7 +37,11 @@ def alibi_slopes(num_heads: int, alibi_bias_max: int = 8) -> torch.Tensor:
 
 class MptHIP(LlamaHIP):
     _shared_prefix_loop = False     # (its many-row loop keeps a copy of the trunk per batch row)
-    supports_fused_gather = False   # (its layer loops read staged rows from the arena: PromptCache.update copies at once)
+    supports_fused_gather = False   # (its layer loops read staged rows from the arena ...)
+    # ... and the copy goes out at the beginning of the first forward (_resolve_arena): behind it the host prepares the step, where an update() that copies at
+    # once, and is timed by events, waits for it.  A question behind 936 staged tokens, 8 layers of 7b: 1 226 us -> 1 103.
+    defers_staging = True
+    _identity: Optional[torch.Tensor] = None
 
     def __init__(self, shape: MptShape, weights: Dict[str, torch.Tensor], device="cuda:0", decode_headroom: int = 256,
                  skinny: bool = True, int8_weights: bool = False):
@@ -187,9 +191,14 @@ class MptHIP(LlamaHIP):
         return ent[4].clone()
 
     def _identity_rotation(self, T: int) -> torch.Tensor:
-        cs = torch.zeros((T, self.D // 2, 2), dtype=torch.float32, device=self.device)
-        cs[..., 0] = 1.0                                        # cos = 1, sin = 0: q and k pass through unrotated
-        return cs
+        """cos = 1, sin = 0: q and k pass through unrotated.  (Up to 512 rows of one table, made once: two launches of a step.)"""
+        cs = self._identity
+        if cs is None or T > cs.shape[0]:
+            cs = torch.zeros((max(T, 512), self.D // 2, 2), dtype=torch.float32, device=self.device)
+            cs[..., 0] = 1.0
+            if T <= 512:
+                self._identity = cs
+        return cs[:T]
 
     # ------------------------------------------------------------------------------------------
     def _forward_dense(self, ids, kpos, arena, B, q_len, past_len, last_token_only, num_layers):
