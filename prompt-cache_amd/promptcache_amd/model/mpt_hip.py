@@ -41,7 +41,6 @@ class MptHIP(LlamaHIP):
     # ... and the copy goes out at the beginning of the first forward (_resolve_arena): behind it the host prepares the step, where an update() that copies at
     # once, and is timed by events, waits for it.  A question behind 936 staged tokens, 8 layers of 7b: 1 226 us -> 1 103.
     defers_staging = True
-    _identity: Optional[torch.Tensor] = None
 
     def __init__(self, shape: MptShape, weights: Dict[str, torch.Tensor], device="cuda:0", decode_headroom: int = 256,
                  skinny: bool = True, int8_weights: bool = False):
@@ -57,6 +56,8 @@ class MptHIP(LlamaHIP):
                 t = torch.from_numpy(t)
             return t.to(device=dev, dtype=self.dtype).contiguous()
 
+        self._identity = torch.zeros((512, self.D // 2, 2), dtype=torch.float32, device=dev)
+        self._identity[..., 0] = 1.0
         self.embed = w("embed")
         self.lnf = w("lnf")
         self.lm_head = self.embed if c.tie_word_embeddings and "lm_head" not in weights else w("lm_head")
@@ -191,14 +192,12 @@ class MptHIP(LlamaHIP):
         return ent[4].clone()
 
     def _identity_rotation(self, T: int) -> torch.Tensor:
-        """cos = 1, sin = 0: q and k pass through unrotated.  (Up to 512 rows of one table, made once: two launches of a step.)"""
-        cs = self._identity
-        if cs is None or T > cs.shape[0]:
-            cs = torch.zeros((max(T, 512), self.D // 2, 2), dtype=torch.float32, device=self.device)
-            cs[..., 0] = 1.0
-            if T <= 512:
-                self._identity = cs
-        return cs[:T]
+        """cos = 1, sin = 0: q and k pass through unrotated.  (Up to 512 rows of one table made with the weights: two launches of a step.)"""
+        if T <= self._identity.shape[0]:
+            return self._identity[:T]
+        cs = torch.zeros((T, self.D // 2, 2), dtype=torch.float32, device=self.device)
+        cs[..., 0] = 1.0
+        return cs
 
     # ------------------------------------------------------------------------------------------
     def _forward_dense(self, ids, kpos, arena, B, q_len, past_len, last_token_only, num_layers):
