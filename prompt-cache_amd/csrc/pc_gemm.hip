@@ -193,6 +193,82 @@ __global__ __launch_bounds__(256) void rmsnorm_frag_kernel(float* __restrict__ x
     }
 }
 
+// The same, a thread per eight columns (2 048 < hidden <= 8 192), and up to eight slabs under way at a time: one trip to memory whatever their number.  Sums go in the
+// order of the form above (thread t's groups t, t + 256, .. one after the other), hence the same bits; the new residual is stored last.
+// What bounds it: the launch, one trip to memory, one sum over the workgroup (two barriers).  takes_wide has the figures.
+template <bool LN>
+__global__ __launch_bounds__(1024) void rmsnorm_frag_wide_kernel(float* __restrict__ x, const _Float16* __restrict__ w,
+                                                                 _Float16* __restrict__ of_hi, _Float16* __restrict__ of_lo,
+                                                                 int hidden, float eps, const float* __restrict__ slabs,
+                                                                 int nslabs, int64_t slab_stride, const _Float16* __restrict__ b) {
+    __shared__ float part[1024];
+    __shared__ float red[2][4];
+    constexpr int CH = 8;
+    const int row = blockIdx.x, tid = threadIdx.x, nv = hidden >> 3, ic = tid < nv ? tid : nv - 1;
+    const bool on = tid < nv;
+    float* xr = x + (int64_t)row * hidden + ic * 8;
+    f4 va = *(const f4*)xr, vb = *(const f4*)(xr + 4);
+    const h8 gw = *(const h8*)(w + ic * 8);
+    h8 bw = h8{0, 0, 0, 0, 0, 0, 0, 0};
+    if (LN && b) bw = *(const h8*)(b + ic * 8);
+    for (int s0 = 0; s0 < nslabs; s0 += CH) {
+        f4 c[CH], d[CH];
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            if (s0 + j < nslabs) {                                // (the same for all: a slab that is not there is not asked for)
+                const float* sp = slabs + (s0 + j) * slab_stride + (int64_t)row * hidden + ic * 8;
+                c[j] = *(const f4*)sp;
+                d[j] = *(const f4*)(sp + 4);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            if (s0 + j < nslabs) {
+                va[0] += c[j][0]; va[1] += c[j][1]; va[2] += c[j][2]; va[3] += c[j][3];
+                vb[0] += d[j][0]; vb[1] += d[j][1]; vb[2] += d[j][2]; vb[3] += d[j][3];
+            }
+        }
+    }
+    const f4 xa = va, xb = vb;
+    auto total = [&](float e, float* sums) {
+        part[tid] = on ? e : 0.f;
+        __syncthreads();
+        if (tid < 256) {
+            float s = 0.f;
+            for (int t = tid; t < (int)blockDim.x; t += 256) s += part[t];
+            s = lanes_sum(s);
+            if ((tid & 63) == 0) sums[tid >> 6] = s;
+        }
+        __syncthreads();
+        return sums[0] + sums[1] + sums[2] + sums[3];
+    };
+    if (LN) {
+        const float mu = total(va[0] + va[1] + va[2] + va[3] + vb[0] + vb[1] + vb[2] + vb[3], red[0]) / (float)hidden;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { va[e] -= mu; vb[e] -= mu; }
+    }
+    const float ss = total(va[0] * va[0] + va[1] * va[1] + va[2] * va[2] + va[3] * va[3] +
+                           vb[0] * vb[0] + vb[1] * vb[1] + vb[2] * vb[2] + vb[3] * vb[3], red[1]);
+    const float rs = rsqrtf(ss / (float)hidden + eps);
+    if (!on) return;
+    h8 hi, lo;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        float v = (float)gw[e] * ((e < 4 ? va[e] : vb[e - 4]) * rs);
+        if (LN) v += (float)bw[e];
+        _Float16 vh, vl;
+        pc_split(v, vh, vl);
+        hi[e] = vh; lo[e] = vl;
+    }
+    const int64_t off = frag_off(row, tid * 8, hidden >> 5);
+    *(h8*)(of_hi + off) = hi;
+    *(h8*)(of_lo + off) = lo;
+    if (nslabs > 0) {
+        *(f4*)xr = xa;
+        *(f4*)(xr + 4) = xb;
+    }
+}
+
 // q|k|v with K split across workgroups (65..288 rows, wide panels): the projection leaves `nslabs` fp32 slabs [M][N] of partial
 // sums in the row-PERMUTED column order of the q|k|v weight image (inside every head, tile j = features 8j..8j+7 then their rotary
 // partners D/2+8j..); this kernel adds the slabs in slice order and does what tile_epilogue<EPI_ROPE> does on a tile: RoPE at the
@@ -377,6 +453,13 @@ PC_EXPORT int pc_gemm(const pc_gemm_args* a, void* stream) {
     return launch_MT(EPI_STORE, p, choose_T(p.ntiles * kslices), p.ntiles, s);
 }
 
+// us, the form of 256 threads / of one thread per eight columns: hidden 5120, four slabs 27 rows 5.0 / 4.4, six 27 rows 6.1 / 4.7, 160 rows 9.8 / 8.9; hidden 4544 4.8 / 4.2;
+// 2080 .. 3072 and 6144 .. 8192 0 to 1.0 less.  Not without slabs (a barrier more: 5120, 27 rows 3.3 / 3.4), nor for three or four at 3073 .. 4096, one trip in both
+// (4.1 / 4.0, layer norm 4.2 / 4.4), nor where a CU has a second row (259 rows of 5120, four slabs 11.7 / 12.9).  8 hidden sizes x 8 counts of slabs x 8 row counts.
+static bool takes_wide(int rows, int hidden, int nslabs) {
+    return rows <= 160 && nslabs > 0 && hidden > 2048 && hidden <= 8192 && !(hidden > 3072 && hidden <= 4096 && (nslabs == 3 || nslabs == 4));
+}
+
 PC_EXPORT int pc_rmsnorm_frag(float* x, const void* weight, void* xf_hi, void* xf_lo, int32_t rows,
                               int32_t hidden, float eps, const float* slabs, int32_t nslabs, void* stream) {
     PC_REQUIRE(rows > 0 && rows <= kRowsMaxM && hidden > 0 && hidden % 32 == 0, PC_ERR_ARG, "pc_rmsnorm_frag: bad sizes");
@@ -384,6 +467,12 @@ PC_EXPORT int pc_rmsnorm_frag(float* x, const void* weight, void* xf_hi, void* x
                "pc_rmsnorm_frag: null pointer");
     PC_REQUIRE(hidden <= 16384, PC_ERR_ARG, "pc_rmsnorm_frag: hidden %d > 16384", hidden);
     const int groups = pc_ceil_div(hidden / 8, 256);
+    if (takes_wide(rows, hidden, nslabs)) {
+        hipLaunchKernelGGL(rmsnorm_frag_wide_kernel<false>, dim3(rows), dim3(pc_ceil_div(hidden / 8, 64) * 64), 0, (hipStream_t)stream, x,
+                           (const _Float16*)weight, (_Float16*)xf_hi, (_Float16*)xf_lo, hidden, eps, slabs, nslabs, (int64_t)rows * hidden,
+                           (const _Float16*)nullptr);
+        return pc_check_launch("rmsnorm_frag_wide_kernel");
+    }
 #define PC_RMS(GV)                                                                                                   \
     hipLaunchKernelGGL(rmsnorm_frag_kernel<GV>, dim3(rows), dim3(256), 0, (hipStream_t)stream, x, (const _Float16*)weight, \
                        (_Float16*)xf_hi, (_Float16*)xf_lo, hidden, eps, slabs, nslabs, (int64_t)rows * hidden,       \
@@ -400,6 +489,12 @@ PC_EXPORT int pc_layernorm_frag(float* x, const void* weight, const void* bias, 
     PC_REQUIRE(x && weight && xf_hi && xf_lo && nslabs >= 0 && (nslabs == 0 || slabs), PC_ERR_ARG,
                "pc_layernorm_frag: null pointer");   /* bias may be NULL */
     const int groups = pc_ceil_div(hidden / 8, 256);
+    if (takes_wide(rows, hidden, nslabs)) {
+        hipLaunchKernelGGL(rmsnorm_frag_wide_kernel<true>, dim3(rows), dim3(pc_ceil_div(hidden / 8, 64) * 64), 0, (hipStream_t)stream, x,
+                           (const _Float16*)weight, (_Float16*)xf_hi, (_Float16*)xf_lo, hidden, eps, slabs, nslabs, (int64_t)rows * hidden,
+                           (const _Float16*)bias);
+        return pc_check_launch("layernorm_frag_wide_kernel");
+    }
 #define PC_LN(GV)                                                                                                    \
     hipLaunchKernelGGL((rmsnorm_frag_kernel<GV, true>), dim3(rows), dim3(256), 0, (hipStream_t)stream, x,            \
                        (const _Float16*)weight, (_Float16*)xf_hi, (_Float16*)xf_lo, hidden, eps, slabs, nslabs,      \

@@ -581,6 +581,34 @@ def test_rmsnorm_frag_matches_oracle(rows, hidden, nslabs):
     np.testing.assert_allclose(got, ref, atol=2e-5, rtol=2e-5)
 
 
+@pytest.mark.parametrize("nslabs", [1, 8, 9])
+@pytest.mark.parametrize("rows,hidden", [(1, 2080), (160, 2080), (17, 4096), (33, 4544), (161, 5120), (3, 8192), (2, 8224)])
+def test_norm_frag_threads_per_column(rows, hidden, nslabs):
+    """A thread per eight columns against 64 bits, at the edges of the sizes that take it: the residual bit for bit, hi + lo to the 2^-21 of the planes and the
+    2^-20 of the row's sums in 32 bits."""
+    n = _n()
+    rng = np.random.default_rng(rows + hidden + nslabs)
+    x = torch.from_numpy(rng.standard_normal((rows, hidden), dtype=np.float32) * 3)
+    sl = torch.from_numpy(rng.standard_normal((nslabs, rows, hidden), dtype=np.float32))
+    w, b = (torch.from_numpy((c + 0.1 * rng.standard_normal(hidden, dtype=np.float32)).astype(np.float16)) for c in (1, 0))
+    xe = x.clone()
+    for s_ in sl:
+        xe += s_
+    v = xe.double()
+    d = v - v.mean(-1, keepdim=True)
+    refs = (v * (v.pow(2).mean(-1, keepdim=True) + 1e-5).rsqrt() * w.double(), d * (d.pow(2).mean(-1, keepdim=True) + 1e-5).rsqrt() * w.double() + b.double())
+    for ln, ref in enumerate(refs):
+        hi = torch.zeros(((rows + 15) // 16, hidden // 32, 64, 8), dtype=torch.float16, device=DEV)
+        lo, xd = torch.zeros_like(hi), x.to(DEV)
+        if ln:
+            n.layernorm_frag(xd, w.to(DEV), b.to(DEV), hi, lo, rows, hidden, 1e-5, sl.to(DEV), nslabs)
+        else:
+            n.rmsnorm_frag(xd, w.to(DEV), hi, lo, rows, hidden, 1e-5, sl.to(DEV), nslabs)
+        assert torch.equal(xd.cpu(), xe)
+        got = (n.from_act_frags(hi, rows).float() + n.from_act_frags(lo, rows).float()).cpu().double()
+        assert float(((got - ref).abs() / (1 + ref.abs())).max()) < 2 ** -20 + 2 ** -21
+
+
 @pytest.mark.parametrize("M,N,K,kq", [(12, 4096, 4096, 4), (12, 4096, 11008, 4), (3, 64, 96, 2), (20, 512, 1376, 3),
                                       (40, 4096, 4096, 4), (64, 4096, 11008, 4), (30, 5120, 13824, 4)])
 def test_gemm_skinny_k_slices(M, N, K, kq):
