@@ -19,7 +19,7 @@ extern "C" {
 
 #define PCB_ABI_VERSION 6
 #define PCB_OK 0
-#define PCB_NOT_TAKEN 1 /* pcb_norm_linear only: sizes or alignments it does not take; nothing was launched */
+#define PCB_NOT_TAKEN 1 /* pcb_norm_linear only: sizes, alignments or overlaps it does not take; nothing was launched */
 #define PCB_ERR_ARG (-2001)
 #define PCB_ERR_HIP_BASE (-3000)
 
@@ -765,8 +765,10 @@ int pcb_attn_step_fits(int32_t dtype, int32_t H, int32_t Hkv, int32_t dim, int32
  *   n_terms > 0 x[r] = sum_j coef[j] * x[j][r]                                       (streams x_stride elements apart, as pcb_mix_norm)
  *   y           t = y[r] * gate[r];  x[r] + t / sqrt(mean(t^2) + eps) * post_gain    (gate E, rows ldg apart, as pcb_post_norm)
  *   x_out[r] = x[r];  the products' rows are x[r] / sqrt(mean(x[r]^2) + eps) * gain (b's: gain2) as E; a->x and b->x are only checked, not read
- * x_out is none of the rows read.  a is a plain store, b one or, with y, a gated unit.  PCB_NOT_TAKEN: beyond a few rows of a
- * few thousand elements, not in whole 16-byte pieces, or so many columns that launches of their own are faster. */
+ * x_out overlaps none of x, y and gate.  What the products store has to lie apart from x, y, gate and x_out too, since every workgroup reads these rows beside others
+ * that store already: a result (y, y2 in fp32) that overlaps one is not taken; rows that row_off2 places are the caller's to keep apart.  a is a plain store, b one or,
+ * with y, a gated unit.  PCB_NOT_TAKEN: that, beyond a few rows of a few thousand elements, not in whole 16-byte pieces, or so many columns that launches of their own
+ * are faster.  pcb_norm_linear_takes: PCB_OK, PCB_NOT_TAKEN or an error, and nothing is launched. */
 typedef struct pcb_row_norm_args {
     uint32_t struct_bytes;
     const float* x;
@@ -786,6 +788,7 @@ typedef struct pcb_row_norm_args {
     float eps;
 } pcb_row_norm_args;
 int pcb_norm_linear(const pcb_row_norm_args* n, const pcb_linear_args* a, const pcb_linear_args* b, void* stream);
+int pcb_norm_linear_takes(const pcb_row_norm_args* n, const pcb_linear_args* a, const pcb_linear_args* b);
 
 /* Recurrences with a matrix state S [dim][vdim] per (slot, head), fp32, zero before position 0.  Per token and head h:
  *   q = q_scale q^, k = k_scale k^        q^, k^: E rows with head h / (H / Hk) at column (h / (H / Hk)) * dim; unit_norm: divided by

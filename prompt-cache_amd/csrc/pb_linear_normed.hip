@@ -258,17 +258,42 @@ static int norm_linear_check(const pcb_row_norm_args* n, const pcb_linear_args* 
     return PCB_OK;
 }
 
-PCB_EXPORT int pcb_norm_linear(const pcb_row_norm_args* n, const pcb_linear_args* a, const pcb_linear_args* b, void* stream) {
+// Every workgroup works out the rows from what they are made of, and nothing orders workgroups: what the products store, and x_out, has to lie apart from that.
+static bool norm_linear_apart(const pcb_row_norm_args& n, const pcb_linear_args& a, const pcb_linear_args* b, bool results) {
+    const int64_t M = a.M, W = a.K;
+    const pcb_span x_out = pcb_rows_span(n.x_out, M, W, W, 4);
+    const pcb_span read[] = {n.table ? pcb_span{} : pcb_rows_span(n.x, 1, 0, (n.n_terms > 0 ? n.n_terms - 1 : 0) * n.x_stride + M * W, 4),
+                             pcb_rows_span(n.y, M, W, W, 4), n.y ? pcb_rows_span(n.gate, M, n.ldg, W, a.dtype == PCB_BF16 ? 2 : 4) : pcb_span{}};
+    for (const pcb_span& s : read) {
+        if (!results && !pcb_apart(x_out, s)) return false;
+        if (results && !(pcb_results_apart(a, s) && (!b || pcb_results_apart(*b, s)))) return false;
+    }
+    return !results || (pcb_results_apart(a, x_out) && (!b || pcb_results_apart(*b, x_out)));
+}
+
+static int norm_linear_route(const pcb_row_norm_args* n, const pcb_linear_args* a, const pcb_linear_args* b, Form* f) {
     const int rc = norm_linear_check(n, a, b);
     if (rc != PCB_OK) return rc;
+    PCB_REQUIRE(norm_linear_apart(*n, *a, b, false), PCB_ERR_ARG, "pcb_norm_linear: x_out overlaps the rows that are read");
     const uintptr_t e4 = a->dtype == PCB_BF16 ? 8 : 16;              // (four elements of E)
     auto takes = [](const pcb_linear_args& q) { return q.n_batch == 0 && !q.row_src && !q.row_dst && !q.row_gate && q.split_n3 <= 0 && pcb_linear_pieces(q); };
     const bool pieces = a->epilogue == PCB_EPI_STORE && takes(*a) && a->K % 64 == 0 &&
                         (!b || (takes(*b) && (b->epilogue == PCB_EPI_STORE || (b->epilogue == PCB_EPI_SILU_MUL && n->y)))) && n->x_stride % 4 == 0 && n->ldg % 4 == 0 &&
                         ((uintptr_t)n->x | (uintptr_t)n->y | (uintptr_t)n->post_gain | (uintptr_t)n->gain | (uintptr_t)n->gain2 | (uintptr_t)n->x_out) % 16 == 0 &&
                         ((uintptr_t)n->gate | (uintptr_t)n->table) % e4 == 0;
-    if (a->M == 0) return PCB_OK;
-    const Form f = form(*n, *a, b);
-    if (!pieces || !f.taken) return PCB_NOT_TAKEN;
+    *f = form(*n, *a, b);
+    return pieces && f->taken && norm_linear_apart(*n, *a, b, true) ? PCB_OK : PCB_NOT_TAKEN;
+}
+
+PCB_EXPORT int pcb_norm_linear_takes(const pcb_row_norm_args* n, const pcb_linear_args* a, const pcb_linear_args* b) {
+    Form f;
+    return norm_linear_route(n, a, b, &f);
+}
+
+PCB_EXPORT int pcb_norm_linear(const pcb_row_norm_args* n, const pcb_linear_args* a, const pcb_linear_args* b, void* stream) {
+    Form f;
+    const int rc = norm_linear_route(n, a, b, &f);
+    if (rc < 0 || a->M == 0) return rc < 0 ? rc : PCB_OK;
+    if (rc != PCB_OK) return rc;
     return a->dtype == PCB_BF16 ? launch<bf16_t>(*n, *a, b, f, (hipStream_t)stream) : launch<float>(*n, *a, b, f, (hipStream_t)stream);
 }

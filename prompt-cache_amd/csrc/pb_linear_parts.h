@@ -117,3 +117,20 @@ inline bool pcb_linear_pieces(const pcb_linear_args& a) {
            a.w_group_stride * es % 16 == 0 &&
            ((uintptr_t)a.x | (uintptr_t)a.w | (uintptr_t)(a.epilogue == PCB_EPI_SILU_MUL ? a.w2 : nullptr)) % 16 == 0;
 }
+
+// Memory that a launch reads or stores: rows of cols elements of es bytes, ld elements apart (a null pointer: nothing)
+struct pcb_span {
+    uintptr_t at;
+    uint64_t bytes;
+};
+inline pcb_span pcb_rows_span(const void* p, int64_t rows, int64_t ld, int64_t cols, int es) {
+    return {(uintptr_t)p, p && rows > 0 ? (uint64_t)((rows - 1) * ld + cols) * es : 0};
+}
+inline bool pcb_apart(const pcb_span& p, const pcb_span& q) { return p.bytes == 0 || q.bytes == 0 || p.at + p.bytes <= q.at || q.at + q.bytes <= p.at; }
+// Whether what an unbatched product stores lies apart from s -- as far as the host can say: not the rows that tables on the device place (row_dst, row_off2, row_off3)
+inline bool pcb_results_apart(const pcb_linear_args& a, const pcb_span& s) {
+    const int es = a.epilogue == PCB_EPI_SCALE_ADD || a.out_f32 || a.dtype == PCB_F32 ? 4 : 2;
+    const int cols = a.split_n > 0 ? a.split_n : a.split_n3 > 0 ? a.split_n3 : a.N;
+    return (a.row_dst || pcb_apart(pcb_rows_span(a.y, a.M, a.ldy, cols, es), s)) &&
+           (!a.y2_f32 || a.split_n <= 0 || pcb_apart(pcb_rows_span(a.y2, a.M, a.head_stride2, a.N - a.split_n, 4), s));
+}

@@ -215,6 +215,7 @@ SIGNATURES = {
     "pcb_embed_norm": (C.c_int, [_vp, _vp, _f32, _i32, C.POINTER(MixNormArgs), _vp]),
     "pcb_linear": (C.c_int, [C.POINTER(LinearArgs), _vp]),
     "pcb_norm_linear": (C.c_int, [C.POINTER(RowNormArgs), C.POINTER(LinearArgs), C.POINTER(LinearArgs), _vp]),
+    "pcb_norm_linear_takes": (C.c_int, [C.POINTER(RowNormArgs), C.POINTER(LinearArgs), C.POINTER(LinearArgs)]),
     "pcb_linear_pair": (C.c_int, [C.POINTER(LinearArgs), C.POINTER(LinearArgs), _vp]),
     "pcb_linear_add2": (C.c_int, [C.POINTER(LinearArgs), C.POINTER(LinearArgs), _vp, _vp, _f32, _vp]),
     "pcb_polynorm": (C.c_int, [_vp, _vp, _vp, _i32, _f32, _i32, _i32, _vp]),
@@ -468,7 +469,8 @@ def linear_add2(a: LinearArgs, b: LinearArgs, z: Optional[torch.Tensor] = None, 
 def norm_linear(a: LinearArgs, b: Optional[LinearArgs], gain: torch.Tensor, gain2: Optional[torch.Tensor], x_out: torch.Tensor, *, eps: float, x=None, coef=None,
                 n_terms: int = 0, table=None, ids=None, scale: float = 1.0, y=None, gate=None, ldg: int = 0, post_gain=None) -> bool:
     """Residual rows -- of a ``table``, the sum of ``n_terms`` streams ``x`` [streams, rows, width], or ``x`` and a gated sublayer's result ``y`` behind its norm
-    -- into ``x_out``, and one or two products (``linear_args``) of the normed rows.  False: not of the sizes that one launch takes, nothing done."""
+    -- into ``x_out``, and one or two products (``linear_args``) of the normed rows.  False: not what one launch takes (sizes, or results that overlap the rows
+    read), nothing done."""
     M, W = a.M, a.K
     for t, nm in ((gain, "gain"), (gain2, "gain2"), (x_out, "x_out"), (x, "x"), (coef, "coef"), (y, "y"), (post_gain, "post_gain")):
         _want(t, torch.float32, "norm_linear " + nm)

@@ -414,9 +414,12 @@ class FivesunHIP(SlotModel):
             else:
                 B.linear_run(a)
 
+        # A layer without a feed-forward leaves its residual gate in its projected rows; where the norm that reads it rides in the next layer's projection, that
+        # one stores elsewhere.
+        mix_in = ("mix_in", "mix_in_next" if T * W <= B.NORM_LINEAR_MAX else "mix_in")
         for i, lw in enumerate(layers):
             l = lw["cfg"]
-            P = self._mat("mix_in", T, lw["w_in"].shape[0], E)
+            P = self._mat(mix_in[i % 2], T, lw["w_in"].shape[0], E)
             project(lw["norm1"], B.linear_args(h, lw["w_in"], P, M=T, bias=lw["b_in"], act_split=lw["act_from"], act2=B.ACT_SIGMOID))
             gate, ldg = getattr(self, "_" + l.kind)(arena, i, l, lw, P, y1, tb, T, R)
             pending = dict(y=y1, gate=gate, ldg=ldg, post_gain=lw["norm1b"])

@@ -377,3 +377,88 @@ def test_layers_and_calls_share_the_rule_of_what_goes_in_segments(heads, dim, vd
     mem = torch.empty(2 * n + 16, dtype=dtype)
     mem = mem[(-mem.data_ptr() % 16) // es:]
     assert B.mlstm_prompt_fits(dim, vdim, n, [mem[a:] for a in at], mem[gate:], 64) == fits
+
+
+# ---- launches of a step whose norm rides in a projection -------------------------------------------------------------------------
+class _NoLaunch:
+    """The blocks library with every call that would launch answered with "done"; what pcb_norm_linear is given is kept."""
+
+    def __init__(self, lib, launches, seen):
+        self.lib, self.launches, self.seen = lib, launches, seen
+
+    def __getattr__(self, name):
+        if name not in self.launches:
+            return getattr(self.lib, name)
+
+        def call(*args):
+            if name == "pcb_norm_linear":
+                self.seen.append([None if a is None else type(a._obj).from_buffer_copy(a._obj) for a in args[:3]])
+            return 0
+        return call
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows", [1, 3])
+def test_a_norms_rows_lie_apart_from_what_its_launch_stores(monkeypatch, rows, dtype):
+    """A layer without a feed-forward leaves its residual gate in its projected rows: the next layer's products, in whose launch the gate is read, store elsewhere."""
+    from promptcache_amd import _blocks as B
+    from promptcache_amd.model.fivesun_hip import FivesunHIP
+    att = dict(heads=4, kv_heads=2, dim=16, vdim=16, scale=0.25, mask=0, rot_base=100.0, rot_dims=16, rot_factor=1.0, v_mix=True)
+    lat = dict(heads=2, kv_heads=1, dim=16, vdim=16, kv_rank=32, rot_dim=16, rot_dims=16, scale=0.2, mask=9, rot_base=50.0, rot_factor=1.0)
+    mem = dict(heads=2, kv_heads=2, dim=16, vdim=16, gate_cap=4.0)
+    s = FivesunShape(vocab_size=60, hidden_size=512, norm_eps=1e-5, embed_scale=3.5, layers=[
+        FivesunLayer("attention", **att), FivesunLayer("attention", **att), FivesunLayer("latent_attention", **lat), FivesunLayer("mlstm", **mem),
+        FivesunLayer("attention", ff=64, **att), FivesunLayer("mlstm", **mem), FivesunLayer("mlstm", **mem), FivesunLayer("latent_attention", **lat)])
+    launches = {n for n, (_, args) in B.SIGNATURES.items() if args and args[-1] is ctypes.c_void_p}
+    seen = []
+    monkeypatch.setattr(B, "_lib", _NoLaunch(B.load(), launches, seen))
+    monkeypatch.setattr(B, "_stream", lambda: 0)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)               # (there is no device here: the tensors lie on the host)
+    m = FivesunHIP(s, W.make_fivesun_weights(s, seed=1), device="cpu", dtype=dtype)
+    m.use_graphs = False
+    ar = m.new_arena(rows, 8)
+    m.forward_rows(ar, [ar.alloc() for _ in range(rows)], [[5]] * rows)
+    assert len(seen) == len(s.layers) + 1
+    es = 2 if dtype == torch.bfloat16 else 4
+    for n, a, b in seen:
+        span = lambda p, ld, cols, size: (p, p + ((rows - 1) * ld + cols) * size)       # noqa: E731
+        read = [span(p, ld, 512, size) for p, ld, size in ((n.x, 512, 4), (n.y, 512, 4), (n.gate, n.ldg, es)) if p]
+        stored = [span(n.x_out, 512, 512, 4)] + [span(q.y, q.ldy, q.N, es) for q in (a, b) if q is not None]
+        for lo, hi in read:
+            assert all(hi <= at or end <= lo for at, end in stored)
+
+
+def test_results_over_the_rows_of_a_norm_go_apart(monkeypatch):
+    """pcb_norm_linear does not take products that store over what the norm reads, and refuses such an x_out; decided on the host, nothing is launched."""
+    from promptcache_amd import _blocks as B
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    M, K, N = 2, 512, 640
+    x, y, gate, gain = torch.zeros(M, K), torch.zeros(M, K), torch.zeros(M, K + 128, dtype=torch.bfloat16), torch.ones(K)
+    out, h, w = torch.zeros(M, K), torch.zeros(M, K, dtype=torch.bfloat16), torch.zeros(N, K, dtype=torch.bfloat16)
+    P, Q = torch.zeros(M, N, dtype=torch.bfloat16), torch.zeros(M, N, dtype=torch.bfloat16)
+    room = torch.zeros(4 * M * K)                                    # streams, and what lies around them
+
+    def asked(a, b=None, x_out=out, streams=None):
+        n = B.RowNormArgs(ctypes.sizeof(B.RowNormArgs), x.data_ptr(), 0, None, 0, None, None, 0, 1.0, y.data_ptr(), gate.data_ptr() + 256, K + 128, gain.data_ptr(),
+                          gain.data_ptr(), gain.data_ptr(), x_out.data_ptr(), 1e-5)
+        if streams is not None:
+            n.x, n.x_stride, n.coef, n.n_terms, n.y, n.gate, n.ldg, n.post_gain = streams.data_ptr(), M * K, gain.data_ptr(), 2, None, None, 0, None
+        return B.load().pcb_norm_linear_takes(ctypes.byref(n), ctypes.byref(a), None if b is None else ctypes.byref(b))
+
+    def product(to):
+        return B.linear_args(h, w, to, M=M)
+    bf = lambda t: t.view(torch.bfloat16).view(-1)                   # noqa: E731
+    assert asked(product(P)) == 0 and asked(product(P), product(Q)) == 0
+    assert asked(product(bf(x)[:M * N].view(M, N))) == B.NOT_TAKEN and asked(product(bf(y)[:M * N].view(M, N))) == B.NOT_TAKEN
+    assert asked(product(gate.view(-1)[:M * N].view(M, N))) == B.NOT_TAKEN
+    assert asked(product(P), product(gate.view(-1)[:M * N].view(M, N))) == B.NOT_TAKEN
+    assert asked(product(bf(out)[:M * N].view(M, N))) == B.NOT_TAKEN
+    tail = bf(room)
+    # two streams of M x K: their last element counts, what begins behind it does not; an fp32 result by its own size
+    assert asked(product(tail[4 * M * K:4 * M * K + M * N].view(M, N)), streams=room) == 0
+    assert asked(product(tail[4 * M * K - 8:4 * M * K - 8 + M * N].view(M, N)), streams=room) == B.NOT_TAKEN
+    assert asked(product(tail[:M * N].view(M, N)), streams=room[M * N // 2:]) == 0
+    assert asked(product(room[:M * N].view(M, N)), streams=room[M * N // 2:]) == B.NOT_TAKEN
+    for over in (x, y, gate.view(torch.float32)):
+        assert asked(product(P), x_out=over) == -2001
+    assert asked(product(P), x_out=room[M * K:], streams=room) == -2001 and asked(product(P), x_out=room[2 * M * K:], streams=room) == 0

@@ -662,6 +662,42 @@ def test_far_positions_in_a_long_prompt_and_after_it(dtype):
     assert rel(torch.cat(got), want) < tol(dtype, 5e-5, 8e-2)
 
 
+def shape_bare(width):
+    """Layers without a feed-forward one after another, of sizes whose norms ride in the next projection's launch at few rows; 2048: more workgroups than
+    fit the chip at a time."""
+    if width == 2048:
+        layers = [att(16, 4, 128, 128, mask=0, v_mix=True), att(16, 4, 128, 128, mask=0, v_mix=True), att(16, 4, 128, 128, mask=0, v_mix=True, ff=96)]
+    else:
+        layers = [att(4, 2, 32, 32, mask=20), lat(4, 32, 16, 32, 64, mask=0), mls(4, 32, 32), mls(2, 32, 64, ff=64), lat(4, 32, 16, 32, 64, mask=9), att(8, 2, 64, 64, mask=0)]
+    return FivesunShape(vocab_size=90, hidden_size=width, norm_eps=1e-6, embed_scale=5.3, layers=layers)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width,rows", [(2048, 1), (2048, 2), (1024, 1), (1024, 4), (512, 1), (512, 3), (512, 8)])
+def test_gates_of_layers_without_a_feed_forward_in_the_next_layers_launch(dtype, width, rows, monkeypatch):
+    """One-token steps, eager and captured, against the same steps with the norms in launches of their own; one request also against the oracle."""
+    from promptcache_amd.model.fivesun_hip import FivesunHIP
+    s = shape_bare(width)
+    w = W.make_fivesun_weights(s, seed=7)
+    m = FivesunHIP(s, w, device=DEV, dtype=dtype)
+    tokens = [toks(6, s.vocab_size, seed=60 + r) for r in range(rows)]
+
+    def steps(graphs):
+        m.use_graphs = graphs
+        ar = m.new_arena(rows, 16)
+        slots = [ar.alloc() for _ in range(rows)]
+        return torch.stack([m.forward_rows(ar, slots, [[t[i]] for t in tokens]) for i in range(6)])
+    eager, captured = steps(False), steps(True)
+    monkeypatch.setattr(B(), "NORM_LINEAR_MAX", 0)
+    m._graphs.clear()
+    # (fp32: other orders of the same sums; bf16: roundings of a row's elements that fall the other way, through all layers)
+    apart = steps(False)
+    assert rel(eager, apart) < tol(dtype, 2e-6, 4e-2) and rel(captured, apart) < tol(dtype, 2e-6, 4e-2)
+    if rows == 1:
+        want = oracle_logits(s, w, tokens[0])[0]
+        assert rel(eager[:, 0], want) < tol(dtype, 3e-5, 0.15) and rel(captured[:, 0], want) < tol(dtype, 3e-5, 0.15)
+
+
 def test_same_rows_same_values_whatever_the_company():
     """float32: a request's logits next to other requests, and on another slot, agree with those it gets alone to summation order."""
     s, w, m = model("wide", torch.float32)
