@@ -140,9 +140,13 @@ typedef struct pcb_linear_args {
     int32_t y2_f32;
 } pcb_linear_args;
 int pcb_linear(const pcb_linear_args* a, void* stream);
-/* pcb_linear(a), pcb_linear(b) for two products of the same rows' count that do not need one another: one launch where both are of few rows (a a plain
- * store, b that or gated), else those two. */
+/* pcb_linear(a), pcb_linear(b) for two products of the same rows' count that do not need one another: one launch where a is a plain store, b that or gated, and both
+ * are of few rows, or in bf16 of more than 64 over the same k and one grid of tiles is the faster; else those two.  Nothing orders the two products within a launch:
+ * results (y, y2 in fp32) that overlap the other's results or the rows and gates it reads go out as two; rows that row_dst, row_off2 or row_off3 place, and rows read
+ * through row_src, are the caller's to keep apart.  pcb_linear_pair_form: 0 for two launches, 1 for one of few rows, 2 .. 6 for one grid of tiles (128 x 128,
+ * 128 x 192, 128 x 256, 256 x 192, 256 x 256), or an error; nothing is launched. */
 int pcb_linear_pair(const pcb_linear_args* a, const pcb_linear_args* b, void* stream);
+int pcb_linear_pair_form(const pcb_linear_args* a, const pcb_linear_args* b);
 /* Two scaled accumulations into the same rows (same M, N, y, ldy; b without a base of its own): pcb_linear(a), then pcb_linear(b), in one launch where
  * there are few rows.  z (fp32 [M][b->K], may be null): b's input is pcb_polynorm(z, coef, eps); b->x is then scratch of that shape, which may or may not
  * be written. */

@@ -191,23 +191,46 @@ int add2(const pcb_linear_args& a, const pcb_linear_args& b, const float* z, con
 
 }  // namespace
 
-PCB_EXPORT int pcb_linear_pair(const pcb_linear_args* a, const pcb_linear_args* b, void* stream) {
-    int rc = pcb_linear_check(a);
-    if (rc == PCB_OK) rc = pcb_linear_check(b);
-    if (rc != PCB_OK) return rc;
-    const bool one = a->dtype == b->dtype && a->M == b->M && a->M > 0 && a->M <= 16 && a->n_batch == 0 && b->n_batch == 0 && a->epilogue == PCB_EPI_STORE &&
-                     b->epilogue != PCB_EPI_SCALE_ADD && pcb_linear_pieces(*a) && pcb_linear_pieces(*b);
+// Whether either product's results lie apart from the other's results and from the rows and gates it reads: in one launch nothing orders the two
+static bool pair_apart(const pcb_linear_args& a, const pcb_linear_args& b) {
+    auto from = [](const pcb_linear_args& p, const pcb_linear_args& q) {         // p's results from what q reads
+        const int es = q.dtype == PCB_BF16 ? 2 : 4;
+        return (q.row_src || pcb_results_apart(p, pcb_rows_span(q.x, q.M, q.ldx, q.K, es))) &&
+               pcb_results_apart(p, pcb_rows_span(q.row_gate, q.M, q.ld_row_gate, 1, es));
+    };
+    const int es = b.out_f32 || b.dtype == PCB_F32 ? 4 : 2, cols = b.split_n > 0 ? b.split_n : b.split_n3 > 0 ? b.split_n3 : b.N;
+    return from(a, b) && from(b, a) && (b.row_dst || pcb_results_apart(a, pcb_rows_span(b.y, b.M, b.ldy, cols, es))) &&
+           (!b.y2_f32 || b.split_n <= 0 || pcb_results_apart(a, pcb_rows_span(b.y2, b.M, b.head_stride2, b.N - b.split_n, 4)));
+}
+
+// How a pair goes out: 0 two launches, 1 one of few rows, 2 + shape one grid of tiles
+static int pair_form(const pcb_linear_args& a, const pcb_linear_args& b) {
+    if (a.dtype != b.dtype || a.M != b.M || a.M <= 0 || a.n_batch != 0 || b.n_batch != 0 || a.epilogue != PCB_EPI_STORE || b.epilogue == PCB_EPI_SCALE_ADD ||
+        !pcb_linear_pieces(a) || !pcb_linear_pieces(b) || !pair_apart(a, b))
+        return 0;
     // (A gated unit in bf16 only up to 80 MB of weights: alone it is faster then.  us, two launches / one, 8 rows, residual gate and gated unit of a width:
     // 2048 15.9 / 14.3, 2560 (66 MB) 24.4 / 21.6, 3072 (94 MB) 28.9 / 29.8, 1 row 13.6 / 12.8, 19.4 / 18.9, 23.4 / 26.5.  9 and 16 rows: bf16 2048 18.7 / 14.7 and
     // 20.0 / 16.0, 2560 29.2 / 22.2 and 32.9 / 25.2; fp32 2048 27.5 / 23.6 and 29.1 / 26.5; plain, 2560 + 8192
     // columns, K = 2048, bf16 18.9 / 15.1 and 20.8 / 17.6.)
-    const bool heavy = a->dtype == PCB_BF16 && b->epilogue == PCB_EPI_SILU_MUL && ((int64_t)a->N * a->K + 2 * (int64_t)b->N * b->K) * 2 > 80000000;
-    if (!one || heavy) {
-        if (a->M > 64 && pcb_linear_tiles_pair(*a, *b, (hipStream_t)stream, &rc)) return rc;
-        rc = pcb_linear(a, stream);
-        return rc == PCB_OK ? pcb_linear(b, stream) : rc;
-    }
-    return a->dtype == PCB_BF16 ? pair<pcb::bf16_t>(*a, *b, (hipStream_t)stream) : pair<float>(*a, *b, (hipStream_t)stream);
+    const bool heavy = a.dtype == PCB_BF16 && b.epilogue == PCB_EPI_SILU_MUL && ((int64_t)a.N * a.K + 2 * (int64_t)b.N * b.K) * 2 > 80000000;
+    if (a.M <= 16) return heavy ? 0 : 1;
+    const int shape = a.M > 64 ? pcb_linear_tiles_pair_shape(a, b) : -1;
+    return shape < 0 ? 0 : 2 + shape;
+}
+
+PCB_EXPORT int pcb_linear_pair_form(const pcb_linear_args* a, const pcb_linear_args* b) {
+    int rc = pcb_linear_check(a);
+    if (rc == PCB_OK) rc = pcb_linear_check(b);
+    return rc == PCB_OK ? pair_form(*a, *b) : rc;
+}
+
+PCB_EXPORT int pcb_linear_pair(const pcb_linear_args* a, const pcb_linear_args* b, void* stream) {
+    const int form = pcb_linear_pair_form(a, b);
+    if (form < 0) return form;
+    if (form >= 2) return pcb_linear_tiles_pair(*a, *b, form - 2, (hipStream_t)stream);
+    if (form == 1) return a->dtype == PCB_BF16 ? pair<pcb::bf16_t>(*a, *b, (hipStream_t)stream) : pair<float>(*a, *b, (hipStream_t)stream);
+    const int rc = pcb_linear(a, stream);
+    return rc == PCB_OK ? pcb_linear(b, stream) : rc;
 }
 
 PCB_EXPORT int pcb_linear_add2(const pcb_linear_args* a, const pcb_linear_args* b, const float* z, const float* coef, float eps, void* stream) {

@@ -5,8 +5,9 @@
 #include "pb_common.h"
 
 int pcb_linear_tiles(const pcb_linear_args& a, hipStream_t stream);
-// two products of the same rows in one grid where that is the better (false: it is not, nothing was launched)
-bool pcb_linear_tiles_pair(const pcb_linear_args& a, const pcb_linear_args& b, hipStream_t stream, int* rc);
+// two products of the same rows in one grid: the tiles for it where that is the better, else -1
+int pcb_linear_tiles_pair_shape(const pcb_linear_args& a, const pcb_linear_args& b);
+int pcb_linear_tiles_pair(const pcb_linear_args& a, const pcb_linear_args& b, int shape, hipStream_t stream);
 // ... and those over some tens or hundreds of rows (pb_linear_waves.hip): which launches whose rows can be read in 16-byte chunks it is the better for
 int64_t pcb_linear_waves_tiles(const pcb_linear_args& a);
 bool pcb_linear_waves_fits(const pcb_linear_args& a);

@@ -460,14 +460,16 @@ static float grid_us(const pcb_linear_args& a, const pcb_linear_args* b, int sha
     return round * ((float)(tiles / 256) + (rest ? 0.5f + (float)rest / 512.0f : 0.0f)) + 0.056f * act * (float)(t.bm * t.bn / 256);
 }
 
-bool pcb_linear_tiles_pair(const pcb_linear_args& a, const pcb_linear_args& b, hipStream_t stream, int* rc) {
+int pcb_linear_tiles_pair_shape(const pcb_linear_args& a, const pcb_linear_args& b) {
     auto fits = [](const pcb_linear_args& q) {
         return q.dtype == PCB_BF16 && q.M > 64 && q.n_groups == 0 && q.n_batch == 0 && !q.row_src && q.ldx < (1 << 22) && q.ldw < (1 << 22) && pcb_linear_pieces(q);
     };
     const bool gated = b.epilogue == PCB_EPI_SILU_MUL;
-    if (!fits(a) || !fits(b) || a.M != b.M || a.K != b.K || a.epilogue != PCB_EPI_STORE || b.epilogue == PCB_EPI_SCALE_ADD || (gated && a.M <= 128)) return false;
+    if (!fits(a) || !fits(b) || a.M != b.M || a.K != b.K || a.epilogue != PCB_EPI_STORE || b.epilogue == PCB_EPI_SCALE_ADD || (gated && a.M <= 128)) return -1;
     const int shape = choose(a, &b);
-    if (grid_us(a, &b, shape) >= 0.97f * (grid_us(a, nullptr, choose(a, nullptr)) + grid_us(b, nullptr, choose(b, nullptr)))) return false;
-    *rc = gated ? dispatch_pair<PCB_EPI_SILU_MUL>(a, b, shape, stream) : dispatch_pair<PCB_EPI_STORE>(a, b, shape, stream);
-    return true;
+    return grid_us(a, &b, shape) < 0.97f * (grid_us(a, nullptr, choose(a, nullptr)) + grid_us(b, nullptr, choose(b, nullptr))) ? shape : -1;
+}
+
+int pcb_linear_tiles_pair(const pcb_linear_args& a, const pcb_linear_args& b, int shape, hipStream_t stream) {
+    return b.epilogue == PCB_EPI_SILU_MUL ? dispatch_pair<PCB_EPI_SILU_MUL>(a, b, shape, stream) : dispatch_pair<PCB_EPI_STORE>(a, b, shape, stream);
 }
