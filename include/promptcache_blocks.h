@@ -5,7 +5,8 @@
  * on the host before it launches anything, launches on `stream` (a hipStream_t) without synchronising, and takes device
  * pointers unless a parameter says otherwise.  `dtype` selects the element type E of weights, activations and cached keys:
  * PCB_BF16 (products on the bf16 matrix cores, fp32 accumulation) or PCB_F32 (32-bit products: the fp32 matrix cores, or three bf16 parts of
- * every operand where a launch has many tiles, whose error is smaller).
+ * every operand where a launch has many tiles, whose error is smaller; results that parts cannot give -- no numbers, or sums in which elements below 2^-110 count -- come
+ * from the fp32 matrix cores there too).
  * Residual streams, norms, scores, softmax weights, router logits and reductions are fp32 in both.
  */
 #ifndef PROMPTCACHE_BLOCKS_H

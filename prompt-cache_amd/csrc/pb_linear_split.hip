@@ -1,12 +1,13 @@
 // pb_linear over many rows in fp32 on the bf16 matrix cores: every operand element as the sum of three bf16 (8 + 8 + 8 bits: hi + mid + lo is the element
-// exactly, but for parts below 2^-126), a product as the six of the nine partial products that reach 2^-26 of it: hi hi in one sum, hi mid, mid hi, mid mid, hi lo, lo hi in
-// another.  What is left out is at most 2^-26 of a term, and a sum of 32 terms is rounded once: against 64 bits 0.46 of the error of the fp32 matrix cores (K = 1024:
-// 1.9e-7 / 4.1e-7), which do 256 multiply-adds a clock and CU where these do 4096 / 6.
+// exactly, but for what an element below 2^-110 has below 2^-133, bf16's smallest; conversions and products keep subnormal numbers), a product as the six of the
+// nine partial products that reach 2^-26 of it: hi hi in one sum, hi mid, mid hi, mid mid, hi lo, lo hi in another.  What is left out is at most 2^-26 of a term,
+// and a sum of 32 terms is rounded once: against 64 bits 0.46 of the error of the fp32 matrix cores (K = 1024: 1.9e-7 / 4.1e-7), which do 256 multiply-adds a
+// clock and CU where these do 4096 / 6.
 //
 // Workgroup = (32 TM) x (16 WN TN) results, 2 x WN waves of TM x TN blocks of 16 x 16.  Per k-step of 32 the rows go global -> registers (two steps ahead), are split
 // there, each element once a workgroup, and lie in two LDS images of three planes; one barrier a k-step that waits for LDS only.
-// What bounds it: issue.  An element's split is 5.5 VALU instructions, a wave of eight in the 128 x 128 tile has 88 of them and 48 MFMAs a step, two waves to a
-// SIMD: 1200 clocks of the one, 1536 of the other, of which next to nothing overlaps (1.39 us a step; the two from different waves: 1.57 of what the slower
+// What bounds it: issue.  An element's split is 5.5 VALU instructions (and its row's largest magnitude half of one, not counted here), a wave of eight in the 128 x 128
+// tile has 88 of them and 48 MFMAs a step, two waves to a SIMD: 1200 clocks of the one, 1536 of the other, of which next to nothing overlaps (1.39 us a step; the two from different waves: 1.57 of what the slower
 // takes).  Products first and then the splits, in every order that was tried, is as good as any finer mix of them (interleaved by hand 49, by the compiler
 // 46, this 45 us where one is 1024 deep).
 #include <type_traits>
@@ -62,7 +63,14 @@ __global__ __launch_bounds__(128 * WN) void linear_split_kernel(pcb_linear_args 
     };
     const int at = sr * 64 + (((tid & 7) >> 1) ^ ((sr >> 2) & 3)) * 16 + (tid & 1) * 8;
     // part q of a chunk, what it leaves stays (the 16-byte chunk c of row r lies at c ^ (r / 4 & 3): a fragment read touches every bank slot)
+    float top[NC];                                                   // the largest magnitude of each chunk's elements so far
+#pragma unroll
+    for (int i = 0; i < NC; ++i) top[i] = 0.0f;
     auto store = [&](f4& r, int i, int q, int buf) {
+        if (q == 0) {                                                // (a NaN is passed over: its sums are no numbers either)
+            asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(top[i]) : "v"(r[0]), "v"(r[1]));
+            asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(top[i]) : "v"(r[2]), "v"(r[3]));
+        }
         const uint2 p = {bf16_pair(r[0], r[1]), bf16_pair(r[2], r[3])};
         if (q < 2) {
             r[0] -= __uint_as_float(p.x << 16);
@@ -143,37 +151,108 @@ __global__ __launch_bounds__(128 * WN) void linear_split_kernel(pcb_linear_args 
     }
 #pragma unroll
     for (int k = 0; k < MF; ++k) product(k);
-    // What is no number here may have a sum: the parts of an infinity (or of a value that rounds to one) make NaN.  And parts below 2^-126 count as zero, which
-    // results below 2^-80 would show.  Such results go element by element.
-    auto total = [&](int i, int j) {
-        f4 v = big[i][j] + small[i][j];
-        bool none = false;
+    // What is no number here may have a sum: the parts of an infinity (or of a value that rounds to one) make NaN.  And what the parts of a sum's elements leave out,
+    // 2^-134 of each at most, is K 2^-133 times the largest element of its row and column: results below 2^26 times that would show it (rows of zeros aside).  A wave
+    // that has such a result works its blocks out on the fp32 matrix cores and takes it from there: a result depends on its own row and column alone.
+    // What that costs, us: nothing but NaN 600 x 5136, K = 1024 134, 2048 x 2048 x 2048 257 (numbers: 54, 96; fp32 matrix cores from the start 78, 147).  The maxima: 2048
+    // columns and K, 2048 rows 94.1 / 95.6, 600 x 2560, K = 1024 29.9 / 31.1, 600 x 5136 48.1 / 48.2.
+    __shared__ __attribute__((aligned(16))) float tops[ROWS];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) none = none || !(fabsf(v[e]) <= 3.4028234663852886e38f) || (fabsf(v[e]) < 0x1p-80f && v[e] != 0.0f);
-        if (none) {
-            const float* x = xrow((wm * TM + i) * 16 + l15);
-#pragma unroll 1
+    for (int i = 0; i < NC; ++i) {
+        float t = top[i];
+#pragma unroll
+        for (int o = 1; o < 8; o <<= 1) t = fmaxf(t, __shfl_xor(t, o, 64));
+        if ((tid & 7) == 0) tops[RI * i + sr] = t;
+    }
+    __syncthreads();
+    // (first against the largest bound of a lane's results, a NaN through a sum of zeros)
+    f4 v[TM][NB], tw[NB];
+    float tx[TM], most = 0.0f, least = __builtin_inff(), none = 0.0f;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) most = fmaxf(most, tx[i] = tops[(wm * TM + i) * 16 + l15]);
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+        tw[j] = *reinterpret_cast<const f4*>(&tops[BM + (j >= TN ? BN : 0) + (wn * TN + j % TN) * 16 + 4 * g]);
+        most = fmaxf(fmaxf(fmaxf(most, tw[j][0]), fmaxf(tw[j][1], tw[j][2])), tw[j][3]);
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            v[i][j] = big[i][j] + small[i][j];
+#pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float* w = wrow((j >= TN ? BN : 0) + (wn * TN + j % TN) * 16 + 4 * g + e);
-                float t = 0.0f, t1 = 0.0f;                           // (two chains, as the fp32 matrix cores have them; K is even)
-#pragma unroll 1
-                for (int k = 0; k < K; k += 2) {
-                    t = __builtin_fmaf(x[k], w[k], t);
-                    t1 = __builtin_fmaf(x[k + 1], w[k + 1], t1);
-                }
-                t += t1;
-                v = e == 0 ? f4{t, v[1], v[2], v[3]} : e == 1 ? f4{v[0], t, v[2], v[3]} : e == 2 ? f4{v[0], v[1], t, v[3]} : f4{v[0], v[1], v[2], t};
+                least = fminf(least, fabsf(v[i][j][e]));
+                none = __builtin_fmaf(v[i][j][e], 0.0f, none);
             }
         }
-        return v;
+    const float share = (float)K * 0x1p-107f;
+    auto lost = [&](int i, int j, int e) {
+        const float r = fabsf(v[i][j][e]), x = tx[i], w = tw[j][e];
+        return !(r <= 3.4028234663852886e38f) || (x > 0.0f && w > 0.0f && r < fmaxf(x, w) * share);
     };
+    bool again = least < most * share || !(none == 0.0f);
+    if (__any(again)) {
+        again = false;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) again = again || lost(i, j, e);
+    }
+    if (__any(again)) {
+        const float *xs[TM], *ws[NB];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) xs[i] = xrow((wm * TM + i) * 16 + l15) + 4 * g;
+#pragma unroll
+        for (int j = 0; j < NB; ++j) ws[j] = wrow((j >= TN ? BN : 0) + (wn * TN + j % TN) * 16 + l15) + 4 * g;
+        f4 nx[TM], nw[NB];
+        auto ask = [&](int k) {                                      // (past K the first ones again, not counted)
+            const int at = k + 4 * g < K ? k : -4 * g;
+#pragma unroll
+            for (int i = 0; i < TM; ++i) nx[i] = *reinterpret_cast<const f4*>(xs[i] + at);
+#pragma unroll
+            for (int j = 0; j < NB; ++j) nw[j] = *reinterpret_cast<const f4*>(ws[j] + at);
+        };
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) big[i][j] = small[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+        ask(0);
+#pragma unroll 1
+        for (int k = 0; k < K; k += 16) {                            // (a lane's four elements are the k of four products; even and odd in sums of their own)
+            const bool in = k + 4 * g < K;
+            f4 x[TM], w[NB];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) x[i] = in ? nx[i] : f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < NB; ++j) w[j] = in ? nw[j] : f4{0.f, 0.f, 0.f, 0.f};
+            if (k + 16 < K) ask(k + 16);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < NB; ++j) {
+                        f4& c = e & 1 ? small[i][j] : big[i][j];
+                        c = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j][e], x[i][e], c, 0, 0, 0);
+                    }
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[i][j][e] = lost(i, j, e) ? big[i][j][e] + small[i][j][e] : v[i][j][e];
+    }
     f4 acc[TM][TN], acc2[TWO ? TM : 1][TWO ? TN : 1];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            acc[i][j] = total(i, j);
-            if (TWO) acc2[TWO ? i : 0][TWO ? j : 0] = total(i, TN + j);
+            acc[i][j] = v[i][j];
+            if (TWO) acc2[TWO ? i : 0][TWO ? j : 0] = v[i][TN + j];
         }
     finish_tile<float, EPI, TM, TN, WN>(a, acc, acc2, m_lo, m_hi, n_lo, wm, wn, g, l15);
 }

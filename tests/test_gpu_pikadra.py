@@ -455,6 +455,45 @@ def test_fp32_products_in_parts_and_what_is_no_number(M, N, K):
     assert bool(((y.double() - z).abs() <= bound * mag)[ok].all())
 
 
+@pytest.mark.parametrize("M,N", [(587, 1026), (587, 2562), (587, 5134)])
+@pytest.mark.parametrize("K", [4, 36, 520])
+@pytest.mark.parametrize("small,large", [(-112, 40), (-118, 60), (-118, 100), (-130, 40), (-130, 60), (-140, 120), (-148, 126), (-104, 100)])
+def test_fp32_products_of_the_smallest_and_the_largest_numbers(M, N, K, small, large):
+    """Elements whose last bits lie below bf16's smallest number, subnormal ones among them, beside large ones: the error bound of fp32 sums, as for
+    ordinary numbers (4 sqrt(K / 32 + 1) 2^-24 of the magnitudes; of subnormal sums each of K roundings may be half of 2^-149), whichever operand is the small
+    one, in some rows or in all, and in the gated unit."""
+    b = B()
+    g = torch.Generator().manual_seed(K + small)
+    bound = 4 * (K / 32 + 1) ** 0.5 * 2.0 ** -24
+
+    def draw(rows, e):
+        return ((torch.rand(rows, K, generator=g, dtype=torch.float64) + 0.5) * (1 - 2 * torch.randint(0, 2, (rows, K), generator=g)) * 2.0 ** e).float().to(DEV)
+
+    def check(x, w):
+        y = torch.full((M, N), float("nan"), device=DEV)
+        b.linear(x, w, y, M=M)
+        x, w = x.double(), w.double().T.contiguous()
+        assert bool(((y.double() - x @ w).abs() <= bound * (x.abs() @ w.abs()) + K * 2.0 ** -150).all())
+    lo, hi = draw(M, small), draw(N, large)
+    check(lo, hi)
+    check(draw(M, large), draw(N, small))
+    mixed = draw(M, 0)
+    mixed[3], mixed[M - 1], mixed[70] = lo[3], lo[70], 0.0
+    mixed[5, K // 2:] = lo[5, K // 2:]
+    if large < 110:                                                  # (sums that fit fp32)
+        check(mixed, hi)
+    else:
+        check(mixed, torch.where(torch.arange(N, device=DEV)[:, None] % 7 == 0, hi * 2.0 ** -20, draw(N, 1)))
+    h = N // 2
+    x, w, w2 = lo, hi[:h].contiguous(), draw(h, large)
+    if small + large < 60 and small + large > -60:                   # (their products fit)
+        t, u = x.double() @ w.double().T.contiguous(), x.double() @ w2.double().T.contiguous()
+        y = torch.full((M, h), float("nan"), device=DEV)
+        b.linear(x, w, y, M=M, epilogue=b.EPI_SILU_MUL, w2=w2, act=b.ACT_RELU)
+        mt, mu = x.double().abs() @ w.double().abs().T.contiguous(), x.double().abs() @ w2.double().abs().T.contiguous()
+        assert bool(((y.double() - torch.relu(t) * u).abs() <= bound * 2.1 * mt * mu + 2.0 ** -149).all())
+
+
 @pytest.mark.parametrize("M,N", [(1, 70), (9, 64), (16, 130), (40, 100), (130, 260), (600, 2564), (2000, 2040)])
 @pytest.mark.parametrize("K", [4, 30, 36, 68, 516])
 def test_fp32_projections_at_every_tile_and_their_edges(M, N, K):
