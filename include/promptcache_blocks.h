@@ -141,6 +141,8 @@ typedef struct pcb_linear_args {
     int32_t y2_f32;
 } pcb_linear_args;
 int pcb_linear(const pcb_linear_args* a, void* stream);
+/* Whether an fp32 launch has its operands split into bf16 parts: 0 no, 1 .. 3 in tiles of 64 x 64, 64 x 128 or 128 x 128 weight rows, or an error; nothing is launched. */
+int pcb_linear_parts_form(const pcb_linear_args* a);
 /* pcb_linear(a), pcb_linear(b) for two products of the same rows' count that do not need one another: one launch where a is a plain store, b that or gated, and both
  * are of few rows, or in bf16 of more than 64 over the same k and one grid of tiles is the faster; else those two.  Nothing orders the two products within a launch:
  * results (y, y2 in fp32) that overlap the other's results or the rows and gates it reads go out as two; rows that row_dst, row_off2 or row_off3 place, and rows read

@@ -509,6 +509,40 @@ bool dma_ok(const pcb_linear_args& a) {
            ((uintptr_t)a.x | (uintptr_t)a.w | (uintptr_t)a.w2) % 16 == 0 && (int64_t)pcb_ceil_div(a.N, 32) * pcb_ceil_div(a.M, 32) < (1 << 30);
 }
 
+// fp32 (1 / 16 of the bf16 rate): bound by the matrix cores, so what counts is that all CUs have the same share of tiles.  Whole rounds of
+// the 256 CUs times a tile's work; a 128 x 128 tile costs 3.8 of 64 x 64 and a 32 x 64 tile 0.575 (us, 64-, 128- and 32-row tiles):
+// 2048 x 2048 x 2048 158 / 149 / 166, 4096 x 4096, K = 1024 299 / 276 / 317, 1200 x 4096, K = 2048 188 / 267 / 203, 600 x 2564, K = 1024
+// 44 / 76 / 47, 600 x 2048, K = 2048 79 / 146 / 68, 130 x 1024, K = 1024 25 / 75 / 17.
+// (32 x 32 tiles, three to a CU, up to 768 of them: 600 x 1024, K = 1024 25.8 -> 21.5, 300 x 1024 18.1 -> 16.3, 200 x 2564 26.5 -> 22.1, 600 x 512,
+// K = 512 10.3 -> 9.6; 600 x 2564 (1539) 42.9, 45.1 so.  What is below a round of the chip or deep is with pb_linear_waves.hip.)
+struct Fp32Tile {
+    int rows;                                                        // (0: 32 x 32)
+    float rounds;
+};
+Fp32Tile fp32_tile(const pcb_linear_args& a, int rows) {
+    const int64_t batch = a.n_batch > 0 ? a.n_batch : 1, extra = a.n_groups / 2;      // (groups: part tiles)
+    auto rounds = [&](int bm, int bn) { return (float)((batch * (pcb_ceil_div(a.M, bm) + extra) * pcb_ceil_div(a.N, bn) + 255) / 256); };
+    const bool gated = a.epilogue == PCB_EPI_SILU_MUL;
+    const int tnw = gated ? 2 : 4;
+    if (!gated && a.n_groups == 0 && batch * pcb_ceil_div(a.M, 32) * pcb_ceil_div(a.N, 32) <= 768) return {0, rounds(32, 32)};
+    const float large = 3.8f * rounds(128, 32 * tnw), mid = rounds(64, 16 * tnw), small = 0.575f * rounds(32, 16 * tnw);
+    if (rows > 64 && large <= mid && large <= small) return {128, rounds(128, 32 * tnw)};
+    return rows > 32 && mid <= small ? Fp32Tile{64, mid} : Fp32Tile{32, rounds(32, 16 * tnw)};
+}
+
+// What a plain or batched launch takes on the fp32 matrix cores, us, by its kernel's rounds of the chip and k-steps of 32 (fitted to 2080 sizes, within 10 %)
+float fp32_us(const pcb_linear_args& a) {
+    const float steps = (float)pcb_ceil_div(a.K, 32);
+    if (pcb_linear_waves_fits(a)) return 0.22f * steps * (float)((pcb_linear_waves_tiles(a) * (a.n_batch > 0 ? a.n_batch : 1) + 255) / 256);
+    const Fp32Tile t = fp32_tile(a, a.M);
+    switch (t.rows) {
+        case 0: return 0.16f * t.rounds * steps + 6.4f;
+        case 128: return (0.25f + 1.92f * t.rounds) * steps + 6.4f + 2.3f * t.rounds;
+        case 64: return (0.1f + 0.545f * t.rounds) * steps + 5.2f + 0.5f * t.rounds;
+        default: return (0.07f + 0.29f * t.rounds) * steps + 5.0f + 0.25f * t.rounds;
+    }
+}
+
 template <typename E, int EPI>
 int dispatch_dma(const pcb_linear_args& a, int rows, hipStream_t stream) {
     // the largest tile that still gives every CU a workgroup; grouped launches count the tiles their rows fill
@@ -516,19 +550,11 @@ int dispatch_dma(const pcb_linear_args& a, int rows, hipStream_t stream) {
     const int64_t batch = a.n_batch > 0 ? a.n_batch : 1;
     auto tiles = [&](int bm, int bn) { return batch * pcb_ceil_div(a.M, bm) * pcb_ceil_div(a.N, bn); };
     if constexpr (sizeof(E) == 4) {
-        // fp32 (1 / 16 of the bf16 rate): bound by the matrix cores, so what counts is that all CUs have the same share of tiles.  Whole rounds of
-        // the 256 CUs times a tile's work; a 128 x 128 tile costs 3.8 of 64 x 64 and a 32 x 64 tile 0.575 (us, 64-, 128- and 32-row tiles):
-        // 2048 x 2048 x 2048 158 / 149 / 166, 4096 x 4096, K = 1024 299 / 276 / 317, 1200 x 4096, K = 2048 188 / 267 / 203, 600 x 2564, K = 1024
-        // 44 / 76 / 47, 600 x 2048, K = 2048 79 / 146 / 68, 130 x 1024, K = 1024 25 / 75 / 17.
-        const int64_t extra = a.n_groups / 2;                        // (groups: part tiles)
-        auto rounds = [&](int bm, int bn) { return (batch * (pcb_ceil_div(a.M, bm) + extra) * pcb_ceil_div(a.N, bn) + 255) / 256; };
-        // (32 x 32 tiles, three to a CU, up to 768 of them: 600 x 1024, K = 1024 25.8 -> 21.5, 300 x 1024 18.1 -> 16.3, 200 x 2564 26.5 -> 22.1, 600 x 512,
-        // K = 512 10.3 -> 9.6; 600 x 2564 (1539) 42.9, 45.1 so.  What is below a round of the chip or deep is with pb_linear_waves.hip.)
+        const Fp32Tile t = fp32_tile(a, rows);
         if constexpr (EPI != PCB_EPI_SILU_MUL)
-            if (a.n_groups == 0 && batch * pcb_ceil_div(a.M, 32) * pcb_ceil_div(a.N, 32) <= 768) return launch_dma<E, EPI, 1, 1, 3>(a, stream);
-        const float large = 3.8f * rounds(128, 32 * TNW), mid = rounds(64, 16 * TNW), small = 0.575f * rounds(32, 16 * TNW);
-        if (rows > 64 && large <= mid && large <= small) return launch_dma<E, EPI, 4, TNW, 2>(a, stream);
-        return rows > 32 && mid <= small ? launch_dma<E, EPI, 2, TNW / 2, 3>(a, stream) : launch_dma<E, EPI, 1, TNW / 2, 3>(a, stream);
+            if (t.rows == 0) return launch_dma<E, EPI, 1, 1, 3>(a, stream);
+        if (t.rows == 128) return launch_dma<E, EPI, 4, TNW, 2>(a, stream);
+        return t.rows == 64 ? launch_dma<E, EPI, 2, TNW / 2, 3>(a, stream) : launch_dma<E, EPI, 1, TNW / 2, 3>(a, stream);
     }
     // (two workgroups of a CU hide each other's loads behind their products; a lone one needs a stage more in flight)
     if (rows > 64 && tiles(128, 32 * TNW) > 256) return launch_dma<E, EPI, 4, TNW, 2>(a, stream);
@@ -588,6 +614,9 @@ FewRows few_rows(const pcb_linear_args& a) {
     const int64_t most = any ? INT64_MAX : add ? (a.K < (bf ? 2048 : 1024) ? 640 : bf || a.M > 4 ? 768 : 1024) : bf || a.M <= 4 ? 1024 : 768;
     return g2 <= most ? FewRows{2, late} : one;
 }
+
+// Whether an fp32 launch of more than sixteen rows, read in 16-byte chunks, has its operands split (pb_linear_split.hip; at a tie, whose error is the smaller)
+bool in_parts(const pcb_linear_args& a) { return pcb_linear_split_fits(a) && pcb_linear_split_us(a) < 1.01f * fp32_us(a); }
 
 template <typename E>
 int dispatch(const pcb_linear_args& a, hipStream_t stream) {
@@ -649,7 +678,7 @@ int dispatch(const pcb_linear_args& a, hipStream_t stream) {
         return pcb_check_launch("linear_skinny_kernel");
     }
     if (dma_ok(a)) {
-        if (sizeof(E) == 4 && pcb_linear_split_fits(a)) return pcb_linear_split(a, stream);
+        if (sizeof(E) == 4 && in_parts(a)) return pcb_linear_split(a, stream);
         if (pcb_linear_waves_fits(a)) return pcb_linear_waves(a, stream);
         // Plain launches whose 128 x 128 tiles reach more than half of the 256 CUs go to the whole-CU tiles of pb_linear_tiles.hip (row strides
         // such that a tile's rows lie within 32-bit offsets); below, the smaller tiles here give more CUs work: 300 x 2048, K = 2048 (48 tiles)
@@ -713,6 +742,12 @@ int pcb_linear_check(const pcb_linear_args* a) {
                 PCB_ERR_ARG, "pcb_linear: bad column-wise destination");
     PCB_REQUIRE(a->split_n > 0 || a->split_n3 > 0 || a->epilogue == PCB_EPI_SCALE_ADD || a->ldy >= a->N, PCB_ERR_ARG, "pcb_linear: ldy < N");
     return PCB_OK;
+}
+
+PCB_EXPORT int pcb_linear_parts_form(const pcb_linear_args* a) {
+    const int rc = pcb_linear_check(a);
+    if (rc != PCB_OK) return rc;
+    return a->dtype == PCB_F32 && a->M > 16 && dma_ok(*a) && in_parts(*a) ? pcb_linear_split_shape(*a) : 0;
 }
 
 PCB_EXPORT int pcb_linear(const pcb_linear_args* a, void* stream) {

@@ -270,27 +270,50 @@ int64_t tiles_of(const pcb_linear_args& a, int rows, int cols) {
     return (int64_t)pcb_ceil_div(a.M, rows) * pcb_ceil_div(W * a.N, cols) * (a.n_batch > 0 ? a.n_batch : 1);
 }
 
+// The tile whose workgroups on the fullest CU cost least, us a k-step of 32: one, two, .. eight of 64 x 64 0.56, 1.02, .. 4.06 (gated, four waves: 0.66, 1.03,
+// .. 3.75), of 64 x 128 0.86, 1.83, .. 7.9, of 128 x 128 1.42, 3.0, 4.6, 6.4 -- the larger, the fewer splits a product.  At 570 sizes (100 .. 2048 rows, 512 ..
+// 10272 columns, K = 256 .. 2048) on average 0.3 % from the fastest of them.
+enum Shape { SMALL = 1, WIDE, LARGE };
+Shape shape_of(const pcb_linear_args& a) {
+    auto on_a_cu = [&](int rows, int cols) { return (float)((tiles_of(a, rows, cols) + 255) / 256); };
+    const bool gated = a.epilogue == PCB_EPI_SILU_MUL;
+    const float large = 1.45f * on_a_cu(128, 128), wide = 0.885f * on_a_cu(64, 128), small = gated ? 0.24f + 0.44f * on_a_cu(64, 64) : 0.52f * on_a_cu(64, 64);
+    return large <= wide && large <= small ? LARGE : wide <= small ? WIDE : SMALL;
+}
+
 template <int EPI>
 int dispatch(const pcb_linear_args& a, hipStream_t stream) {
-    // The tile whose workgroups on the fullest CU cost least, us a k-step of 32: one, two, .. eight of 64 x 64 0.56, 1.02, .. 4.06 (gated, four waves: 0.66, 1.03,
-    // .. 3.75), of 64 x 128 0.86, 1.83, .. 7.9, of 128 x 128 1.42, 3.0, 4.6, 6.4 -- the larger, the fewer splits a product.  At 570 sizes (100 .. 2048 rows, 512 ..
-    // 10272 columns, K = 256 .. 2048) on average 0.3 % from the fastest of them.
-    auto on_a_cu = [&](int rows, int cols) { return (float)((tiles_of(a, rows, cols) + 255) / 256); };
     constexpr bool TWO = EPI == PCB_EPI_SILU_MUL;
-    const float large = 1.45f * on_a_cu(128, 128), wide = 0.885f * on_a_cu(64, 128), small = TWO ? 0.24f + 0.44f * on_a_cu(64, 64) : 0.52f * on_a_cu(64, 64);
-    if (large <= wide && large <= small) return launch<EPI, 4, TWO ? 1 : 2, 4>(a, stream);
-    if (wide <= small) return launch<EPI, 2, TWO ? 1 : 2, 4>(a, stream);
-    if constexpr (TWO)
-        return launch<EPI, 2, 1, 2>(a, stream);
-    else
-        return launch<EPI, 2, 1, 4>(a, stream);
+    switch (shape_of(a)) {
+        case LARGE: return launch<EPI, 4, TWO ? 1 : 2, 4>(a, stream);
+        case WIDE: return launch<EPI, 2, TWO ? 1 : 2, 4>(a, stream);
+        default: return launch<EPI, 2, 1, TWO ? 2 : 4>(a, stream);
+    }
 }
 
 }  // namespace
 
-// From 145 tiles of 64 x 64 on, whatever K: 128 of them 0.70 .. 0.90 of the fp32 matrix cores' speed (tiles of 32 x 32 there, on all CUs), 160 1.01 .. 1.15 of it, 256 1.05 ..
-// 1.30, 480 1.20 .. 1.46.  600 x 5136, K = 1024 78 -> 46.6 us, the gated pair of 2048 60 -> 46.3, 2048 x 2048 x 2048 147 -> 93.4.
+// From 145 tiles of 64 x 64 on (128 of them 0.70 .. 0.90 of the fp32 matrix cores' speed: tiles of 32 x 32 there, on all CUs), where the launch takes less by this
+// estimate than by fp32_us() (pb_linear.hip): fitted to 2080 sizes of 17 .. 2048 rows, 145 .. 2048 such tiles, K = 256 .. 2048, plain and gated.  Slower than the fp32 matrix
+// cores by more than 4 % at five of them (splitting whatever has 145 tiles: at 468, by up to half: 32 rows of 65920 columns, K = 1024 57.4 / 84.5, 600 x 1664 -- two
+// rounds of the chip -- 26.7 / 32.3), on average 0.2 % behind the better of the two.  600 x 5136, K = 1024 78 -> 48.2 us, the gated pair of 2048 60 -> 46.3,
+// 2048 x 2048 x 2048 147 -> 95.6.
 bool pcb_linear_split_fits(const pcb_linear_args& a) { return a.n_groups == 0 && tiles_of(a, 64, 64) > 144; }
+
+int pcb_linear_split_shape(const pcb_linear_args& a) { return shape_of(a); }
+
+float pcb_linear_split_us(const pcb_linear_args& a) {
+    const bool gated = a.epilogue == PCB_EPI_SILU_MUL;
+    const float steps = (float)((a.K + 31) / 32);
+    auto on_a_cu = [&](int rows, int cols) { return (float)((tiles_of(a, rows, cols) + 255) / 256); };
+    switch (shape_of(a)) {
+        case LARGE: return (1.29f * steps + 4.5f) * on_a_cu(128, 128) + 5.0f;
+        case WIDE: return gated ? (0.765f * steps + 3.3f) * on_a_cu(64, 128) + 4.2f : (0.81f * steps + 2.4f) * on_a_cu(64, 128) + 4.7f;
+        default:
+            return gated ? (0.22f + 0.38f * on_a_cu(64, 64)) * steps + 6.2f + 0.75f * on_a_cu(64, 64) :
+                           (0.045f + 0.425f * on_a_cu(64, 64)) * steps + 5.9f + 0.7f * on_a_cu(64, 64);
+    }
+}
 
 int pcb_linear_split(const pcb_linear_args& a, hipStream_t stream) {
     switch (a.epilogue) {

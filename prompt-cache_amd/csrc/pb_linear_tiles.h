@@ -12,6 +12,8 @@ int pcb_linear_tiles_pair(const pcb_linear_args& a, const pcb_linear_args& b, in
 int64_t pcb_linear_waves_tiles(const pcb_linear_args& a);
 bool pcb_linear_waves_fits(const pcb_linear_args& a);
 int pcb_linear_waves(const pcb_linear_args& a, hipStream_t stream);
-// ... and those in fp32 of so many tiles that splitting their operands pays (pb_linear_split.hip)
+// ... and those in fp32 of so many tiles that splitting their operands may pay, with what such a launch takes (pb_linear_split.hip)
 bool pcb_linear_split_fits(const pcb_linear_args& a);
+float pcb_linear_split_us(const pcb_linear_args& a);
+int pcb_linear_split_shape(const pcb_linear_args& a);
 int pcb_linear_split(const pcb_linear_args& a, hipStream_t stream);

@@ -214,6 +214,7 @@ SIGNATURES = {
     "pcb_mix_norm": (C.c_int, [C.POINTER(MixNormArgs), _vp]),
     "pcb_embed_norm": (C.c_int, [_vp, _vp, _f32, _i32, C.POINTER(MixNormArgs), _vp]),
     "pcb_linear": (C.c_int, [C.POINTER(LinearArgs), _vp]),
+    "pcb_linear_parts_form": (C.c_int, [C.POINTER(LinearArgs)]),
     "pcb_norm_linear": (C.c_int, [C.POINTER(RowNormArgs), C.POINTER(LinearArgs), C.POINTER(LinearArgs), _vp]),
     "pcb_norm_linear_takes": (C.c_int, [C.POINTER(RowNormArgs), C.POINTER(LinearArgs), C.POINTER(LinearArgs)]),
     "pcb_linear_pair": (C.c_int, [C.POINTER(LinearArgs), C.POINTER(LinearArgs), _vp]),

@@ -456,7 +456,7 @@ def test_fp32_products_in_parts_and_what_is_no_number(M, N, K):
 
 
 @pytest.mark.parametrize("M,N", [(587, 1026), (587, 2562), (587, 5134)])
-@pytest.mark.parametrize("K", [4, 36, 520])
+@pytest.mark.parametrize("K", [4, 36, 520, 1052])
 @pytest.mark.parametrize("small,large", [(-112, 40), (-118, 60), (-118, 100), (-130, 40), (-130, 60), (-140, 120), (-148, 126), (-104, 100)])
 def test_fp32_products_of_the_smallest_and_the_largest_numbers(M, N, K, small, large):
     """Elements whose last bits lie below bf16's smallest number, subnormal ones among them, beside large ones: the error bound of fp32 sums, as for
@@ -492,6 +492,26 @@ def test_fp32_products_of_the_smallest_and_the_largest_numbers(M, N, K, small, l
         b.linear(x, w, y, M=M, epilogue=b.EPI_SILU_MUL, w2=w2, act=b.ACT_RELU)
         mt, mu = x.double().abs() @ w.double().abs().T.contiguous(), x.double().abs() @ w2.double().abs().T.contiguous()
         assert bool(((y.double() - torch.relu(t) * u).abs() <= bound * 2.1 * mt * mu + 2.0 ** -149).all())
+
+
+# each tile of the kernel that splits its operands, three k-steps and more, whole and ragged; and sizes on the other side of its line
+@pytest.mark.parametrize("gated,M,N,K", [(False, 587, 1540, 228), (False, 587, 2562, 92), (False, 587, 5134, 124), (True, 777, 5134, 92), (True, 587, 1540, 100),
+                                         (True, 587, 2562, 124), (False, 600, 1664, 256), (True, 48, 4672, 512),
+                                         (False, 32, 9280, 64)])
+def test_fp32_products_on_both_sides_of_the_line(gated, M, N, K):
+    """Against 64 bits, to what fp32 sums of K / 32 parts give (4 sqrt(K / 32 + 1) 2^-24 of the magnitudes; the gated unit: of two of them)."""
+    b = B()
+    x, w, w2 = (rnd(r, K, seed=i, scale=K ** -0.25) for i, r in ((1, M), (2, N), (3, N)))
+    bound = 4 * (K / 32 + 1) ** 0.5 * 2.0 ** -24
+    t, u = x.double() @ w.double().T.contiguous(), x.double() @ w2.double().T.contiguous()
+    mt, mu = x.double().abs() @ w.double().abs().T.contiguous(), x.double().abs() @ w2.double().abs().T.contiguous()
+    y = torch.full((M, N), float("nan"), device=DEV)
+    if gated:
+        b.linear(x, w, y, M=M, epilogue=b.EPI_SILU_MUL, w2=w2, act=b.ACT_RELU)
+        assert bool(((y.double() - torch.relu(t) * u).abs() <= bound * 2.1 * mt * mu).all())
+    else:
+        b.linear(x, w, y, M=M)
+        assert bool(((y.double() - t).abs() <= bound * mt).all())
 
 
 @pytest.mark.parametrize("M,N", [(1, 70), (9, 64), (16, 130), (40, 100), (130, 260), (600, 2564), (2000, 2040)])
