@@ -717,7 +717,7 @@ typedef struct pcb_attn_rows_args {
 int pcb_attn_rows(const pcb_attn_rows_args* a, void* stream);
 
 /* One decoding step of an attention layer behind its projection: pcb_head_prep of the step's rows, pcb_attn_rows (latent: pcb_attn_latent) over what is cached and
- * the new row itself; n_splits and part as there (n_splits > 1: a second launch merges).  Every row is the only one of its slot in the step.  tile r = {slot, position, 1, flat row} (int32 x 4, device).
+ * the new row itself; n_splits (less than one: one) and part, in whole 16 bytes, as there (n_splits > 1: a second launch merges).  Every row is the only one of its slot in the step.  tile r = {slot, position, 1, flat row} (int32 x 4, device).
  * p: projected rows, ldp apart; queries from column q_at on, q_head_stride apart: unit-RMS norm, q_gain, a turn of the first rot_dims columns (neighbouring pairs,
  * freqs float64 [rot_dims / 2], times rot_mag); keys from k_at on, k_cols apart, likewise with k_gain; values from v_at on: norm, kept in fp32 in keep (may be null) and
  * mixed with other's by blend[0] (may be null; as in pcb_head_prep_seg).  The new key and value go to k / v as in pcb_attn_rows_args.

@@ -429,10 +429,13 @@ PCB_EXPORT int pcb_attn_step(const pcb_attn_step_args* a, void* stream) {
     PCB_REQUIRE(!a->up || (a->latent && !a->sink && !a->gate && a->up_gate && a->up_dim > 0 && a->up_dim <= 128 && a->up_dim % 8 == 0 && a->part &&
                            (uintptr_t)a->up % 16 == 0 && a->ld_up_gate >= (int64_t)a->H * a->up_dim),
                 PCB_ERR_ARG, "pcb_attn_step: up-projections of a latent's heads, up to 128 columns in eights, with their gates and scratch");
-    PCB_REQUIRE(a->n_splits <= 1 || (a->part && (uintptr_t)a->part % 16 == 0 && a->n_splits <= 64), PCB_ERR_ARG, "pcb_attn_step: up to 64 runs, with their scratch");
+    PCB_REQUIRE((a->n_splits <= 1 && !a->up) || (a->part && (uintptr_t)a->part % 16 == 0 && a->n_splits <= 64), PCB_ERR_ARG,
+                "pcb_attn_step: up to 64 runs, with their scratch in whole 16 bytes");
     const int es = a->dtype == PCB_BF16 ? 2 : 4;
     const int64_t whole = a->k_slot_stride | a->k_head_stride | a->k_row_stride | a->v_slot_stride | a->v_head_stride | a->v_row_stride | a->ldo | (a->latent ? a->ldq : 0);
     PCB_REQUIRE(whole * es % 16 == 0 && ((uintptr_t)a->k | (uintptr_t)a->v | (uintptr_t)a->out | (uintptr_t)a->q) % 16 == 0, PCB_ERR_ARG,
                 "pcb_attn_step: cached rows and results begin at whole 16 bytes");
-    return a->dtype == PCB_BF16 ? dispatch<pcb::bf16_t>(*a, (hipStream_t)stream) : dispatch<float>(*a, (hipStream_t)stream);
+    pcb_attn_step_args q = *a;
+    if (q.n_splits < 1) q.n_splits = 1;                              // (both launches lay the runs out by it)
+    return q.dtype == PCB_BF16 ? dispatch<pcb::bf16_t>(q, (hipStream_t)stream) : dispatch<float>(q, (hipStream_t)stream);
 }

@@ -1054,7 +1054,8 @@ def attn_step(p: torch.Tensor, tiles: torch.Tensor, n_rows: int, k: torch.Tensor
     _want(part, torch.float32, "attn_step part")
     assert up is None or (up.dtype == p.dtype == up_gate.dtype and up.is_contiguous() and up.dim() == 3 and up.shape[0] == H and up.shape[2] == vdim and
                           _reach(up_gate) >= (n_rows - 1) * ld_up_gate + H * up.shape[1])
-    assert (n_splits <= 1 and up is None) or (part is not None and part.numel() >= attn_softmax_part(n_rows, H, n_splits, vdim))
+    n_splits = max(1, n_splits)
+    assert (n_splits == 1 and up is None) or (part is not None and part.numel() >= attn_softmax_part(n_rows, H, n_splits, vdim))
     a = AttnStepArgs(C.sizeof(AttnStepArgs), _code(p), _p(p), p.shape[-1], q_at, q_head_stride, k_at, dim, v_at, _p(q), q.shape[-1] if latent else 0, _p(tiles),
                      n_rows, _p(k), *(int(x) for x in k_strides), _p(v), *(int(x) for x in v_strides), H, Hkv, dim, vdim, int(latent), float(scale),
                      int(window), int(block), _p(sink), _p(gate), ldg, _p(out), out.shape[-1], _p(q_gain), _p(k_gain), float(eps), rot_dims, _p(freqs),

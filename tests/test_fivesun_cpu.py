@@ -462,3 +462,20 @@ def test_results_over_the_rows_of_a_norm_go_apart(monkeypatch):
     for over in (x, y, gate.view(torch.float32)):
         assert asked(product(P), x_out=over) == -2001
     assert asked(product(P), x_out=room[M * K:], streams=room) == -2001 and asked(product(P), x_out=room[2 * M * K:], streams=room) == 0
+
+
+@pytest.mark.parametrize("splits,up,off", [(1, True, 4), (0, True, 8), (2, False, 4), (65, False, 0), (65, True, 0), (1, True, None), (3, False, None)])
+def test_scratch_of_a_decoding_step_is_checked_wherever_it_is_used(splits, up, off):
+    """Whole 16 bytes, up to 64 runs; refused on the host (no device is needed)."""
+    from promptcache_amd import _blocks as B
+    room = torch.zeros(4096)
+    at = room.data_ptr() // 16 * 16 + 16
+    a = B.AttnStepArgs(ctypes.sizeof(B.AttnStepArgs), B.F32)
+    a.p = a.q = a.tiles = a.k = a.v = a.out = a.freqs = at
+    a.ldp, a.ldq, a.ldo, a.n_rows, a.H, a.Hkv, a.dim, a.vdim, a.latent, a.rot_dims = 256, 64, 64, 1, 1, 1, 48, 32, 1, 16
+    a.k_row_stride = a.v_row_stride = 48
+    a.n_splits, a.part = splits, None if off is None else at + off
+    if up:
+        a.up, a.up_dim, a.up_gate, a.ld_up_gate = at, 64, at, 64
+    assert B.load().pcb_attn_step_fits(B.F32, 1, 1, 48, 32, 16, 1)
+    assert B.load().pcb_attn_step(ctypes.byref(a), None) == -2001 and b"scratch" in B.load().pcb_last_error_string()

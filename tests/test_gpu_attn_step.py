@@ -152,3 +152,31 @@ def test_what_is_refused():
         with pytest.raises(RuntimeError, match=why):
             b.attn_step(P, tiles, 1, plane, (4 * row, 4 * row, row), plane.view(-1)[64:], (4 * row, 4 * row, row), 1, 1, dim, 64, 1.0, out, q_at=0, q_head_stride=64, k_at=64,
                         v_at=128, eps=1e-6)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("splits", [0, -3])
+def test_fewer_than_one_run_is_one(dtype, splits):
+    """With the up-projections in the merging launch: what the first launch leaves is found by the second."""
+    import ctypes
+    b, n, H, C, R, up = B(), 3, 4, 64, 16, 24
+    CR, HQ = C + R, H * (8 + R)
+    P, qa, w, gate = rnd(n, HQ + CR, seed=1, dtype=dtype), rnd(n, H * CR, seed=2, dtype=dtype), rnd(H, up, C, seed=3, dtype=dtype), rnd(n, H * up, seed=4, dtype=dtype)
+    plane, freqs = rnd(n, 40, CR, seed=5, dtype=dtype), torch.tensor([0.5 ** i for i in range(R // 2)], dtype=F64, device=DEV)
+    tiles = torch.tensor([[r, 13 * r + 2, 1, r] for r in range(n)], dtype=torch.int32, device=DEV).reshape(-1)
+    lib, got = b.load(), []
+    real = lib.pcb_attn_step
+    for s in (1, splits):
+        part, out = torch.full((b.attn_softmax_part(n, H, 1, C),), float("nan"), device=DEV), torch.zeros(n, H * up, dtype=dtype, device=DEV)
+
+        def call(args, stream):                                  # (the wrapper counts such runs as one itself)
+            args._obj.n_splits = s
+            return real(ctypes.byref(args._obj), stream)
+        try:
+            lib.pcb_attn_step = call
+            b.attn_step(P, tiles, n, plane, (40 * CR, 0, CR), plane, (40 * CR, 0, CR), H, 1, CR, C, 0.1, out, q_at=8, q_head_stride=8 + R, k_at=HQ, q=qa, eps=1e-6,
+                        rot_dims=R, freqs=freqs, part=part, up=w, up_gate=gate, ld_up_gate=H * up, n_splits=s)
+        finally:
+            lib.pcb_attn_step = real
+        got.append(out)
+    assert bool(torch.isfinite(got[0]).all()) and torch.equal(got[0], got[1])
