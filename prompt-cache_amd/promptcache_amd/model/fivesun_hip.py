@@ -381,7 +381,8 @@ class FivesunHIP(SlotModel):
         tb = self._tables(dblob, d)
         layers = self.layers if num_layers is None else self.layers[:num_layers]
         eps = self.config.norm_eps
-        x, spare = self._mat("x", T, W, f32), self._mat("x_next", T, W, f32)
+        few = T * W <= B.NORM_LINEAR_MAX          # the sizes at which a norm may ride in the launch of the products that read it
+        x, spare = self._mat("x", T, W, f32), self._mat("x_next", T, W, f32) if few else None
         h = self._mat("h", T, W, E)
         y1, y2 = self._mat("y1", T, W, f32), self._mat("y2", T, W, f32)
         streams = torch.empty((len(layers), T, W), dtype=f32, device=dev) if return_streams else None
@@ -396,9 +397,9 @@ class FivesunHIP(SlotModel):
             rows, pending = {}, {}
 
         def project(gain, a, b=None):
-            """The products ``a`` and, where given, ``b`` of the normed rows: for one or two rows the norm goes into their launch."""
+            """The products ``a`` and, where given, ``b`` of the normed rows: at few rows (up to eight of 512 columns, two of 2048) the norm goes into their launch."""
             nonlocal x, spare, rows, pending
-            if T * W <= B.NORM_LINEAR_MAX and (rows or pending):
+            if few and (rows or pending):
                 to = x if rows else spare
                 if B.norm_linear(a, b, gain, gain if b else None, to, eps=eps, **(rows or dict(x=x, **pending))):
                     x, spare = to, x if to is spare else spare
@@ -416,7 +417,7 @@ class FivesunHIP(SlotModel):
 
         # A layer without a feed-forward leaves its residual gate in its projected rows; where the norm that reads it rides in the next layer's projection, that
         # one stores elsewhere.
-        mix_in = ("mix_in", "mix_in_next" if T * W <= B.NORM_LINEAR_MAX else "mix_in")
+        mix_in = ("mix_in", "mix_in_next" if few else "mix_in")
         for i, lw in enumerate(layers):
             l = lw["cfg"]
             P = self._mat(mix_in[i % 2], T, lw["w_in"].shape[0], E)

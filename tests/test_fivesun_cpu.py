@@ -397,11 +397,21 @@ class _NoLaunch:
         return call
 
 
+def no_launches(monkeypatch):
+    """Steps on the host whose launches do nothing; -> what pcb_norm_linear is given, call by call."""
+    from promptcache_amd import _blocks as B
+    launches = {n for n, (_, args) in B.SIGNATURES.items() if args and args[-1] is ctypes.c_void_p}
+    seen = []
+    monkeypatch.setattr(B, "_lib", _NoLaunch(B.load(), launches, seen))
+    monkeypatch.setattr(B, "_stream", lambda: 0)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)               # (there is no device here: the tensors lie on the host)
+    return seen
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("rows", [1, 3])
 def test_a_norms_rows_lie_apart_from_what_its_launch_stores(monkeypatch, rows, dtype):
     """A layer without a feed-forward leaves its residual gate in its projected rows: the next layer's products, in whose launch the gate is read, store elsewhere."""
-    from promptcache_amd import _blocks as B
     from promptcache_amd.model.fivesun_hip import FivesunHIP
     att = dict(heads=4, kv_heads=2, dim=16, vdim=16, scale=0.25, mask=0, rot_base=100.0, rot_dims=16, rot_factor=1.0, v_mix=True)
     lat = dict(heads=2, kv_heads=1, dim=16, vdim=16, kv_rank=32, rot_dim=16, rot_dims=16, scale=0.2, mask=9, rot_base=50.0, rot_factor=1.0)
@@ -409,11 +419,7 @@ def test_a_norms_rows_lie_apart_from_what_its_launch_stores(monkeypatch, rows, d
     s = FivesunShape(vocab_size=60, hidden_size=512, norm_eps=1e-5, embed_scale=3.5, layers=[
         FivesunLayer("attention", **att), FivesunLayer("attention", **att), FivesunLayer("latent_attention", **lat), FivesunLayer("mlstm", **mem),
         FivesunLayer("attention", ff=64, **att), FivesunLayer("mlstm", **mem), FivesunLayer("mlstm", **mem), FivesunLayer("latent_attention", **lat)])
-    launches = {n for n, (_, args) in B.SIGNATURES.items() if args and args[-1] is ctypes.c_void_p}
-    seen = []
-    monkeypatch.setattr(B, "_lib", _NoLaunch(B.load(), launches, seen))
-    monkeypatch.setattr(B, "_stream", lambda: 0)
-    monkeypatch.setattr(torch.Tensor, "is_cuda", True)               # (there is no device here: the tensors lie on the host)
+    seen = no_launches(monkeypatch)
     m = FivesunHIP(s, W.make_fivesun_weights(s, seed=1), device="cpu", dtype=dtype)
     m.use_graphs = False
     ar = m.new_arena(rows, 8)
@@ -426,6 +432,22 @@ def test_a_norms_rows_lie_apart_from_what_its_launch_stores(monkeypatch, rows, d
         stored = [span(n.x_out, 512, 512, 4)] + [span(q.y, q.ldy, q.N, es) for q in (a, b) if q is not None]
         for lo, hi in read:
             assert all(hi <= at or end <= lo for at, end in stored)
+
+
+def test_rows_of_a_few_row_step_only_have_their_second_scratch(monkeypatch):
+    """What exists so that a norm may ride in a projection's launch is not allocated for steps in which it cannot."""
+    from promptcache_amd.model.fivesun_hip import FivesunHIP
+    no_launches(monkeypatch)
+    att = dict(heads=4, kv_heads=2, dim=16, vdim=16, scale=0.25, mask=0, rot_base=100.0, rot_dims=16, rot_factor=1.0)
+    s = FivesunShape(vocab_size=60, hidden_size=512, norm_eps=1e-5, embed_scale=3.5, layers=[FivesunLayer("attention", **att), FivesunLayer("attention", **att)])
+    m = FivesunHIP(s, W.make_fivesun_weights(s, seed=1), device="cpu")
+    m.use_graphs = False
+    ar = m.new_arena(1, 300)
+    slot = ar.alloc()
+    m.forward_rows(ar, [slot], [[5] * 200])
+    assert not {"x_next", "mix_in_next"} & set(m._buf)
+    m.forward_rows(ar, [slot], [[5]])
+    assert m._buf["x_next"].numel() == 1024 and m._buf["mix_in_next"].numel() < m._buf["mix_in"].numel()
 
 
 def test_results_over_the_rows_of_a_norm_go_apart(monkeypatch):
