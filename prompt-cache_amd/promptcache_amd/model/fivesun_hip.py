@@ -462,6 +462,13 @@ class FivesunHIP(SlotModel):
         unit = 32 if self.dtype == torch.float32 and n * groups * -(-reach // 32) <= 256 else 64
         return self._splits(n, groups, heads, reach, full, unit, merged)
 
+    def _latent_step(self, n, groups, reach, splits):
+        """Whether a step of ``n`` single tokens goes through ``B.attn_step`` over a latent: it saves a launch, but reads a row twice, as key and as value, where
+        ``B.attn_latent`` reads it once.  us, a layer's step, 16 heads over 192 + 64 columns, head_prep and attn_latent / attn_step: bf16 8 of 8 000 keys 59 / 45, 64 of
+        2 000 71 / 63, of 8 000 103 / 103, 192 of 2 000 94 / 91, 128 of 4 000 102 / 109, 256 of 4 000 170 / 177, 1 024 of 1 000 219 / 213; fp32 64 of 2 000 118 / 102, 128
+        of 4 000 217 / 226, of 8 000 334 / 385, 512 of 1 000 (one run) 255 / 218.  (Heads' own keys: faster at all of 1 .. 1 024 rows, 60 .. 30 000 keys.)"""
+        return n * groups * -(-reach // 64) <= 8000 or (splits == 1 and (self.dtype == torch.float32 or n * groups > 768))
+
     def _attention(self, arena, i, l, lw, P, y, tb, T, R):
         E = self.dtype
         H, G, D, Dv = l.heads, l.kv_heads, l.dim, l.vdim
@@ -524,12 +531,13 @@ class FivesunHIP(SlotModel):
         qa = self._mat("q_latent", T, H * CR, E) if n else None   # per head [W_uk^T q | rotated part]: a query over the cached rows
         reach = min(arena.cap, l.mask or arena.cap)
         full = 768 if CR <= 256 else 512
-        if tb["ones"] and n == T and B.attn_step_fits(E, H, 1, CR, C, Rd, True):
+        # the heads' up-projections and gates ride in the launch that merges: us a step of 16 heads, bf16, without / with it: one of 300 keys 212 / 206, 8 of 300
+        # 287 / 281, 32 of 100 360 / 356, 64 of 60 397 / 396; 8 heads, fp32, two of 300 189 / 183
+        up = T <= 64 and Dv <= 128 and Dv % 8 == 0
+        one = tb["ones"] and n == T and B.attn_step_fits(E, H, 1, CR, C, Rd, True)
+        splits = self._step_splits(T, -(-H // 16), H, reach, full, up) if one else 0
+        if one and self._latent_step(T, -(-H // 16), reach, splits):
             B.linear(P, lw["w_abs"], qa, M=T, n_batch=H, ldx=N, x_batch_stride=DR, ldy=H * CR, y_batch_stride=CR)
-            # the heads' up-projections and gates ride in the launch that merges: us a step of 16 heads, bf16, without / with it: one of 300 keys 212 / 206, 8 of 300
-            # 287 / 281, 32 of 100 360 / 356, 64 of 60 397 / 396; 8 heads, fp32, two of 300 189 / 183
-            up = T <= 64 and Dv <= 128 and Dv % 8 == 0
-            splits = self._step_splits(T, -(-H // 16), H, reach, full, up)
             strides, og, gate = (arena.slot_stride(i), 0, CR), self._mat("mix_gated", T, HV, E), P[:, HQ + CR:]
             kw = dict(q_at=D, q_head_stride=DR, k_at=HQ, q=qa, k_gain=lw["c_gain"], eps=self.config.norm_eps, rot_dims=Rd, freqs=lw["freqs"],
                       rot_mag=lw["rot_mag"], window=l.mask, n_splits=splits)

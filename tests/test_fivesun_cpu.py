@@ -384,13 +384,14 @@ class _NoLaunch:
     """The blocks library with every call that would launch answered with "done"; what pcb_norm_linear is given is kept."""
 
     def __init__(self, lib, launches, seen):
-        self.lib, self.launches, self.seen = lib, launches, seen
+        self.lib, self.launches, self.seen, self.names = lib, launches, seen, []
 
     def __getattr__(self, name):
         if name not in self.launches:
             return getattr(self.lib, name)
 
         def call(*args):
+            self.names.append(name)
             if name == "pcb_norm_linear":
                 self.seen.append([None if a is None else type(a._obj).from_buffer_copy(a._obj) for a in args[:3]])
             return 0
@@ -448,6 +449,27 @@ def test_rows_of_a_few_row_step_only_have_their_second_scratch(monkeypatch):
     assert not {"x_next", "mix_in_next"} & set(m._buf)
     m.forward_rows(ar, [slot], [[5]])
     assert m._buf["x_next"].numel() == 1024 and m._buf["mix_in_next"].numel() < m._buf["mix_in"].numel()
+
+
+@pytest.mark.parametrize("dtype,rows,reach,step", [
+    (torch.bfloat16, 1, 60000, True), (torch.bfloat16, 8, 60000, True), (torch.bfloat16, 64, 8000, True), (torch.bfloat16, 64, 8100, False), (torch.bfloat16, 128, 4000, False),
+    (torch.bfloat16, 192, 2000, True), (torch.bfloat16, 512, 2000, False), (torch.bfloat16, 1024, 1000, True), (torch.float32, 128, 4000, False),
+    (torch.float32, 128, 8000, False), (torch.float32, 512, 1000, True), (torch.float32, 64, 2000, True)])
+def test_steps_over_latents_take_one_launch_where_that_is_the_faster(monkeypatch, dtype, rows, reach, step):
+    """The rule by rows and reach, and the launches of a step on either side of it."""
+    from promptcache_amd import _blocks as B
+    from promptcache_amd.model.fivesun_hip import FivesunHIP
+    lat = dict(heads=2, kv_heads=1, dim=16, vdim=16, kv_rank=32, rot_dim=16, rot_dims=16, scale=0.2, mask=0, rot_base=50.0, rot_factor=1.0)
+    s = FivesunShape(vocab_size=60, hidden_size=64, norm_eps=1e-5, layers=[FivesunLayer("latent_attention", **lat)])
+    no_launches(monkeypatch)
+    m = FivesunHIP(s, W.make_fivesun_weights(s, seed=1), device="cpu", dtype=dtype)
+    m.use_graphs = False
+    splits = m._step_splits(rows, 1, 16, reach, 768, rows <= 64)
+    assert m._latent_step(rows, 1, reach, splits) == step
+    m._latent_step = lambda *a: step
+    ar = m.new_arena(2, 8)
+    m.forward_rows(ar, [ar.alloc(), ar.alloc()], [[5], [6]])
+    assert ("pcb_attn_step" in B._lib.names) == step and ("pcb_attn_latent" in B._lib.names) != step
 
 
 def test_results_over_the_rows_of_a_norm_go_apart(monkeypatch):
