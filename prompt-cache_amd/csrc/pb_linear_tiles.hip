@@ -395,7 +395,7 @@ int launch(const pcb_linear_args& a, const pcb_linear_args* b, hipStream_t strea
 // 2048 rows, K = 2048, 128 x 128 / 128 x 256 / 256 x 256 and what the rule took: N = 2048 20.0 / 28.0 / 42.7 -> 20.0, 8192 84 / 75 / 67 -> 66;
 // 6000 rows, K = 512, N = 2048 21.2 / 24.9 / 22.3 -> 21.9.  Without and with the two of 192 columns: 2048 rows, N = 2560 31.7 / 29.9, 5136 55.3 / 49.7,
 // 10272 106 / 102; 1500 x 3072 31.3 / 25.4; 4096 x 2560 52.0 / 45.4; 2400 x 2048, K = 8192 102 / 91.  (The gated unit's halves are whole pairs of
-// 32-column blocks: not 192.)
+// 32-column blocks: not 192.)  With the present loop at 330 sizes on average 0.8 % from the fastest shape, 8 of them by more than 10 % (by grid_us() below 1.2 %, 11).
 enum Shape { SQUARE, WIDE192, WIDE, TALL192, TALL };
 int choose(const pcb_linear_args& a, const pcb_linear_args* b) {
     const bool gated = (b ? b : &a)->epilogue == PCB_EPI_SILU_MUL;
@@ -444,11 +444,9 @@ int pcb_linear_tiles(const pcb_linear_args& a, hipStream_t stream) {
     }
 }
 
-// Two products in one grid fill the rounds that each leaves part empty.  What a grid takes, us: whole rounds, half a round for a part of one and the rest of it
-// in proportion (a full chip runs at a lower clock), and the activations behind the last products, 0.056 a number and thread: one grid where that is the
-// lesser, by 3 %, than the two products' (gated units beyond 128 rows only).  Over 138 sizes of 65 .. 4800 rows 0.1 % behind the better of the two, two of
-// them by 11 and 13 %.  Apart / in one, us, 2560 and 8192 fp32 columns, K = 2048: 255 rows 38.1 / 25.1, 377 40.1 / 25.4, 679 52.4 / 35.0, 1484 77.8 / 57.7, 2195 120 / 103; 2048
-// with a sigmoid and a gated 4096: 142 rows 32.3 / 24.7, 558 50.9 / 40.1, 2195 124 / 106 (1805 83 / 102: apart); 640 and 2048, K = 512: 310 rows 12.0 / 9.0.
+// What a grid of one or two products takes, us (choose() above ranks shapes by whole rounds of a full chip; this is for comparing grids that fill it differently, and
+// the kernels of smaller tiles): whole rounds, half a round's products for a part of one and the rest of it in proportion (a full chip runs at a lower clock), and
+// the activations behind the last products, 0.056 a number and thread.
 static float grid_us(const pcb_linear_args& a, const pcb_linear_args* b, int shape) {
     static constexpr struct { int bm, bn; float base, step; } T[] = {
         {128, 128, 4.8f, 0.57f}, {128, 192, 7.0f, 0.77f}, {128, 256, 11.0f, 0.88f}, {256, 192, 10.0f, 1.3f}, {256, 256, 12.7f, 1.5f}};
@@ -456,10 +454,29 @@ static float grid_us(const pcb_linear_args& a, const pcb_linear_args* b, int sha
     auto blocks = [&](const pcb_linear_args& q) { return (int64_t)pcb_ceil_div(q.epilogue == PCB_EPI_SILU_MUL ? 2 * q.N : q.N, t.bn); };
     auto acts = [&](const pcb_linear_args& q) { return q.epilogue == PCB_EPI_SILU_MUL ? 0.5f : (q.act | q.act2) ? 1.0f : 0.0f; };
     const int64_t tiles = pcb_ceil_div(a.M, t.bm) * (blocks(a) + (b ? blocks(*b) : 0)), rest = tiles % 256;
-    const float round = t.base + t.step * (float)pcb_ceil_div(a.K, 64), act = b && acts(*b) > acts(a) ? acts(*b) : acts(a);
-    return round * ((float)(tiles / 256) + (rest ? 0.5f + (float)rest / 512.0f : 0.0f)) + 0.056f * act * (float)(t.bm * t.bn / 256);
+    const float steps = t.step * (float)pcb_ceil_div(a.K, 64), act = b && acts(*b) > acts(a) ? acts(*b) : acts(a);
+    const float whole = (float)(tiles / 256), part = rest ? 0.5f + (float)rest / 512.0f : 0.0f;
+    return steps * (whole + part) + t.base * (whole > 0.0f ? whole + part : 1.0f) + 0.056f * act * (float)(t.bm * t.bn / 256);
 }
 
+// ... and a product by itself, through the kernel that pb_linear has for it: waves, these tiles, or tiles of 64 x 64
+static float alone_us(const pcb_linear_args& q) {
+    const float steps = (float)pcb_ceil_div(q.K, 64);
+    const int cols = q.epilogue == PCB_EPI_SILU_MUL ? 2 * q.N : q.N;
+    if (pcb_linear_waves_fits(q)) {
+        const int64_t wgs = pcb_linear_waves_tiles(q);
+        return wgs <= 256 ? 3.5f + (float)wgs / 230.0f + 0.087f * steps : 4.6f + 0.19f * steps;
+    }
+    if ((int64_t)pcb_ceil_div(q.M, 128) * pcb_ceil_div(cols, 128) > 128) return grid_us(q, nullptr, choose(q, nullptr));
+    return (int64_t)pcb_ceil_div(q.M, 64) * pcb_ceil_div(cols, 64) <= 256 ? 4.2f + 0.33f * steps : 4.8f + 0.42f * steps;
+}
+
+// Two products in one grid fill the rounds that each leaves part empty: one grid where that takes 5 % less by these estimates than the two by themselves (gated units
+// beyond 128 rows only; their code is longer, 1.5).  Of 600 sizes that go out in one so -- 65 .. 4800 rows, 64 .. 12000 columns, K = 64 .. 8192 -- two are slower for it,
+// by 8 and 23 %, on average they take 0.79 of the time.  (Judged by this grid's times alone, without the kernels of smaller tiles, 153 of 1160 lost more than 2 %, up
+// to 1.6: 76 rows, K = 8192, 240 and 152 columns 27.3 / 43.9.)
+// Apart / in one, us, 2560 and 8192 fp32 columns, K = 2048: 255 rows 38.1 / 25.1, 377 40.1 / 25.4, 679 52.4 / 35.0, 1484 77.8 / 57.7, 2195 120 / 103; 2048
+// with a sigmoid and a gated 4096: 142 rows 32.3 / 24.7, 558 50.9 / 40.1, 2195 124 / 106 (1805 83 / 102: apart); 640 and 2048, K = 512: 310 rows 12.0 / 9.0.
 int pcb_linear_tiles_pair_shape(const pcb_linear_args& a, const pcb_linear_args& b) {
     auto fits = [](const pcb_linear_args& q) {
         return q.dtype == PCB_BF16 && q.M > 64 && q.n_groups == 0 && q.n_batch == 0 && !q.row_src && q.ldx < (1 << 22) && q.ldw < (1 << 22) && pcb_linear_pieces(q);
@@ -467,7 +484,7 @@ int pcb_linear_tiles_pair_shape(const pcb_linear_args& a, const pcb_linear_args&
     const bool gated = b.epilogue == PCB_EPI_SILU_MUL;
     if (!fits(a) || !fits(b) || a.M != b.M || a.K != b.K || a.epilogue != PCB_EPI_STORE || b.epilogue == PCB_EPI_SCALE_ADD || (gated && a.M <= 128)) return -1;
     const int shape = choose(a, &b);
-    return grid_us(a, &b, shape) < 0.97f * (grid_us(a, nullptr, choose(a, nullptr)) + grid_us(b, nullptr, choose(b, nullptr))) ? shape : -1;
+    return grid_us(a, &b, shape) + (gated ? 1.5f : 0.0f) < 0.95f * (alone_us(a) + alone_us(b)) ? shape : -1;
 }
 
 int pcb_linear_tiles_pair(const pcb_linear_args& a, const pcb_linear_args& b, int shape, hipStream_t stream) {

@@ -65,3 +65,14 @@ def test_a_row_that_is_no_number_stays_alone(bad):
     rows = [r for r in range(M) if r != 17]
     assert bool(torch.isfinite(y1[rows].float()).all()) and bool(torch.isfinite(y2[rows]).all())
     assert not bool(torch.isfinite(y1[17].float()).any()) and not bool(torch.isfinite(y2[17]).any())
+
+
+# what every tile shape of either epilogue takes: (rows, k, columns, of the second product, gated, pcb_linear_pair_form)
+SHAPES = [(111, 96, 91, 66, False, 2), (389, 160, 3884, 4276, False, 3), (654, 160, 1945, 5955, False, 4), (786, 96, 3085, 5896, False, 5),
+          (1032, 96, 3892, 5886, False, 6), (138, 352, 221, 222, True, 2), (290, 352, 3921, 5514, True, 4), (902, 352, 3501, 4123, True, 6)]
+
+
+@pytest.mark.parametrize("M,K,N1,N2,gated,form", SHAPES)
+def test_pairs_of_every_tile_shape(M, K, N1, N2, gated, form):
+    """(That these sizes reach the shapes: test_linear_pair_cpu.py.)"""
+    test_pairs(gated, M, K, N1, N2)
