@@ -190,15 +190,16 @@ __global__ __launch_bounds__(512) void norm_linear_kernel(pcb_row_norm_args n, p
         normed_block<E, EPI, PARTS, U, NC, KIND>(n, n.gain2, b, blockIdx.x - na, false, rows, part, red);
 }
 
-int row_bits(int M) { return M <= 1 ? 0 : M <= 2 ? 1 : M <= 4 ? 2 : 3; }
-
 // Which form takes a launch, and whether one launch is the better one.  us against the launches it stands for, weights from memory, by workgroups.
 // Runs of k: bf16 one up to K = 1024, two beyond (1 row, K = 1024, 2592 columns behind a sublayer -1.8 / -1.2, 10272 -0.7 / +0.5); fp32 one up to K = 512, then two
 // while that is no more than three workgroups a CU, of more than 2048 elements 192 (1 row, K = 1024, the streams' sum, 5376 columns one run +0.8, two -0.6, 10752
 // -0.8 / 0.0; 4 rows 2688 columns -1.2 / -0.1, 1312 behind a sublayer -0.7 / -1.6).
-// Taken up to `most` workgroups, each of which works out the rows again: one chunk a thread, plain 96 .. 384 -0.2 .. -2.2, 672 -0.4 .. -1.6, 1280 -1.2 .. +2.4, 2560
-// +1.4 .. +6.8; gated 768 -1.6 .. -4.4, 1280 -0.7 .. -5.8, 2560 -5.1 .. +3.8; from a table (two launches less) 336 .. 672 -1.5 .. -4.4; two chunks, plain 168 -1.0
-// .. -1.7, 336 -0.7 .. +1.4, 672 -0.3 .. +2.7; gated 384 -1.1 .. -2.0, 640 -3.3 .. +0.1; from a table 336 -1.6 .. -4.1.
+// Taken up to `most` workgroups, each of which works out the rows again -- the more streams they are the sum of, the fewer.  us, launches apart / here, medians of 2060
+// sizes (1 .. 8 rows, K = 64 .. 2048, 16 .. 12000 columns): one chunk a thread, a table up to 640 workgroups -0.3 .. -1.5; behind a sublayer, plain -1.0 .. -2.2, gated to
+// 1280 -0.4 .. -5; two streams to 768 -0.1 .. -1.3; four bf16 to 512 -0.5 .. -1.3, 768 -0.1, fp32 256 -0.8, 512 +0.2; eight 256 -0.6 / -1.0, 512 +0.3 / +0.5, 768 +1.1 /
+// +2.7; twelve bf16 256 -0.7, 640 +1.3, fp32 256 -0.4, 640 +2.6; 24 0.0 .. +5.6.  Two chunks: behind a sublayer -0.7 .. -1.9, four streams 256 -0.3 .. -1.3, eight bf16 192 -0.2,
+// fp32 +0.0 .. +0.7, twelve 0.0 .. +0.9.  fp32 beyond K = 1024: more than two streams +0.3 .. +0.8.  Next to no k: 128 x 7200, 450 workgroups, two streams +0.8.  Slower
+// than apart by more than 2 % at 61 of the 1418 that are taken (by the workgroups alone, whatever the rows are the sum of, at 403 of 2060, by up to 1.9).
 struct Form {
     int parts, chunks;
     bool taken;
@@ -210,7 +211,20 @@ Form form(const pcb_row_norm_args& n, const pcb_linear_args& a, const pcb_linear
     const bool table = n.table, gated = b && b->epilogue == PCB_EPI_SILU_MUL;
     auto groups = [&](int parts) { return (int64_t)pcb_ceil_div(a.N, 16 / parts) + (b ? pcb_ceil_div(b->N, 16 / parts) : 0); };
     if (a.K > 1024 || (a.dtype == PCB_F32 && a.K > 512 && groups(2) <= (f.chunks == 1 ? 768 : 192))) f.parts = 2;
-    const int most = f.chunks == 1 ? (gated || table ? 1280 : 768) : table ? 512 : gated ? 384 : 256;
+    const bool bf = a.dtype == PCB_BF16, one = f.chunks == 1;
+    const int terms = n.n_terms, few = terms <= 12 ? 16 : 0;
+    int most;
+    if (table)
+        most = one ? 768 : bf ? 384 : 256;
+    else if (n.y)
+        most = one ? (gated ? 1280 : 768) : gated ? 384 : 256;
+    else if (!bf && a.K > 1024 && terms > 2)
+        most = few;
+    else if (one)
+        most = terms <= 2 ? 768 : terms <= 4 ? (bf ? 512 : 256) : terms <= 8 || (bf && terms <= 12) ? 256 : few;
+    else
+        most = terms <= 4 ? 256 : bf && terms <= 8 ? 192 : few;
+    if (a.K < 256 && most > (gated ? 768 : 320)) most = gated ? 768 : 320;
     f.taken = groups(f.parts) <= most;
     return f;
 }
