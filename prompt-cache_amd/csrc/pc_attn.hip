@@ -1381,8 +1381,10 @@ PC_EXPORT int64_t pc_attn_workspace_bytes(int32_t B, int32_t H, int32_t D, int32
     int ns = ns_a > ns_b ? ns_a : ns_b;
     // passes of <= kTailMax rows may run in tail mode (pc_attn_fwd_ex with lo_row0 = -1): one more split, always merged
     if (q_len <= kTailMax) {
-        const int nt = tail_stream_splits(B, H, kv_len_max);
+        // (its streams cover the keys in front of the pass, and a tile less of them may take more streams: 15 tiles 15, 16 tiles 8)
+        const int nt = tail_stream_splits(B, H, kv_len_max), np = tail_stream_splits(B, H, kv_len_max - q_len);
         ns = ns > nt ? ns : nt;
+        ns = ns > np ? ns : np;
         ns = (ns < kMaxSplit ? ns : kMaxSplit - 1) + 1;
     }
     // passes of <= 16 rows may take attn_small_kernel: one partial per workgroup (+ the tail's)

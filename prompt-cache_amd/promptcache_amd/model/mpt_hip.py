@@ -39,7 +39,8 @@ class MptHIP(LlamaHIP):
     _shared_prefix_loop = False     # (its many-row loop keeps a copy of the trunk per batch row)
     supports_fused_gather = False   # (its layer loops read staged rows from the arena ...)
     # ... and the copy goes out at the beginning of the first forward (_resolve_arena): behind it the host prepares the step, where an update() that copies at
-    # once, and is timed by events, waits for it.  A question behind 936 staged tokens, 8 layers of 7b: 1 226 us -> 1 103.
+    # once, and is timed by events, waits for it and for all that is under way.  A question behind 936 staged tokens, 8 layers of 7b, us: one after the other
+    # 1 211 -> 1 086, each waited for by itself 1 220 -> 1 197 (new text or the same; one of a length not asked before captures its graph first, 3.6 ms).
     defers_staging = True
 
     def __init__(self, shape: MptShape, weights: Dict[str, torch.Tensor], device="cuda:0", decode_headroom: int = 256,

@@ -407,6 +407,39 @@ def test_attn_17_to_32_rows_over_a_long_cache_matches_the_oracle(B, H, Hkv, D, q
     np.testing.assert_allclose(got, ref, atol=2e-5, rtol=2e-4)
 
 
+@pytest.mark.parametrize("B,H,q_len,past,alibi", [(1, 32, 25, 936, True), (1, 32, 32, 960, True), (1, 32, 17, 1919, True), (1, 64, 20, 440, True), (2, 64, 20, 180, False),
+                                                   (1, 128, 31, 185, False)])
+def test_attn_workspace_holds_a_question_that_ends_in_a_tile_of_its_own(B, H, q_len, past, alibi):
+    """Tail mode in the 64-row kernel where the pass's last key lies in a further key tile than the last staged one: what pc_attn_workspace_bytes asks for is
+    enough (fewer streams may cover a tile more).  Against 64 bits as above."""
+    n = _n()
+    D, cap = 128, past + q_len + 3
+    g = torch.Generator().manual_seed(past)
+    q32, k, v = torch.randn(B, q_len, H, D, generator=g), torch.randn(B, H, cap, D, generator=g).half(), torch.randn(B, H, cap, D, generator=g).half()
+    q = q32.half()
+    ql = (q32 - q.float()).half()
+    klo, vlo = (1e-4 * torch.randn(B, H, q_len, D, generator=g)).half(), (1e-4 * torch.randn(B, H, q_len, D, generator=g)).half()
+    dev = [t.to(DEV) for t in (q, ql, k, v, klo, vlo)]
+    slopes = torch.exp2(-8.0 * torch.arange(1, H + 1) / H)
+    kpos = torch.zeros(B, (cap + 63) // 64 * 64 + 64)                # (whole tiles of columns)
+    kpos[:, :past + q_len] = torch.arange(past + q_len) - (past + q_len - 1.0)
+    ws = torch.full((max(n.attn_workspace_bytes(B, H, D, q_len, past + q_len), 4) // 4,), float("nan"), dtype=torch.float32, device=DEV)
+    oh = torch.full((B, q_len, H * D), float("nan"), dtype=torch.float16, device=DEV)
+    ol = torch.full_like(oh, float("nan"))
+    n.attn_fwd(dev[0], q_len * H * D, H * D, dev[2], dev[3], H * cap * D, cap * D, oh, q_len * H * D, H * D, B, H, H, D, q_len, past, D ** -0.5, ws, q_lo=dev[1],
+               out_lo=ol, kv_lo=(dev[4], dev[5], H * q_len * D, q_len * D, -1),
+               alibi=(kpos.to(DEV), (slopes * 1.4426950408889634).to(DEV)) if alibi else None)
+    kf, vf = k.double()[:, :, :past + q_len].clone(), v.double()[:, :, :past + q_len].clone()
+    kf[:, :, past:] += klo.double()
+    vf[:, :, past:] += vlo.double()
+    s = (q.double() + ql.double()).transpose(1, 2) @ kf.transpose(2, 3) * D ** -0.5
+    if alibi:
+        s = s + slopes.double()[None, :, None, None] * kpos.double()[:, None, None, :past + q_len]
+    s = s.masked_fill(torch.arange(past + q_len)[None, :] > past + torch.arange(q_len)[:, None], float("-inf"))
+    want = (torch.softmax(s, -1) @ vf).transpose(1, 2).reshape(B, q_len, H * D)
+    np.testing.assert_allclose((oh.float() + ol.float()).cpu().numpy(), want.numpy(), atol=2e-5, rtol=2e-4)
+
+
 def test_attn_softmax_rescale_with_key_spike():
     """Force the running max to jump late in the KV stream (online-softmax rescale path) and early
     (later tiles contribute ~0): a spike row in K aligned with one query."""
