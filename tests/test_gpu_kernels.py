@@ -642,6 +642,28 @@ def test_norm_frag_threads_per_column(rows, hidden, nslabs):
         assert float(((got - ref).abs() / (1 + ref.abs())).max()) < 2 ** -20 + 2 ** -21
 
 
+@pytest.mark.parametrize("nslabs", [1, 2, 5, 8, 9])
+@pytest.mark.parametrize("hidden", [2080, 3072, 4096, 4544, 5120, 6656, 8192])
+@pytest.mark.parametrize("ln", [False, True])
+def test_norm_frag_forms_give_the_same_bits(hidden, nslabs, ln):
+    """A row's planes and residual are the same bits in a launch of 160 rows (a thread per eight columns) and in one of 161 (256 threads a row)."""
+    n = _n()
+    g = torch.Generator(device=DEV).manual_seed(hidden + nslabs)
+    x, sl = 3 * torch.randn(161, hidden, generator=g, device=DEV), torch.randn(nslabs, 161, hidden, generator=g, device=DEV)
+    w, b = (1 + 0.1 * torch.randn(hidden, generator=g, device=DEV)).half(), (0.1 * torch.randn(hidden, generator=g, device=DEV)).half()
+    got = []
+    for rows in (160, 161):
+        hi = torch.zeros(((rows + 15) // 16, hidden // 32, 64, 8), dtype=torch.float16, device=DEV)
+        lo, xr = torch.zeros_like(hi), x[:rows].clone()
+        if ln:
+            n.layernorm_frag(xr, w, b, hi, lo, rows, hidden, 1e-5, sl[:, :rows].contiguous(), nslabs)
+        else:
+            n.rmsnorm_frag(xr, w, hi, lo, rows, hidden, 1e-5, sl[:, :rows].contiguous(), nslabs)
+        got.append((xr[:160], n.from_act_frags(hi, rows)[:160], n.from_act_frags(lo, rows)[:160]))
+    for one, other in zip(*got):
+        assert bool(torch.isfinite(one.float()).all()) and torch.equal(one, other)
+
+
 @pytest.mark.parametrize("M,N,K,kq", [(12, 4096, 4096, 4), (12, 4096, 11008, 4), (3, 64, 96, 2), (20, 512, 1376, 3),
                                       (40, 4096, 4096, 4), (64, 4096, 11008, 4), (30, 5120, 13824, 4)])
 def test_gemm_skinny_k_slices(M, N, K, kq):
