@@ -12,7 +12,9 @@
 // to 1.6 GHz; with zeros as operands 256 of them run at 2.2.  MFMAs alone on random operands in registers, 256 CUs: 1.61 PFLOP/s in 32 x 32 x 16, 1.69 in
 // 16 x 16 x 32, and so it is here, 32 x 32 / 16 x 16, us: two planes, 1737 x 12288, K = 4096 306 / 297, 3584 x 4096, K = 11008 530 / 517, 3584 x 12288 599 / 575; one
 // plane, 2048 rows, K = 2048, 128 x 192 tiles 27.1 / 25.9, 128 x 256 34.4 / 33.1, 256 x 256 over 4096 x 4096 x 4096 103.9 / 101.7.  128 x 128 tiles of one plane are not
-// as close to that limit and take 22.4 us for 21.4, 38.4 for 36.2 (2048 x 2048, K = 2048, 4096): 32 x 32.
+// as close to that limit and take 22.4 us for 21.4, 38.4 for 36.2 (2048 x 2048, K = 2048, 4096): 32 x 32.  Nor is anything else where few CUs have a tile: two planes,
+// 70 x 640, K = 5120 (5 tiles) 46.1 / 51.5, 102 x 2560, K = 1024 (20) 14.0 / 15.1, from 64 tiles on equal, 256 and more 0.96 .. 0.99; one plane, 256 x 256 tiles on 192 CUs
+// (1500 x 8192, K = 2048) 47.5 / 48.8, on all 0.95 .. 0.98 (2048 x 8192, K = 8192 194 / 187); over K <= 256 1 .. 3 % more.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -73,9 +75,9 @@ struct Loop {
                     for (int e = 0; e < per; ++e)
                         if (per * (k / gap) + e < R) read_one(buf, un, per * (k / gap) + e);
                 // (no loop here: with one, the unrolled whole passes what the compiler unrolls)
-                constexpr int len = SOON ? 2 * (d1 - d0) : MF;
-                const int n = d0 + k * (d1 - d0) / (len > 0 ? len : 1);
-                if (k < len && n < d0 + (k + 1) * (d1 - d0) / len) stage(n, t, to);
+                constexpr int len = SOON ? 2 * (d1 - d0) : MF, over = len > 0 ? len : 1;
+                const int n = d0 + k * (d1 - d0) / over;
+                if (k < len && n < d0 + (k + 1) * (d1 - d0) / over) stage(n, t, to);
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
