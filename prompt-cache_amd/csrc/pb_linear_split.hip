@@ -66,11 +66,10 @@ __global__ __launch_bounds__(128 * WN) void linear_split_kernel(pcb_linear_args 
     float top[NC];                                                   // the largest magnitude of each chunk's elements so far
 #pragma unroll
     for (int i = 0; i < NC; ++i) top[i] = 0.0f;
+    auto peak = [&](const f4& r, int i, int h) {                     // half h of a chunk (a NaN is passed over: its sums are no numbers either)
+        asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(top[i]) : "v"(r[2 * h]), "v"(r[2 * h + 1]));
+    };
     auto store = [&](f4& r, int i, int q, int buf) {
-        if (q == 0) {                                                // (a NaN is passed over: its sums are no numbers either)
-            asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(top[i]) : "v"(r[0]), "v"(r[1]));
-            asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(top[i]) : "v"(r[2]), "v"(r[3]));
-        }
         const uint2 p = {bf16_pair(r[0], r[1]), bf16_pair(r[2], r[3])};
         if (q < 2) {
             r[0] -= __uint_as_float(p.x << 16);
@@ -99,7 +98,11 @@ __global__ __launch_bounds__(128 * WN) void linear_split_kernel(pcb_linear_args 
         }
     };
     // product k of the six of every pair of blocks: the small ones of a kind one after the other, so that no two neighbours add to the same sum
-    constexpr int MF = 6 * TM * NB;
+    constexpr int MF = 6 * TM * NB, FROM = MF - 2 * NC;
+    // Where a chunk's largest magnitude is taken: behind the last products, one instruction each, ahead of the chunk's split where there are few products.  us, behind /
+    // ahead, K = 4096: 128 x 128 tiles 167 / 172 (without 167), 64 x 128 107.5 / 109 (102.5), 64 x 64 71.2 / 70.0 (68.3); ahead of the products, while their
+    // operands come from LDS, 169.7, 107.5, 73.4.
+    constexpr bool BEHIND = MF >= 24;
     auto product = [&](int k) {
         const int kind = k / (TM * NB), j = k / TM % NB, i = k % TM;
         const int w = kind == 0 ? 2 : kind == 3 || kind == 4 ? 1 : 0, x = kind == 1 ? 2 : kind == 3 || kind == 5 ? 1 : 0;
@@ -113,11 +116,18 @@ __global__ __launch_bounds__(128 * WN) void linear_split_kernel(pcb_linear_args 
         meet();
         read(P);
         auto unit = [&](int u) {
+            if (!BEHIND && u % 3 == 0) peak(raw[1 - P][u / 3], u / 3, 0), peak(raw[1 - P][u / 3], u / 3, 1);
             store(raw[1 - P][u / 3], u / 3, u % 3, 1 - P);
             if (u % 3 == 2) load(raw[1 - P][u / 3], u / 3, s + 3 < steps ? s + 3 : steps - 1);
         };
 #pragma unroll
-        for (int k = 0; k < MF; ++k) product(k);
+        for (int k = 0; k < MF; ++k) {
+            product(k);
+            if (BEHIND && k >= FROM) {
+                __builtin_amdgcn_sched_barrier(0);
+                peak(raw[1 - P][(k - FROM) / 2], (k - FROM) / 2, (k - FROM) & 1);
+            }
+        }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < 3 * NC; ++u) unit(u);
@@ -129,6 +139,7 @@ __global__ __launch_bounds__(128 * WN) void linear_split_kernel(pcb_linear_args 
     }
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
+        for (int h = 0; h < 2; ++h) peak(raw[0][i], i, h);
 #pragma unroll
         for (int q = 0; q < 3; ++q) store(raw[0][i], i, q, 0);
         load(raw[0][i], i, steps > 2 ? 2 : steps - 1);
@@ -154,8 +165,8 @@ __global__ __launch_bounds__(128 * WN) void linear_split_kernel(pcb_linear_args 
     // What is no number here may have a sum: the parts of an infinity (or of a value that rounds to one) make NaN.  And what the parts of a sum's elements leave out,
     // 2^-134 of each at most, is K 2^-133 times the largest element of its row and column: results below 2^26 times that would show it (rows of zeros aside).  A wave
     // that has such a result works its blocks out on the fp32 matrix cores and takes it from there: a result depends on its own row and column alone.
-    // What that costs, us: nothing but NaN 600 x 5136, K = 1024 134, 2048 x 2048 x 2048 257 (numbers: 54, 96; fp32 matrix cores from the start 78, 147).  The maxima: 2048
-    // columns and K, 2048 rows 94.1 / 95.6, 600 x 2560, K = 1024 29.9 / 31.1, 600 x 5136 48.1 / 48.2.
+    // What that costs, us: nothing but NaN 600 x 5136, K = 1024 134, 2048 x 2048 x 2048 257 (numbers: 54, 96; fp32 matrix cores from the start 78, 147).  Without and with
+    // the maxima and this look: 2048 columns and K, 2048 rows 95.8 / 96.7, 600 x 2560, K = 1024 29.9 / 31.0, 600 x 5136 48.0 / 47.5, 400 x 2048 20.0 / 20.8.
     __shared__ __attribute__((aligned(16))) float tops[ROWS];
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
@@ -296,8 +307,8 @@ int dispatch(const pcb_linear_args& a, hipStream_t stream) {
 // From 145 tiles of 64 x 64 on (128 of them 0.70 .. 0.90 of the fp32 matrix cores' speed: tiles of 32 x 32 there, on all CUs), where the launch takes less by this
 // estimate than by fp32_us() (pb_linear.hip): fitted to 2080 sizes of 17 .. 2048 rows, 145 .. 2048 such tiles, K = 256 .. 2048, plain and gated.  Slower than the fp32 matrix
 // cores by more than 4 % at five of them (splitting whatever has 145 tiles: at 468, by up to half: 32 rows of 65920 columns, K = 1024 57.4 / 84.5, 600 x 1664 -- two
-// rounds of the chip -- 26.7 / 32.3), on average 0.2 % behind the better of the two.  600 x 5136, K = 1024 78 -> 48.2 us, the gated pair of 2048 60 -> 46.3,
-// 2048 x 2048 x 2048 147 -> 95.6.
+// rounds of the chip -- 26.7 / 32.3), on average 0.2 % behind the better of the two.  600 x 5136, K = 1024 78 -> 47.5 us, the gated pair of 2048 60 -> 46.3,
+// 2048 x 2048 x 2048 147 -> 96.
 bool pcb_linear_split_fits(const pcb_linear_args& a) { return a.n_groups == 0 && tiles_of(a, 64, 64) > 144; }
 
 int pcb_linear_split_shape(const pcb_linear_args& a) { return shape_of(a); }
