@@ -345,10 +345,10 @@ __global__ __launch_bounds__(64 * SKW) void linear_skinny_kernel(pcb_linear_args
 
 // The few-row products of pb_linear_parts.h, a launch of their own.  LATE: as above.
 // (few_rows() below says which launches take it, and what both cost)
-template <typename E, int EPI, int PARTS, int U, bool LATE>
+template <typename E, int EPI, int PARTS, int U, bool LATE, int G, bool ONCE>
 __global__ __launch_bounds__(512) void linear_parts_kernel(pcb_linear_args a) {
-    __shared__ f4 red[EPI == PCB_EPI_SILU_MUL ? 2 : 1][8][64];
-    parts_block<E, EPI, PARTS, U, LATE>(a, blockIdx.x, red);
+    __shared__ f4 red[EPI == PCB_EPI_SILU_MUL ? 2 * G : G][8][64];
+    parts_block<E, EPI, PARTS, U, LATE, G, ONCE>(a, blockIdx.x, red);
 }
 
 // ---- many rows: both panels travel to LDS by themselves ------------------------------------------------------------------------------
@@ -579,6 +579,7 @@ int launch(const pcb_linear_args& a, hipStream_t stream) {
 struct FewRows {
     int parts;
     bool late;
+    int blocks = 1;                                                  // blocks of 16 / parts columns a workgroup has
 };
 FewRows few_rows(const pcb_linear_args& a) {
     const bool bf = a.dtype == PCB_BF16, gated = a.epilogue == PCB_EPI_SILU_MUL, add = a.epilogue == PCB_EPI_SCALE_ADD;
@@ -597,6 +598,19 @@ FewRows few_rows(const pcb_linear_args& a) {
     // four runs up to three workgroups a CU.  1 row bf16: 2048 x 4096 8.5 / 8.4 / 5.9 / 5.7, 3072 x 2048 6.2 / 5.7 / 5.6 / 5.1; 4 rows, 3072 x 2048 6.5 / 6.3 / 6.3 /
     // 6.2, gated 10.3 / 10.5 / 9.5 / 8.6, 3072 x 1024 5.6 / 4.5 / 4.9 / 4.8, gated 6.8 / 6.5 / 6.6 / 6.5; 1 row fp32 1024 x 2048 9.0 / 7.5 / 5.3 / 4.5
     const bool late = a.epilogue == PCB_EPI_STORE ? bf || a.M <= 2 : gated && bf;
+    // Stores in bf16 of more than a round of eight columns each: two runs and as many blocks of them a workgroup, up to four (deeper k three), as keeps the share of
+    // the busiest CU smallest, the more the better.  Times of the rule before, 8 rows, K = 2048: 2568 columns (2) 0.93, 5136 (3) 0.78, 7424 (4) 0.80, 10272 (3)
+    // 0.76, 32000 (4) 0.72; K = 4096 0.94, 0.77, 0.92 (2), 0.82, 0.74 (2); K = 1024 1.0, 0.89, 0.84, 0.91, 0.79; 4 rows, K = 2048 0.93, 0.89, 0.90, 0.88, 0.86.  One and
+    // two rows only over K <= 1024 (10272 columns 0.85, 32000 0.79; K = 2048 1.02, 1.01).
+    if (bf && a.epilogue == PCB_EPI_STORE && a.n_batch == 0 && a.K % 64 == 0 && a.K >= 1024 && g2 > 256 && (a.M > 2 || a.K <= 1024)) {
+        FewRows f{2, true, 1};
+        int64_t least = 0;
+        for (int blocks = 1; blocks <= (a.K <= 2048 ? 4 : 3); ++blocks) {
+            const int64_t share = (pcb_ceil_div(pcb_ceil_div((int)g2, blocks), 256)) * (int64_t)blocks;
+            if (blocks == 1 || share <= least) f.blocks = blocks, least = share;
+        }
+        return f;
+    }
     if (a.M <= 4 && a.K % 128 == 0 && a.K >= (gated && bf ? 2048 : 1024) && g4 <= (a.M <= 2 || gated || a.K >= 2048 ? 768 : 512)) return {4, late};
     // two runs, of more than four rows not where 16 columns each are one round of the chip and eight are two (there the kernel above over a deep k: 8 rows,
     // K = 4096, 2048 columns 9.6 / 10.3 / 7.1, 2560 9.8 / 10.6 / 10.6, 4096 13.6 / 11.6 / 11.3, 8192 18.3 / 20.1 / 20.4, 16384 35.8 / 36.0 / 36.4)
@@ -636,15 +650,32 @@ int dispatch(const pcb_linear_args& a, hipStream_t stream) {
         const bool late = sizeof(E) == 2 && groups > (a.epilogue == PCB_EPI_SILU_MUL && a.K < 2048 ? 1024 : 768);
         const FewRows few = few_rows(a);
         if (few.parts > 0) {
-            auto go = [&](auto epi, auto p, auto late) {
-                constexpr int EPI = decltype(epi)::value, P = decltype(p)::value;
-                // (fp32: more k-steps in flight cost workgroups)
-                hipLaunchKernelGGL((linear_parts_kernel<E, EPI, P, sizeof(E) == 2 ? 4 : 2, decltype(late)::value>),
-                                   dim3(pcb_ceil_div(a.N, 16 / P), 1, a.n_batch > 0 ? a.n_batch : 1), dim3(512), 0, stream, a);
+            const bool once = pcb_weights_once((a.epilogue == PCB_EPI_SILU_MUL ? 2 : 1) * (int64_t)a.N, a.K, sizeof(E));
+            auto launch = [&](auto epi, auto p, auto late, auto u, auto blocks) {
+                constexpr int EPI = decltype(epi)::value, P = decltype(p)::value, G = decltype(blocks)::value;
+                const dim3 grid(pcb_ceil_div(a.N, 16 / P * G), 1, a.n_batch > 0 ? a.n_batch : 1);
+                if (P > 1 && once)
+                    hipLaunchKernelGGL((linear_parts_kernel<E, EPI, P, decltype(u)::value, decltype(late)::value, G, (P > 1)>), grid, dim3(512), 0, stream, a);
+                else
+                    hipLaunchKernelGGL((linear_parts_kernel<E, EPI, P, decltype(u)::value, decltype(late)::value, G, false>), grid, dim3(512), 0, stream, a);
             };
             using One = std::integral_constant<int, 1>;
             using Two = std::integral_constant<int, 2>;
+            using Three = std::integral_constant<int, 3>;
             using Four = std::integral_constant<int, 4>;
+            // (fp32: more k-steps in flight cost workgroups)
+            auto go = [&](auto epi, auto p, auto late) { launch(epi, p, late, std::integral_constant<int, sizeof(E) == 2 ? 4 : 2>{}, One{}); };
+            if constexpr (sizeof(E) == 2)
+                if (few.blocks > 1) {
+                    using Store = std::integral_constant<int, PCB_EPI_STORE>;
+                    auto sized = [&](auto u) {
+                        few.blocks == 2   ? launch(Store{}, Two{}, std::true_type{}, u, Two{})
+                        : few.blocks == 3 ? launch(Store{}, Two{}, std::true_type{}, u, Three{})
+                                          : launch(Store{}, Two{}, std::true_type{}, u, Four{});
+                    };
+                    a.K <= 1024 ? sized(Two{}) : sized(Four{});
+                    return pcb_check_launch("linear_parts_kernel");
+                }
             auto kind = [&](auto epi) {
                 // (what few_rows() does not ask for is not built: runs side by side are late in a plain store, in bf16 in the gated unit)
                 constexpr bool LATE = decltype(epi)::value == PCB_EPI_STORE || (sizeof(E) == 2 && decltype(epi)::value == PCB_EPI_SILU_MUL);

@@ -92,14 +92,14 @@ __device__ __forceinline__ void normed_block(const pcb_row_norm_args& n, const f
     }
     __builtin_amdgcn_sched_barrier(0);
     // ---- this workgroup's weights (past the end the last k-step again, which is not counted)
-    const int64_t w_at = n_b * a.ldw + 32 * run + 8 * group;
+    const int64_t w_at = n_b * a.ldw + piece_at<E>(run, group);
     const int steps = W / (32 * PARTS);
     Frag<E> fb[U], fc[TWO ? U : 1];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const int s = wave + u * SKW, k = 32 * PARTS * (s < steps ? s : steps - 1);
-        fb[u] = load8((const E*)a.w + w_at + k);
-        if (TWO) fc[u] = load8((const E*)a.w2 + w_at + k);
+        fb[u] = weight_piece<PARTS, (PARTS > 1)>((const E*)a.w + w_at + k);
+        if (TWO) fc[u] = weight_piece<PARTS, (PARTS > 1)>((const E*)a.w2 + w_at + k);
     }
     __builtin_amdgcn_sched_barrier(0);
     // ---- the residual and its norm
@@ -139,12 +139,12 @@ __device__ __forceinline__ void normed_block(const pcb_row_norm_args& n, const f
     lds_barrier();
     // ---- the products
     Sum<E> sum, sum2;
-    const E* xrow = rows + m_a * (W + PAD) + 32 * run + 8 * group;
+    const E* xrow = rows + m_a * (W + PAD) + piece_at<E>(run, group);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const int s = wave + u * SKW;
         if (s >= steps) break;                                       // (uniform over the wave)
-        const Frag<E> fa = load8(xrow + 32 * PARTS * s);
+        const Frag<E> fa = load_piece<PARTS>(xrow + 32 * PARTS * s);
         sum.add(fa, fb[u]);
         if (TWO) sum2.add(fa, fc[u]);
     }

@@ -10,21 +10,21 @@
 namespace {
 using namespace pcb;
 
-// ---- side by side: the first na workgroups are the first product's ---------------------------------------------------------------------
-template <typename E, int EPI, int PARTS, int U>
+// ---- side by side: the first na workgroups are the first product's, GA blocks of columns each ----------------------------------------------
+template <typename E, int EPI, int PARTS, int U, int GA, bool LATE, bool ONCE>
 __global__ __launch_bounds__(512) void linear_pair_kernel(pcb_linear_args a, pcb_linear_args b, int na) {
-    __shared__ f4 red[EPI == PCB_EPI_SILU_MUL ? 2 : 1][8][64];
+    __shared__ f4 red[EPI == PCB_EPI_SILU_MUL ? 2 : GA][8][64];
     if ((int)blockIdx.x < na)
-        parts_block<E, PCB_EPI_STORE, PARTS, U, true>(a, blockIdx.x, red);
+        parts_block<E, PCB_EPI_STORE, PARTS, U, true, GA, ONCE>(a, blockIdx.x, red);
     else
-        parts_block<E, EPI, PARTS, U, EPI == PCB_EPI_STORE>(b, blockIdx.x - na, red);
+        parts_block<E, EPI, PARTS, U, LATE, 1, ONCE>(b, blockIdx.x - na, red);
 }
 
 // ---- one behind the other: y = (base + col_scale (x w^T + bias)) + b.col_scale (b.x b.w^T + b.bias) ------------------------------------------
 // Workgroups and waves as in pb_linear_parts.h, both products' sums side by side.  POLY: the rows of b.x are polynorm(z), worked out where they are
 // used: every workgroup takes the rows' sums itself (eight waves share the rows), beside the first product's loads and with the second's first weights
 // under way.
-template <typename E, int PARTS, int U, bool POLY>
+template <typename E, int PARTS, int U, bool POLY, bool ONCE>
 __global__ __launch_bounds__(512) void linear_add2_kernel(pcb_linear_args a, pcb_linear_args b, const float* __restrict__ z, const float* __restrict__ coef,
                                                           float eps) {
     constexpr int R = 16 / PARTS, SKW = 8;
@@ -32,7 +32,7 @@ __global__ __launch_bounds__(512) void linear_add2_kernel(pcb_linear_args a, pcb
     __shared__ float part[8][3];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, group = lane >> 4, l15 = lane & 15;
     const int M = a.M, N = a.N, n_lo = blockIdx.x * R, run = l15 / R, i = l15 % R;
-    const int n_b = n_lo + i < N ? n_lo + i : N - 1, m_a = i < M ? i : M - 1, at = 32 * run + 8 * group;
+    const int n_b = n_lo + i < N ? n_lo + i : N - 1, m_a = i < M ? i : M - 1, at = piece_at<E>(run, group);
     const E* wa = (const E*)a.w + n_b * a.ldw + at;
     const E* wb = (const E*)b.w + n_b * b.ldw + at;
     const E* xa = (const E*)a.x + m_a * a.ldx + at;
@@ -86,8 +86,8 @@ __global__ __launch_bounds__(512) void linear_add2_kernel(pcb_linear_args a, pcb
         for (int u = 0; u < U; ++u)
             if (s0 + u * SKW < steps_a) {                            // (uniform over the wave)
                 const int k = 32 * PARTS * (s0 + u * SKW);
-                fb[u] = load8(wa + k);
-                fa[u] = load8(xa + k);
+                fb[u] = weight_piece<PARTS, ONCE>(wa + k);
+                fa[u] = load_piece<PARTS>(xa + k);
             }
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -102,11 +102,11 @@ __global__ __launch_bounds__(512) void linear_add2_kernel(pcb_linear_args a, pcb
         for (int u = 0; u < U; ++u)
             if (s0 + u * SKW < steps_b) {
                 const int k = 32 * PARTS * (s0 + u * SKW);
-                fb[u] = load8(wb + k);
+                fb[u] = weight_piece<PARTS, ONCE>(wb + k);
                 if constexpr (POLY)
-                    zv[u][0] = *reinterpret_cast<const f4*>(zrow + k), zv[u][1] = *reinterpret_cast<const f4*>(zrow + k + 4);
+                    zv[u][0] = *reinterpret_cast<const f4*>(zrow + k), zv[u][1] = *reinterpret_cast<const f4*>(zrow + k + (sizeof(E) == 2 ? 4 : 16 * PARTS));
                 else
-                    fa[u] = load8(xb + k);
+                    fa[u] = load_piece<PARTS>(xb + k);
             }
         if constexpr (POLY) {
             if (s0 == wave) {                                        // (every wave comes by exactly once: steps_b >= 8)
@@ -156,31 +156,56 @@ bool splits(const pcb_linear_args& a, int parts) { return a.K % (32 * parts) == 
 
 template <typename E>
 int pair(const pcb_linear_args& a, const pcb_linear_args& b, hipStream_t stream) {
-    auto go = [&](auto epi, auto p) {
-        constexpr int EPI = decltype(epi)::value, P = decltype(p)::value;
-        const int na = pcb_ceil_div(a.N, 16 / P), nb = pcb_ceil_div(b.N, 16 / P);
-        hipLaunchKernelGGL((linear_pair_kernel<E, EPI, P, sizeof(E) == 2 ? 4 : 2>), dim3(na + nb), dim3(512), 0, stream, a, b, na);
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
+    using Four = std::integral_constant<int, 4>;
+    const bool once = pcb_weights_once(a.N + (b.epilogue == PCB_EPI_SILU_MUL ? 2 : 1) * (int64_t)b.N, a.K < b.K ? a.K : b.K, sizeof(E));
+    auto go = [&](auto epi, auto p, auto u, auto ga, auto late) {
+        constexpr int EPI = decltype(epi)::value, P = decltype(p)::value, GA = decltype(ga)::value;
+        const int na = pcb_ceil_div(a.N, 16 / P * GA), nb = pcb_ceil_div(b.N, 16 / P);
+        if (P > 1 && once)
+            hipLaunchKernelGGL((linear_pair_kernel<E, EPI, P, decltype(u)::value, GA, decltype(late)::value, (P > 1)>), dim3(na + nb), dim3(512), 0, stream, a, b, na);
+        else
+            hipLaunchKernelGGL((linear_pair_kernel<E, EPI, P, decltype(u)::value, GA, decltype(late)::value, false>), dim3(na + nb), dim3(512), 0, stream, a, b, na);
         return pcb_check_launch("linear_pair_kernel");
     };
-    // Two runs of k side by side (up to eight rows) while both products together have no more than 8192 weight rows, beyond that up to four rows, not
-    // with a gated bf16 unit.  Weights from memory, us, one run / two: 1 row bf16, 1280 + 4096 columns, K = 1024 5.9 / 5.5, 640 + 2048, K = 512 3.9 / 4.1; 2560 + 8192,
-    // K = 2048 12.9 / 11.2, 8 rows 14.7 / 15.5; 1024 and 2048 gated, K = 1024, 8 rows 6.7 / 6.1, fp32 9.9 / 8.8; 2048 and 4096 gated, K = 2048, 1 row
-    // 12.1 / 12.3, 2 rows fp32 21.8 / 19.7, 8 rows 13.5 / 14.9.  (Four runs lose 2 to 20 % against two at each of these.)  As launches of their own,
-    // the first of each pair: 8.1, 6.4, 13.9, 19.3, 9.9, 13.2, 13.7, 23.3, 16.0.
-    const bool gated = b.epilogue == PCB_EPI_SILU_MUL;
+    // Two runs of k side by side up to eight rows; results' places behind the products where the second is gated, fp32 of many plain columns in one run.
+    // Weights from memory, us, one run (as all were that are not marked *) / two: bf16 1 row, 2048 and 4096 gated, K = 2048 12.5 / 9.4, 8 rows 13.7 / 10.9,
+    // places ahead 14.3; 2560 and 5120, K = 2560 20.3 / 16.8; 2560 + 8192 columns, K = 2048, 8 rows 15.0 / 14.0, 1 row 10.5 * / 9.6; 1024 and 2048 gated, K = 1024, 8
+    // rows 6.5 / 6.7, 4 rows 6.0 / 6.3; 512 + 1024 gated, K = 512 3.7 / 3.9; fp32 5.5 / 4.1; 2048 and 4096 gated, K = 2048, fp32, 2 rows 18.7 * / 16.8 with one
+    // k-step a time and places behind, 8 rows 21.9 * / 19.8; 2560 + 8192 columns, 8 rows 22.8 / 24.4.  The first product's blocks two a workgroup where that is a round
+    // of the chip less: 1536 and 3072 gated, K = 1536, 8 rows 9.1 / 8.0, 3072 and 6144 23.4 / 20.9; 2048 and 4096 10.9 / 11.9.
+    constexpr bool bf = sizeof(E) == 2;
+    const bool gated = b.epilogue == PCB_EPI_SILU_MUL, deep = a.K >= 1024 && b.K >= 1024;
     const int64_t w_rows = (int64_t)a.N + (gated ? 2 : 1) * (int64_t)b.N;
-    const bool two = a.M <= 8 && a.K >= 1024 && b.K >= 1024 && splits(a, 2) && splits(b, 2) &&
-                     (w_rows <= 8192 || (a.M <= 4 && !(gated && sizeof(E) == 2)));
-    auto kind = [&](auto epi) { return two ? go(epi, std::integral_constant<int, 2>{}) : go(epi, std::integral_constant<int, 1>{}); };
-    return b.epilogue == PCB_EPI_STORE ? kind(std::integral_constant<int, PCB_EPI_STORE>{}) : kind(std::integral_constant<int, PCB_EPI_SILU_MUL>{});
+    const bool two = a.M <= 8 && (gated ? !bf || (a.K > 1024 && b.K > 1024) : deep) && splits(a, 2) && splits(b, 2) && (bf || gated || w_rows <= 8192 || a.M <= 4);
+    auto yes = std::true_type{};
+    auto no = std::false_type{};
+    using Plain = std::integral_constant<int, bf ? 4 : 2>;
+    if (!gated) {
+        std::integral_constant<int, PCB_EPI_STORE> epi;
+        return !two ? go(epi, One{}, Plain{}, One{}, yes) : go(epi, Two{}, Plain{}, One{}, std::integral_constant<bool, !bf>{});
+    }
+    std::integral_constant<int, PCB_EPI_SILU_MUL> epi;
+    if (!two) return go(epi, One{}, Plain{}, One{}, no);
+    if constexpr (bf) {
+        const int na = pcb_ceil_div(a.N, 8), nb = pcb_ceil_div(b.N, 8);
+        return pcb_ceil_div(nb + (na + 1) / 2, 256) < pcb_ceil_div(nb + na, 256) ? go(epi, Two{}, Four{}, Two{}, yes) : go(epi, Two{}, Four{}, One{}, yes);
+    } else {
+        return a.K > 1024 && b.K > 1024 ? go(epi, Two{}, One{}, One{}, yes) : go(epi, Two{}, Two{}, One{}, no);
+    }
 }
 
 template <typename E>
 int add2(const pcb_linear_args& a, const pcb_linear_args& b, const float* z, const float* coef, float eps, int parts, hipStream_t stream) {
     constexpr int U = sizeof(E) == 2 ? 4 : 2;
     const dim3 grid(pcb_ceil_div(a.N, 16 / parts));
+    const bool once = pcb_weights_once(2 * (int64_t)a.N, a.K < b.K ? a.K : b.K, sizeof(E));
     auto go = [&](auto p, auto poly) {
-        hipLaunchKernelGGL((linear_add2_kernel<E, decltype(p)::value, U, decltype(poly)::value>), grid, dim3(512), 0, stream, a, b, z, coef, eps);
+        if (once)
+            hipLaunchKernelGGL((linear_add2_kernel<E, decltype(p)::value, U, decltype(poly)::value, true>), grid, dim3(512), 0, stream, a, b, z, coef, eps);
+        else
+            hipLaunchKernelGGL((linear_add2_kernel<E, decltype(p)::value, U, decltype(poly)::value, false>), grid, dim3(512), 0, stream, a, b, z, coef, eps);
         return pcb_check_launch("linear_add2_kernel");
     };
     using Four = std::integral_constant<int, 4>;
@@ -208,11 +233,11 @@ static int pair_form(const pcb_linear_args& a, const pcb_linear_args& b) {
     if (a.dtype != b.dtype || a.M != b.M || a.M <= 0 || a.n_batch != 0 || b.n_batch != 0 || a.epilogue != PCB_EPI_STORE || b.epilogue == PCB_EPI_SCALE_ADD ||
         !pcb_linear_pieces(a) || !pcb_linear_pieces(b) || !pair_apart(a, b))
         return 0;
-    // (A gated unit in bf16 only up to 80 MB of weights: alone it is faster then.  us, two launches / one, 8 rows, residual gate and gated unit of a width:
-    // 2048 15.9 / 14.3, 2560 (66 MB) 24.4 / 21.6, 3072 (94 MB) 28.9 / 29.8, 1 row 13.6 / 12.8, 19.4 / 18.9, 23.4 / 26.5.  9 and 16 rows: bf16 2048 18.7 / 14.7 and
-    // 20.0 / 16.0, 2560 29.2 / 22.2 and 32.9 / 25.2; fp32 2048 27.5 / 23.6 and 29.1 / 26.5; plain, 2560 + 8192
-    // columns, K = 2048, bf16 18.9 / 15.1 and 20.8 / 17.6.)
-    const bool heavy = a.dtype == PCB_BF16 && b.epilogue == PCB_EPI_SILU_MUL && ((int64_t)a.N * a.K + 2 * (int64_t)b.N * b.K) * 2 > 80000000;
+    // (More than four rows of bf16 with many plain columns as two: there each is the faster by itself, with several blocks of columns a workgroup.  us, one launch / two,
+    // 8 rows, 2560 + 8192 columns, K = 2048 14.0 / 14.6, 3840 + 12288, K = 3072 24.9 / 23.8, 5120 + 16384, K = 4096 42.6 / 37.2; gated 3072 and 6144, K = 3072
+    // 20.9 / 25.0, 1 row 17.7 / 20.3, 4096 and 8192 32.2 / 36.6, 16 rows 44.1 / 49.0; fp32 2048 and 4096, 9 and 16 rows 23.6 / 27.5 and 26.5 / 29.1; plain, 2560 + 8192
+    // columns, 9 and 16 rows 15.1 / 18.9 and 17.6 / 20.8.)
+    const bool heavy = a.dtype == PCB_BF16 && b.epilogue == PCB_EPI_STORE && a.M > 4 && a.M <= 8 && ((int64_t)a.N * a.K + (int64_t)b.N * b.K) * 2 > 80000000;
     if (a.M <= 16) return heavy ? 0 : 1;
     const int shape = a.M > 64 ? pcb_linear_tiles_pair_shape(a, b) : -1;
     return shape < 0 ? 0 : 2 + shape;

@@ -31,7 +31,10 @@ struct Sum<float> {
 // runs' sums of R columns each, and what lies beside them is thrown away.  A workgroup then has R columns instead of 16: twice or four times the
 // workgroups where 16 columns each would leave CUs idle, and as many more loads under way per column.  Eight waves split k; a wave requests U k-steps
 // at a time (a loop of single steps waits for each).
-
+// What bounds it: the launch (2.2 us), then the weights at 6 TB/s where nothing stands beside their stream.  An instruction that reads eight rows of
+// 128 bytes (two runs) costs what one that reads a KB in a row does, sixteen rows of 64 bytes 10 to 20 % more (weights alone, 42 MB 8.3 / 8.3 / 9.5 us); the rows
+// themselves are as many bytes a workgroup as its weights at eight rows and eight columns, so several blocks of columns share one reading of them.  8 rows, K = 2048,
+// before / with both, us: 5136 columns (21 MB) 9.1 / 7.1, 10272 14.1 / 10.8, 32000 34.1 / 24.6 (weights alone 21).
 // the waves' sums: lane R i .. of run 0 ends up with what it stores (rows m0 = 4 (lane >> 4) .. + 3 of column lane & 15)
 template <int PARTS>
 __device__ __forceinline__ f4 parts_total(const f4 (*red)[64], int lane) {
@@ -47,25 +50,31 @@ __device__ __forceinline__ f4 parts_total(const f4 (*red)[64], int lane) {
     return acc;
 }
 
-// Workgroup `block` of such a launch, 512 threads; red: [EPI gated ? 2 : 1][8][64].  LATE: where a result goes is worked out behind the products.
-template <typename E, int EPI, int PARTS, int U, bool LATE>
+// Workgroup `block` of such a launch, 512 threads; red: [G, gated 2 G][8][64].  LATE: where a result goes is worked out behind the products.  G: blocks of
+// R columns a workgroup has, which share what it reads of the rows.
+template <typename E, int EPI, int PARTS, int U, bool LATE, int G, bool ONCE>
 __device__ __forceinline__ void parts_block(const pcb_linear_args& a, int block, f4 (*red)[8][64]) {
     constexpr bool TWO = EPI == PCB_EPI_SILU_MUL, ADD = EPI == PCB_EPI_SCALE_ADD;
-    constexpr int R = 16 / PARTS, SKW = 8;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, group = lane >> 4, l15 = lane & 15;
-    const int K = a.K, N = a.N, n_lo = block * R, g = a.n_batch > 0 ? blockIdx.z : 0;
+    constexpr int R = 16 / PARTS, SKW = 8, T = TWO ? 2 : 1;
+    const int tid = threadIdx.x, lane = tid & 63, wave = G > 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6, group = lane >> 4, l15 = lane & 15;
+    const int K = a.K, N = a.N, n_lo = block * (R * G), g = a.n_batch > 0 ? blockIdx.z : 0;
     const int run = l15 / R, i = l15 % R;
-    const int n_b = n_lo + i < N ? n_lo + i : N - 1, m_a = i < a.M ? i : a.M - 1;
+    const int m_a = i < a.M ? i : a.M - 1, at = piece_at<E>(run, group);
     const E* X = (const E*)a.x + g * a.x_batch_stride;
-    const int64_t w_at = g * a.w_group_stride + n_b * a.ldw + 32 * run + 8 * group;
-    const E* wrow = (const E*)a.w + w_at;
-    const E* wrow2 = TWO ? (const E*)a.w2 + w_at : nullptr;
-    const E* xrow = X + (int64_t)(a.row_src ? a.row_src[m_a] : m_a) * a.ldx + 32 * run + 8 * group;
-    // (the lanes that store: rows m0 .. m0 + 3 of column n_b, run 0)
-    const int m0 = 4 * group;
+    const E* wrow[G * T];
+#pragma unroll
+    for (int j = 0; j < G; ++j) {
+        const int n = n_lo + j * R + i < N ? n_lo + j * R + i : N - 1;
+        const int64_t w_at = g * a.w_group_stride + n * a.ldw + at;
+        wrow[j * T] = (const E*)a.w + w_at;
+        if (TWO) wrow[j * T + T - 1] = (const E*)a.w2 + w_at;
+    }
+    const E* xrow = X + (int64_t)(a.row_src ? a.row_src[m_a] : m_a) * a.ldx + at;
+    // (the lanes that store: rows m0 .. m0 + 3 of column n_b, run 0, of a wave's block)
+    const int m0 = 4 * group, mine = n_lo + (G > 1 ? wave * R : 0) + i, n_b = mine < N ? mine : N - 1;
     float bv = 0.0f, bv2 = 0.0f, cs = 0.0f;
     Place to[4] = {};
-    const bool stores = wave == 0 && m0 < R && run == 0;
+    const bool stores = wave < G && m0 < R && run == 0;
     auto places = [&] {
         if (a.bias) bv = to_f32(((const E*)a.bias)[n_b]);
         if (TWO && a.bias2) bv2 = to_f32(((const E*)a.bias2)[n_b]);
@@ -75,38 +84,46 @@ __device__ __forceinline__ void parts_block(const pcb_linear_args& a, int block,
             if (TWO || m0 + r < a.M) to[r] = place<E, EPI>(a, m0 + r < a.M ? m0 + r : a.M - 1, n_b);
     };
     if (!LATE && stores) places();
-    Sum<E> sum, sum2;
+    Sum<E> sum[G * T];
     const int steps = K / (32 * PARTS);
     for (int s0 = wave; s0 < steps; s0 += U * SKW) {
-        Frag<E> fa[U], fb[U], fc[TWO ? U : 1];
+        Frag<E> fa[U], fb[G * T][U];
 #pragma unroll
         for (int u = 0; u < U; ++u)
             if (s0 + u * SKW < steps) {                                // (uniform over the wave)
                 const int k = 32 * PARTS * (s0 + u * SKW);
-                fb[u] = load8(wrow + k);
-                if (TWO) fc[u] = load8(wrow2 + k);
-                fa[u] = load8(xrow + k);
+#pragma unroll
+                for (int j = 0; j < G * T; ++j) fb[j][u] = weight_piece<PARTS, ONCE>(wrow[j] + k);
+                fa[u] = load_piece<PARTS>(xrow + k);
             }
 #pragma unroll
         for (int u = 0; u < U; ++u)
             if (s0 + u * SKW < steps) {
-                sum.add(fa[u], fb[u]);
-                if (TWO) sum2.add(fa[u], fc[u]);
+#pragma unroll
+                for (int j = 0; j < G * T; ++j) sum[j].add(fa[u], fb[j][u]);
             }
     }
     if (LATE && stores) places();
-    red[0][wave][lane] = sum.total();
-    if (TWO) red[1][wave][lane] = sum2.total();
+#pragma unroll
+    for (int j = 0; j < G * T; ++j) red[j][wave][lane] = sum[j].total();
     __syncthreads();
-    if (wave != 0) return;
-    const f4 acc = parts_total<PARTS>(red[0], lane), acc2 = TWO ? parts_total<PARTS>(red[TWO], lane) : f4{};
-    if (!stores || n_lo + i >= N) return;
+    if (wave >= G) return;
+    const int at_red = G > 1 ? wave * T : 0;
+    const f4 acc = parts_total<PARTS>(red[at_red], lane), acc2 = TWO ? parts_total<PARTS>(red[at_red + T - 1], lane) : f4{};
+    if (!stores || mine >= N) return;
 #pragma unroll
     for (int r = 0; r < 4; ++r)
         if (m0 + r < a.M) put<E, EPI>(to[r], finished<E, EPI>(a, to[r], n_b, acc[r], acc2[r], bv, bv2), cs);
 }
 
 }  // namespace pcb
+
+// Whether a launch's weights (K to a row, `rows` rows of es bytes an element) are read past the caches (nontemporal): where they come from a model whose weights
+// do not stay in the 256 MB of the Infinity Cache from one step to the next, as rows of 4 KB in matrices of 8 MB do (bf16 of width 2048), in fp32 of 4 MB
+// (width 1024).  us, through the caches / past them: from memory, 8 rows, K = 2048, 5136 columns 7.9 / 7.1, 10272 11.8 / 10.8, 2048 5.6 / 5.1; fp32, K = 1024, 2 rows,
+// 2568 columns 6.1 / 5.8, a step of two requests 315 without the 4 MB ones, 305 with them; weights that do stay, 1 row, K = 1024 and 4096 added 6.7 / 8.0,
+// 32000 x 1024 12.0 / 13.2.
+inline bool pcb_weights_once(int64_t rows, int64_t K, int es) { return K * es >= 4096 && rows * K * es >= (es == 2 ? 8000000 : 4000000); }
 
 // PCB_OK when the arguments are valid (pb_linear.hip)
 int pcb_linear_check(const pcb_linear_args* a);

@@ -82,3 +82,19 @@ def test_few_rows_at_the_rules_other_borders(M, N, K, dtype):
     scale, want = rnd(N, seed=7), f(y)
     b.linear(x, w, y, M=M, epilogue=b.EPI_SCALE_ADD, col_scale=scale)
     assert rel(y, want + f(scale) * z) < 1e-6
+
+
+# several blocks of eight columns a workgroup: a block more than a round of the chip, last workgroups of one block or a part of it, two, three and four blocks, k of
+# one, two and three trips, weights read past the caches (rows of 4 KB, 4 MB) and not
+@pytest.mark.parametrize("M", [1, 2, 3, 5, 8])
+@pytest.mark.parametrize("N,K", [(2049, 1024), (4609, 1088), (6144, 1984), (8161, 2048), (8193, 2112), (6137, 4096), (16385, 1024)])
+def test_several_blocks_of_columns_a_workgroup(M, N, K):
+    b, f, dtype = B(), lambda t: t.to(F64), torch.bfloat16
+    x, w, bias = rnd(M, K, seed=1, dtype=dtype), rnd(N, K, seed=2, dtype=dtype) * 0.1, rnd(N, seed=3, dtype=dtype)
+    out, y, z = torch.zeros(M + 1, N, dtype=dtype, device=DEV), torch.empty(M, N, device=DEV), f(x) @ f(w).T
+    b.linear(x, w, y, M=M)
+    assert rel(y, z) < 1e-6
+    b.linear(x, w, out, M=M, bias=bias, act_split=N // 3, act2=b.ACT_SIGMOID)
+    want = z + f(bias)
+    want[:, N // 3:] = want[:, N // 3:].sigmoid()
+    assert rel(out[:M], want) < 2.0 ** -8 and not bool(out[M].any())

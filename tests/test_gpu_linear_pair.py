@@ -39,6 +39,14 @@ def test_pairs(M, N, N2, K, K2, dtype):
     assert rel(gate, want.sigmoid()) < max(low, 2e-6) and rel(mid, (f(x2) @ f(v).T).relu() * (f(x2) @ f(v2).T)) < max(low, 2e-6)
 
 
+# two blocks of the first product's columns a workgroup (a round of the chip less), the last one of a part of a block; k of one product beyond the line, of the other not
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M", [1, 5, 8])
+@pytest.mark.parametrize("N,N2,K,K2", [(1540, 3070, 1536, 1536), (1537, 3072, 1600, 1088), (3000, 9, 1088, 1024)])
+def test_pairs_beside_a_gated_unit_of_two_runs(M, N, N2, K, K2, dtype):
+    test_pairs(N=N, N2=N2, K=K, K2=K2, M=M, dtype=dtype)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("M", [1, 2, 3, 5, 8, 9])
 @pytest.mark.parametrize("N,K,ff", [(1024, 1024, 4096), (1001, 512, 1536), (70, 1152, 512), (36, 64, 96)])
