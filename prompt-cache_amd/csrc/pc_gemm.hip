@@ -50,6 +50,7 @@ void set_k_balance(GemmParams& p, int K) {
 int launch_MT(int epi, const GemmParams& p, int T, int units, hipStream_t s) {
     const int mt = pc_ceil_div(p.M, 16);
     if (mt > 4) return launch_rows_epi(epi, p, units, s);
+    if (normed_few_takes(epi, p)) return launch_normed_few(epi, p, units, s);
     if (mt <= 1) return launch_skinny_mt1(epi, p, T, units, s);
     if (mt == 2) return launch_skinny_mt2(epi, p, T, units, s);
     return launch_skinny_mt4(epi, p, T, units, s);

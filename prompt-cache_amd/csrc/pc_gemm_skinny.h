@@ -962,6 +962,11 @@ void launch_w8(const GemmParams& p, dim3 grid, dim3 block, hipStream_t s) {
     }
 }
 
+// the norm inside the launch (pc_gemm_norm.hip): one and two rows, and two to four tiles a workgroup
+bool normed_few_takes(int epi, const GemmParams& p);
+int launch_normed_few(int epi, const GemmParams& p, int units, hipStream_t s);
+int launch_normed(int epi, const GemmParams& p, int T, int units, hipStream_t s);
+
 template <int MT, int T, int EPI>
 int launch_one(const GemmParams& p, int units, hipStream_t s) {
     constexpr int TT = (EPI == EPI_SILU) ? 2 * T : T;
@@ -969,6 +974,10 @@ int launch_one(const GemmParams& p, int units, hipStream_t s) {
     static const int forced = [] { const char* e = getenv("PC_GEMM_U"); return e ? atoi(e) : 0; }();
     const dim3 grid(pc_ceil_div(units, T), p.kslices), block(kThreads);
     const bool two = p.xf_lo != nullptr;
+    // (the norm inside the launch, fp16 weights, one row tile: pc_gemm_norm.hip)
+    constexpr bool kNormed = MT == 1 && T >= 2 && T <= 4 && (EPI == EPI_STORE || EPI == EPI_ROPE || EPI == EPI_SILU);
+    if constexpr (kNormed)
+        if (p.xn && !p.w8) return launch_normed(EPI, p, T, units, s);
 #define PC_GO(UV)                                                                                     \
     do {                                                                                              \
         if (p.w8) {   /* int8 weights: split-precision activations only.  Same k-steps per block as fp16 (half the   */ \
@@ -978,7 +987,7 @@ int launch_one(const GemmParams& p, int units, hipStream_t s) {
             launch_w8<MT, T, EPI, UW, UA>(p, grid, block, s);                                         \
             break;                                                                                    \
         }                                                                                             \
-        if constexpr (MT <= 2 && EPI != EPI_ADD) {                                                    \
+        if constexpr (MT <= 2 && EPI != EPI_ADD && !kNormed) {                                        \
             if (p.xn) {   /* (two row tiles of fp32 rows: eight k-steps of them in flight spill) */       \
                 constexpr int UN = (MT == 2 && (UV) > 4) ? 4 : (UV);                                  \
                 hipLaunchKernelGGL((gemm_skinny_kernel<MT, T, EPI, true, UN, true>), grid, block, 0, s, p); \
