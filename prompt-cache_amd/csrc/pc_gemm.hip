@@ -51,6 +51,20 @@ int launch_MT(int epi, const GemmParams& p, int T, int units, hipStream_t s) {
     const int mt = pc_ceil_div(p.M, 16);
     if (mt > 4) return launch_rows_epi(epi, p, units, s);
     if (normed_few_takes(epi, p)) return launch_normed_few(epi, p, units, s);
+    if (!p.w8 && !p.xn && p.xf_lo) {
+        // Five tiles a workgroup where they fill a round of the chip that eight leave a third empty (13b's down_proj and o_proj in four slices, us, eight / five: 20 rows
+        // 30.3 / 25.3 and 14.6 / 13.2, 40 rows, four 42.5 / 29.5 and 19.5 / 15.9), and up to 32 rows of one slice instead of four where tile images are whole multiples of
+        // 64 KB, since the starts of four of them lie on the same channels (1024 tiles, K = 4096: 12 rows 29.7 / 25.3, 20 rows 30.9 / 26.6, 64 rows 35.7 / 36.4).
+        const bool five = mt <= 2 ? epi != EPI_SILU : epi == EPI_STORE;
+        if (five && T == 8 && pc_ceil_div(units * p.kslices, 5) <= 256) T = 5;
+        if (five && T == 4 && mt <= 2 && p.kslices == 1 && p.KS % 64 == 0) T = 5;
+        if (T == 5 && mt <= 2) return launch_pipe(epi, p, T, units, s);
+        // (33 to 64 rows take three pairs at most: two, where three are a second round of the chip that is emptier.  13b's gate|up, 40 rows 81.5 / 67.2)
+        if (mt > 2 && epi == EPI_SILU && T > 3) {
+            auto busy = [&](int t) { const int wg = pc_ceil_div(units, t); return (float)wg / (float)(256 * pc_ceil_div(wg, 256)); };
+            T = busy(2) > busy(3) ? 2 : 3;
+        }
+    }
     if (mt <= 1) return launch_skinny_mt1(epi, p, T, units, s);
     if (mt == 2) return launch_skinny_mt2(epi, p, T, units, s);
     return launch_skinny_mt4(epi, p, T, units, s);

@@ -260,8 +260,10 @@ int launch_skinny_ks(const void* wf, const void* xf_hi, const void* xf_lo, int M
     switch (tiles_per_wg) {
         case 1: return share > 8 ? launch_ks<1, 16>(kp, s) : launch_ks<1, 8>(kp, s);
         case 2: return share > 8 ? launch_ks<2, 12>(kp, s) : launch_ks<2, 8>(kp, s);
-        case 4: return share > 4 ? launch_ks<4, 8>(kp, s) : launch_ks<4, 4>(kp, s);
-        case 8: return share > 3 ? launch_ks<8, 4>(kp, s) : launch_ks<8, 3>(kp, s);
+        // (four and eight tiles: the next k-step under way while one is multiplied.  13b, 12 rows, three slices of four tiles, down_proj 26.0 us, o_proj 13.4; in blocks of
+        // eight k-steps one after the other spread over two tiles and two slices 41.0 and 18.0.)
+        case 4: return launch_ks<4, 1, true>(kp, s);
+        case 8: return launch_ks<8, 1, true>(kp, s);
         default: break;
     }
     pc_set_error("pc_gemm (ks): ks_tiles %d not in {1, 2, 4, 8}", tiles_per_wg);

@@ -1,0 +1,143 @@
+// Weight-streaming projections of up to 32 rows in two planes, three to five tiles (pairs of tiles) a workgroup: pc_gemm_skinny.h's tiles, K split, reduction and
+// epilogues with the next U k-steps' weights and activations under way while U are multiplied.  (One block of k-steps after the other leaves a wave without a load
+// under way while it multiplies, and more bytes in flight do not make up for it: one or two k-steps of four tiles are what a CU's memory path holds.)
+// us, one block after the other / so, weights from memory: 20 rows, 7b q|k|v 21.3 / 20.4, gate|up 36.5 / 33.1, o_proj in four slices 10.5 / 9.4, down_proj 22.0 / 21.6;
+// 13b gate|up 52.4 / 51.1; 12 rows, 13b q|k|v 28.2 / 28.3, o_proj 16.6 / 12.1 and down_proj 33.0 / 23.7 with five tiles instead of eight.  Weights alone, 7b: 17.1, 28.7,
+// 6.5, 16.2.  Not for 33 rows and more (down_proj 24.0 / 25.4: the activations are the larger part) nor one, two or eight tiles (18.5 / 21.5, 49.6 / 49.5).
+#include <type_traits>
+
+#include "pc_gemm_skinny.h"
+
+using namespace pcg;
+
+namespace {
+
+template <int MT, int T, int EPI, int U>
+__global__ __launch_bounds__(kThreads) void gemm_pipe_kernel(const GemmParams p) {
+    constexpr int TT = EPI == EPI_SILU ? 2 * T : T, TPI = EPI == EPI_SILU ? 2 : 1;       // tiles, tiles of an output item
+    constexpr int kRT = MT * TT < 8 ? MT * TT : 8, IPR = kRT / TPI;                      // tiles, items of a round of the reduction (64 KiB at most)
+    constexpr int NOUT = MT * T, ROUNDS = (NOUT + IPR - 1) / IPR;
+    __shared__ f4 red[kWaves][kRT][64];
+    const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int KS = p.KS, bx = blockIdx.x, by = blockIdx.y;
+    int ks0, ks1;
+    wave_k_range<false>(p, by, wave, ks0, ks1);
+    int tile[TT];
+    wg_tiles<T, EPI>(p, bx, tile);
+    const char* wt[TT];
+#pragma unroll
+    for (int t = 0; t < TT; ++t) wt[t] = (const char*)p.wf + (int64_t)tile[t] * KS * 1024;
+    const int live = p.m_dev ? (*p.m_dev < p.M ? *p.m_dev : p.M) : p.M;
+    bool ok[MT];
+#pragma unroll
+    for (int a = 0; a < MT; ++a) ok[a] = a * 16 + m < live;
+    struct Block {
+        h8 w[U][TT], h[U][MT], l[U][MT];
+    } A, B;
+    auto issue = [&](Block& b, int kb) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            int k = kb + u < ks1 ? kb + u : ks1 - 1;                         // (past the share the last k-step again, not multiplied)
+            k = k < 0 ? 0 : k;
+            const uint32_t at = (uint32_t)k * 1024u + (uint32_t)lane * 16u;
+#pragma unroll
+            for (int t = 0; t < TT; ++t) b.w[u][t] = __builtin_bit_cast(h8, __builtin_nontemporal_load((const u32x4*)(wt[t] + at)));
+#pragma unroll
+            for (int a = 0; a < MT; ++a) {
+                const h8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+                b.h[u][a] = b.l[u][a] = zero;
+                if (ok[a]) {
+                    b.h[u][a] = *(const h8*)((const char*)p.xf_hi + (int64_t)a * KS * 1024 + at);
+                    b.l[u][a] = *(const h8*)((const char*)p.xf_lo + (int64_t)a * KS * 1024 + at);
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    f4 acc[MT][TT];
+#pragma unroll
+    for (int a = 0; a < MT; ++a)
+#pragma unroll
+        for (int t = 0; t < TT; ++t) acc[a][t] = f4{0.f, 0.f, 0.f, 0.f};
+    auto consume = [&](const Block& b, int kb) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (kb + u >= ks1) continue;                                     // (uniform over the wave)
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                for (int a = 0; a < MT; ++a) {
+                    acc[a][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b.w[u][t], b.h[u][a], acc[a][t], 0, 0, 0);
+                    acc[a][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b.w[u][t], b.l[u][a], acc[a][t], 0, 0, 0);
+                }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    issue(A, ks0);
+    for (int kb = ks0; kb < ks1; kb += 2 * U) {
+        issue(B, kb + U);
+        consume(A, kb);
+        if (kb + 2 * U < ks1) issue(A, kb + 2 * U);
+        consume(B, kb + U);
+    }
+    // the waves' shares in wave order, one output item a wave and round
+#pragma unroll
+    for (int r = 0; r < ROUNDS; ++r) {
+        if (r > 0) lds_barrier();
+#pragma unroll
+        for (int i = 0; i < IPR; ++i) {
+            const int item = r * IPR + i;
+            if (item < NOUT) {
+                const int a = item / T, t = item - a * T;
+                red[wave][i * TPI][lane] = acc[a][t];
+                if (EPI == EPI_SILU) red[wave][i * TPI + TPI - 1][lane] = acc[a][TT - T + t];
+            }
+        }
+        lds_barrier();
+        const int item = r * IPR + wave;
+        if (wave < IPR && item < NOUT) {
+            const int a = item / T, t = item - a * T;
+            f4 v = {0.f, 0.f, 0.f, 0.f}, u = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) {
+                v += red[w][wave * TPI][lane];
+                if (EPI == EPI_SILU) u += red[w][wave * TPI + TPI - 1][lane];
+            }
+            tile_epilogue<EPI>(p, v, u, a * 16 + m, bx * T + t, g, by);
+        }
+    }
+}
+
+template <int MT, int T, int EPI>
+int go(const GemmParams& p, int units, hipStream_t s) {
+    constexpr int U = EPI != EPI_SILU && (T == 4 || (MT == 1 && T == 3)) ? 2 : 1;
+    hipLaunchKernelGGL((gemm_pipe_kernel<MT, T, EPI, U>), dim3(pc_ceil_div(units, T), p.kslices), dim3(kThreads), 0, s, p);
+    return pc_check_launch("gemm_pipe_kernel");
+}
+
+template <int MT, int T>
+int by_epi(int epi, const GemmParams& p, int units, hipStream_t s) {
+    switch (epi) {
+        case EPI_STORE: return go<MT, T, EPI_STORE>(p, units, s);
+        case EPI_ADD: return go<MT, T, EPI_ADD>(p, units, s);
+        case EPI_SILU:
+            if constexpr (T <= 4) return go<MT, T, EPI_SILU>(p, units, s);
+            return PC_ERR_ARG;
+        case EPI_ROPE: return go<MT, T, EPI_ROPE>(p, units, s);
+        default: return go<MT, T, EPI_GELU>(p, units, s);
+    }
+}
+
+template <int MT>
+int by_tiles(int epi, const GemmParams& p, int T, int units, hipStream_t s) {
+    return T == 3 ? by_epi<MT, 3>(epi, p, units, s) : T == 4 ? by_epi<MT, 4>(epi, p, units, s) : by_epi<MT, 5>(epi, p, units, s);
+}
+
+}  // namespace
+
+namespace pcg {
+int launch_pipe(int epi, const GemmParams& p, int T, int units, hipStream_t s) {
+    return p.M <= 16 ? by_tiles<1>(epi, p, T, units, s) : by_tiles<2>(epi, p, T, units, s);
+}
+}  // namespace pcg

@@ -966,6 +966,8 @@ void launch_w8(const GemmParams& p, dim3 grid, dim3 block, hipStream_t s) {
 bool normed_few_takes(int epi, const GemmParams& p);
 int launch_normed_few(int epi, const GemmParams& p, int units, hipStream_t s);
 int launch_normed(int epi, const GemmParams& p, int T, int units, hipStream_t s);
+// two planes, up to 32 rows, three to five tiles a workgroup (pc_gemm_pipe.hip)
+int launch_pipe(int epi, const GemmParams& p, int T, int units, hipStream_t s);
 
 template <int MT, int T, int EPI>
 int launch_one(const GemmParams& p, int units, hipStream_t s) {
@@ -974,6 +976,10 @@ int launch_one(const GemmParams& p, int units, hipStream_t s) {
     static const int forced = [] { const char* e = getenv("PC_GEMM_U"); return e ? atoi(e) : 0; }();
     const dim3 grid(pc_ceil_div(units, T), p.kslices), block(kThreads);
     const bool two = p.xf_lo != nullptr;
+    // (two planes without the norm, three and four tiles of up to two row tiles: pc_gemm_pipe.hip)
+    constexpr bool kPiped = MT <= 2 && (T == 3 || T == 4);
+    if constexpr (kPiped)
+        if (two && !p.xn && !p.w8) return launch_pipe(EPI, p, T, units, s);
     // (the norm inside the launch, fp16 weights, one row tile: pc_gemm_norm.hip)
     constexpr bool kNormed = MT == 1 && T >= 2 && T <= 4 && (EPI == EPI_STORE || EPI == EPI_ROPE || EPI == EPI_SILU);
     if constexpr (kNormed)
@@ -994,8 +1000,10 @@ int launch_one(const GemmParams& p, int units, hipStream_t s) {
                 break;                                                                                \
             }                                                                                         \
         }                                                                                             \
-        if (two) hipLaunchKernelGGL((gemm_skinny_kernel<MT, T, EPI, true, UV>), grid, block, 0, s, p); \
-        else hipLaunchKernelGGL((gemm_skinny_kernel<MT, T, EPI, false, UV>), grid, block, 0, s, p);    \
+        if constexpr (!kPiped) {                                                                      \
+            if (two) { hipLaunchKernelGGL((gemm_skinny_kernel<MT, T, EPI, true, UV>), grid, block, 0, s, p); break; } \
+        }                                                                                             \
+        hipLaunchKernelGGL((gemm_skinny_kernel<MT, T, EPI, false, UV>), grid, block, 0, s, p);         \
     } while (0)
 #ifdef PC_DEV_SWEEPS   // block-depth sweeps (tools/gemm_n4096_sweep.py): ~500 extra kernel instantiations, not in the product build
     if constexpr (MT * TT <= 2) {
@@ -1037,6 +1045,7 @@ int launch_T(const GemmParams& p, int T, int units, hipStream_t s) {
     constexpr int kMaxT8 = 8 / MT / (EPI == EPI_SILU ? 2 : 1);     // int8 images: at most 8 accumulator tiles (launch_w8)
     if (p.w8 && T > kMaxT8) T = kMaxT8;
     if constexpr (kMaxT >= 8) { if (T >= 8) return launch_one<MT, 8, EPI>(p, units, s); }
+    if constexpr (MT == 4 && EPI == EPI_STORE) { if (T == 5) return launch_one<MT, 5, EPI>(p, units, s); }
     if constexpr (kMaxT >= 4) { if (T >= 4) return launch_one<MT, 4, EPI>(p, units, s); }
     if constexpr (kMaxT >= 3) { if (T == 3) return launch_one<MT, 3, EPI>(p, units, s); }
     if constexpr (kMaxT >= 2) { if (T >= 2) return launch_one<MT, 2, EPI>(p, units, s); }

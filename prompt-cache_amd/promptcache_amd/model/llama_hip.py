@@ -311,8 +311,13 @@ class LlamaHIP:
         # Measured at 12 rows (tools/ks_micro.py, in-graph): down_proj (K = 11008) 22.75 -> 20.16 us at 2 tiles x 2 slices, every
         # other shape of either projection loses to the one-tile launch (o_proj 9.4 -> 10.4 .. 13.5 us; one row: 19.0 -> 20.3 us):
         # the in-launch reduction costs ~3 us, only the long-K launch with its 2:1 activation traffic earns it back.
-        self.ks_o, self.ks_down = _ks("PC_KS_O", ""), _ks("PC_KS_DOWN", "2,2")
-        self.ks_min_rows = 5       # ... and only with more than 4 rows (decode keeps the one-tile launch)
+        # Where a tile each is more than the 256 CUs (hidden 5120: 320), whichever of these fills a round of them, o_proj and one row included: 4 x 3, 240
+        # workgroups; us, one tile (two of them a workgroup) / 2 x 2 / 4 x 3, down_proj 12 rows 35.4 / 41.0 / 26.0, 1 row 30.2 / 40.1 / 24.9, o_proj 12 rows
+        # 14.9 / 18.0 / 13.4, 1 row 13.1 / 17.7 / 12.8.
+        tiles = -(-shape.hidden_size // 16)
+        fits = [f"{t},{k}" for t, k in ((4, 3), (4, 2), (8, 3)) if tiles > 256 and 200 <= -(-tiles // t) * k <= 256][:1]
+        self.ks_o, self.ks_down = _ks("PC_KS_O", fits[0] if fits else ""), _ks("PC_KS_DOWN", fits[0] if fits else "2,2")
+        self.ks_min_rows = 1 if fits else 5      # ... and, where a tile each is one round, only with more than 4 rows (decode keeps the one-tile launch)
         self._ks_state = None      # (scratch, counters), lazily
         self._kv_only = False      # set per call (see __call__)
         self._past_lens = None     # set per call: per-row past lengths of a ragged-prefix encode batch
