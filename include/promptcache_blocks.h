@@ -20,7 +20,7 @@ extern "C" {
 
 #define PCB_ABI_VERSION 6
 #define PCB_OK 0
-#define PCB_NOT_TAKEN 1 /* pcb_norm_linear only: sizes, alignments or overlaps it does not take; nothing was launched */
+#define PCB_NOT_TAKEN 1 /* pcb_norm_linear and pcb_norm_stream only: sizes, alignments or overlaps it does not take; nothing was launched */
 #define PCB_ERR_ARG (-2001)
 #define PCB_ERR_HIP_BASE (-3000)
 
@@ -796,6 +796,10 @@ typedef struct pcb_row_norm_args {
 } pcb_row_norm_args;
 int pcb_norm_linear(const pcb_row_norm_args* n, const pcb_linear_args* a, const pcb_linear_args* b, void* stream);
 int pcb_norm_linear_takes(const pcb_row_norm_args* n, const pcb_linear_args* a, const pcb_linear_args* b);
+/* The same, and the same checks, for more elements (8 rows of 2048) or more columns, one workgroup a CU.  PCB_NOT_TAKEN as there; pcb_norm_linear is the faster one where
+ * it takes a launch. */
+int pcb_norm_stream(const pcb_row_norm_args* n, const pcb_linear_args* a, const pcb_linear_args* b, void* stream);
+int pcb_norm_stream_takes(const pcb_row_norm_args* n, const pcb_linear_args* a, const pcb_linear_args* b);
 
 /* Recurrences with a matrix state S [dim][vdim] per (slot, head), fp32, zero before position 0.  Per token and head h:
  *   q = q_scale q^, k = k_scale k^        q^, k^: E rows with head h / (H / Hk) at column (h / (H / Hk)) * dim; unit_norm: divided by

@@ -260,20 +260,8 @@ int launch(const pcb_row_norm_args& n, const pcb_linear_args& a, const pcb_linea
 
 }  // namespace
 
-static int norm_linear_check(const pcb_row_norm_args* n, const pcb_linear_args* a, const pcb_linear_args* b) {
-    int rc = pcb_linear_check(a);
-    if (rc == PCB_OK && b) rc = pcb_linear_check(b);
-    if (rc != PCB_OK) return rc;
-    PCB_REQUIRE(n && n->struct_bytes == sizeof(pcb_row_norm_args), PCB_ERR_ARG, "pcb_norm_linear: struct size mismatch");
-    PCB_REQUIRE(n->x_out && n->gain && (!b || n->gain2) && (n->table ? n->ids && n->vocab > 0 && !n->y : n->x && n->x != n->x_out) &&
-                    (n->table || n->y ? n->n_terms == 0 : n->n_terms > 0 && n->coef) && (!n->y || (n->gate && n->post_gain && n->ldg >= a->K)),
-                PCB_ERR_ARG, "pcb_norm_linear: rows of a table, a sum of streams, or a residual and a gated sublayer's result; x_out is neither's");
-    PCB_REQUIRE(!b || (a->dtype == b->dtype && a->M == b->M && a->K == b->K), PCB_ERR_ARG, "pcb_norm_linear: products of the same rows");
-    return PCB_OK;
-}
-
 // Every workgroup works out the rows from what they are made of, and nothing orders workgroups: what the products store, and x_out, has to lie apart from that.
-static bool norm_linear_apart(const pcb_row_norm_args& n, const pcb_linear_args& a, const pcb_linear_args* b, bool results) {
+bool pcb_norm_linear_apart(const pcb_row_norm_args& n, const pcb_linear_args& a, const pcb_linear_args* b, bool results) {
     const int64_t M = a.M, W = a.K;
     const pcb_span x_out = pcb_rows_span(n.x_out, M, W, W, 4);
     const pcb_span read[] = {n.table ? pcb_span{} : pcb_rows_span(n.x, 1, 0, (n.n_terms > 0 ? n.n_terms - 1 : 0) * n.x_stride + M * W, 4),
@@ -285,18 +273,34 @@ static bool norm_linear_apart(const pcb_row_norm_args& n, const pcb_linear_args&
     return !results || (pcb_results_apart(a, x_out) && (!b || pcb_results_apart(*b, x_out)));
 }
 
-static int norm_linear_route(const pcb_row_norm_args* n, const pcb_linear_args* a, const pcb_linear_args* b, Form* f) {
-    const int rc = norm_linear_check(n, a, b);
-    if (rc != PCB_OK) return rc;
-    PCB_REQUIRE(norm_linear_apart(*n, *a, b, false), PCB_ERR_ARG, "pcb_norm_linear: x_out overlaps the rows that are read");
-    const uintptr_t e4 = a->dtype == PCB_BF16 ? 8 : 16;              // (four elements of E)
+// Whether what the rows are made of, and the products, can be read in pieces, and the results go where these kernels put them
+bool pcb_norm_linear_pieces(const pcb_row_norm_args& n, const pcb_linear_args& a, const pcb_linear_args* b) {
+    const uintptr_t e4 = a.dtype == PCB_BF16 ? 8 : 16;              // (four elements of E)
     auto takes = [](const pcb_linear_args& q) { return q.n_batch == 0 && !q.row_src && !q.row_dst && !q.row_gate && q.split_n3 <= 0 && pcb_linear_pieces(q); };
-    const bool pieces = a->epilogue == PCB_EPI_STORE && takes(*a) && a->K % 64 == 0 &&
-                        (!b || (takes(*b) && (b->epilogue == PCB_EPI_STORE || (b->epilogue == PCB_EPI_SILU_MUL && n->y)))) && n->x_stride % 4 == 0 && n->ldg % 4 == 0 &&
-                        ((uintptr_t)n->x | (uintptr_t)n->y | (uintptr_t)n->post_gain | (uintptr_t)n->gain | (uintptr_t)n->gain2 | (uintptr_t)n->x_out) % 16 == 0 &&
-                        ((uintptr_t)n->gate | (uintptr_t)n->table) % e4 == 0;
+    return a.epilogue == PCB_EPI_STORE && takes(a) && a.K % 64 == 0 &&
+           (!b || (takes(*b) && (b->epilogue == PCB_EPI_STORE || (b->epilogue == PCB_EPI_SILU_MUL && n.y)))) && n.x_stride % 4 == 0 && n.ldg % 4 == 0 &&
+           ((uintptr_t)n.x | (uintptr_t)n.y | (uintptr_t)n.post_gain | (uintptr_t)n.gain | (uintptr_t)n.gain2 | (uintptr_t)n.x_out) % 16 == 0 &&
+           ((uintptr_t)n.gate | (uintptr_t)n.table) % e4 == 0;
+}
+
+int pcb_norm_linear_check(const pcb_row_norm_args* n, const pcb_linear_args* a, const pcb_linear_args* b) {
+    int rc = pcb_linear_check(a);
+    if (rc == PCB_OK && b) rc = pcb_linear_check(b);
+    if (rc != PCB_OK) return rc;
+    PCB_REQUIRE(n && n->struct_bytes == sizeof(pcb_row_norm_args), PCB_ERR_ARG, "pcb_norm_linear: struct size mismatch");
+    PCB_REQUIRE(n->x_out && n->gain && (!b || n->gain2) && (n->table ? n->ids && n->vocab > 0 && !n->y : n->x && n->x != n->x_out) &&
+                    (n->table || n->y ? n->n_terms == 0 : n->n_terms > 0 && n->coef) && (!n->y || (n->gate && n->post_gain && n->ldg >= a->K)),
+                PCB_ERR_ARG, "pcb_norm_linear: rows of a table, a sum of streams, or a residual and a gated sublayer's result; x_out is neither's");
+    PCB_REQUIRE(!b || (a->dtype == b->dtype && a->M == b->M && a->K == b->K), PCB_ERR_ARG, "pcb_norm_linear: products of the same rows");
+    PCB_REQUIRE(pcb_norm_linear_apart(*n, *a, b, false), PCB_ERR_ARG, "pcb_norm_linear: x_out overlaps the rows that are read");
+    return PCB_OK;
+}
+
+static int norm_linear_route(const pcb_row_norm_args* n, const pcb_linear_args* a, const pcb_linear_args* b, Form* f) {
+    const int rc = pcb_norm_linear_check(n, a, b);
+    if (rc != PCB_OK) return rc;
     *f = form(*n, *a, b);
-    return pieces && f->taken && norm_linear_apart(*n, *a, b, true) ? PCB_OK : PCB_NOT_TAKEN;
+    return f->taken && pcb_norm_linear_pieces(*n, *a, b) && pcb_norm_linear_apart(*n, *a, b, true) ? PCB_OK : PCB_NOT_TAKEN;
 }
 
 PCB_EXPORT int pcb_norm_linear_takes(const pcb_row_norm_args* n, const pcb_linear_args* a, const pcb_linear_args* b) {

@@ -151,3 +151,9 @@ inline bool pcb_results_apart(const pcb_linear_args& a, const pcb_span& s) {
     return (a.row_dst || pcb_apart(pcb_rows_span(a.y, a.M, a.ldy, cols, es), s)) &&
            (!a.y2_f32 || a.split_n <= 0 || pcb_apart(pcb_rows_span(a.y2, a.M, a.head_stride2, a.N - a.split_n, 4), s));
 }
+
+// What pcb_norm_linear and pcb_norm_stream ask of their arguments (pb_linear_normed.hip): PCB_OK when they are valid; whether their kernels can read and place them;
+// whether x_out (results: what the products store) lies apart from what the rows are made of
+int pcb_norm_linear_check(const pcb_row_norm_args* n, const pcb_linear_args* a, const pcb_linear_args* b);
+bool pcb_norm_linear_pieces(const pcb_row_norm_args& n, const pcb_linear_args& a, const pcb_linear_args* b);
+bool pcb_norm_linear_apart(const pcb_row_norm_args& n, const pcb_linear_args& a, const pcb_linear_args* b, bool results);

@@ -17,7 +17,7 @@ _lib: Optional[C.CDLL] = None
 BF16, F32 = 0, 1
 EPI_STORE, EPI_SILU_MUL, EPI_SCALE_ADD = 0, 1, 2
 ACT_NONE, ACT_SILU, ACT_SIGMOID, ACT_RELU2, ACT_SOFTPLUS, ACT_SOFTCAP, ACT_RELU, ACT_GELU_TANH, ACT_LOGSIGMOID, ACT_SCALE = range(10)
-NOT_TAKEN, NORM_LINEAR_MAX = 1, 4096                               # (what norm_linear takes: rows x columns)
+NOT_TAKEN, NORM_LINEAR_MAX = 1, 16384                              # (what norm_linear takes: rows x columns)
 NORM_NONE, NORM_RMS, NORM_DYT = 0, 1, 2
 SCORE_SIGMOID, SCORE_SOFTMAX = 0, 1
 ABI_VERSION = 6
@@ -217,6 +217,8 @@ SIGNATURES = {
     "pcb_linear_parts_form": (C.c_int, [C.POINTER(LinearArgs)]),
     "pcb_norm_linear": (C.c_int, [C.POINTER(RowNormArgs), C.POINTER(LinearArgs), C.POINTER(LinearArgs), _vp]),
     "pcb_norm_linear_takes": (C.c_int, [C.POINTER(RowNormArgs), C.POINTER(LinearArgs), C.POINTER(LinearArgs)]),
+    "pcb_norm_stream": (C.c_int, [C.POINTER(RowNormArgs), C.POINTER(LinearArgs), C.POINTER(LinearArgs), _vp]),
+    "pcb_norm_stream_takes": (C.c_int, [C.POINTER(RowNormArgs), C.POINTER(LinearArgs), C.POINTER(LinearArgs)]),
     "pcb_linear_pair": (C.c_int, [C.POINTER(LinearArgs), C.POINTER(LinearArgs), _vp]),
     "pcb_linear_pair_form": (C.c_int, [C.POINTER(LinearArgs), C.POINTER(LinearArgs)]),
     "pcb_linear_add2": (C.c_int, [C.POINTER(LinearArgs), C.POINTER(LinearArgs), _vp, _vp, _f32, _vp]),
@@ -469,10 +471,10 @@ def linear_add2(a: LinearArgs, b: LinearArgs, z: Optional[torch.Tensor] = None, 
 
 
 def norm_linear(a: LinearArgs, b: Optional[LinearArgs], gain: torch.Tensor, gain2: Optional[torch.Tensor], x_out: torch.Tensor, *, eps: float, x=None, coef=None,
-                n_terms: int = 0, table=None, ids=None, scale: float = 1.0, y=None, gate=None, ldg: int = 0, post_gain=None) -> bool:
+                n_terms: int = 0, table=None, ids=None, scale: float = 1.0, y=None, gate=None, ldg: int = 0, post_gain=None, many: bool = False) -> bool:
     """Residual rows -- of a ``table``, the sum of ``n_terms`` streams ``x`` [streams, rows, width], or ``x`` and a gated sublayer's result ``y`` behind its norm
     -- into ``x_out``, and one or two products (``linear_args``) of the normed rows.  False: not what one launch takes (sizes, or results that overlap the rows
-    read), nothing done."""
+    read), nothing done.  ``many``: many columns, as of a vocabulary (the form for few of them is not asked)."""
     M, W = a.M, a.K
     for t, nm in ((gain, "gain"), (gain2, "gain2"), (x_out, "x_out"), (x, "x"), (coef, "coef"), (y, "y"), (post_gain, "post_gain")):
         _want(t, torch.float32, "norm_linear " + nm)
@@ -487,7 +489,10 @@ def norm_linear(a: LinearArgs, b: Optional[LinearArgs], gain: torch.Tensor, gain
         assert x.dim() == 3 and x.shape[0] >= n_terms and x.shape[1] >= M and x.shape[2] == W and coef.numel() >= n_terms
     n = RowNormArgs(C.sizeof(RowNormArgs), _p(x), x.stride(0) if n_terms else 0, _p(coef), n_terms, _p(table), _p(ids), table.shape[0] if table is not None else 0,
                     float(scale), _p(y), _p(gate), ldg, _p(post_gain), _p(gain), _p(gain2), _p(x_out), float(eps))
-    rc = load().pcb_norm_linear(C.byref(n), C.byref(a), None if b is None else C.byref(b), _stream())
+    args = (C.byref(n), C.byref(a), None if b is None else C.byref(b), _stream())
+    rc = NOT_TAKEN if many else load().pcb_norm_linear(*args)
+    if rc == NOT_TAKEN:
+        rc = load().pcb_norm_stream(*args)
     if rc != NOT_TAKEN:
         check(rc, "pcb_norm_linear")
     return rc != NOT_TAKEN

@@ -347,7 +347,7 @@ class FivesunHIP(SlotModel):
             np.add(st.row_slot * (g * cap * d), st.row_pos * d, out=offs[k])
         dims = dict(T=T, R=R, n_want=int(want_rows.size), n32=n32, o64=o64, sizes=sizes, tile=tile, ones=max(counts) == 1,
                     longest=max((starts[b] + counts[b] for b in {*big, *rebuilt}), default=0),
-                    seg=min(seg, max(counts)) if chunks else 0)
+                    seg=min(seg, max(counts)) if chunks else 0, every=want_rows.size == T and bool((want_rows == np.arange(T)).all()))
         res = self._decode_graphed(arena, blob, dims) if graphed else None
         if res is None:
             dblob = torch.from_numpy(blob).to(dev)
@@ -438,8 +438,11 @@ class FivesunHIP(SlotModel):
         if d["n_want"]:
             nw = d["n_want"]
             hn = self._mat("hn", nw, W, E)
+            logit = B.linear_args(hn, self.head, logits, M=nw)
+            if few and pending and d["every"] and B.norm_linear(logit, None, self.final_norm, None, spare, eps=eps, x=x, many=True, **pending):
+                return (logits, streams) if return_streams else logits
             step(self.final_norm, hn, rows=tb["want"], n_rows=nw)
-            B.linear(hn, self.head, logits, M=nw)
+            B.linear_run(logit)
         return (logits, streams) if return_streams else logits
 
     # ---- mixers (each gets its projected rows P, leaves its result in y, fp32 [T, W], and returns where the residual gate's sigmoid lies) --------------------

@@ -163,7 +163,7 @@ class KazolornHIP(SlotModel):
             dblob = torch.from_numpy(blob).to(dev)
             logits = torch.empty((n_want, V), dtype=f32, device=dev)
             res = self._run(arena, T, dblob, n32, o64, sigs, tiles, tiles.shape[0], tiles64.shape[0], n_want, max_kv, logits,
-                            num_layers, return_streams)
+                            num_layers, return_streams, every=n_want == T and bool((want_rows == np.arange(T)).all()))
         for s_, c in zip(slots, counts):
             arena.lengths[s_] += c
         if picked is not None:
@@ -171,9 +171,9 @@ class KazolornHIP(SlotModel):
         return res
 
     def _run(self, arena, T, dblob, n32, o64, sigs, tiles, n_tiles, n64, n_want, max_kv, logits, num_layers=None,
-             return_streams=False):
+             return_streams=False, every=False):
         """The device side of a step: every launch of the forward, reading the step's tables from ``dblob`` (token ids, the two
-        tile tables, wanted rows as int32, then the cache offsets of every row as int64)."""
+        tile tables, wanted rows as int32, then the cache offsets of every row as int64).  ``every``: the wanted rows are all rows, in order."""
         dev, E, f32 = self.device, self.dtype, torch.float32
         W, V = self.W, self.V
         d32 = dblob[:n32 * 4].view(torch.int32)
@@ -247,8 +247,11 @@ class KazolornHIP(SlotModel):
             streams[L - 1].copy_(x)
         if n_want:
             hn = self._mat("hn", n_want, W, E)
-            B.mix_norm(hist, L + 1, layers[-1]["dwa"], self.final_norm, hn, rows=want_d, eps=eps, n_rows=n_want)
-            B.linear(hn, self.head, logits, M=n_want)
+            logit = B.linear_args(hn, self.head, logits, M=n_want)
+            if not (every and T * W <= B.NORM_LINEAR_MAX and
+                    B.norm_linear(logit, None, self.final_norm, None, x, eps=eps, x=hist, coef=layers[-1]["dwa"], n_terms=L + 1, many=True)):
+                B.mix_norm(hist, L + 1, layers[-1]["dwa"], self.final_norm, hn, rows=want_d, eps=eps, n_rows=n_want)
+                B.linear_run(logit)
         return (logits, streams) if return_streams else logits
 
     # ---- decode steps as captured graphs -----------------------------------------------------------------------------------------
@@ -283,10 +286,10 @@ class KazolornHIP(SlotModel):
             saved, self._buf = self._buf, ent["bufs"]             # the graph owns its scratch: later, larger steps may regrow the shared one
             try:
                 args = (arena, T, ent["dev"], n32, o64, sigs, None, T, T, T, cap, ent["logits"])
-                self._run(*args)                                  # eager first: sizes every scratch buffer, and is this step's result
+                self._run(*args, every=True)                      # eager first: sizes every scratch buffer, and is this step's result
                 torch.cuda.synchronize()
                 with graph_capture(self.device) as g:
-                    self._run(*args)
+                    self._run(*args, every=True)
                 ent["graph"] = g
             finally:
                 self._buf = saved
