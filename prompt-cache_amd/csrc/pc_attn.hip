@@ -47,119 +47,144 @@ __device__ __forceinline__ int row_past_len(const AttnParams& p, int b) {
 #ifndef PC_TAIL_MAX
 #define PC_TAIL_MAX 32
 #endif
-constexpr int kTailMax = PC_TAIL_MAX;   // most rows of one prefill pass the tail workgroup handles (NT = 16 or 32 below)
+constexpr int kTailMax = PC_TAIL_MAX;   // most rows of one prefill pass the tail workgroup handles
 
-// The attention of <= NT new query rows over the <= NT rows their own pass appended (keys past_len + j, j <= qi), for one
-// head, as a split-KV partial (m, l, O) in the log2 domain.  All fp32 FMAs on (q_hi + q_lo), (K + K_lo), (V + V_lo): the
-// reference computes the pass in fp32 (llama2.py:361-388), only the STAGED rows are fp16 there.  It runs in the
-// workgroup of an extra split while the other splits stream the staged keys, so its 2-5 us hide under their ~10 us.
+// The attention of <= 16 RT new query rows over the rows their own pass appended (keys past_len + j, j <= qi), for one head, as a
+// split-KV partial (m, l, O) in the log2 domain.  Q, K and V are the 32-bit values that their two planes hold (the reference
+// computes the pass in fp32, llama2.py:361-388; only the STAGED rows are fp16 there): every score is the sum of all four
+// products of planes, P is split in three (11 bits each, so all of its 24) and meets both planes of V.
+// It runs in the workgroup of an extra split while the other splits stream the staged keys, so its time hides under theirs --
+// if it is short.  Bound by its chain (past length, rows, softmax, V back transposed), so the work is on the matrix cores:
+// wave = (row tile, share of the head's dims), K fragments straight from memory, V by LDS-DMA into a tile of 32 rows (hi, lo).
+// As fp32 FMAs on rows in LDS the 32-row form read five float4 of LDS for 16 FMAs and was the launch's last workgroup: us per
+// layer with the merge, 32 heads x 128, 308 / 936 / 1725 staged keys: 27 rows 14.2 -> 13.2, 14.6 -> 14.5, 16.2 -> 16.1, 100 staged keys 12.5 -> 9.0.
 // (Residual tiles inside the streaming kernel instead cost 32 VGPRs -- the second resident workgroup per CU, or spills --
 // and a straggler split: 13.3 -> 15.9 .. 25 us per launch on the persona prompt; the same arithmetic inside the merge
 // kernel lengthened the serial merge by 1.1 us per layer.)
-// 256 threads = NT rows x LPR lanes; a lane owns JPT = NT / LPR keys in the score phase and D / LPR output dims after it.
-// LDS: qs / ks / vs are [NT][D] fp32 (qs, ks with the float4 column XOR-swizzled by the row: the lanes of a row group
-// read different rows of one column; unswizzled they share a bank), ps is [NT][NT].
-template <int D, int NT, bool ALIBI, bool WT = false>   // WT: the partial leaves through write-through stores (fused merge)
-__device__ __forceinline__ void attn_tail_block(const AttnParams& p, float* __restrict__ qs, float* __restrict__ ks,
-                                                float* __restrict__ vs, float* __restrict__ ps, int b, int h, int split) {
-    constexpr int CPR = D / 8;             // 16-byte fp16 chunks per row
-    constexpr int F4R = D / 4;             // float4 columns per fp32 row
-    constexpr int SWZ = F4R >= 16 ? 15 : F4R - 1;
-    constexpr int LPR = kThreads / NT;     // lanes per query row (16 / 8)
-    constexpr int JPT = NT / LPR;          // keys per lane (1 / 4)
-    constexpr int DPT = D / LPR;           // output dims per lane in the O phase
-    static_assert(NT * LPR == kThreads && JPT * LPR == NT && DPT * LPR == D && DPT % 2 == 0, "tail thread map");
-    const int tid = threadIdx.x, q_len = p.q_len;
+constexpr int kTailKeys = 32;                                       // rows of the V tile (16 RT of them used)
+template <int D> constexpr int tail_halfs() { return 2 * kTailKeys * D; }
+template <int D, int RT, bool ALIBI, bool WT = false>   // WT: the partial leaves through write-through stores (fused merge)
+__device__ __forceinline__ void attn_tail_block(const AttnParams& p, _Float16* __restrict__ vt, int b, int h, int split) {
+    constexpr int KS = D / 32, DB = D / 16, CPR = D / 8;
+    constexpr int NP = 4 / RT, DPW = (DB + NP - 1) / NP;           // waves of a row tile, head-dim blocks of one of them
+    constexpr int VCH = 2 * kTailKeys * CPR / kThreads;            // 16-byte V chunks per thread, both planes
+    static_assert((RT == 1 || RT == 2) && VCH >= 1, "tail shape");
+    const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4, q_len = p.q_len;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), rt = wave % RT, part = wave / RT;
     const int past = row_past_len(p, 0);
     const int hkv = h / (p.H / p.Hkv);
     const _Float16* kb = p.k + b * p.kv_bs + (int64_t)hkv * p.kv_hs + (int64_t)past * D;
     const _Float16* vb = p.v + b * p.kv_bs + (int64_t)hkv * p.kv_hs + (int64_t)past * D;
     const _Float16* klb = p.k_lo + b * p.lo_bs + (int64_t)hkv * p.lo_hs;
     const _Float16* vlb = p.v_lo + b * p.lo_bs + (int64_t)hkv * p.lo_hs;
-    for (int idx = tid; idx < NT * CPR; idx += kThreads) {
-        const int row = idx / CPR, c = idx - row * CPR;
-        const int rc = row < q_len ? row : q_len - 1;          // clamped: unconditional loads
-        const int64_t qoff = b * p.q_bs + (int64_t)rc * p.q_ts + (int64_t)h * D + c * 8;
-        const h8 qh = *(const h8*)(p.q + qoff);
-        h8 ql = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (p.q_lo) ql = *(const h8*)(p.q_lo + qoff);
-        const h8 kk = *(const h8*)(kb + (int64_t)rc * D + c * 8), kl = *(const h8*)(klb + (int64_t)rc * D + c * 8);
-        const h8 vv = *(const h8*)(vb + (int64_t)rc * D + c * 8), vl = *(const h8*)(vlb + (int64_t)rc * D + c * 8);
+    // ---- every load first; rows behind the pass re-read its last one (their P is 0, and uninitialised rows could hold NaNs) ----
+    const int qi = rt * 16 + n, qc = qi < q_len ? qi : q_len - 1;
+    h8 qh[KS], ql[KS], kh[RT][KS], kl[RT][KS];
+    const int64_t qoff = b * p.q_bs + (int64_t)qc * p.q_ts + (int64_t)h * D + g * 8;
+    const _Float16* qlo = p.q_lo ? p.q_lo : p.q;                   // (no lo plane: a finite stand-in, zeroed below)
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            f4 q4, k4, v4;
+    for (int ks = 0; ks < KS; ++ks) {
+        qh[ks] = *(const h8*)(p.q + qoff + ks * 32);
+        ql[ks] = *(const h8*)(qlo + qoff + ks * 32);
+    }
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                q4[e] = (float)qh[half * 4 + e] + (float)ql[half * 4 + e];
-                k4[e] = (float)kk[half * 4 + e] + (float)kl[half * 4 + e];
-                v4[e] = (float)vv[half * 4 + e] + (float)vl[half * 4 + e];
+    for (int t = 0; t < RT; ++t) {
+        const int j = t * 16 + n < q_len ? t * 16 + n : q_len - 1;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            kh[t][ks] = *(const h8*)(kb + (int64_t)j * D + ks * 32 + g * 8);
+            kl[t][ks] = *(const h8*)(klb + (int64_t)j * D + ks * 32 + g * 8);
+        }
+    }
+    f4 kp[RT];
+    if constexpr (ALIBI) {
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int j = t * 16 + g * 4 + r;
+                kp[t][r] = p.slopes[h] * p.key_pos[b * p.kp_bs + past + (j < q_len ? j : q_len - 1)];
             }
-            const int col = ((2 * c + half) ^ (row & SWZ)) * 4;
-            *(f4*)(qs + row * D + col) = q4;
-            *(f4*)(ks + row * D + col) = k4;
-            *(f4*)(vs + row * D + (2 * c + half) * 4) = v4;      // read row-wise below: no swizzle
+    }
+    // V rows rotated by 32 B per row (see attn_fwd_kernel), first the hi plane's 32 rows, then the lo plane's
+#pragma unroll
+    for (int i = 0; i < VCH; ++i) {
+        const int c = (i * 4 + wave) * 64 + lane, prow = c / CPR, row = prow & (kTailKeys - 1), pos = c - prow * CPR;
+        const int col = (pos - 2 * (row & 7)) & (CPR - 1), rr = row < q_len ? row : q_len - 1;
+        const _Float16* src = prow < kTailKeys ? vb : vlb;
+        glds16(src + (int64_t)rr * D + col * 8, (char*)vt + (i * 4 + wave) * 1024);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (!p.q_lo) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) { h8 z = {0, 0, 0, 0, 0, 0, 0, 0}; ql[ks] = z; }
+    }
+    float sv[RT][4], m = kNegBig;
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        f4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl[t][ks], ql[ks], acc, 0, 0, 0);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl[t][ks], qh[ks], acc, 0, 0, 0);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[t][ks], ql[ks], acc, 0, 0, 0);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[t][ks], qh[ks], acc, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float s = acc[r] * p.scale_log2;
+            if (ALIBI) s += kp[t][r];
+            const bool vis = qi < q_len && t * 16 + g * 4 + r <= qi;          // causal inside the pass
+            sv[t][r] = vis ? s : kNegBig;
+            m = fmaxf(m, sv[t][r]);
         }
     }
-    __syncthreads();
-    const int qi = tid / LPR, jl = tid - qi * LPR;               // (query row, lane in the row group)
-    float acc[JPT];
-#pragma unroll
-    for (int u = 0; u < JPT; ++u) acc[u] = 0.f;
-#pragma unroll 8
-    for (int d4 = 0; d4 < F4R; ++d4) {
-        const f4 a = *(const f4*)(qs + qi * D + ((d4 ^ (qi & SWZ)) * 4));
-#pragma unroll
-        for (int u = 0; u < JPT; ++u) {
-            const int j = jl + u * LPR;
-            const f4 k4 = *(const f4*)(ks + j * D + ((d4 ^ (j & SWZ)) * 4));
-            acc[u] += a[0] * k4[0] + a[1] * k4[1] + a[2] * k4[2] + a[3] * k4[3];
-        }
-    }
-    float sv[JPT];
-    float m = kNegBig;
-#pragma unroll
-    for (int u = 0; u < JPT; ++u) {
-        const int j = jl + u * LPR;
-        sv[u] = acc[u] * p.scale_log2;
-        if (ALIBI) sv[u] += p.slopes[h] * p.key_pos[b * p.kp_bs + past + (j < q_len ? j : q_len - 1)];
-        const bool vis = qi < q_len && j <= qi;                  // causal inside the pass
-        sv[u] = vis ? sv[u] : kNegBig;
-        m = fmaxf(m, sv[u]);
-    }
-#pragma unroll
-    for (int off = LPR / 2; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+    m = fmaxf(m, __shfl_xor(m, 16));
+    m = fmaxf(m, __shfl_xor(m, 32));
     float l = 0.f;
+    h8 p0 = {0, 0, 0, 0, 0, 0, 0, 0}, p1 = p0, p2 = p0;            // P in three pieces; half t of the k-step = keys of row tile t
 #pragma unroll
-    for (int u = 0; u < JPT; ++u) {
-        const int j = jl + u * LPR;
-        const float pj = (qi < q_len && j <= qi) ? exp2f(sv[u] - m) : 0.f;
-        l += pj;
-        ps[qi * NT + j] = pj;
-    }
+    for (int t = 0; t < RT; ++t)
 #pragma unroll
-    for (int off = LPR / 2; off > 0; off >>= 1) l += __shfl_xor(l, off);
+        for (int r = 0; r < 4; ++r) {
+            const bool vis = qi < q_len && t * 16 + g * 4 + r <= qi;
+            const float e = vis ? exp2f(sv[t][r] - m) : 0.f;
+            l += e;
+            const _Float16 a0 = (_Float16)e;
+            const float e1 = e - (float)a0;
+            const _Float16 a1 = (_Float16)e1;
+            p0[t * 4 + r] = a0; p1[t * 4 + r] = a1; p2[t * 4 + r] = (_Float16)(e1 - (float)a1);
+        }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
     const int64_t slot = (((int64_t)b * p.H + h) * p.nsplit + split) * q_len + qi;
-    if (jl == 0 && qi < q_len) {
+    if (part == 0 && g == 0 && qi < q_len) {
         if (WT) st_wt2(p.part_ml + slot * 2, m, l);
         else { p.part_ml[slot * 2] = m; p.part_ml[slot * 2 + 1] = l; }
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // this wave's share of the V tile has landed, then everyone's
     __syncthreads();
-    float o[DPT];
 #pragma unroll
-    for (int e = 0; e < DPT; ++e) o[e] = 0.f;
-#pragma unroll 4
-    for (int jj = 0; jj < NT; ++jj) {
-        const float w = ps[qi * NT + jj];
-#pragma unroll
-        for (int e = 0; e < DPT; ++e) o[e] += w * vs[jj * D + jl * DPT + e];
-    }
-    if (qi < q_len) {
-        if (WT) {
-#pragma unroll
-            for (int e = 0; e < DPT; e += 2) st_wt2(p.part_o + slot * D + jl * DPT + e, o[e], o[e + 1]);
-        } else {
-#pragma unroll
-            for (int e = 0; e < DPT; ++e) p.part_o[slot * D + jl * DPT + e] = o[e];
+    for (int u = 0; u < DPW; ++u) {
+        const int db = part * DPW + u;
+        if (db >= DB) break;                                       // (wave-uniform)
+        const int vrow = g * 4 + (n >> 2);                         // (row + 16 has the same rotation)
+        const _Float16* vp = vt + vrow * D + ((db * 16 + (n & 3) * 4 + 16 * (vrow & 7)) & (D - 1));
+        const h4 h0 = lds_tr_read(vp), h1 = lds_tr_read(vp + 16 * D);
+        const h4 l0 = lds_tr_read(vp + kTailKeys * D), l1 = lds_tr_read(vp + (kTailKeys + 16) * D);
+        const h8 vh = {h0[0], h0[1], h0[2], h0[3], h1[0], h1[1], h1[2], h1[3]};
+        const h8 vl = {l0[0], l0[1], l0[2], l0[3], l1[0], l1[1], l1[2], l1[3]};
+        f4 o = {0.f, 0.f, 0.f, 0.f};
+        o = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, p2, o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, p1, o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, p0, o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, p1, o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, p0, o, 0, 0, 0);
+        if (qi < q_len) {
+            float* dst = p.part_o + slot * D + db * 16 + g * 4;
+            if constexpr (WT) { st_wt2(dst, o[0], o[1]); st_wt2(dst + 2, o[2], o[3]); }
+            else *(f4*)dst = o;
         }
     }
 }
@@ -197,12 +222,10 @@ __device__ __forceinline__ void attn_fwd_body(const AttnParams p) {
     constexpr int LPT = kTK * CPR / kThreads;  // 16-byte loads per thread per tile per tensor
     static_assert(LPT >= 1, "tile too small for 256 threads");
 
-    // (the split-precision variants without residual tiles also host attn_tail_block's fp32 buffers in these two)
-    constexpr int kKlElems = (HP && !KVLO && 4 * kTailMax * D > kTK * D) ? 4 * kTailMax * D : kTK * D;
-    constexpr int kVlElems = (HP && !KVLO && 2 * (kTailMax * D + kTailMax * kTailMax) > kTK * D)
-                                 ? 2 * (kTailMax * D + kTailMax * kTailMax) : kTK * D;
-    __shared__ __attribute__((aligned(16))) _Float16 Kl[kKlElems];
-    __shared__ __attribute__((aligned(16))) _Float16 Vl[kVlElems];
+    // (the split-precision variants without residual tiles also host attn_tail_block's V tile in the first)
+    static_assert(tail_halfs<D>() <= kTK * D, "the tail's V tile lives in the K tile");
+    __shared__ __attribute__((aligned(16))) _Float16 Kl[kTK * D];
+    __shared__ __attribute__((aligned(16))) _Float16 Vl[kTK * D];
     __shared__ __attribute__((aligned(16))) _Float16 Kll[KVLO ? kTK * D : 8];     // residual tiles (KVLO)
     __shared__ __attribute__((aligned(16))) _Float16 Vll[KVLO ? kTK * D : 8];
 
@@ -236,12 +259,8 @@ __device__ __forceinline__ void attn_fwd_body(const AttnParams p) {
         if (p.tail) {
             nsp = p.nsplit - 1;
             if (split == nsp) {           // workgroup-uniform: the extra split takes the pass's own rows
-                static_assert(sizeof(Kl) >= 2 * kTailMax * D * sizeof(float) &&
-                              sizeof(Vl) >= (kTailMax * D + kTailMax * kTailMax) * sizeof(float), "tail buffers live in the K / V tiles");
-                if (q_len <= 16 || kTailMax == 16)
-                    attn_tail_block<D, 16, ALIBI>(p, (float*)Kl, (float*)Kl + 16 * D, (float*)Vl, (float*)Vl + 16 * D, b, h, split);
-                else
-                    attn_tail_block<D, kTailMax, ALIBI>(p, (float*)Kl, (float*)Kl + kTailMax * D, (float*)Vl, (float*)Vl + kTailMax * D, b, h, split);
+                if (q_len <= 16) attn_tail_block<D, 1, ALIBI>(p, Kl, b, h, split);
+                else attn_tail_block<D, 2, ALIBI>(p, Kl, b, h, split);
                 return;
             }
         }
@@ -873,7 +892,7 @@ __device__ __forceinline__ void small_arrive_merge(const AttnParams& p, int b, i
 // (The launch is sized to ONE workgroup per CU -- small_nstream -- so the staging variant, which keeps the K fragments alive until
 // they are stored, takes the registers of a one-wave-per-SIMD kernel instead of spilling at 256.)
 // RT: 16-row tiles of query rows per wave (1: <= 16 new rows; 2: 17..32 -- every K fragment and V tile read serves both tiles;
-// one workgroup per CU, as the staging variant).
+// one workgroup per CU, as the staging variant).  p.small_rt = 2: 17..32 rows as RT = 1, a workgroup for each row tile.
 template <int D, bool ALIBI, int NS, bool GATHER = false, int RT = 1>
 __global__ __launch_bounds__(kThreads, (GATHER || RT > 1) ? 1 : 2) void attn_small_kernel(const AttnParams p) {
     constexpr bool FUSE = NS > 0;
@@ -882,10 +901,9 @@ __global__ __launch_bounds__(kThreads, (GATHER || RT > 1) ? 1 : 2) void attn_sma
     constexpr int KS = D / 32, DB = D / 16, CPR = D / 8;
     constexpr int LPW = kTK * CPR / 64;              // 16-byte V chunks per lane per tile
     constexpr int kTileHalfs = kTK * D;
-    constexpr int kTailRows = 16 * RT;
-    constexpr int kTailBytes = (2 * kTailRows * D + kTailRows * D + kTailRows * kTailRows) * 4;
+    static_assert(tail_halfs<D>() <= 4 * kTileHalfs, "the tail's V tile lives in the waves' tiles");
     constexpr int kMergeBytes = RT * (4 * (D / 16) * 64 * 4 + 4 * 16 * 2) * 4;      // the four waves' (O, m, l) per row tile
-    constexpr int kLds0 = 4 * kTileHalfs * 2 > kTailBytes ? 4 * kTileHalfs * 2 : kTailBytes;
+    constexpr int kLds0 = 4 * kTileHalfs * 2;
     constexpr int kLdsBytes = kLds0 > kMergeBytes ? kLds0 : kMergeBytes;
     constexpr int kTabBytes = GATHER ? 4 * kTK * 16 : 0;           // row-table entries of the four waves' tiles
     __shared__ __attribute__((aligned(16))) char smem[kLdsBytes + 16 + kTabBytes];
@@ -894,19 +912,22 @@ __global__ __launch_bounds__(kThreads, (GATHER || RT > 1) ? 1 : 2) void attn_sma
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = blockIdx.y;
-    const int b = blockIdx.z / p.nsplit, split = blockIdx.z - b * p.nsplit;
+    const int nz = p.nbatch * p.nsplit, tile0 = RT == 1 ? blockIdx.z / nz : 0;       // (small_rt: one row tile a workgroup)
+    const int bz = (int)blockIdx.z - tile0 * nz;
+    const int b = bz / p.nsplit, split = bz - b * p.nsplit;
     const int hkv = h / (p.H / p.Hkv);
     const int q_len = p.q_len;
     const int past_len = row_past_len(p, 0);
     const int nstream = p.tail ? p.nsplit - 1 : p.nsplit;
     auto stamp = [&](int slot) {
-        if (p.trace && lane == 0)
-            p.trace[((((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * 4 + wave) * 4) + slot] = wall_clock64();
+        if (p.trace && lane == 0 && tile0 == 0)
+            p.trace[((((int64_t)bz * gridDim.y + blockIdx.y) * 4 + wave) * 4) + slot] = wall_clock64();
     };
     stamp(0);
-    if (p.tail && split == nstream) {                 // workgroup-uniform: the pass's own rows, fp32
-        float* f = (float*)smem;
-        attn_tail_block<D, kTailRows, ALIBI, FUSE>(p, f, f + kTailRows * D, f + 2 * kTailRows * D, f + 3 * kTailRows * D, b, h, split);
+    if (p.tail && split == nstream) {                 // workgroup-uniform: the pass's own rows
+        if (tile0 > 0) return;                        // (the first row tile's workgroup takes both)
+        if (RT == 2 || (!FUSE && q_len > kSmallQ)) attn_tail_block<D, 2, ALIBI, FUSE>(p, (_Float16*)smem, b, h, split);
+        else attn_tail_block<D, 1, ALIBI, FUSE>(p, (_Float16*)smem, b, h, split);
         if constexpr (FUSE) small_arrive_merge<D, NS>(p, b, h, s_last);
         return;
     }
@@ -918,7 +939,7 @@ __global__ __launch_bounds__(kThreads, (GATHER || RT > 1) ? 1 : 2) void attn_sma
     int qi[RT], row_vis_end[RT];                                   // this lane's query row of each row tile
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-        qi[rt] = rt * 16 + n;
+        qi[rt] = (tile0 + rt) * 16 + n;
         row_vis_end[rt] = qi[rt] < q_len ? (p.tail ? past_len : past_len + qi[rt] + 1) : 0;
     }
 
@@ -956,7 +977,7 @@ __global__ __launch_bounds__(kThreads, (GATHER || RT > 1) ? 1 : 2) void attn_sma
     _Float16* Vw = (_Float16*)smem + wave * kTileHalfs;            // this wave's V tile
     char* Vwb = smem + wave * kTileHalfs * 2;                      // (the same, as the wave-uniform LDS-DMA base)
     [[maybe_unused]] u32x4* etab = (u32x4*)(smem + kLdsBytes + 16) + wave * kTK;   // GATHER: this wave's 64 row-table entries
-    [[maybe_unused]] const bool g_writer = GATHER && (h % (p.H / p.Hkv)) == 0;        // one query head per kv head stages
+    [[maybe_unused]] const bool g_writer = GATHER && (h % (p.H / p.Hkv)) == 0 && tile0 == 0;   // one query head per kv head stages
     [[maybe_unused]] const uint64_t g_koff = GATHER ? (uint64_t)(uint32_t)(p.g_kplane + hkv) : 0;
     [[maybe_unused]] const uint64_t g_voff = GATHER ? (uint64_t)(uint32_t)(p.g_vplane + hkv) : 0;
 
@@ -1032,7 +1053,10 @@ __global__ __launch_bounds__(kThreads, (GATHER || RT > 1) ? 1 : 2) void attn_sma
                     acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qfl[rt][ks], acc, 0, 0, 0);
                 }
                 f4 kb4 = {0.f, 0.f, 0.f, 0.f};
-                if (ALIBI) kb4 = *(const f4*)(kpos + key0 + kb * 16 + g * 4);
+                if (ALIBI) {                             // (keys past k1 are masked: no position behind their group of four is read)
+                    const int at = key0 + kb * 16 + g * 4, last = (k1 - 1) & ~3;
+                    kb4 = *(const f4*)(kpos + (at < last ? at : last));
+                }
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int key = key0 + kb * 16 + g * 4 + r;
@@ -1165,13 +1189,18 @@ __global__ __launch_bounds__(kThreads, (GATHER || RT > 1) ? 1 : 2) void attn_sma
 // Streaming workgroups per head of attn_small_kernel (each = 4 key slices): ONE workgroup per CU in total, the tail workgroup
 // of each head included -- 8 + 1 splits x 32 heads = 288 workgroups put a second workgroup on 32 of the 256 CUs and the launch
 // waits for those: 7 + 1 (exactly 256) runs the persona step 1.7 % faster end to end (3.908 -> 3.844 ms, profiles/r03_*).
-int small_nstream(int B, int H, int tail = 0) {
+// Fewer over a short cache: a wave of three streams has one tile up to 768 keys, as one of seven has, and every stream more is a
+// partial of all rows that is written and merged.  us with the merge, 32 heads, all / fewer: 308 keys, 3 rows 8.7 / 8.3, 12 rows
+// 9.7 / 8.8, 27 rows 13.2 / 11.9, 700 keys 9.2 / 9.0, 10.2 / 9.5, 13.6 / 12.5, 936 keys, 16 rows 11.3 / 10.8; one row 308 keys 8.0 / 8.3,
+// two rows 700 keys 9.0 / 9.2, 1200 keys, 4 rows 11.2 / 11.5 (five streams; 8 heads, 936 keys 9.1 / 9.4).
+int small_nstream(int B, int H, int tail = 0, int q_len = 1, int keys = 1 << 20) {
     static const int forced = [] { const char* e = getenv("PC_ATTN_SMALL_WG"); return e ? atoi(e) : 0; }();
     if (forced > 0) return forced < 15 ? forced : 15;
     int ns = 256 / (B * H) - tail;
     if (ns < 1) ns = 1;
     if (ns > 15) ns = 15;
-    return ns;
+    const int few = keys <= 768 && q_len >= 3 ? 3 : keys <= 1024 && q_len >= kSmallQ ? 5 : ns;
+    return ns < few ? ns : few;
 }
 
 // Merge split-KV partials: out = sum_i 2^(m_i - m*) O_i / sum_i 2^(m_i - m*) l_i.
@@ -1270,7 +1299,7 @@ int choose_nsplit(int B, int H, int q_len, int kv_len, bool hp) {
     return ns;
 }
 
-// Streaming splits of a tail-mode launch of the 64-row kernel (<= 32 new rows, their own keys in the tail workgroup's fp32 pass):
+// Streaming splits of a tail-mode launch of the 64-row kernel (<= 32 new rows, their own keys in the tail workgroup):
 // the merge launch runs anyway, the streams cover the staged keys only, and what a short question over a SHORT cache pays is the
 // serial walk of one workgroup over its key tiles -- choose_nsplit's "two tiles per split at least" left 5 tiles to one workgroup
 // at 300 staged keys.  Here: as many streams as there are tiles while the grid stays within two workgroups per CU, then the
@@ -1299,7 +1328,7 @@ int launch_attn(const AttnParams& p0, int B, hipStream_t stream) {
     p.nqblk = pc_ceil_div(p.q_len, rows32 ? kQB32 : kQB);
     p.nbatch = B;
     p.xcd_remap = (!p.small && p.nsplit == 1 && p.nqblk >= (rows32 ? 2 : 4) && !no_remap) ? 1 : 0;
-    dim3 grid(p.nqblk, p.H, B * p.nsplit);
+    dim3 grid(p.nqblk, p.H, B * p.nsplit * (p.small ? p.small_rt : 1));
     if (p.xcd_remap) grid = dim3(8 * p.nqblk * ((p.H * B + 7) / 8), 1, 1);
     const bool ring = D == 128 && ring_eligible(p, D);      // (attn_fwd_impl chose p.nsplit for it)
 #ifdef PC_DEV_SWEEPS      // (the merge inside the launch: built, bit-reproducible, and no faster than the second launch in three rounds of
@@ -1324,11 +1353,12 @@ int launch_attn(const AttnParams& p0, int B, hipStream_t stream) {
         if (rrc != PC_OK) return rrc;
     } else if (p.small && p.rows) {       // stage while reading (pc_attn gather_rows)
         if (p.key_pos) hipLaunchKernelGGL((attn_small_kernel<D, true, 0, true>), grid, dim3(kThreads), 0, stream, p);
-        else if (p.q_len > kSmallQ) hipLaunchKernelGGL((attn_small_kernel<D, false, 0, true, 2>), grid, dim3(kThreads), 0, stream, p);
+        else if (p.q_len > kSmallQ * p.small_rt) hipLaunchKernelGGL((attn_small_kernel<D, false, 0, true, 2>), grid, dim3(kThreads), 0, stream, p);
         else hipLaunchKernelGGL((attn_small_kernel<D, false, 0, true>), grid, dim3(kThreads), 0, stream, p);
     } else if (p.small) {
-        if (p.key_pos) hipLaunchKernelGGL((attn_small_kernel<D, true, 0>), grid, dim3(kThreads), 0, stream, p);
-        else if (p.q_len > kSmallQ) hipLaunchKernelGGL((attn_small_kernel<D, false, 0, false, 2>), grid, dim3(kThreads), 0, stream, p);
+        if (p.key_pos && p.q_len > kSmallQ * p.small_rt) hipLaunchKernelGGL((attn_small_kernel<D, true, 0, false, 2>), grid, dim3(kThreads), 0, stream, p);
+        else if (p.key_pos) hipLaunchKernelGGL((attn_small_kernel<D, true, 0>), grid, dim3(kThreads), 0, stream, p);
+        else if (p.q_len > kSmallQ * p.small_rt) hipLaunchKernelGGL((attn_small_kernel<D, false, 0, false, 2>), grid, dim3(kThreads), 0, stream, p);
         else hipLaunchKernelGGL((attn_small_kernel<D, false, 0>), grid, dim3(kThreads), 0, stream, p);
     } else if (rows32) {
         if (p.key_pos) hipLaunchKernelGGL((attn_fwd32_kernel<D, true>), grid, dim3(kThreads), 0, stream, p);
@@ -1449,7 +1479,7 @@ int attn_fwd_impl(const void* q, const void* q_lo, int64_t q_batch_stride, int64
     p.H = H; p.Hkv = Hkv; p.q_len = q_len; p.past_len = past_len;
     p.scale_log2 = softmax_scale * 1.4426950408889634f;
     p.nsplit = choose_nsplit(B, H, q_len, past_len + q_len, q_len <= kQB || q_lo != nullptr);
-    p.tail = 0; p.small = 0;
+    p.tail = 0; p.small = 0; p.small_rt = 1;
     // (a pass the ring kernel takes carries its own rows as residual tiles in the stream: no fp32 tail workgroup)
     const bool ring_first = ring_eligible(p, D);
     p.tail = (!ring_first && k_lo && lo_row0 == -1 && q_len <= kTailMax && !past_lens) ? 1 : 0;
@@ -1457,13 +1487,18 @@ int attn_fwd_impl(const void* q, const void* q_lo, int64_t q_batch_stride, int64
     // launches that carry residual tiles in the stream (decode over a residual tail, lo_row0 != -1).
     static const bool small_off = [] { const char* e = getenv("PC_ATTN_NO_SMALL"); return e && e[0] == '1'; }();
     // 17..32 rows in tail mode take the same kernel with two row tiles per wave (every K fragment and V tile serves both;
-    // two-launch form, no ALiBi instantiation); PC_ATTN_SMALL2=0: the 64-row kernel, as in rounds 1-3
+    // two-launch form); PC_ATTN_SMALL2=0: the 64-row kernel, as in rounds 1-3
     static const bool small2_off = [] { const char* e = getenv("PC_ATTN_SMALL2"); return e && e[0] == '0'; }();
-    const bool small2 = !small2_off && q_len > kSmallQ && q_len <= 2 * kSmallQ && p.tail && !key_pos && !counters;
+    const bool small2 = !small2_off && q_len > kSmallQ && q_len <= 2 * kSmallQ && p.tail && !counters;
     bool small = !small_off && (q_len <= kSmallQ || small2) && !past_lens && (!k_lo || p.tail) && past_len + q_len >= 256;
     if (small) {
-        const int ns = small_nstream(B, H, p.tail) + p.tail;
+        const int ns = small_nstream(B, H, p.tail, q_len, p.tail ? past_len : past_len + q_len) + p.tail;
         if (ns >= 2) p.nsplit = ns; else small = false;
+        // A workgroup for each row tile while these are at most a round and a quarter of the CUs: two row tiles in one are a chain of
+        // twice the products and merges for the same keys.  us with the merge, 27 rows, one workgroup / two: 32 heads, 308 keys 11.8 /
+        // 9.5, 700 12.5 / 10.1, 40 heads 12.2 / 11.4, 13.5 / 12.9; behind that (32 heads, 936 keys 13.8 / 13.7, 2500 20.7 / 21.7) the same
+        // keys cross the chip twice.
+        if (q_len > kSmallQ && 2 * B * H * p.nsplit <= 320) p.small_rt = 2;
     }
     p.small = small ? 1 : 0;
     // staging while reading lives in attn_small_kernel's two-launch form and in the tail-mode instantiation of the 64-row kernel
@@ -1471,7 +1506,9 @@ int attn_fwd_impl(const void* q, const void* q_lo, int64_t q_batch_stride, int64
     const bool mid_gather = !small && p.tail && !ring_first && !key_pos && !pre_k && q_len <= kQB;
     // ... and in the ring kernel (more than 32 split-precision rows at head_dim 128, no shared prefix, one past length)
     const bool ring_gather = !small && ring_eligible(p, D) && !pre_k && !past_lens;
-    const bool can_gather = (small || mid_gather || ring_gather) && (small ? !counters : true) && B == 1 && past_len > 0;
+    // (17..32 rows with ALiBi: no staging form)
+    const bool small_gather = small && !(key_pos && q_len > kSmallQ);
+    const bool can_gather = (small_gather || mid_gather || ring_gather) && (small ? !counters : true) && B == 1 && past_len > 0;
     if (gather_ok) { *gather_ok = can_gather ? 1 : 0; return PC_OK; }
     PC_REQUIRE(!gather_rows || can_gather, PC_ERR_ARG,
                "pc_attn: gather_rows needs B = 1 and a launch of <= %d query rows in tail mode, <= %d rows over >= 256 keys without counters, or a split-precision launch of >= %d rows at head_dim 128 (ask pc_attn_gather_ok)", kTailMax, kSmallQ, ring_min_rows());

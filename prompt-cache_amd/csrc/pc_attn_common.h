@@ -50,9 +50,10 @@ struct AttnParams {
     int32_t H, Hkv, q_len, past_len, nsplit;
     // tail != 0 (lo_row0 < 0 and q_len <= kTailMax: prefill of a short prompt over a staged cache): splits
     // 0 .. nsplit-2 stream the STAGED keys [0, past_len) only; the workgroup of split nsplit-1 computes the attention over
-    // the rows this pass appended in fp32 (attn_tail_block) and leaves it as one more partial for the merge kernel.
+    // the rows this pass appended (attn_tail_block) and leaves it as one more partial for the merge kernel.
     int32_t tail;
     int32_t small;          // attn_small_kernel launch (host-side dispatch flag)
+    int32_t small_rt;       // ... workgroups per stream of keys, 16 query rows each (2: 17..32 rows, a row tile a workgroup)
     int32_t formal_handoff; // fused merge: acq_rel arrival (the C++-memory-model form, env PC_FORMAL_HANDOFF=1) instead of relaxed + vmcnt(0)
     int32_t xcd_remap, nqblk, nbatch;
     // (host) the staged keys go to attn_wide_kernel in `nsplit - 1` slices, the keys this pass appended to attn_ring_kernel in its
