@@ -224,7 +224,7 @@ class DibizenHIP(SlotModel):
                     n_chains=chains.shape[0])
         res = self._decode_graphed(arena, blob, dims) if graphed else None
         if res is None:
-            dblob = torch.from_numpy(blob).to(dev)
+            dblob = self._upload(blob)
             logits = torch.empty((dims["n_want"], V), dtype=f32, device=dev)
             res = self._run(arena, dblob, dims, logits, num_layers, return_streams)
         for s_, c in zip(slots, counts):

@@ -350,7 +350,7 @@ class FivesunHIP(SlotModel):
                     seg=min(seg, max(counts)) if chunks else 0, every=want_rows.size == T and bool((want_rows == np.arange(T)).all()))
         res = self._decode_graphed(arena, blob, dims) if graphed else None
         if res is None:
-            dblob = torch.from_numpy(blob).to(dev)
+            dblob = self._upload(blob)
             logits = torch.empty((dims["n_want"], self.V), dtype=torch.float32, device=dev)
             res = self._run(arena, dblob, dims, logits, num_layers, return_streams)
         for s_, c in zip(slots, counts):

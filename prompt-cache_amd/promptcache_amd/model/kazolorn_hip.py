@@ -23,6 +23,7 @@ and the logits are ``head . rms(sum_j dwa_last[j] X_j) g`` for the rows that wer
 from __future__ import annotations
 
 import os
+from itertools import chain
 from typing import Dict, List, Optional, Sequence
 
 import numpy as np
@@ -126,25 +127,31 @@ class KazolornHIP(SlotModel):
         W, V = self.W, self.V
 
         # host-side tables of the step, one upload
-        ids = np.fromiter((t for req in tokens for t in req), dtype=np.int32, count=T)
+        ids = np.fromiter(chain.from_iterable(tokens), dtype=np.int32, count=T)
         if ids.size and (ids.min() < 0 or ids.max() >= V):
             raise ValueError("token id outside the vocabulary")
-        row_slot = np.repeat(np.asarray(slots, dtype=np.int64), counts)
-        row_pos = np.concatenate([np.arange(st, st + c, dtype=np.int64) for st, c in zip(starts, counts)])
-        row0 = np.concatenate([[0], np.cumsum(counts)])
-        tiles = []
-        for b, (s, st, c) in enumerate(zip(slots, starts, counts)):
-            for q in range(0, c, 16):
-                tiles.append((s, st + q, min(16, c - q), int(row0[b]) + q))
-        tiles = np.asarray(tiles, dtype=np.int32).reshape(-1, 4)
-        tiles64 = np.asarray([(s, st + q, min(64, c - q), int(row0[b]) + q) for b, (s, st, c) in enumerate(zip(slots, starts, counts))
-                              for q in range(0, c, 64)], dtype=np.int32).reshape(-1, 4)
         for b, ws in enumerate(want):
             if any(not 0 <= int(w) < counts[b] for w in ws):
                 raise ValueError("a wanted place lies outside its request's tokens")
         # one-token steps run as a captured graph whose launches have fixed sizes: logits of every row, picked from afterwards
         graphed = (self.use_graphs and T <= self.GRAPH_MAX_ROWS and all(c == 1 for c in counts) and num_layers is None
                    and not return_streams)
+        if graphed:                                               # (a row of its own for each request: no loops over tiles)
+            row_slot, row_pos, row0 = np.asarray(slots, dtype=np.int64), np.asarray(starts, dtype=np.int64), range(T)
+            tiles = np.empty((T, 4), dtype=np.int32)
+            tiles[:, 0], tiles[:, 1], tiles[:, 2], tiles[:, 3] = row_slot, row_pos, 1, row0
+            tiles64 = tiles
+        else:
+            row_slot = np.repeat(np.asarray(slots, dtype=np.int64), counts)
+            row_pos = np.concatenate([np.arange(st, st + c, dtype=np.int64) for st, c in zip(starts, counts)])
+            row0 = np.concatenate([[0], np.cumsum(counts)])
+            tiles = []
+            for b, (s, st, c) in enumerate(zip(slots, starts, counts)):
+                for q in range(0, c, 16):
+                    tiles.append((s, st + q, min(16, c - q), int(row0[b]) + q))
+            tiles = np.asarray(tiles, dtype=np.int32).reshape(-1, 4)
+            tiles64 = np.asarray([(s, st + q, min(64, c - q), int(row0[b]) + q) for b, (s, st, c) in enumerate(zip(slots, starts, counts))
+                                  for q in range(0, c, 64)], dtype=np.int32).reshape(-1, 4)
         picked = None
         if graphed and any(len(ws) != 1 for ws in want):
             picked = [b for b, ws in enumerate(want) for _ in ws]
@@ -160,7 +167,7 @@ class KazolornHIP(SlotModel):
         n_want = int(want_rows.size)
         res = self._decode_graphed(arena, T, blob, n32, o64, sigs) if graphed else None
         if res is None:
-            dblob = torch.from_numpy(blob).to(dev)
+            dblob = self._upload(blob)
             logits = torch.empty((n_want, V), dtype=f32, device=dev)
             res = self._run(arena, T, dblob, n32, o64, sigs, tiles, tiles.shape[0], tiles64.shape[0], n_want, max_kv, logits,
                             num_layers, return_streams, every=n_want == T and bool((want_rows == np.arange(T)).all()))

@@ -199,7 +199,7 @@ class PikadraHIP(SlotModel):
                     longest=max((st.starts[b] + st.counts[b] for b in big), default=0))
         res = self._decode_graphed(arena, blob, dims) if graphed else None
         if res is None:
-            dblob = torch.from_numpy(blob).to(dev)
+            dblob = self._upload(blob)
             logits = torch.empty((dims["n_want"], self.V), dtype=torch.float32, device=dev)
             res = self._run(arena, dblob, dims, logits, num_layers, return_streams)
         for s_, c in zip(slots, st.counts):

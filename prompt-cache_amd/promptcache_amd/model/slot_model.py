@@ -3,6 +3,7 @@
 and the adapters' ``model(input_ids, past_key_values=...)`` convention is served on top of that."""
 from __future__ import annotations
 
+from itertools import chain
 from typing import List, Optional
 
 import numpy as np
@@ -42,7 +43,7 @@ class StepRows:
             raise ValueError("every request of a step brings at least one token")
         self.counts, self.T, self.R = counts, sum(counts), len(counts)
         self.want = [[c - 1] for c in counts] if want is None else want
-        self.ids = np.fromiter((t for req in tokens for t in req), dtype=np.int32, count=self.T)
+        self.ids = np.fromiter(chain.from_iterable(tokens), dtype=np.int32, count=self.T)
         if self.T and (self.ids.min() < 0 or self.ids.max() >= vocab):
             raise ValueError("token id outside the vocabulary")
         for b, ws in enumerate(self.want):
@@ -84,6 +85,17 @@ class SlotModel:
         if t is None or t.numel() < n:
             t = self._buf[name] = torch.zeros(max(n, 64), dtype=torch.int32, device=self.device)
         return t
+
+    def _upload(self, blob: np.ndarray) -> torch.Tensor:
+        """The step's tables (bytes) on the device, through a pinned block that the host allocator hands out again once the copy is done.  From pageable
+        memory the copy waits for all that is under way on the stream: 16.4 us instead of 7.9 with nothing there, and each prompt began on an idle chip."""
+        if torch.device(self.device).type != "cuda":
+            return torch.from_numpy(blob).to(self.device)
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("a step's tables are new each time: it cannot be captured")
+        host = torch.empty(blob.size, dtype=torch.uint8, pin_memory=True)
+        host.numpy()[:] = blob
+        return host.to(self.device, non_blocking=True)
 
     # ---- one-token steps as captured graphs (models whose step is ``_run(arena, device tables, dims, logits)``) ------------------
     def _decode_graphed(self, arena, blob, d):
