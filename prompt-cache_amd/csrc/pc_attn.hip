@@ -1516,7 +1516,7 @@ int attn_fwd_impl(const void* q, const void* q_lo, int64_t q_batch_stride, int64
                "pc_attn: gather_rows must be 16-byte aligned, planes non-negative");
     p.rows = gather_rows; p.g_kplane = g_kplane; p.g_vplane = g_vplane;
     if (ring_eligible(p, D)) p.nsplit = ring_nsplit(B, H, q_len, past_len + q_len);
-    p.wide = 0; p.wide_nsplit = 0; p.own_only = 0;
+    p.wide = 0; p.wide_nsplit = 0;
     if (!small && wide_eligible(p, D, B)) { p.wide = 1; p.nsplit = wide_nsplit(H, q_len, past_len) + 1; }
     if (p.tail && !small) {
         p.nsplit = tail_stream_splits(B, H, past_len);

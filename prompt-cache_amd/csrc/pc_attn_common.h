@@ -56,9 +56,9 @@ struct AttnParams {
     int32_t small_rt;       // ... workgroups per stream of keys, 16 query rows each (2: 17..32 rows, a row tile a workgroup)
     int32_t formal_handoff; // fused merge: acq_rel arrival (the C++-memory-model form, env PC_FORMAL_HANDOFF=1) instead of relaxed + vmcnt(0)
     int32_t xcd_remap, nqblk, nbatch;
-    // (host) the staged keys go to attn_wide_kernel in `nsplit - 1` slices, the keys this pass appended to attn_ring_kernel in its
-    // own_only mode as partial nsplit - 1 (pc_attn_wide.hip)
-    int32_t wide, wide_nsplit, own_only;
+    // (host) attn_wide_kernel takes the staged keys in `nsplit - 1` slices and the keys this pass appended, by attn_ring_body in its
+    // own_only mode, as partial nsplit - 1 (pc_attn_wide.hip)
+    int32_t wide, wide_nsplit;
     int32_t defer_merge;    // (host) leave the split-KV partials in the workspace: the consumer merges them (pc_gemm_q8 part_o)
     int32_t* nsplit_out;    // (host) where pc_attn reports how many partials per row it left (1: the output planes are final)
     float scale_log2;

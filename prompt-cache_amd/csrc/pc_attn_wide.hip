@@ -21,13 +21,17 @@
 //     stage-while-reading (pc_attn gather_rows) as in the ring kernel: sources from the row table, rows not in the arena yet are
 //     stored from the stage that just landed.
 //   * only STAGED keys (exact fp16, every one visible to every row): no residual planes, no causal mask -- the keys this pass
-//     appended go to attn_ring_kernel in its own-rows mode as one more partial, and attn_combine_kernel merges (pc_attn.hip).
+//     appended are one more partial, by workgroups that run attn_ring_body in its own-rows mode, and attn_combine_kernel merges
+//     (pc_attn.hip).  These workgroups are the last of the same launch: 240 of 256 CUs have a slice of 40 heads, the others take one of
+//     them after the other.  us with the merge, a launch of their own / here: 40 heads over 8 258 keys, 130 / 259 / 500 rows 88.6 / 85.5,
+//     120.1 / 119.6 (143 / 138 while the keys are staged), 196.8 / 191.1, 32 heads over 8 000, 130 rows 73.3 / 69.6, 8 heads over 9 000,
+//     200 rows 63.4 / 48.1.
 // Replaces LlamaAttention.forward's core over the cached keys, promptcache/model/llama2.py:368-398.
 // Roofline: MFMA.  flops = 4 * H * D * q * staged keys * (2 planes of Q / P).
 #include <type_traits>
 #include <utility>
 
-#include "pc_attn_common.h"
+#include "pc_attn_ring_dev.h"
 
 namespace pca {
 namespace {
@@ -64,13 +68,23 @@ __device__ __forceinline__ float vmax3(float a, float b, float c) { float r; asm
 // not own (zero Q fragments) is never stored.
 template <bool GATHER, int R>
 __global__ __launch_bounds__(kWThreads) void attn_wide_kernel(const AttnParams p) {
-    __shared__ __attribute__((aligned(16))) char lds[kWNst * kWStage];
     constexpr int D = WD, KS = WKS, DB = WDB, CPR = WCPR;
+    constexpr int RQ = R < 2 ? R : 2;
+    constexpr int NQL = kWaves * R < kWGroups ? kWaves * R : kWGroups;
+    // LDS: the ring of tiles, the lo plane of Q, both planes of the third groups' Q, row-table entries; the workgroups of the own rows: two of their stages
+    constexpr int kQlo = kWNst * kWStage, kQhi2 = kQlo + NQL * KS * 1024, kGtab = kQhi2 + (R == 3 ? (kWGroups - 2 * kWaves) * KS * 1024 : 0);
+    constexpr int kWide = kGtab + (GATHER ? kWaves * 2048 : 0);
+    __shared__ __attribute__((aligned(16))) char lds[kWide > 2 * kStage ? kWide : 2 * kStage];
+    // grid: q-block, head, slice of the staged keys; behind these the q-blocks and heads of the own rows
+    const int nwide = p.nqblk * p.H * p.wide_nsplit, bid = blockIdx.x;
+    if (bid >= nwide) {
+        attn_ring_body<true, false, false>(p, lds, lds, RingGrid{bid - nwide, 0, 0, (p.q_len + kRingQB - 1) / kRingQB, 1, 1, 1});
+        return;
+    }
 
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, gq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // grid: x = q-block, y = head, z = slice of the staged keys
-    const int qblk = blockIdx.x, h = blockIdx.y, split = blockIdx.z;
+    const int qblk = bid % p.nqblk, h = bid / p.nqblk % p.H, split = bid / p.nqblk / p.H;
     const int hkv = h / (p.H / p.Hkv);
     const int q_len = p.q_len;
     int past_len_v = p.past_len;
@@ -98,12 +112,8 @@ __global__ __launch_bounds__(kWThreads) void attn_wide_kernel(const AttnParams p
     // ---- Q fragments of every group of this wave.  Registers: the hi plane of its first two groups.  LDS, in FRAGMENT order (each
     // lane reads back the 16 bytes it wrote: wave-private regions, no bank conflicts, no barrier): the lo plane of all of them and
     // both planes of the third group (only waves 0 and 1 can have one: kWGroups = 18) ----
-    constexpr int RQ = R < 2 ? R : 2;
-    constexpr int NQL = kWaves * R < kWGroups ? kWaves * R : kWGroups;
-    __shared__ __attribute__((aligned(16))) char qlo_lds[NQL * KS * 1024];
-    __shared__ __attribute__((aligned(16))) char qhi2_lds[R == 3 ? (kWGroups - 2 * kWaves) * KS * 1024 : 16];
-    char* const my_qlo = qlo_lds + wave * (KS * 1024) + lane * 16;        // + group g of this wave: (g * kWaves) * KS * 1024
-    [[maybe_unused]] char* const my_qhi2 = qhi2_lds + (wave & 1) * (KS * 1024) + lane * 16;
+    char* const my_qlo = lds + kQlo + wave * (KS * 1024) + lane * 16;        // + group g of this wave: (g * kWaves) * KS * 1024
+    [[maybe_unused]] char* const my_qhi2 = lds + kQhi2 + (wave & 1) * (KS * 1024) + lane * 16;
     h8 qf[RQ][KS];
     static_for<R>([&](auto gi) {
         constexpr int g = decltype(gi)::value;
@@ -134,7 +144,7 @@ __global__ __launch_bounds__(kWThreads) void attn_wide_kernel(const AttnParams p
     // ---- staging: wave-instruction j (0, 1) of a plane covers rows 4 (8 j + wave) .. + 4 (1 KiB); lane l: row + (l >> 4), position
     // l & 15.  (row & 15 = (4 wave + (l >> 4)) & 15 for both j: one swizzle per lane)
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
-    __shared__ __attribute__((aligned(16))) char gtab[GATHER ? kWaves * 2048 : 16];
+    [[maybe_unused]] char* const gtab = lds + (GATHER ? kGtab : 0);
     [[maybe_unused]] const uint32_t gtab0 = GATHER ? (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)gtab + wave * 2048 : 0;
     [[maybe_unused]] uint64_t g_nost[3][2] = {{~0ull, ~0ull}, {~0ull, ~0ull}, {~0ull, ~0ull}};    // do-not-store lane masks: [0] the tile being multiplied, [1] landing, [2] just issued
     auto lane_row = [&](int l) { return 4 * wave + (l >> 4); };                     // + 32 j
@@ -427,7 +437,7 @@ __global__ __launch_bounds__(kWThreads) void attn_wide_kernel(const AttnParams p
                     }
                 }
             }
-            tr_slot = (p.trace && i == 8 && blockIdx.x + blockIdx.y + blockIdx.z == 0) ? 0 : -1;
+            tr_slot = (p.trace && i == 8 && bid == 0) ? 0 : -1;
             if (my_ng > 0) tile((const _Float16*)buf, (const _Float16*)(buf + kWPlane), key0 + kTK - 1 > last_key, key0);
             if (tr_slot >= 0) tr_slot = 12;
             stamp();
@@ -474,8 +484,8 @@ __global__ __launch_bounds__(kWThreads) void attn_wide_kernel(const AttnParams p
 }  // namespace
 
 // Launches the wide kernel takes the STAGED keys of: what the ring kernel takes (head_dim 128, split-precision Q, no ALiBi), one batch
-// row, one past length, no shared prefix, residual planes for the pass's own rows -- and a shape where it pays: the three launches
-// (slices, own rows, merge of up to 16 partials) cost ~25 us more fixed time than the ring kernel's two, which the shared K / V pass
+// row, one past length, no shared prefix, residual planes for the pass's own rows -- and a shape where it pays: the two launches
+// (slices and own rows, merge of up to 16 partials; measured as three) cost ~25 us more fixed time than the ring kernel's two, which the shared K / V pass
 // earns back from ~6 k staged keys and 128 rows on (tools/wide_sweep.py, profiles/r06_wide_sweep.txt: 40 heads over 8 258 keys,
 // 130 / 259 / 288 / 512 rows: 0.89 / 0.84 / 0.84 / 0.92 x the ring kernel's time; 32 heads over 4 390 keys: 1.0-1.2 x, over
 // 2 048: 1.2-1.4 x).  PC_ATTN_WIDE_MIN / PC_ATTN_WIDE_MIN_ROWS move the thresholds, PC_ATTN_NO_WIDE=1 switches it off.
@@ -510,7 +520,9 @@ int launch_attn_wide(const AttnParams& p0, hipStream_t stream) {
     AttnParams p = p0;
     p.wide_nsplit = p.nsplit - 1;
     p.nqblk = wide_nqblk(p.q_len);
-    const dim3 grid(p.nqblk, p.H, p.wide_nsplit), block(kWThreads);
+    // (workgroups of the own rows as pc_attn_ring_dev.h deals them to the XCDs)
+    const int own = 8 * pc_ceil_div(p.q_len, kRingQB) * pc_ceil_div(p.H, 8);
+    const dim3 grid(p.nqblk * p.H * p.wide_nsplit + own), block(kWThreads);
     const int ngroups = pc_ceil_div(p.q_len, 16), gpb = pc_ceil_div(ngroups, p.nqblk), R = pc_ceil_div(gpb, kWaves);
 #define PC_WIDE(RV)                                                                                       \
     do {                                                                                                  \
@@ -523,13 +535,7 @@ int launch_attn_wide(const AttnParams& p0, hipStream_t stream) {
         default: PC_WIDE(3); break;
     }
 #undef PC_WIDE
-    int rc = pc_check_launch("attn_wide_kernel");
-    if (rc != PC_OK) return rc;
-    // the keys this pass appended (residual planes, causal mask): the ring kernel over [past_len, kv_len) as the last partial
-    AttnParams r = p0;
-    r.rows = nullptr;
-    r.own_only = 1;
-    return launch_attn_ring(r, 1, stream);
+    return pc_check_launch("attn_wide_kernel");
 }
 
 }  // namespace pca
