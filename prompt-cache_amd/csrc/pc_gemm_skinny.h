@@ -1040,10 +1040,14 @@ int launch_one(const GemmParams& p, int units, hipStream_t s) {
 // the activation planes, so that traffic is (#workgroups x planes) and at MT = 4 it exceeds the weights'.
 template <int MT, int EPI>
 int launch_T(const GemmParams& p, int T, int units, hipStream_t s) {
-    constexpr int kMaxT = (MT == 4 ? 6 : 8) / (EPI == EPI_SILU ? 2 : 1);
+    // (33 to 64 rows: eight tiles for plain stores only, whose 128 accumulator registers have nothing beside them; a vocabulary of 2000 tiles, one round instead of two of
+    // workgroups that read 1 MB of activations each, us, four / eight: K = 4096, 33 rows 58.7 / 51.8, 48 61.5 / 53.2, 64 67.6 / 57.5, K = 5120, 48 77.0 / 67.5;
+    // one plane, K = 5120, 33 rows 63.4 / 65.8)
+    constexpr int kMaxT = (MT == 4 && EPI != EPI_STORE ? 6 : 8) / (EPI == EPI_SILU ? 2 : 1);
     if (T > kMaxT) T = kMaxT;
     constexpr int kMaxT8 = 8 / MT / (EPI == EPI_SILU ? 2 : 1);     // int8 images: at most 8 accumulator tiles (launch_w8)
     if (p.w8 && T > kMaxT8) T = kMaxT8;
+    if (MT == 4 && !p.xf_lo && T > 6) T = 6;
     if constexpr (kMaxT >= 8) { if (T >= 8) return launch_one<MT, 8, EPI>(p, units, s); }
     if constexpr (MT == 4 && EPI == EPI_STORE) { if (T == 5) return launch_one<MT, 5, EPI>(p, units, s); }
     if constexpr (kMaxT >= 4) { if (T >= 4) return launch_one<MT, 4, EPI>(p, units, s); }

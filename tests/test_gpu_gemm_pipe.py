@@ -76,3 +76,16 @@ def test_slices_added_in_the_launch(M, N, K, S, T):
     for k in range(1, 4):
         n.gemm_skinny_ks(wf, hi, lo, M, N, K, y, N, S, T, scratch, counters)
         assert rel(y, 1 + k * want) < 2e-6 and not bool(counters.any())
+
+
+# 33 to 64 rows, more tiles than a round of six a workgroup holds: eight, the last workgroup with fewer; one plane too
+@pytest.mark.parametrize("M", [33, 47, 64])
+@pytest.mark.parametrize("N,K", [(32000, 96), (32016, 288), (24592, 32)])
+def test_vocabularies(M, N, K):
+    n = _n()
+    wf, hi, lo, want = operands(M, N, K)
+    y = torch.zeros((M, N), device=DEV)
+    n.gemm_skinny(wf, hi, lo, M, N, K, n.EPI_STORE, y=y, ldy=N)
+    assert rel(y, want) < 1e-6
+    n.gemm_skinny(wf, hi, None, M, N, K, n.EPI_STORE, y=y, ldy=N)          # (rows rounded to 11 bits: a uniform error of 2^-12 at most, 2^-12 / sqrt(3) in the mean)
+    assert rel(y, want) < 2.0 ** -12
