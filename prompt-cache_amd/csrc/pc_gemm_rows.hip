@@ -1,5 +1,7 @@
 // 65..512-row weight-streaming projections (gemm_rows_kernel): long questions in front of a staged cache
 // (replaces the nn.Linear calls of promptcache/model/llama2.py:345-347, :405, :242 at q = 65..512; see pc_gemm_skinny.h).
+#include <type_traits>
+
 #include "pc_gemm_skinny.h"
 
 namespace pcg {
@@ -348,7 +350,7 @@ int launch_rows(const GemmParams& p_in, int units, hipStream_t s) {
         else if constexpr ((TTV) <= 6) hipLaunchKernelGGL((gemm_rows_kernel<TTV, EPI, 4, false>), grid, block, 0, s, p); \
         return pc_check_launch("gemm_rows_kernel");                                                        \
     } while (0)
-    // Wide panels (round 3): up to 288 rows (two blocks of them up to 512) with split-precision planes, a workgroup takes EIGHT weight tiles (128 columns; four
+    // Wide panels (round 3): up to 288 rows (two blocks of them up to 512) with split-precision planes, a workgroup takes up to EIGHT weight tiles (128 columns; four
     // gate/up pairs) instead of four.  What bounds this kernel at a few hundred rows is the activation planes every workgroup
     // re-reads from L2 (13b, 256 rows: 5.2 MB per workgroup against 0.65 MB of weights; launch time = HBM time of the weights +
     // 1.2 us per row): half as many workgroups re-read half as much.  The accumulators of eight tiles need 156 registers, i.e.
@@ -363,7 +365,7 @@ int launch_rows(const GemmParams& p_in, int units, hipStream_t s) {
         // then read twice (once from L2), the activations of a row block by half as many workgroups
         const int nz = mt <= 18 ? 1 : 2;
         if (two && !no_wide && !forced && mt <= 36 && (EPI != EPI_ROPE || wide_rope || nz == 2)) {
-            constexpr int TV = (EPI == EPI_SILU) ? 4 : 8;
+            [[maybe_unused]] constexpr int TV = (EPI == EPI_SILU) ? 4 : 8;
             GemmParams pz = p;
             pz.zrows = nz == 1 ? 0 : 16 * pc_ceil_div(mt, 2);
             const int rw = pc_ceil_div(pc_ceil_div(mt, nz), 2);
@@ -382,14 +384,21 @@ int launch_rows(const GemmParams& p_in, int units, hipStream_t s) {
             // an odd number of row tiles in one block (259 rows = 17 tiles): the odd tile goes to the three staging waves (XT: LDS-DMA
             // ring of five 30-KiB stages) instead of a ninth compute wave on the SIMD that already runs two.  PC_ROWS_XT=0: off
             static const bool xt_on = [] { const char* e = getenv("PC_ROWS_XT"); return !(e && e[0] == '0'); }();
-            if (xt_on && nz == 1 && (mt & 1) && mt >= 5) {
-                hipLaunchKernelGGL((gemm_rows_kernel<8, EPI, 2, true, 3, 3, 2, 768, 5, true>), dim3(pc_ceil_div(units, TV), p.kslices, 1),
-                                   dim3((mt / 2 + 3) * 64), 0, s, pz);
+            auto go = [&](auto tt) {
+                constexpr int TT = decltype(tt)::value, T = EPI == EPI_SILU ? TT / 2 : TT;
+                if (xt_on && nz == 1 && (mt & 1) && mt >= 5)
+                    hipLaunchKernelGGL((gemm_rows_kernel<TT, EPI, 2, true, 3, 3, 2, 768, 5, true>), dim3(pc_ceil_div(units, T), p.kslices, 1), dim3((mt / 2 + 3) * 64), 0, s, pz);
+                else
+                    hipLaunchKernelGGL((gemm_rows_kernel<TT, EPI, 2, true, 3, 3, 2, 768>), dim3(pc_ceil_div(units, T), p.kslices, nz), dim3((rw + 3) * 64), 0, s, pz);
                 return pc_check_launch("gemm_rows_kernel");
-            }
-            hipLaunchKernelGGL((gemm_rows_kernel<8, EPI, 2, true, 3, 3, 2, 768>), dim3(pc_ceil_div(units, TV), p.kslices, nz),
-                               dim3((rw + 3) * 64), 0, s, pz);
-            return pc_check_launch("gemm_rows_kernel");
+            };
+            // Six or four tiles a workgroup where that is no further round of the chip: eight leave CUs empty.  us, 80 / 150 / 259 rows, eight / so: 7b gate|up (172 / 230
+            // workgroups) 56.0 / 51.5, 79.0 / 71.0, 98.1 / 94.9, 7b q|k|v in two slices (192 / 256) 31.5 / 29.4, 45.1 / 42.1, 58.4 / 55.5, MPT's first feed-forward product
+            // (128 / 256) 64.6 / 44.2, 85.8 / 59.2, 105.5 / 83.7; a round more: 13b gate|up (216 / 288) 74.1 / 102.3, 104.4 / 152.1, 138.9 / 210.7.
+            auto rounds = [&](int tt) { return pc_ceil_div(pc_ceil_div(units, EPI == EPI_SILU ? tt / 2 : tt) * p.kslices * nz, 256); };
+            if (rounds(4) == rounds(8)) return go(std::integral_constant<int, 4>{});
+            if (rounds(6) == rounds(8)) return go(std::integral_constant<int, 6>{});
+            return go(std::integral_constant<int, 8>{});
         }
     }
     const int work = units * p.kslices;
