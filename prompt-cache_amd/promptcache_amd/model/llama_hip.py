@@ -662,6 +662,12 @@ class LlamaHIP:
             return max(1, min(8 if T <= 128 else 6, 256 // (blocks * -(-N // 128))))
         return self.kslices
 
+    def qkv_kslices(self, T: int, KQ: int) -> int:
+        """K slices of q|k|v beside ``KQ`` of the others: 65..288 rows cut K in two, as the 128-column panels are half as many as the CUs, and the rotation /
+        append runs over the two slabs (pc_gemm: q|k|v epilogue with kslices = 2)."""
+        wide = self.SKINNY_MAX_ROWS < T <= 288 and KQ != self.kslices and lw0_fp16(self.layers)
+        return int(os.environ.get("PC_ROWS_QKV_KS", "2")) if wide else 1
+
     def _proj(self, a_hi, a_lo, lw: dict, key: str, M: int, N: int, K: int, epi: int, **out) -> None:
         """One many-row projection on the hand-written MFMA kernel (pc_gemm_dense.hip): ``(a_hi + a_lo) @ W^T`` with the
         epilogue fused.  int8 mode: ``lw[key]`` holds the int8 codes as fp16 (exact) and the per-output scales
@@ -1474,9 +1480,7 @@ class LlamaHIP:
         # partial sums; the next RMSNorm launch folds them into the residual stream (x += sum of slabs).
         KQ = self.rows_kslices(T, hid)
         slabs = torch.empty((KQ, T, hid), dtype=torch.float32, device=dev)
-        # ... and so does q|k|v there: its 128-column panels are half as many as the CUs, so K is cut in two and the rotation /
-        # append runs over the two slabs (pc_gemm: q|k|v epilogue with kslices = 2)
-        QS = int(os.environ.get("PC_ROWS_QKV_KS", "2")) if (self.SKINNY_MAX_ROWS < T <= 288 and KQ != self.kslices and lw0_fp16(self.layers)) else 1
+        QS = self.qkv_kslices(T, KQ)
         qkv_slabs = torch.empty((QS, T, W), dtype=torch.float32, device=dev) if QS > 1 else None
         pending = 0                                   # slabs waiting to be added to x
         layers = self.layers if num_layers is None else self.layers[:num_layers]

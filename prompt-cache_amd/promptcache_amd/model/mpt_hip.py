@@ -297,6 +297,9 @@ class MptHIP(LlamaHIP):
         ch, cl = planes(inter)
         KQ = self.rows_kslices(T, hid)
         slabs = torch.empty((KQ, T, hid), dtype=f32, device=dev)
+        # (6 layers of 7b, questions of 70 / 150 / 288 rows, us, one launch / slices and the append behind them: 1202 / 1181, 1695 / 1663, 2548 / 2485)
+        QS = self.qkv_kslices(T, KQ)
+        qkv_slabs = torch.empty((QS, T, 3 * hid), dtype=f32, device=dev) if QS > 1 else None
         pending = 0
         tail = self._tail_for(arena, past_dev)
         layers = self.layers if num_layers is None else self.layers[:num_layers]
@@ -306,7 +309,7 @@ class MptHIP(LlamaHIP):
             kvlo, lo_base = tail(li)
             n.gemm_qkv_rope(lw["wqkv_f"], xh, xl, T, hid, cs, q16, q16l, hid, kp, vp, arena.batch_stride,
                             arena.head_stride, B, H, H, D, q_len, past_len, arena.cap, past_dev, kv_lo=kvlo and kvlo[:4],
-                            lo_base=lo_base, wscale=lw["wqkv_s"])
+                            lo_base=lo_base, wscale=lw["wqkv_s"], kslices=QS, scratch=qkv_slabs)
             n.attn_fwd(q16, q_len * hid, hid, kp, vp, arena.batch_stride, arena.head_stride, None, 0, 0,
                        B, H, H, D, q_len, past_len, self.softmax_scale, ws, past_len_dev=past_dev, out_frag=(ah, al),
                        q_lo=q16l, alibi=alibi, kv_lo=kvlo)
