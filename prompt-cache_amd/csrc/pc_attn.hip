@@ -1332,7 +1332,7 @@ int launch_attn(const AttnParams& p0, int B, hipStream_t stream) {
     if (p.xcd_remap) grid = dim3(8 * p.nqblk * ((p.H * B + 7) / 8), 1, 1);
     const bool ring = D == 128 && ring_eligible(p, D);      // (attn_fwd_impl chose p.nsplit for it)
 #ifdef PC_DEV_SWEEPS      // (the merge inside the launch: built, bit-reproducible, and no faster than the second launch in three rounds of
-                          // measurements (DESIGN.md 3.2) -- dev builds only; the product library ignores `counters` and merges in a second launch)
+                          // measurements -- dev builds only; the product library ignores `counters` and merges in a second launch)
     if (!ring && p.small && p.counters) {
         // one launch: the last-arriving workgroup of each head merges the partials (no attn_combine_kernel)
 #define PC_SMALL_FUSED(NSV)                                                                                          \

@@ -5,7 +5,7 @@
 // Q and P as split-precision pairs, residual tiles of the K / V rows that carry them) -- what changes is how the keys get to
 // the matrix cores:
 //   * workgroup = 8 waves = 128 query rows of one head (attn_fwd_kernel: 4 waves, 64 rows): a K / V tile crosses L2 -> LDS
-//     once per 128 rows.  At 259 rows over 8.3 k staged keys attn_fwd_kernel moves 872 MB of tiles per
+//     once per 128 rows.  At 259 rows over 8.3 k staged keys (13b) attn_fwd_kernel moves 872 MB of tiles per
 //     layer for 45 GFLOP -- it is bound by that stream, not by the MFMAs (19 % busy).
 //   * tiles travel by global_load_lds (16 B per lane, lane-linear destination; the K XOR swizzle and the V row rotation are
 //     applied to the SOURCE address of each lane): no staging registers (attn_fwd_kernel holds 64 VGPRs of them and sits at
@@ -231,9 +231,9 @@ __device__ __forceinline__ void attn_ring_body(const AttnParams& p, char* const 
     };
     // Who stores: every workgroup of a kv head's group streams the same staged keys (they lie in front of every query row), so
     // the landed stages are dealt out over all of them -- stage i leaves with writer i mod g_nw.  The stores are issued in front
-    // of the stage's arithmetic, which hides their completion; a light last q-block (config 4's 259 rows = 128 + 128 + 3) has no
+    // of the stage's arithmetic, which hides their completion; a light last q-block (259 rows = 128 + 128 + 3) has no
     // arithmetic to hide it behind but is one memory round trip per stage ahead of the others anyway.  (One writer per kv head:
-    // +47 us per launch at config 4, all stages to the light block: +43 us, dealt out: see profiles/r04_variants.txt.)
+    // +47 us per launch at that shape, all stages to the light block: +43 us, dealt out: see profiles/r04_variants.txt.)
     [[maybe_unused]] int g_w = -1, g_nw = 1;
     if constexpr (GATHER) {
         const int group = p.H / p.Hkv, nqb = grid.nqblk;

@@ -1,4 +1,4 @@
-// A long question over a LONG staged cache (259 new rows over 8 258 staged keys at the 13b shape): the STAGED
+// A long question over a LONG staged cache (13b: 259 new rows over 8 258 staged keys at the 13b shape): the STAGED
 // keys of a many-row split-precision launch at head_dim 128 -- ALL query rows of a head (up to 288) in one workgroup.
 //
 // What attn_ring_kernel (pc_attn_ring.hip) pays at that shape: 128 query rows per workgroup make 259 rows three q-blocks per head
