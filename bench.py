@@ -249,7 +249,7 @@ def gemm_rooflines(lm, T: int):
     gu_avg, gu_min, gu_n = us("gu")
     nb_gu = 2 * inter * hid * 2
     tr, src = _pmc_traffic("gemm_skinny_gate_up", sig)
-    gate_up = {"kernel": "gemm_skinny_kernel<1,3,EPI_SILU,NORM> (gate|up projection with RMSNorm and SiLU*up fused): the largest "
+    gate_up = {"kernel": "normed_kernel<3,EPI_SILU> (gate|up projection with RMSNorm and SiLU*up fused): the largest "
                          "single kernel of the timed step by time", "bound": "hbm",
                "achieved": nb_gu / (gu_avg * 1e-6) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                "frac": nb_gu / (gu_avg * 1e-6) / 1e9 / HBM_PEAK_GBS, "traffic": tr, "traffic_source": src,
@@ -271,7 +271,7 @@ def gemm_rooflines(lm, T: int):
             "algorithmic_bytes_per_launch": (nb_o + nb_d) / 2, "avg_launch_us": (o_avg + d_avg) / 2, "o_proj_us": o_avg,
             "down_proj_us": d_avg, "min_launch_us": min(o_min, d_min), "launches_timed": 2 * o_n,
             "launches_per_step": 2 * c.num_hidden_layers, "how": how}
-        extra["roofline_qkv"] = {"kernel": "gemm_skinny_kernel<1,3,EPI_ROPE,NORM> (q|k|v + RMSNorm + RoPE + in-place KV append)",
+        extra["roofline_qkv"] = {"kernel": "normed_kernel<3,EPI_ROPE> (q|k|v + RMSNorm + RoPE + in-place KV append)",
                                  "bound": "hbm", "achieved": nb_q / (q_avg * 1e-6) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                  "frac": nb_q / (q_avg * 1e-6) / 1e9 / HBM_PEAK_GBS, "traffic": _pmc_traffic("gemm_skinny_qkv", sig)[0],
                                  "traffic_source": _pmc_traffic("gemm_skinny_qkv", sig)[1],

@@ -53,7 +53,7 @@ tab = {
                         "hbm_bytes_per_launch": (lambda o, d: (o + d) // 2 if o and d else (o or d))(pick("gemm_skinny_kernel<1, 1, 1"),
                                                                                                     pick("gemm_skinny_ks_kernel")),
                         "source": src + " (average of o_proj = gemm_skinny_kernel<1,1,EPI_ADD> and down_proj = gemm_skinny_ks_kernel)"},
-    "gemm_skinny_gate_up": {"signature": "T=12,hid=4096,inter=11008", "hbm_bytes_per_launch": pick("gemm_skinny_kernel<1, 3, 2"), "source": src},
+    "gemm_skinny_gate_up": {"signature": "T=12,hid=4096,inter=11008", "hbm_bytes_per_launch": pick("normed_kernel<3, 2"), "source": src},
 }
 c = pick("attn_combine_kernel")
 # the timed step's attention since round 4: the staging variant (module K/V read once, staged rows written as they pass)
@@ -64,7 +64,7 @@ a = pick("attn_small_kernel<128, false, 0, false, 1>")          # (only present 
 if a and c:
     tab["attn_cached"] = {"signature": "H=32,Hkv=32,D=128,q=12,S=1725", "hbm_bytes_per_launch": a + c,
                           "source": src + " (attn_small_kernel + attn_combine_kernel)"}
-tab["gemm_skinny_qkv"] = {"signature": "T=12,hid=4096,inter=11008", "hbm_bytes_per_launch": pick("gemm_skinny_kernel<1, 3, 3"),
+tab["gemm_skinny_qkv"] = {"signature": "T=12,hid=4096,inter=11008", "hbm_bytes_per_launch": pick("normed_kernel<3, 3"),
                           "source": src + " (q|k|v + RMSNorm + RoPE + KV append)"}
 # --config4: one more pair of passes over bench.py --config 4 for the ring attention of its step (13b, 259 rows over 8 258 keys)
 if "--config4" in sys.argv:
