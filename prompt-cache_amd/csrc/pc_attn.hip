@@ -52,12 +52,14 @@ constexpr int kTailMax = PC_TAIL_MAX;   // most rows of one prefill pass the tai
 // The attention of <= 16 RT new query rows over the rows their own pass appended (keys past_len + j, j <= qi), for one head, as a
 // split-KV partial (m, l, O) in the log2 domain.  Q, K and V are the 32-bit values that their two planes hold (the reference
 // computes the pass in fp32, llama2.py:361-388; only the STAGED rows are fp16 there): every score is the sum of all four
-// products of planes, P is split in three (11 bits each, so all of its 24) and meets both planes of V.
+// products of planes, P is split in three pieces and meets both planes of V.  The pieces are scaled by 2^15, 2^27 and 2^39, with
+// a sum of products each: fp16 ends at 2^-24, so unscaled ones keep P to 2^-25 and no key of less weight than that (24 bits from
+// 1/2 on, 12 of P = 2^-12); these keep all 24 down to 2^-40, and 2^-64 at any size.
 // It runs in the workgroup of an extra split while the other splits stream the staged keys, so its time hides under theirs --
 // if it is short.  Bound by its chain (past length, rows, softmax, V back transposed), so the work is on the matrix cores:
 // wave = (row tile, share of the head's dims), K fragments straight from memory, V by LDS-DMA into a tile of 32 rows (hi, lo).
 // As fp32 FMAs on rows in LDS the 32-row form read five float4 of LDS for 16 FMAs and was the launch's last workgroup: us per
-// layer with the merge, 32 heads x 128, 308 / 936 / 1725 staged keys: 27 rows 14.2 -> 13.2, 14.6 -> 14.5, 16.2 -> 16.1, 100 staged keys 12.5 -> 9.0.
+// layer with the merge, 32 heads x 128, 308 / 936 / 1725 staged keys: 27 rows 14.2 -> 13.2, 14.6 -> 14.5, 16.2 -> 16.1, 100 staged keys 12.5 -> 9.3 (9.0 with unscaled pieces in one sum).
 // (Residual tiles inside the streaming kernel instead cost 32 VGPRs -- the second resident workgroup per CU, or spills --
 // and a straggler split: 13.3 -> 15.9 .. 25 us per launch on the persona prompt; the same arithmetic inside the merge
 // kernel lengthened the serial merge by 1.1 us per layer.)
@@ -151,10 +153,11 @@ __device__ __forceinline__ void attn_tail_block(const AttnParams& p, _Float16* _
             const bool vis = qi < q_len && t * 16 + g * 4 + r <= qi;
             const float e = vis ? exp2f(sv[t][r] - m) : 0.f;
             l += e;
-            const _Float16 a0 = (_Float16)e;
-            const float e1 = e - (float)a0;
+            const float e0 = e * 0x1p15f;                          // (e <= 1; a piece leaves at most 8 to the next one: 2^15 again)
+            const _Float16 a0 = (_Float16)e0;
+            const float e1 = (e0 - (float)a0) * 0x1p12f;
             const _Float16 a1 = (_Float16)e1;
-            p0[t * 4 + r] = a0; p1[t * 4 + r] = a1; p2[t * 4 + r] = (_Float16)(e1 - (float)a1);
+            p0[t * 4 + r] = a0; p1[t * 4 + r] = a1; p2[t * 4 + r] = (_Float16)((e1 - (float)a1) * 0x1p12f);
         }
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
@@ -175,12 +178,14 @@ __device__ __forceinline__ void attn_tail_block(const AttnParams& p, _Float16* _
         const h4 l0 = lds_tr_read(vp + kTailKeys * D), l1 = lds_tr_read(vp + (kTailKeys + 16) * D);
         const h8 vh = {h0[0], h0[1], h0[2], h0[3], h1[0], h1[1], h1[2], h1[3]};
         const h8 vl = {l0[0], l0[1], l0[2], l0[3], l1[0], l1[1], l1[2], l1[3]};
-        f4 o = {0.f, 0.f, 0.f, 0.f};
-        o = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, p2, o, 0, 0, 0);
-        o = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, p1, o, 0, 0, 0);
-        o = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, p0, o, 0, 0, 0);
-        o = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, p1, o, 0, 0, 0);
-        o = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, p0, o, 0, 0, 0);
+        const f4 zero = {0.f, 0.f, 0.f, 0.f};
+        f4 o0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, p0, zero, 0, 0, 0);
+        f4 o1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, p1, zero, 0, 0, 0);
+        f4 o2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, p2, zero, 0, 0, 0);
+        o0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, p0, o0, 0, 0, 0);
+        o1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, p1, o1, 0, 0, 0);
+        o2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, p2, o2, 0, 0, 0);
+        const f4 o = ((o2 * 0x1p-12f + o1) * 0x1p-12f + o0) * 0x1p-15f;
         if (qi < q_len) {
             float* dst = p.part_o + slot * D + db * 16 + g * 4;
             if constexpr (WT) { st_wt2(dst, o[0], o[1]); st_wt2(dst + 2, o[2], o[3]); }
