@@ -207,6 +207,9 @@ typedef struct pc_attn_args {
 int pc_attn(const pc_attn_args* args, void* stream);
 /* 1 when pc_attn would run `args` (gather_rows ignored) on a kernel that implements gather_rows, else 0 */
 int pc_attn_gather_ok(const pc_attn_args* args);
+/* The launch (key splits, kernel) that pc_attn chooses for a pass with q_lo behind one past length, as one number to compare (0: sizes it refuses); lo_row0: -1 or -2 as
+ * above, 0 without k_lo.  A captured launch keeps this choice whatever past_len_dev says at a replay. */
+int pc_attn_form(int32_t B, int32_t H, int32_t D, int32_t q_len, int32_t past_len, int32_t lo_row0, int32_t alibi);
 
 /* ---------------------------------------------------------------------------------------------
  * Elementwise / reduction pieces of the layer stack, fused for the small-q prefill (q_len rows):

@@ -1438,6 +1438,55 @@ static thread_local unsigned long long* g_attn_trace = nullptr;
 PC_EXPORT int pc_dev_attn_trace(void* buf) { g_attn_trace = (unsigned long long*)buf; return PC_OK; }
 
 namespace {
+// Which launch takes a pass: key splits, the kernel of few rows and its workgroups a row tile, the tail workgroup, the wide kernel.  From sizes and from which operands there are
+// alone (past_len: the host's).  Whether it can stage while reading.
+bool choose_launch(AttnParams& p, int D, int B) {
+    const int H = p.H, q_len = p.q_len, past_len = p.past_len;
+    p.nsplit = choose_nsplit(B, H, q_len, past_len + q_len, q_len <= kQB || p.q_lo != nullptr);
+    p.tail = 0; p.small = 0; p.small_rt = 1;
+    // (a pass the ring kernel takes carries its own rows as residual tiles in the stream: no fp32 tail workgroup)
+    const bool ring_first = ring_eligible(p, D);
+    p.tail = (!ring_first && p.k_lo && p.lo_row0 == -1 && q_len <= kTailMax && !p.past_lens) ? 1 : 0;
+    // <= 16 rows over a long cache: one key slice per WAVE, partials merged per workgroup (attn_small_kernel).  Not for
+    // launches that carry residual tiles in the stream (decode over a residual tail, lo_row0 != -1).
+    static const bool small_off = [] { const char* e = getenv("PC_ATTN_NO_SMALL"); return e && e[0] == '1'; }();
+    // 17..32 rows in tail mode take the same kernel with two row tiles per wave (every K fragment and V tile serves both;
+    // two-launch form); PC_ATTN_SMALL2=0: the 64-row kernel, as in rounds 1-3
+    static const bool small2_off = [] { const char* e = getenv("PC_ATTN_SMALL2"); return e && e[0] == '0'; }();
+    const bool small2 = !small2_off && q_len > kSmallQ && q_len <= 2 * kSmallQ && p.tail && !p.counters;
+    bool small = !small_off && (q_len <= kSmallQ || small2) && !p.past_lens && (!p.k_lo || p.tail) && past_len + q_len >= 256;
+    if (small) {
+        const int ns = small_nstream(B, H, p.tail, q_len, p.tail ? past_len : past_len + q_len) + p.tail;
+        if (ns >= 2) p.nsplit = ns; else small = false;
+        // A workgroup for each row tile while these are at most a round and a quarter of the CUs: two row tiles in one are a chain of
+        // twice the products and merges for the same keys.  us with the merge, 27 rows, one workgroup / two: 32 heads, 308 keys 11.8 /
+        // 9.5, 700 12.5 / 10.1, 40 heads 12.2 / 11.4, 13.5 / 12.9; behind that (32 heads, 936 keys 13.8 / 13.7, 2500 20.7 / 21.7) the same
+        // keys cross the chip twice.
+        if (q_len > kSmallQ && 2 * B * H * p.nsplit <= 320) p.small_rt = 2;
+    }
+    p.small = small ? 1 : 0;
+    // staging while reading lives in attn_small_kernel's two-launch form and in the tail-mode instantiation of the 64-row kernel
+    // (17..32 new rows: one q-block, the streaming splits cover staged keys only); one batch row
+    const bool mid_gather = !small && p.tail && !ring_first && !p.key_pos && !p.pre_k && q_len <= kQB;
+    // ... and in the ring kernel (more than 32 split-precision rows at head_dim 128, no shared prefix, one past length)
+    const bool ring_gather = !small && ring_eligible(p, D) && !p.pre_k && !p.past_lens;
+    // (17..32 rows with ALiBi: no staging form)
+    const bool small_gather = small && !(p.key_pos && q_len > kSmallQ);
+    const bool can_gather = (small_gather || mid_gather || ring_gather) && (small ? !p.counters : true) && B == 1 && past_len > 0;
+    if (ring_eligible(p, D)) p.nsplit = ring_nsplit(B, H, q_len, past_len + q_len);
+    p.wide = 0; p.wide_nsplit = 0;
+    if (!small && wide_eligible(p, D, B)) { p.wide = 1; p.nsplit = wide_nsplit(H, q_len, past_len) + 1; }
+    if (p.tail && !small) {
+        p.nsplit = tail_stream_splits(B, H, past_len);
+        // one more split for the tail workgroup -- taken from the streaming splits when the total would cross into the
+        // next instantiation of the merge kernel (4 / 8 / 16 / 32 partials per row)
+        int ms = p.nsplit;
+        if (ms >= 4 && (ms & (ms - 1)) == 0) ms -= 1;
+        p.nsplit = ms + 1;
+    }
+    return can_gather;
+}
+
 int attn_fwd_impl(const void* q, const void* q_lo, int64_t q_batch_stride, int64_t q_token_stride, const void* k,
                   const void* v, int64_t kv_batch_stride, int64_t kv_head_stride, void* out,
                   int64_t out_batch_stride, int64_t out_token_stride, int32_t B, int32_t H, int32_t Hkv,
@@ -1483,54 +1532,13 @@ int attn_fwd_impl(const void* q, const void* q_lo, int64_t q_batch_stride, int64
     p.k_lo = (const _Float16*)k_lo; p.v_lo = (const _Float16*)v_lo; p.lo_bs = lo_bs; p.lo_hs = lo_hs; p.lo_row0 = lo_row0;
     p.H = H; p.Hkv = Hkv; p.q_len = q_len; p.past_len = past_len;
     p.scale_log2 = softmax_scale * 1.4426950408889634f;
-    p.nsplit = choose_nsplit(B, H, q_len, past_len + q_len, q_len <= kQB || q_lo != nullptr);
-    p.tail = 0; p.small = 0; p.small_rt = 1;
-    // (a pass the ring kernel takes carries its own rows as residual tiles in the stream: no fp32 tail workgroup)
-    const bool ring_first = ring_eligible(p, D);
-    p.tail = (!ring_first && k_lo && lo_row0 == -1 && q_len <= kTailMax && !past_lens) ? 1 : 0;
-    // <= 16 rows over a long cache: one key slice per WAVE, partials merged per workgroup (attn_small_kernel).  Not for
-    // launches that carry residual tiles in the stream (decode over a residual tail, lo_row0 != -1).
-    static const bool small_off = [] { const char* e = getenv("PC_ATTN_NO_SMALL"); return e && e[0] == '1'; }();
-    // 17..32 rows in tail mode take the same kernel with two row tiles per wave (every K fragment and V tile serves both;
-    // two-launch form); PC_ATTN_SMALL2=0: the 64-row kernel, as in rounds 1-3
-    static const bool small2_off = [] { const char* e = getenv("PC_ATTN_SMALL2"); return e && e[0] == '0'; }();
-    const bool small2 = !small2_off && q_len > kSmallQ && q_len <= 2 * kSmallQ && p.tail && !counters;
-    bool small = !small_off && (q_len <= kSmallQ || small2) && !past_lens && (!k_lo || p.tail) && past_len + q_len >= 256;
-    if (small) {
-        const int ns = small_nstream(B, H, p.tail, q_len, p.tail ? past_len : past_len + q_len) + p.tail;
-        if (ns >= 2) p.nsplit = ns; else small = false;
-        // A workgroup for each row tile while these are at most a round and a quarter of the CUs: two row tiles in one are a chain of
-        // twice the products and merges for the same keys.  us with the merge, 27 rows, one workgroup / two: 32 heads, 308 keys 11.8 /
-        // 9.5, 700 12.5 / 10.1, 40 heads 12.2 / 11.4, 13.5 / 12.9; behind that (32 heads, 936 keys 13.8 / 13.7, 2500 20.7 / 21.7) the same
-        // keys cross the chip twice.
-        if (q_len > kSmallQ && 2 * B * H * p.nsplit <= 320) p.small_rt = 2;
-    }
-    p.small = small ? 1 : 0;
-    // staging while reading lives in attn_small_kernel's two-launch form and in the tail-mode instantiation of the 64-row kernel
-    // (17..32 new rows: one q-block, the streaming splits cover staged keys only); one batch row
-    const bool mid_gather = !small && p.tail && !ring_first && !key_pos && !pre_k && q_len <= kQB;
-    // ... and in the ring kernel (more than 32 split-precision rows at head_dim 128, no shared prefix, one past length)
-    const bool ring_gather = !small && ring_eligible(p, D) && !pre_k && !past_lens;
-    // (17..32 rows with ALiBi: no staging form)
-    const bool small_gather = small && !(key_pos && q_len > kSmallQ);
-    const bool can_gather = (small_gather || mid_gather || ring_gather) && (small ? !counters : true) && B == 1 && past_len > 0;
+    const bool can_gather = choose_launch(p, D, B);
     if (gather_ok) { *gather_ok = can_gather ? 1 : 0; return PC_OK; }
     PC_REQUIRE(!gather_rows || can_gather, PC_ERR_ARG,
                "pc_attn: gather_rows needs B = 1 and a launch of <= %d query rows in tail mode, <= %d rows over >= 256 keys without counters, or a split-precision launch of >= %d rows at head_dim 128 (ask pc_attn_gather_ok)", kTailMax, kSmallQ, ring_min_rows());
     PC_REQUIRE(!gather_rows || (((uintptr_t)gather_rows & 15) == 0 && g_kplane >= 0 && g_vplane >= 0), PC_ERR_ARG,
                "pc_attn: gather_rows must be 16-byte aligned, planes non-negative");
     p.rows = gather_rows; p.g_kplane = g_kplane; p.g_vplane = g_vplane;
-    if (ring_eligible(p, D)) p.nsplit = ring_nsplit(B, H, q_len, past_len + q_len);
-    p.wide = 0; p.wide_nsplit = 0;
-    if (!small && wide_eligible(p, D, B)) { p.wide = 1; p.nsplit = wide_nsplit(H, q_len, past_len) + 1; }
-    if (p.tail && !small) {
-        p.nsplit = tail_stream_splits(B, H, past_len);
-        // one more split for the tail workgroup -- taken from the streaming splits when the total would cross into the
-        // next instantiation of the merge kernel (4 / 8 / 16 / 32 partials per row)
-        int ms = p.nsplit;
-        if (ms >= 4 && (ms & (ms - 1)) == 0) ms -= 1;
-        p.nsplit = ms + 1;
-    }
     p.part_o = nullptr; p.part_ml = nullptr;
     if (p.nsplit > 1) {
         const int64_t slots = (int64_t)B * H * p.nsplit * q_len;
@@ -1584,6 +1592,20 @@ PC_EXPORT int pc_attn(const pc_attn_args* a, void* stream) {
                          a->lo_head_stride, a->lo_row0, stream, a->past_lens, a->counters, a->prefix_k, a->prefix_v,
                          a->prefix_k_lo, a->prefix_v_lo, a->prefix_head_stride, a->gather_rows, a->gather_k_plane, a->gather_v_plane, nullptr,
                          a->defer_merge, a->nsplit_out);
+}
+
+// The launch that pc_attn chooses for a pass in split precision behind one past length, as one number (0: a pass that it refuses).  A captured launch keeps its shape whatever
+// length the device holds at a replay, so a graph stands for the lengths that ask for the same one.
+PC_EXPORT int pc_attn_form(int32_t B, int32_t H, int32_t D, int32_t q_len, int32_t past_len, int32_t lo_row0, int32_t alibi) {
+    if (!(D == 32 || D == 64 || D == 128) || B <= 0 || H <= 0 || q_len <= 0 || past_len < 0) return 0;
+    static const _Float16 some[8] = {};                              // (only whether a plane is there counts)
+    AttnParams p = {};
+    p.q = p.q_lo = some;
+    if (lo_row0 < 0) p.k_lo = p.v_lo = some;
+    if (alibi) p.key_pos = p.slopes = (const float*)some;
+    p.H = p.Hkv = H; p.q_len = q_len; p.past_len = past_len; p.lo_row0 = lo_row0;
+    choose_launch(p, D, B);
+    return p.nsplit | (p.small ? 1 << 8 : 0) | (p.small_rt == 2 ? 1 << 9 : 0) | (p.tail ? 1 << 10 : 0) | (p.wide ? 1 << 11 : 0) | (D == 128 && ring_eligible(p, D) ? 1 << 12 : 0);
 }
 
 // Whether pc_attn would run this launch shape on a kernel that implements gather_rows (the field itself is ignored here).

@@ -124,6 +124,7 @@ SIGNATURES = {
     "pc_rope_append": (C.c_int, [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp,
                                  _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _vp]),
     "pc_attn_workspace_bytes": (C.c_int64, [_i32, _i32, _i32, _i32, _i32]),
+    "pc_attn_form": (C.c_int, [_i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "pc_rope_append_ex": (C.c_int, [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp,
                                     _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _i64, _i64, _i32, _i64, _vp]),
     "pc_rmsnorm_split": (C.c_int, [_vp, _vp, _vp, _vp, _i32, _i32, _f32, _vp]),
@@ -299,6 +300,11 @@ def rope_append(q, q_bs, q_ts, q_out, qo_bs, qo_ts, k_new, v_new, n_bs, n_ts, k_
 
 def attn_workspace_bytes(B: int, H: int, D: int, q_len: int, kv_len_max: int) -> int:
     return int(load().pc_attn_workspace_bytes(B, H, D, q_len, kv_len_max))
+
+
+def attn_form(B: int, H: int, D: int, q_len: int, past_len: int, lo_row0: int, alibi: int = 0) -> int:
+    """The launch ``attn_fwd`` chooses for a pass in split precision (``q_lo``) behind ``past_len`` rows, as one number; ``lo_row0``: -1 / -2 as there, 0 without ``kv_lo``."""
+    return load().pc_attn_form(B, H, D, q_len, past_len, lo_row0, alibi)
 
 
 def _attn_args(q, q_bs, q_ts, k, v, kv_bs, kv_hs, out, o_bs, o_ts, B, H, Hkv, D, q_len, past_len, scale,

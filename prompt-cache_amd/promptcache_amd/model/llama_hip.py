@@ -332,7 +332,7 @@ class LlamaHIP:
         self._pre = None            # set per captured forward: (fp32 residual stream, rotation table) from pc_prefill_prologue
         self.fused_prologue = os.environ.get("PC_FUSED_PROLOGUE", "1") != "0"
         self.stats = {"fused_gather": 0}     # forwards that carried out a pending staging inside their attention launches
-        self._gather_ok_cache, self._nsplit_cache = {}, {}
+        self._gather_ok_cache, self._form_cache = {}, {}
         # hipGraphs for the 65..512-row forward as well (B = 1, 16-row buckets): nine launches per layer from Python are host-bound
         # at 7b and ~100 rows (PC_GRAPH_MID=0: launched eagerly, as in rounds 1-3)
         self.graph_mid = os.environ.get("PC_GRAPH_MID", "1") != "0"
@@ -1181,13 +1181,18 @@ class LlamaHIP:
             self._gather_ok_cache[ck] = ok
         return ok
 
-    def _nsplit_key(self, B: int, q_len: int, kv_len: int) -> int:
-        k = (B, q_len, kv_len)
-        v = self._nsplit_cache.get(k)
+    _alibi = 0                                               # (1: scores carry position biases)
+
+    def _attn_form(self, B: int, q_len: int, past_len: int) -> int:
+        """The attention launch of a forward in the current tail mode (``pc_attn_form``).  A captured one keeps its splits and kernel wherever it is replayed, so a graph
+        stands for the staged lengths that ask for the same.  (The size of the workspace does not tell: 16 rows of 32 heads behind 650 and 1 300 rows share it, three streams
+        of keys and seven.)"""
+        k = (B, q_len, past_len, self._lo_mode)
+        v = self._form_cache.get(k)
         if v is None:
-            if len(self._nsplit_cache) > 4096:
-                self._nsplit_cache.clear()
-            v = self._nsplit_cache[k] = _native.attn_workspace_bytes(B, self.H, self.D, q_len, kv_len)   # monotone in the split count
+            if len(self._form_cache) > 4096:
+                self._form_cache.clear()
+            v = self._form_cache[k] = _native.attn_form(B, self.H, self.D, q_len, past_len, -self._lo_mode, self._alibi)
         return v
 
     def _graph_key(self, arena, B, q_len, past_len, last_token_only, num_layers, gather):
@@ -1195,7 +1200,7 @@ class LlamaHIP:
         tail = arena.tail_lo if mode else None
         # (a staging forward captures the address of the arena's row table as well: a NEW arena that happens to land on the freed
         # buffer address of an old one must not replay a graph that writes through the old arena's freed row table)
-        return (B, q_len, arena.buf.data_ptr(), arena.cap, self._nsplit_key(B, q_len, past_len + q_len), bool(last_token_only), num_layers,
+        return (B, q_len, arena.buf.data_ptr(), arena.cap, self._attn_form(B, q_len, past_len), bool(last_token_only), num_layers,
                 self.fuse_norm, self.use_chain, mode, tail.data_ptr() if mode else 0, tail.shape[4] if mode else 0,
                 arena.row_table().data_ptr() if gather else 0)
 
@@ -1378,9 +1383,8 @@ class LlamaHIP:
         """The captured graph of ONE greedy decode step over ``arena`` (forward of the token in the loop state + argmax +
         state advance), keyed like ``_graphed_skinny``."""
         n = _native
-        nsplit_key = n.attn_workspace_bytes(1, self.H, self.D, 1, past_len + 1)
         mode = self._lo_mode
-        key = ("loop", arena.buf.data_ptr(), arena.cap, nsplit_key, self.fuse_norm, self.use_chain, mode,
+        key = ("loop", arena.buf.data_ptr(), arena.cap, self._attn_form(1, 1, past_len), self.fuse_norm, self.use_chain, mode,
                arena.tail_lo.data_ptr() if mode else 0, arena.tail_lo.shape[4] if mode else 0)
         ent = self._graphs.pop(key, None)
         if ent is not None:

@@ -36,6 +36,7 @@ def alibi_slopes(num_heads: int, alibi_bias_max: int = 8) -> torch.Tensor:
 
 
 class MptHIP(LlamaHIP):
+    _alibi = 1
     _shared_prefix_loop = False     # (its many-row loop keeps a copy of the trunk per batch row)
     supports_fused_gather = False   # (its layer loops read staged rows from the arena ...)
     # ... and the copy goes out at the beginning of the first forward (_resolve_arena): behind it the host prepares the step, where an update() that copies at
@@ -146,11 +147,9 @@ class MptHIP(LlamaHIP):
         return CausalLMOutput(logits=logits, past_key_values=arena.views() if use_cache else None)
 
     def _graphed_mpt(self, ids, position_ids, arena, B, q_len, past_len, last_token_only, num_layers):
-        n = _native
         kv_len = past_len + q_len
-        nsplit_key = n.attn_workspace_bytes(B, self.H, self.D, q_len, kv_len)
         mode = self._lo_mode
-        key = (B, q_len, arena.buf.data_ptr(), arena.cap, nsplit_key, bool(last_token_only), num_layers, mode,
+        key = (B, q_len, arena.buf.data_ptr(), arena.cap, self._attn_form(B, q_len, past_len), bool(last_token_only), num_layers, mode,
                arena.tail_lo.data_ptr() if mode else 0, arena.tail_lo.shape[4] if mode else 0)
         ent = self._graphs.pop(key, None)
         fresh = ent is None
