@@ -13,10 +13,15 @@
 
 namespace pcg {
 
+// dev: PC_GEMM_T, a number of tiles for every launch that has a kernel of so many (fewer otherwise); 0: the rules below and in launch_MT
+static int forced_T() {
+    static const int forced = [] { const char* e = getenv("PC_GEMM_T"); return e ? atoi(e) : 0; }();
+    return forced;
+}
+
 // tiles (or gate/up pairs) per workgroup: fill ~256 CUs with one round of workgroups where possible
 int choose_T(int units) {
-    static const int forced = [] { const char* e = getenv("PC_GEMM_T"); return e ? atoi(e) : 0; }();
-    if (forced > 0) return forced;
+    if (forced_T() > 0) return forced_T();
     // smallest T in {1,2,3,4,8} whose grid fits one round of 256 CUs (a partial second round idles most of
     // the chip: 344 workgroups ran at 4.4 TB/s where 230 run the same bytes in one round)
     const int cand[5] = {1, 2, 3, 4, 8};
@@ -50,17 +55,18 @@ void set_k_balance(GemmParams& p, int K) {
 int launch_MT(int epi, const GemmParams& p, int T, int units, hipStream_t s) {
     const int mt = pc_ceil_div(p.M, 16);
     if (mt > 4) return launch_rows_epi(epi, p, units, s);
-    if (normed_few_takes(epi, p)) return launch_normed_few(epi, p, units, s);
+    const bool forced = forced_T() > 0;
+    if (!forced && normed_few_takes(epi, p)) return launch_normed_few(epi, p, units, s);
     if (!p.w8 && !p.xn && p.xf_lo) {
         // Five tiles a workgroup where they fill a round of the chip that eight leave a third empty (13b's down_proj and o_proj in four slices, us, eight / five: 20 rows
         // 30.3 / 25.3 and 14.6 / 13.2, 40 rows, four 42.5 / 29.5 and 19.5 / 15.9), and up to 32 rows of one slice instead of four where tile images are whole multiples of
         // 64 KB, since the starts of four of them lie on the same channels (1024 tiles, K = 4096: 12 rows 29.7 / 25.3, 20 rows 30.9 / 26.6, 64 rows 35.7 / 36.4).
         const bool five = mt <= 2 ? epi != EPI_SILU : epi == EPI_STORE;
-        if (five && T == 8 && pc_ceil_div(units * p.kslices, 5) <= 256) T = 5;
-        if (five && T == 4 && mt <= 2 && p.kslices == 1 && p.KS % 64 == 0) T = 5;
-        if (T == 5 && mt <= 2) return launch_pipe(epi, p, T, units, s);
+        if (five && !forced && T == 8 && pc_ceil_div(units * p.kslices, 5) <= 256) T = 5;
+        if (five && !forced && T == 4 && mt <= 2 && p.kslices == 1 && p.KS % 64 == 0) T = 5;
+        if (five && T == 5 && mt <= 2) return launch_pipe(epi, p, T, units, s);
         // (33 to 64 rows take three pairs at most: two, where three are a second round of the chip that is emptier.  13b's gate|up, 40 rows 81.5 / 67.2)
-        if (mt > 2 && epi == EPI_SILU && T > 3) {
+        if (mt > 2 && epi == EPI_SILU && T > 3 && !forced) {
             auto busy = [&](int t) { const int wg = pc_ceil_div(units, t); return (float)wg / (float)(256 * pc_ceil_div(wg, 256)); };
             T = busy(2) > busy(3) ? 2 : 3;
         }

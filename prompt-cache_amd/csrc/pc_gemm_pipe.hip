@@ -123,6 +123,7 @@ int by_epi(int epi, const GemmParams& p, int units, hipStream_t s) {
         case EPI_ADD: return go<MT, T, EPI_ADD>(p, units, s);
         case EPI_SILU:
             if constexpr (T <= 4) return go<MT, T, EPI_SILU>(p, units, s);
+            pc_set_error("pc_gemm (pipe): no gated unit with %d pairs a workgroup", T);
             return PC_ERR_ARG;
         case EPI_ROPE: return go<MT, T, EPI_ROPE>(p, units, s);
         default: return go<MT, T, EPI_GELU>(p, units, s);
