@@ -26,13 +26,15 @@ __device__ __forceinline__ h8 weight(const char* tile, int ks, int lane) {
 }
 
 // the eight waves' sums of the workgroup's tiles in wave order, scaled by 1 / rms, to the epilogue: one tile (pair) a wave
-template <int T, int EPI>
+template <int T, int EPI, bool TRACE>
 __device__ __forceinline__ void reduce_normed(const GemmParams& p, const f4 (&acc)[EPI == EPI_SILU ? 2 * T : T], f4 (*red)[EPI == EPI_SILU ? 2 * T : T][64],
                                               const float (*ssl)[16], int wave, int lane, int m, int g) {
     constexpr int TT = EPI == EPI_SILU ? 2 * T : T;
 #pragma unroll
     for (int t = 0; t < TT; ++t) red[wave][t][lane] = acc[t];
+    if (TRACE) trace_stamp(p, blockIdx.x, 0, wave, 1);
     lds_barrier();
+    if (TRACE) trace_stamp(p, blockIdx.x, 0, wave, 2);
     if (wave >= T) return;
     f4 v = {0.f, 0.f, 0.f, 0.f}, u = {0.f, 0.f, 0.f, 0.f};
     float tot = 0.f;
@@ -46,9 +48,10 @@ __device__ __forceinline__ void reduce_normed(const GemmParams& p, const f4 (&ac
     v *= rs;
     u *= rs;
     tile_epilogue<EPI>(p, v, u, m, (int)blockIdx.x * T + wave, g, 0);
+    if (TRACE) { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); trace_stamp(p, blockIdx.x, 0, wave, 3); }
 }
 
-template <int T, int EPI, int U>
+template <int T, int EPI, int U, bool TRACE>
 __global__ __launch_bounds__(kThreads) void normed_few_kernel(const GemmParams p) {
     constexpr int TT = EPI == EPI_SILU ? 2 * T : T;
     extern __shared__ __attribute__((aligned(16))) _Float16 pieces[];       // per wave: [row][hi, lo][ld]
@@ -56,6 +59,7 @@ __global__ __launch_bounds__(kThreads) void normed_few_kernel(const GemmParams p
     __shared__ float ssl[kWaves][16];
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (TRACE) trace_stamp(p, blockIdx.x, 0, wave, 0);
     const int KS = p.KS, M = p.M;
     const int live = p.m_dev ? (*p.m_dev < M ? *p.m_dev : M) : M;           // (rows behind them are never read)
     int ks0, ks1;
@@ -151,10 +155,10 @@ __global__ __launch_bounds__(kThreads) void normed_few_kernel(const GemmParams p
         consume(wB, kb + U);
         __builtin_amdgcn_sched_barrier(0);
     }
-    reduce_normed<T, EPI>(p, acc, red, ssl, wave, lane, m, g);
+    reduce_normed<T, EPI, TRACE>(p, acc, red, ssl, wave, lane, m, g);
 }
 
-template <int T, int EPI>
+template <int T, int EPI, bool TRACE>
 __global__ __launch_bounds__(kThreads) void normed_kernel(const GemmParams p) {
     constexpr int TT = EPI == EPI_SILU ? 2 * T : T;
     __shared__ f4 red[kWaves][TT][64];
@@ -162,6 +166,7 @@ __global__ __launch_bounds__(kThreads) void normed_kernel(const GemmParams p) {
     __shared__ __attribute__((aligned(16))) _Float16 gain[kWaves * kGamHalfs];
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (TRACE) trace_stamp(p, blockIdx.x, 0, wave, 0);
     const int KS = p.KS;
     const int live = p.m_dev ? (*p.m_dev < p.M ? *p.m_dev : p.M) : p.M;
     int ks0, ks1;
@@ -221,22 +226,26 @@ __global__ __launch_bounds__(kThreads) void normed_kernel(const GemmParams p) {
     ss += __shfl_xor(ss, 16);
     ss += __shfl_xor(ss, 32);
     if (g == 0) ssl[wave][m] = ss;
-    reduce_normed<T, EPI>(p, acc, red, ssl, wave, lane, m, g);
+    reduce_normed<T, EPI, TRACE>(p, acc, red, ssl, wave, lane, m, g);
 }
 
-template <int T, int EPI>
+// (pc_dev_gemm_trace: kernels of their own, since the places to stamp at cost 1 or 2 % of the shortest launches)
+template <int T, int EPI, bool TRACE>
 int go_few(const GemmParams& p, int units, size_t lds, hipStream_t s) {
     constexpr int U = EPI == EPI_SILU ? 1 : 4;
     static const hipError_t raised =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(normed_few_kernel<T, EPI, U>), hipFuncAttributeMaxDynamicSharedMemorySize, kFewLds);
+        hipFuncSetAttribute(reinterpret_cast<const void*>(normed_few_kernel<T, EPI, U, TRACE>), hipFuncAttributeMaxDynamicSharedMemorySize, kFewLds);
     (void)raised;
-    hipLaunchKernelGGL((normed_few_kernel<T, EPI, U>), dim3(pc_ceil_div(units, T)), dim3(kThreads), lds, s, p);
+    hipLaunchKernelGGL((normed_few_kernel<T, EPI, U, TRACE>), dim3(pc_ceil_div(units, T)), dim3(kThreads), lds, s, p);
     return pc_check_launch("normed_few_kernel");
 }
 
 template <int T, int EPI>
 int go(const GemmParams& p, int units, hipStream_t s) {
-    hipLaunchKernelGGL((normed_kernel<T, EPI>), dim3(pc_ceil_div(units, T)), dim3(kThreads), 0, s, p);
+    if (p.trace)
+        hipLaunchKernelGGL((normed_kernel<T, EPI, true>), dim3(pc_ceil_div(units, T)), dim3(kThreads), 0, s, p);
+    else
+        hipLaunchKernelGGL((normed_kernel<T, EPI, false>), dim3(pc_ceil_div(units, T)), dim3(kThreads), 0, s, p);
     return pc_check_launch("normed_kernel");
 }
 
@@ -267,7 +276,13 @@ int launch_normed_few(int epi, const GemmParams& p, int units, hipStream_t s) {
     const size_t lds = few_lds(p);
     auto sized = [&](auto t) {
         constexpr int TV = decltype(t)::value;
-        return epi == EPI_STORE ? go_few<TV, EPI_STORE>(p, units, lds, s) : epi == EPI_ROPE ? go_few<TV, EPI_ROPE>(p, units, lds, s) : go_few<TV, EPI_SILU>(p, units, lds, s);
+        auto go = [&](auto e) {
+            constexpr int EPI = decltype(e)::value;
+            return p.trace ? go_few<TV, EPI, true>(p, units, lds, s) : go_few<TV, EPI, false>(p, units, lds, s);
+        };
+        return epi == EPI_STORE  ? go(std::integral_constant<int, EPI_STORE>{})
+               : epi == EPI_ROPE ? go(std::integral_constant<int, EPI_ROPE>{})
+                                 : go(std::integral_constant<int, EPI_SILU>{});
     };
     return T == 1 ? sized(std::integral_constant<int, 1>{}) : T == 2 ? sized(std::integral_constant<int, 2>{}) : sized(std::integral_constant<int, 3>{});
 }

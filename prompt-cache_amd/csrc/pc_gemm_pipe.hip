@@ -12,7 +12,8 @@ using namespace pcg;
 
 namespace {
 
-template <int MT, int T, int EPI, int U>
+// TRACE (pc_dev_gemm_trace): a kernel of its own, since the places to stamp at cost 2 % of o_proj's
+template <int MT, int T, int EPI, int U, bool TRACE>
 __global__ __launch_bounds__(kThreads) void gemm_pipe_kernel(const GemmParams p) {
     constexpr int TT = EPI == EPI_SILU ? 2 * T : T, TPI = EPI == EPI_SILU ? 2 : 1;       // tiles, tiles of an output item
     constexpr int kRT = MT * TT < 8 ? MT * TT : 8, IPR = kRT / TPI;                      // tiles, items of a round of the reduction (64 KiB at most)
@@ -21,6 +22,7 @@ __global__ __launch_bounds__(kThreads) void gemm_pipe_kernel(const GemmParams p)
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int KS = p.KS, bx = blockIdx.x, by = blockIdx.y;
+    if (TRACE) trace_stamp(p, bx, by, wave, 0);
     int ks0, ks1;
     wave_k_range<false>(p, by, wave, ks0, ks1);
     int tile[TT];
@@ -81,6 +83,7 @@ __global__ __launch_bounds__(kThreads) void gemm_pipe_kernel(const GemmParams p)
         if (kb + 2 * U < ks1) issue(A, kb + 2 * U);
         consume(B, kb + U);
     }
+    if (TRACE) trace_stamp(p, bx, by, wave, 1);
     // the waves' shares in wave order, one output item a wave and round
 #pragma unroll
     for (int r = 0; r < ROUNDS; ++r) {
@@ -95,6 +98,7 @@ __global__ __launch_bounds__(kThreads) void gemm_pipe_kernel(const GemmParams p)
             }
         }
         lds_barrier();
+        if (TRACE && r == 0) trace_stamp(p, bx, by, wave, 2);
         const int item = r * IPR + wave;
         if (wave < IPR && item < NOUT) {
             const int a = item / T, t = item - a * T;
@@ -107,12 +111,17 @@ __global__ __launch_bounds__(kThreads) void gemm_pipe_kernel(const GemmParams p)
             tile_epilogue<EPI>(p, v, u, a * 16 + m, bx * T + t, g, by);
         }
     }
+    if (TRACE) { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); trace_stamp(p, bx, by, wave, 3); }
 }
 
 template <int MT, int T, int EPI>
 int go(const GemmParams& p, int units, hipStream_t s) {
     constexpr int U = EPI != EPI_SILU && (T == 4 || (MT == 1 && T == 3)) ? 2 : 1;
-    hipLaunchKernelGGL((gemm_pipe_kernel<MT, T, EPI, U>), dim3(pc_ceil_div(units, T), p.kslices), dim3(kThreads), 0, s, p);
+    const dim3 grid(pc_ceil_div(units, T), p.kslices);
+    if (p.trace)
+        hipLaunchKernelGGL((gemm_pipe_kernel<MT, T, EPI, U, true>), grid, dim3(kThreads), 0, s, p);
+    else
+        hipLaunchKernelGGL((gemm_pipe_kernel<MT, T, EPI, U, false>), grid, dim3(kThreads), 0, s, p);
     return pc_check_launch("gemm_pipe_kernel");
 }
 
