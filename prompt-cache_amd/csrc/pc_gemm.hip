@@ -59,11 +59,14 @@ int launch_MT(int epi, const GemmParams& p, int T, int units, hipStream_t s) {
     if (!forced && normed_few_takes(epi, p)) return launch_normed_few(epi, p, units, s);
     if (!p.w8 && !p.xn && p.xf_lo) {
         // Five tiles a workgroup where they fill a round of the chip that eight leave a third empty (13b's down_proj and o_proj in four slices, us, eight / five: 20 rows
-        // 30.3 / 25.3 and 14.6 / 13.2, 40 rows, four 42.5 / 29.5 and 19.5 / 15.9), and up to 32 rows of one slice instead of four where tile images are whole multiples of
-        // 64 KB, since the starts of four of them lie on the same channels (1024 tiles, K = 4096: 12 rows 29.7 / 25.3, 20 rows 30.9 / 26.6, 64 rows 35.7 / 36.4).
+        // 30.3 / 25.3 and 14.6 / 13.2, 40 rows, four 42.5 / 29.5 and 19.5 / 15.9), and up to 32 rows of one slice instead of four where tile images are 64 KB (up to
+        // 16 rows) or 128 KB, since the starts of four of them lie on the same channels, of more than 840 tiles, since five leave more CUs empty.  us, four / five: K = 4096, 1024
+        // tiles, 5 rows 29.8 / 25.6, 12 29.2 / 26.4, 20 30.7 / 27.7, 32 31.8 / 29.2, 864 tiles 25.4 / 22.7, 26.0 / 24.4, 27.8 / 26.7, 29.1 / 28.9, 800 tiles 22.7 / 21.7,
+        // 23.6 / 23.6, 25.7 / 26.6, 27.6 / 29.1; K = 2048, 992 tiles 14.9 / 13.4, 15.2 / 14.3, 16.0 / 15.9, 16.5 / 16.8, 864 tiles 12.9 / 11.7, 13.2 / 12.8, 14.1 / 14.4,
+        // 14.7 / 15.1; K = 6144, 992 tiles 34.4 / 36.4, 35.1 / 38.2, 38.2 / 40.4, 40.6 / 43.4; K = 8192 44.5 / 48.1, 44.6 / 49.2, 47.7 / 50.0, 50.8 / 52.7.
         const bool five = mt <= 2 ? epi != EPI_SILU : epi == EPI_STORE;
         if (five && !forced && T == 8 && pc_ceil_div(units * p.kslices, 5) <= 256) T = 5;
-        if (five && !forced && T == 4 && mt <= 2 && p.kslices == 1 && p.KS % 64 == 0) T = 5;
+        if (five && !forced && T == 4 && mt <= 2 && p.kslices == 1 && units > 840 && (p.KS == 128 || (p.KS == 64 && mt == 1))) T = 5;
         if (five && T == 5 && mt <= 2) return launch_pipe(epi, p, T, units, s);
         // (33 to 64 rows take three pairs at most: two, where three are a second round of the chip that is emptier.  13b's gate|up, 40 rows 81.5 / 67.2)
         if (mt > 2 && epi == EPI_SILU && T > 3 && !forced) {

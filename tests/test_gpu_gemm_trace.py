@@ -48,3 +48,14 @@ def test_two_planes(M, N, K, slices, workgroups):
     n.gemm_skinny(wf, hi, lo, M, N, K, n.EPI_STORE, y=z, ldy=N, kslices=slices)
     look(stamped(lambda: n.gemm_skinny(wf, hi, lo, M, N, K, n.EPI_STORE, y=y, ldy=N, kslices=slices)), workgroups)
     assert torch.equal(y, z)
+
+
+# five tiles a workgroup only where they are the faster: images of 64 KB (up to 16 rows) and 128 KB, more than 840 tiles
+@pytest.mark.parametrize("M,K,tiles,each", [(5, 4096, 1024, 5), (20, 4096, 841, 5), (32, 4096, 864, 5), (20, 4096, 832, 4), (12, 4096, 800, 4), (12, 2048, 1024, 5), (20, 2048, 1024, 4),
+                                            (12, 6144, 1000, 4), (20, 8192, 1000, 4), (12, 4128, 1000, 4)])
+def test_five_tiles_a_workgroup(M, K, tiles, each):
+    n, N = _n(), 16 * tiles
+    wf, hi, lo, want = operands(M, N, K)
+    y = torch.zeros((M, N), device=DEV)
+    look(stamped(lambda: n.gemm_skinny(wf, hi, lo, M, N, K, n.EPI_STORE, y=y, ldy=N)), -(-tiles // each))
+    assert float((y.double() - want).norm() / want.norm()) < 1e-6
