@@ -12,8 +12,11 @@ using namespace pcg;
 
 namespace {
 
+// ODD: shares of an odd number of blocks, where the second of the last pair is not there (and not read; asked for unseen, as the other shares' all are, it cost as much as one
+// that counts.  us, unseen / so: 800 tiles, 12 and 32 rows, K = 512 6.1 / 5.0 and 7.5 / 5.8, K = 1536 11.6 / 10.4 and 14.5 / 12.4, K = 2560 16.5 / 15.1 and 20.7 / 18.8; even ones the
+// other way round, K = 1024, 12 rows 8.0 / 8.2, o_proj in four slices 9.0 / 9.3).
 // TRACE (pc_dev_gemm_trace): a kernel of its own, since the places to stamp at cost 2 % of o_proj's
-template <int MT, int T, int EPI, int U, bool TRACE>
+template <int MT, int T, int EPI, int U, bool ODD, bool TRACE>
 __global__ __launch_bounds__(kThreads) void gemm_pipe_kernel(const GemmParams p) {
     constexpr int TT = EPI == EPI_SILU ? 2 * T : T, TPI = EPI == EPI_SILU ? 2 : 1;       // tiles, tiles of an output item
     constexpr int kRT = MT * TT < 8 ? MT * TT : 8, IPR = kRT / TPI;                      // tiles, items of a round of the reduction (64 KiB at most)
@@ -78,7 +81,7 @@ __global__ __launch_bounds__(kThreads) void gemm_pipe_kernel(const GemmParams p)
     };
     issue(A, ks0);
     for (int kb = ks0; kb < ks1; kb += 2 * U) {
-        issue(B, kb + U);
+        if (!ODD || kb + U < ks1) issue(B, kb + U);
         consume(A, kb);
         if (kb + 2 * U < ks1) issue(A, kb + 2 * U);
         consume(B, kb + U);
@@ -118,10 +121,13 @@ template <int MT, int T, int EPI>
 int go(const GemmParams& p, int units, hipStream_t s) {
     constexpr int U = EPI != EPI_SILU && (T == 4 || (MT == 1 && T == 3)) ? 2 : 1;
     const dim3 grid(pc_ceil_div(units, T), p.kslices);
+    const bool odd = pc_ceil_div(pc_ceil_div(pc_ceil_div(p.KS, p.kslices), kWaves), U) & 1;
     if (p.trace)
-        hipLaunchKernelGGL((gemm_pipe_kernel<MT, T, EPI, U, true>), grid, dim3(kThreads), 0, s, p);
+        hipLaunchKernelGGL((gemm_pipe_kernel<MT, T, EPI, U, true, true>), grid, dim3(kThreads), 0, s, p);
+    else if (odd)
+        hipLaunchKernelGGL((gemm_pipe_kernel<MT, T, EPI, U, true, false>), grid, dim3(kThreads), 0, s, p);
     else
-        hipLaunchKernelGGL((gemm_pipe_kernel<MT, T, EPI, U, false>), grid, dim3(kThreads), 0, s, p);
+        hipLaunchKernelGGL((gemm_pipe_kernel<MT, T, EPI, U, false, false>), grid, dim3(kThreads), 0, s, p);
     return pc_check_launch("gemm_pipe_kernel");
 }
 
