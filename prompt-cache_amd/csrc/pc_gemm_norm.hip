@@ -255,8 +255,10 @@ size_t few_lds(const GemmParams& p) { return (size_t)p.M * 2 * (pc_ceil_div(p.KS
 
 namespace pcg {
 
+// Not plain results over a share of up to four k-steps a wave (us, 1 row, blocks of k-steps / so: K = 512, 300 and 800 tiles 4.4 / 4.8 and 5.9 / 7.7, K = 1024 5.4 / 5.3 and
+// 8.0 / 9.1; K = 1152 0.90 and 0.96 of it, 1536 6.4 / 5.7 and 10.6 / 9.6, 2048 7.5 / 6.6 and 14.4 / 11.3; gated, K = 512, 300 and 860 pairs 5.9 / 5.5 and 8.7 / 7.9).
 bool normed_few_takes(int epi, const GemmParams& p) {
-    return p.xn && !p.w8 && p.M <= kFewRows && p.kslices == 1 && p.kskew == 0 && (epi == EPI_STORE || epi == EPI_ROPE || epi == EPI_SILU) && few_lds(p) <= kFewLds;
+    return p.xn && (epi == EPI_SILU || p.KS > 4 * kWaves) && !p.w8 && p.M <= kFewRows && p.kslices == 1 && p.kskew == 0 && (epi == EPI_STORE || epi == EPI_ROPE || epi == EPI_SILU) && few_lds(p) <= kFewLds;
 }
 
 // Tiles (pairs of tiles) a workgroup: the number that leaves the fewest of the chip's 256 CUs without one in the last round, of 3 (of 2, where tile images are not
@@ -285,6 +287,22 @@ int launch_normed_few(int epi, const GemmParams& p, int units, hipStream_t s) {
                                  : go(std::integral_constant<int, EPI_SILU>{});
     };
     return T == 1 ? sized(std::integral_constant<int, 1>{}) : T == 2 ? sized(std::integral_constant<int, 2>{}) : sized(std::integral_constant<int, 3>{});
+}
+
+// Where single k-steps, the next under way, are the faster: not where a block of four holds a wave's whole share; over more than 4096 of K only over odd multiples of 512 (else tiles
+// begin on the same channels, and the more steps a workgroup asks for at a time the better); two tiles a workgroup, few bytes under way, only with the loads of ten rows
+// beside them.  us, blocks of four / so, at 3, 8 and 16 rows: plain, 300 tiles (two), K = 512 4.5 / 4.4, 4.8 / 4.8, 5.3 / 5.0, K = 1024 5.5 / 6.2, 5.9 / 6.5, 6.6 / 6.6, K = 2048
+// 7.5 / 8.8, 8.1 / 8.9, 9.9 / 9.6, K = 4096 12.1 / 14.3, 13.2 / 14.4, 15.8 / 15.2, K = 5120 15.6 / 19.3, 16.4 / 18.0, 18.8 / 19.2, K = 8192 21.6 / 26.4, 24.0 / 26.9, 26.5 / 27.2; 640
+// (three), K = 1024 1.07, 1.05, 1.00 of it, K = 1536 0.92, 0.88, 0.87, 4096 0.95, 1.00, 0.95, 5120 1.04, 1.08, 1.05, 8192 1.07, 1.10, 1.07, 11008 1.06, 1.06, 1.02; 960 (four) 4096 0.99,
+// 1.01, 0.93, 5120 1.02, 1.03, 1.00, 8192 1.03, 1.05, 1.02, 13824 0.96, 0.96, 0.92; gated, 688 pairs (three), K = 4096 31.3 / 32.0, 31.7 / 31.8, 33.2 / 32.0, 640, K = 1024 1.02, 1.02, 0.99,
+// K = 2048 0.93, 0.91, 0.90, 5120 1.01, 1.02, 1.01, 8192 1.09, 1.08, 1.06; 864 (four), K = 4096 44.5 / 45.4, 43.3 / 44.3, 43.5 / 43.8, 5120 53.1 / 52.1, 51.0 / 49.8, 52.7 / 50.7.  (Where a
+// launch's weights lie moves such times by up to 3 %.)
+bool normed_takes(int epi, const GemmParams& p, int T) {
+    const int share = pc_ceil_div(p.KS, kWaves);
+    const bool far = p.KS % 32 == 16;
+    if (epi == EPI_SILU) return T == 4 ? p.KS % 128 != 0 : share <= 16 ? share != 4 && (p.KS % 128 != 0 || p.M > 9) : far;
+    if (share <= 4) return share <= 2;
+    return T > 2 ? share <= 16 || far : share <= 16 && p.M > 9;
 }
 
 // (two to four tiles, or pairs of tiles, a workgroup)

@@ -153,6 +153,17 @@ int by_tiles(int epi, const GemmParams& p, int T, int units, hipStream_t s) {
 }  // namespace
 
 namespace pcg {
+// Three and four tiles: plain results over up to 4096 of K a slice, beyond only over odd multiples of 512 (else tiles begin on the same channels, and the more steps a workgroup asks
+// for at a time the better); gated ones of up to sixteen rows not where a block of four k-steps holds a wave's share, nor over multiples of 4096.  us, one block after the
+// other / so: 560 and 800 tiles, 4 rows, K = 2048 9.2 / 8.9 and 13.0 / 12.7, 4096 14.8 / 14.9 and 23.4 / 23.6, 5120 17.7 / 18.6 and 23.4 / 23.8, 7168 23.5 / 24.5 and 31.1 / 32.0;
+// 32 rows, K = 2048 11.5 / 11.6 and 14.8 / 14.3, 4096 19.0 / 19.7 and 26.1 / 26.8, 5120 23.5 / 25.3 and 30.4 / 31.2, 7168 31.6 / 34.1 and 40.9 / 42.5; 20 rows, K = 6656, 640 and 900
+// tiles 28.9 / 28.0 and 35.2 / 34.7, 11008 46.8 / 48.8 and 61.2 / 62.8; gated, 688 pairs, 12 rows, K = 1024 11.4 / 12.0, 2048 17.3 / 16.3, 4096 29.7 / 30.8, 5120 40.0 / 38.8, 32
+// rows, 640 pairs, K = 5120 43.2 / 42.0.  (Where a launch's weights lie moves such times by up to 3 %.)
+bool pipe_takes(int epi, const GemmParams& p) {
+    if (epi == EPI_SILU) return p.M > 16 || (pc_ceil_div(p.KS, kWaves) != 4 && p.KS % 128 != 0);
+    return p.KS <= 128 * p.kslices || p.KS % 32 == 16;
+}
+
 int launch_pipe(int epi, const GemmParams& p, int T, int units, hipStream_t s) {
     return p.M <= 16 ? by_tiles<1>(epi, p, T, units, s) : by_tiles<2>(epi, p, T, units, s);
 }

@@ -965,8 +965,10 @@ void launch_w8(const GemmParams& p, dim3 grid, dim3 block, hipStream_t s) {
 // the norm inside the launch (pc_gemm_norm.hip): one and two rows, and two to four tiles a workgroup
 bool normed_few_takes(int epi, const GemmParams& p);
 int launch_normed_few(int epi, const GemmParams& p, int units, hipStream_t s);
+bool normed_takes(int epi, const GemmParams& p, int T);
 int launch_normed(int epi, const GemmParams& p, int T, int units, hipStream_t s);
 // two planes, up to 32 rows, three to five tiles a workgroup (pc_gemm_pipe.hip)
+bool pipe_takes(int epi, const GemmParams& p);
 int launch_pipe(int epi, const GemmParams& p, int T, int units, hipStream_t s);
 
 template <int MT, int T, int EPI>
@@ -977,13 +979,13 @@ int launch_one(const GemmParams& p, int units, hipStream_t s) {
     const dim3 grid(pc_ceil_div(units, T), p.kslices), block(kThreads);
     const bool two = p.xf_lo != nullptr;
     // (two planes without the norm, three and four tiles of up to two row tiles: pc_gemm_pipe.hip)
-    constexpr bool kPiped = MT <= 2 && (T == 3 || T == 4);
-    if constexpr (kPiped)
-        if (two && !p.xn && !p.w8) return launch_pipe(EPI, p, T, units, s);
+    if constexpr (MT <= 2 && (T == 3 || T == 4))
+        if (two && !p.xn && !p.w8 && pipe_takes(EPI, p)) return launch_pipe(EPI, p, T, units, s);
     // (the norm inside the launch, fp16 weights, one row tile: pc_gemm_norm.hip)
-    constexpr bool kNormed = MT == 1 && T >= 2 && T <= 4 && (EPI == EPI_STORE || EPI == EPI_ROPE || EPI == EPI_SILU);
-    if constexpr (kNormed)
-        if (p.xn && !p.w8) return launch_normed(EPI, p, T, units, s);
+    if constexpr (MT == 1 && T >= 2 && T <= 4 && (EPI == EPI_STORE || EPI == EPI_ROPE || EPI == EPI_SILU))
+        if (p.xn && !p.w8 && normed_takes(EPI, p, T)) return launch_normed(EPI, p, T, units, s);
+    // (... which take every gated launch of two row tiles in two planes)
+    [[maybe_unused]] constexpr bool kPiped = MT == 2 && (T == 3 || T == 4) && EPI == EPI_SILU;
 #define PC_GO(UV)                                                                                     \
     do {                                                                                              \
         if (p.w8) {   /* int8 weights: split-precision activations only.  Same k-steps per block as fp16 (half the   */ \
@@ -993,7 +995,7 @@ int launch_one(const GemmParams& p, int units, hipStream_t s) {
             launch_w8<MT, T, EPI, UW, UA>(p, grid, block, s);                                         \
             break;                                                                                    \
         }                                                                                             \
-        if constexpr (MT <= 2 && EPI != EPI_ADD && !kNormed) {                                        \
+        if constexpr (MT <= 2 && EPI != EPI_ADD) {                                                     \
             if (p.xn) {   /* (two row tiles of fp32 rows: eight k-steps of them in flight spill) */       \
                 constexpr int UN = (MT == 2 && (UV) > 4) ? 4 : (UV);                                  \
                 hipLaunchKernelGGL((gemm_skinny_kernel<MT, T, EPI, true, UN, true>), grid, block, 0, s, p); \

@@ -50,3 +50,16 @@ def test_gated(M, inter, K):
     want = torch.nn.functional.silu(z[:, :inter]) * z[:, inter:]
     got = n.from_act_frags(hi, M).double() + n.from_act_frags(lo, M).double()
     assert float((got - want).norm() / want.norm()) < 2e-6     # (and the exponential's 1e-6)
+
+
+# either side of the lines between single k-steps and blocks of four: shares of two, three, four and five k-steps, nine and ten rows at two tiles a workgroup, 4096 and more of K
+@pytest.mark.parametrize("M", [1, 9, 10])
+@pytest.mark.parametrize("N,K", [(4800, 512), (4800, 544), (10240, 1024), (10240, 1056), (15376, 1056), (4800, 4096), (4800, 4128), (10240, 4608), (10240, 5120), (12832, 4608)])
+def test_store_on_either_side_of_the_lines(M, N, K):
+    test_store(M, N, K)
+
+
+@pytest.mark.parametrize("M", [3, 9, 10])
+@pytest.mark.parametrize("inter,K", [(4800, 1024), (4800, 1056), (11008, 4096), (11008, 4128), (11008, 4608), (13824, 4096), (13824, 4160)])
+def test_gated_on_either_side_of_the_lines(M, inter, K):
+    test_gated(M, inter, K)

@@ -89,3 +89,16 @@ def test_vocabularies(M, N, K):
     assert rel(y, want) < 1e-6
     n.gemm_skinny(wf, hi, None, M, N, K, n.EPI_STORE, y=y, ldy=N)          # (rows rounded to 11 bits: a uniform error of 2^-12 at most, 2^-12 / sqrt(3) in the mean)
     assert rel(y, want) < 2.0 ** -12
+
+
+# either side of the lines between the next k-steps under way and blocks one after the other: shares of an odd and an even number of blocks, 4096 and more of K, gated ones
+@pytest.mark.parametrize("M", [12, 16, 17, 32])
+@pytest.mark.parametrize("N,K,slices", [(8992, 768, 1), (12832, 1536, 1), (12832, 4096, 1), (12832, 4128, 1), (8992, 4608, 1), (8992, 5120, 1), (4096, 2560, 4)])
+def test_stores_on_either_side_of_the_lines(M, N, K, slices):
+    test_stores_and_sums(M, N, K, slices)
+
+
+@pytest.mark.parametrize("M", [16, 17])
+@pytest.mark.parametrize("inter,K", [(11008, 1024), (11008, 1056), (11008, 4096), (13824, 4096), (13824, 4128)])
+def test_gated_on_either_side_of_the_lines(M, inter, K):
+    test_gated(M, inter, K)
