@@ -224,6 +224,25 @@ class GreedyLoop:
         return e0.elapsed_time(e1)
 
 
+def ks_forms(hidden: int):
+    """(o_proj, down_proj, fewest rows): tiles a workgroup and slices of K of the N = hidden projections of up to 16 rows that are reduced inside their launch
+    (pc_gemm_skinny_ks); None: a tile a workgroup (EPI_ADD)."""
+    # Measured at 12 rows (tools/ks_micro.py, in-graph): down_proj (K = 11008) 22.75 -> 20.16 us at 2 tiles x 2 slices, every
+    # other shape of either projection loses to the one-tile launch (o_proj 9.4 -> 10.4 .. 13.5 us; one row: 19.0 -> 20.3 us):
+    # the in-launch reduction costs ~3 us, only the long-K launch with its 2:1 activation traffic earns it back.
+    # Where a tile each is more than the 256 CUs (hidden 5120: 320), whichever of these fills a round of them, o_proj included.  4 x 3 (hidden 4240 .. 5440) at any number
+    # of rows, the others (4 x 2 for 6352 .. 8192, 8 x 3 for 8464 .. 10880) beyond eight, where the rows are a second reading of the planes for a tile each.  us, one tile (two of them
+    # a workgroup) / these, o_proj and down_proj, 1 row: hidden 4608 12.3 / 11.3 and 26.4 / 23.8, 5120 13.1 / 12.9 and 30.5 / 25.1, 5376 14.8 / 13.6 and 31.1 / 27.3, 6656 17.9 / 18.2 and
+    # 42.8 / 43.3, 7168 19.0 / 19.7 and 47.8 / 49.6, 8192 27.3 / 29.0 and 71.2 / 74.7, 8704 28.9 / 28.6 and 69.4 / 65.2, 10752 37.6 / 39.5 and 93.6 / 96.7; 12 rows: 5120 15.1 / 13.4
+    # and 35.8 / 26.2, 6656 20.5 / 19.6 and 48.6 / 45.2, 7168 21.6 / 21.1 and 54.6 / 52.0, 8192 29.2 / 27.6 and 79.5 / 75.3, 8704 32.7 / 29.4 and 80.0 / 67.2, 10752 41.6 / 39.7 and
+    # 105.0 / 96.1; 8 rows as one, 9 as twelve (7168 47.4 / 49.3, 54.4 / 51.9).  (2 x 2 loses everywhere here: 5120, 12 rows 18.4 and 41.5.)
+    tiles = -(-hidden // 16)
+    for t, k in ((4, 3), (4, 2), (8, 3)):
+        if tiles > 256 and 200 <= -(-tiles // t) * k <= 256:
+            return (t, k), (t, k), 1 if (t, k) == (4, 3) else 9
+    return None, (2, 2), 5
+
+
 class LlamaHIP:
     """Weights live on one MI355X in fp16; ``wqkv`` and ``wgu`` are the row-concatenated q|k|v and
     gate|up projections so each is one GEMM."""
@@ -303,21 +322,14 @@ class LlamaHIP:
         # 3.933 ms fused against 3.907 / 3.908 ms with attn_combine_kernel (gpurun_out/r3b)
         self._attn_counters = torch.zeros(8192, dtype=torch.int32, device=self.device) \
             if os.environ.get("PC_ATTN_FUSED", "0") == "1" else None
-        # N = hidden projections of the <= 16-row stack with K split across workgroups and the reduction inside the launch
-        # (pc_gemm_skinny_ks): "tiles,slices" per projection, empty = the one-tile-per-workgroup EPI_ADD launch
-        def _ks(env, default):
-            v = os.environ.get(env, default)
+        # (tools/ks_micro.py; "tiles,slices", empty: the one-tile launch)
+        def _ks(v):
             return tuple(int(t) for t in v.split(",")) if v else None
-        # Measured at 12 rows (tools/ks_micro.py, in-graph): down_proj (K = 11008) 22.75 -> 20.16 us at 2 tiles x 2 slices, every
-        # other shape of either projection loses to the one-tile launch (o_proj 9.4 -> 10.4 .. 13.5 us; one row: 19.0 -> 20.3 us):
-        # the in-launch reduction costs ~3 us, only the long-K launch with its 2:1 activation traffic earns it back.
-        # Where a tile each is more than the 256 CUs (hidden 5120: 320), whichever of these fills a round of them, o_proj and one row included: 4 x 3, 240
-        # workgroups; us, one tile (two of them a workgroup) / 2 x 2 / 4 x 3, down_proj 12 rows 35.4 / 41.0 / 26.0, 1 row 30.2 / 40.1 / 24.9, o_proj 12 rows
-        # 14.9 / 18.0 / 13.4, 1 row 13.1 / 17.7 / 12.8.
-        tiles = -(-shape.hidden_size // 16)
-        fits = [f"{t},{k}" for t, k in ((4, 3), (4, 2), (8, 3)) if tiles > 256 and 200 <= -(-tiles // t) * k <= 256][:1]
-        self.ks_o, self.ks_down = _ks("PC_KS_O", fits[0] if fits else ""), _ks("PC_KS_DOWN", fits[0] if fits else "2,2")
-        self.ks_min_rows = 1 if fits else 5      # ... and, where a tile each is one round, only with more than 4 rows (decode keeps the one-tile launch)
+        self.ks_o, self.ks_down, self.ks_min_rows = ks_forms(shape.hidden_size)
+        if "PC_KS_O" in os.environ:
+            self.ks_o = _ks(os.environ["PC_KS_O"])
+        if "PC_KS_DOWN" in os.environ:
+            self.ks_down = _ks(os.environ["PC_KS_DOWN"])
         self._ks_state = None      # (scratch, counters), lazily
         self._kv_only = False      # set per call (see __call__)
         self._past_lens = None     # set per call: per-row past lengths of a ragged-prefix encode batch
