@@ -187,34 +187,36 @@ __device__ __forceinline__ Frag<float> load8(const float* p) {
 }
 // A lane's part of a k-step of which PARTS lie side by side (pb_linear_parts.h), from `piece_at` on in the row: such that every load instruction of a wave
 // reads whole 64-byte lines, PARTS of them in a row.  bf16: eight neighbouring elements; fp32: four, and the four 16 PARTS elements on (any order of k is
-// as good, as long as both operands have it).
-template <typename E>
+// as good, as long as both operands have it).  NEAR: eight neighbours in fp32 too, both halves of a line in two instructions one after the other: where a workgroup has the
+// lines of two matrices of sixteen rows under way (a gated unit in one run; us, 12 and 16 rows, weights from memory, lines apart / near: K = 768, 512 columns 7.93 / 7.22 and 1.09 of it,
+// K = 2048, 2048 columns 1.06 and 1.08, 4096 1.01 and 1.02 of it; beside another product the other way round, 0.95).
+template <typename E, bool NEAR = false>
 __device__ __forceinline__ int piece_at(int run, int group) {
-    return sizeof(E) == 2 ? 32 * run + 8 * group : 16 * run + 4 * group;
+    return sizeof(E) == 2 || NEAR ? 32 * run + 8 * group : 16 * run + 4 * group;
 }
-template <int PARTS>
+template <int PARTS, bool NEAR = false>
 __device__ __forceinline__ Frag<bf16_t> load_piece(const bf16_t* p) { return load8(p); }
-template <int PARTS>
+template <int PARTS, bool NEAR = false>
 __device__ __forceinline__ Frag<float> load_piece(const float* p) {
     Frag<float> f;
-    const f4 a = *reinterpret_cast<const f4*>(p), b = *reinterpret_cast<const f4*>(p + 16 * PARTS);
+    const f4 a = *reinterpret_cast<const f4*>(p), b = *reinterpret_cast<const f4*>(p + (NEAR ? 4 : 16 * PARTS));
 #pragma unroll
     for (int e = 0; e < 4; ++e) f.v[e] = a[e], f.v[4 + e] = b[e];
     return f;
 }
 // The same of weights; ONCE: nontemporal loads, for weights that are not in the caches and will not stay there
-template <int PARTS, bool ONCE>
+template <int PARTS, bool ONCE, bool NEAR = false>
 __device__ __forceinline__ Frag<bf16_t> weight_piece(const bf16_t* p) {
     if (!ONCE) return load_piece<PARTS>(p);
     Frag<bf16_t> f;
     f.v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
     return f;
 }
-template <int PARTS, bool ONCE>
+template <int PARTS, bool ONCE, bool NEAR = false>
 __device__ __forceinline__ Frag<float> weight_piece(const float* p) {
-    if (!ONCE) return load_piece<PARTS>(p);
+    if (!ONCE) return load_piece<PARTS, NEAR>(p);
     Frag<float> f;
-    const f4 a = __builtin_nontemporal_load(reinterpret_cast<const f4*>(p)), b = __builtin_nontemporal_load(reinterpret_cast<const f4*>(p + 16 * PARTS));
+    const f4 a = __builtin_nontemporal_load(reinterpret_cast<const f4*>(p)), b = __builtin_nontemporal_load(reinterpret_cast<const f4*>(p + (NEAR ? 4 : 16 * PARTS)));
 #pragma unroll
     for (int e = 0; e < 4; ++e) f.v[e] = a[e], f.v[4 + e] = b[e];
     return f;

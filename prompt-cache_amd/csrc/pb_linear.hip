@@ -348,7 +348,7 @@ __global__ __launch_bounds__(64 * SKW) void linear_skinny_kernel(pcb_linear_args
 template <typename E, int EPI, int PARTS, int U, bool LATE, int G, bool ONCE>
 __global__ __launch_bounds__(512) void linear_parts_kernel(pcb_linear_args a) {
     __shared__ f4 red[EPI == PCB_EPI_SILU_MUL ? 2 * G : G][8][64];
-    parts_block<E, EPI, PARTS, U, LATE, G, ONCE>(a, blockIdx.x, red);
+    parts_block<E, EPI, PARTS, U, LATE, G, ONCE, sizeof(E) == 4 && EPI == PCB_EPI_SILU_MUL && PARTS == 1>(a, blockIdx.x, red);
 }
 
 // ---- many rows: both panels travel to LDS by themselves ------------------------------------------------------------------------------

@@ -51,15 +51,15 @@ __device__ __forceinline__ f4 parts_total(const f4 (*red)[64], int lane) {
 }
 
 // Workgroup `block` of such a launch, 512 threads; red: [G, gated 2 G][8][64].  LATE: where a result goes is worked out behind the products.  G: blocks of
-// R columns a workgroup has, which share what it reads of the rows.
-template <typename E, int EPI, int PARTS, int U, bool LATE, int G, bool ONCE>
+// R columns a workgroup has, which share what it reads of the rows.  NEAR: load_piece().
+template <typename E, int EPI, int PARTS, int U, bool LATE, int G, bool ONCE, bool NEAR = false>
 __device__ __forceinline__ void parts_block(const pcb_linear_args& a, int block, f4 (*red)[8][64]) {
     constexpr bool TWO = EPI == PCB_EPI_SILU_MUL, ADD = EPI == PCB_EPI_SCALE_ADD;
     constexpr int R = 16 / PARTS, SKW = 8, T = TWO ? 2 : 1;
     const int tid = threadIdx.x, lane = tid & 63, wave = G > 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6, group = lane >> 4, l15 = lane & 15;
     const int K = a.K, N = a.N, n_lo = block * (R * G), g = a.n_batch > 0 ? blockIdx.z : 0;
     const int run = l15 / R, i = l15 % R;
-    const int m_a = i < a.M ? i : a.M - 1, at = piece_at<E>(run, group);
+    const int m_a = i < a.M ? i : a.M - 1, at = piece_at<E, NEAR>(run, group);
     const E* X = (const E*)a.x + g * a.x_batch_stride;
     const E* wrow[G * T];
 #pragma unroll
@@ -93,8 +93,8 @@ __device__ __forceinline__ void parts_block(const pcb_linear_args& a, int block,
             if (s0 + u * SKW < steps) {                                // (uniform over the wave)
                 const int k = 32 * PARTS * (s0 + u * SKW);
 #pragma unroll
-                for (int j = 0; j < G * T; ++j) fb[j][u] = weight_piece<PARTS, ONCE>(wrow[j] + k);
-                fa[u] = load_piece<PARTS>(xrow + k);
+                for (int j = 0; j < G * T; ++j) fb[j][u] = weight_piece<PARTS, ONCE, NEAR>(wrow[j] + k);
+                fa[u] = load_piece<PARTS, NEAR>(xrow + k);
             }
 #pragma unroll
         for (int u = 0; u < U; ++u)
