@@ -602,15 +602,8 @@ FewRows few_rows(const pcb_linear_args& a) {
     // the busiest CU smallest, the more the better.  Times of the rule before, 8 rows, K = 2048: 2568 columns (2) 0.93, 5136 (3) 0.78, 7424 (4) 0.80, 10272 (3)
     // 0.76, 32000 (4) 0.72; K = 4096 0.94, 0.77, 0.92 (2), 0.82, 0.74 (2); K = 1024 1.0, 0.89, 0.84, 0.91, 0.79; 4 rows, K = 2048 0.93, 0.89, 0.90, 0.88, 0.86.  One and
     // two rows only over K <= 1024 (10272 columns 0.85, 32000 0.79; K = 2048 1.02, 1.01).
-    if (bf && a.epilogue == PCB_EPI_STORE && a.n_batch == 0 && a.K % 64 == 0 && a.K >= 1024 && g2 > 256 && (a.M > 2 || a.K <= 1024)) {
-        FewRows f{2, true, 1};
-        int64_t least = 0;
-        for (int blocks = 1; blocks <= (a.K <= 2048 ? 4 : 3); ++blocks) {
-            const int64_t share = (pcb_ceil_div(pcb_ceil_div((int)g2, blocks), 256)) * (int64_t)blocks;
-            if (blocks == 1 || share <= least) f.blocks = blocks, least = share;
-        }
-        return f;
-    }
+    if (bf && a.epilogue == PCB_EPI_STORE && a.n_batch == 0 && a.K % 64 == 0 && a.K >= 1024 && g2 > 256 && (a.M > 2 || a.K <= 1024))
+        return {2, true, pcb_parts_blocks(g2, a.K).blocks};
     if (a.M <= 4 && a.K % 128 == 0 && a.K >= (gated && bf ? 2048 : 1024) && g4 <= (a.M <= 2 || gated || a.K >= 2048 ? 768 : 512)) return {4, late};
     // two runs, of more than four rows not where 16 columns each are one round of the chip and eight are two (there the kernel above over a deep k: 8 rows,
     // K = 4096, 2048 columns 9.6 / 10.3 / 7.1, 2560 9.8 / 10.6 / 10.6, 4096 13.6 / 11.6 / 11.3, 8192 18.3 / 20.1 / 20.4, 16384 35.8 / 36.0 / 36.4)

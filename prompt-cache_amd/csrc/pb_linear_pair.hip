@@ -169,16 +169,21 @@ int pair(const pcb_linear_args& a, const pcb_linear_args& b, hipStream_t stream)
             hipLaunchKernelGGL((linear_pair_kernel<E, EPI, P, decltype(u)::value, GA, decltype(late)::value, false>), dim3(na + nb), dim3(512), 0, stream, a, b, na);
         return pcb_check_launch("linear_pair_kernel");
     };
-    // Two runs of k side by side up to eight rows; results' places behind the products where the second is gated, fp32 of many plain columns in one run.
-    // Weights from memory, us, one run (as all were that are not marked *) / two: bf16 1 row, 2048 and 4096 gated, K = 2048 12.5 / 9.4, 8 rows 13.7 / 10.9,
-    // places ahead 14.3; 2560 and 5120, K = 2560 20.3 / 16.8; 2560 + 8192 columns, K = 2048, 8 rows 15.0 / 14.0, 1 row 10.5 * / 9.6; 1024 and 2048 gated, K = 1024, 8
-    // rows 6.5 / 6.7, 4 rows 6.0 / 6.3; 512 + 1024 gated, K = 512 3.7 / 3.9; fp32 5.5 / 4.1; 2048 and 4096 gated, K = 2048, fp32, 2 rows 18.7 * / 16.8 with one
-    // k-step a time and places behind, 8 rows 21.9 * / 19.8; 2560 + 8192 columns, 8 rows 22.8 / 24.4.  The first product's blocks two a workgroup where that is a round
-    // of the chip less: 1536 and 3072 gated, K = 1536, 8 rows 9.1 / 8.0, 3072 and 6144 23.4 / 20.9; 2048 and 4096 10.9 / 11.9.
+    // Two runs of k side by side up to eight rows, while the workgroups are not too many for a k of so few steps; results' places behind the products where the second is gated,
+    // ahead of them over a k of up to 1536.  Weights from memory, us, one run (as all were that are not marked *) / two: bf16 1 row, 2048 and 4096 gated, K = 2048
+    // 12.5 / 9.4, 8 rows 13.7 / 10.9, places ahead 14.3; 2560 and 5120, K = 2560 20.3 / 16.8; 2560 + 8192 columns, K = 2048, 8 rows 15.0 / 14.0, 1 row 10.5 * / 9.6; K = 1024, places ahead, 512
+    // and 512 gated, 1 and 8 rows 5.2 / 4.4 and 6.3 / 5.3, 1024 and 1024 5.6 / 4.9 and 6.6 / 5.8, 1024 and 2048 8 rows 6.5 / 6.1 (behind 6.7), 2700 and 2700 8.3 / 9.8, K = 1152, 2048 and 2048, 1 and 8 rows, ahead and behind 5.8 / 6.4 and 6.9 / 7.4, K = 1536 0.98 and 0.99 of it; plain, 8 rows, K = 1024,
+    // 3072 + 9216 columns 1.00 / 1.08, 8192 + 24576 1.00 / 1.07, K = 1536 3072 + 9216 1.00 / 1.08, K = 2048 1.00 / 0.97; 512 + 1024 gated, K = 512 3.7 / 3.9; fp32 5.5 / 4.1, 2048 and 2048
+    // gated, K = 512 1.00 / 0.92, 2700 and 2700 8.4 / 9.2, 3072 and 3072, K = 512, 8 rows 8.4 / 9.9, 8192 and 8192 14.8 / 20.0, K = 768 20.1 / 25.7, K = 1024, 4 and 8 rows 1.00 / 0.97 and 1.00 / 1.16; 2048 and 4096
+    // gated, K = 2048, fp32, 2 rows 18.7 * / 16.8 with one k-step a time and places behind, 8 rows 21.9 * / 19.8; 2560 + 8192 columns, 8 rows 22.8 / 24.4.  The first product's blocks two a
+    // workgroup where that is a round of the chip less: 1536 and 3072 gated, K = 1536, 8 rows 9.1 / 8.0, 3072 and 6144 23.4 / 20.9; 2048 and 4096 10.9 / 11.9.
     constexpr bool bf = sizeof(E) == 2;
-    const bool gated = b.epilogue == PCB_EPI_SILU_MUL, deep = a.K >= 1024 && b.K >= 1024;
+    const bool gated = b.epilogue == PCB_EPI_SILU_MUL;
+    const int K = a.K < b.K ? a.K : b.K;
     const int64_t w_rows = (int64_t)a.N + (gated ? 2 : 1) * (int64_t)b.N;
-    const bool two = a.M <= 8 && (gated ? !bf || (a.K > 1024 && b.K > 1024) : deep) && splits(a, 2) && splits(b, 2) && (bf || gated || w_rows <= 8192 || a.M <= 4);
+    const bool few = w_rows <= 7168, two = a.M <= 8 && splits(a, 2) && splits(b, 2) &&
+                                           (gated ? (bf ? K > 1024 || (K == 1024 && few) : K > 1024 || few || (K == 1024 && (w_rows <= 16384 || a.M <= 4)))
+                                                  : K >= 1024 && (w_rows <= 8192 || a.M <= 4 || (bf && K > 1536)));
     auto yes = std::true_type{};
     auto no = std::false_type{};
     using Plain = std::integral_constant<int, bf ? 4 : 2>;
@@ -189,10 +194,11 @@ int pair(const pcb_linear_args& a, const pcb_linear_args& b, hipStream_t stream)
     std::integral_constant<int, PCB_EPI_SILU_MUL> epi;
     if (!two) return go(epi, One{}, Plain{}, One{}, no);
     if constexpr (bf) {
+        if (K < 1536 && few) return go(epi, Two{}, Four{}, One{}, no);
         const int na = pcb_ceil_div(a.N, 8), nb = pcb_ceil_div(b.N, 8);
         return pcb_ceil_div(nb + (na + 1) / 2, 256) < pcb_ceil_div(nb + na, 256) ? go(epi, Two{}, Four{}, Two{}, yes) : go(epi, Two{}, Four{}, One{}, yes);
     } else {
-        return a.K > 1024 && b.K > 1024 ? go(epi, Two{}, One{}, One{}, yes) : go(epi, Two{}, Two{}, One{}, no);
+        return K > 1024 ? go(epi, Two{}, One{}, One{}, yes) : go(epi, Two{}, Two{}, One{}, no);
     }
 }
 
@@ -233,11 +239,14 @@ static int pair_form(const pcb_linear_args& a, const pcb_linear_args& b) {
     if (a.dtype != b.dtype || a.M != b.M || a.M <= 0 || a.n_batch != 0 || b.n_batch != 0 || a.epilogue != PCB_EPI_STORE || b.epilogue == PCB_EPI_SCALE_ADD ||
         !pcb_linear_pieces(a) || !pcb_linear_pieces(b) || !pair_apart(a, b))
         return 0;
-    // (More than four rows of bf16 with many plain columns as two: there each is the faster by itself, with several blocks of columns a workgroup.  us, one launch / two,
-    // 8 rows, 2560 + 8192 columns, K = 2048 14.0 / 14.6, 3840 + 12288, K = 3072 24.9 / 23.8, 5120 + 16384, K = 4096 42.6 / 37.2; gated 3072 and 6144, K = 3072
-    // 20.9 / 25.0, 1 row 17.7 / 20.3, 4096 and 8192 32.2 / 36.6, 16 rows 44.1 / 49.0; fp32 2048 and 4096, 9 and 16 rows 23.6 / 27.5 and 26.5 / 29.1; plain, 2560 + 8192
-    // columns, 9 and 16 rows 15.1 / 18.9 and 17.6 / 20.8.)
-    const bool heavy = a.dtype == PCB_BF16 && b.epilogue == PCB_EPI_STORE && a.M > 4 && a.M <= 8 && ((int64_t)a.N * a.K + (int64_t)b.N * b.K) * 2 > 80000000;
+    // (More than four rows of bf16 with many plain columns as two, where the busiest CU has no more blocks of columns then: each is the faster by itself, with several of them a
+    // workgroup.  us, one launch / two, 8 rows, 2560 + 8192 columns, K = 2048 14.0 / 14.6, 5136 + 15408, K = 2048 22.4 / 20.7, 8192 + 24576, K = 1536 26.9 / 23.5, 3840 + 12288, K = 3072
+    // 24.9 / 23.8, 2700 + 8100, K = 4096 24.4 / 22.9, 3072 + 9216, K = 4096 (six blocks / two and five) 26.2 / 29.5, 5120 + 16384 42.6 / 37.2; gated 3072 and 6144, K = 3072 20.9 / 25.0, 1 row
+    // 17.7 / 20.3, 4096 and 8192 32.2 / 36.6, 16 rows 44.1 / 49.0; fp32 2048 and 4096, 9 and 16 rows 23.6 / 27.5 and 26.5 / 29.1; plain, 2560 + 8192 columns, 9 and 16 rows
+    // 15.1 / 18.9 and 17.6 / 20.8.)
+    const int ga = pcb_ceil_div(a.N, 8), gb = pcb_ceil_div(b.N, 8);
+    const bool heavy = a.dtype == PCB_BF16 && b.epilogue == PCB_EPI_STORE && a.M > 4 && a.M <= 8 && ((int64_t)a.N * a.K + (int64_t)b.N * b.K) * 2 > 80000000 &&
+                       pcb_parts_blocks(ga, a.K).share + pcb_parts_blocks(gb, b.K).share <= pcb_ceil_div(ga + gb, 256);
     if (a.M <= 16) return heavy ? 0 : 1;
     const int shape = a.M > 64 ? pcb_linear_tiles_pair_shape(a, b) : -1;
     return shape < 0 ? 0 : 2 + shape;

@@ -125,6 +125,19 @@ __device__ __forceinline__ void parts_block(const pcb_linear_args& a, int block,
 // 32000 x 1024 12.0 / 13.2.
 inline bool pcb_weights_once(int64_t rows, int64_t K, int es) { return K * es >= 4096 && rows * K * es >= (es == 2 ? 8000000 : 4000000); }
 
+// How many of `groups` blocks of columns a workgroup has so that the busiest CU has the fewest, the more the better, up to four (deeper k three); how many it then has
+struct pcb_blocks {
+    int blocks;
+    int64_t share;
+};
+inline pcb_blocks pcb_parts_blocks(int64_t groups, int64_t K) {
+    pcb_blocks f{1, 0};
+    for (int n = 1; n <= (K <= 2048 ? 4 : 3); ++n) {
+        const int64_t share = ((groups + n - 1) / n + 255) / 256 * n;
+        if (n == 1 || share <= f.share) f = {n, share};
+    }
+    return f;
+}
 // PCB_OK when the arguments are valid (pb_linear.hip)
 int pcb_linear_check(const pcb_linear_args* a);
 // whether a launch's rows can be read in 16-byte pieces, whole k-steps

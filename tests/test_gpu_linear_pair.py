@@ -47,6 +47,15 @@ def test_pairs_beside_a_gated_unit_of_two_runs(M, N, N2, K, K2, dtype):
     test_pairs(N=N, N2=N2, K=K, K2=K2, M=M, dtype=dtype)
 
 
+# either side of the lines between one run and two: 1024 of k (results' places ahead), just more and just fewer, 7168 weight rows of a gated unit and 8192 plain ones, in fp32 16384 over 1024
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M", [4, 5, 8])
+@pytest.mark.parametrize("N,N2,K,K2", [(1024, 3072, 1024, 1024), (1024, 3073, 1024, 1088), (1040, 3064, 512, 512), (1040, 3065, 512, 960), (2048, 7168, 1024, 1024), (2048, 7170, 1024, 1024),
+                                       (1024, 3072, 1472, 1472), (1025, 7168, 1536, 1600)])
+def test_pairs_on_either_side_of_the_lines(M, N, N2, K, K2, dtype):
+    test_pairs(N=N, N2=N2, K=K, K2=K2, M=M, dtype=dtype)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("M", [1, 2, 3, 5, 8, 9])
 @pytest.mark.parametrize("N,K,ff", [(1024, 1024, 4096), (1001, 512, 1536), (70, 1152, 512), (36, 64, 96)])
