@@ -308,11 +308,15 @@ int launch(const pcb_row_norm_args& n, const pcb_linear_args& a, const pcb_linea
 // faster where there are few of them, and up to K = 512, where a run of weights is less than what finding it costs: bf16 gated, 1 row, K = 384, 72 and 2200 columns 4.2, here 5.8).
 // us, launches apart / here, medians of 900 random sizes: K = 576 .. 1024 and 1600 .. 2048 a table or behind a sublayer 0.62 .. 0.97 of it, one fp32 size in 60 1.04; between them
 // waves have a third k-step, or not, in registers for four: bf16, 5 rows, K = 1088, 4176 columns 8.5 / 9.8, fp32, 2 rows, 13000 columns 17.2 / 20.2.  The streams' sum is worked
-// out by every workgroup: up to 32768 elements of all streams of more than 256 runs of weights 0.75 .. 1.03, of fewer up to 12288 0.8 .. 0.97, beyond 1.05 .. 1.5.
+// out by every workgroup: up to 32768 elements of all streams of more than 256 runs of weights 0.75 .. 1.03 (of K = 576 .. 768 up to 20480: 8 rows, five streams, 5136 columns, bf16, K = 576 1.01,
+// 16000 1.16, fp32 1.03 and 1.09), of fewer up to 12288 0.8 .. 0.97, beyond 1.05 .. 1.5.  A vocabulary's runs of a short k go by faster in launches of their own, several blocks of columns a
+// workgroup: 32000 columns, bf16, 1 row, K = 576 12.1 / 14.6, 768 13.5 / 15.3, 960 1.00, 1024 0.97, 4 rows, K = 576 13.4 / 14.9, 704 1.01, 8 rows 1.05, 0.95, fp32, 1 row 1.01 .. 1.06 and 0.97; 16000 columns, the
+// sum of five streams, bf16, 1 row, K = 576 1.12, 704 1.04, 832 0.99.
 bool faster(const pcb_row_norm_args& n, const pcb_linear_args& a, const pcb_linear_args* b) {
     const int64_t elems = (int64_t)a.K << (a.M <= 1 ? 0 : a.M <= 2 ? 1 : a.M <= 4 ? 2 : 3);
     const int64_t runs = pcb_ceil_div(a.N, R) + (b ? (int64_t)pcb_ceil_div(b->N, R) * (b->epilogue == PCB_EPI_SILU_MUL ? 2 : 1) : 0);
-    return (a.K > 1536 || (a.K > 512 && a.K <= 1024)) && n.n_terms * elems <= (runs > CUS ? 32768 : 12288);
+    const int least = runs > 3000 ? (a.dtype == PCB_F32 ? 704 : a.M <= 2 ? 960 : a.M <= 4 ? 768 : 704) : runs > 1500 && n.n_terms > 0 && a.dtype == PCB_BF16 ? 768 : 0;
+    return (a.K > 1536 || (a.K > 512 && a.K <= 1024)) && a.K >= least && n.n_terms * elems <= (runs <= CUS ? 12288 : a.K <= 768 ? 20480 : 32768);
 }
 
 int route(const pcb_row_norm_args* n, const pcb_linear_args* a, const pcb_linear_args* b) {

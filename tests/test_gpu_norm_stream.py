@@ -81,6 +81,28 @@ def test_norm_stream(dtype, kind, M, K, N1, N2):
         close(y2[:M], torch.nn.functional.silu(want) * (n2 @ w3.to(d).T + b3.to(d)) if kind == "gated" else want)
 
 
+# a vocabulary's columns of a short k, and many streams of one: whether the launch is taken, by type, rows and k
+@pytest.mark.parametrize("dtype,kind,M,K,N,taken", [
+    (torch.bfloat16, "post", 1, 896, 24008, False), (torch.bfloat16, "post", 1, 960, 24008, True), (torch.bfloat16, "post", 4, 704, 24008, False), (torch.bfloat16, "post", 3, 768, 24008, True),
+    (torch.bfloat16, "post", 8, 640, 24008, False), (torch.bfloat16, "post", 5, 704, 24008, True), (torch.bfloat16, "post", 1, 576, 24000, True), (torch.float32, "post", 2, 640, 24008, False),
+    (torch.float32, "post", 2, 704, 24008, True), (torch.bfloat16, "mix2", 1, 704, 12008, False), (torch.bfloat16, "mix2", 1, 768, 12008, True), (torch.bfloat16, "mix2", 1, 704, 12000, True),
+    (torch.float32, "mix2", 1, 576, 12008, True), (torch.bfloat16, "mix5", 8, 576, 2064, False), (torch.bfloat16, "mix5", 4, 768, 2064, True)])
+def test_short_k_of_many_columns(dtype, kind, M, K, N, taken):
+    x, gain = torch.randn(5, M, K, device=DEV), torch.ones(K, device=DEV)
+    h, w, y = torch.empty(M, K, dtype=dtype, device=DEV), (torch.randn(N, K, device=DEV) * K ** -0.5).to(dtype), torch.full((M, N), 7.0, device=DEV)
+    t, gate, n = torch.randn(M, K, device=DEV), torch.rand(M, K, device=DEV).to(dtype), int(kind[3:]) if kind[:3] == "mix" else 0
+    src = dict(x=x, coef=gain[:5], n_terms=n) if n else dict(x=x[0], y=t, gate=gate, ldg=K, post_gain=gain)
+    assert B.norm_linear(B.linear_args(h, w, y, M=M), None, gain, None, torch.empty(M, K, device=DEV), eps=1e-5, many=True, **src) == taken
+    if not taken:
+        assert bool((y == 7).all())
+        return
+    d = torch.float64
+    row = x[:n].to(d).sum(0) if n else x[0].to(d) + rms(t.to(d) * gate.to(d), gain.to(d), 1e-5)
+    want = rms(row, gain.to(d), 1e-5) @ w.to(d).T
+    tol = 4e-6 * 5 * (1 + want.abs()) if dtype == torch.float32 else 6 * 2 ** -9 * 1.5 * (1 + want.abs())      # (as in test_norm_stream; sums are stored in fp32)
+    assert bool(((y.to(d) - want).abs() <= tol).all())
+
+
 def test_what_it_does_not_take():
     """Sizes beyond its own, and results over the rows that are read: refused or not taken, and nothing done."""
     def ask(M, K, N, y=None, xo=None, act=torch.bfloat16):
