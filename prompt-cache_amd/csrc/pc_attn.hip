@@ -1463,6 +1463,11 @@ bool choose_launch(AttnParams& p, int D, int B) {
         // 9.5, 700 12.5 / 10.1, 40 heads 12.2 / 11.4, 13.5 / 12.9; behind that (32 heads, 936 keys 13.8 / 13.7, 2500 20.7 / 21.7) the same
         // keys cross the chip twice.
         if (q_len > kSmallQ && 2 * B * H * p.nsplit <= 320) p.small_rt = 2;
+        // ALiBi, 17..32 rows: the 64-row kernel where a wave of few streams would walk more than one tile of 64 keys with the positions' loads in its
+        // chain.  us with the merge, 17 rows, this kernel / that one, 32 heads x 128 over 1725 keys 16.5 / 16.4, 2100 21.5 / 19.0, 4000 29.6 / 26.6, 40 heads, 1100
+        // 15.8 / 15.6, 1400 20.6 / 17.5, 28 heads, 2500 1.13 of the other's time (20 and 24 heads 0.71 and 0.88; head dims 32 and 64: mostly below 0.95).
+        const int streams = p.nsplit - p.tail;
+        if (D == 128 && p.key_pos && q_len > kSmallQ && streams <= 8 && past_len > 4 * kTK * streams) { small = false; p.small_rt = 1; }
     }
     p.small = small ? 1 : 0;
     // staging while reading lives in attn_small_kernel's two-launch form and in the tail-mode instantiation of the 64-row kernel

@@ -49,3 +49,14 @@ def test_every_launch_fits_its_workspace_and_modes_differ():
     assert n.attn_form(1, 32, 128, 12, 1700, -1) != n.attn_form(1, 32, 128, 12, 1700, 0)
     for bad in ((0, 32, 128, 1, 1), (1, 0, 128, 1, 1), (1, 32, 96, 1, 1), (1, 32, 128, 0, 1), (1, 32, 128, 1, -1)):
         assert n.attn_form(*bad, 0) == 0
+
+
+@pytest.mark.parametrize("H,past", [(28, 2048), (32, 1792), (40, 1280), (64, 768)])
+def test_positions_in_a_chain_of_tiles(H, past):
+    """17 to 32 rows with ALiBi leave the kernel of few rows where a wave has a second tile (head dim 128)."""
+    n = _n()
+    plain = n.attn_form(1, H, 128, 27, past, -1, 0), n.attn_form(1, H, 128, 27, past + 1, -1, 0)
+    alibi = n.attn_form(1, H, 128, 27, past, -1, 1), n.attn_form(1, H, 128, 27, past + 1, -1, 1)
+    assert alibi[0] == plain[0] and plain[1] == plain[0] and alibi[1] != alibi[0]
+    assert n.attn_form(1, H, 64, 27, past + 1, -1, 1) == n.attn_form(1, H, 64, 27, past, -1, 1)
+    assert n.attn_form(1, H, 128, 16, past + 1, -1, 1) == n.attn_form(1, H, 128, 16, past, -1, 1)

@@ -17,7 +17,8 @@ def _n():
     (4, 2, 128, 1, 1), (4, 4, 64, 5, 40), (8, 8, 32, 16, 100), (4, 2, 128, 17, 3), (2, 2, 64, 32, 238), (32, 32, 128, 31, 60),       # the 64-row kernel beside the tail
     (32, 32, 128, 2, 254), (32, 32, 128, 3, 253), (8, 2, 128, 15, 768), (8, 2, 128, 16, 769), (40, 40, 128, 16, 1024), (40, 40, 128, 16, 1025),
     (32, 32, 128, 17, 239), (32, 32, 128, 27, 308), (8, 2, 64, 31, 768), (16, 16, 32, 32, 769), (40, 40, 128, 29, 700), (40, 40, 128, 32, 769),
-    (54, 54, 128, 18, 300), (64, 64, 128, 20, 300), (32, 32, 128, 25, 1024), (32, 8, 128, 32, 1300)])
+    (54, 54, 128, 18, 300), (64, 64, 128, 20, 300), (32, 32, 128, 25, 1024), (32, 8, 128, 32, 1300),
+    (40, 40, 128, 17, 1280), (40, 40, 128, 32, 1281), (40, 40, 64, 30, 1281)])                                     # (ALiBi, a wave's second tile: the 64-row kernel)
 def test_a_few_rows_over_a_staged_cache(H, Hkv, D, q_len, past, alibi):
     n = _n()
     kv, g = past + q_len, torch.Generator().manual_seed(1000 * past + q_len)
