@@ -68,6 +68,10 @@ int launch_MT(int epi, const GemmParams& p, int T, int units, hipStream_t s) {
         if (five && !forced && T == 8 && pc_ceil_div(units * p.kslices, 5) <= 256) T = 5;
         if (five && !forced && T == 4 && mt <= 2 && p.kslices == 1 && units > 840 && (p.KS == 128 || (p.KS == 64 && mt == 1))) T = 5;
         if (five && T == 5 && mt <= 2) return launch_pipe(epi, p, T, units, s);
+        // (33 to 64 rows: no eight tiles (launch_T) of a slice of K below 1536, nor in slices that are more than a round of the chip: what a workgroup begins with is not
+        // earned back.  us, 48 rows, four / eight: 2000 tiles, K = 1024 21.0 / 22.7, K = 1536 27.0 / 25.0; four slices, K = 4096, 768 tiles 30.1 / 37.0, K = 3072, 576 tiles 20.3 / 26.3,
+        // two of them 23.2 / 17.3; three slices, K = 5120, 960 tiles 39.7 / 45.6, two 41.5 / 35.9, K = 4096, 1536 tiles 50.3 / 54.4)
+        if (mt > 2 && epi == EPI_STORE && !forced && T == 8 && (p.KS < 48 * p.kslices || (p.kslices > 1 && units * p.kslices > 8 * 256))) T = 4;
         // (33 to 64 rows take three pairs at most: two, where three are a second round of the chip that is emptier.  13b's gate|up, 40 rows 81.5 / 67.2)
         if (mt > 2 && epi == EPI_SILU && T > 3 && !forced) {
             auto busy = [&](int t) { const int wg = pc_ceil_div(units, t); return (float)wg / (float)(256 * pc_ceil_div(wg, 256)); };

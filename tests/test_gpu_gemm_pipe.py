@@ -78,7 +78,7 @@ def test_slices_added_in_the_launch(M, N, K, S, T):
         assert rel(y, 1 + k * want) < 2e-6 and not bool(counters.any())
 
 
-# 33 to 64 rows, more tiles than a round of six a workgroup holds: eight, the last workgroup with fewer; one plane too
+# 33 to 64 rows, a vocabulary of a short k (four tiles a workgroup), the last workgroup with fewer; one plane too
 @pytest.mark.parametrize("M", [33, 47, 64])
 @pytest.mark.parametrize("N,K", [(32000, 96), (32016, 288), (24592, 32)])
 def test_vocabularies(M, N, K):
@@ -102,3 +102,10 @@ def test_stores_on_either_side_of_the_lines(M, N, K, slices):
 @pytest.mark.parametrize("inter,K", [(11008, 1024), (11008, 1056), (11008, 4096), (13824, 4096), (13824, 4128)])
 def test_gated_on_either_side_of_the_lines(M, inter, K):
     test_gated(M, inter, K)
+
+
+# eight tiles a workgroup from K = 1536 on, in slices only while they are one round of the chip
+@pytest.mark.parametrize("M", [33, 47, 64])
+@pytest.mark.parametrize("N,K,slices", [(32016, 1504, 1), (32016, 1536, 1), (24592, 1568, 1), (9232, 3072, 2), (9232, 3008, 2), (15360, 4608, 3)])
+def test_vocabularies_on_either_side_of_the_lines(M, N, K, slices):
+    test_stores_and_sums(M, N, K, slices)
