@@ -605,8 +605,9 @@ FewRows few_rows(const pcb_linear_args& a) {
     if (bf && a.epilogue == PCB_EPI_STORE && a.n_batch == 0 && a.K % 64 == 0 && a.K >= 1024 && g2 > 256 && (a.M > 2 || a.K <= 1024))
         return {2, true, pcb_parts_blocks(g2, a.K).blocks};
     if (a.M <= 4 && a.K % 128 == 0 && a.K >= (gated && bf ? 2048 : 1024) && g4 <= (a.M <= 2 || gated || a.K >= 2048 ? 768 : 512)) return {4, late};
-    // two runs, of more than four rows not where 16 columns each are one round of the chip and eight are two (there the kernel above over a deep k: 8 rows,
-    // K = 4096, 2048 columns 9.6 / 10.3 / 7.1, 2560 9.8 / 10.6 / 10.6, 4096 13.6 / 11.6 / 11.3, 8192 18.3 / 20.1 / 20.4, 16384 35.8 / 36.0 / 36.4)
+    // (From here on, in bf16: sums into rows, the gated unit, batches, and plain stores of one and two rows over K > 1024 or of no more than a round.)
+    // Two runs, of more than four rows not where 16 columns each are one round of the chip and eight are two (there the kernel above over a deep k; stores of 8 rows
+    // over K = 4096, which a batch has as well: 2048 columns 9.6 / 10.3 / 7.1, 2560 9.8 / 10.6 / 10.6, 4096 13.6 / 11.6 / 11.3, 8192 18.3 / 20.1 / 20.4, 16384 35.8 / 36.0 / 36.4)
     if (a.K % 64 != 0 || a.K < (bf ? 1024 : 512)) return one;
     if (a.M > 4 && !gated) {
         const bool hole = g2 > 256 && g2 <= 400;
@@ -614,8 +615,8 @@ FewRows few_rows(const pcb_linear_args& a) {
         if (hole) return one;
     }
     // ... and while the chip has places for them: accumulations in bf16 8 rows, 4096 x 1024 5.6 / 4.9 / 5.1, 8192 x 1024 6.7 / 7.0 / 7.5, 8192 x 2048 10.8 / 11.7 /
-    // 11.5; stores in bf16 up to six rows at any size (32000 x 2048, 1 row 30.0 / 27.8 / 23.6, 5 rows 32.1 / 31.1 / 29.8, 8 rows 34.3 / 34.6 / 35.1), in fp32 two (2 rows
-    // 33.7 / 27.0 / 26.4); fp32, K = 2048, 4 rows, 8192 columns 20.1 / 17.3 / 17.5, 8 rows, 6144 20.4 / 16.9 / 15.8, 8192 21.8 / 18.1 / 19.9; 4 rows added, K = 512, 4096
+    // 11.5; stores in bf16 at any size (32000 x 2048, 1 row 30.0 / 27.8 / 23.6), batches of them up to six rows (the same columns, 5 rows 32.1 / 31.1 / 29.8, 8 rows 34.3 / 34.6 /
+    // 35.1), in fp32 two (2 rows 33.7 / 27.0 / 26.4); fp32, K = 2048, 4 rows, 8192 columns 20.1 / 17.3 / 17.5, 8 rows, 6144 20.4 / 16.9 / 15.8, 8192 21.8 / 18.1 / 19.9; 4 rows added, K = 512, 4096
     // columns 5.7 / 5.0 / 5.2, 8192 7.3 / 6.4 / 6.9
     const bool any = bf ? (add ? a.K >= 2048 && a.M <= 4 : gated || a.M <= 6) : a.epilogue == PCB_EPI_STORE && a.M <= 2;
     const int64_t most = any ? INT64_MAX : add ? (a.K < (bf ? 2048 : 1024) ? 640 : bf || a.M > 4 ? 768 : 1024) : bf || a.M <= 4 ? 1024 : 768;

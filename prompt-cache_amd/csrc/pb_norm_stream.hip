@@ -82,6 +82,8 @@ __device__ __forceinline__ void store_result(const Product& p, int m, int col, i
 template <typename E, int EPI, int U, int NC, int KIND>
 __global__ __launch_bounds__(512) void norm_stream_kernel(Launch n) {
     constexpr int TB = EPI == PCB_EPI_SILU_MUL ? 2 : 1;
+    // (weights past the caches, fp32 and the deepest k.  us, past / through them: fp32, 1 row, K = 768, 5136 columns from memory 8.2 / 9.1, from the Infinity Cache 8.2 / 8.5, 32000
+    // from memory 21.7 / 22.8, K = 576 19.7 / 21.0; where 32000 columns stay there, 98 and 74 MB that nothing else displaces, 21.1 / 20.2, 19.6 / 18.7)
     constexpr bool ONCE = U == 4 || sizeof(E) == 4;
     __shared__ f4 red[2][D][SKW][64];
     __shared__ __attribute__((aligned(16))) E rows[NC * CHUNK + MAX_ROWS * PAD];

@@ -1196,8 +1196,9 @@ __global__ __launch_bounds__(kThreads, (GATHER || RT > 1) ? 1 : 2) void attn_sma
 // waits for those: 7 + 1 (exactly 256) runs the persona step 1.7 % faster end to end (3.908 -> 3.844 ms, profiles/r03_*).
 // Fewer over a short cache: a wave of three streams has one tile up to 768 keys, as one of seven has, and every stream more is a
 // partial of all rows that is written and merged.  us with the merge, 32 heads, all / fewer: 308 keys, 3 rows 8.7 / 8.3, 12 rows
-// 9.7 / 8.8, 27 rows 13.2 / 11.9, 700 keys 9.2 / 9.0, 10.2 / 9.5, 13.6 / 12.5, 936 keys, 16 rows 11.3 / 10.8; one row 308 keys 8.0 / 8.3,
-// two rows 700 keys 9.0 / 9.2, 1200 keys, 4 rows 11.2 / 11.5 (five streams; 8 heads, 936 keys 9.1 / 9.4).
+// 9.7 / 8.8, 27 rows 13.2 / 11.9, 700 keys 9.2 / 9.0, 10.2 / 9.5, 13.6 / 12.5, 936 keys, 16 rows 11.3 / 10.8 (8 heads,
+// the most streams there are: 10.05 / 9.89).  All of them where fewer were slower: one row 308 keys 8.0 / 8.3, two rows 700 keys 9.0 / 9.2, five streams of 4 rows over
+// 1200 keys 11.2 / 11.5 and, of 8 heads, 936 keys 9.1 / 9.4.
 int small_nstream(int B, int H, int tail = 0, int q_len = 1, int keys = 1 << 20) {
     static const int forced = [] { const char* e = getenv("PC_ATTN_SMALL_WG"); return e ? atoi(e) : 0; }();
     if (forced > 0) return forced < 15 ? forced : 15;

@@ -365,7 +365,6 @@ int launch_rows(const GemmParams& p_in, int units, hipStream_t s) {
         // then read twice (once from L2), the activations of a row block by half as many workgroups
         const int nz = mt <= 18 ? 1 : 2;
         if (two && !no_wide && !forced && mt <= 36 && (EPI != EPI_ROPE || wide_rope || nz == 2)) {
-            [[maybe_unused]] constexpr int TV = (EPI == EPI_SILU) ? 4 : 8;
             GemmParams pz = p;
             pz.zrows = nz == 1 ? 0 : 16 * pc_ceil_div(mt, 2);
             const int rw = pc_ceil_div(pc_ceil_div(mt, nz), 2);
@@ -373,13 +372,11 @@ int launch_rows(const GemmParams& p_in, int units, hipStream_t s) {
             // (LDS-DMA ring staging, round 6: the same time as register staging in the step -- config 4 21.96 / 21.93 ms against
             // 21.93 / 21.83 -- because a CU's weight stream is capped near 13.5 GB/s whatever is in flight; profiles/r06_variants.txt r6s)
             static const int ring = [] { const char* e = getenv("PC_ROWS_RING"); return e ? atoi(e) : 0; }();
-            if (ring == 6)
-                hipLaunchKernelGGL((gemm_rows_kernel<8, EPI, 2, true, 3, 3, 2, 768, 6>), dim3(pc_ceil_div(units, TV), p.kslices, nz),
-                                   dim3((rw + 3) * 64), 0, s, pz);
-            else if (ring == 3)
-                hipLaunchKernelGGL((gemm_rows_kernel<8, EPI, 2, true, 3, 6, 2, 768, 3>), dim3(pc_ceil_div(units, TV), p.kslices, nz),
-                                   dim3((rw + 3) * 64), 0, s, pz);
-            else
+            constexpr int TV = (EPI == EPI_SILU) ? 4 : 8;
+            const dim3 rgrid(pc_ceil_div(units, TV), p.kslices, nz), rblock((rw + 3) * 64);
+            if (ring == 6) hipLaunchKernelGGL((gemm_rows_kernel<8, EPI, 2, true, 3, 3, 2, 768, 6>), rgrid, rblock, 0, s, pz);
+            if (ring == 3) hipLaunchKernelGGL((gemm_rows_kernel<8, EPI, 2, true, 3, 6, 2, 768, 3>), rgrid, rblock, 0, s, pz);
+            if (ring == 6 || ring == 3) return pc_check_launch("gemm_rows_kernel");
 #endif
             // an odd number of row tiles in one block (259 rows = 17 tiles): the odd tile goes to the three staging waves (XT: LDS-DMA
             // ring of five 30-KiB stages) instead of a ninth compute wave on the SIMD that already runs two.  PC_ROWS_XT=0: off

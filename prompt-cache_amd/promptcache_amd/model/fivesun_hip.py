@@ -397,7 +397,7 @@ class FivesunHIP(SlotModel):
             rows, pending = {}, {}
 
         def project(gain, a, b=None):
-            """The products ``a`` and, where given, ``b`` of the normed rows: at few rows (up to eight of 512 columns, two of 2048) the norm goes into their launch."""
+            """The products ``a`` and, where given, ``b`` of the normed rows: at few rows (up to eight of 2048 columns) the norm goes into their launch."""
             nonlocal x, spare, rows, pending
             if few and (rows or pending):
                 to = x if rows else spare

@@ -210,7 +210,7 @@ class KazolornHIP(SlotModel):
                 z, act = self._mat("z", T, l.ff, f32), self._mat("act", T, l.ff, E)
                 up = B.linear_args(h2, lw["up"], z, M=T)
             rows = dict(x=hist, n_terms=i + 1, coef=layers[i - 1]["dwa"]) if i else dict(table=self.embed, ids=ids_d)
-            # (few rows, up to eight of 512 columns, two of 2048: the embedding or the streams' sum and the norms in the launch of the layer's first products)
+            # (few rows, up to eight of 2048 columns: the embedding or the streams' sum and the norms in the launch of the layer's first products)
             if not (up and T * W <= B.NORM_LINEAR_MAX and B.norm_linear(qk, up, lw["g1"], lw["g2"], base, eps=eps, **rows)):
                 norms = (lw["g1"], h1, lw.get("g2"), h2 if has_ff else None)
                 if i:
