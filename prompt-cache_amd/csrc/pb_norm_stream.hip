@@ -228,13 +228,13 @@ __global__ __launch_bounds__(512) void norm_stream_kernel(Launch n) {
         const int k = wave + s * SKW;
         fa[s] = load_piece<2>(xrow + 64 * (k < steps ? k : steps - 1));
     }
-    auto total_of = [&](const f4 (*w)[64]) {
-        float s = 0.0f;
+    auto total_of = [&](const f4 (*w)[64]) {                         // (the waves' sums of each run of k, then the runs': as parts_total() has them, to the bit)
+        float s[2] = {0.0f, 0.0f};
 #pragma unroll
-        for (int p = 0; p < 2; ++p)
+        for (int v = 0; v < SKW; ++v)
 #pragma unroll
-            for (int v = 0; v < SKW; ++v) s += ((const float*)&w[v][(m + 8 * p) / 4 * 16 + cl + 8 * p])[m & 3];
-        return s;
+            for (int p = 0; p < 2; ++p) s[p] += ((const float*)&w[v][(m + 8 * p) / 4 * 16 + cl + 8 * p])[m & 3];
+        return s[0] + s[1];
     };
     for (int u0 = 0, par = 0; u0 < total; u0 += D, par ^= 1) {
         const int slot = (wave - u0) & (SKW - 1), u = u0 + (slot & (D - 1));       // (the waves take turns at the results)

@@ -103,6 +103,22 @@ def test_short_k_of_many_columns(dtype, kind, M, K, N, taken):
     assert bool(((y.to(d) - want).abs() <= tol).all())
 
 
+@pytest.mark.parametrize("dtype,M,K,N", [(torch.bfloat16, 8, 2048, 5136), (torch.bfloat16, 3, 1024, 5136), (torch.float32, 8, 1024, 2048)])
+def test_sums_are_those_of_the_products_launch(dtype, M, K, N):
+    """Two runs of k, each summed over the waves, then one and the other: the bits of the products' own launch over the same normed rows (read out by weights of one)."""
+    x, t = torch.randn(M, K, device=DEV), torch.randn(M, K, device=DEV)
+    gate, gain = torch.rand(M, K, device=DEV).to(dtype), torch.randn(K, device=DEV)
+    got = []
+    for w in (torch.eye(K, device=DEV, dtype=dtype), (torch.randn(N, K, device=DEV) * K ** -0.5).to(dtype)):
+        y = torch.full((M, w.shape[0]), float("nan"), device=DEV)
+        assert B.norm_linear(B.linear_args(torch.empty(M, K, dtype=dtype, device=DEV), w, y, M=M), None, gain, None, torch.empty(M, K, device=DEV), eps=1e-5, x=x, y=t, gate=gate, ldg=K,
+                             post_gain=gain, many=True)
+        got.append(y)
+    want = torch.empty(M, N, device=DEV)
+    B.linear(got[0].to(dtype), w, want, M=M)
+    assert torch.equal(got[1], want)
+
+
 def test_what_it_does_not_take():
     """Sizes beyond its own, and results over the rows that are read: refused or not taken, and nothing done."""
     def ask(M, K, N, y=None, xo=None, act=torch.bfloat16):
