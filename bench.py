@@ -190,7 +190,7 @@ def gemm_rooflines(lm, T: int):
     the captured graph cannot be bracketed by events; the in-graph durations are in profiles/ (rocprofv3).  32 distinct weight
     sets (13 GB) are cycled, so nothing is served from the 256 MB Infinity Cache.
     -> (dominant, extra): `dominant` = the gate|up projection (RMSNorm + SiLU*up fused), the largest single kernel of the timed
-    step by time (profiles/r03_bench_kernel_stats.txt); `extra` = {"roofline_nhidden": o_proj + down_proj with the residual add
+    step by time (profiles/bench_kernel_stats.txt); `extra` = {"roofline_nhidden": o_proj + down_proj with the residual add
     as the step dispatches them, "roofline_qkv": q|k|v + RMSNorm + RoPE + append}."""
     import torch
     from promptcache_amd import _native as n
@@ -244,7 +244,7 @@ def gemm_rooflines(lm, T: int):
 
     how = ("HIP events on the launch stream around eager launches on each layer's weights right after the timed region (kernels "
            "inside the captured hipGraph of the timed step cannot be bracketed; event pairs include ~2 us of launch gap); the "
-           "in-graph average of the same kernel is in profiles/r03_bench_kernel_stats.txt")
+           "in-graph average of the same kernel is in profiles/bench_kernel_stats.txt")
     sig = f"T={T},hid={hid},inter={inter}"
     gu_avg, gu_min, gu_n = us("gu")
     nb_gu = 2 * inter * hid * 2
@@ -396,7 +396,7 @@ def attn_many_roofline(lm, q_len: int, S: int):
     wide = S >= int(os.environ.get("PC_ATTN_WIDE_MIN", "6144")) and q_len >= int(os.environ.get("PC_ATTN_WIDE_MIN_ROWS", "128")) \
         and os.environ.get("PC_ATTN_NO_WIDE") != "1"
     res = {"kernel": (("attn_wide_kernel<GATHER, R> over the staged keys (all query rows of a head per workgroup, key slices; "
-                       "pc_attn_wide.hip) + attn_ring_kernel<KVLO> over the pass's own rows" if wide else "attn_ring_kernel<KVLO, GATHER>") +
+                       "pc_attn_wide.hip), the pass's own rows in workgroups of the same launch" if wide else "attn_ring_kernel<KVLO, GATHER>") +
                       (" (stages while it reads: pc_attn gather_rows)" if staging else "")) +
                      " + attn_combine_kernel (pc_attn, > 64 split-precision rows): ALL launches of one pc_attn call inside the events",
            "staging": staging, "bound": "mfma", "achieved": flops / (avg * 1e-6) / 1e12, "peak": MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
@@ -1337,7 +1337,7 @@ def main():
                          "fused_gather_forwards": int(lm.hf_model.stats.get("fused_gather", 0)),
                          "host_glue_ms": ttft_ms - (process_ms[len(process_ms) // 2] + prefill_ms[len(prefill_ms) // 2]),
                          "what": "host_glue_ms = ms_per_step - (median process interval + median first-lm() interval)"}
-    # `roofline` = the time-dominant hand-written kernel of the timed step (largest share in profiles/r03_bench_kernel_stats.txt)
+    # `roofline` = the time-dominant hand-written kernel of the timed step (largest share in profiles/bench_kernel_stats.txt)
     if rank == 0 and not args.no_context:
         result["roofline"], extra_rf = gemm_rooflines(lm, q)
         result.update(extra_rf)
