@@ -47,7 +47,7 @@ __device__ __forceinline__ void reduce_normed(const GemmParams& p, const f4 (&ac
     const float rs = rsqrtf(tot / (float)(p.KS * 32) + p.eps);
     v *= rs;
     u *= rs;
-    tile_epilogue<EPI>(p, v, u, m, (int)blockIdx.x * T + wave, g, 0);
+    tile_epilogue_of<EPI, TRACE>(p, v, u, m, (int)blockIdx.x * T + wave, g, 0);
     if (TRACE) { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); trace_stamp(p, blockIdx.x, 0, wave, 3); }
 }
 
@@ -243,7 +243,7 @@ int go_few(const GemmParams& p, int units, size_t lds, hipStream_t s) {
 template <int T, int EPI>
 int go(const GemmParams& p, int units, hipStream_t s) {
     if (p.trace)
-        hipLaunchKernelGGL((normed_kernel<T, EPI, true>), dim3(pc_ceil_div(units, T)), dim3(kThreads), 0, s, p);
+        hipLaunchKernelGGL((normed_kernel<T, traced_epi(EPI), true>), dim3(pc_ceil_div(units, T)), dim3(kThreads), 0, s, traced(p, EPI));
     else
         hipLaunchKernelGGL((normed_kernel<T, EPI, false>), dim3(pc_ceil_div(units, T)), dim3(kThreads), 0, s, p);
     return pc_check_launch("normed_kernel");
@@ -280,7 +280,7 @@ int launch_normed_few(int epi, const GemmParams& p, int units, hipStream_t s) {
         constexpr int TV = decltype(t)::value;
         auto go = [&](auto e) {
             constexpr int EPI = decltype(e)::value;
-            return p.trace ? go_few<TV, EPI, true>(p, units, lds, s) : go_few<TV, EPI, false>(p, units, lds, s);
+            return p.trace ? go_few<TV, traced_epi(EPI), true>(traced(p, EPI), units, lds, s) : go_few<TV, EPI, false>(p, units, lds, s);
         };
         return epi == EPI_STORE  ? go(std::integral_constant<int, EPI_STORE>{})
                : epi == EPI_ROPE ? go(std::integral_constant<int, EPI_ROPE>{})

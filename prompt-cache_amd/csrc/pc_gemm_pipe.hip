@@ -111,7 +111,7 @@ __global__ __launch_bounds__(kThreads) void gemm_pipe_kernel(const GemmParams p)
                 v += red[w][wave * TPI][lane];
                 if (EPI == EPI_SILU) u += red[w][wave * TPI + TPI - 1][lane];
             }
-            tile_epilogue<EPI>(p, v, u, a * 16 + m, bx * T + t, g, by);
+            tile_epilogue_of<EPI, TRACE>(p, v, u, a * 16 + m, bx * T + t, g, by);
         }
     }
     if (TRACE) { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); trace_stamp(p, bx, by, wave, 3); }
@@ -123,7 +123,7 @@ int go(const GemmParams& p, int units, hipStream_t s) {
     const dim3 grid(pc_ceil_div(units, T), p.kslices);
     const bool odd = pc_ceil_div(pc_ceil_div(pc_ceil_div(p.KS, p.kslices), kWaves), U) & 1;
     if (p.trace)
-        hipLaunchKernelGGL((gemm_pipe_kernel<MT, T, EPI, U, true, true>), grid, dim3(kThreads), 0, s, p);
+        hipLaunchKernelGGL((gemm_pipe_kernel<MT, T, traced_epi(EPI), U, true, true>), grid, dim3(kThreads), 0, s, traced(p, EPI));
     else if (odd)
         hipLaunchKernelGGL((gemm_pipe_kernel<MT, T, EPI, U, true, false>), grid, dim3(kThreads), 0, s, p);
     else

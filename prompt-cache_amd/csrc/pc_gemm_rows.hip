@@ -342,10 +342,7 @@ int launch_rows(const GemmParams& p_in, int units, hipStream_t s) {
         constexpr int TV = (EPI == EPI_SILU) ? (TTV) / 2 : (TTV);                                          \
         const dim3 grid(pc_ceil_div(units, TV), p.kslices);                                                \
         if (two) {                                                                                         \
-            if constexpr ((TTV) <= 4) {                                                                    \
-                if (narrow) hipLaunchKernelGGL((gemm_rows_kernel<TTV, EPI, 2, true>), grid, block, 0, s, p); \
-                else hipLaunchKernelGGL((gemm_rows_kernel<TTV, EPI, 4, true>), grid, block, 0, s, p);      \
-            }                                                                                              \
+            if constexpr ((TTV) <= 4) hipLaunchKernelGGL((gemm_rows_kernel<TTV, EPI, 2, true>), grid, block, 0, s, p); \
         } else if (narrow) hipLaunchKernelGGL((gemm_rows_kernel<TTV, EPI, 2, false>), grid, block, 0, s, p); \
         else if constexpr ((TTV) <= 6) hipLaunchKernelGGL((gemm_rows_kernel<TTV, EPI, 4, false>), grid, block, 0, s, p); \
         return pc_check_launch("gemm_rows_kernel");                                                        \
@@ -364,7 +361,8 @@ int launch_rows(const GemmParams& p_in, int units, hipStream_t s) {
         // 289..512 rows: two row blocks per column panel (grid.z), each within the 9 compute waves -- the weights of a panel are
         // then read twice (once from L2), the activations of a row block by half as many workgroups
         const int nz = mt <= 18 ? 1 : 2;
-        if (two && !no_wide && !forced && mt <= 36 && (EPI != EPI_ROPE || wide_rope || nz == 2)) {
+        // (more than 384 rows in two planes have no other kernel, whatever the switches say)
+        if (two && (!narrow || (!no_wide && !forced && (EPI != EPI_ROPE || wide_rope || nz == 2)))) {
             GemmParams pz = p;
             pz.zrows = nz == 1 ? 0 : 16 * pc_ceil_div(mt, 2);
             const int rw = pc_ceil_div(pc_ceil_div(mt, nz), 2);

@@ -107,6 +107,7 @@ struct GemmParams {
     int32_t kskew, prio_alt;
     // dev: per-wave wall-clock stamps [grid.x * grid.y][kWaves][4] (entry, K loop done, reduced, done); pc_dev_gemm_trace
     unsigned long long* trace;
+    int32_t trace_epi;   // (the epilogue of a traced launch whose kernel is built for plain results only: tile_epilogue_of)
 };
 
 __device__ __forceinline__ void trace_stamp(const GemmParams& p, int bx, int by, int wave, int slot) {
@@ -596,6 +597,28 @@ __device__ __forceinline__ void alt_prio(const GemmParams& p, int wave, int& blk
     }
 }
 
+// tile_epilogue of a kernel that is built once more for pc_dev_gemm_trace: with stamps it stands for all epilogues of one result a row and column (22 kernels
+// instead of 46: the library's kernels are counted), and each launch says which
+template <int EPI, bool TRACE>
+__device__ __forceinline__ void tile_epilogue_of(const GemmParams& p, f4 v, f4 u, int row, int unit, int g, int slice) {
+    if constexpr (TRACE && EPI != EPI_SILU) {
+        switch (p.trace_epi) {
+            case EPI_ADD: return tile_epilogue<EPI_ADD>(p, v, u, row, unit, g, slice);
+            case EPI_ROPE: return tile_epilogue<EPI_ROPE>(p, v, u, row, unit, g, slice);
+            case EPI_GELU: return tile_epilogue<EPI_GELU>(p, v, u, row, unit, g, slice);
+            default: return tile_epilogue<EPI_STORE>(p, v, u, row, unit, g, slice);
+        }
+    } else {
+        tile_epilogue<EPI>(p, v, u, row, unit, g, slice);
+    }
+}
+inline GemmParams traced(const GemmParams& p, int epi) {
+    GemmParams q = p;
+    q.trace_epi = epi;
+    return q;
+}
+constexpr int traced_epi(int epi) { return epi == EPI_SILU ? EPI_SILU : EPI_STORE; }
+
 // weight tile ids of workgroup bx (clamped: a clamped duplicate tile recomputes a valid tile and is not stored)
 template <int T, int EPI>
 __device__ __forceinline__ void wg_tiles(const GemmParams& p, int bx, int (&tile)[(EPI == EPI_SILU) ? 2 * T : T]) {
@@ -974,8 +997,7 @@ int launch_pipe(int epi, const GemmParams& p, int T, int units, hipStream_t s);
 template <int MT, int T, int EPI>
 int launch_one(const GemmParams& p, int units, hipStream_t s) {
     constexpr int TT = (EPI == EPI_SILU) ? 2 * T : T;
-    constexpr int UD = (MT * TT >= 16) ? 1 : (MT * TT >= 8) ? 2 : (MT * TT >= 3 ? 4 : 8);     // default depth
-    static const int forced = [] { const char* e = getenv("PC_GEMM_U"); return e ? atoi(e) : 0; }();
+    constexpr int UD = (MT * TT >= 16) ? 1 : (MT * TT >= 8) ? 2 : 4;     // default depth
     const dim3 grid(pc_ceil_div(units, T), p.kslices), block(kThreads);
     const bool two = p.xf_lo != nullptr;
     // (two planes without the norm, three and four tiles of up to two row tiles: pc_gemm_pipe.hip)
@@ -1007,7 +1029,8 @@ int launch_one(const GemmParams& p, int units, hipStream_t s) {
         }                                                                                             \
         hipLaunchKernelGGL((gemm_skinny_kernel<MT, T, EPI, false, UV>), grid, block, 0, s, p);         \
     } while (0)
-#ifdef PC_DEV_SWEEPS   // block-depth sweeps (tools/gemm_n4096_sweep.py): ~500 extra kernel instantiations, not in the product build
+#ifdef PC_DEV_SWEEPS   // PC_GEMM_U, block-depth sweeps (tools/gemm_n4096_sweep.py): ~500 extra kernel instantiations, not in the product build
+    static const int forced = [] { const char* e = getenv("PC_GEMM_U"); return e ? atoi(e) : 0; }();
     if constexpr (MT * TT <= 2) {
         if (forced == 16) { PC_GO(16); return pc_check_launch("gemm_skinny_kernel"); }
     }
@@ -1017,20 +1040,14 @@ int launch_one(const GemmParams& p, int units, hipStream_t s) {
     }
     if (forced == 2) { PC_GO(2); return pc_check_launch("gemm_skinny_kernel"); }
 #endif
-    if constexpr (MT * TT <= 2) {
-        // one or two tiles per workgroup (the N = hidden projections): measured in-graph on the 7b shapes
-        // (tools/gemm_n4096_sweep.py), k-steps per block 4 / 8 / 16: o_proj 9.3 / 9.8 / 9.5 us at 12 rows, 8.0 / 8.9 / 8.9 at
-        // one row; down_proj 24.3 / 24.7 / 23.2 at 12 rows, 19.1 / 20.9 / 21.8 at one row -- shallow blocks win except for
-        // the long-K launch with its activation loads (more than 4 rows), which wants the deep one
-        if (!forced) {
-            // (the deep block only where it was measured: one tile, one row tile, residual add = down_proj; every other
-            // shape with U = 16 spills 100 .. 480 B per lane)
-            if constexpr (MT == 1 && TT == 1 && EPI == EPI_ADD) {
-                if (p.M > 4 && p.KS >= 256) { PC_GO(16); return pc_check_launch("gemm_skinny_kernel"); }
-            }
-            PC_GO(4);
-            return pc_check_launch("gemm_skinny_kernel");
-        }
+    // one or two tiles per workgroup (the N = hidden projections): measured in-graph on the 7b shapes
+    // (tools/gemm_n4096_sweep.py), k-steps per block 4 / 8 / 16: o_proj 9.3 / 9.8 / 9.5 us at 12 rows, 8.0 / 8.9 / 8.9 at
+    // one row; down_proj 24.3 / 24.7 / 23.2 at 12 rows, 19.1 / 20.9 / 21.8 at one row -- shallow blocks win except for
+    // the long-K launch with its activation loads (more than 4 rows), which wants the deep one
+    // (the deep block only where it was measured: one tile, one row tile, residual add = down_proj; every other
+    // shape with U = 16 spills 100 .. 480 B per lane)
+    if constexpr (MT == 1 && TT == 1 && EPI == EPI_ADD) {
+        if (p.M > 4 && p.KS >= 256) { PC_GO(16); return pc_check_launch("gemm_skinny_kernel"); }
     }
     PC_GO(UD);
 #undef PC_GO

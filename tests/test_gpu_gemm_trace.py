@@ -50,6 +50,22 @@ def test_two_planes(M, N, K, slices, workgroups):
     assert torch.equal(y, z)
 
 
+@pytest.mark.parametrize("M", [5, 20])
+@pytest.mark.parametrize("N,K", [(12288, 1120), (13824, 4096)])           # three and five tiles a workgroup
+def test_epilogues(M, N, K):
+    """A traced kernel stands for several epilogues: the sum into rows and the activation leave what their own kernels leave."""
+    n = _n()
+    wf, hi, lo, _ = operands(M, N, K)
+    y, z = torch.ones((M, N), device=DEV), torch.ones((M, N), device=DEV)
+    n.gemm_skinny(wf, hi, lo, M, N, K, n.EPI_ADD, y=z, ldy=N)
+    assert stamped(lambda: n.gemm_skinny(wf, hi, lo, M, N, K, n.EPI_ADD, y=y, ldy=N)).shape[0] >= 173
+    assert torch.equal(y, z)
+    frags = [torch.zeros(((M + 15) // 16, N // 32, 64, 8), dtype=torch.float16, device=DEV) for _ in range(4)]
+    n.gemm_skinny(wf, hi, lo, M, N, K, n.EPI_GELU, of_hi=frags[0], of_lo=frags[1])
+    stamped(lambda: n.gemm_skinny(wf, hi, lo, M, N, K, n.EPI_GELU, of_hi=frags[2], of_lo=frags[3]))
+    assert torch.equal(frags[0], frags[2]) and torch.equal(frags[1], frags[3]) and bool(frags[0].any())
+
+
 # five tiles a workgroup only where they are the faster: images of 64 KB (up to 16 rows) and 128 KB, more than 840 tiles
 @pytest.mark.parametrize("M,K,tiles,each", [(5, 4096, 1024, 5), (20, 4096, 841, 5), (32, 4096, 864, 5), (20, 4096, 832, 4), (12, 4096, 800, 4), (12, 2048, 1024, 5), (20, 2048, 1024, 4),
                                             (12, 6144, 1000, 4), (20, 8192, 1000, 4), (12, 4128, 1000, 4)])
