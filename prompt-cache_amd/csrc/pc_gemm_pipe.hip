@@ -159,8 +159,11 @@ namespace pcg {
 // 32 rows, K = 2048 11.5 / 11.6 and 14.8 / 14.3, 4096 19.0 / 19.7 and 26.1 / 26.8, 5120 23.5 / 25.3 and 30.4 / 31.2, 7168 31.6 / 34.1 and 40.9 / 42.5; 20 rows, K = 6656, 640 and 900
 // tiles 28.9 / 28.0 and 35.2 / 34.7, 11008 46.8 / 48.8 and 61.2 / 62.8; gated, 688 pairs, 12 rows, K = 1024 11.4 / 12.0, 2048 17.3 / 16.3, 4096 29.7 / 30.8, 5120 40.0 / 38.8, 32
 // rows, 640 pairs, K = 5120 43.2 / 42.0.  (Where a launch's weights lie moves such times by up to 3 %.)
-bool pipe_takes(int epi, const GemmParams& p) {
+// Three tiles over an odd multiple of 1024 (3072; of 1024 it makes no difference) not with more than 24 rows, whose operands have a second line in every group of lanes.  us, one block after
+// the other / so, K = 3072, 520, 640 and 768 tiles: 32 rows 15.5 / 16.6, 16.5 / 17.4, 17.9 / 18.4, 24 rows 14.8 / 15.2, 15.9 / 16.0, 17.4 / 17.2; K = 2560 and 3584, 32 rows 0.95 to 1.01 of it.
+bool pipe_takes(int epi, const GemmParams& p, int T) {
     if (epi == EPI_SILU) return p.M > 16 || (pc_ceil_div(p.KS, kWaves) != 4 && p.KS % 128 != 0);
+    if (T == 3 && p.M > 24 && p.kslices == 1 && p.KS > 32 && p.KS % 64 == 32) return false;
     return p.KS <= 128 * p.kslices || p.KS % 32 == 16;
 }
 

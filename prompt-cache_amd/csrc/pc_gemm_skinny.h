@@ -991,7 +991,7 @@ int launch_normed_few(int epi, const GemmParams& p, int units, hipStream_t s);
 bool normed_takes(int epi, const GemmParams& p, int T);
 int launch_normed(int epi, const GemmParams& p, int T, int units, hipStream_t s);
 // two planes, up to 32 rows, three to five tiles a workgroup (pc_gemm_pipe.hip)
-bool pipe_takes(int epi, const GemmParams& p);
+bool pipe_takes(int epi, const GemmParams& p, int T);
 int launch_pipe(int epi, const GemmParams& p, int T, int units, hipStream_t s);
 
 template <int MT, int T, int EPI>
@@ -1002,7 +1002,7 @@ int launch_one(const GemmParams& p, int units, hipStream_t s) {
     const bool two = p.xf_lo != nullptr;
     // (two planes without the norm, three and four tiles of up to two row tiles: pc_gemm_pipe.hip)
     if constexpr (MT <= 2 && (T == 3 || T == 4))
-        if (two && !p.xn && !p.w8 && pipe_takes(EPI, p)) return launch_pipe(EPI, p, T, units, s);
+        if (two && !p.xn && !p.w8 && pipe_takes(EPI, p, T)) return launch_pipe(EPI, p, T, units, s);
     // (the norm inside the launch, fp16 weights, one row tile: pc_gemm_norm.hip)
     if constexpr (MT == 1 && T >= 2 && T <= 4 && (EPI == EPI_STORE || EPI == EPI_ROPE || EPI == EPI_SILU))
         if (p.xn && !p.w8 && normed_takes(EPI, p, T)) return launch_normed(EPI, p, T, units, s);

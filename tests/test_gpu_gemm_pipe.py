@@ -98,6 +98,11 @@ def test_stores_on_either_side_of_the_lines(M, N, K, slices):
     test_stores_and_sums(M, N, K, slices)
 
 
+@pytest.mark.parametrize("M,N,K", [(24, 8336, 3072), (25, 8336, 3072), (32, 12288, 3072), (25, 12544, 3072)])
+def test_more_than_24_rows_over_an_odd_multiple_of_1024(M, N, K):
+    test_stores_and_sums(M, N, K, 1)
+
+
 @pytest.mark.parametrize("M", [16, 17])
 @pytest.mark.parametrize("inter,K", [(11008, 1024), (11008, 1056), (11008, 4096), (13824, 4096), (13824, 4128)])
 def test_gated_on_either_side_of_the_lines(M, inter, K):
