@@ -17,25 +17,6 @@ using namespace pcb;
 constexpr int CHUNK = 2048, MAX_ROWS = 8, PAD = 8;    // (a row in LDS begins 8 elements behind the end of the one before)
 enum { TABLE, POST, MIX };                                           // (MIX + t: a sum whose last t streams, or all of up to t, are under way at a time)
 
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }   // (loads stay under way)
-
-// the sum over a row's waves: 8 >> log2 rows of them, row r's from r (8 >> log2 rows) on
-__device__ __forceinline__ float row_total(float s, float* part, int wave, int lane, int per, int r) {
-    s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0xb1, 0xf, 0xf, true));       // quad_perm [1,0,3,2]
-    s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x4e, 0xf, 0xf, true));       // quad_perm [2,3,0,1]
-    s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x141, 0xf, 0xf, true));      // row_half_mirror
-    s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x140, 0xf, 0xf, true));      // row_mirror
-    s += __shfl_xor(s, 16, 64);
-    s += __shfl_xor(s, 32, 64);
-    if (lane == 0) part[wave] = s;
-    lds_barrier();
-    const f4 lo = *(const f4*)part, hi = *(const f4*)(part + 4);
-    s = 0.0f;
-#pragma unroll
-    for (int w = 0; w < 8; ++w) s += (unsigned)(w - r * per) < (unsigned)per ? (w < 4 ? lo[w & 3] : hi[w & 3]) : 0.0f;
-    return s;
-}
-
 // U: k-steps a wave takes of its run, all under way at a time (fewer count); NC: chunks of four columns a thread works out
 template <typename E, int EPI, int PARTS, int U, int NC, int KIND>
 __device__ __forceinline__ void normed_block(const pcb_row_norm_args& n, const float* gain, const pcb_linear_args& a, int block, bool keeps, E* rows,

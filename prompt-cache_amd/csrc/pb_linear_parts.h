@@ -116,6 +116,26 @@ __device__ __forceinline__ void parts_block(const pcb_linear_args& a, int block,
         if (m0 + r < a.M) put<E, EPI>(to[r], finished<E, EPI>(a, to[r], n_b, acc[r], acc2[r], bv, bv2), cs);
 }
 
+// ---- the norm in the launch of its products (pb_linear_normed.hip, pb_norm_stream.hip) ----
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }   // (loads stay under way)
+
+// the sum over a row's waves: 8 >> log2 rows of them, row r's from r (8 >> log2 rows) on
+__device__ __forceinline__ float row_total(float s, float* part, int wave, int lane, int per, int r) {
+    s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0xb1, 0xf, 0xf, true));       // quad_perm [1,0,3,2]
+    s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x4e, 0xf, 0xf, true));       // quad_perm [2,3,0,1]
+    s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x141, 0xf, 0xf, true));      // row_half_mirror
+    s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x140, 0xf, 0xf, true));      // row_mirror
+    s += __shfl_xor(s, 16, 64);
+    s += __shfl_xor(s, 32, 64);
+    if (lane == 0) part[wave] = s;
+    lds_barrier();
+    const f4 lo = *(const f4*)part, hi = *(const f4*)(part + 4);
+    s = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) s += (unsigned)(w - r * per) < (unsigned)per ? (w < 4 ? lo[w & 3] : hi[w & 3]) : 0.0f;
+    return s;
+}
+
 }  // namespace pcb
 
 // Whether a launch's weights (K to a row, `rows` rows of es bytes an element) are read past the caches (nontemporal): where they come from a model whose weights

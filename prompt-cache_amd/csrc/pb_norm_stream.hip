@@ -18,18 +18,6 @@ using namespace pcb;
 constexpr int CHUNK = 2048, MAX_ROWS = 8, PAD = 8, R = 8, SKW = 8, D = 2, CUS = 256;      // (a row in LDS begins 8 elements behind the end of the one before)
 enum { TABLE, POST, MIX };                                           // what the rows are made of
 
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }   // (loads stay under way)
-
-__device__ __forceinline__ float row_sum(float s) {                                      // over a wave
-    s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0xb1, 0xf, 0xf, true));       // quad_perm [1,0,3,2]
-    s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x4e, 0xf, 0xf, true));       // quad_perm [2,3,0,1]
-    s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x141, 0xf, 0xf, true));      // row_half_mirror
-    s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x140, 0xf, 0xf, true));      // row_mirror
-    s += __shfl_xor(s, 16, 64);
-    s += __shfl_xor(s, 32, 64);
-    return s;
-}
-
 // Who has which blocks of R columns.  A workgroup has those b_step or a_step apart: b_each of the second product's, the first b_more one more; a_each of the first's, a_more one
 // more, from the workgroup on whom the second's did not reach.  apart > 0 (products of different gains): so many workgroups have the second's, the others the first's.
 struct Deal {
@@ -187,14 +175,7 @@ __global__ __launch_bounds__(512) void norm_stream_kernel(Launch n) {
         float s = 0.0f;
 #pragma unroll
         for (int k = 0; k < NC; ++k) s += on[k] ? (x[k][0] * x[k][0] + x[k][1] * x[k][1]) + (x[k][2] * x[k][2] + x[k][3] * x[k][3]) : 0.0f;
-        s = row_sum(s);
-        if (lane == 0) where[wave] = s;
-        lds_barrier();
-        const f4 lo = *(const f4*)where, hi = *(const f4*)(where + 4);
-        s = 0.0f;
-#pragma unroll
-        for (int w = 0; w < SKW; ++w) s += (unsigned)(w - r * per) < (unsigned)per ? (w < 4 ? lo[w & 3] : hi[w & 3]) : 0.0f;
-        return 1.0f / sqrtf(s / (float)W + n.eps);
+        return 1.0f / sqrtf(row_total(s, where, wave, lane, per, r) / (float)W + n.eps);
     };
     if constexpr (KIND == TABLE) {
 #pragma unroll
